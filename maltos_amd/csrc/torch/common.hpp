@@ -1,0 +1,131 @@
+// Host side between torch tensors and the C ABI (include/maltos_hip.h): shared helpers of the sources in this folder.
+//
+// What an eager training step pays per operator besides its kernels is host time: an operator whose implementation,
+// autograd formula and argument checks are Python costs 40-60 us per call (forward and backward together), several times
+// the kernel it launches at small sizes.  Here the same operators are C++ from the Python entry point to the launch.
+#pragma once
+#include <ATen/ATen.h>
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+#include <tuple>
+#include <vector>
+
+#include "../../../include/maltos_hip.h"
+
+namespace maltos {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::Edge;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+[[noreturn]] void raise_status(int status);  // the exception maltos_amd._lib.check raises for this status
+inline void check(int status) {
+  if (C10_UNLIKELY(status != MLTS_OK)) raise_status(status);
+}
+
+inline int dtype_code(const Tensor& t) {
+  if (t.scalar_type() == at::kBFloat16) return MLTS_BF16;
+  if (t.scalar_type() == at::kFloat) return MLTS_F32;
+  TORCH_CHECK_VALUE(false, "maltos_amd kernels take float32 or bfloat16 tensors, got ", t.scalar_type());
+}
+
+inline void require_gpu(const Tensor& t) {
+  TORCH_CHECK(!t.defined() || t.is_cuda(), "maltos_amd ops run on the GPU only (there is no CPU fallback); got a host tensor");
+}
+inline void require_gpu(const OptTensor& t) {
+  if (t.has_value()) require_gpu(*t);
+}
+
+inline mlts_stream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+inline bool stream_is_capturing() {
+  return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
+
+inline const void* ptr(const Tensor& t) { return t.const_data_ptr(); }
+inline void* mptr(const Tensor& t) { return t.mutable_data_ptr(); }
+inline const void* ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->const_data_ptr() : nullptr; }
+
+inline Tensor workspace(int64_t bytes, const Tensor& like) {
+  if (bytes <= 0) return Tensor();
+  return at::empty({bytes}, like.options().dtype(at::kByte));
+}
+
+// contiguous without a copy where it already is (Tensor::contiguous does the same but goes through the dispatcher)
+inline Tensor dense(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+// the kernels take any (batch, head, seq) strides but need a contiguous head_dim
+inline Tensor dense_last(const Tensor& t) { return t.stride(-1) == 1 || t.size(-1) == 1 ? t : t.contiguous(); }
+
+struct Strides3 {
+  int64_t v[3];
+  explicit Strides3(const Tensor& t) : v{t.stride(0), t.stride(1), t.stride(2)} {}
+};
+
+// [B, H, S, D] over [B, S, H, D] storage: the layout a projection output is transposed from and back to
+inline Tensor bshd_empty(int64_t B, int64_t H, int64_t S, int64_t D, const at::TensorOptions& opts) {
+  return at::empty_strided({B, H, S, D}, {S * H * D, D, H * D, 1}, opts);
+}
+
+// ---- raw launches (no autograd) -----------------------------------------------------------------------------------
+std::tuple<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, const Tensor& v, int64_t mask_mode, double scale,
+                                             const OptTensor& q_pos, const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq);
+std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                                      const Tensor& lse, int64_t mask_mode, double scale, const OptTensor& q_pos,
+                                                      const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq);
+std::tuple<Tensor, Tensor> rope_pair(const Tensor& xa, const Tensor& xb, const Tensor& cos, const Tensor& sin, const OptTensor& positions,
+                                     int64_t position_offset, bool inverse, bool in_place);
+Tensor swiglu_rows(const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t cols);
+Tensor swiglu_rows_backward(const Tensor& dh, const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t cols);
+Tensor grad_sum_slices(const Tensor& parts, const OptTensor& out, bool accumulate);
+
+void bind_ops(pybind11::module& m);    // ops.cpp
+void bind_llama(pybind11::module& m);  // llama.cpp
+
+// A backward formula over saved tensors.  The tensors are unpacked first, with autograd as it is (an unpack hook may run a
+// checkpointed forward again), then `backward` runs without autograd recording.
+struct Formula : public Node {
+  explicit Formula(size_t count) : saved_(count) {}
+  virtual variable_list backward(variable_list&& grads, const std::vector<Tensor>& saved) = 0;
+  void save(size_t slot, const Tensor& t, bool is_output = false) {
+    saved_[slot] = SavedVariable(t, is_output);
+    if (is_output) outputs_ |= uint32_t{1} << slot;
+  }
+  void save(size_t slot, const OptTensor& t) {
+    if (t.has_value()) save(slot, *t);
+  }
+  variable_list apply(variable_list&& grads) final {
+    before_unpack(grads);
+    std::vector<Tensor> values(saved_.size());
+    for (size_t i = 0; i < saved_.size(); ++i) values[i] = saved_[i].unpack((outputs_ >> i) & 1 ? getptr() : nullptr);
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    return backward(std::move(grads), values);
+  }
+  virtual void before_unpack(const variable_list&) {}
+  void release_variables() override {
+    for (SavedVariable& s : saved_) s.reset_data();
+  }
+
+ private:
+  std::vector<SavedVariable> saved_;
+  uint32_t outputs_ = 0;
+};
+
+inline OptTensor optional_tensor(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; }
+
+template <typename F>
+std::shared_ptr<F> make_formula() {
+  return std::shared_ptr<F>(new F(), torch::autograd::deleteNode);
+}
+
+}  // namespace maltos

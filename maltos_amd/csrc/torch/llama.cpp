@@ -1,0 +1,468 @@
+// The projections, the MLP and the rotary + attention block of maltos_amd/llama.py as C++ autograd nodes, and the record of
+// which parameters' gradients a backward pass has written.
+#include <algorithm>
+#include <cmath>
+#include <mutex>
+#include <numeric>
+#include <unordered_map>
+
+#include "common.hpp"
+
+namespace maltos {
+namespace {
+
+using torch::autograd::collect_next_edges;
+using torch::autograd::compute_requires_grad;
+using torch::autograd::set_history;
+
+// ---- which parameters received a gradient -------------------------------------------------------------------------------
+// Backward formulas that add into a bound `.grad` return no gradient to autograd, so an optimizer that skips parameters
+// without a gradient has to be told another way: a GradMarks holds one flag per parameter it was made for, and listeners
+// collect the parameters themselves.  Set from autograd's device thread without the interpreter lock.
+struct GradMarks;
+std::mutex& marks_mutex = *new std::mutex;  // (never destroyed, like the two below: marks may be released at exit)
+auto& marks_by_param = *new std::unordered_map<const c10::TensorImpl*, std::vector<std::pair<GradMarks*, size_t>>>;
+auto& listeners = *new std::vector<std::vector<Tensor>*>;
+
+struct GradMarks {
+  std::vector<Tensor> params;  // kept alive: their addresses are the keys
+  std::vector<uint8_t> written;
+
+  explicit GradMarks(std::vector<Tensor> ps) : params(std::move(ps)), written(params.size(), 0) {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    for (size_t i = 0; i < params.size(); ++i) marks_by_param[params[i].unsafeGetTensorImpl()].emplace_back(this, i);
+  }
+  GradMarks(const GradMarks&) = delete;
+  ~GradMarks() {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    for (const Tensor& p : params) {
+      auto it = marks_by_param.find(p.unsafeGetTensorImpl());
+      if (it == marks_by_param.end()) continue;
+      auto& v = it->second;
+      v.erase(std::remove_if(v.begin(), v.end(), [this](const auto& e) { return e.first == this; }), v.end());
+      if (v.empty()) marks_by_param.erase(it);
+    }
+  }
+  std::vector<bool> list() const {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    return std::vector<bool>(written.begin(), written.end());
+  }
+  bool all() const {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    return std::find(written.begin(), written.end(), 0) == written.end();
+  }
+  void fill(bool value) {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    std::fill(written.begin(), written.end(), value);
+  }
+};
+
+void notify_grad_written(const Tensor& param) {
+  std::lock_guard<std::mutex> lock(marks_mutex);
+  auto it = marks_by_param.find(param.unsafeGetTensorImpl());
+  if (it != marks_by_param.end())
+    for (auto& [marks, i] : it->second) marks->written[i] = 1;
+  for (std::vector<Tensor>* seen : listeners) seen->push_back(param);
+}
+
+struct GradListener {
+  std::vector<Tensor> seen;
+  bool active = false;
+  void start() {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    if (!active) listeners.push_back(&seen);
+    active = true;
+  }
+  std::vector<Tensor> stop() {
+    std::lock_guard<std::mutex> lock(marks_mutex);
+    listeners.erase(std::remove(listeners.begin(), listeners.end(), &seen), listeners.end());
+    active = false;
+    return seen;
+  }
+  GradListener() = default;
+  GradListener(const GradListener&) = delete;
+  ~GradListener() { stop(); }
+};
+
+// ---- parameters that share one flat buffer --------------------------------------------------------------------------------
+// Whether every parameter's `.grad` (or the parameter itself) still is the view of `flat` at its offset: what the flat
+// optimizer layouts ask several times a step, for every parameter of the model.
+struct FlatViews {
+  std::vector<Tensor> params;
+  std::vector<int64_t> offsets;
+  FlatViews(std::vector<Tensor> ps, std::vector<int64_t> offs) : params(std::move(ps)), offsets(std::move(offs)) {}
+  bool grads_are_views_of(const Tensor& flat) const {
+    const char* base = static_cast<const char*>(flat.const_data_ptr());
+    const int64_t size = flat.element_size();
+    for (size_t i = 0; i < params.size(); ++i) {
+      const Tensor& g = params[i].grad();
+      if (!g.defined() || g.scalar_type() != flat.scalar_type() || !g.is_contiguous() || g.const_data_ptr() != base + offsets[i] * size) return false;
+    }
+    return true;
+  }
+  bool grads_defined() const {
+    for (const Tensor& p : params)
+      if (!p.grad().defined()) return false;
+    return true;
+  }
+};
+
+// ---- products -------------------------------------------------------------------------------------------------------------
+// Number of K-splits for dW = dY^T X.  The product has only out * in outputs but `rows` (= tokens) terms each: for the
+// LLaMA-50M projections (512..1536 wide, 16384 tokens) a single GEMM fills a quarter of the 256 CUs and runs at ~85
+// TFLOP/s, the same work as a batch of 8-16 row slices reaches 300-600 TFLOP/s on MI355X.
+int64_t weight_grad_splits(int64_t rows, int64_t out_features, int64_t in_features) {
+  const int64_t tiles = ((out_features + 255) / 256) * ((in_features + 255) / 256);
+  int64_t splits = 1;
+  while (splits < 16 && tiles * splits < 128 && rows % (splits * 2) == 0 && rows / (splits * 2) >= 1024) splits *= 2;
+  return splits;
+}
+
+// dW = dy2^T x2 for [rows, out] / [rows, in] operands, as a batch of row-slice products where that fills the chip better.
+// With `grad` (the gradient buffer the weight already owns, a view of a flat gradient buffer) dW is added into it in the
+// pass that finishes it and nothing is returned.
+Tensor weight_grad(const Tensor& x2, const Tensor& dy2, const Tensor& grad) {
+  const int64_t splits = weight_grad_splits(x2.size(0), dy2.size(1), x2.size(1));
+  if (splits > 1 && x2.is_contiguous() && dy2.is_contiguous()) {
+    const int64_t rows = x2.size(0) / splits;
+    Tensor part = at::bmm(dy2.view({splits, rows, dy2.size(1)}).transpose(1, 2), x2.view({splits, rows, x2.size(1)}));
+    Tensor dw = grad_sum_slices(part, grad.defined() ? OptTensor(grad) : std::nullopt, grad.defined());  // fp32 sum, rounded once
+    return grad.defined() ? Tensor() : dw;
+  }
+  if (grad.defined()) {
+    Tensor g = grad;
+    g.addmm_(dy2.t(), x2);
+    return Tensor();
+  }
+  return at::mm(dy2.t(), x2);
+}
+
+Tensor rows2d(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
+
+Tensor project(const Tensor& x, const Tensor& weight) {
+  if (x.dim() == 2 || !x.is_contiguous()) return at::linear(x, weight);
+  c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = weight.size(0);
+  return at::mm(rows2d(x), weight.t()).view(shape);
+}
+
+// the gradient buffer that a product may be added into, or undefined
+Tensor bound_grad(const Tensor& weight, bool into_grad) {
+  if (!into_grad) return Tensor();
+  const Tensor& g = weight.grad();
+  if (!g.defined() || !g.is_contiguous() || g.scalar_type() != weight.scalar_type() || g.sizes() != weight.sizes()) return Tensor();
+  return g;
+}
+
+struct LinearBackward final : Formula {
+  enum { X, W, COUNT };
+  bool into_grad = false;
+  LinearBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosLinearBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    const Tensor &x = s[X], &w = s[W], &dy = g[0];
+    if (!dy.defined()) return {Tensor(), Tensor()};
+    Tensor dx, dw;
+    const Tensor dy2 = rows2d(dy);
+    if (task_should_compute_output(0)) dx = at::mm(dy2, w).view(x.sizes());
+    if (task_should_compute_output(1)) {
+      const Tensor grad = bound_grad(w, into_grad);
+      dw = weight_grad(rows2d(x), dy2, grad);
+      if (grad.defined()) notify_grad_written(w);  // autograd's hooks on the weight see no gradient for what was added here
+    }
+    return {dx, dw};
+  }
+};
+
+Tensor linear(const Tensor& x, const Tensor& weight, bool into_grad) {
+  std::shared_ptr<LinearBackward> fn;
+  if (compute_requires_grad(x, weight)) {
+    fn = make_formula<LinearBackward>();
+    fn->set_next_edges(collect_next_edges(x, weight));
+    fn->save(fn->X, x), fn->save(fn->W, weight);
+    fn->into_grad = into_grad;
+  }
+  Tensor y;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    y = project(x, weight);
+  }
+  if (fn) set_history(y, fn);
+  return y;
+}
+
+// ---- projections that share their input, run as ONE product over adjacent weights -----------------------------------------
+// q_proj / k_proj / v_proj (and gate_proj / up_proj) read the same activations.  When their weights are adjacent row blocks
+// of one allocation (what the flat optimizer layouts make of them), they ARE one [sum of out_features, in_features] matrix,
+// and the three (two) products are one: at LLaMA-50M sizes a 512-wide product has 128 output tiles for 256 compute units,
+// the 1536-wide one fills the chip, and the backward's three input-gradient products and their two additions become one.
+struct Adjacent {
+  Tensor weight;                     // [R, in]; undefined: the parameters are not adjacent
+  Tensor grad;                       // their gradients as one matrix like `weight`, when those are adjacent in the same order
+  std::vector<int64_t> first;        // output column of parameter i's first row
+  std::vector<size_t> order;         // parameters by address
+  std::vector<std::pair<const void*, const void*>> key;  // addresses of the parameters and their gradients this was made for
+
+  explicit Adjacent(const std::vector<Tensor>& params) {
+    for (const Tensor& p : params) key.push_back(addresses(p));
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    const Tensor& p0 = params[0];
+    for (const Tensor& p : params)
+      if (p.dim() != 2 || !p.is_cuda() || !p.is_contiguous() || p.scalar_type() != p0.scalar_type() || p.size(1) != p0.size(1) || !p.requires_grad()) return;
+    order.resize(params.size());
+    std::iota(order.begin(), order.end(), size_t{0});
+    std::sort(order.begin(), order.end(), [&](size_t i, size_t j) { return key[i].first < key[j].first; });
+    first.resize(params.size());
+    int64_t rows = 0;
+    const char* next = static_cast<const char*>(key[order[0]].first);
+    for (size_t i : order) {
+      if (key[i].first != next || !params[i].storage().is_alias_of(p0.storage())) return;
+      first[i] = rows;
+      rows += params[i].size(0);
+      next += params[i].nbytes();
+    }
+    const Tensor& base = params[order[0]];
+    weight = base.as_strided({rows, base.size(1)}, {base.size(1), 1}, base.storage_offset());
+    const Tensor g0 = params[order[0]].grad();
+    next = nullptr;
+    for (size_t i : order) {
+      const Tensor& g = params[i].grad();
+      if (!g.defined() || !g.is_contiguous() || g.scalar_type() != p0.scalar_type() || g.sizes() != params[i].sizes() ||
+          (next && key[i].second != next) || !g.storage().is_alias_of(g0.storage()))
+        return;
+      next = static_cast<const char*>(key[i].second) + g.nbytes();
+    }
+    grad = g0.as_strided(weight.sizes(), weight.strides(), g0.storage_offset());
+  }
+  static std::pair<const void*, const void*> addresses(const Tensor& p) {
+    const Tensor& g = p.grad();
+    return {p.const_data_ptr(), g.defined() ? g.const_data_ptr() : nullptr};
+  }
+  bool made_for(const std::vector<Tensor>& params) const {
+    if (params.size() != key.size()) return false;
+    for (size_t i = 0; i < params.size(); ++i)
+      if (addresses(params[i]) != key[i]) return false;
+    return true;
+  }
+};
+using AdjacentPtr = std::shared_ptr<Adjacent>;
+
+// the [rows, sum of widths] matrix whose column ranges the given [..., width_i] tensors are, in this order, when they are
+// such views of one dense buffer; undefined otherwise (then the caller copies them together)
+Tensor adjacent_columns(const std::vector<Tensor>& parts, const std::vector<size_t>& order) {
+  const Tensor& first = parts[order[0]];
+  const int64_t dims = first.dim();
+  int64_t total = 0;
+  for (size_t i : order) total += parts[i].size(-1);
+  int64_t offset = first.storage_offset();
+  for (size_t i : order) {
+    const Tensor& p = parts[i];
+    if (p.dim() != dims || p.scalar_type() != first.scalar_type() || !p.storage().is_alias_of(first.storage()) || p.storage_offset() != offset ||
+        (p.size(-1) > 1 && p.stride(-1) != 1))
+      return Tensor();
+    int64_t step = total;
+    for (int64_t d = dims - 2; d >= 0; --d) {
+      if (p.size(d) != first.size(d) || (p.size(d) > 1 && p.stride(d) != step)) return Tensor();
+      step *= p.size(d);
+    }
+    offset += p.size(-1);
+  }
+  const int64_t rows = first.numel() / first.size(-1);
+  return first.as_strided({rows, total}, {total, 1}, first.storage_offset());
+}
+
+// dW of the common matrix: added into the adjacent gradients, or returned as one gradient per parameter
+variable_list adjacent_weight_grads(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, const Tensor& x2, const Tensor& dy2) {
+  variable_list out(weights.size());
+  const Tensor grad = into_grad ? a.grad : Tensor();
+  const Tensor dw = weight_grad(x2, dy2, grad);
+  if (grad.defined()) {
+    for (const Tensor& w : weights) notify_grad_written(w);
+  } else {
+    for (size_t i = 0; i < weights.size(); ++i) out[i] = dw.narrow(0, a.first[i], weights[i].size(0));
+  }
+  return out;
+}
+
+struct AdjacentLinearsBackward final : Formula {
+  enum { X, COUNT };
+  AdjacentPtr rows;
+  bool into_grad = false;
+  std::vector<Tensor> weights;
+  AdjacentLinearsBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosAdjacentLinearsBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    const Tensor x2 = rows2d(s[X]);
+    bool all = true, any = false;
+    for (const Tensor& dy : g) all = all && dy.defined(), any = any || dy.defined();
+    variable_list out(1 + weights.size());
+    if (!any) return out;
+    Tensor dy2;
+    if (all) {
+      dy2 = adjacent_columns(g, rows->order);  // already side by side (attention's joint gradient buffer)?
+      if (!dy2.defined()) {
+        std::vector<Tensor> parts;
+        for (size_t i : rows->order) parts.push_back(g[i].reshape({-1, g[i].size(-1)}));
+        // one launch, through the Python function so that whoever counts the copies of a step sees this one
+        pybind11::gil_scoped_acquire gil;
+        dy2 = pybind11::module_::import("torch").attr("cat")(parts, 1).cast<Tensor>();
+      }
+    } else {
+      dy2 = at::empty({x2.size(0), rows->weight.size(0)}, x2.options());
+      for (size_t i = 0; i < weights.size(); ++i) {
+        Tensor part = dy2.narrow(1, rows->first[i], weights[i].size(0));
+        if (g[i].defined()) part.copy_(g[i].reshape({-1, g[i].size(-1)}));
+        else part.zero_();
+      }
+    }
+    if (task_should_compute_output(0)) out[0] = at::mm(dy2, rows->weight).view(s[X].sizes());
+    variable_list dws = adjacent_weight_grads(*rows, weights, into_grad, x2, dy2);
+    std::move(dws.begin(), dws.end(), out.begin() + 1);
+    return out;
+  }
+};
+
+template <typename F>
+std::shared_ptr<F> adjacent_formula(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
+  auto fn = make_formula<F>();
+  torch::autograd::edge_list edges = collect_next_edges(x);
+  for (const Tensor& w : weights) edges.push_back(torch::autograd::impl::gradient_edge(w));
+  fn->set_next_edges(std::move(edges));
+  fn->save(fn->X, x);
+  fn->rows = rows, fn->weights = weights, fn->into_grad = into_grad;
+  return fn;
+}
+
+// (x W_0^T, x W_1^T, ...) from one product with the parameters' common matrix, as column slices of it
+std::vector<Tensor> adjacent_linears(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
+  std::vector<Tensor> out(weights.size());
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    const Tensor y = project(x, rows->weight);
+    for (size_t i = 0; i < weights.size(); ++i) out[i] = y.narrow(-1, rows->first[i], weights[i].size(0));
+  }
+  if (at::GradMode::is_enabled()) {
+    const auto fn = adjacent_formula<AdjacentLinearsBackward>(x, rows, weights, into_grad);
+    for (const Tensor& o : out) set_history(o, fn);
+  }
+  return out;
+}
+
+// round(silu(x W_gate^T)) * (x W_up^T) (models/llama.py:205-206) with the two projections as one product; the backward
+// writes d gate and d up side by side, so that the input gradient is one product as well
+struct GateUpBackward final : Formula {
+  enum { X, GU, COUNT };
+  AdjacentPtr rows;
+  bool into_grad = false;
+  std::vector<Tensor> weights;
+  GateUpBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosGateUpBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    if (!g[0].defined()) return variable_list(3);
+    const Tensor dgu = swiglu_rows_backward(g[0], s[GU], rows->first[0], rows->first[1], weights[0].size(0));
+    const Tensor dgu2 = rows2d(dgu);
+    variable_list out(3);
+    if (task_should_compute_output(0)) out[0] = at::mm(dgu2, rows->weight).view(s[X].sizes());
+    variable_list dws = adjacent_weight_grads(*rows, weights, into_grad, rows2d(s[X]), dgu2);
+    std::move(dws.begin(), dws.end(), out.begin() + 1);
+    return out;
+  }
+};
+
+Tensor gate_up(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
+  Tensor gu, h;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    gu = project(x, rows->weight);
+    h = swiglu_rows(gu, rows->first[0], rows->first[1], weights[0].size(0));
+  }
+  if (at::GradMode::is_enabled()) {
+    const auto fn = adjacent_formula<GateUpBackward>(x, rows, weights, into_grad);
+    fn->save(fn->GU, gu);
+    set_history(h, fn);
+  }
+  return h;
+}
+
+// ---- attention(rotary(q), rotary(k), v) (models/llama.py:143-150) as one node ---------------------------------------------
+// The same kernels as the separate ops, hence the same values.  What the node adds is the layout of its backward: dQ, dK and
+// dV are head ranges of one [B, S, Hq + 2 Hkv, D] buffer and the rotation of dQ / dK back is done in place there (the buffer
+// is the node's own until it returns), so the gradient of q/k/v projections that run as one product arrives as one matrix.
+struct RopeAttentionBackward final : Formula {
+  enum { Q, K, V, OUT, LSE, COS, SIN, ROPE_POSITIONS, POSITIONS, SEQUENCES, COUNT };
+  int64_t position_offset = 0, mask_mode = 0;
+  double scale = 0;
+  RopeAttentionBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosRopeAttentionBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    if (!g[0].defined()) return variable_list(3);
+    const OptTensor pos = optional_tensor(s[POSITIONS]), seq = optional_tensor(s[SEQUENCES]);
+    auto [dq, dk, dv] = attention_backward(g[0], s[Q], s[K], s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq);
+    rope_pair(dq, dk, s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset, true, true);
+    return {dq, dk, dv};
+  }
+};
+
+Tensor rope_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cos, const Tensor& sin, const OptTensor& rope_positions,
+                      int64_t position_offset, const OptTensor& positions, const OptTensor& sequences) {
+  std::shared_ptr<RopeAttentionBackward> fn;
+  Tensor out;
+  const int64_t mask_mode = positions.has_value() ? MLTS_MASK_DOC : MLTS_MASK_CAUSAL;
+  const double scale = std::pow(static_cast<double>(q.size(-1)), -0.5);
+  if (compute_requires_grad(q, k, v)) {
+    fn = make_formula<RopeAttentionBackward>();
+    fn->set_next_edges(collect_next_edges(q, k, v));
+    fn->save(fn->V, v);
+    fn->save(fn->COS, cos), fn->save(fn->SIN, sin);
+    fn->save(fn->ROPE_POSITIONS, rope_positions), fn->save(fn->POSITIONS, positions), fn->save(fn->SEQUENCES, sequences);
+    fn->position_offset = position_offset, fn->mask_mode = mask_mode, fn->scale = scale;
+  }
+  Tensor qr, kr, lse;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    std::tie(qr, kr) = rope_pair(q, k, cos, sin, rope_positions, position_offset, false, false);
+    std::tie(out, lse) = attention_forward(qr, kr, v, mask_mode, scale, positions, positions, sequences, sequences);
+  }
+  if (fn) {
+    set_history(out, fn);
+    fn->save(fn->Q, qr), fn->save(fn->K, kr), fn->save(fn->LSE, lse), fn->save(fn->OUT, out, true);
+  }
+  return out;
+}
+
+}  // namespace
+
+void bind_llama(pybind11::module& m) {
+  using torch::wrap_pybind_function;
+  namespace py = pybind11;
+  m.def("linear", wrap_pybind_function(linear));
+  m.def("adjacent_linears", wrap_pybind_function(adjacent_linears));
+  m.def("gate_up", wrap_pybind_function(gate_up));
+  m.def("weight_grad_splits", wrap_pybind_function(weight_grad_splits));
+  m.def("adjacent_columns", wrap_pybind_function([](const std::vector<Tensor>& parts) {
+          std::vector<size_t> order(parts.size());
+          std::iota(order.begin(), order.end(), size_t{0});
+          const Tensor t = adjacent_columns(parts, order);
+          return t.defined() ? OptTensor(t) : std::nullopt;
+        }));
+  py::class_<Adjacent, AdjacentPtr>(m, "Adjacent")
+      .def(py::init<const std::vector<Tensor>&>())
+      .def("made_for", &Adjacent::made_for)
+      .def_property_readonly("adjacent", [](const Adjacent& a) { return a.weight.defined(); })
+      .def_property_readonly("weight", [](const Adjacent& a) { return a.weight.defined() ? OptTensor(a.weight) : std::nullopt; })
+      .def_property_readonly("grad", [](const Adjacent& a) { return a.grad.defined() ? OptTensor(a.grad) : std::nullopt; });
+  m.def("rope_attention", wrap_pybind_function(rope_attention));
+  m.def("notify_grad_written", wrap_pybind_function(notify_grad_written));
+  py::class_<GradMarks>(m, "GradMarks")
+      .def(py::init<std::vector<Tensor>>())
+      .def("list", &GradMarks::list)
+      .def("all", &GradMarks::all)
+      .def("fill", &GradMarks::fill);
+  py::class_<GradListener>(m, "GradListener").def(py::init<>()).def("start", &GradListener::start).def("stop", &GradListener::stop);
+  py::class_<FlatViews>(m, "FlatViews")
+      .def(py::init<std::vector<Tensor>, std::vector<int64_t>>())
+      .def("grads_are_views_of", &FlatViews::grads_are_views_of)
+      .def("grads_defined", &FlatViews::grads_defined);
+}
+
+}  // namespace maltos

@@ -24,6 +24,7 @@ import torch
 import torch.nn as nn
 
 from . import ops
+from ._native import native
 
 
 # Which parameters received a gradient in this step.  With gradients bound to a flat buffer `param.grad` is never None,
@@ -31,28 +32,24 @@ from . import ops
 # writes a parameter's gradient says so.  Autograd's own accumulation says it through a post-accumulate-grad hook that
 # the flat optimizer layout registers; code that adds into `param.grad` itself (HipLinear.accumulate_into_grad, a
 # replayed HIP graph, a reduce-scatter into a shard's gradient) calls notify_grad_written.
-_GRAD_WRITE_LISTENERS: list[list] = []
-
-
+# The record itself is kept by the extension (csrc/torch/llama.cpp), where backward formulas reach it without the interpreter.
 def notify_grad_written(param: torch.Tensor) -> None:
-    mark = param.__dict__.get("_maltos_hip_grad_written")
-    if mark is not None:
-        mark()
-    for seen in _GRAD_WRITE_LISTENERS:
-        seen.append(param)
+    native().notify_grad_written(param)
 
 
 class grad_write_listener:
     """`with grad_write_listener() as seen:` collects the parameters whose gradient is reported written inside the block
-    (what a recorder of a backward pass keeps, to report the same parameters again after every replay)."""
+    (what a recorder of a backward pass keeps, to report the same parameters again after every replay).  `seen` is filled
+    when the block ends."""
 
     def __enter__(self) -> list:
         self._seen: list = []
-        _GRAD_WRITE_LISTENERS.append(self._seen)
+        self._listener = native().GradListener()
+        self._listener.start()
         return self._seen
 
     def __exit__(self, *exc) -> None:
-        _GRAD_WRITE_LISTENERS.remove(self._seen)
+        self._seen.extend(self._listener.stop())
 
 
 def _is_flat_neighbour(prev: torch.Tensor, nxt: torch.Tensor) -> bool:
@@ -73,16 +70,26 @@ class _Segment:
         self.bound_grad = flat_g
         self.exp_avg = torch.zeros(self.numel, dtype=torch.float32, device=flat_p.device)
         self.exp_avg_sq = torch.zeros(self.numel, dtype=torch.float32, device=flat_p.device)
+        # every parameter's state["step"] is a view of one host tensor, so that a step counts all of them at once
+        self.steps = torch.zeros(len(params))
+        self.step_views = list(self.steps.unbind(0))
+        self._steps_np = self.steps.numpy()
+        self.views = native().FlatViews(params, offsets) if flat_g is not None else None
+
+    def common_step(self, state) -> int | None:
+        """The step count that all parameters share, or None if they differ (a parameter was skipped in an earlier step for
+        want of a gradient, or somebody put another tensor into its state)."""
+        if any(state[p]["step"] is not view for p, view in zip(self.params, self.step_views)):
+            return None
+        first = self._steps_np[0]
+        return int(first) if (self._steps_np == first).all() else None
 
     def flat_grad(self) -> torch.Tensor | None:
         """The grads as one flat tensor laid out like flat_p, or None if they are scattered."""
+        if self.views is not None:
+            return self.bound_grad if self.views.grads_are_views_of(self.bound_grad) else None
         grads = [p.grad for p in self.params]
         if any(g is None or not g.is_contiguous() or g.dtype != torch.float32 for g in grads):
-            return None
-        if self.bound_grad is not None:
-            base = self.bound_grad.data_ptr()
-            if all(g.data_ptr() == base + off * 4 for g, off in zip(grads, self.offsets)):
-                return self.bound_grad
             return None
         if any(off != sum(p.numel() for p in self.params[:i]) for i, off in enumerate(self.offsets)):
             return None
@@ -140,7 +147,7 @@ class FusedAdamW(torch.optim.Optimizer):
         self._segments.clear()
 
     def _adopt_state(self, seg: _Segment) -> None:
-        for p, off in zip(seg.params, seg.offsets):
+        for i, (p, off) in enumerate(zip(seg.params, seg.offsets)):
             st = self.state[p]
             n = p.numel()
             views = (seg.exp_avg[off:off + n].view_as(p), seg.exp_avg_sq[off:off + n].view_as(p))
@@ -148,12 +155,9 @@ class FusedAdamW(torch.optim.Optimizer):
                 views[0].copy_(st["exp_avg"])
                 views[1].copy_(st["exp_avg_sq"])
             st["exp_avg"], st["exp_avg_sq"] = views
-            if "step" not in st:
-                st["step"] = torch.tensor(0.0)
-            elif not torch.is_tensor(st["step"]):
-                st["step"] = torch.tensor(float(st["step"]))
-            else:
-                st["step"] = st["step"].detach().to("cpu", torch.float32)
+            if "step" in st:
+                seg.step_views[i].fill_(float(st["step"]))
+            st["step"] = seg.step_views[i]
 
     def _build_segments(self, group_index: int, group: dict[str, Any]) -> list[_Segment]:
         params = [p for p in group["params"] if p.requires_grad]
@@ -207,13 +211,11 @@ class FusedAdamW(torch.optim.Optimizer):
                          weight_decay=float(group["weight_decay"]), sq_norm=sq_norm, max_norm=max_norm)
             for seg in self._segments[gi]:
                 flat_g = seg.flat_grad()
-                # one launch over the whole segment needs one step count (the bias corrections are launch arguments);
-                # the counts differ once a parameter was skipped in an earlier step for want of a gradient
-                steps = {float(self.state[p]["step"]) for p in seg.params}
-                if flat_g is not None and len(steps) == 1:
-                    for p in seg.params:
-                        self.state[p]["step"] += 1
-                    ops.adamw_step_(seg.flat_p, flat_g, seg.exp_avg, seg.exp_avg_sq, step=int(steps.pop()) + 1,
+                # one launch over the whole segment needs one step count (the bias corrections are launch arguments)
+                step = seg.common_step(self.state) if flat_g is not None else None
+                if step is not None:
+                    seg.steps += 1
+                    ops.adamw_step_(seg.flat_p, flat_g, seg.exp_avg, seg.exp_avg_sq, step=step + 1,
                                     p_lowp=self._shadow.get(seg.flat_p.data_ptr()), **hyper)
                     continue
                 shadow = self._shadow.get(seg.flat_p.data_ptr())
@@ -290,11 +292,13 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
         self.grad_sq_norm: torch.Tensor | None = None  # device fp64 scalar, filled by copy_master_params(fuse_norm=True)
         del total
         # flat layout: which parameters' gradients were written since the last zero_grad (see notify_grad_written)
-        self._grad_written = [False] * len(model_params)
+        self._marks = None
         if self._flat_model:
-            for i, p in enumerate(model_params):
-                p.__dict__["_maltos_hip_grad_written"] = lambda i=i: self._grad_written.__setitem__(i, True)
-                p.register_post_accumulate_grad_hook(notify_grad_written)
+            self._marks = native().GradMarks(model_params)
+            self._model_views = native().FlatViews(model_params, self._offsets)
+            self._master_views = native().FlatViews(self.master_params, self._offsets)
+            for p in model_params:
+                p.register_post_accumulate_grad_hook(native().notify_grad_written)
 
     # ---- helpers --------------------------------------------------------------------------
     def _bind_model_grads(self) -> None:
@@ -305,10 +309,7 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
     def _grads_are_flat(self) -> bool:
         if not self._flat_model:
             return False
-        assert self.flat_model_grad is not None
-        base = self.flat_model_grad.data_ptr()
-        return all(p.grad is not None and p.grad.data_ptr() == base + off * 2 and p.grad.is_contiguous()
-                   for p, off in zip(self.model_params, self._offsets))
+        return self._model_views.grads_are_views_of(self.flat_model_grad)
 
     def model_param_for(self, param: nn.Parameter) -> nn.Parameter:
         return self._model_param_by_master_id.get(id(param), param)
@@ -318,7 +319,8 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
         gradient this step.  Parameters nobody reported are skipped by `step()`, as parameters whose `.grad` is None
         are by the reference (runtime/optim.py:46-50)."""
         if params is None:
-            self._grad_written = [True] * len(self.model_params)
+            if self._marks is not None:
+                self._marks.fill(True)
             return
         for p in params:
             notify_grad_written(p)
@@ -334,10 +336,10 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
                 sq = torch.empty((), dtype=torch.float64, device=self.flat_master.device)
             ops.grad_to_f32_(self.flat_master_grad, self.flat_model_grad, sq_out=sq)
             self.grad_sq_norm = sq
-            for mp in self.master_params:
-                if mp.grad is None:
-                    off = self._offsets[self.master_params.index(mp)]
-                    mp.grad = self.flat_master_grad[off:off + mp.numel()].view_as(mp)
+            if not self._master_views.grads_defined():
+                for mp, off in zip(self.master_params, self._offsets):
+                    if mp.grad is None:
+                        mp.grad = self.flat_master_grad[off:off + mp.numel()].view_as(mp)
         else:
             self.grad_sq_norm = None
             for p, mp, off in zip(self.model_params, self.master_params, self._offsets):
@@ -361,11 +363,11 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
 
     def step(self, closure=None):
         self.copy_master_params()
-        partial = self._flat_model and self._grads_are_flat() and not all(self._grad_written)
+        partial = self._flat_model and self._grads_are_flat() and not self._marks.all()
         if partial:
             # parameters without a gradient this step are left alone (no weight decay, no moment decay, no step count),
             # like parameters whose .grad is None in the reference; the others are then stepped one launch each
-            for mp, written in zip(self.master_params, self._grad_written):
+            for mp, written in zip(self.master_params, self._marks.list()):
                 if not written:
                     mp.grad = None
         try:
@@ -376,7 +378,7 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
                     if mp.grad is None:
                         mp.grad = self.flat_master_grad[off:off + mp.numel()].view_as(mp)
         # the fused step has written the bf16 model copy of everything it stepped
-        fused_writeback = self._fused and self._flat_model and (partial or all(mp.grad is not None for mp in self.master_params))
+        fused_writeback = self._fused and self._flat_model and (partial or self._master_views.grads_defined())
         if not fused_writeback:
             with torch.no_grad():
                 for p, mp in zip(self.model_params, self.master_params):
@@ -388,8 +390,9 @@ class MasterWeightsOptimizer(torch.optim.Optimizer):
         if self._flat_model:
             assert self.flat_model_grad is not None
             self.flat_model_grad.zero_()
-            self._bind_model_grads()
-            self._grad_written = [False] * len(self.model_params)
+            if not self._grads_are_flat():
+                self._bind_model_grads()
+            self._marks.fill(False)
         else:
             for p in self.model_params:
                 if set_to_none:
