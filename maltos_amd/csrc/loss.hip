@@ -1,7 +1,10 @@
-// Causal cross-entropy: loss and d(logits) from ONE read of the logits.  A block owns one row,
-// stages it in LDS (a 32000-entry bf16 row is 62.5 KiB of the CU's 160 KiB), reduces max and
-// sum-exp with 64-lane shuffles, then streams the gradient out.  Rows whose label is the ignore
+// Causal cross-entropy: loss and d(logits) from ONE read of the logits.  A block owns one row, keeps it in registers,
+// reduces max and sum-exp with 64-lane shuffles, then streams the gradient out.  Rows whose label is the ignore
 // index are never read: their gradient is zero.
+//
+// A vocabulary that the vector width does not divide (50257) leaves rows that start anywhere within 16 bytes: a row is
+// then walked as a short head, aligned 16-byte vectors, and a short tail, whose at most 2 * (vector - 1) single elements go to
+// one lane each.
 #include "common.hpp"
 
 namespace {
@@ -47,112 +50,37 @@ __global__ __launch_bounds__(1024) void ce_count_kernel(const int64_t* __restric
   }
 }
 
-// STAGED: the row lives in dynamic LDS between the passes; otherwise it is re-read from global
-// memory (L2) -- used only when a row does not fit.
-template <typename T, bool STAGED, bool VEC>
-__global__ __launch_bounds__(kCeThreads) void ce_row_kernel(const T* logits,  // may be dlogits (gradient in place)
-                                                            const int64_t* __restrict__ labels, T* dlogits,
-                                                            float* __restrict__ row_loss,
-                                                            const int32_t* __restrict__ count, int vocab,
-                                                            int64_t ignore_index) {
-  constexpr int N = Vec16<T>::N;
-  extern __shared__ __attribute__((aligned(16))) unsigned char ce_smem[];
-  __shared__ float red[kCeWaves];
-  T* srow = reinterpret_cast<T*>(ce_smem);
-  const int64_t row = blockIdx.x;
-  const int64_t label = labels[row];
-  const T* zr = logits + row * vocab;
-  T* dr = dlogits + row * vocab;
-  const int nvec = VEC ? vocab / N : 0;
+// A row as a head of single elements, whole aligned vectors and a tail of single elements.  Logits and gradient rows have the
+// same split because both buffers start 16-byte aligned (checked by the launcher).
+template <typename T>
+struct CeRow {
+  static constexpr int N = Vec16<T>::N;
+  int head, nvec, singles, vocab;
+  __device__ __forceinline__ CeRow(int64_t row, int vocab_) : vocab(vocab_) {
+    const int off = static_cast<int>((row * vocab) & (N - 1));
+    head = min(vocab, off ? N - off : 0);
+    nvec = (vocab - head) / N;
+    singles = vocab - nvec * N;
+  }
+  // column of single element t < singles (head first, then tail)
+  __device__ __forceinline__ int single(int t) const { return t < head ? t : t + nvec * N; }
+};
 
-  if (label == ignore_index) {
-    if (threadIdx.x == 0) row_loss[row] = 0.f;
-    if (VEC) {
-      Vec16<T> z;
+template <typename T>
+__device__ __forceinline__ void ce_zero_row(T* dr, const CeRow<T>& r) {
+  Vec16<T> z;
 #pragma unroll
-      for (int j = 0; j < N; ++j) z.set(j, 0.f);
-      for (int c = threadIdx.x; c < nvec; c += kCeThreads) reinterpret_cast<Vec16<T>*>(dr)[c] = z;
-    } else {
-      for (int c = threadIdx.x; c < vocab; c += kCeThreads) dr[c] = from_f32<T>(0.f);
-    }
-    return;
-  }
-  const bool label_ok = label >= 0 && label < vocab;
-
-  // pass 1: load (and stage), running max
-  float mx = -INFINITY;
-  if (VEC) {
-    for (int c = threadIdx.x; c < nvec; c += kCeThreads) {
-      Vec16<T> t;
-      t.v = __builtin_nontemporal_load(reinterpret_cast<const decltype(t.v)*>(zr) + c);
-      if (STAGED) reinterpret_cast<Vec16<T>*>(srow)[c] = t;
-#pragma unroll
-      for (int j = 0; j < N; ++j) mx = fmaxf(mx, t.get(j));
-    }
-  } else {
-    for (int c = threadIdx.x; c < vocab; c += kCeThreads) {
-      T t = zr[c];
-      if (STAGED) srow[c] = t;
-      mx = fmaxf(mx, to_f32<T>(t));
-    }
-  }
-  mx = block_max(mx, red);  // the barrier inside also publishes the staged row
-  const T* src = STAGED ? srow : zr;
-
-  // pass 2: sum exp
-  const float mxs = mx * kLog2e;
-  float se = 0.f;
-  if (VEC) {
-    for (int c = threadIdx.x; c < nvec; c += kCeThreads) {
-      Vec16<T> t = reinterpret_cast<const Vec16<T>*>(src)[c];
-#pragma unroll
-      for (int j = 0; j < N; ++j) se += exp2f(t.get(j) * kLog2e - mxs);
-    }
-  } else {
-    for (int c = threadIdx.x; c < vocab; c += kCeThreads) se += exp2f(to_f32<T>(src[c]) * kLog2e - mxs);
-  }
-  // read before the barrier inside block_sum: behind it other threads may already be storing gradients over the row
-  float label_logit = 0.f;
-  if (threadIdx.x == 0 && label_ok) label_logit = to_f32<T>(src[label]);
-  se = block_sum(se, red);
-  const float lse = mx + logf(se);
-  if (threadIdx.x == 0) {
-    row_loss[row] = label_ok ? lse - label_logit : NAN;
-  }
-
-  // pass 3: gradient
-  const int cnt = *count;
-  const float inv = 1.0f / static_cast<float>(cnt > 0 ? cnt : 1);
-  const float lses = lse * kLog2e;
-  if (VEC) {
-    const int lvec = label_ok ? static_cast<int>(label / N) : -1;
-    const int lsub = label_ok ? static_cast<int>(label % N) : 0;
-    for (int c = threadIdx.x; c < nvec; c += kCeThreads) {
-      Vec16<T> t = reinterpret_cast<const Vec16<T>*>(src)[c];
-      Vec16<T> o;
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        float p = exp2f(t.get(j) * kLog2e - lses);
-        if (c == lvec && j == lsub) p -= 1.0f;
-        o.set(j, p * inv);
-      }
-      __builtin_nontemporal_store(o.v, reinterpret_cast<decltype(o.v)*>(dr) + c);
-    }
-  } else {
-    for (int c = threadIdx.x; c < vocab; c += kCeThreads) {
-      float p = exp2f(to_f32<T>(src[c]) * kLog2e - lses);
-      if (c == label) p -= 1.0f;
-      dr[c] = from_f32<T>(p * inv);
-    }
-  }
+  for (int j = 0; j < CeRow<T>::N; ++j) z.set(j, 0.f);
+  for (int c = threadIdx.x; c < r.nvec; c += kCeThreads) __builtin_nontemporal_store(z.v, reinterpret_cast<decltype(z.v)*>(dr + r.head) + c);
+  if (static_cast<int>(threadIdx.x) < r.singles) dr[r.single(threadIdx.x)] = from_f32<T>(0.f);
 }
 
-// Row kept in registers: NV 16-byte vectors per lane (a 32000-entry bf16 row is 8 per lane of a 512-lane block), all
-// loads of a row issued before the first use.  No LDS beyond the reduction scratch, so four or more rows are in
-// flight per CU instead of the two that fit when rows are staged in LDS (six wavefronts per SIMD = three blocks per CU
-// is the register budget that still compiles without spills for eight vectors per lane).
+// Row kept in registers: NV 16-byte vectors per lane (a 32000-entry bf16 row is 8 per lane of a 512-lane block), all loads of a
+// row issued before the first use.  No LDS beyond the reduction scratch: three blocks per CU up to eight vectors per lane (the
+// register budget that still compiles without spills), two with sixteen.
+// bf16 1021 x 50257: 180 us with one 2-byte access per lane, 50 us (4.1 TB/s) in this form.
 template <typename T, int NV>
-__global__ __launch_bounds__(kCeThreads, 6) void ce_row_reg_kernel(const T* logits,  // may be dlogits (gradient in place)
+__global__ __launch_bounds__(kCeThreads, NV > 8 ? 4 : 6) void ce_row_reg_kernel(const T* logits,  // may be dlogits (gradient in place)
                                                                 const int64_t* __restrict__ labels, T* dlogits,
                                                                 float* __restrict__ row_loss,
                                                                 const int32_t* __restrict__ count, int vocab,
@@ -161,60 +89,58 @@ __global__ __launch_bounds__(kCeThreads, 6) void ce_row_reg_kernel(const T* logi
   __shared__ float red[kCeWaves];
   const int64_t row = blockIdx.x;
   const int64_t label = labels[row];
+  const CeRow<T> r(row, vocab);
   const T* zr = logits + row * vocab;
   T* dr = dlogits + row * vocab;
-  const int nvec = vocab / N;
+  const int tid = threadIdx.x;
   if (label == ignore_index) {
-    if (threadIdx.x == 0) row_loss[row] = 0.f;
-    Vec16<T> z;
-#pragma unroll
-    for (int j = 0; j < N; ++j) z.set(j, 0.f);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int c = threadIdx.x + i * kCeThreads;
-      if (c < nvec) __builtin_nontemporal_store(z.v, reinterpret_cast<decltype(z.v)*>(dr) + c);
-    }
+    if (tid == 0) row_loss[row] = 0.f;
+    ce_zero_row<T>(dr, r);
     return;
   }
   const bool label_ok = label >= 0 && label < vocab;
+  const bool has_single = tid < r.singles;
+  const int single_col = has_single ? r.single(tid) : 0;
   Vec16<T> t[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = threadIdx.x + i * kCeThreads;
-    if (c < nvec) t[i].v = __builtin_nontemporal_load(reinterpret_cast<const decltype(t[i].v)*>(zr) + c);
+    const int c = tid + i * kCeThreads;
+    if (c < r.nvec) t[i].v = __builtin_nontemporal_load(reinterpret_cast<const decltype(t[i].v)*>(zr + r.head) + c);
   }
+  const float single = has_single ? to_f32<T>(zr[single_col]) : -INFINITY;
   float label_logit = 0.f;
-  if (threadIdx.x == 0 && label_ok) label_logit = to_f32<T>(zr[label]);
-  float mx = -INFINITY;
+  if (tid == 0 && label_ok) label_logit = to_f32<T>(zr[label]);
+  float mx = single;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    if (threadIdx.x + i * kCeThreads < nvec) {
+    if (tid + i * kCeThreads < r.nvec) {
 #pragma unroll
       for (int j = 0; j < N; ++j) mx = fmaxf(mx, t[i].get(j));
     }
   }
   mx = block_max(mx, red);
   const float mxs = mx * kLog2e;
-  float se = 0.f;
+  float se = has_single ? exp2f(single * kLog2e - mxs) : 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    if (threadIdx.x + i * kCeThreads < nvec) {
+    if (tid + i * kCeThreads < r.nvec) {
 #pragma unroll
       for (int j = 0; j < N; ++j) se += exp2f(t[i].get(j) * kLog2e - mxs);
     }
   }
   se = block_sum(se, red);
   const float lse = mx + logf(se);
-  if (threadIdx.x == 0) row_loss[row] = label_ok ? lse - label_logit : NAN;
+  if (tid == 0) row_loss[row] = label_ok ? lse - label_logit : NAN;
   const int cnt = *count;
   const float inv = 1.0f / static_cast<float>(cnt > 0 ? cnt : 1);
   const float lses = lse * kLog2e;
-  const int lvec = label_ok ? static_cast<int>(label / N) : -1;
-  const int lsub = label_ok ? static_cast<int>(label % N) : 0;
+  const int lcol = label_ok ? static_cast<int>(label) - r.head : -1;  // negative: the label is in the head (or nowhere)
+  const int lvec = lcol >= 0 ? lcol / N : -1;
+  const int lsub = lcol >= 0 ? lcol % N : 0;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = threadIdx.x + i * kCeThreads;
-    if (c < nvec) {
+    const int c = tid + i * kCeThreads;
+    if (c < r.nvec) {
       Vec16<T> o;
 #pragma unroll
       for (int j = 0; j < N; ++j) {
@@ -222,8 +148,91 @@ __global__ __launch_bounds__(kCeThreads, 6) void ce_row_reg_kernel(const T* logi
         if (c == lvec && j == lsub) p -= 1.0f;
         o.set(j, p * inv);
       }
-      __builtin_nontemporal_store(o.v, reinterpret_cast<decltype(o.v)*>(dr) + c);
+      __builtin_nontemporal_store(o.v, reinterpret_cast<decltype(o.v)*>(dr + r.head) + c);
     }
+  }
+  if (has_single) {
+    float p = exp2f(single * kLog2e - lses);
+    if (single_col == label) p -= 1.0f;
+    dr[single_col] = from_f32<T>(p * inv);
+  }
+}
+
+// Rows that do not fit the registers of a block (more than 65536 bf16 or 32768 fp32 entries), and buffers that are not 16-byte
+// aligned (VEC = false: single elements throughout): max and sum in one pass (a running maximum per lane), the gradient in a
+// second one that reads the row again.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kCeThreads) void ce_row_stream_kernel(const T* logits,  // may be dlogits (gradient in place)
+                                                                   const int64_t* __restrict__ labels, T* dlogits,
+                                                                   float* __restrict__ row_loss,
+                                                                   const int32_t* __restrict__ count, int vocab,
+                                                                   int64_t ignore_index) {
+  constexpr int N = Vec16<T>::N;
+  __shared__ float red[kCeWaves];
+  const int64_t row = blockIdx.x;
+  const int64_t label = labels[row];
+  CeRow<T> r(row, vocab);
+  if (!VEC) r.head = 0, r.nvec = 0, r.singles = vocab;
+  const T* zr = logits + row * vocab;
+  T* dr = dlogits + row * vocab;
+  if (label == ignore_index) {
+    if (threadIdx.x == 0) row_loss[row] = 0.f;
+    if (VEC) {
+      ce_zero_row<T>(dr, r);
+    } else {
+      for (int c = threadIdx.x; c < vocab; c += kCeThreads) dr[c] = from_f32<T>(0.f);
+    }
+    return;
+  }
+  const bool label_ok = label >= 0 && label < vocab;
+  float m = -INFINITY, se = 0.f;
+  auto take = [&](const float* x, int n) {
+    float top = m;
+    for (int j = 0; j < n; ++j) top = fmaxf(top, x[j]);
+    const float base = top == -INFINITY ? 0.f : top;
+    if (top > m) se *= exp2f((m - base) * kLog2e), m = top;
+    for (int j = 0; j < n; ++j) se += exp2f((x[j] - base) * kLog2e);
+  };
+  for (int c = threadIdx.x; c < r.nvec; c += kCeThreads) {
+    const Vec16<T> t = reinterpret_cast<const Vec16<T>*>(zr + r.head)[c];
+    float x[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) x[j] = t.get(j);
+    take(x, N);
+  }
+  for (int c = threadIdx.x; c < r.singles; c += kCeThreads) {
+    const float x = to_f32<T>(zr[r.single(c)]);
+    take(&x, 1);
+  }
+  // read before the barriers: behind the last one other threads may already be storing gradients over the row
+  float label_logit = 0.f;
+  if (threadIdx.x == 0 && label_ok) label_logit = to_f32<T>(zr[label]);
+  const float mx = block_max(m, red);
+  se = block_sum(m == -INFINITY ? 0.f : se * exp2f((m - mx) * kLog2e), red);
+  const float lse = mx + logf(se);
+  if (threadIdx.x == 0) row_loss[row] = label_ok ? lse - label_logit : NAN;
+  const int cnt = *count;
+  const float inv = 1.0f / static_cast<float>(cnt > 0 ? cnt : 1);
+  const float lses = lse * kLog2e;
+  const int lcol = label_ok ? static_cast<int>(label) - r.head : -1;
+  const int lvec = lcol >= 0 ? lcol / N : -1;
+  const int lsub = lcol >= 0 ? lcol % N : 0;
+  for (int c = threadIdx.x; c < r.nvec; c += kCeThreads) {
+    const Vec16<T> t = reinterpret_cast<const Vec16<T>*>(zr + r.head)[c];
+    Vec16<T> o;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      float p = exp2f(t.get(j) * kLog2e - lses);
+      if (c == lvec && j == lsub) p -= 1.0f;
+      o.set(j, p * inv);
+    }
+    __builtin_nontemporal_store(o.v, reinterpret_cast<decltype(o.v)*>(dr + r.head) + c);
+  }
+  for (int s = threadIdx.x; s < r.singles; s += kCeThreads) {
+    const int c = r.single(s);
+    float p = exp2f(to_f32<T>(zr[c]) * kLog2e - lses);
+    if (c == label) p -= 1.0f;
+    dr[c] = from_f32<T>(p * inv);
   }
 }
 
@@ -271,50 +280,26 @@ __global__ __launch_bounds__(256) void scale_by_scalar_vec_kernel(T* x, const fl
   if (blockIdx.x == 0 && tail < n) x[tail] = from_f32<T>(to_f32<T>(x[tail]) * s);
 }
 
-constexpr int64_t kMaxStagedBytes = 128 * 1024;
-
 template <typename T>
-int ce_launch(const void* logits, const int64_t* labels, void* dlogits, float* row_loss, const int32_t* count,
-              int64_t rows, int vocab, int64_t ignore_index, hipStream_t st) {
+void ce_launch(const void* logits, const int64_t* labels, void* dlogits, float* row_loss, const int32_t* count,
+               int64_t rows, int vocab, int64_t ignore_index, hipStream_t st) {
   constexpr int N = Vec16<T>::N;
-  const bool vec = (vocab % N == 0) && mlts_aligned16(logits) && mlts_aligned16(dlogits);
-  const int64_t row_bytes = static_cast<int64_t>(vocab) * static_cast<int64_t>(sizeof(T));
-  const bool staged = row_bytes <= kMaxStagedBytes;
-  const size_t smem = staged ? static_cast<size_t>((row_bytes + 15) & ~15LL) : 0;
+  const bool aligned = mlts_aligned16(logits) && mlts_aligned16(dlogits);
   const T* lg = static_cast<const T*>(logits);
   T* dl = static_cast<T*>(dlogits);
-  if (vec && vocab / N <= 8 * kCeThreads) {  // the row fits the registers of one block
-    const int per_lane = (vocab / N + kCeThreads - 1) / kCeThreads;
-#define MLTS_CE_REG(NV)                                                                                              \
-  hipLaunchKernelGGL((ce_row_reg_kernel<T, NV>), dim3((unsigned)rows), dim3(kCeThreads), 0, st, lg, labels, dl, row_loss, \
-                     count, vocab, ignore_index)
-    if (per_lane <= 1) MLTS_CE_REG(1);
-    else if (per_lane <= 2) MLTS_CE_REG(2);
-    else if (per_lane <= 4) MLTS_CE_REG(4);
-    else MLTS_CE_REG(8);
+  const int per_lane = (vocab / N + kCeThreads - 1) / kCeThreads;  // whole vectors of a row per lane
+#define MLTS_CE(KERN) \
+  hipLaunchKernelGGL((KERN), dim3((unsigned)rows), dim3(kCeThreads), 0, st, lg, labels, dl, row_loss, count, vocab, ignore_index)
+#define MLTS_CE_REG(NV) MLTS_CE((ce_row_reg_kernel<T, NV>))
+  if (!aligned) MLTS_CE((ce_row_stream_kernel<T, false>));
+  else if (per_lane <= 1) MLTS_CE_REG(1);
+  else if (per_lane <= 2) MLTS_CE_REG(2);
+  else if (per_lane <= 4) MLTS_CE_REG(4);
+  else if (per_lane <= 8) MLTS_CE_REG(8);
+  else if (per_lane <= 16) MLTS_CE_REG(16);
+  else MLTS_CE((ce_row_stream_kernel<T, true>));
 #undef MLTS_CE_REG
-    return MLTS_OK;
-  }
-#define MLTS_CE_LAUNCH(ST, VC)                                                                                      \
-  do {                                                                                                              \
-    auto kern = ce_row_kernel<T, ST, VC>;                                                                           \
-    if (smem > 48 * 1024) {                                                                                         \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                                       \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));       \
-      if (e != hipSuccess) {                                                                                        \
-        mlts_set_error("mlts_ce_fwd_bwd: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));         \
-        return MLTS_ERR_LAUNCH;                                                                                     \
-      }                                                                                                             \
-    }                                                                                                               \
-    hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kCeThreads), smem, st, lg, labels, dl, row_loss, count,     \
-                       vocab, ignore_index);                                                                        \
-  } while (0)
-  if (staged && vec) MLTS_CE_LAUNCH(true, true);
-  else if (staged) MLTS_CE_LAUNCH(true, false);
-  else if (vec) MLTS_CE_LAUNCH(false, true);
-  else MLTS_CE_LAUNCH(false, false);
-#undef MLTS_CE_LAUNCH
-  return MLTS_OK;
+#undef MLTS_CE
 }
 
 }  // namespace
@@ -335,10 +320,8 @@ extern "C" int mlts_ce_fwd_bwd(const void* logits, const int64_t* labels, void* 
   hipLaunchKernelGGL(ce_count_kernel, dim3(1), dim3(1024), 0, st, labels, rows, ignore_index, count_out);
   if (rows > 0) {
     MltsKernelTimer timer("ce", st);
-    int rc = dtype == MLTS_BF16
-                 ? ce_launch<bf16_t>(logits, labels, dlogits, row_loss, count_out, rows, vocab, ignore_index, st)
-                 : ce_launch<float>(logits, labels, dlogits, row_loss, count_out, rows, vocab, ignore_index, st);
-    if (rc != MLTS_OK) return rc;
+    if (dtype == MLTS_BF16) ce_launch<bf16_t>(logits, labels, dlogits, row_loss, count_out, rows, vocab, ignore_index, st);
+    else ce_launch<float>(logits, labels, dlogits, row_loss, count_out, rows, vocab, ignore_index, st);
   }
   hipLaunchKernelGGL(ce_loss_reduce_kernel, dim3(1), dim3(kCeThreads), 0, st, row_loss, rows, count_out, loss_out);
   return mlts_check_launch("mlts_ce_fwd_bwd");
@@ -355,7 +338,7 @@ extern "C" int mlts_scale_by_device_scalar(void* x, const float* scale, int64_t 
     const int64_t per = dtype == MLTS_BF16 ? 8 : 4;
     const int64_t n_vec = n / per;
     int64_t blocks = (n_vec + 255) / 256;
-    blocks = blocks < 1 ? 1 : (blocks > 8192 ? 8192 : blocks);
+    blocks = blocks < 1 ? 1 : (blocks > 1024 ? 1024 : blocks);  // four per CU stream as fast, and leave early in the usual case
     if (dtype == MLTS_BF16)
       hipLaunchKernelGGL(scale_by_scalar_vec_kernel<bf16_t>, dim3((unsigned)blocks), dim3(256), 0, st, static_cast<bf16_t*>(x), scale, n_vec, n);
     else

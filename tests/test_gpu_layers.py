@@ -273,6 +273,30 @@ def test_cross_entropy_over_its_logits(dev, dtype, rows, vocab):
         other.backward()
 
 
+@pytest.mark.parametrize("vocab", [1, 7, 9, 4095, 4099, 32769, 50257, 65543, 65553])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_cross_entropy_rows_at_any_alignment(dev, dtype, vocab):
+    """Rows that start anywhere within 16 bytes, labels in the head, the vectors and the tail of a row, sizes around the lines
+    between rows kept in registers and rows read twice; over the logits and into a separate buffer alike."""
+    rows = 11
+    gen = torch.Generator().manual_seed(vocab)
+    logits = (torch.randn(rows, vocab, generator=gen) * 3).to(dtype).to(dev)
+    labels = torch.randint(0, vocab, (rows,), generator=gen)
+    labels[0], labels[1], labels[2] = 0, vocab - 1, -100
+    labels = labels.to(dev)
+    ref = logits.float().detach().requires_grad_(True)
+    want = torch.nn.functional.cross_entropy(ref, labels, ignore_index=-100, reduction="sum") / (rows - 1)
+    want.backward()
+    for overwrite in (False, True):
+        x = logits.clone()
+        leaf = x.requires_grad_(True)
+        loss = ops.cross_entropy(leaf * 1, labels, overwrite_logits=overwrite)
+        (grad,) = torch.autograd.grad(loss, leaf)
+        assert abs(loss.item() - want.item()) <= 1e-5 * max(1.0, abs(want.item()))
+        tol = dict(rtol=1e-4, atol=1e-7) if dtype == torch.float32 else dict(rtol=2.0 ** -7, atol=1e-6)
+        torch.testing.assert_close(grad.float(), ref.grad, **tol)
+
+
 def test_cross_entropy_without_targets_is_zero(dev):
     lg = torch.randn(2, 3, 5, device=dev, requires_grad=True)
     loss = ops.cross_entropy(lg, torch.full((2, 3), -100, device=dev))
