@@ -210,8 +210,8 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_dw_reduce_kernel(const float
 }
 
 int rmsnorm_bwd_blocks(int64_t rows) {
-  int64_t b = (rows + 31) / 32;  // >= 32 rows per block keeps the partial buffer small
-  if (b > 256) b = 256;          // one block per CU: more blocks only lengthen the reduction of their dw partials
+  int64_t b = (rows + 3) / 4;  // few rows: a wavefront each, four to a block, before any wavefront takes a second one
+  if (b > 256) b = 256;        // one block per CU: more blocks only lengthen the reduction of their dw partials
   if (b < 1) b = 1;
   return static_cast<int>(b);
 }
@@ -454,7 +454,25 @@ int rmsnorm_bwd_t(const void* dy, const void* x, const void* w, const float* rst
   const int chunks = (hidden / Vec16<T>::N + MLTS_WAVE - 1) / MLTS_WAVE;  // <= kMaxChunks, checked by the caller
 #define MLTS_RMS_BWD(CH, R, NW) \
   rmsnorm_bwd_launch<T, CH, R, NW>(dy, x, w, rstd, dres, dx, partial, rows, hidden, blocks, rows_per_block, st)
-  if (chunks <= 2) {
+  if (rows_per_block <= 16) {
+    // few rows: four wavefronts per block, as many rows of each in flight as it has (1021 x 768: 25 -> 5 us; blocks of at least
+    // 32 rows had left seven of eight CUs without one)
+    const int per_wave = (rows_per_block + 3) / 4;
+    if (chunks <= 1) {
+      if (per_wave >= 4) MLTS_RMS_BWD(1, 4, 4);
+      else if (per_wave >= 2) MLTS_RMS_BWD(1, 2, 4);
+      else MLTS_RMS_BWD(1, 1, 4);
+    } else if (chunks <= 2) {
+      if (per_wave >= 4) MLTS_RMS_BWD(2, 4, 4);
+      else if (per_wave >= 2) MLTS_RMS_BWD(2, 2, 4);
+      else MLTS_RMS_BWD(2, 1, 4);
+    } else if (chunks <= 4) {
+      if (per_wave >= 2) MLTS_RMS_BWD(4, 2, 4);
+      else MLTS_RMS_BWD(4, 1, 4);
+    } else {
+      MLTS_RMS_BWD(8, 1, 4);
+    }
+  } else if (chunks <= 2) {
     // rows of one wavefront (of 16 per block) per pass: as many as it has, up to 8 vectors per operand and lane
     const int per_wave = (rows_per_block + 15) / 16;
     if (chunks <= 1) {

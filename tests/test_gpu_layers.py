@@ -297,6 +297,21 @@ def test_cross_entropy_rows_at_any_alignment(dev, dtype, vocab):
         torch.testing.assert_close(grad.float(), ref.grad, **tol)
 
 
+@pytest.mark.parametrize("rows", [1, 3, 5, 1023, 1025, 2049, 4097])
+@pytest.mark.parametrize("hidden", [768, 2048, 4096])
+def test_rmsnorm_backward_few_rows(dev, rows, hidden):
+    """Row counts around the lines between the block shapes of the backward kernel."""
+    gen = torch.Generator().manual_seed(rows)
+    x, dy = (torch.randn(rows, hidden, generator=gen).bfloat16().to(dev) for _ in range(2))
+    w = (1 + 0.1 * torch.randn(hidden, generator=gen)).bfloat16().to(dev)
+    xf, wf = x.float().requires_grad_(True), w.float().requires_grad_(True)
+    torch.nn.functional.rms_norm(xf, (hidden,), wf, 1e-5).backward(dy.float())
+    _, rstd = torch.ops.maltos.rmsnorm_fwd(x, w, 1e-5)
+    dx, dw = torch.ops.maltos.rmsnorm_bwd(dy, x, w, rstd)
+    torch.testing.assert_close(dx.float(), xf.grad, rtol=2.0 ** -7, atol=2e-2)
+    torch.testing.assert_close(dw.float(), wf.grad, rtol=2.0 ** -7, atol=2.0 ** -8 * rows ** 0.5 + 1e-2)
+
+
 def test_cross_entropy_without_targets_is_zero(dev):
     lg = torch.randn(2, 3, 5, device=dev, requires_grad=True)
     loss = ops.cross_entropy(lg, torch.full((2, 3), -100, device=dev))
