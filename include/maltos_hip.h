@@ -101,7 +101,7 @@ int64_t mlts_attn_bwd_workspace_bytes(const mlts_attn_shape* s, int accumulate_f
  * mlts_attn_shape::doc_plan; the calls then skip their pre-pass (three small launches, 28 us at B=2, S=8192) and
  * mlts_attn_*_workspace_bytes no longer include it.  The plan must not be rewritten while a call that uses it is in
  * flight.  No counterpart in the reference, whose callers rebuild the varlen metadata per call
- * (runtime/layers/flash_utils.py:566-640).  Returns 0 bytes / does nothing for shapes the generic kernels serve. */
+ * (runtime/layers/flash_utils.py:566-640).  Returns 0 bytes / does nothing for shapes the 16-row kernels serve. */
 int64_t mlts_attn_doc_plan_bytes(const mlts_attn_shape* s);
 int mlts_attn_doc_plan(const mlts_attn_shape* s, void* plan, int64_t plan_bytes, mlts_stream_t stream);
 

@@ -1,5 +1,5 @@
 // C-ABI entry points for attention: argument validation on the host, workspace carving, kernel
-// selection (bf16 head_dim 64/128 -> MFMA kernels, everything else -> generic fp32-ALU kernels) and
+// selection (bf16 head_dim 64/128 -> the 32-row kernels, everything else -> the 16-row kernels) and
 // the log-sum-exp block merge.
 #include <mutex>
 
@@ -9,8 +9,8 @@ int mlts_attn_fwd_bf16_dma(const AttnParams& p, int D, int mode, hipStream_t st)
 int64_t mlts_attn_bwd_dkdv_split_workspace(int64_t B, int64_t Hq, int64_t Sq);                             // attn_bwd_split.hip
 int mlts_attn_bwd_dkdv_bf16_split(AttnBwdParams bp, int D, int mode, void* workspace, bool lse2_ready, hipStream_t st);    // attn_bwd_split.hip
 int mlts_attn_bwd_dq_bf16_tr(const AttnBwdParams& bp, int D, int mode, hipStream_t st);                    // attn_bwd_dq_tr.hip
-int mlts_attn_generic_fwd(const AttnParams& p, int D, int dtype, int mode, hipStream_t st);
-int mlts_attn_generic_bwd(const AttnBwdParams& bp, int D, int dtype, int mode, hipStream_t st);
+int mlts_attn_tile16_fwd(AttnParams p, int D, int dtype, int mode, hipStream_t st);                        // attn_tile16.hip
+int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int dtype, int mode, hipStream_t st);                    // attn_tile16.hip
 int mlts_attn_delta(const void* dout, const int64_t* dos, const void* o, const int64_t* os, float* delta, int B, int H,
                     int S, int D, int dtype, hipStream_t st);
 
@@ -230,13 +230,16 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
     MLTS_REQUIRE(do_stride[2] < kMaxRowStride, "%s: the sequence stride of dout must be below 2^24 elements", who);
   }
   void* lse2_ws = ws;
+  if (!uses_mfma(s)) {
+    bp.delta_out = delta;
+    return mlts_attn_tile16_bwd(bp, s->D, s->dtype, s->mask_mode, st);
+  }
   // the recomputing dQ kernel forms delta itself from 16-byte chunks of the O rows
-  const bool stats_in_dq = uses_mfma(s) && s->Sk > 0 && mlts_aligned16(o) && strides_aligned(s->o_stride, 2);
+  const bool stats_in_dq = s->Sk > 0 && mlts_aligned16(o) && strides_aligned(s->o_stride, 2);
   if (s->Sq > 0 && !stats_in_dq) {
     int rc = mlts_attn_delta(dout, do_stride, o, s->o_stride, delta, s->B, s->Hq, s->Sq, s->D, s->dtype, st);
     if (rc != MLTS_OK) return rc;
   }
-  if (!uses_mfma(s)) return mlts_attn_generic_bwd(bp, s->D, s->dtype, s->mask_mode, st);
   return attn_bwd_bf16(bp, s->D, s->mask_mode, delta, lse2_ws, stats_in_dq, st);
 }
 
@@ -579,7 +582,7 @@ extern "C" int mlts_attn_doc_plan(const mlts_attn_shape* s, void* plan, int64_t 
   mlts_attn_shape t = *s;
   t.doc_plan = nullptr;
   const int64_t need = stats_bytes(&t, true);
-  if (need == 0) return MLTS_OK;  // a shape the generic kernels serve: they evaluate the mask themselves
+  if (need == 0) return MLTS_OK;  // a shape the 16-row kernels serve: they evaluate the mask themselves
   MLTS_REQUIRE(plan && plan_bytes >= need, "mlts_attn_doc_plan: plan buffer too small (%lld < %lld)", (long long)plan_bytes,
                (long long)need);
   MLTS_REQUIRE(mlts_aligned16(plan), "mlts_attn_doc_plan: the plan buffer must be 16-byte aligned");
@@ -621,7 +624,7 @@ extern "C" int mlts_attn_fwd(const mlts_attn_shape* s, const void* q, const void
     setup_stats(p, s, false, static_cast<char*>(workspace), st);
     return mlts_attn_fwd_bf16_dma(p, s->D, s->mask_mode, st);
   }
-  return mlts_attn_generic_fwd(p, s->D, s->dtype, s->mask_mode, st);
+  return mlts_attn_tile16_fwd(p, s->D, s->dtype, s->mask_mode, st);
 }
 
 extern "C" int mlts_attn_bwd(const mlts_attn_shape* s, const void* dout, const int64_t do_stride[3], const void* q,

@@ -326,6 +326,15 @@ def test_generic_head_dims(dev, D):
         run_case(dev, torch.bfloat16, 1, 2, 2, 70, 70, D, ops.MASK_DOC, seed=D + 1)
 
 
+@pytest.mark.parametrize("B,H,Hkv,Sq,Sk", [(1, 1, 1, 1, 1), (1, 2, 1, 15, 17), (2, 4, 2, 33, 129), (3, 8, 8, 300, 300), (8, 12, 6, 513, 513)])
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.float32, 65), (torch.float32, 160), (torch.bfloat16, 32), (torch.bfloat16, 100)])
+def test_sixteen_row_kernels_at_tile_edges(dev, dtype, D, B, H, Hkv, Sq, Sk):
+    """Remainders of the 16-row, 32-unit and 64-tile sizes, head dims inside their padding, rows that are not 16-byte aligned
+    (D=65), and grids on both sides of the lines between 16, 32 and 64 rows per workgroup."""
+    for mode in (ops.MASK_CAUSAL, ops.MASK_NONE) + ((ops.MASK_DOC,) if Sq == Sk and B < 8 else ()):
+        run_case(dev, dtype, B, H, Hkv, Sq, Sk, D, mode, seed=Sq + D)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_padding_rows_give_zeros_and_no_nan(dev, dtype):
     o, lse = run_case(dev, dtype, 2, 2, 2, 200, 200, 64, ops.MASK_DOC, seed=77, max_doc=50, pad_tail=37)
