@@ -256,6 +256,18 @@ int mlts_grad_sum_slices(void* out, const void* parts, int32_t dtype, int32_t sl
  * runtime/plugins/zero_common.py:324-329).  workspace: MLTS_SQNORM_WS_BYTES. */
 int mlts_sq_norm(const float* x, int64_t n, double* sq_out, void* workspace, mlts_stream_t stream);
 
+/* The norm, scaling and AdamW passes over a list of fp32 tensors (host arrays of device pointers and element counts) in one
+ * launch per 48 tensors, for parameters that do not share a flat buffer: what the reference's optimizer does per parameter
+ * (torch's multi-tensor AdamW, train/cli.py:420-443; runtime/plugins/grad_clip.py:30-77).  Workspace of the norm:
+ * mlts_list_sq_norm_workspace_bytes. */
+int64_t mlts_list_sq_norm_workspace_bytes(const int64_t* sizes, int32_t count);
+int mlts_list_sq_norm(const float* const* tensors, const int64_t* sizes, int32_t count, double* sq_out, void* workspace,
+                      int64_t workspace_bytes, mlts_stream_t stream);
+int mlts_list_scale(float* const* tensors, const int64_t* sizes, int32_t count, float scale, mlts_stream_t stream);
+int mlts_list_adamw_step(float* const* p, const float* const* g, float* const* m, float* const* v, const int64_t* sizes,
+                         int32_t count, float lr, float beta1, float beta2, float eps, float weight_decay, int64_t step,
+                         float grad_scale, const double* sq_norm, float max_norm, mlts_stream_t stream);
+
 /* x *= scale (runtime/plugins/grad_clip.py:55-58). */
 int mlts_scale(float* x, float scale, int64_t n, mlts_stream_t stream);
 

@@ -108,6 +108,13 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "mlts_grad_to_f32": (C.c_int, [_P, _P, C.c_int32, C.c_int64, C.c_int, _P, _P, _P]),
     "mlts_grad_sum_slices": (C.c_int, [_P, _P, C.c_int32, C.c_int32, C.c_int64, C.c_int, _P]),
     "mlts_sq_norm": (C.c_int, [_P, C.c_int64, _P, _P, _P]),
+    "mlts_list_sq_norm_workspace_bytes": (C.c_int64, [_P, C.c_int32]),
+    "mlts_list_sq_norm": (C.c_int, [_P, _P, C.c_int32, _P, _P, C.c_int64, _P]),
+    "mlts_list_scale": (C.c_int, [_P, _P, C.c_int32, C.c_float, _P]),
+    "mlts_list_adamw_step": (
+        C.c_int,
+        [_P, _P, _P, _P, _P, C.c_int32, C.c_float, C.c_float, C.c_float, C.c_float, C.c_float, C.c_int64, C.c_float, _P, C.c_float, _P],
+    ),
     "mlts_scale": (C.c_int, [_P, C.c_float, C.c_int64, _P]),
     "mlts_adamw_step": (
         C.c_int,

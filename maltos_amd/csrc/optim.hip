@@ -205,6 +205,147 @@ __global__ __launch_bounds__(kThreads) void grad_bf16_to_f32_vec_kernel(float* _
   if (SQ) block_sum_f64_store(acc, partial + blockIdx.x);
 }
 
+// ---- the same passes over a list of tensors --------------------------------------------------------------------------------
+// Parameters that do not share a flat buffer would take a launch (for the norm two and an addition) each: 39 tensors of the tiny
+// fp32 model were 195 launches of 1.5-5 us, 0.5 ms of GPU time and 1.5 ms of host time per step.  A launch takes up to kListMax
+// tensors by value; tensor t owns blocks [first[t], first[t + 1]), `chunk` elements each.
+constexpr int kListMax = 48;
+
+struct TensorList {
+  int count, chunk;
+  int first[kListMax + 1];
+  int64_t n[kListMax];
+};
+__device__ __forceinline__ int list_tensor(const TensorList& l) {  // the tensor of this block (wave-uniform: scalar compares)
+  const int b = blockIdx.x;
+  int t = 0;
+  while (t + 1 < l.count && b >= l.first[t + 1]) ++t;
+  return t;
+}
+
+struct ConstPtrs {
+  const float* p[kListMax];
+};
+struct AdamPtrs {
+  float* p[kListMax];
+  const float* g[kListMax];
+  float* m[kListMax];
+  float* v[kListMax];
+};
+
+__global__ __launch_bounds__(kThreads) void list_sq_norm_kernel(const TensorList l, const ConstPtrs ptrs, double* partial) {
+  const int t = list_tensor(l);
+  const float* x = ptrs.p[t];
+  const int64_t begin = static_cast<int64_t>(blockIdx.x - l.first[t]) * l.chunk;
+  const int64_t end = min(begin + l.chunk, l.n[t]);
+  double acc = 0.0;
+  int64_t i = begin;
+  if ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) {  // (chunks are whole vectors)
+    const int64_t whole = begin + ((end - begin) & ~int64_t{3});
+    for (int64_t j = begin + 4 * threadIdx.x; j < whole; j += 4 * kThreads) {
+      const f32x4 q = *reinterpret_cast<const f32x4*>(x + j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = fma(static_cast<double>(q[e]), static_cast<double>(q[e]), acc);
+    }
+    i = whole;
+  }
+  for (i += threadIdx.x; i < end; i += kThreads) acc = fma(static_cast<double>(x[i]), static_cast<double>(x[i]), acc);
+  block_sum_f64_store(acc, partial + blockIdx.x);
+}
+
+__global__ __launch_bounds__(kThreads) void list_scale_kernel(const TensorList l, const ConstPtrs ptrs, float s) {
+  const int t = list_tensor(l);
+  float* x = const_cast<float*>(ptrs.p[t]);
+  const int64_t begin = static_cast<int64_t>(blockIdx.x - l.first[t]) * l.chunk;
+  const int64_t end = min(begin + l.chunk, l.n[t]);
+  int64_t i = begin;
+  if ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
+    const int64_t whole = begin + ((end - begin) & ~int64_t{3});
+    for (int64_t j = begin + 4 * threadIdx.x; j < whole; j += 4 * kThreads) {
+      f32x4 q = *reinterpret_cast<f32x4*>(x + j);
+      q *= s;
+      *reinterpret_cast<f32x4*>(x + j) = q;
+    }
+    i = whole;
+  }
+  for (i += threadIdx.x; i < end; i += kThreads) x[i] *= s;
+}
+
+__global__ __launch_bounds__(kThreads) void list_adamw_kernel(const TensorList l, const AdamPtrs ptrs, AdamArgs a) {
+  const int t = list_tensor(l);
+  float *p = ptrs.p[t], *m = ptrs.m[t], *v = ptrs.v[t];
+  const float* g = ptrs.g[t];
+  const float c = clip_coef(a);
+  const int64_t begin = static_cast<int64_t>(blockIdx.x - l.first[t]) * l.chunk;
+  const int64_t end = min(begin + l.chunk, l.n[t]);
+  int64_t i = begin;
+  if (((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(g)) & 15u) == 0) {
+    const int64_t whole = begin + ((end - begin) & ~int64_t{3});
+    for (int64_t j = begin + 4 * threadIdx.x; j < whole; j += 4 * kThreads) {
+      f32x4 pp = *reinterpret_cast<f32x4*>(p + j), mm = *reinterpret_cast<f32x4*>(m + j), vv = *reinterpret_cast<f32x4*>(v + j);
+      const f32x4 gg = *reinterpret_cast<const f32x4*>(g + j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float pe = pp[e], me = mm[e], ve = vv[e];
+        adam_update(pe, gg[e], me, ve, a, c);
+        pp[e] = pe, mm[e] = me, vv[e] = ve;
+      }
+      *reinterpret_cast<f32x4*>(p + j) = pp;
+      *reinterpret_cast<f32x4*>(m + j) = mm;
+      *reinterpret_cast<f32x4*>(v + j) = vv;
+    }
+    i = whole;
+  }
+  for (i += threadIdx.x; i < end; i += kThreads) {
+    float pe = p[i], me = m[i], ve = v[i];
+    adam_update(pe, g[i], me, ve, a, c);
+    p[i] = pe, m[i] = me, v[i] = ve;
+  }
+}
+
+// Elements per block such that all tensors together take about `most` blocks: small tensors get one block of 4096 elements or
+// less, a large one its share.  The norm keeps one partial sum per block.
+constexpr int kListBlocks = 8192, kListNormBlocks = 1024;
+int64_t list_chunk(const int64_t* sizes, int count, int most) {
+  int64_t total = 0;
+  for (int i = 0; i < count; ++i) total += sizes[i];
+  int64_t chunk = (total + most - 1) / most;
+  chunk = (chunk + 1023) / 1024 * 1024;
+  return chunk < 4096 ? 4096 : chunk;
+}
+// returns the number of blocks of the launch, or -1 when one tensor needs more than 2^30 of them
+int64_t list_fill(TensorList& l, const int64_t* sizes, int count, int64_t chunk) {
+  l.count = count;
+  l.chunk = static_cast<int>(chunk);
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    l.first[i] = static_cast<int>(blocks);
+    l.n[i] = sizes[i];
+    blocks += (sizes[i] + chunk - 1) / chunk;
+    if (blocks > (int64_t{1} << 30)) return -1;
+  }
+  l.first[count] = static_cast<int>(blocks);
+  return blocks;
+}
+
+bool adam_args(AdamArgs& a, float lr, float beta1, float beta2, float eps, float weight_decay, int64_t step, float grad_scale,
+               const double* sq_norm, float max_norm) {
+  if (step < 1 || !(beta1 >= 0.f && beta1 < 1.f && beta2 >= 0.f && beta2 < 1.f)) return false;
+  a.lr = lr;
+  a.beta1 = beta1;
+  a.beta2 = beta2;
+  a.eps = eps;
+  a.weight_decay = weight_decay;
+  const double bc1 = 1.0 - pow(static_cast<double>(beta1), static_cast<double>(step));
+  const double bc2 = 1.0 - pow(static_cast<double>(beta2), static_cast<double>(step));
+  a.step_size = static_cast<float>(static_cast<double>(lr) / bc1);
+  a.bc2_sqrt = static_cast<float>(sqrt(bc2));
+  a.grad_scale = grad_scale;
+  a.max_norm = max_norm;
+  a.sq_norm = sq_norm;
+  return true;
+}
+
 int grid_for(int64_t work_items, int max_blocks) {
   int64_t b = (work_items + kThreads - 1) / kThreads;
   if (b < 1) b = 1;
@@ -224,18 +365,7 @@ extern "C" int mlts_adamw_step(float* p, const float* g, float* m, float* v, voi
   MLTS_REQUIRE(beta1 >= 0.f && beta1 < 1.f && beta2 >= 0.f && beta2 < 1.f, "mlts_adamw_step: betas must be in [0, 1)");
   hipStream_t st = static_cast<hipStream_t>(stream);
   AdamArgs a;
-  a.lr = lr;
-  a.beta1 = beta1;
-  a.beta2 = beta2;
-  a.eps = eps;
-  a.weight_decay = weight_decay;
-  const double bc1 = 1.0 - pow(static_cast<double>(beta1), static_cast<double>(step));
-  const double bc2 = 1.0 - pow(static_cast<double>(beta2), static_cast<double>(step));
-  a.step_size = static_cast<float>(static_cast<double>(lr) / bc1);
-  a.bc2_sqrt = static_cast<float>(sqrt(bc2));
-  a.grad_scale = grad_scale;
-  a.max_norm = max_norm;
-  a.sq_norm = sq_norm;
+  adam_args(a, lr, beta1, beta2, eps, weight_decay, step, grad_scale, sq_norm, max_norm);
   bf16_t* plow = static_cast<bf16_t*>(p_lowp);
 
   const bool vec_ok = mlts_aligned16(p) && mlts_aligned16(g) && mlts_aligned16(m) && mlts_aligned16(v) &&
@@ -284,6 +414,85 @@ extern "C" int mlts_sq_norm(const float* x, int64_t n, double* sq_out, void* wor
   }
   hipLaunchKernelGGL(sq_norm_stage2, dim3(1), dim3(kThreads), 0, st, partial, blocks, sq_out);
   return mlts_check_launch("mlts_sq_norm");
+}
+
+extern "C" int64_t mlts_list_sq_norm_workspace_bytes(const int64_t* sizes, int32_t count) {
+  if (!sizes || count <= 0) return 0;
+  const int64_t chunk = list_chunk(sizes, count, kListNormBlocks);
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) blocks += (sizes[i] + chunk - 1) / chunk;
+  return (blocks > 0 ? blocks : 1) * static_cast<int64_t>(sizeof(double));
+}
+
+extern "C" int mlts_list_sq_norm(const float* const* tensors, const int64_t* sizes, int32_t count, double* sq_out, void* workspace,
+                                 int64_t workspace_bytes, mlts_stream_t stream) {
+  MLTS_REQUIRE(count > 0 && tensors && sizes && sq_out && workspace, "mlts_list_sq_norm: empty list or null pointer");
+  for (int i = 0; i < count; ++i) MLTS_REQUIRE(sizes[i] >= 0 && (sizes[i] == 0 || tensors[i]), "mlts_list_sq_norm: bad tensor %d", i);
+  MLTS_REQUIRE(workspace_bytes >= mlts_list_sq_norm_workspace_bytes(sizes, count), "mlts_list_sq_norm: workspace too small");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  double* partial = static_cast<double*>(workspace);
+  const int64_t chunk = list_chunk(sizes, count, kListNormBlocks);
+  int64_t done = 0;
+  for (int at = 0; at < count; at += kListMax) {
+    const int k = count - at < kListMax ? count - at : kListMax;
+    TensorList l;
+    ConstPtrs ptrs;
+    for (int i = 0; i < k; ++i) ptrs.p[i] = tensors[at + i];
+    const int64_t blocks = list_fill(l, sizes + at, k, chunk);
+    MLTS_REQUIRE(blocks >= 0, "mlts_list_sq_norm: tensors too large");
+    if (blocks > 0) hipLaunchKernelGGL(list_sq_norm_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, l, ptrs, partial + done);
+    done += blocks;
+  }
+  hipLaunchKernelGGL(sq_norm_stage2, dim3(1), dim3(kThreads), 0, st, partial, static_cast<int>(done), sq_out);
+  return mlts_check_launch("mlts_list_sq_norm");
+}
+
+extern "C" int mlts_list_scale(float* const* tensors, const int64_t* sizes, int32_t count, float scale, mlts_stream_t stream) {
+  MLTS_REQUIRE(count >= 0 && (count == 0 || (tensors && sizes)), "mlts_list_scale: null pointer");
+  for (int i = 0; i < count; ++i) MLTS_REQUIRE(sizes[i] >= 0 && (sizes[i] == 0 || tensors[i]), "mlts_list_scale: bad tensor %d", i);
+  if (count == 0) return MLTS_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t chunk = list_chunk(sizes, count, kListBlocks);
+  for (int at = 0; at < count; at += kListMax) {
+    const int k = count - at < kListMax ? count - at : kListMax;
+    TensorList l;
+    ConstPtrs ptrs;
+    for (int i = 0; i < k; ++i) ptrs.p[i] = tensors[at + i];
+    const int64_t blocks = list_fill(l, sizes + at, k, chunk);
+    MLTS_REQUIRE(blocks >= 0, "mlts_list_scale: tensors too large");
+    if (blocks > 0) hipLaunchKernelGGL(list_scale_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, l, ptrs, scale);
+  }
+  return mlts_check_launch("mlts_list_scale");
+}
+
+extern "C" int mlts_list_adamw_step(float* const* p, const float* const* g, float* const* m, float* const* v, const int64_t* sizes, int32_t count,
+                                    float lr, float beta1, float beta2, float eps, float weight_decay, int64_t step, float grad_scale,
+                                    const double* sq_norm, float max_norm, mlts_stream_t stream) {
+  MLTS_REQUIRE(count >= 0 && (count == 0 || (p && g && m && v && sizes)), "mlts_list_adamw_step: null pointer");
+  for (int i = 0; i < count; ++i)
+    MLTS_REQUIRE(sizes[i] >= 0 && (sizes[i] == 0 || (p[i] && g[i] && m[i] && v[i])), "mlts_list_adamw_step: bad tensor %d", i);
+  AdamArgs a;
+  MLTS_REQUIRE(adam_args(a, lr, beta1, beta2, eps, weight_decay, step, grad_scale, sq_norm, max_norm),
+               "mlts_list_adamw_step: step is the 1-based step count and betas are in [0, 1)");
+  if (count == 0) return MLTS_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  MltsKernelTimer timer("adamw", st);
+  const int64_t chunk = list_chunk(sizes, count, kListBlocks);
+  for (int at = 0; at < count; at += kListMax) {
+    const int k = count - at < kListMax ? count - at : kListMax;
+    TensorList l;
+    AdamPtrs ptrs;
+    for (int i = 0; i < k; ++i) {
+      ptrs.p[i] = p[at + i];
+      ptrs.g[i] = g[at + i];
+      ptrs.m[i] = m[at + i];
+      ptrs.v[i] = v[at + i];
+    }
+    const int64_t blocks = list_fill(l, sizes + at, k, chunk);
+    MLTS_REQUIRE(blocks >= 0, "mlts_list_adamw_step: tensors too large");
+    if (blocks > 0) hipLaunchKernelGGL(list_adamw_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, l, ptrs, a);
+  }
+  return mlts_check_launch("mlts_list_adamw_step");
 }
 
 extern "C" int mlts_scale(float* x, float scale, int64_t n, mlts_stream_t stream) {

@@ -554,6 +554,49 @@ Tensor scale_(const Tensor& x, double scale) {
   return x;
 }
 
+// the same passes over lists of tensors
+struct FlatList {
+  std::vector<void*> ptrs;
+  std::vector<int64_t> sizes;
+  FlatList(const std::vector<Tensor>& ts, const char* what) {
+    for (const Tensor& t : ts) {
+      require_gpu(t);
+      flat_f32(t, what);
+      ptrs.push_back(mptr(t));
+      sizes.push_back(t.numel());
+    }
+  }
+};
+
+Tensor list_sq_norm(const std::vector<Tensor>& xs) {
+  TORCH_CHECK_VALUE(!xs.empty(), "no tensors");
+  const FlatList l(xs, "x");
+  Tensor out = at::empty({}, xs[0].options().dtype(at::kDouble));
+  const int64_t bytes = mlts_list_sq_norm_workspace_bytes(l.sizes.data(), l.sizes.size());
+  Tensor ws = workspace(bytes, xs[0]);
+  check(mlts_list_sq_norm(reinterpret_cast<const float* const*>(l.ptrs.data()), l.sizes.data(), l.sizes.size(), out.mutable_data_ptr<double>(),
+                          mptr(ws), bytes, current_stream()));
+  return out;
+}
+
+void list_scale_(const std::vector<Tensor>& xs, double scale) {
+  const FlatList l(xs, "x");
+  check(mlts_list_scale(reinterpret_cast<float* const*>(l.ptrs.data()), l.sizes.data(), l.sizes.size(), scale, current_stream()));
+}
+
+void list_adamw_step_(const std::vector<Tensor>& p, const std::vector<Tensor>& g, const std::vector<Tensor>& m, const std::vector<Tensor>& v, double lr,
+                      double beta1, double beta2, double eps, double weight_decay, int64_t step, const OptTensor& sq_norm, double max_norm) {
+  require_gpu(sq_norm);
+  TORCH_CHECK_VALUE(!sq_norm.has_value() || (sq_norm->scalar_type() == at::kDouble && sq_norm->numel() == 1), "sq_norm must be a float64 scalar tensor");
+  const FlatList lp(p, "param"), lg(g, "grad"), lm(m, "exp_avg"), lv(v, "exp_avg_sq");
+  TORCH_CHECK_VALUE(lp.sizes == lg.sizes && lp.sizes == lm.sizes && lp.sizes == lv.sizes,
+                    "param, grad, exp_avg, exp_avg_sq must have the same number of elements");
+  check(mlts_list_adamw_step(reinterpret_cast<float* const*>(lp.ptrs.data()), reinterpret_cast<const float* const*>(lg.ptrs.data()),
+                             reinterpret_cast<float* const*>(lm.ptrs.data()), reinterpret_cast<float* const*>(lv.ptrs.data()), lp.sizes.data(),
+                             lp.sizes.size(), lr, beta1, beta2, eps, weight_decay, step, 1.0, static_cast<const double*>(ptr(sq_norm)), max_norm,
+                             current_stream()));
+}
+
 Tensor grad_to_f32_(const Tensor& dst, const Tensor& src, bool accumulate, const OptTensor& sq_out) {
   require_gpu(dst), require_gpu(src), require_gpu(sq_out);
   flat_f32(dst, "dst");
@@ -971,6 +1014,9 @@ void bind_ops(pybind11::module& m) {
   m.def("adamw_step_", wrap_pybind_function(adamw_step_));
   m.def("sq_norm", wrap_pybind_function(sq_norm));
   m.def("scale_", wrap_pybind_function(scale_));
+  m.def("list_sq_norm", wrap_pybind_function(list_sq_norm));
+  m.def("list_scale_", wrap_pybind_function(list_scale_));
+  m.def("list_adamw_step_", wrap_pybind_function(list_adamw_step_));
   m.def("grad_to_f32_", wrap_pybind_function(grad_to_f32_));
   m.def("grad_sum_slices", wrap_pybind_function(grad_sum_slices));
   m.def("set_doc_plan_cache_entries", wrap_pybind_function(set_doc_plan_cache_entries));

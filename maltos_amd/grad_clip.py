@@ -37,11 +37,7 @@ def global_grad_sq_norm(optimizer: torch.optim.Optimizer) -> torch.Tensor | None
     grads = _grad_tensors(optimizer)
     if not grads:
         return None
-    total = torch.zeros((), dtype=torch.float64, device=grads[0].device)
-    for g in grads:
-        g32 = g if g.dtype == torch.float32 and g.is_contiguous() else g.to(torch.float32).contiguous()
-        total += ops.sq_norm(g32.view(-1))
-    return total
+    return ops.list_sq_norm([g if g.dtype == torch.float32 and g.is_contiguous() else g.to(torch.float32).contiguous() for g in grads])
 
 
 def clip_grad_norm_(optimizer: torch.optim.Optimizer, max_norm: float) -> float | None:
@@ -58,10 +54,11 @@ def clip_grad_norm_(optimizer: torch.optim.Optimizer, max_norm: float) -> float 
         if flat is not None:
             ops.scale_(flat, clip_coef)
         else:
-            for g in _grad_tensors(optimizer):
-                if g.dtype == torch.float32 and g.is_contiguous():
-                    ops.scale_(g.view(-1), clip_coef)
-                else:
+            flat32 = lambda g: g.is_cuda and g.dtype == torch.float32 and g.is_contiguous()
+            grads = _grad_tensors(optimizer)
+            ops.list_scale_([g for g in grads if flat32(g)], clip_coef)
+            for g in grads:
+                if not flat32(g):
                     g.mul_(clip_coef)
     return global_norm
 

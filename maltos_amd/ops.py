@@ -333,6 +333,21 @@ def scale_(x: torch.Tensor, scale: float) -> torch.Tensor:
     return native().scale_(x, scale)
 
 
+def list_sq_norm(xs: list[torch.Tensor]) -> torch.Tensor:
+    """`sq_norm` over all of the float32 tensors together: one launch per 48 of them and one that adds the parts."""
+    return native().list_sq_norm(xs)
+
+
+def list_scale_(xs: list[torch.Tensor], scale: float) -> None:
+    native().list_scale_(xs, scale)
+
+
+def list_adamw_step_(p, g, m, v, *, lr: float, beta1: float, beta2: float, eps: float, weight_decay: float, step: int,
+                     sq_norm: torch.Tensor | None = None, max_norm: float = 0.0) -> None:
+    """`adamw_step_` over lists of tensors that share a step count: one launch per 48 of them."""
+    native().list_adamw_step_(p, g, m, v, lr, beta1, beta2, eps, weight_decay, step, sq_norm, max_norm)
+
+
 def grad_sum_slices(parts: torch.Tensor, out: torch.Tensor | None = None, *, accumulate: bool = False) -> torch.Tensor:
     """parts [slices, ...] -> sum over the slices, added in fp32 and rounded once; with `out` the result is written
     there (accumulate=True: added onto what `out` holds)."""

@@ -70,19 +70,7 @@ class _Segment:
         self.bound_grad = flat_g
         self.exp_avg = torch.zeros(self.numel, dtype=torch.float32, device=flat_p.device)
         self.exp_avg_sq = torch.zeros(self.numel, dtype=torch.float32, device=flat_p.device)
-        # every parameter's state["step"] is a view of one host tensor, so that a step counts all of them at once
-        self.steps = torch.zeros(len(params))
-        self.step_views = list(self.steps.unbind(0))
-        self._steps_np = self.steps.numpy()
         self.views = native().FlatViews(params, offsets) if flat_g is not None else None
-
-    def common_step(self, state) -> int | None:
-        """The step count that all parameters share, or None if they differ (a parameter was skipped in an earlier step for
-        want of a gradient, or somebody put another tensor into its state)."""
-        if any(state[p]["step"] is not view for p, view in zip(self.params, self.step_views)):
-            return None
-        first = self._steps_np[0]
-        return int(first) if (self._steps_np == first).all() else None
 
     def flat_grad(self) -> torch.Tensor | None:
         """The grads as one flat tensor laid out like flat_p, or None if they are scattered."""
@@ -91,12 +79,32 @@ class _Segment:
         grads = [p.grad for p in self.params]
         if any(g is None or not g.is_contiguous() or g.dtype != torch.float32 for g in grads):
             return None
-        if any(off != sum(p.numel() for p in self.params[:i]) for i, off in enumerate(self.offsets)):
+        if self.offsets[-1] + self.params[-1].numel() != sum(p.numel() for p in self.params):   # padding between the parameters
             return None
         for a, b in zip(grads, grads[1:]):
             if not _is_flat_neighbour(a, b):
                 return None
         return grads[0].as_strided((self.numel,), (1,))
+
+
+class _GroupLayout:
+    """The segments of one parameter group.  Every parameter's state["step"] is a view of one host tensor, so that a step counts
+    all of them at once."""
+
+    def __init__(self, segments: list[_Segment]) -> None:
+        self.segments = segments
+        self.params = [p for seg in segments for p in seg.params]
+        self.steps = torch.zeros(len(self.params))
+        self.step_views = list(self.steps.unbind(0))
+        self._steps_np = self.steps.numpy()
+
+    def common_step(self, state) -> int | None:
+        """The step count that all parameters share, or None if they differ (a parameter was skipped in an earlier step for
+        want of a gradient, or somebody put another tensor into its state)."""
+        if not self.params or any(state[p]["step"] is not view for p, view in zip(self.params, self.step_views)):
+            return None
+        first = self._steps_np[0]
+        return int(first) if (self._steps_np == first).all() else None
 
 
 class FusedAdamW(torch.optim.Optimizer):
@@ -123,7 +131,7 @@ class FusedAdamW(torch.optim.Optimizer):
         if weight_decay < 0:
             raise ValueError(f"Invalid weight_decay value: {weight_decay}")
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
-        self._segments: dict[int, list[_Segment]] = {}
+        self._segments: dict[int, _GroupLayout] = {}
         self._shadow: dict[int, torch.Tensor] = {}
         self._clip: tuple[torch.Tensor, float] | None = None
         self._bound = None
@@ -146,20 +154,23 @@ class FusedAdamW(torch.optim.Optimizer):
         self._bound = (flat_p, flat_g, list(params), list(offsets))
         self._segments.clear()
 
-    def _adopt_state(self, seg: _Segment) -> None:
-        for i, (p, off) in enumerate(zip(seg.params, seg.offsets)):
-            st = self.state[p]
-            n = p.numel()
-            views = (seg.exp_avg[off:off + n].view_as(p), seg.exp_avg_sq[off:off + n].view_as(p))
-            if "exp_avg" in st:  # state restored from a checkpoint: keep its values
-                views[0].copy_(st["exp_avg"])
-                views[1].copy_(st["exp_avg_sq"])
-            st["exp_avg"], st["exp_avg_sq"] = views
-            if "step" in st:
-                seg.step_views[i].fill_(float(st["step"]))
-            st["step"] = seg.step_views[i]
+    def _adopt_state(self, layout: _GroupLayout) -> None:
+        step_views = iter(layout.step_views)
+        for seg in layout.segments:
+            for p, off in zip(seg.params, seg.offsets):
+                st = self.state[p]
+                n = p.numel()
+                views = (seg.exp_avg[off:off + n].view_as(p), seg.exp_avg_sq[off:off + n].view_as(p))
+                if "exp_avg" in st:  # state restored from a checkpoint: keep its values
+                    views[0].copy_(st["exp_avg"])
+                    views[1].copy_(st["exp_avg_sq"])
+                st["exp_avg"], st["exp_avg_sq"] = views
+                step = next(step_views)
+                if "step" in st:
+                    step.fill_(float(st["step"]))
+                st["step"] = step
 
-    def _build_segments(self, group_index: int, group: dict[str, Any]) -> list[_Segment]:
+    def _build_segments(self, group_index: int, group: dict[str, Any]) -> _GroupLayout:
         params = [p for p in group["params"] if p.requires_grad]
         for p in params:
             if not p.is_cuda or p.dtype != torch.float32 or not p.is_contiguous():
@@ -187,9 +198,9 @@ class FusedAdamW(torch.optim.Optimizer):
                 run.append(p)
             if run:
                 close(run)
-        for seg in segments:
-            self._adopt_state(seg)
-        return segments
+        layout = _GroupLayout(segments)
+        self._adopt_state(layout)
+        return layout
 
     def load_state_dict(self, state_dict: dict[str, Any]) -> None:
         super().load_state_dict(state_dict)
@@ -209,15 +220,21 @@ class FusedAdamW(torch.optim.Optimizer):
             beta1, beta2 = group["betas"]
             hyper = dict(lr=float(group["lr"]), beta1=float(beta1), beta2=float(beta2), eps=float(group["eps"]),
                          weight_decay=float(group["weight_decay"]), sq_norm=sq_norm, max_norm=max_norm)
-            for seg in self._segments[gi]:
-                flat_g = seg.flat_grad()
-                # one launch over the whole segment needs one step count (the bias corrections are launch arguments)
-                step = seg.common_step(self.state) if flat_g is not None else None
-                if step is not None:
-                    seg.steps += 1
-                    ops.adamw_step_(seg.flat_p, flat_g, seg.exp_avg, seg.exp_avg_sq, step=step + 1,
-                                    p_lowp=self._shadow.get(seg.flat_p.data_ptr()), **hyper)
-                    continue
+            layout = self._segments[gi]
+            flat_grads = [seg.flat_grad() for seg in layout.segments]
+            # launches over whole segments need one step count (the bias corrections are launch arguments)
+            step = layout.common_step(self.state) if all(g is not None for g in flat_grads) else None
+            if step is not None:
+                layout.steps += 1
+                if len(layout.segments) == 1 or self._shadow:
+                    for seg, g in zip(layout.segments, flat_grads):
+                        ops.adamw_step_(seg.flat_p, g, seg.exp_avg, seg.exp_avg_sq, step=step + 1,
+                                        p_lowp=self._shadow.get(seg.flat_p.data_ptr()), **hyper)
+                else:   # parameters in allocations of their own: all of them in one launch
+                    ops.list_adamw_step_([seg.flat_p for seg in layout.segments], flat_grads, [seg.exp_avg for seg in layout.segments],
+                                         [seg.exp_avg_sq for seg in layout.segments], step=step + 1, **hyper)
+                continue
+            for seg in layout.segments:
                 shadow = self._shadow.get(seg.flat_p.data_ptr())
                 for p, offset in zip(seg.params, seg.offsets):
                     n = p.numel()

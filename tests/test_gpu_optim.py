@@ -57,6 +57,30 @@ def test_fused_adamw_matches_library_fp32(dev):
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-7)
 
 
+@pytest.mark.parametrize("count,biggest", [(1, 7), (3, 4096), (48, 5000), (49, 4097), (100, 300000)])
+def test_list_passes_equal_the_flat_ones(dev, count, biggest):
+    """Norm, scaling and AdamW over a list of tensors: sizes around a block's elements, an unaligned view, more tensors than one
+    launch takes."""
+    from maltos_amd import ops
+
+    gen = torch.Generator().manual_seed(count)
+    sizes = [1 + int(torch.randint(0, biggest, (1,), generator=gen)) for _ in range(count - 1)] + [biggest]
+    make = lambda: [torch.randn(n + 1, generator=gen).to(dev)[(i == 0):][:n] for i, n in enumerate(sizes)]
+    p, g, m, v = make(), make(), make(), [t.abs() for t in make()]
+    want_sq = sum(float(t.double().pow(2).sum()) for t in g)
+    sq = ops.list_sq_norm(g)
+    assert abs(float(sq) - want_sq) <= 1e-12 * want_sq
+    hyper = dict(lr=1e-3, beta1=0.9, beta2=0.95, eps=1e-8, weight_decay=0.1, step=3, sq_norm=sq, max_norm=1.0)
+    flat = [[t.clone() for t in ts] for ts in (p, g, m, v)]
+    for args in zip(*flat):
+        ops.adamw_step_(*args, **hyper)
+    ops.list_adamw_step_(p, g, m, v, **hyper)
+    for mine, want in zip((p, m, v), (flat[0], flat[2], flat[3])):
+        assert all(torch.equal(a, b) for a, b in zip(mine, want))
+    ops.list_scale_(g, 0.25)
+    assert all(torch.equal(a, b * 0.25) for a, b in zip(g, flat[1]))
+
+
 @pytest.mark.parametrize("inner", ["fused", "stock"])
 @pytest.mark.parametrize("flat", [True, False])
 def test_master_weights_optimizer_bf16(dev, inner, flat):
