@@ -256,6 +256,22 @@ int mlts_grad_sum_slices(void* out, const void* parts, int32_t dtype, int32_t sl
  * runtime/plugins/zero_common.py:324-329).  workspace: MLTS_SQNORM_WS_BYTES. */
 int mlts_sq_norm(const float* x, int64_t n, double* sq_out, void* workspace, mlts_stream_t stream);
 
+/* Matrix products of the linear layers (models/llama.py:69-75,134-142,196-206 and their gradients, which the reference leaves to
+ * the vendor library through torch): C[M, N] = A B, row major, fp32 accumulation, one rounding.
+ *   MLTS_GEMM_NT  A[M, K] B[N, K]   y = x W^T
+ *   MLTS_GEMM_NN  A[M, K] B[K, N]   dx = dy W
+ *   MLTS_GEMM_TN  A[K, M] B[K, N]   dW = dy^T x; C dense
+ * ld*: elements between rows.  accumulate != 0: added onto C in fp32 before the rounding.  mlts_gemm_supports: NULL, or why a
+ * product is not served (alignment of 16 bytes along rows, operands below 2 GiB).  Workspace: mlts_gemm_workspace_bytes (the
+ * fp32 parts of a contraction that is split over workgroups; 0 for most). */
+#define MLTS_GEMM_NT 0
+#define MLTS_GEMM_NN 1
+#define MLTS_GEMM_TN 2
+const char* mlts_gemm_supports(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc);
+int64_t mlts_gemm_workspace_bytes(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K);
+int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb,
+              void* c, int64_t ldc, int32_t accumulate, void* workspace, int64_t workspace_bytes, mlts_stream_t stream);
+
 /* The norm, scaling and AdamW passes over a list of fp32 tensors (host arrays of device pointers and element counts) in one
  * launch per 48 tensors, for parameters that do not share a flat buffer: what the reference's optimizer does per parameter
  * (torch's multi-tensor AdamW, train/cli.py:420-443; runtime/plugins/grad_clip.py:30-77).  Workspace of the norm:

@@ -89,6 +89,10 @@ Tensor swiglu_rows(const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t c
 Tensor swiglu_rows_backward(const Tensor& dh, const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t cols);
 Tensor grad_sum_slices(const Tensor& parts, const OptTensor& out, bool accumulate);
 
+bool own_product(int form, const Tensor& a, const Tensor& b);  // whether `product` runs on the own kernels: by size, type, layout
+// a, b as the form (MLTS_GEMM_*) says -> [M, N], written to `out` (or added onto it) if that is given
+Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out = Tensor(), bool accumulate = false);  // products.cpp
+
 void bind_ops(pybind11::module& m);    // ops.cpp
 void bind_llama(pybind11::module& m);  // llama.cpp
 

@@ -118,32 +118,29 @@ int64_t weight_grad_splits(int64_t rows, int64_t out_features, int64_t in_featur
   return splits;
 }
 
-// dW = dy2^T x2 for [rows, out] / [rows, in] operands, as a batch of row-slice products where that fills the chip better.
-// With `grad` (the gradient buffer the weight already owns, a view of a flat gradient buffer) dW is added into it in the
-// pass that finishes it and nothing is returned.
+// dW = dy2^T x2 for [rows, out] / [rows, in] operands, large ones as a batch of row-slice products where that fills the chip
+// better.  With `grad` (the gradient buffer the weight already owns, a view of a flat gradient buffer) dW is added into it in
+// the pass that finishes it and nothing is returned.
 Tensor weight_grad(const Tensor& x2, const Tensor& dy2, const Tensor& grad) {
   const int64_t splits = weight_grad_splits(x2.size(0), dy2.size(1), x2.size(1));
-  if (splits > 1 && x2.is_contiguous() && dy2.is_contiguous()) {
+  if (splits > 1 && x2.is_contiguous() && dy2.is_contiguous() && !own_product(MLTS_GEMM_TN, dy2, x2)) {
     const int64_t rows = x2.size(0) / splits;
     Tensor part = at::bmm(dy2.view({splits, rows, dy2.size(1)}).transpose(1, 2), x2.view({splits, rows, x2.size(1)}));
     Tensor dw = grad_sum_slices(part, grad.defined() ? OptTensor(grad) : std::nullopt, grad.defined());  // fp32 sum, rounded once
     return grad.defined() ? Tensor() : dw;
   }
-  if (grad.defined()) {
-    Tensor g = grad;
-    g.addmm_(dy2.t(), x2);
-    return Tensor();
-  }
-  return at::mm(dy2.t(), x2);
+  Tensor dw = product(MLTS_GEMM_TN, dy2, x2, grad, grad.defined());
+  return grad.defined() ? Tensor() : dw;
 }
 
 Tensor rows2d(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
 
 Tensor project(const Tensor& x, const Tensor& weight) {
-  if (x.dim() == 2 || !x.is_contiguous()) return at::linear(x, weight);
+  if (x.dim() == 2 && x.is_contiguous()) return product(MLTS_GEMM_NT, x, weight);
+  if (!x.is_contiguous()) return at::linear(x, weight);
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = weight.size(0);
-  return at::mm(rows2d(x), weight.t()).view(shape);
+  return product(MLTS_GEMM_NT, rows2d(x), weight).view(shape);
 }
 
 // the gradient buffer that a product may be added into, or undefined
@@ -164,7 +161,7 @@ struct LinearBackward final : Formula {
     if (!dy.defined()) return {Tensor(), Tensor()};
     Tensor dx, dw;
     const Tensor dy2 = rows2d(dy);
-    if (task_should_compute_output(0)) dx = at::mm(dy2, w).view(x.sizes());
+    if (task_should_compute_output(0)) dx = product(MLTS_GEMM_NN, dy2, w).view(x.sizes());
     if (task_should_compute_output(1)) {
       const Tensor grad = bound_grad(w, into_grad);
       dw = weight_grad(rows2d(x), dy2, grad);
@@ -315,7 +312,7 @@ struct AdjacentLinearsBackward final : Formula {
         else part.zero_();
       }
     }
-    if (task_should_compute_output(0)) out[0] = at::mm(dy2, rows->weight).view(s[X].sizes());
+    if (task_should_compute_output(0)) out[0] = product(MLTS_GEMM_NN, dy2, rows->weight).view(s[X].sizes());
     variable_list dws = adjacent_weight_grads(*rows, weights, into_grad, x2, dy2);
     std::move(dws.begin(), dws.end(), out.begin() + 1);
     return out;
@@ -362,7 +359,7 @@ struct GateUpBackward final : Formula {
     const Tensor dgu = swiglu_rows_backward(g[0], s[GU], rows->first[0], rows->first[1], weights[0].size(0));
     const Tensor dgu2 = rows2d(dgu);
     variable_list out(3);
-    if (task_should_compute_output(0)) out[0] = at::mm(dgu2, rows->weight).view(s[X].sizes());
+    if (task_should_compute_output(0)) out[0] = product(MLTS_GEMM_NN, dgu2, rows->weight).view(s[X].sizes());
     variable_list dws = adjacent_weight_grads(*rows, weights, into_grad, rows2d(s[X]), dgu2);
     std::move(dws.begin(), dws.end(), out.begin() + 1);
     return out;
@@ -436,6 +433,10 @@ void bind_llama(pybind11::module& m) {
   using torch::wrap_pybind_function;
   namespace py = pybind11;
   m.def("linear", wrap_pybind_function(linear));
+  m.def("product", wrap_pybind_function([](int form, const Tensor& a, const Tensor& b, const OptTensor& out, bool accumulate) {
+          at::AutoDispatchBelowADInplaceOrView below_autograd;
+          return product(form, a, b, out.value_or(Tensor()), accumulate);
+        }), py::arg("form"), py::arg("a"), py::arg("b"), py::arg("out") = py::none(), py::arg("accumulate") = false);
   m.def("adjacent_linears", wrap_pybind_function(adjacent_linears));
   m.def("gate_up", wrap_pybind_function(gate_up));
   m.def("weight_grad_splits", wrap_pybind_function(weight_grad_splits));

@@ -1,0 +1,57 @@
+// Matrix products of the linear layers: the kernels of csrc/gemm.hip up to a size, the vendor library through torch above it.
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+
+#include "common.hpp"
+
+namespace maltos {
+namespace {
+
+// M * N * K up to which the own kernels run.  A product through torch costs 18 us of host time, a call here 5, and that is what
+// small steps wait for: up to a few thousand rows of a 512-wide model the host is behind the GPU.  There the own kernels are
+// the faster ones on the GPU as well (1023 x 512 x 32000, dx: 45 us against the library's 145; 512-wide: 9 against 12).  From
+// 16384 x 512 x 512 on a step fills the GPU for longer than the host needs, and the library's kernels, with the shipped
+// per-shape selection, are ahead: a training step of that size took 90 us more of 9500 with its 512-wide products done here.
+constexpr double kOwnLimit = 4.0e9;
+
+struct Sizes {
+  int64_t M, N, K;
+  Sizes(int form, const Tensor& a, const Tensor& b)
+      : M(form == MLTS_GEMM_TN ? a.size(1) : a.size(0)), N(form == MLTS_GEMM_NT ? b.size(0) : b.size(1)), K(form == MLTS_GEMM_TN ? a.size(0) : a.size(1)) {}
+};
+
+bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
+bool plain(const Tensor& t) { return t.is_cuda() && t.dim() == 2 && (t.stride(1) == 1 || t.size(1) == 1) && !at::isTensorSubclassLike(t); }
+
+Tensor library_product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
+  const Tensor x = form == MLTS_GEMM_TN ? a.t() : a, y = form == MLTS_GEMM_NT ? b.t() : b;
+  if (!out.defined()) return at::mm(x, y);
+  Tensor o = out;
+  return accumulate ? o.addmm_(x, y) : at::mm_out(o, x, y);
+}
+
+}  // namespace
+
+bool own_product(int form, const Tensor& a, const Tensor& b) {
+  const Sizes z(form, a, b);
+  return static_cast<double>(z.M) * static_cast<double>(z.N) * static_cast<double>(z.K) <= kOwnLimit && z.M > 0 && z.N > 0 && z.K > 0 && plain(a) &&
+         plain(b) && a.scalar_type() == b.scalar_type() && (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) &&
+         mlts_gemm_supports(form, dtype_code(a), z.M, z.N, z.K, a.stride(0), b.stride(0), z.N) == nullptr && aligned(a) && aligned(b) &&
+         !c10::impl::dispatch_mode_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA);
+}
+
+Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
+  if (!own_product(form, a, b) || (out.defined() && !(plain(out) && out.is_contiguous() && aligned(out) && out.scalar_type() == a.scalar_type())))
+    return library_product(form, a, b, out, accumulate);
+  const Sizes z(form, a, b);
+  Tensor c = out.defined() ? out : at::empty({z.M, z.N}, a.options());
+  const int dtype = dtype_code(a);
+  const int64_t ws_bytes = mlts_gemm_workspace_bytes(form, dtype, z.M, z.N, z.K);
+  Tensor ws = workspace(ws_bytes, a);
+  check(mlts_gemm(form, dtype, z.M, z.N, z.K, ptr(a), a.stride(0), ptr(b), b.stride(0), mptr(c), z.N, accumulate,
+                  ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
+  return c;
+}
+
+}  // namespace maltos
