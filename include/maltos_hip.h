@@ -183,7 +183,18 @@ int mlts_add_rmsnorm_fwd(const void* x, const void* res, void* sum_out, const vo
 int mlts_add_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* rstd, const void* dres, void* dx,
                          void* dw, void* workspace, int64_t workspace_bytes, int64_t rows, int32_t hidden, int32_t dtype,
                          mlts_stream_t stream);
+/* Both (dres NULL: no residual path), with the weight gradient added onto dw in fp32 and rounded once. */
+int mlts_rmsnorm_bwd_accumulate(const void* dy, const void* x, const void* w, const float* rstd, const void* dres, void* dx,
+                                void* dw, void* workspace, int64_t workspace_bytes, int64_t rows, int32_t hidden,
+                                int32_t dtype, mlts_stream_t stream);
 
+
+/* Token-embedding gradient (nn.Embedding, models/llama.py:238): dw[ids[t]] += dy[t].  ids int64 [n] (ids outside
+ * [0, vocab) are skipped: the forward lookup rejects them), dy [n, hidden], dw [vocab, hidden]; equal ids are summed in fp32 in a fixed order and added onto dw with one rounding.
+ * mlts_embedding_bwd_supports: NULL, or why these sizes are not taken. */
+const char* mlts_embedding_bwd_supports(int64_t n, int64_t hidden, int64_t vocab, int32_t dtype);
+int mlts_embedding_bwd(const int64_t* ids, const void* dy, void* dw, int64_t n, int64_t hidden, int64_t vocab, int32_t dtype,
+                       mlts_stream_t stream);
 
 /* Interleaved-pair rotary embedding (models/llama.py:89-94,134-144):
  *   (x[2i], x[2i+1]) -> (x[2i] c - x[2i+1] s, x[2i] s + x[2i+1] c), c/s = cos/sin[pos, i],

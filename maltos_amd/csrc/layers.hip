@@ -182,9 +182,10 @@ __global__ __launch_bounds__(NW * MLTS_WAVE) void rmsnorm_bwd_kernel(const T* __
 
 // dw[col] = sum over the per-block partial rows, in a fixed order: a block owns 32 columns, its 8 groups of 32
 // lanes each add every 8th partial row (four loads in flight), then the 8 group sums are added through LDS.
+// accumulate: added onto dw instead, in fp32, rounded once.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void rmsnorm_dw_reduce_kernel(const float* __restrict__ dw_partial, int nblocks,
-                                                                     int hidden, T* __restrict__ dw) {
+                                                                     int hidden, T* __restrict__ dw, int accumulate) {
   __shared__ float part[8][32];
   const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
   const int col = blockIdx.x * 32 + c;
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_dw_reduce_kernel(const float
     float s = part[0][c];
 #pragma unroll
     for (int i = 1; i < 8; ++i) s += part[i][c];
-    dw[col] = from_f32<T>(s);
+    dw[col] = from_f32<T>(accumulate ? s + to_f32<T>(dw[col]) : s);
   }
 }
 
@@ -447,7 +448,7 @@ void rmsnorm_bwd_launch(const void* dy, const void* x, const void* w, const floa
 
 template <typename T>
 int rmsnorm_bwd_t(const void* dy, const void* x, const void* w, const float* rstd, const void* dres, void* dx, void* dw,
-                  float* partial, int64_t rows, int hidden, hipStream_t st) {
+                  int accumulate, float* partial, int64_t rows, int hidden, hipStream_t st) {
   const int blocks = rmsnorm_bwd_blocks(rows);
   const int rows_per_block = static_cast<int>((rows + blocks - 1) / blocks);
   MltsKernelTimer timer("rmsnorm_bwd", st);
@@ -492,7 +493,7 @@ int rmsnorm_bwd_t(const void* dy, const void* x, const void* w, const float* rst
   }
 #undef MLTS_RMS_BWD
   hipLaunchKernelGGL(rmsnorm_dw_reduce_kernel<T>, dim3((hidden + 31) / 32), dim3(kThreads), 0, st,
-                     partial, blocks, hidden, static_cast<T*>(dw));
+                     partial, blocks, hidden, static_cast<T*>(dw), accumulate);
   return mlts_check_launch("mlts_rmsnorm_bwd");
 }
 
@@ -603,8 +604,8 @@ extern "C" int64_t mlts_rmsnorm_bwd_workspace_bytes(int64_t rows, int32_t hidden
 
 namespace {
 int rmsnorm_bwd_checked(const char* who, const void* dy, const void* x, const void* w, const float* rstd, const void* dres,
-                        void* dx, void* dw, void* workspace, int64_t workspace_bytes, int64_t rows, int32_t hidden,
-                        int32_t dtype, mlts_stream_t stream) {
+                        void* dx, void* dw, int32_t accumulate, void* workspace, int64_t workspace_bytes, int64_t rows,
+                        int32_t hidden, int32_t dtype, mlts_stream_t stream) {
   MLTS_REQUIRE(known_dtype(dtype), "%s: unknown dtype %d", who, dtype);
   MLTS_REQUIRE(rows > 0 && hidden > 0, "%s: bad shape rows=%lld hidden=%d", who, (long long)rows, hidden);
   const int n = elem_per_vec(dtype);
@@ -618,15 +619,15 @@ int rmsnorm_bwd_checked(const char* who, const void* dy, const void* x, const vo
                who, (long long)workspace_bytes, (long long)mlts_rmsnorm_bwd_workspace_bytes(rows, hidden));
   hipStream_t st = static_cast<hipStream_t>(stream);
   float* partial = static_cast<float*>(workspace);
-  return dtype == MLTS_BF16 ? rmsnorm_bwd_t<bf16_t>(dy, x, w, rstd, dres, dx, dw, partial, rows, hidden, st)
-                            : rmsnorm_bwd_t<float>(dy, x, w, rstd, dres, dx, dw, partial, rows, hidden, st);
+  return dtype == MLTS_BF16 ? rmsnorm_bwd_t<bf16_t>(dy, x, w, rstd, dres, dx, dw, accumulate, partial, rows, hidden, st)
+                            : rmsnorm_bwd_t<float>(dy, x, w, rstd, dres, dx, dw, accumulate, partial, rows, hidden, st);
 }
 }  // namespace
 
 extern "C" int mlts_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* rstd, void* dx, void* dw,
                                 void* workspace, int64_t workspace_bytes, int64_t rows, int32_t hidden, int32_t dtype,
                                 mlts_stream_t stream) {
-  return rmsnorm_bwd_checked("mlts_rmsnorm_bwd", dy, x, w, rstd, nullptr, dx, dw, workspace, workspace_bytes, rows, hidden,
+  return rmsnorm_bwd_checked("mlts_rmsnorm_bwd", dy, x, w, rstd, nullptr, dx, dw, 0, workspace, workspace_bytes, rows, hidden,
                              dtype, stream);
 }
 
@@ -634,7 +635,14 @@ extern "C" int mlts_add_rmsnorm_bwd(const void* dy, const void* x, const void* w
                                     void* dx, void* dw, void* workspace, int64_t workspace_bytes, int64_t rows,
                                     int32_t hidden, int32_t dtype, mlts_stream_t stream) {
   MLTS_REQUIRE(dres, "mlts_add_rmsnorm_bwd: null pointer");
-  return rmsnorm_bwd_checked("mlts_add_rmsnorm_bwd", dy, x, w, rstd, dres, dx, dw, workspace, workspace_bytes, rows,
+  return rmsnorm_bwd_checked("mlts_add_rmsnorm_bwd", dy, x, w, rstd, dres, dx, dw, 0, workspace, workspace_bytes, rows,
+                             hidden, dtype, stream);
+}
+
+extern "C" int mlts_rmsnorm_bwd_accumulate(const void* dy, const void* x, const void* w, const float* rstd, const void* dres,
+                                           void* dx, void* dw, void* workspace, int64_t workspace_bytes, int64_t rows,
+                                           int32_t hidden, int32_t dtype, mlts_stream_t stream) {
+  return rmsnorm_bwd_checked("mlts_rmsnorm_bwd_accumulate", dy, x, w, rstd, dres, dx, dw, 1, workspace, workspace_bytes, rows,
                              hidden, dtype, stream);
 }
 

@@ -93,6 +93,15 @@ bool own_product(int form, const Tensor& a, const Tensor& b);  // whether `produ
 // a, b as the form (MLTS_GEMM_*) says -> [M, N], written to `out` (or added onto it) if that is given
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out = Tensor(), bool accumulate = false);  // products.cpp
 
+void notify_grad_written(const Tensor& param);  // llama.cpp: the parameter's gradient buffer was written past autograd
+// the gradient buffer a weight already owns and a backward formula may add into, or undefined
+inline Tensor bound_grad(const Tensor& weight, bool into_grad) {
+  if (!into_grad) return Tensor();
+  const Tensor& g = weight.grad();
+  if (!g.defined() || !g.is_contiguous() || g.scalar_type() != weight.scalar_type() || g.sizes() != weight.sizes()) return Tensor();
+  return g;
+}
+
 void bind_ops(pybind11::module& m);    // ops.cpp
 void bind_llama(pybind11::module& m);  // llama.cpp
 

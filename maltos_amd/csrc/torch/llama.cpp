@@ -57,6 +57,8 @@ struct GradMarks {
   }
 };
 
+}  // namespace
+
 void notify_grad_written(const Tensor& param) {
   std::lock_guard<std::mutex> lock(marks_mutex);
   auto it = marks_by_param.find(param.unsafeGetTensorImpl());
@@ -64,6 +66,8 @@ void notify_grad_written(const Tensor& param) {
     for (auto& [marks, i] : it->second) marks->written[i] = 1;
   for (std::vector<Tensor>* seen : listeners) seen->push_back(param);
 }
+
+namespace {
 
 struct GradListener {
   std::vector<Tensor> seen;
@@ -143,14 +147,6 @@ Tensor project(const Tensor& x, const Tensor& weight) {
   return product(MLTS_GEMM_NT, rows2d(x), weight).view(shape);
 }
 
-// the gradient buffer that a product may be added into, or undefined
-Tensor bound_grad(const Tensor& weight, bool into_grad) {
-  if (!into_grad) return Tensor();
-  const Tensor& g = weight.grad();
-  if (!g.defined() || !g.is_contiguous() || g.scalar_type() != weight.scalar_type() || g.sizes() != weight.sizes()) return Tensor();
-  return g;
-}
-
 struct LinearBackward final : Formula {
   enum { X, W, COUNT };
   bool into_grad = false;
@@ -183,6 +179,45 @@ Tensor linear(const Tensor& x, const Tensor& weight, bool into_grad) {
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     y = project(x, weight);
+  }
+  if (fn) set_history(y, fn);
+  return y;
+}
+
+// ---- token embedding --------------------------------------------------------------------------------------------------------
+struct EmbeddingBackward final : Formula {
+  enum { IDS, W, COUNT };
+  bool into_grad = false;
+  EmbeddingBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosEmbeddingBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    if (!g[0].defined()) return {Tensor()};
+    const Tensor &w = s[W], ids = dense(s[IDS].scalar_type() == at::kLong ? s[IDS] : s[IDS].to(at::kLong)), dy = dense(g[0]);
+    const int64_t n = ids.numel(), vocab = w.size(0), hidden = w.size(1);
+    if ((w.scalar_type() != at::kBFloat16 && w.scalar_type() != at::kFloat) || dy.scalar_type() != w.scalar_type() ||
+        mlts_embedding_bwd_supports(n, hidden, vocab, dtype_code(w)) != nullptr)
+      return {at::embedding_dense_backward(dy, ids, vocab, -1, false)};
+    const Tensor grad = bound_grad(w, into_grad);
+    Tensor dw = grad.defined() ? grad : at::zeros({vocab, hidden}, w.options());
+    check(mlts_embedding_bwd(ids.const_data_ptr<int64_t>(), ptr(dy), mptr(dw), n, hidden, vocab, dtype_code(w), current_stream()));
+    if (!grad.defined()) return {dw};
+    notify_grad_written(w);
+    return {Tensor()};
+  }
+};
+
+Tensor embedding(const Tensor& weight, const Tensor& ids, bool into_grad) {
+  std::shared_ptr<EmbeddingBackward> fn;
+  if (compute_requires_grad(weight)) {
+    fn = make_formula<EmbeddingBackward>();
+    fn->set_next_edges(collect_next_edges(weight));
+    fn->save(fn->IDS, ids), fn->save(fn->W, weight);
+    fn->into_grad = into_grad;
+  }
+  Tensor y;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    y = at::embedding(weight, ids);
   }
   if (fn) set_history(y, fn);
   return y;
@@ -433,6 +468,7 @@ void bind_llama(pybind11::module& m) {
   using torch::wrap_pybind_function;
   namespace py = pybind11;
   m.def("linear", wrap_pybind_function(linear));
+  m.def("embedding", wrap_pybind_function(embedding));
   m.def("product", wrap_pybind_function([](int form, const Tensor& a, const Tensor& b, const OptTensor& out, bool accumulate) {
           at::AutoDispatchBelowADInplaceOrView below_autograd;
           return product(form, a, b, out.value_or(Tensor()), accumulate);

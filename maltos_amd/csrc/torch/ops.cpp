@@ -9,6 +9,8 @@
 #include <mutex>
 #include <vector>
 
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+
 #include "common.hpp"
 
 namespace maltos {
@@ -368,6 +370,19 @@ std::tuple<Tensor, Tensor> add_rmsnorm_bwd(const Tensor& dy_in, const Tensor& dr
   return {dx, dw};
 }
 
+// dx, with dw added onto the gradient buffer the weight already owns; dres may be undefined
+Tensor rmsnorm_bwd_into(const Tensor& dy_in, const Tensor& dres_in, const Tensor& x_in, const Tensor& w_in, const Tensor& rstd, Tensor grad) {
+  const Tensor x = dense(x_in), dy = dense(dy_in), w = dense(w_in), dres = dres_in.defined() ? dense(dres_in) : dres_in;
+  const int64_t rows = rows_of(x), hidden = x.size(-1);
+  Tensor dx = at::empty(x.sizes(), x.options());
+  if (rows == 0) return dx;
+  const int64_t ws_bytes = mlts_rmsnorm_bwd_workspace_bytes(rows, hidden);
+  Tensor ws = workspace(ws_bytes, x);
+  check(mlts_rmsnorm_bwd_accumulate(ptr(dy), ptr(x), ptr(w), rstd.const_data_ptr<float>(), dres.defined() ? ptr(dres) : nullptr, mptr(dx), mptr(grad),
+                                    mptr(ws), ws_bytes, rows, hidden, dtype_code(x), current_stream()));
+  return dx;
+}
+
 // ---- RoPE -----------------------------------------------------------------------------------------------------------
 void check_tables(const Tensor& x, const Tensor& cos, const Tensor& sin) {
   const int64_t half = x.size(3) / 2;
@@ -690,20 +705,34 @@ std::tuple<Tensor, Tensor> attn_fwd_autograd(const Tensor& q, const Tensor& k, c
   return {o, lse};
 }
 
+// into_grad: the weight's gradient is added into the buffer it already owns, as the products of the linear layers do it.  A
+// weight with tensor hooks is left to autograd, so that the hooks see its gradient.
+Tensor norm_grad_buffer(const Tensor& w, bool into_grad) {
+  return into_grad && torch::autograd::impl::hooks(w).empty() && !c10::impl::dispatch_mode_enabled() ? bound_grad(w, true) : Tensor();
+}
+
 struct RmsNormBackward final : Formula {
   enum { X, W, RSTD, COUNT };
+  bool into_grad = false;
   RmsNormBackward() : Formula(COUNT) {}
   std::string name() const override { return "MaltosRmsNormBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    const Tensor grad = task_should_compute_output(1) && g[0].defined() ? norm_grad_buffer(s[W], into_grad) : Tensor();
+    if (grad.defined()) {
+      Tensor dx = rmsnorm_bwd_into(g[0], Tensor(), s[X], s[W], s[RSTD], grad);
+      notify_grad_written(s[W]);
+      return {dx, Tensor()};
+    }
     auto [dx, dw] = op::rmsnorm_bwd().call(g[0].defined() ? g[0] : at::zeros_like(s[X]), s[X], s[W], s[RSTD]);
     return {dx, dw};
   }
 };
 
-std::tuple<Tensor, Tensor> rmsnorm_fwd_autograd(const Tensor& x, const Tensor& w, double eps) {
+std::tuple<Tensor, Tensor> rmsnorm_recorded(const Tensor& x, const Tensor& w, double eps, bool into_grad) {
   std::shared_ptr<RmsNormBackward> fn;
   if (compute_requires_grad(x, w)) {
     fn = make_formula<RmsNormBackward>();
+    fn->into_grad = into_grad;
     fn->set_next_edges(collect_next_edges(x, w));
     fn->save(fn->X, x), fn->save(fn->W, w);
   }
@@ -724,19 +753,26 @@ std::tuple<Tensor, Tensor> rmsnorm_fwd_autograd(const Tensor& x, const Tensor& w
 // addends receive the same gradient.
 struct AddRmsNormBackward final : Formula {
   enum { H, W, RSTD, COUNT };
+  bool into_grad = false;
   AddRmsNormBackward() : Formula(COUNT) {}
   std::string name() const override { return "MaltosAddRmsNormBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[1].defined()) return {g[0], g[0], Tensor()};
+    if (const Tensor grad = task_should_compute_output(2) ? norm_grad_buffer(s[W], into_grad) : Tensor(); grad.defined()) {
+      Tensor dx = rmsnorm_bwd_into(g[1], g[0], s[H], s[W], s[RSTD], grad);
+      notify_grad_written(s[W]);
+      return {dx, dx, Tensor()};
+    }
     auto [dx, dw] = g[0].defined() ? op::add_rmsnorm_bwd().call(g[1], g[0], s[H], s[W], s[RSTD]) : op::rmsnorm_bwd().call(g[1], s[H], s[W], s[RSTD]);
     return {dx, dx, dw};
   }
 };
 
-std::tuple<Tensor, Tensor, Tensor> add_rmsnorm_fwd_autograd(const Tensor& x, const Tensor& res, const Tensor& w, double eps) {
+std::tuple<Tensor, Tensor, Tensor> add_rmsnorm_recorded(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad) {
   std::shared_ptr<AddRmsNormBackward> fn;
   if (compute_requires_grad(x, res, w)) {
     fn = make_formula<AddRmsNormBackward>();
+    fn->into_grad = into_grad;
     fn->set_next_edges(collect_next_edges(x, res, w));
     fn->save(fn->W, w);
   }
@@ -752,6 +788,11 @@ std::tuple<Tensor, Tensor, Tensor> add_rmsnorm_fwd_autograd(const Tensor& x, con
     fn->save(fn->H, h, true), fn->save(fn->RSTD, rstd, true);
   }
   return {h, y, rstd};
+}
+
+std::tuple<Tensor, Tensor> rmsnorm_fwd_autograd(const Tensor& x, const Tensor& w, double eps) { return rmsnorm_recorded(x, w, eps, false); }
+std::tuple<Tensor, Tensor, Tensor> add_rmsnorm_fwd_autograd(const Tensor& x, const Tensor& res, const Tensor& w, double eps) {
+  return add_rmsnorm_recorded(x, res, w, eps, false);
 }
 
 struct RopeBackward final : Formula {
@@ -955,9 +996,11 @@ std::tuple<Tensor, Tensor, Tensor> py_attention_backward(const Tensor& dout, con
   at::AutoDispatchBelowADInplaceOrView below_autograd;
   return attention_backward(dout, q, k, v, o, lse, mask_mode, resolve_scale(scale, q), q_pos, k_pos, q_seq, k_seq);
 }
-Tensor py_rms_norm(const Tensor& x, const Tensor& w, double eps) { return std::get<0>(op::rmsnorm_fwd().call(x, w, eps)); }
-std::tuple<Tensor, Tensor> py_add_rms_norm(const Tensor& x, const Tensor& res, const Tensor& w, double eps) {
-  auto [h, y, rstd] = op::add_rmsnorm_fwd().call(x, res, w, eps);
+Tensor py_rms_norm(const Tensor& x, const Tensor& w, double eps, bool into_grad) {
+  return std::get<0>(into_grad && at::GradMode::is_enabled() ? rmsnorm_recorded(x, w, eps, true) : op::rmsnorm_fwd().call(x, w, eps));
+}
+std::tuple<Tensor, Tensor> py_add_rms_norm(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad) {
+  auto [h, y, rstd] = into_grad && at::GradMode::is_enabled() ? add_rmsnorm_recorded(x, res, w, eps, true) : op::add_rmsnorm_fwd().call(x, res, w, eps);
   return {h, y};
 }
 Tensor py_rope(const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& positions, int64_t offset) {
@@ -1000,8 +1043,9 @@ void bind_ops(pybind11::module& m) {
   m.def("attention_backward_accumulate", wrap_pybind_function(attention_backward_accumulate));
   m.def("attention_backward_ring_block", wrap_pybind_function(attention_backward_ring_block));
   m.def("attention_merge_", wrap_pybind_function(attention_merge_));
-  m.def("rms_norm", wrap_pybind_function(py_rms_norm));
-  m.def("add_rms_norm", wrap_pybind_function(py_add_rms_norm));
+  namespace py = pybind11;
+  m.def("rms_norm", wrap_pybind_function(py_rms_norm), py::arg("x"), py::arg("w"), py::arg("eps"), py::arg("into_grad") = false);
+  m.def("add_rms_norm", wrap_pybind_function(py_add_rms_norm), py::arg("x"), py::arg("res"), py::arg("w"), py::arg("eps"), py::arg("into_grad") = false);
   m.def("rope", wrap_pybind_function(py_rope));
   m.def("rope_pair", wrap_pybind_function(py_rope_pair));
   m.def("rope_pair_", wrap_pybind_function(rope_pair_));

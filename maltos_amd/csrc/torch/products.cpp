@@ -15,6 +15,13 @@ namespace {
 // per-shape selection, are ahead: a training step of that size took 90 us more of 9500 with its 512-wide products done here.
 constexpr double kOwnLimit = 4.0e9;
 
+// Above it they still run for dx = dy W with so long a contraction that it is split over workgroups (dx of an lm_head): the
+// library does not split those (us, 512 wide, 32000 terms: 1024 rows 47 against 160, 8192 rows 270 against 346).
+bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K) {
+  return static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K) <= kOwnLimit ||
+         (form == MLTS_GEMM_NN && mlts_gemm_workspace_bytes(form, dtype, M, N, K) > 0);
+}
+
 struct Sizes {
   int64_t M, N, K;
   Sizes(int form, const Tensor& a, const Tensor& b)
@@ -35,8 +42,8 @@ Tensor library_product(int form, const Tensor& a, const Tensor& b, const Tensor&
 
 bool own_product(int form, const Tensor& a, const Tensor& b) {
   const Sizes z(form, a, b);
-  return static_cast<double>(z.M) * static_cast<double>(z.N) * static_cast<double>(z.K) <= kOwnLimit && z.M > 0 && z.N > 0 && z.K > 0 && plain(a) &&
-         plain(b) && a.scalar_type() == b.scalar_type() && (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) &&
+  return z.M > 0 && z.N > 0 && z.K > 0 && plain(a) && plain(b) && a.scalar_type() == b.scalar_type() &&
+         (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) && within_own_range(form, dtype_code(a), z.M, z.N, z.K) &&
          mlts_gemm_supports(form, dtype_code(a), z.M, z.N, z.K, a.stride(0), b.stride(0), z.N) == nullptr && aligned(a) && aligned(b) &&
          !c10::impl::dispatch_mode_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA);
 }

@@ -3,8 +3,8 @@
 Counterpart of the reference's models/llama.py:30-330 with identical module and parameter names
 (embed_tokens, layers.N.self_attn.{q,k,v,o}_proj, layers.N.mlp.{gate,up,down}_proj,
 layers.N.{input,post_attention}_layernorm, norm, lm_head), so state dicts are interchangeable.
-RMSNorm, RoPE, attention, SwiGLU and the loss are the `maltos::` custom ops; the projections and the
-embedding stay on the vendor GEMM library through torch.  Attention consumes the [B, H, S, D] views
+RMSNorm, RoPE, attention, SwiGLU and the loss are the `maltos::` custom ops; the projections run on the own
+product kernels up to a size and on the vendor library through torch above it (csrc/torch/products.cpp).  Attention consumes the [B, H, S, D] views
 of the projection outputs in place and keeps K/V at their native head count.
 """
 from __future__ import annotations
@@ -101,24 +101,61 @@ class HipLinear(nn.Linear):
         return native().linear(x, self.weight, bool(self.accumulate_into_grad))
 
 
+class LlamaEmbedding(nn.Embedding):
+    """embed_tokens (reference: nn.Embedding, models/llama.py:238).  `accumulate_into_grad` as in HipLinear, except that a
+    weight with tensor hooks, or tied to the lm_head, keeps its gradient with autograd."""
+
+    accumulate_into_grad = False
+
+    def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
+        plain = self.padding_idx is None and self.max_norm is None and not self.scale_grad_by_freq and not self.sparse
+        if not plain or not self.weight.is_cuda:
+            return super().forward(input_ids)
+        return native().embedding(self.weight, input_ids, self.accumulate_into_grad and not self.weight._backward_hooks)
+
+
+class LlamaHead(nn.Linear):
+    """The lm_head (reference: nn.Linear, models/llama.py:242-243).  `accumulate_into_grad` as in LlamaEmbedding."""
+
+    accumulate_into_grad = False
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if self.bias is not None or not x.is_cuda or torch.is_autocast_enabled("cuda"):
+            return F.linear(x, self.weight, self.bias)
+        return native().linear(x, self.weight, self.accumulate_into_grad and not self.weight._backward_hooks)
+
+
 def set_grad_accumulation_into_buffers(model: nn.Module, enabled: bool = True) -> int:
-    """Switches `HipLinear.accumulate_into_grad` on every HipLinear of `model`; returns how many were switched."""
+    """Switches `HipLinear.accumulate_into_grad` on every HipLinear of `model`, and returns how many were switched.  The
+    norms and, when untied, the embedding and the lm_head follow (weights with tensor hooks excepted)."""
     count = 0
     for module in model.modules():
         if isinstance(module, HipLinear):
             module.accumulate_into_grad = bool(enabled)
             count += 1
+        elif isinstance(module, LlamaRMSNorm):
+            module.accumulate_into_grad = bool(enabled)
+        elif isinstance(module, LlamaForCausalLM):
+            untied = module.lm_head.weight is not module.embed_tokens.weight
+            module.lm_head.accumulate_into_grad = module.embed_tokens.accumulate_into_grad = bool(enabled) and untied
     return count
 
 
 class LlamaRMSNorm(nn.Module):
+    accumulate_into_grad = False   # see HipLinear; a weight with tensor hooks keeps its gradient with autograd
+
     def __init__(self, hidden_size: int, eps: float) -> None:
         super().__init__()
         self.weight = nn.Parameter(torch.ones(hidden_size))
         self.eps = eps
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.rms_norm(x, self.weight, self.eps)
+        return native().rms_norm(x, self.weight, self.eps, self.accumulate_into_grad)
+
+
+def _add_norm(norm: nn.Module, x: torch.Tensor, residual: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(h, norm of h) with h = x + residual."""
+    return native().add_rms_norm(x, residual, norm.weight, norm.eps, getattr(norm, "accumulate_into_grad", False))
 
 
 class LlamaRotaryEmbedding(nn.Module):
@@ -266,9 +303,9 @@ class LlamaDecoderLayer(nn.Module):
         if pending is None:
             normed = ln1(x)
         else:
-            x, normed = ops.add_rms_norm(x, pending, ln1.weight, ln1.eps)
+            x, normed = _add_norm(ln1, x, pending)
         attn_out = self.self_attn(normed, position_offset=position_offset, position_ids=position_ids, sequence_ids=sequence_ids)
-        x, normed = ops.add_rms_norm(x, attn_out, ln2.weight, ln2.eps)
+        x, normed = _add_norm(ln2, x, attn_out)
         return x, self.mlp(normed)
 
 
@@ -276,10 +313,10 @@ class LlamaForCausalLM(nn.Module):
     def __init__(self, config: LlamaConfig) -> None:
         super().__init__()
         self.config = config
-        self.embed_tokens = nn.Embedding(config.vocab_size, config.hidden_size)
+        self.embed_tokens = LlamaEmbedding(config.vocab_size, config.hidden_size)
         self.layers = nn.ModuleList([LlamaDecoderLayer(config) for _ in range(config.num_hidden_layers)])
         self.norm = LlamaRMSNorm(config.hidden_size, config.rms_norm_eps)
-        self.lm_head = nn.Linear(config.hidden_size, config.vocab_size, bias=False)
+        self.lm_head = LlamaHead(config.hidden_size, config.vocab_size, bias=False)
         if config.tie_word_embeddings:
             self.lm_head.weight = self.embed_tokens.weight
 
@@ -319,7 +356,7 @@ class LlamaForCausalLM(nn.Module):
             for layer in self.layers:
                 x, pending = layer(x, position_offset=position_offset, position_ids=position_ids, sequence_ids=sequence_ids,
                                    pending=pending, defer_residual=True)
-            _, normed = ops.add_rms_norm(x, pending, self.norm.weight, self.norm.eps)
+            _, normed = _add_norm(self.norm, x, pending)
         else:
             for layer in self.layers:
                 x = layer(x, position_offset=position_offset, position_ids=position_ids, sequence_ids=sequence_ids)

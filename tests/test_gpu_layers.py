@@ -531,3 +531,49 @@ def test_more_than_two_to_the_31_elements(dev):
     assert all(torch.equal(x[:4096], y) for x, y in zip((p, m, v), first))
     assert all(torch.equal(x[mid[0]:mid[1]], y) for x, y in zip((p, m, v), mid[2:]))
     assert all(torch.equal(x[last[0]:], y) for x, y in zip((p, m, v), last[1:]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,hidden,vocab,common", [(1, 8, 5, 0), (63, 520, 300, 0), (1025, 512, 32000, 0), (3000, 256, 1000, 1500), (16384, 512, 32000, 200),
+                                                   (28672, 64, 257, 20000), (28673, 64, 257, 0)])
+def test_embedding_gradient(dev, dtype, n, hidden, vocab, common):
+    """Rows of equal ids summed in fp32: few and many tokens, ids of thousands of tokens, and more tokens than one list holds."""
+    from maltos_amd._native import native
+    gen = torch.Generator().manual_seed(n)
+    ids = torch.randint(0, vocab, (n,), generator=gen)
+    ids[torch.randperm(n, generator=gen)[:common]] = vocab - 1
+    dy = torch.randn(n, hidden, generator=gen).to(dtype)
+    want = torch.zeros(vocab, hidden, dtype=torch.float64).index_add_(0, ids, dy.double())
+    w = torch.zeros(vocab, hidden, dtype=dtype, device=dev, requires_grad=True)
+    rel = 3e-3 if dtype == torch.bfloat16 else 1e-6
+    native().embedding(w, ids.to(dev), False).backward(dy.to(dev))
+    assert (w.grad.cpu().double() - want).norm() <= rel * want.norm()
+    first = w.grad.clone()
+    for _ in range(2):   # added onto the gradient buffer that is there, the same every time
+        w.grad.copy_(first)
+        native().embedding(w, ids.to(dev), True).backward(dy.to(dev))
+        assert (w.grad.cpu().double() - 2 * want).norm() <= 2 * rel * want.norm()
+        second = w.grad.clone() if _ == 0 else second
+    assert torch.equal(w.grad, second)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_norm_embedding_and_head_gradients_into_buffers(dev, dtype):
+    """With gradient buffers bound, their gradients are autograd's; a weight with a tensor hook stays with autograd."""
+    from maltos_amd.llama import LlamaConfig, LlamaForCausalLM, set_grad_accumulation_into_buffers
+    config = LlamaConfig(vocab_size=200, hidden_size=64, intermediate_size=96, num_hidden_layers=2, num_attention_heads=2)
+    torch.manual_seed(3)
+    plain = LlamaForCausalLM(config).to(dev, dtype)
+    into = LlamaForCausalLM(config).to(dev, dtype)
+    into.load_state_dict(plain.state_dict())
+    set_grad_accumulation_into_buffers(into)
+    for p in into.parameters():
+        p.grad = torch.zeros_like(p)
+    seen = []
+    into.layers[0].input_layernorm.weight.register_hook(lambda g: seen.append(g))
+    ids = torch.randint(0, 200, (2, 40), device=dev)
+    for m in (plain, into):
+        m({"input_ids": ids, "labels": ids}).backward()
+    assert len(seen) == 1 and seen[0] is not None
+    for (name, a), b in zip(plain.named_parameters(), into.parameters()):
+        assert torch.equal(a.grad, b.grad), name
