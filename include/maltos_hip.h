@@ -282,6 +282,21 @@ const char* mlts_gemm_supports(int32_t form, int32_t dtype, int64_t M, int64_t N
 int64_t mlts_gemm_workspace_bytes(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K);
 int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb,
               void* c, int64_t ldc, int32_t accumulate, void* workspace, int64_t workspace_bytes, mlts_stream_t stream);
+/* Up to four products in one call, small ones in one launch.  A product of the NN form may be the sum over up to three
+ * segments a[i] b[i] (the input gradient of layers that share their input), in bf16 with the roundings of separate products. */
+typedef struct {
+  int32_t form, segments, accumulate;
+  int64_t M, N;
+  int64_t k[3];
+  const void *a[3], *b[3];
+  int64_t lda[3], ldb[3];
+  void* c;
+  int64_t ldc;
+} mlts_gemm_product;
+int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* products, int32_t count, int32_t dtype);
+int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
+                    mlts_stream_t stream);
+
 
 /* The norm, scaling and AdamW passes over a list of fp32 tensors (host arrays of device pointers and element counts) in one
  * launch per 48 tensors, for parameters that do not share a flat buffer: what the reference's optimizer does per parameter

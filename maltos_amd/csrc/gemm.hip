@@ -16,6 +16,8 @@
 // that a lane holds four neighbouring columns of one row of C, and leaves through LDS in whole row segments.
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int FORM_NT = MLTS_GEMM_NT, FORM_NN = MLTS_GEMM_NN, FORM_TN = MLTS_GEMM_TN;
@@ -110,49 +112,90 @@ struct Slab {
   }
 };
 
-struct GemmArgs {
+// One product of a launch, as small as can be: kernel arguments are read from host memory.  (Operands are smaller than 2 GiB, so
+// their strides and lengths fit 32 bits.)
+struct Product {
   const void *a, *b;
   void* c;
-  float* partial;   // split contraction: [slices][M][N] fp32 in place of c
-  int64_t lda, ldb, ldc;
+  float* partial;  // split contraction: [slices][M][N] fp32 in place of c
+  int lda, ldb, ldc, K;
+  int k_slice;     // contraction elements per slice (a multiple of the slab)
   int M, N;
-  int64_t K, k_slice;  // contraction elements per slice (a multiple of the slab)
   int tiles_m, tiles_n, slices;
-  int accumulate;
+  int form, accumulate;
+};
+// The contraction of the NN form may be a concatenation (dx = sum dy_i W_i of layers that share their input): what follows the
+// first part.  In bf16 each part is rounded, and added to the parts before it in bf16: the values of separate products whose
+// results are added, bit for bit.
+constexpr int kMaxSegments = 3, kMaxProducts = 4;
+struct MoreSegments {
+  const void *a[kMaxSegments - 1], *b[kMaxSegments - 1];
+  int lda[kMaxSegments - 1], ldb[kMaxSegments - 1], K[kMaxSegments - 1];
+  int count, product;  // how many, of which product
 };
 
-template <typename T, int FORM, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_kernel(const GemmArgs g) {
-  constexpr int WAVES_N = BN / WN, WAVES = (BM / WM) * WAVES_N, THREADS = WAVES * 64;
-  constexpr int MB = WM / 32, NB = WN / 32;
-  constexpr int SETS = MB * NB >= 8 ? 1 : 2;  // (eight accumulator blocks leave no registers for a second set)
+// Consecutive workgroups go to the eight XCDs in turn; each XCD gets a contiguous run of a product's tiles, walked along N, so
+// that the workgroups that share rows of A share an L2.
+__device__ __forceinline__ int tile_of(int block, int tiles) {
+  const int per = tiles >> 3, rest = tiles & 7, xcd = block & 7, pos = block >> 3;
+  return pos < per + (xcd < rest) ? xcd * per + min(xcd, rest) + pos : -1;
+}
+
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG>
+struct TileShape {
+  static constexpr int WAVES_N = BN / WN, WAVES = (BM / WM) * WAVES_N * KG, THREADS = WAVES * 64;
+  static constexpr int MB = WM / 32, NB = WN / 32;
+  static constexpr int SETS = MB * NB >= 8 ? 1 : 2;  // (eight accumulator blocks leave no registers for a second set)
   typedef Slab<T, BM, FORM != FORM_TN, THREADS, SETS> SA;
   typedef Slab<T, BN, FORM == FORM_NT, THREADS, SETS> SB;
-  constexpr int STAGE = SA::BYTES + SB::BYTES;
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  static constexpr int STAGE = SA::BYTES + SB::BYTES;
+  static constexpr int OUT = WAVES * 32 * (WN + 4) * 4 + (KG > 1 ? (WAVES - WAVES / KG) * MB * NB * 4096 : 0);
+  static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
+};
+
+// One tile of one product.  KG > 1: the wavefronts form KG groups that share the tile and each multiply their part of every
+// slab; the groups' sums are joined through LDS in a fixed order.
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS>
+__device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs) {
+  typedef TileShape<T, FORM, BM, BN, WM, WN, KG> S;
+  constexpr int WAVES_N = S::WAVES_N, MB = S::MB, NB = S::NB, SETS = S::SETS, STAGE = S::STAGE;
+  typedef typename S::SA SA;
+  typedef typename S::SB SB;
+  constexpr int BK = Elem<T>::BK, STEPS = 4 / KG;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = (wave / WAVES_N) * WM, wn = (wave % WAVES_N) * WN;
-
-  // Consecutive workgroups go to the eight XCDs in turn; each XCD gets a contiguous run of tiles, walked along N, so that the
-  // workgroups that share rows of A share an L2.
-  const int tiles = g.tiles_m * g.tiles_n * g.slices;
-  int tile = static_cast<int>(blockIdx.x);
-  {
-    const int per = tiles >> 3, rest = tiles & 7, xcd = tile & 7, pos = tile >> 3;
-    tile = xcd * per + min(xcd, rest) + pos;
-  }
+  const int group = KG > 1 ? wave / (S::WAVES / KG) : 0, member = KG > 1 ? wave % (S::WAVES / KG) : wave;
+  const int wm = (member / WAVES_N) * WM, wn = (member % WAVES_N) * WN;
   const int slice = tile / (g.tiles_m * g.tiles_n);
   tile -= slice * (g.tiles_m * g.tiles_n);
   const int m0 = (tile / g.tiles_n) * BM, n0 = (tile % g.tiles_n) * BN;
-  const int64_t k_begin = slice * g.k_slice, k_end = min(g.K, k_begin + g.k_slice);
 
   SA sa;
   SB sb;
-  if (FORM == FORM_TN) sa.init(static_cast<const T*>(g.a) + m0, g.lda, g.K, g.M - m0, k_begin);
-  else sa.init(static_cast<const T*>(g.a) + static_cast<int64_t>(m0) * g.lda, g.lda, g.M - m0, g.K, k_begin);
-  if (FORM == FORM_NT) sb.init(static_cast<const T*>(g.b) + static_cast<int64_t>(n0) * g.ldb, g.ldb, g.N - n0, g.K, k_begin);
-  else sb.init(static_cast<const T*>(g.b) + n0, g.ldb, g.K, g.N - n0, k_begin);
+  int k_left = 0;                  // contraction elements of the segment behind the slab that is fetched next
+  int seg = 0, seg_slabs = 0;      // segments opened after the first, slabs of the open one that are not fetched yet
+  auto open = [&](const void* a, int64_t lda, const void* b, int64_t ldb, int64_t K, int64_t k_begin, int64_t k_end) {
+    if (FORM == FORM_TN) sa.init(static_cast<const T*>(a) + m0, lda, K, g.M - m0, k_begin);
+    else sa.init(static_cast<const T*>(a) + m0 * lda, lda, g.M - m0, K, k_begin);
+    if (FORM == FORM_NT) sb.init(static_cast<const T*>(b) + n0 * ldb, ldb, g.N - n0, K, k_begin);
+    else sb.init(static_cast<const T*>(b) + n0, ldb, K, g.N - n0, k_begin);
+    k_left = static_cast<int>(k_end - k_begin);
+    seg_slabs = (k_left + BK - 1) / BK;
+  };
+  const int k_begin = slice * g.k_slice;
+  open(g.a, g.lda, g.b, g.ldb, g.K, k_begin, min(g.K, k_begin + g.k_slice));
+  int slabs = seg_slabs;
+  if constexpr (SEGMENTS)
+    for (int i = 0; i < segs; ++i) slabs += (more.K[i] + BK - 1) / BK;
+  auto next_slab = [&] {  // before the first chunk of a slab is fetched
+    if constexpr (SEGMENTS) {
+      while (seg_slabs == 0 && seg < segs) {
+        open(more.a[seg], more.lda[seg], more.b[seg], more.ldb[seg], more.K[seg], 0, more.K[seg]);
+        ++seg;
+      }
+      --seg_slabs;
+    }
+  };
 
   f32x16 acc[MB][NB];
 #pragma unroll
@@ -163,70 +206,137 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_kernel(const 
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
   // One slab ahead in LDS, the next SETS in registers: chunk c of slab s + 1 goes to the other stage and its registers fetch
-  // chunk c of slab s + 1 + SETS, a quarter of the chunks behind the products of each fragment step.  (Past the end: zeros, never
-  // multiplied.)  With one set a load has the time of one slab to arrive, which short contractions out of HBM exceed.
+  // chunk c of slab s + 1 + SETS, spread behind the products of the fragment steps.  (Past the end: zeros, never multiplied.)
+  // With one set a load has the time of one slab to arrive, which short contractions out of HBM exceed; more than two sets
+  // bring nothing (1024 x 512 x 512: 5.2 us with 2, 4, 5.5 with 6).
   constexpr int CHUNKS = SA::PER + SB::PER;
   auto store = [&](int set, int c, unsigned char* stage) {
     if (c < SA::PER) sa.store(set, c, stage);
     else sb.store(set, c - SA::PER, stage + SA::BYTES);
   };
-  auto fetch = [&](int set, int c, int k_left) {
+  auto fetch = [&](int set, int c) {
     if (c < SA::PER) sa.fetch(set, c, k_left);
     else sb.fetch(set, c - SA::PER, k_left);
   };
-  const int slabs = static_cast<int>((k_end - k_begin + Elem<T>::BK - 1) / Elem<T>::BK);
-  int k_left = static_cast<int>(k_end - k_begin);
 #pragma unroll
   for (int f = 0; f < SETS; ++f) {
+    next_slab();
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) fetch(f, c, k_left);
-    k_left -= Elem<T>::BK;
+    for (int c = 0; c < CHUNKS; ++c) fetch(f, c);
+    k_left -= BK;
   }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) store(0, c, lds);
+  next_slab();
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) fetch(0, c, k_left);
+  for (int c = 0; c < CHUNKS; ++c) fetch(0, c);
+  constexpr bool FOLD = SEGMENTS && sizeof(T) == 2;
+  f32x16 parts[FOLD ? MB : 1][FOLD ? NB : 1];  // sum of the parts before
+  int part = 0, part_end = FOLD ? (g.K + BK - 1) / BK : 0;
+  auto fold = [&] {
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float v = to_f32<T>(from_f32<T>(acc[i][j][e]));
+            parts[i][j][e] = part == 0 ? v : to_f32<T>(from_f32<T>(parts[i][j][e] + v));
+            acc[i][j][e] = 0.f;
+          }
+    }
+  };
   auto slab = [&](int s, int set) {  // set: registers of slab s + 1
-    k_left -= Elem<T>::BK;
+    k_left -= BK;
+    next_slab();
     __syncthreads();  // stage s & 1 is written everywhere, and nobody reads the other one any more
     const unsigned char* la = lds + (s & 1) * STAGE;
     const unsigned char* lb = la + SA::BYTES;
     unsigned char* next = lds + (~s & 1) * STAGE;
-    typename Elem<T>::frag fa[2][MB], fb[2][NB];
+    typename Elem<T>::frag fa[2][MB], fb[2][NB];  // (reading the whole slab's first instead changes nothing)
     auto read = [&](int ks) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) fb[ks & 1][j] = SB::fragment(lb, wn + 32 * j, ks, lane);
+      for (int j = 0; j < NB; ++j) fb[ks & 1][j] = SB::fragment(lb, wn + 32 * j, group * STEPS + ks, lane);
 #pragma unroll
-      for (int i = 0; i < MB; ++i) fa[ks & 1][i] = SA::fragment(la, wm + 32 * i, ks, lane);
+      for (int i = 0; i < MB; ++i) fa[ks & 1][i] = SA::fragment(la, wm + 32 * i, group * STEPS + ks, lane);
     };
     read(0);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks < 3) read(ks + 1);
+    for (int ks = 0; ks < STEPS; ++ks) {
+      if (ks + 1 < STEPS) read(ks + 1);
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) acc[i][j] = Elem<T>::mma(fb[ks & 1][j], fa[ks & 1][i], acc[i][j]);
 #pragma unroll
-      for (int c = ks * CHUNKS / 4; c < (ks + 1) * CHUNKS / 4; ++c) {
+      for (int c = ks * CHUNKS / STEPS; c < (ks + 1) * CHUNKS / STEPS; ++c) {
         store(set, c, next);
-        fetch(set, c, k_left);
+        fetch(set, c);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  auto after = [&](int s) {  // slab s was multiplied: the last of its part?
+    if constexpr (FOLD)
+      while (part < segs && s + 1 == part_end) {
+        fold();
+        part_end += (more.K[part++] + BK - 1) / BK;
+      }
+  };
+  if constexpr (FOLD) after(-1);
   if constexpr (SETS == 1) {
     for (int s = 0; s < slabs; ++s) slab(s, 0);
   } else {
     for (int s = 0; s < slabs; s += 2) {
       slab(s, 1);
-      if (s + 1 < slabs) slab(s + 1, 0);
+      after(s);
+      if (s + 1 < slabs) {
+        slab(s + 1, 0);
+        after(s + 1);
+      }
+    }
+  }
+  if constexpr (FOLD) {
+    if (segs > 0) {
+      fold();
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = parts[i][j];
     }
   }
 
   // acc[i][j][4 q + r]: row wm + 32 i + l % 32 of C, column wn + 32 j + 8 q + 4 hh + r.  Out through LDS, 32 rows at a time.
   __syncthreads();
   constexpr int ROW = WN + 4;  // floats
+  if constexpr (KG > 1) {
+    f32x4* sums = reinterpret_cast<f32x4*>(lds + S::WAVES * 32 * ROW * 4);  // [group - 1][member][block][quad][lane]
+    if (group > 0) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            sums[(((wave - S::WAVES / KG) * MB * NB + i * NB + j) * 4 + q) * 64 + lane] =
+                f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int o = 0; o < KG - 1; ++o)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 v = sums[(((o * (S::WAVES / KG) + member) * MB * NB + i * NB + j) * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] += v[r];
+          }
+  }
   float* stage = reinterpret_cast<float*>(lds) + wave * 32 * ROW;
   constexpr int LPR = WN / 4;         // lanes per row, four columns each
   constexpr int RPP = 64 / LPR;       // rows per pass
@@ -274,166 +384,355 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_kernel(const 
   }
 }
 
-// C (+)= sum of the slices' fp32 partial products, one rounding
-template <typename T, bool ACC>
-__global__ __launch_bounds__(256) void gemm_join_kernel(T* __restrict__ c, const float* __restrict__ partial, int slices, int64_t n4) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_kernel(const Product g) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n * g.slices);
+  if (tile >= 0) gemm_tile<T, FORM, BM, BN, WM, WN, KG, false>(g, tile, lds, MoreSegments{}, 0);
+}
+
+// Several small products in one launch: what a linear layer's backward needs (dx and dW), or projections that share their input.
+// Each alone leaves most of the chip idle and pays a launch: 1024 x 512 x 512 dx and dW are 128 and 64 tiles for 256 CUs.
+enum { FORMS_NT, FORMS_NN, FORMS_ANY, FORMS_SEGMENTS };  // the products' forms, as far as they change the code
+struct Products {
+  int first[kMaxProducts];  // the first workgroup of each; past the last one INT_MAX
+  Product p[kMaxProducts];
+  MoreSegments more;
+};
+template <typename T, int FORMS, int BM, int BN, int KG>
+__global__ __launch_bounds__(256) void gemm_multi_kernel(const Products ps) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int block = static_cast<int>(blockIdx.x);
+  int i = 0, first = ps.first[0];
+#pragma unroll
+  for (int k = 1; k < kMaxProducts; ++k)
+    if (block >= ps.first[k]) i = k, first = ps.first[k];
+  const Product& g = ps.p[i];
+  const int tile = tile_of(block - first, g.tiles_m * g.tiles_n * g.slices);
+  if (tile < 0) return;
+  if (FORMS == FORMS_NT || (FORMS != FORMS_NN && g.form == FORM_NT)) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
+  else if (FORMS == FORMS_NN || g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, 32, 32, KG, FORMS == FORMS_SEGMENTS>(g, tile, lds, ps.more, i == ps.more.product ? ps.more.count : 0);
+  else gemm_tile<T, FORM_TN, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
+}
+
+// C (+)= sum of the slices' fp32 partial products, one rounding; up to kMaxProducts outputs
+struct Joins {
+  struct Output {
+    void* c;
+    const float* partial;
+    int slices, accumulate, first_block;
+    int64_t n4;  // groups of four elements
+  } p[kMaxProducts];
+  int count;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void gemm_join_kernel(const Joins js) {
+  int o = 0;
+  while (o + 1 < js.count && static_cast<int>(blockIdx.x) >= js.p[o + 1].first_block) ++o;
+  const auto& g = js.p[o];
+  const int64_t i = static_cast<int64_t>(static_cast<int>(blockIdx.x) - g.first_block) * 256 + threadIdx.x, n4 = g.n4;
   if (i >= n4) return;
   typedef T t4 __attribute__((ext_vector_type(4)));
-  const f32x4* p = reinterpret_cast<const f32x4*>(partial) + i;
+  const f32x4* p = reinterpret_cast<const f32x4*>(g.partial) + i;
+  t4* c = reinterpret_cast<t4*>(g.c) + i;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
   int k = 0;
-  for (; k + 4 <= slices; k += 4) {
+  for (; k + 4 <= g.slices; k += 4) {
     f32x4 v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) v[u] = p[static_cast<int64_t>(k + u) * n4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) s += v[u];
   }
-  for (; k < slices; ++k) s += p[static_cast<int64_t>(k) * n4];
-  t4 o;
-  if (ACC) o = reinterpret_cast<const t4*>(c)[i];
+  for (; k < g.slices; ++k) s += p[static_cast<int64_t>(k) * n4];
+  t4 out;
+  if (g.accumulate) {
+    const t4 old = *c;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(ACC ? s[e] + to_f32<T>(o[e]) : s[e]);
-  reinterpret_cast<t4*>(c)[i] = o;
+    for (int e = 0; e < 4; ++e) s[e] += to_f32<T>(old[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out[e] = from_f32<T>(s[e]);
+  *c = out;
 }
 
-struct Plan {
-  int tile;    // 0: 64 x 64, 1: 128 x 128, 2: 256 x 128, 3: 256 x 256
-  int slices;
-  int64_t k_slice;
-};
+// ---- which tile, which split ----------------------------------------------------------------------------------------------
+constexpr int kSmall = 0;  // a tile of the multi kernel; 1: 128 x 128, 2: 256 x 128, 3: 256 x 256
 constexpr int kTileM[4] = {64, 128, 256, 256}, kTileN[4] = {64, 128, 128, 256};
-
-// The largest tile that still gives every CU a workgroup; a product with fewer tiles than CUs is split along its contraction
-// where that is long.  Best of all tiles and splits (us): NT 16384 x 512 x 512 256x128 15.6 (128x128 16.7, 64x64 19.2, 256x256
-// 21.6); NT 16384 x 2752 x 512 256x256 66 (76, 96, 77); NN 1023 x 512 x 32000 256x128 in 16 parts 45 (unsplit 210); TN 512 x
-// 512 x 16384 in 32 parts 24 (128x128 in 16: 23); TN 2752 x 512 x 16384 in 4 parts 70 (256x256 in 8: 68); TN 512 x 512 x 1023
-// 64x64 unsplit 10.1 (in 4: 12.7).
-Plan make_plan(int64_t M, int64_t N, int64_t K, int bk, bool dense) {
-  auto tiles = [&](int t) { return ((M + kTileM[t] - 1) / kTileM[t]) * ((N + kTileN[t] - 1) / kTileN[t]); };
-  const int64_t slabs = (K + bk - 1) / bk;
-  Plan p{0, 1, 0};
-  auto split = [&](int64_t least_slabs) {
-    while (tiles(p.tile) * p.slices * 2 <= 256 && slabs / (p.slices * 2) >= least_slabs) p.slices *= 2;
-  };
-  if (tiles(3) >= 240) {
-    p.tile = 3;
-  } else if (tiles(2) >= 256) {
-    p.tile = 2;
-  } else if (slabs >= 64 && tiles(2) * (slabs / 8) >= 192) {
-    p.tile = 2;
-    split(8);
-  } else if (tiles(1) >= 256) {
-    p.tile = 1;
-  } else {
-    split(bk == 64 ? 16 : 8);
-  }
-  if (N % 4 || !dense) p.slices = 1;
-  p.k_slice = (slabs + p.slices - 1) / p.slices * bk;
-  p.slices = p.k_slice > 0 ? static_cast<int>((K + p.k_slice - 1) / p.k_slice) : 1;
-  if (p.slices < 1) p.slices = 1;
-  return p;
+int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+int slab_of(int dtype) { return dtype == MLTS_BF16 ? 64 : 32; }
+int64_t slabs_of(const mlts_gemm_product& p, int bk) {
+  int64_t n = 0;
+  for (int i = 0; i < p.segments; ++i) n += (p.k[i] + bk - 1) / bk;
+  return n;
 }
 
-template <typename T, int FORM, int BM, int BN, int WM, int WN>
-int launch_tile(const GemmArgs& g, hipStream_t st) {
-  constexpr int WAVES = (BM / WM) * (BN / WN), THREADS = WAVES * 64;
-  constexpr int stages = 2 * (Slab<T, BM, FORM != FORM_TN, THREADS, 1>::BYTES + Slab<T, BN, FORM == FORM_NT, THREADS, 1>::BYTES);
-  constexpr int out = WAVES * 32 * (WN + 4) * 4;
-  constexpr int bytes = stages > out ? stages : out;
-  static_assert(bytes <= 160 * 1024, "LDS");
-  auto kern = gemm_kernel<T, FORM, BM, BN, WM, WN>;
-  static MltsLdsOptIn opt_in;
-  if (bytes > 48 * 1024) {
-    if (hipError_t e = opt_in.reserve(reinterpret_cast<const void*>(kern), bytes); e != hipSuccess) {
-      mlts_set_error("mlts_gemm: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
-      return MLTS_ERR_LAUNCH;
-    }
+void set_slices(Product& g, int64_t slices, int64_t slabs, int bk) {
+  const int64_t part = std::max<int64_t>(1, (slabs + slices - 1) / slices);
+  g.k_slice = static_cast<int>(part * bk);
+  g.slices = static_cast<int>(std::max<int64_t>(1, (slabs + part - 1) / part));
+}
+
+// A product that runs alone takes the largest tile that still gives every CU a workgroup; one with fewer tiles than CUs is split
+// along its contraction where that is long.  Best of all tiles and splits (us): NT 16384 x 512 x 512 256x128 15.6 (128x128 16.7,
+// 64x64 19.2, 256x256 21.6); NT 16384 x 2752 x 512 256x256 66 (76, 96, 77); NN 1023 x 512 x 32000 256x128 in 16 parts 45 (unsplit
+// 210); TN 512 x 512 x 16384 in 32 parts 24 (128x128 in 16: 23); TN 2752 x 512 x 16384 in 4 parts 70 (256x256 in 8: 68).
+int choose_tile(const mlts_gemm_product& p, int dtype, int64_t* slices) {
+  const int64_t slabs = slabs_of(p, slab_of(dtype)), t2 = tiles_of(p.M, p.N, 256, 128);
+  *slices = 1;
+  if (p.segments > 1) return kSmall;
+  if (tiles_of(p.M, p.N, 256, 256) >= 240) return 3;
+  if (t2 >= 256) return 2;
+  if (dtype == MLTS_BF16 && slabs >= 64 && t2 * (slabs / 8) >= 192) {
+    while (t2 * *slices * 2 <= 256 && slabs / (*slices * 2) >= 8) *slices *= 2;
+    return 2;
   }
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g.tiles_m * g.tiles_n * g.slices)), dim3(THREADS), bytes, st, g);
+  return tiles_of(p.M, p.N, 128, 128) >= 256 ? 1 : kSmall;
+}
+bool splittable(const mlts_gemm_product& p) { return p.segments == 1 && p.N % 4 == 0 && p.ldc == p.N; }
+
+// The small products of a launch together: tiles of 64 x 64, or in fp32 also of 32 x 32, whose four wavefronts share a tile along
+// the contraction (us, 64 x 64 / 32 x 32: NT 2048 x 256 x 256 8.2 / 6.3, NN 1000 x 512 x 1376 31.4 / 17.1, 500 x 256 x 256 7.9 /
+// 4.6, but 2048 x 1376 x 512 29.8 / 32.4).  chain: us a workgroup takes for a slab; busy: us of a CU for each slab when it has
+// several workgroups (measured).
+struct SmallShape {
+  int size;
+  double chain, busy;
+};
+constexpr SmallShape kBf16Shape{64, 0.26, 0.16}, kF32Shape{64, 0.65, 0.5}, kF32Fine{32, 0.31, 0.16};
+
+// Slices of each product, and the estimated time: the longest chain of slabs, or the product on all 256 CUs if that is longer, and
+// what a split costs: a launch that joins the slices and their fp32 sums written and read.  A weight gradient's split does not
+// depend on what shares its launch, so that its bits do not either.  (us: NN 1024 x 512 x 2752 whole 14.8, in
+// two 13.0, in four 14.5; TN 512 x 512 x 2048 whole 12.0, in four 9.5; TN 512 x 512 x 1024 whole 7.6, in two 8.3; fp32 TN 256 x 256 x
+// 2048 whole 20.5, in eight 8.9; fp32 NN 1000 x 512 x 1376 whole 17.1, in two 20.3.)
+double small_slices(const mlts_gemm_product* const* ps, int count, int dtype, const SmallShape& shape, int64_t* slices) {
+  const int bk = slab_of(dtype);
+  double longest = 0;
+  for (int i = 0; i < count; ++i) {
+    const int64_t slabs = slabs_of(*ps[i], bk), tiles = tiles_of(ps[i]->M, ps[i]->N, shape.size, shape.size);
+    const int company = count > 1 && ps[i]->form == FORM_NN ? 2 : 1;  // beside dx runs a dW of the same size
+    const double whole = static_cast<double>(tiles * slabs * company) * shape.busy / 256;
+    auto cost = [&](int64_t s) {
+      return std::max(shape.chain * static_cast<double>(slabs) / static_cast<double>(s), whole) +
+             (s > 1 ? 2.5 + 8.0 * static_cast<double>(s * ps[i]->M * ps[i]->N) / 3.5e6 : 0.0);
+    };
+    slices[i] = 1;
+    for (int64_t s = 2; splittable(*ps[i]) && s <= 16 && slabs / s >= 4; s *= 2)
+      if (cost(s) < cost(slices[i])) slices[i] = s;
+    longest = std::max(longest, cost(slices[i]));
+  }
+  return longest;
+}
+
+struct LaunchPlan {
+  int tile[kMaxProducts];
+  int64_t slices[kMaxProducts];
+  const mlts_gemm_product* small[kMaxProducts];
+  int small_at[kMaxProducts], smalls = 0;
+  SmallShape shape;
+  int64_t workspace = 0;  // bytes
+  LaunchPlan(const mlts_gemm_product* ps, int count, int dtype) : shape(dtype == MLTS_BF16 ? kBf16Shape : kF32Shape) {
+    for (int i = 0; i < count; ++i) {
+      tile[i] = choose_tile(ps[i], dtype, &slices[i]);
+      if (tile[i] == kSmall) small_at[smalls] = i, small[smalls++] = &ps[i];
+      else if (!splittable(ps[i])) slices[i] = 1;
+    }
+    if (smalls) {
+      int64_t s[kMaxProducts], fine[kMaxProducts];
+      const double coarse = small_slices(small, smalls, dtype, shape, s);
+      if (dtype == MLTS_F32 && small_slices(small, smalls, dtype, kF32Fine, fine) < coarse) shape = kF32Fine, std::copy(fine, fine + smalls, s);
+      for (int i = 0; i < smalls; ++i) slices[small_at[i]] = s[i];
+    }
+    for (int i = 0; i < count; ++i)
+      if (slices[i] > 1) workspace += ps[i].M * ps[i].N * 4 * slices[i];
+  }
+};
+
+template <typename S>
+int opt_in_lds(MltsLdsOptIn& once, const void* kern, int bytes, S what) {
+  if (bytes <= 48 * 1024) return MLTS_OK;
+  if (hipError_t e = once.reserve(kern, bytes); e != hipSuccess) {
+    mlts_set_error("%s: cannot reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+    return MLTS_ERR_LAUNCH;
+  }
   return MLTS_OK;
 }
 
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG = 1>
+int launch_tile(const Product& g, hipStream_t st) {
+  typedef TileShape<T, FORM, BM, BN, WM, WN, KG> S;
+  static_assert(S::LDS <= 160 * 1024, "LDS");
+  auto kern = gemm_kernel<T, FORM, BM, BN, WM, WN, KG>;
+  static MltsLdsOptIn once;
+  if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm"); rc != MLTS_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g.tiles_m * g.tiles_n * g.slices)), dim3(S::THREADS), S::LDS, st, g);
+  return MLTS_OK;
+}
 template <typename T, int FORM>
-int launch_form(int tile, const GemmArgs& g, hipStream_t st) {
-  if (tile == 0) return launch_tile<T, FORM, 64, 64, 32, 32>(g, st);
+int launch_form(int tile, const SmallShape& shape, const Product& g, hipStream_t st) {
   if (tile == 1) return launch_tile<T, FORM, 128, 128, 64, 64>(g, st);
   if (tile == 2) return launch_tile<T, FORM, 256, 128, 64, 64>(g, st);
-  return launch_tile<T, FORM, 256, 256, 128, 64>(g, st);
+  if (tile == 3) return launch_tile<T, FORM, 256, 256, 128, 64>(g, st);
+  if constexpr (sizeof(T) == 4) {
+    if (shape.size == 32) return launch_tile<T, FORM, 32, 32, 32, 32, 4>(g, st);
+  }
+  return launch_tile<T, FORM, 64, 64, 32, 32>(g, st);
+}
+template <typename T>
+int launch_alone(int tile, const SmallShape& shape, const Product& g, hipStream_t st) {
+  if (g.form == FORM_NT) return launch_form<T, FORM_NT>(tile, shape, g, st);
+  return g.form == FORM_NN ? launch_form<T, FORM_NN>(tile, shape, g, st) : launch_form<T, FORM_TN>(tile, shape, g, st);
 }
 
-bool small_enough(int64_t lines, int64_t ld, int es) { return lines * ld * es < (int64_t{1} << 31) - 4096; }
+template <typename T, int FORMS, int BM, int BN, int KG>
+int launch_small(const Products& ps, int blocks, hipStream_t st) {
+  constexpr int nt = TileShape<T, FORM_NT, BM, BN, 32, 32, KG>::LDS, nn = TileShape<T, FORM_NN, BM, BN, 32, 32, KG>::LDS,
+                tn = TileShape<T, FORM_TN, BM, BN, 32, 32, KG>::LDS;
+  constexpr int bytes = FORMS == FORMS_NT ? nt : FORMS == FORMS_NN ? nn : std::max(nt, std::max(nn, tn));
+  static_assert(TileShape<T, FORM_NT, BM, BN, 32, 32, KG>::THREADS == 256, "four wavefronts");
+  auto kern = gemm_multi_kernel<T, FORMS, BM, BN, KG>;
+  static MltsLdsOptIn once;
+  if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), bytes, "mlts_gemm"); rc != MLTS_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), bytes, st, ps);
+  return MLTS_OK;
+}
+template <typename T, int BM, int BN, int KG>
+int launch_small_forms(int forms, const Products& ps, int blocks, hipStream_t st) {
+  switch (forms) {
+    case FORMS_NT: return launch_small<T, FORMS_NT, BM, BN, KG>(ps, blocks, st);
+    case FORMS_NN: return launch_small<T, FORMS_NN, BM, BN, KG>(ps, blocks, st);
+    case FORMS_ANY: return launch_small<T, FORMS_ANY, BM, BN, KG>(ps, blocks, st);
+    default: return launch_small<T, FORMS_SEGMENTS, BM, BN, KG>(ps, blocks, st);
+  }
+}
+
+const char* why_not(const mlts_gemm_product& p, int dtype) {
+  if (p.form < FORM_NT || p.form > FORM_TN) return "unknown form";
+  if (p.segments < 1 || p.segments > (p.form == FORM_NN ? kMaxSegments : 1)) return "bad number of segments";
+  if (p.M < 0 || p.N < 0 || p.M > 0x7fffffff || p.N > 0x7fffffff) return "bad shape";
+  if (p.ldc < p.N || p.ldc > 0x7fffffff) return "row strides must be at least the row length and fit 32 bits";
+  const int es = dtype == MLTS_BF16 ? 2 : 4, v = 16 / es;
+  const bool a_kc = p.form != FORM_TN, b_kc = p.form == FORM_NT;
+  for (int i = 0; i < p.segments; ++i) {
+    const int64_t K = p.k[i];
+    if (K < 0 || K > 0x7fffffff || p.lda[i] > 0x7fffffff || p.ldb[i] > 0x7fffffff) return "bad shape";
+    if (p.lda[i] % v || p.ldb[i] % v) return "operand rows must be 16-byte aligned";
+    if ((a_kc || b_kc) && K % v) return "the contraction must be a multiple of 16 bytes";
+    if (p.lda[i] < (a_kc ? K : p.M) || p.ldb[i] < (b_kc ? K : p.N)) return "row strides must be at least the row length";
+    const int64_t limit = (int64_t{1} << 31) - 4096;
+    if ((a_kc ? p.M : K) * p.lda[i] * es >= limit || (b_kc ? p.N : K) * p.ldb[i] * es >= limit) return "operands of 2 GiB or more";
+  }
+  return nullptr;
+}
+
+mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
+                         int32_t accumulate) {
+  mlts_gemm_product p{};
+  p.form = form, p.segments = 1, p.accumulate = accumulate;
+  p.M = M, p.N = N, p.k[0] = K;
+  p.a[0] = a, p.lda[0] = lda, p.b[0] = b, p.ldb[0] = ldb, p.c = c, p.ldc = ldc;
+  return p;
+}
+
+template <typename T>
+int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hipStream_t st) {
+  const LaunchPlan plan(ps, count, dtype);
+  Products joint{};
+  Joins joins{};
+  int blocks = 0, join_blocks = 0, smalls = 0;
+  bool all_nt = true, all_nn = true, segments = false;
+  std::fill(joint.first, joint.first + kMaxProducts, 0x7fffffff);
+  MltsKernelTimer timer("gemm", st);
+  for (int i = 0; i < count; ++i) {
+    const mlts_gemm_product& p = ps[i];
+    const bool small = plan.tile[i] == kSmall;
+    const int bm = small ? plan.shape.size : kTileM[plan.tile[i]], bn = small ? plan.shape.size : kTileN[plan.tile[i]];
+    Product g{};
+    g.a = p.a[0], g.b = p.b[0], g.c = p.c;
+    g.lda = static_cast<int>(p.lda[0]), g.ldb = static_cast<int>(p.ldb[0]), g.ldc = static_cast<int>(p.ldc), g.K = static_cast<int>(p.k[0]);
+    g.form = p.form, g.accumulate = p.accumulate != 0;
+    g.M = static_cast<int>(p.M), g.N = static_cast<int>(p.N);
+    g.tiles_m = static_cast<int>((p.M + bm - 1) / bm), g.tiles_n = static_cast<int>((p.N + bn - 1) / bn);
+    const int64_t slabs = slabs_of(p, slab_of(dtype));
+    set_slices(g, plan.slices[i], slabs, slab_of(dtype));
+    if (p.segments > 1) {
+      g.k_slice = g.K;
+      for (int k = 1; k < p.segments; ++k) {
+        joint.more.a[k - 1] = p.a[k], joint.more.b[k - 1] = p.b[k];
+        joint.more.lda[k - 1] = static_cast<int>(p.lda[k]), joint.more.ldb[k - 1] = static_cast<int>(p.ldb[k]), joint.more.K[k - 1] = static_cast<int>(p.k[k]);
+      }
+      joint.more.count = p.segments - 1, joint.more.product = smalls;
+    }
+    const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices;
+    MLTS_REQUIRE(blocks + tiles < (int64_t{1} << 30), "mlts_gemm: too many tiles");
+    if (tiles == 0) continue;
+    if (plan.slices[i] > 1) {
+      g.partial = workspace;
+      workspace += p.M * p.N * plan.slices[i];
+      joins.p[joins.count++] = {p.c, g.partial, g.slices, g.accumulate, join_blocks, p.M * p.N / 4};
+      join_blocks += static_cast<int>((p.M * p.N / 4 + 255) / 256);
+    }
+    if (small && count > 1) {
+      all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN, segments = segments || p.segments > 1;
+      joint.first[smalls] = blocks;
+      blocks += static_cast<int>((tiles + 7) / 8 * 8);  // (whole rounds over the XCDs, so that each product starts at the first)
+      joint.p[smalls++] = g;
+    } else if (int rc = launch_alone<T>(plan.tile[i], plan.shape, g, st); rc != MLTS_OK) {
+      return rc;
+    }
+  }
+  if (smalls) {
+    const int forms = segments ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
+    int rc;
+    if constexpr (sizeof(T) == 2) rc = launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
+    else if (plan.shape.size == 64) rc = launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
+    else rc = launch_small_forms<T, 32, 32, 4>(forms, joint, blocks, st);
+    if (rc != MLTS_OK) return rc;
+  }
+  if (joins.count) hipLaunchKernelGGL(gemm_join_kernel<T>, dim3(static_cast<unsigned>(join_blocks)), dim3(256), 0, st, joins);
+  return mlts_check_launch("mlts_gemm");
+}
 
 }  // namespace
 
 extern "C" const char* mlts_gemm_supports(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc) {
   if (dtype != MLTS_BF16 && dtype != MLTS_F32) return "dtype must be MLTS_F32 or MLTS_BF16";
-  if (form < FORM_NT || form > FORM_TN) return "unknown form";
-  if (M < 0 || N < 0 || K < 0 || M > 0x7fffffff || N > 0x7fffffff) return "bad shape";
-  const int es = dtype == MLTS_BF16 ? 2 : 4, v = 16 / es;
-  if (lda % v || ldb % v) return "operand rows must be 16-byte aligned";
-  const bool a_kc = form != FORM_TN, b_kc = form == FORM_NT;
-  if ((a_kc || b_kc) && K % v) return "the contraction must be a multiple of 16 bytes";
-  if (lda < (a_kc ? K : M) || ldb < (b_kc ? K : N) || ldc < N) return "row strides must be at least the row length";
-  if (!small_enough(a_kc ? M : K, lda, es) || !small_enough(b_kc ? N : K, ldb, es)) return "operands of 2 GiB or more";
-  return nullptr;
+  return why_not(single(form, M, N, K, nullptr, lda, nullptr, ldb, nullptr, ldc, 0), dtype);
 }
 
 extern "C" int64_t mlts_gemm_workspace_bytes(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0) return 0;
-  const Plan p = make_plan(M, N, K, dtype == MLTS_BF16 ? 64 : 32, true);
-  return p.slices > 1 ? M * N * 4 * p.slices : 0;
+  const mlts_gemm_product p = single(form, M, N, K, nullptr, 0, nullptr, 0, nullptr, N, 0);
+  return M <= 0 || N <= 0 ? 0 : LaunchPlan(&p, 1, dtype).workspace;
+}
+
+extern "C" int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* products, int32_t count, int32_t dtype) {
+  return count < 1 || count > kMaxProducts ? 0 : LaunchPlan(products, count, dtype).workspace;
+}
+
+extern "C" int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
+                               mlts_stream_t stream) {
+  MLTS_REQUIRE(dtype == MLTS_BF16 || dtype == MLTS_F32, "mlts_gemm: unknown dtype %d", dtype);
+  MLTS_REQUIRE(products && count >= 1 && count <= kMaxProducts, "mlts_gemm: 1 to %d products in a call", kMaxProducts);
+  for (int i = 0; i < count; ++i) {
+    const mlts_gemm_product& p = products[i];
+    const char* why = why_not(p, dtype);
+    MLTS_REQUIRE(why == nullptr, "mlts_gemm: %s", why);
+    if (p.M == 0 || p.N == 0) continue;
+    MLTS_REQUIRE(p.c && mlts_aligned16(p.c), "mlts_gemm: pointers must be 16-byte aligned and not null");
+    for (int k = 0; k < p.segments; ++k)
+      MLTS_REQUIRE(p.k[k] == 0 || (p.a[k] && p.b[k] && mlts_aligned16(p.a[k]) && mlts_aligned16(p.b[k])),
+                   "mlts_gemm: pointers must be 16-byte aligned and not null");
+  }
+  const int64_t need = mlts_gemm_multi_workspace_bytes(products, count, dtype);
+  MLTS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && mlts_aligned16(workspace)), "mlts_gemm: workspace too small or unaligned");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  float* ws = static_cast<float*>(workspace);
+  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, ws, st) : run<float>(products, count, dtype, ws, st);
 }
 
 extern "C" int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb,
                          void* c, int64_t ldc, int32_t accumulate, void* workspace, int64_t workspace_bytes, mlts_stream_t stream) {
-  const char* why = mlts_gemm_supports(form, dtype, M, N, K, lda, ldb, ldc);
-  MLTS_REQUIRE(why == nullptr, "mlts_gemm: %s", why);
-  if (M == 0 || N == 0) return MLTS_OK;
-  MLTS_REQUIRE(c && (K == 0 || (a && b)), "mlts_gemm: null pointer");
-  MLTS_REQUIRE(mlts_aligned16(a) && mlts_aligned16(b) && mlts_aligned16(c), "mlts_gemm: pointers must be 16-byte aligned");
-  const Plan p = make_plan(M, N, K, dtype == MLTS_BF16 ? 64 : 32, ldc == N);
-  GemmArgs g{};
-  g.a = a;
-  g.b = b;
-  g.c = c;
-  g.lda = lda;
-  g.ldb = ldb;
-  g.ldc = ldc;
-  g.M = static_cast<int>(M);
-  g.N = static_cast<int>(N);
-  g.K = K;
-  g.k_slice = p.k_slice;
-  g.slices = p.slices;
-  g.accumulate = accumulate != 0;
-  g.tiles_m = static_cast<int>((M + kTileM[p.tile] - 1) / kTileM[p.tile]);
-  g.tiles_n = static_cast<int>((N + kTileN[p.tile] - 1) / kTileN[p.tile]);
-  MLTS_REQUIRE(static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices < (int64_t{1} << 31), "mlts_gemm: too many tiles");
-  if (p.slices > 1) {
-    MLTS_REQUIRE(workspace && workspace_bytes >= M * N * 4 * p.slices && mlts_aligned16(workspace), "mlts_gemm: workspace too small or unaligned");
-    g.partial = static_cast<float*>(workspace);
-  }
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  MltsKernelTimer timer("gemm", st);
-  int rc;
-  if (dtype == MLTS_BF16)
-    rc = form == FORM_NT ? launch_form<bf16_t, FORM_NT>(p.tile, g, st)
-         : form == FORM_NN ? launch_form<bf16_t, FORM_NN>(p.tile, g, st) : launch_form<bf16_t, FORM_TN>(p.tile, g, st);
-  else
-    rc = form == FORM_NT ? launch_form<float, FORM_NT>(p.tile, g, st)
-         : form == FORM_NN ? launch_form<float, FORM_NN>(p.tile, g, st) : launch_form<float, FORM_TN>(p.tile, g, st);
-  if (rc != MLTS_OK) return rc;
-  if (p.slices > 1) {
-    const int64_t n4 = M * N / 4;
-    const dim3 grid(static_cast<unsigned>((n4 + 255) / 256));
-    if (dtype == MLTS_BF16) {
-      if (accumulate) hipLaunchKernelGGL((gemm_join_kernel<bf16_t, true>), grid, dim3(256), 0, st, static_cast<bf16_t*>(c), g.partial, p.slices, n4);
-      else hipLaunchKernelGGL((gemm_join_kernel<bf16_t, false>), grid, dim3(256), 0, st, static_cast<bf16_t*>(c), g.partial, p.slices, n4);
-    } else {
-      if (accumulate) hipLaunchKernelGGL((gemm_join_kernel<float, true>), grid, dim3(256), 0, st, static_cast<float*>(c), g.partial, p.slices, n4);
-      else hipLaunchKernelGGL((gemm_join_kernel<float, false>), grid, dim3(256), 0, st, static_cast<float*>(c), g.partial, p.slices, n4);
-    }
-  }
-  return mlts_check_launch("mlts_gemm");
+  const mlts_gemm_product p = single(form, M, N, K, a, lda, b, ldb, c, ldc, accumulate);
+  return mlts_gemm_multi(&p, 1, dtype, workspace, workspace_bytes, stream);
 }

@@ -93,6 +93,17 @@ bool own_product(int form, const Tensor& a, const Tensor& b);  // whether `produ
 // a, b as the form (MLTS_GEMM_*) says -> [M, N], written to `out` (or added onto it) if that is given
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out = Tensor(), bool accumulate = false);  // products.cpp
 
+bool own_output(const Tensor& out, const Tensor& a);  // whether the own kernels can write a product with `a` to `out`
+// Products that run on the own kernels (own_product, own_output), in one call: small ones in one launch.
+struct ProductList {
+  mlts_gemm_product items[4];
+  int count = 0;
+  Tensor like;
+  void add(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate);
+  void add_segment(const Tensor& a, const Tensor& b);  // NN: the last product also gets + a b
+  void run() const;
+};
+
 void notify_grad_written(const Tensor& param);  // llama.cpp: the parameter's gradient buffer was written past autograd
 // the gradient buffer a weight already owns and a backward formula may add into, or undefined
 inline Tensor bound_grad(const Tensor& weight, bool into_grad) {

@@ -122,6 +122,8 @@ int64_t weight_grad_splits(int64_t rows, int64_t out_features, int64_t in_featur
   return splits;
 }
 
+Tensor rows2d(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
+
 // dW = dy2^T x2 for [rows, out] / [rows, in] operands, large ones as a batch of row-slice products where that fills the chip
 // better.  With `grad` (the gradient buffer the weight already owns, a view of a flat gradient buffer) dW is added into it in
 // the pass that finishes it and nothing is returned.
@@ -137,14 +139,28 @@ Tensor weight_grad(const Tensor& x2, const Tensor& dy2, const Tensor& grad) {
   return grad.defined() ? Tensor() : dw;
 }
 
-Tensor rows2d(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
-
 Tensor project(const Tensor& x, const Tensor& weight) {
   if (x.dim() == 2 && x.is_contiguous()) return product(MLTS_GEMM_NT, x, weight);
   if (!x.is_contiguous()) return at::linear(x, weight);
   c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = weight.size(0);
   return product(MLTS_GEMM_NT, rows2d(x), weight).view(shape);
+}
+
+// dx = dy2 w and dw = dy2^T x2 (added into `grad` if that is defined, and then not returned): in one launch where both run on
+// the own kernels, as neither fills the chip at the sizes they are used for
+std::pair<Tensor, Tensor> input_and_weight_grad(const Tensor& dy2, const Tensor& w, const Tensor& x2, const Tensor& grad) {
+  if (own_product(MLTS_GEMM_NN, dy2, w) && own_product(MLTS_GEMM_TN, dy2, x2) && (!grad.defined() || own_output(grad, x2))) {
+    Tensor dx = at::empty({dy2.size(0), w.size(1)}, dy2.options());
+    Tensor dw = grad.defined() ? grad : at::empty(w.sizes(), dy2.options());
+    ProductList list;
+    list.add(MLTS_GEMM_TN, dy2, x2, dw, grad.defined());  // the longer contraction first
+    list.add(MLTS_GEMM_NN, dy2, w, dx, false);
+    list.run();
+    return {dx, grad.defined() ? Tensor() : dw};
+  }
+  Tensor dx = product(MLTS_GEMM_NN, dy2, w);
+  return {dx, weight_grad(x2, dy2, grad)};
 }
 
 struct LinearBackward final : Formula {
@@ -157,10 +173,16 @@ struct LinearBackward final : Formula {
     if (!dy.defined()) return {Tensor(), Tensor()};
     Tensor dx, dw;
     const Tensor dy2 = rows2d(dy);
-    if (task_should_compute_output(0)) dx = product(MLTS_GEMM_NN, dy2, w).view(x.sizes());
-    if (task_should_compute_output(1)) {
-      const Tensor grad = bound_grad(w, into_grad);
-      dw = weight_grad(rows2d(x), dy2, grad);
+    const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
+    const Tensor grad = need_dw ? bound_grad(w, into_grad) : Tensor();
+    if (need_dx && need_dw) {
+      std::tie(dx, dw) = input_and_weight_grad(dy2, w, rows2d(x), grad);
+      dx = dx.view(x.sizes());
+    } else if (need_dx) {
+      dx = product(MLTS_GEMM_NN, dy2, w).view(x.sizes());
+    }
+    if (need_dw) {
+      if (!need_dx) dw = weight_grad(rows2d(x), dy2, grad);
       if (grad.defined()) notify_grad_written(w);  // autograd's hooks on the weight see no gradient for what was added here
     }
     return {dx, dw};
@@ -228,11 +250,15 @@ Tensor embedding(const Tensor& weight, const Tensor& ids, bool into_grad) {
 // of one allocation (what the flat optimizer layouts make of them), they ARE one [sum of out_features, in_features] matrix,
 // and the three (two) products are one: at LLaMA-50M sizes a 512-wide product has 128 output tiles for 256 compute units,
 // the 1536-wide one fills the chip, and the backward's three input-gradient products and their two additions become one.
+// Parameters that are not adjacent still share their input: at sizes where the products run on the own kernels, all of a pass are
+// one launch, and the outputs are column ranges of one buffer as above (`rows` then has no `weight`).
 struct Adjacent {
   Tensor weight;                     // [R, in]; undefined: the parameters are not adjacent
   Tensor grad;                       // their gradients as one matrix like `weight`, when those are adjacent in the same order
   std::vector<int64_t> first;        // output column of parameter i's first row
-  std::vector<size_t> order;         // parameters by address
+  std::vector<size_t> order;         // parameters by output column
+  int64_t width = 0;                 // their rows together
+  bool similar = false;              // not adjacent, but of one input width and type: may run as a group
   std::vector<std::pair<const void*, const void*>> key;  // addresses of the parameters and their gradients this was made for
 
   explicit Adjacent(const std::vector<Tensor>& params) {
@@ -240,19 +266,26 @@ struct Adjacent {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     const Tensor& p0 = params[0];
     for (const Tensor& p : params)
-      if (p.dim() != 2 || !p.is_cuda() || !p.is_contiguous() || p.scalar_type() != p0.scalar_type() || p.size(1) != p0.size(1) || !p.requires_grad()) return;
+      if (p.dim() != 2 || !p.is_cuda() || !p.is_contiguous() || p.scalar_type() != p0.scalar_type() || p.size(1) != p0.size(1)) return;
     order.resize(params.size());
-    std::iota(order.begin(), order.end(), size_t{0});
-    std::sort(order.begin(), order.end(), [&](size_t i, size_t j) { return key[i].first < key[j].first; });
     first.resize(params.size());
+    std::iota(order.begin(), order.end(), size_t{0});
+    for (size_t i = 0; i < params.size(); ++i) first[i] = width, width += params[i].size(0);
+    similar = params.size() <= 3;
+    for (const Tensor& p : params)
+      if (!p.requires_grad()) return;
+    std::vector<size_t> in_order = order;
+    std::sort(in_order.begin(), in_order.end(), [&](size_t i, size_t j) { return key[i].first < key[j].first; });
+    std::vector<int64_t> at(params.size());
     int64_t rows = 0;
-    const char* next = static_cast<const char*>(key[order[0]].first);
-    for (size_t i : order) {
+    const char* next = static_cast<const char*>(key[in_order[0]].first);
+    for (size_t i : in_order) {
       if (key[i].first != next || !params[i].storage().is_alias_of(p0.storage())) return;
-      first[i] = rows;
+      at[i] = rows;
       rows += params[i].size(0);
       next += params[i].nbytes();
     }
+    order = in_order, first = at;
     const Tensor& base = params[order[0]];
     weight = base.as_strided({rows, base.size(1)}, {base.size(1), 1}, base.storage_offset());
     const Tensor g0 = params[order[0]].grad();
@@ -303,16 +336,79 @@ Tensor adjacent_columns(const std::vector<Tensor>& parts, const std::vector<size
   return first.as_strided({rows, total}, {total, 1}, first.storage_offset());
 }
 
-// dW of the common matrix: added into the adjacent gradients, or returned as one gradient per parameter
-variable_list adjacent_weight_grads(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, const Tensor& x2, const Tensor& dy2) {
-  variable_list out(weights.size());
-  const Tensor grad = into_grad ? a.grad : Tensor();
-  const Tensor dw = weight_grad(x2, dy2, grad);
-  if (grad.defined()) {
-    for (const Tensor& w : weights) notify_grad_written(w);
+// whether the products with these parameters, not adjacent, run as one launch
+bool runs_as_group(const Adjacent& a, const Tensor& x, const std::vector<Tensor>& weights) {
+  if (!a.similar || a.weight.defined() || !x.is_cuda() || !x.is_contiguous() || x.dim() < 2 || x.numel() == 0) return false;
+  const Tensor x2 = rows2d(x);
+  for (size_t i = 0; i < weights.size(); ++i)
+    if (a.first[i] * x.element_size() % 16 || weights[i].size(1) != x.size(-1) || !own_product(MLTS_GEMM_NT, x2, weights[i])) return false;
+  return a.width * x.element_size() % 16 == 0;
+}
+
+// x times all of the parameters, transposed: their outputs side by side
+Tensor project_all(const Tensor& x, const Adjacent& rows, const std::vector<Tensor>& weights) {
+  if (rows.weight.defined()) return project(x, rows.weight);
+  c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = rows.width;
+  Tensor y = at::empty(shape, x.options());
+  const Tensor x2 = rows2d(x), y2 = rows2d(y);
+  ProductList list;
+  for (size_t i = 0; i < weights.size(); ++i) list.add(MLTS_GEMM_NT, x2, weights[i], y2.narrow(1, rows.first[i], weights[i].size(0)), false);
+  list.run();
+  return y;
+}
+
+// The input gradient (if asked for), then one gradient per parameter: added into the gradient buffers where into_grad allows it,
+// and then undefined.  dy2: the outputs' gradients side by side.
+variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, bool need_dx, const Tensor& x, const Tensor& dy2) {
+  variable_list out(1 + weights.size());
+  const Tensor x2 = rows2d(x);
+  if (a.weight.defined()) {
+    const Tensor grad = into_grad ? a.grad : Tensor();
+    Tensor dw;
+    if (need_dx) std::tie(out[0], dw) = input_and_weight_grad(dy2, a.weight, x2, grad);
+    else dw = weight_grad(x2, dy2, grad);
+    for (size_t i = 0; i < weights.size(); ++i) {
+      if (grad.defined()) notify_grad_written(weights[i]);
+      else out[1 + i] = dw.narrow(0, a.first[i], weights[i].size(0));
+    }
   } else {
-    for (size_t i = 0; i < weights.size(); ++i) out[i] = dw.narrow(0, a.first[i], weights[i].size(0));
+    std::vector<Tensor> parts, into;
+    bool own = true;
+    for (size_t i = 0; i < weights.size(); ++i) {
+      parts.push_back(dy2.narrow(1, a.first[i], weights[i].size(0)));
+      into.push_back(bound_grad(weights[i], into_grad && weights[i].requires_grad()));
+      own = own && own_product(MLTS_GEMM_NN, parts[i], weights[i]) && own_product(MLTS_GEMM_TN, parts[i], x2) &&
+            (!into[i].defined() || own_output(into[i], x2));
+    }
+    if (own) {
+      ProductList list;
+      for (size_t i = 0; i < weights.size(); ++i) {
+        Tensor dw = into[i].defined() ? into[i] : at::empty(weights[i].sizes(), dy2.options());
+        list.add(MLTS_GEMM_TN, parts[i], x2, dw, into[i].defined());
+        if (!into[i].defined()) out[1 + i] = dw;
+      }
+      if (need_dx) {
+        out[0] = at::empty(x2.sizes(), dy2.options());
+        for (size_t i = weights.size(); i-- > 0;) {  // last one first: the order in which autograd adds them up
+          if (i + 1 == weights.size()) list.add(MLTS_GEMM_NN, parts[i], weights[i], out[0], false);
+          else list.add_segment(parts[i], weights[i]);
+        }
+      }
+      list.run();
+    } else {
+      for (size_t i = weights.size(); i-- > 0;) {
+        if (need_dx) {
+          Tensor dx = product(MLTS_GEMM_NN, parts[i], weights[i]);
+          out[0] = out[0].defined() ? out[0].add_(dx) : dx;
+        }
+        out[1 + i] = weight_grad(x2, parts[i], into[i]);
+      }
+    }
+    for (size_t i = 0; i < weights.size(); ++i)
+      if (into[i].defined()) notify_grad_written(weights[i]);
   }
+  if (out[0].defined()) out[0] = out[0].view(x.sizes());
   return out;
 }
 
@@ -324,7 +420,6 @@ struct AdjacentLinearsBackward final : Formula {
   AdjacentLinearsBackward() : Formula(COUNT) {}
   std::string name() const override { return "MaltosAdjacentLinearsBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
-    const Tensor x2 = rows2d(s[X]);
     bool all = true, any = false;
     for (const Tensor& dy : g) all = all && dy.defined(), any = any || dy.defined();
     variable_list out(1 + weights.size());
@@ -340,19 +435,20 @@ struct AdjacentLinearsBackward final : Formula {
         dy2 = pybind11::module_::import("torch").attr("cat")(parts, 1).cast<Tensor>();
       }
     } else {
-      dy2 = at::empty({x2.size(0), rows->weight.size(0)}, x2.options());
+      dy2 = at::empty({rows2d(s[X]).size(0), rows->width}, s[X].options());
       for (size_t i = 0; i < weights.size(); ++i) {
         Tensor part = dy2.narrow(1, rows->first[i], weights[i].size(0));
         if (g[i].defined()) part.copy_(g[i].reshape({-1, g[i].size(-1)}));
         else part.zero_();
       }
     }
-    if (task_should_compute_output(0)) out[0] = product(MLTS_GEMM_NN, dy2, rows->weight).view(s[X].sizes());
-    variable_list dws = adjacent_weight_grads(*rows, weights, into_grad, x2, dy2);
-    std::move(dws.begin(), dws.end(), out.begin() + 1);
-    return out;
+    return grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dy2);
   }
 };
+
+bool any_requires_grad(const std::vector<Tensor>& ts) {
+  return std::any_of(ts.begin(), ts.end(), [](const Tensor& t) { return t.requires_grad(); });
+}
 
 template <typename F>
 std::shared_ptr<F> adjacent_formula(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
@@ -365,15 +461,15 @@ std::shared_ptr<F> adjacent_formula(const Tensor& x, const AdjacentPtr& rows, co
   return fn;
 }
 
-// (x W_0^T, x W_1^T, ...) from one product with the parameters' common matrix, as column slices of it
+// (x W_0^T, x W_1^T, ...) as column slices of one buffer: one product with the parameters' common matrix, or their group
 std::vector<Tensor> adjacent_linears(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
   std::vector<Tensor> out(weights.size());
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    const Tensor y = project(x, rows->weight);
+    const Tensor y = project_all(x, *rows, weights);
     for (size_t i = 0; i < weights.size(); ++i) out[i] = y.narrow(-1, rows->first[i], weights[i].size(0));
   }
-  if (at::GradMode::is_enabled()) {
+  if (at::GradMode::is_enabled() && (compute_requires_grad(x) || any_requires_grad(weights))) {
     const auto fn = adjacent_formula<AdjacentLinearsBackward>(x, rows, weights, into_grad);
     for (const Tensor& o : out) set_history(o, fn);
   }
@@ -393,11 +489,7 @@ struct GateUpBackward final : Formula {
     if (!g[0].defined()) return variable_list(3);
     const Tensor dgu = swiglu_rows_backward(g[0], s[GU], rows->first[0], rows->first[1], weights[0].size(0));
     const Tensor dgu2 = rows2d(dgu);
-    variable_list out(3);
-    if (task_should_compute_output(0)) out[0] = product(MLTS_GEMM_NN, dgu2, rows->weight).view(s[X].sizes());
-    variable_list dws = adjacent_weight_grads(*rows, weights, into_grad, rows2d(s[X]), dgu2);
-    std::move(dws.begin(), dws.end(), out.begin() + 1);
-    return out;
+    return grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dgu2);
   }
 };
 
@@ -405,10 +497,10 @@ Tensor gate_up(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tenso
   Tensor gu, h;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    gu = project(x, rows->weight);
+    gu = project_all(x, *rows, weights);
     h = swiglu_rows(gu, rows->first[0], rows->first[1], weights[0].size(0));
   }
-  if (at::GradMode::is_enabled()) {
+  if (at::GradMode::is_enabled() && (compute_requires_grad(x) || any_requires_grad(weights))) {
     const auto fn = adjacent_formula<GateUpBackward>(x, rows, weights, into_grad);
     fn->save(fn->GU, gu);
     set_history(h, fn);
@@ -485,6 +577,7 @@ void bind_llama(pybind11::module& m) {
   py::class_<Adjacent, AdjacentPtr>(m, "Adjacent")
       .def(py::init<const std::vector<Tensor>&>())
       .def("made_for", &Adjacent::made_for)
+      .def("runs_as_group", &runs_as_group)
       .def_property_readonly("adjacent", [](const Adjacent& a) { return a.weight.defined(); })
       .def_property_readonly("weight", [](const Adjacent& a) { return a.weight.defined() ? OptTensor(a.weight) : std::nullopt; })
       .def_property_readonly("grad", [](const Adjacent& a) { return a.grad.defined() ? OptTensor(a.grad) : std::nullopt; });

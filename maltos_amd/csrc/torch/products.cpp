@@ -49,8 +49,7 @@ bool own_product(int form, const Tensor& a, const Tensor& b) {
 }
 
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
-  if (!own_product(form, a, b) || (out.defined() && !(plain(out) && out.is_contiguous() && aligned(out) && out.scalar_type() == a.scalar_type())))
-    return library_product(form, a, b, out, accumulate);
+  if (!own_product(form, a, b) || (out.defined() && !own_output(out, a))) return library_product(form, a, b, out, accumulate);
   const Sizes z(form, a, b);
   Tensor c = out.defined() ? out : at::empty({z.M, z.N}, a.options());
   const int dtype = dtype_code(a);
@@ -59,6 +58,34 @@ Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bo
   check(mlts_gemm(form, dtype, z.M, z.N, z.K, ptr(a), a.stride(0), ptr(b), b.stride(0), mptr(c), z.N, accumulate,
                   ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
   return c;
+}
+
+bool own_output(const Tensor& out, const Tensor& a) {
+  return plain(out) && aligned(out) && out.scalar_type() == a.scalar_type() && out.stride(0) >= out.size(1);
+}
+
+void ProductList::add(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
+  const Sizes z(form, a, b);
+  mlts_gemm_product& p = items[count++];
+  p = {};
+  p.form = form, p.accumulate = accumulate;
+  p.M = z.M, p.N = z.N, p.c = mptr(out), p.ldc = out.size(0) > 1 ? out.stride(0) : z.N;
+  add_segment(a, b);
+  like = a;
+}
+
+void ProductList::add_segment(const Tensor& a, const Tensor& b) {
+  mlts_gemm_product& p = items[count - 1];
+  const int i = p.segments++;
+  p.k[i] = Sizes(p.form, a, b).K;
+  p.a[i] = ptr(a), p.lda[i] = a.stride(0), p.b[i] = ptr(b), p.ldb[i] = b.stride(0);
+}
+
+void ProductList::run() const {
+  const int dtype = dtype_code(like);
+  const int64_t ws_bytes = mlts_gemm_multi_workspace_bytes(items, count, dtype);
+  Tensor ws = workspace(ws_bytes, like);
+  check(mlts_gemm_multi(items, count, dtype, ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
 }
 
 }  // namespace maltos

@@ -57,15 +57,21 @@ class LlamaConfig:
 # The projections, the MLP and the rotary + attention block are C++ autograd nodes (csrc/torch/llama.cpp).  Projections that
 # share their input (q/k/v; gate/up) run as ONE product there whenever their weights are adjacent row blocks of one
 # allocation (what the flat optimizer layouts make of them: MasterWeightsOptimizer(flat=True), Zero1FlatBuffers): they ARE one
-# [sum of out_features, in_features] matrix.  Parameter names, shapes and values are untouched; without adjacency the
-# projections run one by one as in the reference (models/llama.py:134-142,196-206).
-def _fused_rows(holder: nn.Module, params: list[nn.Parameter]):
-    """The parameters as one matrix (`weight`, and `grad` when their gradients are adjacent too), kept on the module until a
-    parameter or gradient moves; None when they are not adjacent."""
+# [sum of out_features, in_features] matrix.  Parameter names, shapes and values are untouched.  Otherwise the projections run
+# one by one as in the reference (models/llama.py:134-142,196-206).
+#
+# Without adjacency, and at sizes where the own product kernels run, the products of a pass are still one launch, and their
+# input gradient is formed in one sum.
+def _fused_rows(holder: nn.Module, modules: list[nn.Module], params: list[nn.Parameter], x: torch.Tensor):
+    """The parameters as one matrix (`weight`, and `grad` when their gradients are adjacent too) or as a group of such that
+    share a launch, kept on the module until a parameter or gradient moves; None when they run one by one."""
     rows = holder.__dict__.get("_maltos_hip_fused_rows")
     if rows is None or not rows.made_for(params):
         rows = holder.__dict__["_maltos_hip_fused_rows"] = native().Adjacent(params)
-    return rows if rows.adjacent else None
+    if rows.adjacent:
+        return rows
+    plain = all(type(m) is HipLinear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks) for m in modules)
+    return rows if plain and rows.runs_as_group(x, params) else None
 
 
 def _adjacent_columns(parts: list[torch.Tensor]) -> torch.Tensor | None:
@@ -235,8 +241,8 @@ class LlamaAttention(nn.Module):
         fused = None
         if self.fuse_projections and x.is_cuda and _fusable(projections):
             weights = [m.weight for m in projections]
-            fused = _fused_rows(self, weights)
-        if fused is not None:   # one product over the three adjacent weights
+            fused = _fused_rows(self, projections, weights, x)
+        if fused is not None:   # one product over the three adjacent weights, or one launch
             q, k, v = native().adjacent_linears(x, fused, weights, all(m.accumulate_into_grad for m in projections))
         else:
             q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
@@ -274,7 +280,7 @@ class LlamaMLP(nn.Module):
         pair = [self.gate_proj, self.up_proj]
         if self.fuse_projections and x.is_cuda and _fusable(pair) and self.gate_proj.out_features % (16 // x.element_size()) == 0:
             weights = [self.gate_proj.weight, self.up_proj.weight]
-            fused = _fused_rows(self, weights)
+            fused = _fused_rows(self, pair, weights, x)
             if fused is not None:
                 return self.down_proj(native().gate_up(x, fused, weights, all(m.accumulate_into_grad for m in pair)))
         return self.down_proj(ops.swiglu(self.gate_proj(x), self.up_proj(x)))

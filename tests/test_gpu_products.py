@@ -58,3 +58,22 @@ def test_products_left_to_the_library(dev):
         want = expected(NT, a, b)
         assert (native().product(NT, a, b).double() - want).norm() <= 5e-3 * want.norm()
     assert _lib.lib().mlts_gemm_supports(NT, _lib.MLTS_BF16, 64, 64, 33, 33, 33, 64) is not None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,hidden,widths", [(8, 64, (64, 32, 32)), (333, 136, (96, 72, 40)), (1023, 512, (512, 256, 256)), (2048, 256, (688, 688)), (4104, 512, (1376, 1376))])
+def test_group_of_projections(dev, dtype, rows, hidden, widths):
+    """Projections that share their input, weights not adjacent: outputs, one input gradient over all of them, weight gradients."""
+    gen = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, hidden, generator=gen).to(dtype).to(dev).requires_grad_(True)
+    ws = [torch.randn(n, hidden, generator=gen).to(dtype).to(dev).requires_grad_(True) for n in widths]
+    dys = [torch.randn(rows, n, generator=gen).to(dtype).to(dev) for n in widths]
+    group = native().Adjacent(ws)
+    assert not group.adjacent and group.runs_as_group(x, ws)
+    ys = native().adjacent_linears(x, group, ws, False)
+    grads = torch.autograd.grad(ys, (x, *ws), dys)
+    rel = 4e-3 if dtype == torch.bfloat16 else 2e-6
+    xd, wd, dd = x.detach().double(), [w.detach().double() for w in ws], [d.double() for d in dys]
+    want = [xd @ w.t() for w in wd] + [sum(d @ w for d, w in zip(dd, wd))] + [d.t() @ xd for d in dd]
+    for got, w in zip([*ys, *grads], want):
+        assert (got.detach().double() - w).norm() <= rel * w.norm()
