@@ -89,6 +89,10 @@ Tensor swiglu_rows(const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t c
 Tensor swiglu_rows_backward(const Tensor& dh, const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t cols);
 Tensor grad_sum_slices(const Tensor& parts, const OptTensor& out, bool accumulate);
 
+// with autograd; into_grad: the weight's gradient is added into the buffer it owns
+Tensor rms_norm(const Tensor& x, const Tensor& w, double eps, bool into_grad);
+std::tuple<Tensor, Tensor> add_rms_norm(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad);  // (sum, its norm)
+
 bool own_product(int form, const Tensor& a, const Tensor& b);  // whether `product` runs on the own kernels: by size, type, layout
 // a, b as the form (MLTS_GEMM_*) says -> [M, N], written to `out` (or added onto it) if that is given
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out = Tensor(), bool accumulate = false);  // products.cpp

@@ -6,6 +6,11 @@
 #include <numeric>
 #include <unordered_map>
 
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/autograd/python_variable.h>
+
 #include "common.hpp"
 
 namespace maltos {
@@ -554,11 +559,289 @@ Tensor rope_attention(const Tensor& q, const Tensor& k, const Tensor& v, const T
   return out;
 }
 
+// ---- the layers of a model ------------------------------------------------------------------------------------------------
+// What a decoder layer is made of (models/llama.py:217-231) as four autograd nodes and no Python: the two norms above and the two
+// blocks below, with the kernels and the values of the modules one by one.  At a thousand tokens a layer's kernels take 60 us
+// forward, calling its modules one after the other 110 us of host time, and the views between them cost the backward pass
+// another 20.
+
+// [B, H, S, D] over [B, S, H, D] storage (or a column range of wider rows) as [B * S, H * D] rows
+Tensor as_rows(const Tensor& t) {
+  return t.as_strided({t.size(0) * t.size(2), t.size(1) * t.size(3)}, {t.stride(2), 1}, t.storage_offset());
+}
+// columns col .. col + heads * dim of [B, S, width] rows as [B, heads, S, dim]
+Tensor as_heads(const Tensor& rows, int64_t batch, int64_t seq, int64_t width, int64_t col, int64_t heads, int64_t dim) {
+  return rows.as_strided({batch, heads, seq, dim}, {seq * width, dim, width, 1}, rows.storage_offset() + col);
+}
+
+struct BlockWeights {
+  AdjacentPtr rows;              // of the projections that share the block's input
+  std::vector<Tensor> in;        // q, k, v or gate, up
+  Tensor out;                    // o or down
+  bool into_grad_in = false, into_grad_out = false;
+};
+
+template <typename F>
+std::shared_ptr<F> block_formula(const Tensor& x, const BlockWeights& w) {
+  auto fn = adjacent_formula<F>(x, w.rows, w.in, w.into_grad_in);
+  fn->add_next_edge(torch::autograd::impl::gradient_edge(w.out));
+  fn->save(fn->OUT_W, w.out);
+  fn->into_grad_out = w.into_grad_out;
+  return fn;
+}
+bool recorded(const Tensor& x, const BlockWeights& w) {
+  return at::GradMode::is_enabled() && (compute_requires_grad(x, w.out) || any_requires_grad(w.in));
+}
+
+// The last projection of a block: the gradients of its input and weight
+std::pair<Tensor, Tensor> output_grads(const Tensor& dy, const Tensor& w, const Tensor& rows, bool into_grad) {
+  const Tensor grad = bound_grad(w, into_grad && w.requires_grad());
+  auto grads = input_and_weight_grad(rows2d(dense(dy)), w, rows, grad);
+  if (grad.defined()) notify_grad_written(w);
+  return grads;
+}
+
+struct AttentionBlockBackward final : Formula {
+  enum { X, Q, K, V, OUT, LSE, COS, SIN, ROPE_POSITIONS, POSITIONS, SEQUENCES, OUT_W, COUNT };
+  AdjacentPtr rows;
+  std::vector<Tensor> weights;
+  bool into_grad = false, into_grad_out = false;
+  int64_t position_offset = 0, mask_mode = 0;
+  double scale = 0;
+  AttentionBlockBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosAttentionBlockBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    if (!g[0].defined()) return variable_list(5);
+    const Tensor &q = s[Q], &k = s[K];
+    const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+    auto [dvo, dwo] = output_grads(g[0], s[OUT_W], as_rows(s[OUT]), into_grad_out);
+    const OptTensor pos = optional_tensor(s[POSITIONS]), seq = optional_tensor(s[SEQUENCES]);
+    auto [dq, dk, dv] = attention_backward(as_heads(dvo, B, S, H * D, 0, H, D), q, k, s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq);
+    rope_pair(dq, dk, s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset, true, true);
+    const std::vector<Tensor> parts = {as_rows(dq), as_rows(dk), as_rows(dv)};
+    Tensor dqkv = adjacent_columns(parts, rows->order);
+    if (!dqkv.defined()) {
+      std::vector<Tensor> ordered;
+      for (size_t i : rows->order) ordered.push_back(parts[i]);
+      dqkv = at::cat(ordered, 1);
+    }
+    variable_list out = grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dqkv);
+    out.push_back(dwo);
+    return out;
+  }
+};
+
+struct Positions {
+  int64_t offset = 0;
+  OptTensor rope, ids, sequences;  // int32 rotary positions; positions and sequence ids of a document mask
+};
+
+Tensor attention_block(const Tensor& x, const BlockWeights& w, int64_t heads, int64_t kv_heads, const Tensor& cos, const Tensor& sin, const Positions& p) {
+  const int64_t B = x.size(0), S = x.size(1), D = w.in[0].size(0) / heads, width = w.rows->width;
+  const int64_t mask_mode = p.ids.has_value() ? MLTS_MASK_DOC : MLTS_MASK_CAUSAL;
+  const double scale = std::pow(static_cast<double>(D), -0.5);
+  Tensor q, k, v, qr, kr, out, lse, y;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    const Tensor qkv = project_all(x, *w.rows, w.in);
+    q = as_heads(qkv, B, S, width, w.rows->first[0], heads, D);
+    k = as_heads(qkv, B, S, width, w.rows->first[1], kv_heads, D);
+    v = as_heads(qkv, B, S, width, w.rows->first[2], kv_heads, D);
+    std::tie(qr, kr) = rope_pair(q, k, cos, sin, p.rope, p.offset, false, false);
+    std::tie(out, lse) = attention_forward(qr, kr, v, mask_mode, scale, p.ids, p.ids, p.sequences, p.sequences);
+    y = product(MLTS_GEMM_NT, as_rows(out), w.out).view({B, S, w.out.size(0)});
+  }
+  if (recorded(x, w)) {
+    auto fn = block_formula<AttentionBlockBackward>(x, w);
+    fn->save(fn->Q, qr), fn->save(fn->K, kr), fn->save(fn->V, v), fn->save(fn->OUT, out), fn->save(fn->LSE, lse);
+    fn->save(fn->COS, cos), fn->save(fn->SIN, sin);
+    fn->save(fn->ROPE_POSITIONS, p.rope), fn->save(fn->POSITIONS, p.ids), fn->save(fn->SEQUENCES, p.sequences);
+    fn->position_offset = p.offset, fn->mask_mode = mask_mode, fn->scale = scale;
+    set_history(y, fn);
+  }
+  return y;
+}
+
+struct MlpBlockBackward final : Formula {
+  enum { X, GU, H, OUT_W, COUNT };
+  AdjacentPtr rows;
+  std::vector<Tensor> weights;
+  bool into_grad = false, into_grad_out = false;
+  MlpBlockBackward() : Formula(COUNT) {}
+  std::string name() const override { return "MaltosMlpBlockBackward"; }
+  variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    if (!g[0].defined()) return variable_list(4);
+    auto [dh, dw] = output_grads(g[0], s[OUT_W], rows2d(s[H]), into_grad_out);
+    const Tensor dgu = swiglu_rows_backward(dh.view(s[H].sizes()), s[GU], rows->first[0], rows->first[1], weights[0].size(0));
+    variable_list out = grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], rows2d(dgu));
+    out.push_back(dw);
+    return out;
+  }
+};
+
+Tensor mlp_block(const Tensor& x, const BlockWeights& w) {
+  Tensor gu, h, y;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    gu = project_all(x, *w.rows, w.in);
+    h = swiglu_rows(gu, w.rows->first[0], w.rows->first[1], w.in[0].size(0));
+    y = project(h, w.out);
+  }
+  if (recorded(x, w)) {
+    auto fn = block_formula<MlpBlockBackward>(x, w);
+    fn->save(fn->GU, gu), fn->save(fn->H, h);
+    set_history(y, fn);
+  }
+  return y;
+}
+
+// A borrowed look at a module: its attributes without going through Python's attribute lookup.
+struct ModuleView {
+  PyObject* module;
+  PyObject* dict;
+  explicit ModuleView(PyObject* m) : module(m) {
+    PyObject** p = m ? _PyObject_GetDictPtr(m) : nullptr;
+    dict = p ? *p : nullptr;
+  }
+  PyObject* item(const char* name) const { return dict ? PyDict_GetItemString(dict, name) : nullptr; }
+  PyObject* in(const char* table, const char* name) const {
+    PyObject* t = item(table);
+    return t && PyDict_Check(t) ? PyDict_GetItemString(t, name) : nullptr;
+  }
+  // exactly of this class, and nothing hangs on its call
+  bool stock(const pybind11::handle& type) const {
+    if (!dict || reinterpret_cast<PyObject*>(Py_TYPE(module)) != type.ptr() || item("forward")) return false;
+    for (const char* hooks : {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"}) {
+      PyObject* h = item(hooks);
+      if (!h || !PyDict_Check(h) || PyDict_Size(h) != 0) return false;
+    }
+    return true;
+  }
+  Tensor tensor(const char* table, const char* name) const {
+    PyObject* t = in(table, name);
+    return t && THPVariable_CheckExact(t) ? THPVariable_Unpack(t) : t && THPVariable_Check(t) ? THPVariable_Unpack(t) : Tensor();
+  }
+  bool flag(const char* name) const {  // on the instance or its class
+    PyObject* v = item(name);
+    if (v) return PyObject_IsTrue(v) == 1;
+    v = PyObject_GetAttrString(reinterpret_cast<PyObject*>(Py_TYPE(module)), name);
+    if (!v) PyErr_Clear();
+    const bool on = v && PyObject_IsTrue(v) == 1;
+    Py_XDECREF(v);
+    return on;
+  }
+  int64_t integer(const char* name) const {
+    PyObject* v = item(name);
+    return v && PyLong_Check(v) ? PyLong_AsLongLong(v) : 0;
+  }
+};
+
+// The rows of `params` (see Adjacent), kept on the module until a parameter or gradient moves
+AdjacentPtr rows_of_module(const ModuleView& m, const std::vector<Tensor>& params) {
+  static const char* const kept = "_maltos_hip_fused_rows";
+  if (PyObject* r = m.item(kept); r && r != Py_None) {
+    AdjacentPtr rows = pybind11::cast<AdjacentPtr>(pybind11::handle(r));
+    if (rows->made_for(params)) return rows;
+  }
+  auto rows = std::make_shared<Adjacent>(params);
+  PyDict_SetItemString(m.dict, kept, pybind11::cast(rows).ptr());
+  return rows;
+}
+
+struct LayerParts {
+  BlockWeights attention, mlp;
+  Tensor norm1, norm2, cos, sin;
+  double eps1 = 0, eps2 = 0;
+  bool into_norm1 = false, into_norm2 = false;
+  int64_t heads = 0, kv_heads = 0;
+};
+
+// types: the classes of the stock modules; backends: the attention backend names that route to the kernels here
+bool read_layer(PyObject* layer, const pybind11::dict& types, const pybind11::handle& backends, const Tensor& x, LayerParts& out) {
+  auto child = [](const ModuleView& m, const char* name) { return ModuleView(m.in("_modules", name)); };
+  auto type = [&](const char* name) { return pybind11::handle(PyDict_GetItemString(types.ptr(), name)); };
+  const ModuleView l(layer);
+  if (!l.stock(type("layer"))) return false;
+  const ModuleView attn = child(l, "self_attn"), mlp = child(l, "mlp"), n1 = child(l, "input_layernorm"), n2 = child(l, "post_attention_layernorm");
+  if (!attn.stock(type("attention")) || !mlp.stock(type("mlp")) || !n1.stock(type("norm")) || !n2.stock(type("norm"))) return false;
+  const ModuleView core = child(attn, "attn_core"), rotary = child(attn, "rotary_emb");
+  if (!core.stock(type("core")) || !rotary.stock(type("rotary"))) return false;
+  PyObject* backend = core.item("attention_backend");
+  if (!backend || PySequence_Contains(backends.ptr(), backend) != 1) return false;
+  if (!attn.flag("fuse_projections") || !attn.flag("fuse_rope_attention") || !mlp.flag("fuse_projections")) return false;
+
+  auto fits = [&](const Tensor& t, int64_t dims) {
+    return t.defined() && t.dim() == dims && t.is_cuda() && t.scalar_type() == x.scalar_type() && t.is_contiguous() && t.device() == x.device();
+  };
+  auto block = [&](const ModuleView& m, std::initializer_list<const char*> ins, const char* last, BlockWeights& w) {
+    w.into_grad_in = true;
+    for (const char* name : ins) {
+      const ModuleView p = child(m, name);
+      w.in.push_back(p.stock(type("linear")) && p.in("_parameters", "bias") == Py_None ? p.tensor("_parameters", "weight") : Tensor());
+      if (!fits(w.in.back(), 2)) return false;
+      w.into_grad_in = w.into_grad_in && p.flag("accumulate_into_grad");
+    }
+    const ModuleView p = child(m, last);
+    w.out = p.stock(type("linear")) && p.in("_parameters", "bias") == Py_None ? p.tensor("_parameters", "weight") : Tensor();
+    w.into_grad_out = p.dict && p.flag("accumulate_into_grad");
+    if (!fits(w.out, 2) || w.in[0].size(1) != x.size(-1)) return false;
+    w.rows = rows_of_module(m, w.in);
+    return w.rows->weight.defined() || runs_as_group(*w.rows, x, w.in);
+  };
+  if (!block(attn, {"q_proj", "k_proj", "v_proj"}, "o_proj", out.attention) || !block(mlp, {"gate_proj", "up_proj"}, "down_proj", out.mlp)) return false;
+  const auto &a = out.attention, &m = out.mlp;
+  out.heads = attn.integer("num_heads"), out.kv_heads = attn.integer("num_kv_heads");
+  const int64_t dim = attn.integer("head_dim");
+  if (out.heads <= 0 || out.kv_heads <= 0 || dim <= 0 || dim > 192 || a.in[0].size(0) != out.heads * dim || a.in[1].size(0) != out.kv_heads * dim ||
+      a.in[2].size(0) != out.kv_heads * dim || a.out.size(1) != out.heads * dim || a.out.size(0) != x.size(-1))
+    return false;
+  if (m.in[0].size(0) != m.in[1].size(0) || m.out.size(1) != m.in[0].size(0) || m.out.size(0) != x.size(-1) ||
+      m.in[0].size(0) % (16 / x.element_size()) != 0)
+    return false;
+  out.cos = rotary.tensor("_buffers", "cos"), out.sin = rotary.tensor("_buffers", "sin");
+  out.norm1 = n1.tensor("_parameters", "weight"), out.norm2 = n2.tensor("_parameters", "weight");
+  PyObject *e1 = n1.item("eps"), *e2 = n2.item("eps");
+  if (!fits(out.cos, 2) || !fits(out.sin, 2) || !fits(out.norm1, 1) || !fits(out.norm2, 1) || !e1 || !e2 || !PyFloat_Check(e1) || !PyFloat_Check(e2))
+    return false;
+  out.eps1 = PyFloat_AsDouble(e1), out.eps2 = PyFloat_AsDouble(e2);
+  out.into_norm1 = n1.flag("accumulate_into_grad"), out.into_norm2 = n2.flag("accumulate_into_grad");
+  return true;
+}
+
+// (x, pending) after all layers of a ModuleList's table, the last residual add left to whoever normalises next; None where a
+// layer is not made of stock modules, something hooks into one, or its projections run one by one
+pybind11::object run_layers(const pybind11::dict& layers, const pybind11::dict& types, const pybind11::object& backends, const Tensor& x_in,
+                            int64_t position_offset, const OptTensor& rope_positions, const OptTensor& positions, const OptTensor& sequences) {
+  if (!x_in.is_cuda() || x_in.dim() != 3 || !x_in.is_contiguous() || x_in.numel() == 0 || at::isTensorSubclassLike(x_in) ||
+      (x_in.scalar_type() != at::kBFloat16 && x_in.scalar_type() != at::kFloat) || c10::impl::dispatch_mode_enabled() ||
+      at::autocast::is_autocast_enabled(at::kCUDA))
+    return pybind11::none();
+  std::vector<LayerParts> parts(PyDict_Size(layers.ptr()));
+  size_t count = 0;
+  for (auto item : layers)
+    if (!read_layer(item.second.ptr(), types, backends, x_in, parts[count++])) return pybind11::none();
+  const Positions where{position_offset, rope_positions, positions, sequences};
+  Tensor x = x_in, pending;
+  {
+    pybind11::gil_scoped_release no_gil;
+    for (const LayerParts& l : parts) {
+      Tensor normed;
+      if (pending.defined()) std::tie(x, normed) = add_rms_norm(x, pending, l.norm1, l.eps1, l.into_norm1);
+      else normed = rms_norm(x, l.norm1, l.eps1, l.into_norm1);
+      const Tensor attn = attention_block(normed, l.attention, l.heads, l.kv_heads, l.cos, l.sin, where);
+      std::tie(x, normed) = add_rms_norm(x, attn, l.norm2, l.eps2, l.into_norm2);
+      pending = mlp_block(normed, l.mlp);
+    }
+  }
+  return pybind11::make_tuple(x, pending);
+}
+
 }  // namespace
 
 void bind_llama(pybind11::module& m) {
   using torch::wrap_pybind_function;
   namespace py = pybind11;
+  m.def("run_layers", wrap_pybind_function(run_layers));
   m.def("linear", wrap_pybind_function(linear));
   m.def("embedding", wrap_pybind_function(embedding));
   m.def("product", wrap_pybind_function([](int form, const Tensor& a, const Tensor& b, const OptTensor& out, bool accumulate) {
@@ -576,6 +859,8 @@ void bind_llama(pybind11::module& m) {
         }));
   py::class_<Adjacent, AdjacentPtr>(m, "Adjacent")
       .def(py::init<const std::vector<Tensor>&>())
+      // (kept on modules, which are copied and pickled: a copy makes its own)
+      .def("__reduce__", [](const Adjacent&) { return py::make_tuple(py::type::of(py::none()), py::tuple()); })
       .def("made_for", &Adjacent::made_for)
       .def("runs_as_group", &runs_as_group)
       .def_property_readonly("adjacent", [](const Adjacent& a) { return a.weight.defined(); })

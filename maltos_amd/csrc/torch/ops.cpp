@@ -996,13 +996,6 @@ std::tuple<Tensor, Tensor, Tensor> py_attention_backward(const Tensor& dout, con
   at::AutoDispatchBelowADInplaceOrView below_autograd;
   return attention_backward(dout, q, k, v, o, lse, mask_mode, resolve_scale(scale, q), q_pos, k_pos, q_seq, k_seq);
 }
-Tensor py_rms_norm(const Tensor& x, const Tensor& w, double eps, bool into_grad) {
-  return std::get<0>(into_grad && at::GradMode::is_enabled() ? rmsnorm_recorded(x, w, eps, true) : op::rmsnorm_fwd().call(x, w, eps));
-}
-std::tuple<Tensor, Tensor> py_add_rms_norm(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad) {
-  auto [h, y, rstd] = into_grad && at::GradMode::is_enabled() ? add_rmsnorm_recorded(x, res, w, eps, true) : op::add_rmsnorm_fwd().call(x, res, w, eps);
-  return {h, y};
-}
 Tensor py_rope(const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& positions, int64_t offset) {
   return op::rope().call(x, cos, sin, positions, offset, false);
 }
@@ -1035,6 +1028,14 @@ size_t doc_plan_cache_size() {
 
 }  // namespace
 
+Tensor rms_norm(const Tensor& x, const Tensor& w, double eps, bool into_grad) {
+  return std::get<0>(into_grad && at::GradMode::is_enabled() ? rmsnorm_recorded(x, w, eps, true) : op::rmsnorm_fwd().call(x, w, eps));
+}
+std::tuple<Tensor, Tensor> add_rms_norm(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad) {
+  auto [h, y, rstd] = into_grad && at::GradMode::is_enabled() ? add_rmsnorm_recorded(x, res, w, eps, true) : op::add_rmsnorm_fwd().call(x, res, w, eps);
+  return {h, y};
+}
+
 void bind_ops(pybind11::module& m) {
   using torch::wrap_pybind_function;
   m.def("attention", wrap_pybind_function(py_attention));
@@ -1044,8 +1045,8 @@ void bind_ops(pybind11::module& m) {
   m.def("attention_backward_ring_block", wrap_pybind_function(attention_backward_ring_block));
   m.def("attention_merge_", wrap_pybind_function(attention_merge_));
   namespace py = pybind11;
-  m.def("rms_norm", wrap_pybind_function(py_rms_norm), py::arg("x"), py::arg("w"), py::arg("eps"), py::arg("into_grad") = false);
-  m.def("add_rms_norm", wrap_pybind_function(py_add_rms_norm), py::arg("x"), py::arg("res"), py::arg("w"), py::arg("eps"), py::arg("into_grad") = false);
+  m.def("rms_norm", wrap_pybind_function(rms_norm), py::arg("x"), py::arg("w"), py::arg("eps"), py::arg("into_grad") = false);
+  m.def("add_rms_norm", wrap_pybind_function(add_rms_norm), py::arg("x"), py::arg("res"), py::arg("w"), py::arg("eps"), py::arg("into_grad") = false);
   m.def("rope", wrap_pybind_function(py_rope));
   m.def("rope_pair", wrap_pybind_function(py_rope_pair));
   m.def("rope_pair_", wrap_pybind_function(rope_pair_));

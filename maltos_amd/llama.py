@@ -16,7 +16,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
-from .attention_backend import AttentionBackend, causal_attention, hip_fallback_reason, uses_hip_kernels, validate_attention_backend
+from .attention_backend import _HIP_BACKENDS, AttentionBackend, causal_attention, hip_fallback_reason, uses_hip_kernels, validate_attention_backend
 from .attn_masking_utils import canonical_position_ids, canonical_sequence_ids
 from .constants import (HIDDEN_STATES_KEY, INPUT_IDS_KEY, LABELS_KEY, LOSS_WEIGHT_KEY, POSITION_IDS_KEY,
                         POSITION_OFFSET_KEY, SEQUENCE_IDS_KEY)
@@ -181,6 +181,11 @@ class LlamaRotaryEmbedding(nn.Module):
         return self.cos, self.sin
 
 
+def _one_document(positions: torch.Tensor) -> torch.Tensor:
+    """Sequence ids of rows that come with positions only: one document per row."""
+    return ops.derived_from(positions, "_maltos_hip_zero_ids", lambda pos: torch.zeros(pos.shape, dtype=torch.int32, device=pos.device))
+
+
 class HipAttentionCore(nn.Module):
     """`attn_core` of LlamaAttention: (q, k, v, position_offset, position_ids, sequence_ids) -> out."""
 
@@ -253,9 +258,8 @@ class LlamaAttention(nn.Module):
         if (self.fuse_rope_attention and type(core) is HipAttentionCore and uses_hip_kernels(core.attention_backend)
                 and hip_fallback_reason(q) is None):
             positions, sequences = core.row_ids(q, position_offset, position_ids, sequence_ids)
-            if positions is not None and sequences is None:   # positions only: one document per row
-                sequences = ops.derived_from(positions, "_maltos_hip_zero_ids",
-                                             lambda pos: torch.zeros(pos.shape, dtype=torch.int32, device=pos.device))
+            if positions is not None and sequences is None:
+                sequences = _one_document(positions)
             if rope_pos is not None:
                 rope_pos = ops._ids32(rope_pos, batch, seq_len, "position_ids")
             vo = native().rope_attention(q, k, v, cos, sin, rope_pos, int(position_offset), positions, sequences)
@@ -315,6 +319,11 @@ class LlamaDecoderLayer(nn.Module):
         return x, self.mlp(normed)
 
 
+# what native().run_layers takes a layer apart into
+_STOCK_MODULES = {"layer": LlamaDecoderLayer, "attention": LlamaAttention, "core": HipAttentionCore, "rotary": LlamaRotaryEmbedding,
+                  "mlp": LlamaMLP, "norm": LlamaRMSNorm, "linear": HipLinear}
+
+
 class LlamaForCausalLM(nn.Module):
     def __init__(self, config: LlamaConfig) -> None:
         super().__init__()
@@ -358,10 +367,14 @@ class LlamaForCausalLM(nn.Module):
                                                   position_offset=position_offset, device=x.device)
             sequence_ids = canonical_sequence_ids(sequence_ids, batch_size=x.size(0), seq_len=x.size(1), device=x.device)
         if self.config.fuse_residual_norm and x.is_cuda and len(self.layers) > 0:
-            pending = None
-            for layer in self.layers:
-                x, pending = layer(x, position_offset=position_offset, position_ids=position_ids, sequence_ids=sequence_ids,
-                                   pending=pending, defer_residual=True)
+            done = self._layers_at_once(x, position_offset, position_ids, sequence_ids)
+            if done is not None:
+                x, pending = done
+            else:
+                pending = None
+                for layer in self.layers:
+                    x, pending = layer(x, position_offset=position_offset, position_ids=position_ids, sequence_ids=sequence_ids,
+                                       pending=pending, defer_residual=True)
             _, normed = _add_norm(self.norm, x, pending)
         else:
             for layer in self.layers:
@@ -376,6 +389,17 @@ class LlamaForCausalLM(nn.Module):
         own = self.config.loss_overwrites_logits and not self.lm_head._forward_hooks
         loss = causal_cross_entropy(logits, labels, overwrite_logits=own and logits.is_cuda and logits.is_contiguous())
         return loss if loss_weight is None else loss * float(loss_weight)
+
+    def _layers_at_once(self, x, position_offset, position_ids, sequence_ids):
+        """(x, pending) after all layers without leaving C++, or None: only layers of the modules above, as they are and with
+        nothing hooked into them, can be run that way."""
+        if type(self.layers) is not nn.ModuleList or x.dim() != 3 or torch.nn.modules.module._has_any_global_hook():
+            return None
+        rope_pos = sequences = None
+        if position_ids is not None:
+            rope_pos = ops._ids32(position_ids, x.size(0), x.size(1), "position_ids")
+            sequences = sequence_ids if sequence_ids is not None else _one_document(position_ids)
+        return native().run_layers(self.layers._modules, _STOCK_MODULES, _HIP_BACKENDS, x, int(position_offset), rope_pos, position_ids, sequences)
 
     def context_parallel_spec(self) -> list[str]:
         """Module paths whose `attn_core` a context-parallel plugin swaps (reference :311-314)."""

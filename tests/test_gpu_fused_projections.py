@@ -131,3 +131,32 @@ def test_rope_pair_in_place_equals_the_copying_form(dev):
             ops.rope_pair_(mine[:, :4], mine[:, 4:6], cos, sin, positions=positions, position_offset=3, inverse=inverse)
             assert torch.equal(mine[:, :4], want[0]) and torch.equal(mine[:, 4:6], want[1])
             assert torch.equal(mine[:, 6:], untouched)
+
+
+@pytest.mark.parametrize("dtype,flat,packed", [(torch.bfloat16, True, False), (torch.bfloat16, False, True), (torch.float32, False, False)])
+def test_layers_at_once_equal_the_modules_one_by_one(dev, dtype, flat, packed):
+    """The layers in one call (stock modules, no hooks) against the same model called module by module (a hook on one layer)."""
+    import copy
+    cfg = LlamaConfig(vocab_size=512, hidden_size=256, intermediate_size=688, num_hidden_layers=2, num_attention_heads=4,
+                      num_key_value_heads=2, max_position_embeddings=128, rms_norm_eps=1e-5)
+    torch.manual_seed(5)
+    at_once = LlamaForCausalLM(cfg).to(dev).to(dtype)
+    one_by_one = copy.deepcopy(at_once)
+    calls = []
+    one_by_one.layers[1].register_forward_hook(lambda *a: calls.append(1))
+    if flat:
+        for m in (at_once, one_by_one):
+            m.opt = MasterWeightsOptimizer(m.parameters(), optimizer_factory=lambda ps: FusedAdamW(ps, lr=1e-3), flat=True)
+            set_grad_accumulation_into_buffers(m)
+    ids = torch.randint(0, 512, (2, 101), generator=torch.Generator().manual_seed(1)).to(dev)
+    batch = {"input_ids": ids, "labels": ids.clone()}
+    if packed:
+        batch["position_ids"] = (torch.arange(101, device=dev) % 40).expand(2, 101).contiguous()
+        batch["sequence_ids"] = (torch.arange(101, device=dev) // 40).expand(2, 101).contiguous()
+    for m in (at_once, one_by_one):
+        m(batch).backward()
+    assert len(calls) == 1 and at_once(batch).equal(one_by_one(batch))
+    for (name, p), q in zip(at_once.named_parameters(), one_by_one.named_parameters()):
+        assert torch.equal(p.grad, q[1].grad), name
+    if not flat:   # what the modules keep does not stand in the way of a copy
+        assert copy.deepcopy(at_once)(batch).equal(at_once(batch))
