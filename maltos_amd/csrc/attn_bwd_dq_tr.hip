@@ -1,6 +1,6 @@
 // Attention backward, dQ, head_dim 64 and 128, bf16: the version of attn_bwd_dq.hip with one LDS copy per tile.
 //
-// Same decomposition (a workgroup of 8 wavefronts owns 256 query rows of one (batch, head), each wavefront 32 of
+// Same decomposition (a workgroup of 8, or 4, wavefronts owns 256, or 128, query rows of one (batch, head), each wavefront 32 of
 // them, Q and dO stay in registers, it walks the visible keys in tiles of 64 and recomputes the scores transposed so
 // that a lane owns one query and LSE / delta are per-lane scalars):
 //     S^T  = K Q^T             A = K rows (LDS)              B = Q  (registers)
@@ -16,13 +16,12 @@
 namespace {
 
 constexpr int BN = 64;
-constexpr int WAVES = 8;
-constexpr int THREADS = WAVES * 64;
-constexpr int BM = WAVES * 32;
 constexpr int STAGES = 2;
 
-template <int D>
+template <int D, int WAVES>
 struct DqCfg {
+  static constexpr int THREADS = WAVES * 64;
+  static constexpr int BM = WAVES * 32;
   static constexpr int KS = D / 16;
   static constexpr int DB = D / 32;
   static constexpr int RB = D * 2;                     // bytes per tile row
@@ -34,7 +33,7 @@ struct DqCfg {
   static constexpr int META_OFF = DELTA_OFF + BM * 4;  // document masks: per stage k_pos[64] then k_seq[64], int32
   static constexpr int META_BYTES = 2 * BN * 4;
   static constexpr int LDS_BYTES = META_OFF + STAGES * META_BYTES;
-  static constexpr int NLD = BN * CPR / THREADS;       // 16-byte chunks per thread and tile (2 or 1)
+  static constexpr int NLD = BN * CPR / THREADS;       // 16-byte chunks per thread and tile (4, 2 or 1)
 };
 
 typedef int v4i32 __attribute__((ext_vector_type(4)));
@@ -96,9 +95,10 @@ __device__ __forceinline__ bf16x8 as_frag(v2i32 lo, v2i32 hi) {
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3));
 }
 
-template <int D, int MODE>
-__global__ __launch_bounds__(THREADS) void attn_bwd_dq_tr_kernel(const AttnBwdParams bp) {
-  using C = DqCfg<D>;
+template <int D, int MODE, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 2) void attn_bwd_dq_tr_kernel(const AttnBwdParams bp) {
+  using C = DqCfg<D, WAVES>;
+  constexpr int THREADS = C::THREADS, BM = C::BM, BM_SHIFT = WAVES == 8 ? 8 : 7;
   constexpr int KS = C::KS, DB = C::DB, RB = C::RB, CPR = C::CPR, TILE_BYTES = C::TILE_BYTES, STAGE_BYTES = C::STAGE_BYTES,
                 NLD = C::NLD;
   const AttnParams& p = bp.a;
@@ -124,13 +124,13 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_tr_kernel(const AttnBwdPa
     }
   }
   const int hq0 = (bh % hgroups) << pack_shift;  // first head of the workgroup
-  const int hq = MODE == MLTS_MASK_DOC ? hq0 + __builtin_amdgcn_readfirstlane((wave * 32) >> (8 - pack_shift)) : hq0;
+  const int hq = MODE == MLTS_MASK_DOC ? hq0 + __builtin_amdgcn_readfirstlane((wave * 32) >> (BM_SHIFT - pack_shift)) : hq0;
   const int hkv = hq0 / (p.Hq / p.Hkv);
   const int q0 = qt * rows_per_head;
   const int wq0 = MODE == MLTS_MASK_DOC ? q0 + ((wave * 32) & (rows_per_head - 1)) : q0 + wave * 32;
   const int qrow = wq0 + l32;
 
-  // (workgroup tile row -> head hq0 + (row >> (8 - pack_shift)), query q0 + (row & (rows_per_head - 1)))
+  // (workgroup tile row -> head hq0 + (row >> (BM_SHIFT - pack_shift)), query q0 + (row & (rows_per_head - 1)))
   const bf16_t* Q = static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq0 * p.qs[1];
   const bf16_t* dO = static_cast<const bf16_t*>(bp.dout) + b * bp.dos[0] + hq0 * bp.dos[1];
   const bf16_t* K = static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_tr_kernel(const AttnBwdPa
     const int c = tid + n * THREADS;
     const int row = c / CPR;
     const int col = ((c % CPR) ^ swz<D>(row & 15)) * 8;
-    const int hrow = MODE == MLTS_MASK_DOC ? row >> (8 - pack_shift) : 0;
+    const int hrow = MODE == MLTS_MASK_DOC ? row >> (BM_SHIFT - pack_shift) : 0;
     const int64_t r = min(q0 + (MODE == MLTS_MASK_DOC ? row & (rows_per_head - 1) : row), p.Sq - 1);
     pro_q[n] = *reinterpret_cast<const v4i32*>(Q + hrow * p.qs[1] + r * p.qs[2] + col);
     pro_d[n] = *reinterpret_cast<const v4i32*>(dO + hrow * bp.dos[1] + r * bp.dos[2] + col);
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_tr_kernel(const AttnBwdPa
       const int c = tid + n * THREADS;
       const int row = c / CPR;
       const int col = ((c % CPR) ^ swz<D>(row & 15)) * 8;
-      const int hrow = MODE == MLTS_MASK_DOC ? row >> (8 - pack_shift) : 0;
+      const int hrow = MODE == MLTS_MASK_DOC ? row >> (BM_SHIFT - pack_shift) : 0;
       const int64_t r = min(q0 + (MODE == MLTS_MASK_DOC ? row & (rows_per_head - 1) : row), p.Sq - 1);
       pro_o[n] = *reinterpret_cast<const v4i32*>(O + hrow * p.os[1] + r * p.os[2] + col);
     }
@@ -266,9 +266,15 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_tr_kernel(const AttnBwdPa
     const uint32_t a = lds0 + stage * STAGE_BYTES + tid * 16;
     lds_write_b128<0>(a, stg_k[0]);
     lds_write_b128<TILE_BYTES>(a, stg_v[0]);
-    if (NLD == 2) {
-      lds_write_b128<THREADS * 16>(a, stg_k[NLD - 1]);
-      lds_write_b128<TILE_BYTES + THREADS * 16>(a, stg_v[NLD - 1]);
+    if constexpr (NLD >= 2) {
+      lds_write_b128<THREADS * 16>(a, stg_k[1]);
+      lds_write_b128<TILE_BYTES + THREADS * 16>(a, stg_v[1]);
+    }
+    if constexpr (NLD == 4) {
+      lds_write_b128<2 * THREADS * 16>(a, stg_k[2]);
+      lds_write_b128<TILE_BYTES + 2 * THREADS * 16>(a, stg_v[2]);
+      lds_write_b128<3 * THREADS * 16>(a, stg_k[3]);
+      lds_write_b128<TILE_BYTES + 3 * THREADS * 16>(a, stg_v[3]);
     }
   };
 
@@ -575,31 +581,42 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_tr_kernel(const AttnBwdPa
   }
 }
 
-template <int D, int MODE>
+template <int D, int MODE, int WAVES>
 int launch(AttnBwdParams bp, hipStream_t st) {
-  auto kern = attn_bwd_dq_tr_kernel<D, MODE>;
-  constexpr int lds_bytes = DqCfg<D>::LDS_BYTES;
+  auto kern = attn_bwd_dq_tr_kernel<D, MODE, WAVES>;
+  constexpr int lds_bytes = DqCfg<D, WAVES>::LDS_BYTES;
   static MltsLdsOptIn lds_opt_in;
   if (hipError_t e = lds_opt_in.reserve(reinterpret_cast<const void*>(kern), lds_bytes); e != hipSuccess) {
     mlts_set_error("mlts_attn_bwd: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     return MLTS_ERR_LAUNCH;
   }
-  if (MODE != MLTS_MASK_DOC) bp.a.head_pack_shift = 0;  // (set with the block order by the caller's pre-pass otherwise)
-  const int rows = BM >> bp.a.head_pack_shift;
+  const int rows = (WAVES * 32) >> bp.a.head_pack_shift;
   bp.a.nqt = (bp.a.Sq + rows - 1) / rows;
   const int64_t blocks = static_cast<int64_t>(bp.a.nqt) * bp.a.B * (bp.a.Hq >> bp.a.head_pack_shift);
   if (blocks > 0) {
     MltsKernelTimer timer("attn_bwd_dq", st);
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), lds_bytes, st, bp);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(WAVES * 64), lds_bytes, st, bp);
   }
   return mlts_check_launch("mlts_attn_bwd");
 }
 
+template <int D, int MODE>
+int launch_size(AttnBwdParams bp, hipStream_t st) {
+  if (MODE != MLTS_MASK_DOC) bp.a.head_pack_shift = 0;  // (set with the block order by the caller's pre-pass otherwise)
+  // Few workgroups: 128 rows each instead of 256 (same bits; us before / after: 8 heads x 1023 packed 22.9 / 19.5, 24 x 777
+  // causal 20.9 / 18.5, 8 x 200 10.9 / 9.6, 8 x 4096 82.3 / 72.4).  Not at head_dim 128, where twice the staging registers
+  // per thread spill: 8 x 1024 39.6 / 48.9.
+  if constexpr (D == 64) {
+    if (mlts_attn_halved_workgroups(bp.a)) return launch<D, MODE, 4>(bp, st);
+  }
+  return launch<D, MODE, 8>(bp, st);
+}
+
 template <int D>
 int launch_mode(const AttnBwdParams& bp, int mode, hipStream_t st) {
-  if (mode == MLTS_MASK_NONE) return launch<D, MLTS_MASK_NONE>(bp, st);
-  if (mode == MLTS_MASK_CAUSAL) return launch<D, MLTS_MASK_CAUSAL>(bp, st);
-  return launch<D, MLTS_MASK_DOC>(bp, st);
+  if (mode == MLTS_MASK_NONE) return launch_size<D, MLTS_MASK_NONE>(bp, st);
+  if (mode == MLTS_MASK_CAUSAL) return launch_size<D, MLTS_MASK_CAUSAL>(bp, st);
+  return launch_size<D, MLTS_MASK_DOC>(bp, st);
 }
 
 }  // namespace

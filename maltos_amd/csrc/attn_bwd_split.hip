@@ -1,9 +1,9 @@
 // Attention backward, dK and dV, head_dim 64 and 128, bf16: two-role workgroup.
 //
-// A workgroup owns 128 keys of one (batch, kv head) and walks the 64-row query tiles that can see them (all
-// query heads of the GQA group); its EIGHT wavefronts come in two roles per 32-key block kb = wave % 4:
-//     role 0 (wave < 4):   S = Q K^T,  P = exp2(S c - lse2)  ->  dV += P^T dO      and hands P (bf16) over in LDS
-//     role 1 (wave >= 4):  delta - dO V^T,  -dS = P (delta - dO V^T)  ->  -dK += (-dS)^T Q     one tile behind
+// A workgroup owns 128 keys (small grids: 64) of one (batch, kv head) and walks the 64-row query tiles that can see them
+// (all query heads of the GQA group); its EIGHT (four) wavefronts come in two roles per 32-key block kb = wave % KB:
+//     role 0 (wave < KB):   S = Q K^T,  P = exp2(S c - lse2)  ->  dV += P^T dO      and hands P (bf16) over in LDS
+//     role 1 (wave >= KB): delta - dO V^T,  -dS = P (delta - dO V^T)  ->  -dK += (-dS)^T Q     one tile behind
 //                          (per barrier interval: dS of tile k-1, dP of tile k, then the dK products of tile k-1)
 // Each role keeps one operand (K or -V) and one accumulator (dV or dK) in registers, so a wavefront fits in
 // 256 registers, two wavefronts share a SIMD, the matrix instructions take plain VGPR accumulators (no AGPR
@@ -21,15 +21,15 @@
 
 namespace {
 
-constexpr int BKV = 128;
 constexpr int BQ = 64;
-constexpr int WAVES = 8;
-constexpr int THREADS = WAVES * 64;
 constexpr int STAGES = 3;
-constexpr int PBUF_BYTES = 4 * 64 * 16;  // P hand-over: [2 buffers][4 key blocks][4 fragments][64 lanes] x 16 B
+constexpr int PBUF_BYTES = 4 * 64 * 16;  // P hand-over: [2 buffers][KB key blocks][4 fragments][64 lanes] x 16 B
 
-template <int D>
+// KB: 32-key blocks per workgroup, each with its two wavefronts
+template <int D, int KB>
 struct SplitCfg {
+  static constexpr int BKV = KB * 32;
+  static constexpr int THREADS = KB * 128;
   static constexpr int KS = D / 16;                  // k-steps of the S / dP products
   static constexpr int DB = D / 32;                  // 32-column blocks of dV / dK
   static constexpr int RB = D * 2;                   // bytes per tile row
@@ -38,8 +38,8 @@ struct SplitCfg {
   static constexpr int STAT_OFF = 2 * TILE_BYTES;    // lse2[64], delta[64] (fp32); the rest of the stage's last KiB is unused
   static constexpr int STAGE_BYTES = STAT_OFF + 4 * BQ * 4;
   static constexpr int PBUF_OFF = STAGES * STAGE_BYTES;
-  static constexpr int LDS_BYTES = PBUF_OFF + 2 * 4 * PBUF_BYTES;
-  static constexpr int NLD = BQ * CPR / THREADS;     // 16-byte chunks per thread and tile (2 or 1)
+  static constexpr int LDS_BYTES = PBUF_OFF + 2 * KB * PBUF_BYTES;
+  static constexpr int NLD = BQ * CPR / THREADS;     // 16-byte chunks per thread and tile (4, 2 or 1)
 };
 
 typedef int v4i32 __attribute__((ext_vector_type(4)));
@@ -114,16 +114,17 @@ __global__ __launch_bounds__(256) void lse2_kernel(const float* __restrict__ lse
   }
 }
 
-template <int D, int MODE>
-__global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const AttnBwdParams bp, const float* __restrict__ lse2) {
-  using C = SplitCfg<D>;
+template <int D, int MODE, int KB>
+__global__ __launch_bounds__(KB * 128, 2) void attn_bwd_dkdv_split_kernel(const AttnBwdParams bp, const float* __restrict__ lse2) {
+  using C = SplitCfg<D, KB>;
+  constexpr int BKV = C::BKV, THREADS = C::THREADS;
   constexpr int KS = C::KS, DB = C::DB, RB = C::RB, CPR = C::CPR, TILE_BYTES = C::TILE_BYTES, STAT_OFF = C::STAT_OFF,
                 STAGE_BYTES = C::STAGE_BYTES, PBUF_OFF = C::PBUF_OFF, NLD = C::NLD;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5, l16 = lane & 15;
-  const int role = wave >> 2, kb = wave & 3;
+  const int role = wave / KB, kb = wave % KB;
 
   const int nbh = p.B * p.Hkv;
   const int bid = blockIdx.x;
@@ -166,15 +167,16 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const Attn
   }
   const int span = qt_begin < nqt ? nqt - qt_begin : 0;
 
-  int4 kstats[2];
+  constexpr int KT = BKV / 64;  // 64-key tiles
+  int4 kstats[KT];
   if (MODE == MLTS_MASK_DOC) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < KT; ++i) {
       const int t = (kv0 >> 6) + i;
       kstats[i] = t < p.nk_stats ? p.k_stats[static_cast<int64_t>(b) * p.nk_stats + t] : make_int4(0x7fffffff, 0, 0, -2);
     }
   }
-  const int4 wk_stats = MODE == MLTS_MASK_DOC ? ((kb >> 1) ? kstats[1] : kstats[0]) : make_int4(0, 0, 0, 0);
+  const int4 wk_stats = MODE == MLTS_MASK_DOC ? ((kb >> 1) ? kstats[KT - 1] : kstats[0]) : make_int4(0, 0, 0, 0);
   // document masks: the lane's key has one 64-bit word per query tile (bit i = query i of the tile sees the key),
   // formed by a pre-pass for the tiles that classify() calls masked; role 0 fetches it along with the tile
   const unsigned long long* vis_row = nullptr;
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const Attn
   auto first_needed = [&](Pos x) -> Pos {  // x itself or the next position whose tile is needed
     if (MODE != MLTS_MASK_DOC) return x;
     while (!at_end(x)) {
-      const int q = doc_scan_next<2, false>(scan, x.qt, span, span, q_stats_row, kstats, wk_stats, lane);
+      const int q = doc_scan_next<KT, false>(scan, x.qt, span, span, q_stats_row, kstats, wk_stats, lane);
       if (q < span) {
         x.qt = q;
         return x;
@@ -278,9 +280,15 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const Attn
     const uint32_t a = stg_lane + stage * STAGE_BYTES;
     lds_write_b128<0>(a, stg_q[0]);
     lds_write_b128<TILE_BYTES>(a, stg_d[0]);
-    if (NLD == 2) {
-      lds_write_b128<THREADS * 16>(a, stg_q[NLD - 1]);
-      lds_write_b128<TILE_BYTES + THREADS * 16>(a, stg_d[NLD - 1]);
+    if constexpr (NLD >= 2) {
+      lds_write_b128<THREADS * 16>(a, stg_q[1]);
+      lds_write_b128<TILE_BYTES + THREADS * 16>(a, stg_d[1]);
+    }
+    if constexpr (NLD == 4) {
+      lds_write_b128<2 * THREADS * 16>(a, stg_q[2]);
+      lds_write_b128<TILE_BYTES + 2 * THREADS * 16>(a, stg_d[2]);
+      lds_write_b128<3 * THREADS * 16>(a, stg_q[3]);
+      lds_write_b128<TILE_BYTES + 3 * THREADS * 16>(a, stg_d[3]);
     }
     if (tid < 2 * BQ)
       asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(lds0_ + stage * STAGE_BYTES + tid * 4), "v"(stg_s), "n"(STAT_OFF));
@@ -670,14 +678,14 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const Attn
       drain_and_barrier();
       if (!at_end(itn)) stage_load(itn);
       const int q0 = (qt_begin + it.qt) * BQ;
-      const int pbuf = (k & 1) * (4 * PBUF_BYTES);
+      const int pbuf = (k & 1) * (KB * PBUF_BYTES);
       if (ROLE == 0) {
         // one instance of the tile body (with several, the register allocator keeps the accumulators twice); the
         // mask is a branch around VALU work inside it.  Without a mask mode nothing needs masking: keys past Sk are
         // never stored and queries past Sq have lse2 = +inf.
         if (cls != TILE_SKIP) role0_tile(MODE != MLTS_MASK_NONE && cls == TILE_MASKED, q0, stage, pbuf, vis);
       } else {
-        if (prev_active) role1_ds(pbuf ^ (4 * PBUF_BYTES));
+        if (prev_active) role1_ds(pbuf ^ (KB * PBUF_BYTES));
         if (cls != TILE_SKIP) role1_dp(stage);
         if (prev_active) role1_dk(prev_stage);
       }
@@ -690,7 +698,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const Attn
     }
     drain_and_barrier();
     if (ROLE == 1 && prev_active) {
-      role1_ds(((k - 1) & 1) * (4 * PBUF_BYTES));
+      role1_ds(((k - 1) & 1) * (KB * PBUF_BYTES));
       role1_dk(prev_stage);
     }
     last_stage = prev_stage;
@@ -772,28 +780,43 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dkdv_split_kernel(const Attn
   }
 }
 
-template <int D, int MODE>
-int launch(const AttnBwdParams& bp, const float* lse2, hipStream_t st) {
-  auto kern = attn_bwd_dkdv_split_kernel<D, MODE>;
-  constexpr int lds_bytes = SplitCfg<D>::LDS_BYTES;
+template <int D, int MODE, int KB>
+int launch(AttnBwdParams bp, const float* lse2, hipStream_t st) {
+  auto kern = attn_bwd_dkdv_split_kernel<D, MODE, KB>;
+  constexpr int lds_bytes = SplitCfg<D, KB>::LDS_BYTES;
   static MltsLdsOptIn lds_opt_in;
   if (hipError_t e = lds_opt_in.reserve(reinterpret_cast<const void*>(kern), lds_bytes); e != hipSuccess) {
     mlts_set_error("mlts_attn_bwd: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     return MLTS_ERR_LAUNCH;
   }
+  bp.nkt = (bp.a.Sk + KB * 32 - 1) / (KB * 32);
   const int64_t blocks = static_cast<int64_t>(bp.nkt) * bp.a.B * bp.a.Hkv;
   if (blocks > 0) {
     MltsKernelTimer timer("attn_bwd_dkdv", st);
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), lds_bytes, st, bp, lse2);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(KB * 128), lds_bytes, st, bp, lse2);
   }
   return mlts_check_launch("mlts_attn_bwd");
 }
 
+template <int D, int MODE>
+int launch_size(AttnBwdParams bp, const float* lse2, hipStream_t st) {
+  // At most 128 workgroups of 128 keys leave half of the CUs idle: 64 keys each then (same bits; us before / after: 8 heads x
+  // 1023 packed 20.8 / 17.8, 8 x 200 causal 8.5 / 7.5, 4 x 2048 unmasked 42.8 / 33.7, 2 key heads for 8 x 1023 66.6 / 56.1).
+  // Not at head_dim 128, where twice the staging registers per thread spill: 8 x 1024 33.2 / 37.1.
+  if constexpr (D == 64) {
+    if (static_cast<int64_t>((bp.a.Sk + 127) / 128) * bp.a.B * bp.a.Hkv <= 128) {
+      bp.a.kblock_order = nullptr;  // all workgroups run at once (and the order is that of 128-key blocks)
+      return launch<D, MODE, 2>(bp, lse2, st);
+    }
+  }
+  return launch<D, MODE, 4>(bp, lse2, st);
+}
+
 template <int D>
 int launch_mode(const AttnBwdParams& bp, int mode, const float* lse2, hipStream_t st) {
-  if (mode == MLTS_MASK_NONE) return launch<D, MLTS_MASK_NONE>(bp, lse2, st);
-  if (mode == MLTS_MASK_CAUSAL) return launch<D, MLTS_MASK_CAUSAL>(bp, lse2, st);
-  return launch<D, MLTS_MASK_DOC>(bp, lse2, st);
+  if (mode == MLTS_MASK_NONE) return launch_size<D, MLTS_MASK_NONE>(bp, lse2, st);
+  if (mode == MLTS_MASK_CAUSAL) return launch_size<D, MLTS_MASK_CAUSAL>(bp, lse2, st);
+  return launch_size<D, MLTS_MASK_DOC>(bp, lse2, st);
 }
 
 }  // namespace
@@ -804,7 +827,6 @@ int64_t mlts_attn_bwd_dkdv_split_workspace(int64_t B, int64_t Hq, int64_t Sq) { 
 // lse2_ready: the workspace already holds lse2 (written by the dQ kernel that ran before).
 int mlts_attn_bwd_dkdv_bf16_split(AttnBwdParams bp, int D, int mode, void* workspace, bool lse2_ready, hipStream_t st) {
   const AttnParams& p = bp.a;
-  bp.nkt = (p.Sk + BKV - 1) / BKV;
   float* lse2 = static_cast<float*>(workspace);
   const int64_t n = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
   if (!lse2_ready)

@@ -1,6 +1,6 @@
 // Attention forward, head_dim 64 and 128, bf16.
 //
-// S^T = K Q^T, P in registers, O^T = V^T P^T, eight wavefronts x 32 query rows; K and V tiles travel
+// S^T = K Q^T, P in registers, O^T = V^T P^T, eight (small grids: four) wavefronts x 32 query rows; K and V tiles travel
 // global -> LDS with the 16-byte LDS-DMA loads
 // (global_load_lds_dwordx4: no staging registers, no ds_write, no VALU work) into a four-stage ring, so a
 // tile's loads are issued two tiles ahead of its use.  Tiles are stored row major; V^T fragments come from
@@ -16,12 +16,9 @@
 namespace {
 
 constexpr int BN = 64;
-constexpr int WAVES = 8;
-constexpr int THREADS = WAVES * 64;
-constexpr int BM = WAVES * 32;
 constexpr int STAGES = 4;
 
-template <int D>
+template <int D, int WAVES>
 struct FwdCfg {
   static constexpr int KS = D / 16;
   static constexpr int DB = D / 32;
@@ -94,9 +91,10 @@ __device__ __forceinline__ void both_halves(float x, float& lo, float& hi) {
   asm("v_mov_b32 %0, %2\n\tv_mov_b32 %1, %2\n\ts_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "=&v"(lo), "=&v"(hi) : "v"(x));
 }
 
-template <int D, int MODE>
-__global__ __launch_bounds__(THREADS) void attn_fwd_dma_kernel(const AttnParams p) {
-  using C = FwdCfg<D>;
+template <int D, int MODE, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 2) void attn_fwd_dma_kernel(const AttnParams p) {
+  using C = FwdCfg<D, WAVES>;
+  constexpr int BM = WAVES * 32, BM_SHIFT = WAVES == 8 ? 8 : 7;
   constexpr int KS = C::KS, DB = C::DB, RB = C::RB, CPR = C::CPR, TILE_BYTES = C::TILE_BYTES, STAGE_BYTES = C::STAGE_BYTES,
                 PPW = C::PPW, META_OFF = C::META_OFF, META_BYTES = C::META_BYTES;
   // DMA instructions per wavefront and tile; with document masks one more: 16 of the tile's 128 position / sequence ids
@@ -127,7 +125,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_dma_kernel(const AttnParams 
       b = e % p.B;
     }
   }
-  const int hq = ((bh % hgroups) << pack_shift) + ((wave * 32) >> (8 - pack_shift));
+  const int hq = ((bh % hgroups) << pack_shift) + ((wave * 32) >> (BM_SHIFT - pack_shift));
   const int hkv = hq / (p.Hq / p.Hkv);
   const int q0 = qt * rows_per_head;
   const int wq0 = q0 + ((wave * 32) & (rows_per_head - 1));
@@ -246,7 +244,8 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_dma_kernel(const AttnParams 
   // keeps the matrix cores busy.  sync() number k (k = 0, 1, ...) means "the k-th needed tile has landed everywhere";
   // the load of tile k + 2 is issued right behind it into ring stage (k + 2) % 4, which held tile k - 2: the early
   // wavefronts finished it two syncs ago, the late ones read its V before their QK(k - 1), i.e. before this sync.
-  const bool late = wave >= WAVES / 2;
+  // (Four wavefronts have a SIMD each and are all early.)
+  const bool late = WAVES == 8 && wave >= WAVES / 2;
   int inflight = 0, istage = 0;
   int ji = next_tile(scan_load, 0);
   auto issue_next = [&]() {
@@ -578,31 +577,40 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_dma_kernel(const AttnParams 
   }
 }
 
-template <int D, int MODE>
+template <int D, int MODE, int WAVES>
 int launch(AttnParams p, hipStream_t st) {
-  auto kern = attn_fwd_dma_kernel<D, MODE>;
-  constexpr int lds_bytes = FwdCfg<D>::LDS_BYTES;
+  auto kern = attn_fwd_dma_kernel<D, MODE, WAVES>;
+  constexpr int lds_bytes = FwdCfg<D, WAVES>::LDS_BYTES;
   static MltsLdsOptIn lds_opt_in;
   if (hipError_t e = lds_opt_in.reserve(reinterpret_cast<const void*>(kern), lds_bytes); e != hipSuccess) {
     mlts_set_error("mlts_attn_fwd: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     return MLTS_ERR_LAUNCH;
   }
-  if (MODE != MLTS_MASK_DOC) p.head_pack_shift = 0;  // (set with the block order by the caller's pre-pass otherwise)
-  const int rows = BM >> p.head_pack_shift;
+  const int rows = (WAVES * 32) >> p.head_pack_shift;
   p.nqt = (p.Sq + rows - 1) / rows;
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * (p.Hq >> p.head_pack_shift);
   {
     MltsKernelTimer timer("attn_fwd", st);
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), lds_bytes, st, p);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(WAVES * 64), lds_bytes, st, p);
   }
   return mlts_check_launch("mlts_attn_fwd");
 }
 
+template <int D, int MODE>
+int launch_size(AttnParams p, hipStream_t st) {
+  if (MODE != MLTS_MASK_DOC) p.head_pack_shift = 0;  // (set with the block order by the caller's pre-pass otherwise)
+  // At most 128 workgroups of 256 rows leave half of the CUs idle, and the two wavefronts of a SIMD wait for each other's
+  // arithmetic: 128 rows each then (same bits; us before / after: 8 heads x 1023 packed, head_dim 64 23.6 / 19.2; 24 x 777
+  // causal 19.0 / 16.7; 8 x 200 10.8 / 8.3; 8 x 4096 75.6 / 68.4; 8 x 3500 unmasked, head_dim 128 91.8 / 80.2).
+  if (mlts_attn_halved_workgroups(p)) return launch<D, MODE, 4>(p, st);
+  return launch<D, MODE, 8>(p, st);
+}
+
 template <int D>
 int launch_mode(const AttnParams& p, int mode, hipStream_t st) {
-  if (mode == MLTS_MASK_NONE) return launch<D, MLTS_MASK_NONE>(p, st);
-  if (mode == MLTS_MASK_CAUSAL) return launch<D, MLTS_MASK_CAUSAL>(p, st);
-  return launch<D, MLTS_MASK_DOC>(p, st);
+  if (mode == MLTS_MASK_NONE) return launch_size<D, MLTS_MASK_NONE>(p, st);
+  if (mode == MLTS_MASK_CAUSAL) return launch_size<D, MLTS_MASK_CAUSAL>(p, st);
+  return launch_size<D, MLTS_MASK_DOC>(p, st);
 }
 
 }  // namespace

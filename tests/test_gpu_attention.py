@@ -159,6 +159,31 @@ def test_document_mask_long_row_equals_causal_attention_per_document(dev, D):
                 check(got[sl], want, torch.bfloat16, f"{tag} {name} against the oracle")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mode", [ops.MASK_NONE, ops.MASK_CAUSAL, ops.MASK_DOC])
+@pytest.mark.parametrize("Hq,Hkv,Sq,Sk", [(12, 12, 333, 333), (12, 6, 257, 130), (8, 2, 65, 321)])
+def test_small_grids_equal_large_ones(dev, D, mode, Hq, Hkv, Sq, Sk):
+    """Workgroups of half the rows or keys take the calls that would leave half of the CUs idle: every batch row of a call on
+    the other side of that line (more than 128 workgroups of 256 rows, and of 128 keys) has the bits of a call on it alone."""
+    B = 1 + 128 // min(Hkv * ((Sk + 127) // 128), Hq // 4 * ((Sq + 63) // 64))
+    gen = torch.Generator().manual_seed(Hq + Sq)
+    q, k, v, do = (bshd(B, H, S, D, gen, torch.bfloat16).to(dev) for H, S in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk), (Hq, Sq)))
+    k = k.contiguous()  # (another order of strides than the rest)
+    ids = {}
+    if mode == ops.MASK_DOC:
+        (qp, qs), (kp, ks) = (tuple(t.to(dev) for t in make_docs(B, S, gen, 150, pad_tail=5)) for S in (Sq, Sk))
+        ids = dict(q_pos=qp, k_pos=kp, q_seq=qs, k_seq=ks)
+    o, lse = ops.attention_forward(q, k, v, mask_mode=mode, **ids)
+    grads = ops.attention_backward(do, q, k, v, o, lse, mask_mode=mode, **ids)
+    for b in (0, B // 2, B - 1):
+        row = slice(b, b + 1)
+        one = {name: t[row] for name, t in ids.items()}
+        o1, lse1 = ops.attention_forward(q[row], k[row], v[row], mask_mode=mode, **one)
+        assert torch.equal(o[row], o1) and torch.equal(lse[row], lse1), b
+        for got, want, name in zip(grads, ops.attention_backward(do[row], q[row], k[row], v[row], o1, lse1, mask_mode=mode, **one), ("dQ", "dK", "dV")):
+            assert torch.equal(got[row], want), (b, name)
+
+
 @pytest.mark.parametrize("seed", range(10))
 def test_document_mask_drawn_shapes(dev, seed):
     """Drawn batch sizes, head groupings (1, 2, 3, 4, 8 query heads per KV head: the forward and dQ workgroups take one,
