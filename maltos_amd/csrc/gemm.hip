@@ -225,6 +225,22 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
     for (int c = 0; c < CHUNKS; ++c) fetch(f, c);
     k_left -= BK;
   }
+  // What the result is added to, for small tiles: fetched here, behind the first slabs, where the end of the tile would wait for
+  // it (a gradient that was last touched a step ago; dW and dx of a 512-wide layer at 1023 tokens: four launches a layer, 40 us
+  // of a training step of 8 layers).
+  constexpr int LPR = WN / 4, RPP = 64 / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
+  constexpr bool EARLY = MB * NB == 1;
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  t4 old[EARLY ? PASSES : 1];
+  const int c4 = (lane % LPR) * 4, col = n0 + wn + c4;
+  const bool whole = col + 4 <= g.N && (g.ldc & 3) == 0;
+  if (EARLY && g.accumulate && !g.partial && whole && group == 0) {
+#pragma unroll
+    for (int r = 0; r < PASSES; ++r) {
+      const int row = m0 + wm + r * RPP + lane / LPR;
+      if (row < g.M) old[EARLY ? r : 0] = *reinterpret_cast<const t4*>(static_cast<const T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col);
+    }
+  }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) store(0, c, lds);
   next_slab();
@@ -338,9 +354,6 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
           }
   }
   float* stage = reinterpret_cast<float*>(lds) + wave * 32 * ROW;
-  constexpr int LPR = WN / 4;         // lanes per row, four columns each
-  constexpr int RPP = 64 / LPR;       // rows per pass
-  const int c4 = (lane % LPR) * 4, col = n0 + wn + c4;
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
 #pragma unroll
@@ -352,7 +365,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
       }
     // (a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
 #pragma unroll
-    for (int r = 0; r < 32 / RPP; ++r) {
+    for (int r = 0; r < PASSES; ++r) {
       const int rr = r * RPP + lane / LPR, row = m0 + wm + 32 * i + rr;
       f32x4 v = *reinterpret_cast<const f32x4*>(stage + rr * ROW + c4);
       if (row >= g.M || col >= g.N) continue;
@@ -366,12 +379,11 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
         continue;
       }
       T* p = static_cast<T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col;
-      typedef T t4 __attribute__((ext_vector_type(4)));
-      if (col + 4 <= g.N && (g.ldc & 3) == 0) {
+      if (whole) {
         if (g.accumulate) {
-          const t4 old = *reinterpret_cast<const t4*>(p);
+          const t4 before = EARLY ? old[EARLY ? r : 0] : *reinterpret_cast<const t4*>(p);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += to_f32<T>(old[e]);
+          for (int e = 0; e < 4; ++e) v[e] += to_f32<T>(before[e]);
         }
         t4 w;
 #pragma unroll
