@@ -604,10 +604,11 @@ template <int D, int MODE>
 int launch_size(AttnBwdParams bp, hipStream_t st) {
   if (MODE != MLTS_MASK_DOC) bp.a.head_pack_shift = 0;  // (set with the block order by the caller's pre-pass otherwise)
   // Few workgroups: 128 rows each instead of 256 (same bits; us before / after: 8 heads x 1023 packed 22.9 / 19.5, 24 x 777
-  // causal 20.9 / 18.5, 8 x 200 10.9 / 9.6, 8 x 4096 82.3 / 72.4).  Not at head_dim 128, where twice the staging registers
+  // causal 20.9 / 18.5, 8 x 200 10.9 / 9.6, 8 x 4096 82.3 / 72.4), with a mask up to 256 of the large ones (64 x 1024 causal 29.1 /
+  // 26.7, 32 x 2048 49.1 / 45.9), without one up to 128 (64 x 1024 31.4 / 34.1).  Not at head_dim 128, where twice the staging registers
   // per thread spill: 8 x 1024 39.6 / 48.9.
   if constexpr (D == 64) {
-    if (mlts_attn_halved_workgroups(bp.a)) return launch<D, MODE, 4>(bp, st);
+    if (mlts_attn_halved_workgroups(bp.a, MODE == MLTS_MASK_NONE ? 128 : 256)) return launch<D, MODE, 4>(bp, st);
   }
   return launch<D, MODE, 8>(bp, st);
 }

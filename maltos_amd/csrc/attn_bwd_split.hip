@@ -800,11 +800,13 @@ int launch(AttnBwdParams bp, const float* lse2, hipStream_t st) {
 
 template <int D, int MODE>
 int launch_size(AttnBwdParams bp, const float* lse2, hipStream_t st) {
-  // At most 128 workgroups of 128 keys leave half of the CUs idle: 64 keys each then (same bits; us before / after: 8 heads x
-  // 1023 packed 20.8 / 17.8, 8 x 200 causal 8.5 / 7.5, 4 x 2048 unmasked 42.8 / 33.7, 2 key heads for 8 x 1023 66.6 / 56.1).
+  // At most 128 workgroups of 128 keys leave half of the CUs idle; with a mask, whose workgroups differ in length, halves are ahead
+  // up to 256 (unmasked they are not, 32 x 1024 28.2 / 30.0): 64 keys each then (same bits; us before / after: 8 heads x
+  // 1023 packed 20.8 / 17.8, 8 x 200 causal 8.5 / 7.5, 4 x 2048 unmasked 42.8 / 33.7, 2 key heads for 8 x 1023 66.6 / 56.1; 168
+  // workgroups: 24 x 777 causal 21.8 / 18.0; 256: 32 x 1000 packed 23.5 / 22.0).
   // Not at head_dim 128, where twice the staging registers per thread spill: 8 x 1024 33.2 / 37.1.
   if constexpr (D == 64) {
-    if (static_cast<int64_t>((bp.a.Sk + 127) / 128) * bp.a.B * bp.a.Hkv <= 128) {
+    if (static_cast<int64_t>((bp.a.Sk + 127) / 128) * bp.a.B * bp.a.Hkv <= (MODE == MLTS_MASK_NONE ? 128 : 256)) {
       bp.a.kblock_order = nullptr;  // all workgroups run at once (and the order is that of 128-key blocks)
       return launch<D, MODE, 2>(bp, lse2, st);
     }

@@ -145,11 +145,12 @@ inline int mlts_doc_head_pack_shift(int Hq, int Hkv) {
   return group % 4 == 0 ? 2 : group % 2 == 0 ? 1 : 0;
 }
 
-// Forward and dQ: do the workgroups get 128 query rows (four wavefronts) instead of 256 (eight)?  Sets p up for them.
-inline bool mlts_attn_halved_workgroups(AttnParams& p) {
+// Forward and dQ: do the workgroups get 128 query rows (four wavefronts) instead of 256 (eight), because there would be at most
+// `limit` of those?  Sets p up for them.
+inline bool mlts_attn_halved_workgroups(AttnParams& p, int64_t limit) {
   const int rows = 256 >> p.head_pack_shift;
   const int64_t blocks = static_cast<int64_t>((p.Sq + rows - 1) / rows) * p.B * (p.Hq >> p.head_pack_shift);
-  if (blocks > 128) return false;
+  if (blocks > limit) return false;
   // (a wavefront looks at the statistics of 64 rows, so a head keeps at least that many)
   if (p.head_pack_shift > 1) p.head_pack_shift = 1;
   p.qblock_order = nullptr;  // all run at once (and the order is that of the other size's blocks)

@@ -601,8 +601,10 @@ int launch_size(AttnParams p, hipStream_t st) {
   if (MODE != MLTS_MASK_DOC) p.head_pack_shift = 0;  // (set with the block order by the caller's pre-pass otherwise)
   // At most 128 workgroups of 256 rows leave half of the CUs idle, and the two wavefronts of a SIMD wait for each other's
   // arithmetic: 128 rows each then (same bits; us before / after: 8 heads x 1023 packed, head_dim 64 23.6 / 19.2; 24 x 777
-  // causal 19.0 / 16.7; 8 x 200 10.8 / 8.3; 8 x 4096 75.6 / 68.4; 8 x 3500 unmasked, head_dim 128 91.8 / 80.2).
-  if (mlts_attn_halved_workgroups(p)) return launch<D, MODE, 4>(p, st);
+  // causal 19.0 / 16.7; 8 x 200 10.8 / 8.3; 8 x 4096 75.6 / 68.4; 8 x 3500 unmasked, head_dim 128 91.8 / 80.2).  At head_dim 64
+  // two of them fit a CU, and up to 256 of the large ones they are still ahead (64 x 1024 causal 25.2 / 23.5, 32 x 1500 35.3 /
+  // 30.3, 24 x 2048 unmasked 46.8 / 43.7); at head_dim 128 they are not (24 x 2048 unmasked 65 / 97).
+  if (mlts_attn_halved_workgroups(p, D == 64 ? 256 : 128)) return launch<D, MODE, 4>(p, st);
   return launch<D, MODE, 8>(p, st);
 }
 

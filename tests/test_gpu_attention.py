@@ -164,8 +164,8 @@ def test_document_mask_long_row_equals_causal_attention_per_document(dev, D):
 @pytest.mark.parametrize("Hq,Hkv,Sq,Sk", [(12, 12, 333, 333), (12, 6, 257, 130), (8, 2, 65, 321)])
 def test_small_grids_equal_large_ones(dev, D, mode, Hq, Hkv, Sq, Sk):
     """Workgroups of half the rows or keys take the calls that would leave half of the CUs idle: every batch row of a call on
-    the other side of that line (more than 128 workgroups of 256 rows, and of 128 keys) has the bits of a call on it alone."""
-    B = 1 + 128 // min(Hkv * ((Sk + 127) // 128), Hq // 4 * ((Sq + 63) // 64))
+    the other side of that line (more than 256 workgroups of 256 rows, and of 128 keys) has the bits of a call on it alone."""
+    B = 1 + 256 // min(Hkv * ((Sk + 127) // 128), Hq // 4 * ((Sq + 63) // 64))
     gen = torch.Generator().manual_seed(Hq + Sq)
     q, k, v, do = (bshd(B, H, S, D, gen, torch.bfloat16).to(dev) for H, S in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk), (Hq, Sq)))
     k = k.contiguous()  # (another order of strides than the rest)
