@@ -492,7 +492,7 @@ struct GateUpBackward final : Formula {
   std::string name() const override { return "MaltosGateUpBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(3);
-    const Tensor dgu = swiglu_rows_backward(g[0], s[GU], rows->first[0], rows->first[1], weights[0].size(0));
+    const Tensor dgu = swiglu_rows_backward(g[0], dense(s[GU]), rows->first[0], rows->first[1], weights[0].size(0));
     const Tensor dgu2 = rows2d(dgu);
     return grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dgu2);
   }
@@ -565,9 +565,13 @@ Tensor rope_attention(const Tensor& q, const Tensor& k, const Tensor& v, const T
 // forward, calling its modules one after the other 110 us of host time, and the views between them cost the backward pass
 // another 20.
 
-// [B, H, S, D] over [B, S, H, D] storage (or a column range of wider rows) as [B * S, H * D] rows
+// [B, H, S, D] as [B * S, H * D] rows: a view of [B, S, H, D] storage (or a column range of wider rows), a copy of any other layout
+// (a saved tensor may come back from the user's hooks in another one)
 Tensor as_rows(const Tensor& t) {
-  return t.as_strided({t.size(0) * t.size(2), t.size(1) * t.size(3)}, {t.stride(2), 1}, t.storage_offset());
+  const int64_t B = t.size(0), H = t.size(1), S = t.size(2), D = t.size(3);
+  if (t.stride(3) == 1 && t.stride(1) == D && t.stride(2) >= H * D && t.stride(0) == S * t.stride(2))
+    return t.as_strided({B * S, H * D}, {t.stride(2), 1}, t.storage_offset());
+  return t.transpose(1, 2).reshape({B * S, H * D});
 }
 // columns col .. col + heads * dim of [B, S, width] rows as [B, heads, S, dim]
 Tensor as_heads(const Tensor& rows, int64_t batch, int64_t seq, int64_t width, int64_t col, int64_t heads, int64_t dim) {
@@ -672,7 +676,7 @@ struct MlpBlockBackward final : Formula {
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(4);
     auto [dh, dw] = output_grads(g[0], s[OUT_W], rows2d(s[H]), into_grad_out);
-    const Tensor dgu = swiglu_rows_backward(dh.view(s[H].sizes()), s[GU], rows->first[0], rows->first[1], weights[0].size(0));
+    const Tensor dgu = swiglu_rows_backward(dh.view(s[H].sizes()), dense(s[GU]), rows->first[0], rows->first[1], weights[0].size(0));
     variable_list out = grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], rows2d(dgu));
     out.push_back(dw);
     return out;

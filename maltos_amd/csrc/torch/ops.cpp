@@ -901,9 +901,10 @@ struct CrossEntropyBackward final : Formula {
   void before_unpack(const variable_list& g) override { TORCH_CHECK(!consumed || !g[0].defined(), twice); }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return {Tensor()};
-    op::scale_by_scalar_().call(s[0], g[0]);
+    const Tensor dlogits = dense(s[0]);
+    op::scale_by_scalar_().call(dlogits, g[0]);
     consumed = true;
-    return {s[0].detach()};
+    return {dlogits.detach()};
   }
 };
 

@@ -1,0 +1,52 @@
+"""How the autograd nodes of the model and the operators behave beside the plain backward pass: saved-tensor hooks, frozen and
+shared parameters, second derivatives, tangents."""
+import pytest
+import torch
+
+from maltos_amd.llama import LlamaConfig, LlamaForCausalLM
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(dev, dtype=torch.bfloat16, **config):
+    cfg = dict(vocab_size=512, hidden_size=256, intermediate_size=688, num_hidden_layers=2, num_attention_heads=4,
+               num_key_value_heads=2, max_position_embeddings=128, rms_norm_eps=1e-5) | config
+    torch.manual_seed(5)
+    return LlamaForCausalLM(LlamaConfig(**cfg)).to(dev).to(dtype)
+
+
+def _batch(dev):
+    ids = torch.randint(0, 512, (2, 101), generator=torch.Generator().manual_seed(1)).to(dev)
+    return {"input_ids": ids, "labels": ids.clone()}
+
+
+def _contiguous(t):
+    return torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
+
+
+def _transposed(t):   # the same values, memory order of the dimensions reversed except for the last
+    if t.dim() < 3:
+        return _contiguous(t)
+    order = [*reversed(range(t.dim() - 1)), t.dim() - 1]
+    return _contiguous(t.permute(order)).permute([order.index(d) for d in range(t.dim())])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("pack", ["host", "contiguous", "transposed"])
+@pytest.mark.parametrize("seq", [101, 1])
+def test_saved_tensors_may_come_back_in_another_layout(dev, dtype, pack, seq):
+    model, batch = _model(dev, dtype), _batch(dev)
+    batch = {k: v[:, :seq].contiguous() for k, v in batch.items()}
+    model(batch).backward()
+    want = [p.grad.clone() for p in model.parameters()]
+    model.zero_grad()
+    if pack == "host":
+        hooks = torch.autograd.graph.save_on_cpu(pin_memory=True)
+    else:
+        hooks = torch.autograd.graph.saved_tensors_hooks(_contiguous if pack == "contiguous" else _transposed, lambda t: t)
+    with hooks:
+        loss = model(batch)
+    loss.backward()
+    for (name, p), w in zip(model.named_parameters(), want):
+        # the same kernels on the same values, the products' operands copied at most
+        assert torch.equal(p.grad, w), name
