@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -109,9 +110,10 @@ struct ProductList {
 };
 
 void notify_grad_written(const Tensor& param);  // llama.cpp: the parameter's gradient buffer was written past autograd
-// the gradient buffer a weight already owns and a backward formula may add into, or undefined
+// the gradient buffer a weight already owns and a backward formula may add into, or undefined (a backward pass that is itself
+// recorded leaves the adding to autograd: what the buffer holds has no history)
 inline Tensor bound_grad(const Tensor& weight, bool into_grad) {
-  if (!into_grad) return Tensor();
+  if (!into_grad || at::GradMode::is_enabled()) return Tensor();
   const Tensor& g = weight.grad();
   if (!g.defined() || !g.is_contiguous() || g.scalar_type() != weight.scalar_type() || g.sizes() != weight.sizes()) return Tensor();
   return g;
@@ -121,7 +123,8 @@ void bind_ops(pybind11::module& m);    // ops.cpp
 void bind_llama(pybind11::module& m);  // llama.cpp
 
 // A backward formula over saved tensors.  The tensors are unpacked first, with autograd as it is (an unpack hook may run a
-// checkpointed forward again), then `backward` runs without autograd recording.
+// checkpointed forward again), then `backward` runs without autograd recording.  A backward pass that is to be differentiated
+// itself (create_graph) goes to `recorded_backward`.
 struct Formula : public Node {
   explicit Formula(size_t count) : saved_(count) {}
   virtual variable_list backward(variable_list&& grads, const std::vector<Tensor>& saved) = 0;
@@ -136,10 +139,32 @@ struct Formula : public Node {
     before_unpack(grads);
     std::vector<Tensor> values(saved_.size());
     for (size_t i = 0; i < saved_.size(); ++i) values[i] = saved_[i].unpack((outputs_ >> i) & 1 ? getptr() : nullptr);
+    if (at::GradMode::is_enabled()) return recorded_backward(std::move(grads), values);
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     return backward(std::move(grads), values);
   }
   virtual void before_unpack(const variable_list&) {}
+  // The backward kernels have no derivatives: their results carry an error as history, so that a second derivative raises where
+  // its terms would be missing.  Formulas made of differentiable operators override this.
+  virtual variable_list recorded_backward(variable_list&& grads, const std::vector<Tensor>& saved) {
+    torch::autograd::edge_list sources;
+    for (const Tensor& g : grads)
+      if (g.defined() && g.requires_grad()) sources.push_back(torch::autograd::impl::gradient_edge(g));
+    for (const Edge& e : next_edges())
+      if (e.is_valid()) sources.push_back(e);
+    variable_list out;
+    {
+      at::AutoDispatchBelowADInplaceOrView below_autograd;
+      out = backward(std::move(grads), saved);
+      for (Tensor& t : out)
+        if (t.defined()) t = t.detach();  // (a result may be one of the gradients, or stand there twice)
+    }
+    const auto error = std::shared_ptr<Node>(new torch::autograd::Error(name() + ": maltos_amd has no second derivative of this operator", std::move(sources)),
+                                             torch::autograd::deleteNode);
+    for (const Tensor& t : out)
+      if (t.defined()) torch::autograd::set_history(t, error);
+    return out;
+  }
   void release_variables() override {
     for (SavedVariable& s : saved_) s.reset_data();
   }

@@ -192,6 +192,12 @@ struct LinearBackward final : Formula {
     }
     return {dx, dw};
   }
+  variable_list recorded_backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    const Tensor &x = s[X], &w = s[W], &dy = g[0];
+    if (!dy.defined()) return {Tensor(), Tensor()};
+    return {task_should_compute_output(0) ? at::matmul(dy, w) : Tensor(),
+            task_should_compute_output(1) ? at::mm(rows2d(dy).t(), rows2d(x)) : Tensor()};
+  }
 };
 
 Tensor linear(const Tensor& x, const Tensor& weight, bool into_grad) {
@@ -230,6 +236,9 @@ struct EmbeddingBackward final : Formula {
     if (!grad.defined()) return {dw};
     notify_grad_written(w);
     return {Tensor()};
+  }
+  variable_list recorded_backward(variable_list&& g, const std::vector<Tensor>& s) override {
+    return {g[0].defined() ? at::embedding_dense_backward(g[0], s[IDS], s[W].size(0), -1, false) : Tensor()};
   }
 };
 
@@ -369,7 +378,7 @@ variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights
   variable_list out(1 + weights.size());
   const Tensor x2 = rows2d(x);
   if (a.weight.defined()) {
-    const Tensor grad = into_grad ? a.grad : Tensor();
+    const Tensor grad = into_grad && !at::GradMode::is_enabled() ? a.grad : Tensor();
     Tensor dw;
     if (need_dx) std::tie(out[0], dw) = input_and_weight_grad(dy2, a.weight, x2, grad);
     else dw = weight_grad(x2, dy2, grad);

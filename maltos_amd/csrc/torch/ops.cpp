@@ -805,6 +805,7 @@ struct RopeBackward final : Formula {
     if (!g[0].defined()) return {Tensor()};
     return {op::rope().call(g[0], s[COS], s[SIN], optional_tensor(s[POSITIONS]), position_offset, !inverse)};
   }
+  variable_list recorded_backward(variable_list&& g, const std::vector<Tensor>& s) override { return backward(std::move(g), s); }
 };
 
 Tensor rope_autograd(const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& positions, int64_t position_offset, bool inverse) {
@@ -841,6 +842,7 @@ struct RopePairBackward final : Formula {
       if (g[i].defined()) out[i] = op::rope().call(g[i], s[COS], s[SIN], pos, position_offset, !inverse);
     return out;
   }
+  variable_list recorded_backward(variable_list&& g, const std::vector<Tensor>& s) override { return backward(std::move(g), s); }
 };
 
 std::tuple<Tensor, Tensor> rope_pair_autograd(const Tensor& xa, const Tensor& xb, const Tensor& cos, const Tensor& sin, const OptTensor& positions,

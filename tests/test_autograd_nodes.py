@@ -1,0 +1,74 @@
+"""CPU tests of the C++ autograd nodes: what they do when a backward pass is itself differentiated.  The products and the embedding run
+through torch on host tensors, the operators on meta tensors (shapes only): no kernel is launched."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from maltos_amd import ops  # noqa: F401  (registers the operators)
+from maltos_amd._native import native
+
+
+def _second(f, leaves):
+    """Gradient of a penalty on the first derivatives."""
+    first = torch.autograd.grad((f(*leaves) ** 3).sum(), leaves, create_graph=True)
+    return torch.autograd.grad(sum((g ** 2).sum() for g in first), leaves)
+
+
+@pytest.mark.parametrize("into_grad", [False, True])
+@pytest.mark.parametrize("shape", [(5, 6), (2, 3, 6), (6,)])
+def test_second_derivative_of_the_linear_layer(shape, into_grad):
+    gen = torch.Generator().manual_seed(1)
+    x, w = torch.randn(shape, generator=gen, dtype=torch.double), torch.randn(4, 6, generator=gen, dtype=torch.double)
+    leaves = x.requires_grad_(True), w.requires_grad_(True)
+    if into_grad:
+        w.grad = torch.zeros_like(w)
+    dx, dw = _second(lambda x, w: native().linear(x, w, into_grad), leaves)
+    if into_grad:   # the last pass, which is not recorded, adds its own part to the buffer
+        dw = dw + w.grad
+    for got, want in zip((dx, dw), _second(F.linear, leaves)):
+        assert torch.allclose(got, want, rtol=1e-12)
+    if into_grad:   # a recorded pass adds to .grad with history, as torch does
+        (native().linear(x, w, True) ** 2).sum().backward(create_graph=True)
+        assert w.grad.grad_fn is not None
+
+
+def test_second_derivative_of_the_embedding():
+    gen = torch.Generator().manual_seed(2)
+    w = torch.randn(7, 4, generator=gen, dtype=torch.double).requires_grad_(True)
+    ids = torch.tensor([[1, 2, 2], [0, 6, 1]])
+    (got,), (want,) = (_second(f, (w,)) for f in (lambda w: native().embedding(w, ids, False), lambda w: F.embedding(ids, w)))
+    assert torch.allclose(got, want, rtol=1e-12)
+
+
+def _meta(*shape):
+    return torch.empty(shape, device="meta", requires_grad=True)
+
+
+_OPS = {
+    "attn_fwd": lambda: (lambda q, k, v: torch.ops.maltos.attn_fwd(q, k, v, 1, 0.5, None, None, None, None)[0], [_meta(1, 2, 4, 8) for _ in range(3)]),
+    "rmsnorm_fwd": lambda: (lambda x, w: torch.ops.maltos.rmsnorm_fwd(x, w, 1e-5)[0], [_meta(3, 8), _meta(8)]),
+    "add_rmsnorm_fwd": lambda: (lambda x, r, w: sum(torch.ops.maltos.add_rmsnorm_fwd(x, r, w, 1e-5)[:2]), [_meta(3, 8), _meta(3, 8), _meta(8)]),
+    "swiglu_fwd": lambda: (torch.ops.maltos.swiglu_fwd, [_meta(3, 8), _meta(3, 8)]),
+    "ce_fwd_bwd": lambda: (lambda x: torch.ops.maltos.ce_fwd_bwd(x, torch.zeros(3, dtype=torch.long, device="meta"), -100)[0], [_meta(3, 8)]),
+}
+
+
+@pytest.mark.parametrize("name", _OPS)
+def test_a_second_derivative_without_a_formula_raises(name):
+    f, leaves = _OPS[name]()
+    for wanted in range(len(leaves)):
+        first = torch.autograd.grad(f(*leaves).sum() ** 2, leaves, create_graph=True)   # (recording alone is fine)
+        with pytest.raises(RuntimeError, match="no second derivative"):
+            torch.autograd.grad(sum(g.sum() ** 2 for g in first), leaves[wanted], allow_unused=True)
+    with pytest.raises(RuntimeError, match="no second derivative"):
+        first = torch.autograd.grad(f(*leaves).sum() ** 2, leaves, create_graph=True)
+        sum(g.sum() ** 2 for g in first).backward()
+
+
+def test_rotations_are_differentiable_twice():
+    cos, sin = torch.empty(4, 4, device="meta"), torch.empty(4, 4, device="meta")
+    for f, leaves in ((lambda x: torch.ops.maltos.rope(x, cos, sin, None, 0, False), [_meta(1, 2, 4, 8)]),
+                      (lambda a, b: sum(torch.ops.maltos.rope_pair(a, b, cos, sin, None, 0, False)), [_meta(1, 2, 4, 8), _meta(1, 2, 4, 8)])):
+        first = torch.autograd.grad((f(*leaves) ** 2).sum(), leaves, create_graph=True)
+        second = torch.autograd.grad(sum((g ** 2).sum() for g in first), leaves)
+        assert [g.shape for g in second] == [t.shape for t in leaves]

@@ -50,3 +50,18 @@ def test_saved_tensors_may_come_back_in_another_layout(dev, dtype, pack, seq):
     for (name, p), w in zip(model.named_parameters(), want):
         # the same kernels on the same values, the products' operands copied at most
         assert torch.equal(p.grad, w), name
+
+
+def test_gradient_penalty_through_the_model_raises(dev):
+    """No term of a second derivative is dropped without a word: the nodes of the layers have no second derivative."""
+    model, batch = _model(dev), _batch(dev)
+    weights = [p for p in model.parameters()]
+    loss = model(batch)
+    first = torch.autograd.grad(loss, weights, create_graph=True)
+    model.zero_grad()
+    model(batch).backward()
+    for g, p in zip(first, weights):   # (recording alone changes nothing; sums of products in another order)
+        assert (g.detach().float() - p.grad.float()).norm() <= 1e-2 * p.grad.float().norm()
+    for g in (first[0], first[3], first[-1]):   # embedding, a projection, the head
+        with pytest.raises(RuntimeError, match="no second derivative"):
+            torch.autograd.grad(g.float().square().sum(), weights, allow_unused=True, retain_graph=True)
