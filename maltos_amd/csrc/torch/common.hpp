@@ -49,6 +49,13 @@ inline void require_gpu(const OptTensor& t) {
   if (t.has_value()) require_gpu(*t);
 }
 
+// Forward-mode tangents: the kernels have no formula for them, and an output without one reads as a derivative of zero.
+inline bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(0).defined(); }
+template <typename... T>
+void refuse_tangents(const char* what, const T&... tensors) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!(has_tangent(tensors) || ...), what, ": maltos_amd has no forward-mode derivative of this operator");
+}
+
 inline mlts_stream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 inline bool stream_is_capturing() {
   return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;

@@ -200,7 +200,11 @@ struct LinearBackward final : Formula {
   }
 };
 
+// What the nodes below know nothing of (tangents, tensors of function transforms and other subclasses) is left to torch's operators
+bool ordinary(const Tensor& t) { return !has_tangent(t) && !at::isTensorSubclassLike(t); }
+
 Tensor linear(const Tensor& x, const Tensor& weight, bool into_grad) {
+  if (!ordinary(x) || !ordinary(weight)) return at::linear(x, weight);
   std::shared_ptr<LinearBackward> fn;
   if (compute_requires_grad(x, weight)) {
     fn = make_formula<LinearBackward>();
@@ -243,6 +247,7 @@ struct EmbeddingBackward final : Formula {
 };
 
 Tensor embedding(const Tensor& weight, const Tensor& ids, bool into_grad) {
+  if (!ordinary(weight) || !ordinary(ids)) return at::embedding(weight, ids);
   std::shared_ptr<EmbeddingBackward> fn;
   if (compute_requires_grad(weight)) {
     fn = make_formula<EmbeddingBackward>();
@@ -460,6 +465,15 @@ struct AdjacentLinearsBackward final : Formula {
   }
 };
 
+// the nodes of several projections have no counterpart in torch to fall back to
+void refuse_function_transforms(const char* what, const Tensor& x, const std::vector<Tensor>& weights = {}) {
+  auto wrapped = [](const Tensor& t) { return t.key_set().has(c10::DispatchKey::FuncTorchBatched) || t.key_set().has(c10::DispatchKey::FuncTorchGradWrapper); };
+  bool any = wrapped(x);
+  refuse_tangents(what, x);
+  for (const Tensor& w : weights) refuse_tangents(what, w), any = any || wrapped(w);
+  TORCH_CHECK_NOT_IMPLEMENTED(!any, what, ": maltos_amd has no rule of this operator for function transforms");
+}
+
 bool any_requires_grad(const std::vector<Tensor>& ts) {
   return std::any_of(ts.begin(), ts.end(), [](const Tensor& t) { return t.requires_grad(); });
 }
@@ -477,6 +491,7 @@ std::shared_ptr<F> adjacent_formula(const Tensor& x, const AdjacentPtr& rows, co
 
 // (x W_0^T, x W_1^T, ...) as column slices of one buffer: one product with the parameters' common matrix, or their group
 std::vector<Tensor> adjacent_linears(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
+  refuse_function_transforms("adjacent_linears", x, weights);
   std::vector<Tensor> out(weights.size());
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
@@ -508,6 +523,7 @@ struct GateUpBackward final : Formula {
 };
 
 Tensor gate_up(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
+  refuse_function_transforms("gate_up", x, weights);
   Tensor gu, h;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
@@ -543,6 +559,7 @@ struct RopeAttentionBackward final : Formula {
 
 Tensor rope_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cos, const Tensor& sin, const OptTensor& rope_positions,
                       int64_t position_offset, const OptTensor& positions, const OptTensor& sequences) {
+  refuse_function_transforms("rope_attention", q, {k, v, cos, sin});
   std::shared_ptr<RopeAttentionBackward> fn;
   Tensor out;
   const int64_t mask_mode = positions.has_value() ? MLTS_MASK_DOC : MLTS_MASK_CAUSAL;
@@ -784,7 +801,7 @@ bool read_layer(PyObject* layer, const pybind11::dict& types, const pybind11::ha
   if (!attn.flag("fuse_projections") || !attn.flag("fuse_rope_attention") || !mlp.flag("fuse_projections")) return false;
 
   auto fits = [&](const Tensor& t, int64_t dims) {
-    return t.defined() && t.dim() == dims && t.is_cuda() && t.scalar_type() == x.scalar_type() && t.is_contiguous() && t.device() == x.device();
+    return t.defined() && ordinary(t) && t.dim() == dims && t.is_cuda() && t.scalar_type() == x.scalar_type() && t.is_contiguous() && t.device() == x.device();
   };
   auto block = [&](const ModuleView& m, std::initializer_list<const char*> ins, const char* last, BlockWeights& w) {
     w.into_grad_in = true;
@@ -825,7 +842,7 @@ bool read_layer(PyObject* layer, const pybind11::dict& types, const pybind11::ha
 // layer is not made of stock modules, something hooks into one, or its projections run one by one
 pybind11::object run_layers(const pybind11::dict& layers, const pybind11::dict& types, const pybind11::object& backends, const Tensor& x_in,
                             int64_t position_offset, const OptTensor& rope_positions, const OptTensor& positions, const OptTensor& sequences) {
-  if (!x_in.is_cuda() || x_in.dim() != 3 || !x_in.is_contiguous() || x_in.numel() == 0 || at::isTensorSubclassLike(x_in) ||
+  if (!x_in.is_cuda() || x_in.dim() != 3 || !x_in.is_contiguous() || x_in.numel() == 0 || !ordinary(x_in) ||
       (x_in.scalar_type() != at::kBFloat16 && x_in.scalar_type() != at::kFloat) || c10::impl::dispatch_mode_enabled() ||
       at::autocast::is_autocast_enabled(at::kCUDA))
     return pybind11::none();

@@ -684,6 +684,7 @@ struct AttnBackward final : Formula {
 
 std::tuple<Tensor, Tensor> attn_fwd_autograd(const Tensor& q, const Tensor& k, const Tensor& v, int64_t mask_mode, double scale,
                                              const OptTensor& q_pos, const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq) {
+  refuse_tangents("attn_fwd", q, k, v);
   std::shared_ptr<AttnBackward> fn;
   if (compute_requires_grad(q, k, v)) {
     fn = make_formula<AttnBackward>();
@@ -729,6 +730,7 @@ struct RmsNormBackward final : Formula {
 };
 
 std::tuple<Tensor, Tensor> rmsnorm_recorded(const Tensor& x, const Tensor& w, double eps, bool into_grad) {
+  refuse_tangents("rmsnorm_fwd", x, w);
   std::shared_ptr<RmsNormBackward> fn;
   if (compute_requires_grad(x, w)) {
     fn = make_formula<RmsNormBackward>();
@@ -769,6 +771,7 @@ struct AddRmsNormBackward final : Formula {
 };
 
 std::tuple<Tensor, Tensor, Tensor> add_rmsnorm_recorded(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad) {
+  refuse_tangents("add_rmsnorm_fwd", x, res, w);
   std::shared_ptr<AddRmsNormBackward> fn;
   if (compute_requires_grad(x, res, w)) {
     fn = make_formula<AddRmsNormBackward>();
@@ -809,6 +812,7 @@ struct RopeBackward final : Formula {
 };
 
 Tensor rope_autograd(const Tensor& x, const Tensor& cos, const Tensor& sin, const OptTensor& positions, int64_t position_offset, bool inverse) {
+  refuse_tangents("rope", x, cos, sin);
   std::shared_ptr<RopeBackward> fn;
   if (compute_requires_grad(x)) {
     fn = make_formula<RopeBackward>();
@@ -847,6 +851,7 @@ struct RopePairBackward final : Formula {
 
 std::tuple<Tensor, Tensor> rope_pair_autograd(const Tensor& xa, const Tensor& xb, const Tensor& cos, const Tensor& sin, const OptTensor& positions,
                                               int64_t position_offset, bool inverse) {
+  refuse_tangents("rope_pair", xa, xb, cos, sin);
   std::shared_ptr<RopePairBackward> fn;
   if (compute_requires_grad(xa, xb)) {
     fn = make_formula<RopePairBackward>();
@@ -878,6 +883,7 @@ struct SwigluBackward final : Formula {
 };
 
 Tensor swiglu_fwd_autograd(const Tensor& gate, const Tensor& up) {
+  refuse_tangents("swiglu_fwd", gate, up);
   std::shared_ptr<SwigluBackward> fn;
   if (compute_requires_grad(gate, up)) {
     fn = make_formula<SwigluBackward>();
@@ -911,6 +917,7 @@ struct CrossEntropyBackward final : Formula {
 };
 
 std::tuple<Tensor, Tensor, Tensor> ce_fwd_bwd_autograd(const Tensor& logits, const Tensor& labels, int64_t ignore_index) {
+  refuse_tangents("ce_fwd_bwd", logits);
   std::shared_ptr<CrossEntropyBackward> fn;
   if (compute_requires_grad(logits)) {
     fn = make_formula<CrossEntropyBackward>();
@@ -935,6 +942,7 @@ std::tuple<Tensor, Tensor, Tensor> ce_fwd_bwd_autograd(const Tensor& logits, con
 // logits-sized tensor.  For callers that own the logits and never look at them again; not an operator, because one that
 // overwrites an argument it is differentiated by has no functional form to register.
 Tensor cross_entropy_over_logits(const Tensor& logits, const Tensor& labels, int64_t ignore_index) {
+  refuse_tangents("ce_fwd_bwd", logits);
   std::shared_ptr<CrossEntropyBackward> fn;
   if (compute_requires_grad(logits)) {
     fn = make_formula<CrossEntropyBackward>();

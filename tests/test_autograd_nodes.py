@@ -1,4 +1,5 @@
-"""CPU tests of the C++ autograd nodes: what they do when a backward pass is itself differentiated.  The products and the embedding run
+"""CPU tests of the C++ autograd nodes: what they do when a backward pass is itself differentiated, with forward-mode tangents and under
+function transforms.  The products and the embedding run
 through torch on host tensors, the operators on meta tensors (shapes only): no kernel is launched."""
 import pytest
 import torch
@@ -72,3 +73,48 @@ def test_rotations_are_differentiable_twice():
         first = torch.autograd.grad((f(*leaves) ** 2).sum(), leaves, create_graph=True)
         second = torch.autograd.grad(sum((g ** 2).sum() for g in first), leaves)
         assert [g.shape for g in second] == [t.shape for t in leaves]
+
+
+@pytest.mark.parametrize("f,shapes", [(lambda x, w: native().linear(x, w, False), [(5, 6), (4, 6)]),
+                                      (lambda w: native().embedding(w, torch.tensor([[1, 2, 2], [0, 6, 1]]), False), [(7, 4)])], ids=["linear", "embedding"])
+def test_tangents_and_transforms_of_the_linear_layer_and_the_embedding(f, shapes):
+    plain = {2: lambda x, w: F.linear(x, w), 1: lambda w: F.embedding(torch.tensor([[1, 2, 2], [0, 6, 1]]), w)}[len(shapes)]
+    gen = torch.Generator().manual_seed(3)
+    values, tangents = ([torch.randn(s, generator=gen, dtype=torch.double) for s in shapes] for _ in range(2))
+    for requires_grad in (False, True):
+        leaves = [v.clone().requires_grad_(requires_grad) for v in values]
+        with torch.autograd.forward_ad.dual_level():
+            for only in range(len(shapes)):   # one tangent at a time
+                args = [torch.autograd.forward_ad.make_dual(v, t) if i == only else v for i, (v, t) in enumerate(zip(leaves, tangents))]
+                got, want = (torch.autograd.forward_ad.unpack_dual(g(*args)).tangent for g in (f, plain))
+                assert torch.allclose(got, want)
+    for got, want in ((torch.func.jvp(g, tuple(values), tuple(tangents))[1] for g in (f, plain)),
+                      (torch.func.grad(lambda *a: (g(*a) ** 2).sum())(*values) for g in (f, plain)),
+                      (torch.func.vmap(g, in_dims=(0, *[None] * (len(shapes) - 1)))(torch.stack([values[0]] * 2), *values[1:]) for g in (f, plain))):
+        assert torch.allclose(got, want)
+
+
+@pytest.mark.parametrize("requires_grad", [False, True])
+@pytest.mark.parametrize("name", _OPS)
+def test_a_tangent_without_a_formula_raises(name, requires_grad):
+    f, leaves = _OPS[name]()
+    leaves = [t.detach().requires_grad_(requires_grad) for t in leaves]
+    with torch.autograd.forward_ad.dual_level():
+        for only in range(len(leaves)):
+            args = [torch.autograd.forward_ad.make_dual(t, torch.empty_like(t)) if i == only else t for i, t in enumerate(leaves)]
+            with pytest.raises(NotImplementedError, match="forward-mode"):
+                f(*args)
+
+
+def test_tangents_through_rotations_and_joint_projections_raise():
+    cos, sin = torch.empty(4, 4, device="meta"), torch.empty(4, 4, device="meta")
+    x = torch.empty(1, 2, 4, 8, device="meta")
+    group = native().Adjacent([torch.empty(4, 6)])
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.empty_like(x))
+        rows = torch.autograd.forward_ad.make_dual(torch.empty(3, 6), torch.empty(3, 6))
+        for call in (lambda: torch.ops.maltos.rope(dual, cos, sin, None, 0, False), lambda: torch.ops.maltos.rope_pair(x, dual, cos, sin, None, 0, False),
+                     lambda: native().rope_attention(x, x, dual, cos, sin, None, 0, None, None), lambda: native().cross_entropy_over_logits(rows, rows, 0),
+                     lambda: native().adjacent_linears(rows, group, [torch.empty(4, 6)], False), lambda: native().gate_up(rows, group, [torch.empty(4, 6)], False)):
+            with pytest.raises(NotImplementedError, match="forward-mode"):
+                call()

@@ -65,3 +65,12 @@ def test_gradient_penalty_through_the_model_raises(dev):
     for g in (first[0], first[3], first[-1]):   # embedding, a projection, the head
         with pytest.raises(RuntimeError, match="no second derivative"):
             torch.autograd.grad(g.float().square().sum(), weights, allow_unused=True, retain_graph=True)
+
+
+@pytest.mark.parametrize("name", ["layers.1.self_attn.q_proj.weight", "layers.0.mlp.down_proj.weight", "layers.1.input_layernorm.weight", "embed_tokens.weight"])
+def test_tangent_of_a_weight_is_not_dropped_by_the_model(dev, name):
+    model, batch = _model(dev), _batch(dev)
+    weights = dict(model.named_parameters())
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="forward-mode"):
+        dual = torch.autograd.forward_ad.make_dual(weights[name].detach(), torch.ones_like(weights[name]))
+        torch.func.functional_call(model, {name: dual}, (batch,))
