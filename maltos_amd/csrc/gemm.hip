@@ -650,11 +650,23 @@ mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const vo
 template <typename T>
 int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hipStream_t st) {
   const LaunchPlan plan(ps, count, dtype);
-  Products joint{};
+  Products joint;
   Joins joins{};
-  int blocks = 0, join_blocks = 0, smalls = 0;
-  bool all_nt = true, all_nn = true, segments = false;
-  std::fill(joint.first, joint.first + kMaxProducts, 0x7fffffff);
+  int blocks, join_blocks = 0, smalls;
+  bool all_nt, all_nn;
+  auto clear = [&] {
+    joint = {};
+    std::fill(joint.first, joint.first + kMaxProducts, 0x7fffffff);
+    blocks = smalls = 0, all_nt = all_nn = true;
+  };
+  auto launch = [&] {  // what `joint` holds
+    if (!smalls) return static_cast<int>(MLTS_OK);
+    const int forms = joint.more.count ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
+    if constexpr (sizeof(T) == 2) return launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
+    else if (plan.shape.size == 64) return launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
+    else return launch_small_forms<T, 32, 32, 4>(forms, joint, blocks, st);
+  };
+  clear();
   MltsKernelTimer timer("gemm", st);
   for (int i = 0; i < count; ++i) {
     const mlts_gemm_product& p = ps[i];
@@ -668,7 +680,13 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hip
     g.tiles_m = static_cast<int>((p.M + bm - 1) / bm), g.tiles_n = static_cast<int>((p.N + bn - 1) / bn);
     const int64_t slabs = slabs_of(p, slab_of(dtype));
     set_slices(g, plan.slices[i], slabs, slab_of(dtype));
+    const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices;
+    if (tiles == 0) continue;
     if (p.segments > 1) {
+      if (joint.more.count) {  // a launch has room for the segments of one product
+        if (int rc = launch(); rc != MLTS_OK) return rc;
+        clear();
+      }
       g.k_slice = g.K;
       for (int k = 1; k < p.segments; ++k) {
         joint.more.a[k - 1] = p.a[k], joint.more.b[k - 1] = p.b[k];
@@ -676,17 +694,15 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hip
       }
       joint.more.count = p.segments - 1, joint.more.product = smalls;
     }
-    const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices;
     MLTS_REQUIRE(blocks + tiles < (int64_t{1} << 30), "mlts_gemm: too many tiles");
-    if (tiles == 0) continue;
     if (plan.slices[i] > 1) {
       g.partial = workspace;
       workspace += p.M * p.N * plan.slices[i];
       joins.p[joins.count++] = {p.c, g.partial, g.slices, g.accumulate, join_blocks, p.M * p.N / 4};
       join_blocks += static_cast<int>((p.M * p.N / 4 + 255) / 256);
     }
-    if (small && count > 1) {
-      all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN, segments = segments || p.segments > 1;
+    if (small && (count > 1 || p.segments > 1)) {
+      all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN;
       joint.first[smalls] = blocks;
       blocks += static_cast<int>((tiles + 7) / 8 * 8);  // (whole rounds over the XCDs, so that each product starts at the first)
       joint.p[smalls++] = g;
@@ -694,14 +710,7 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hip
       return rc;
     }
   }
-  if (smalls) {
-    const int forms = segments ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
-    int rc;
-    if constexpr (sizeof(T) == 2) rc = launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
-    else if (plan.shape.size == 64) rc = launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
-    else rc = launch_small_forms<T, 32, 32, 4>(forms, joint, blocks, st);
-    if (rc != MLTS_OK) return rc;
-  }
+  if (int rc = launch(); rc != MLTS_OK) return rc;
   if (joins.count) hipLaunchKernelGGL(gemm_join_kernel<T>, dim3(static_cast<unsigned>(join_blocks)), dim3(256), 0, st, joins);
   return mlts_check_launch("mlts_gemm");
 }

@@ -1,5 +1,7 @@
 """GPU parity of the matrix products of the linear layers (mlts_gemm) with fp32 / fp64 torch products: remainders of every tile
 and slab, split contractions, strided operands, accumulation, and what is left to the library."""
+import ctypes
+
 import pytest
 import torch
 
@@ -77,3 +79,44 @@ def test_group_of_projections(dev, dtype, rows, hidden, widths):
     want = [xd @ w.t() for w in wd] + [sum(d @ w for d, w in zip(dd, wd))] + [d.t() @ xd for d in dd]
     for got, w in zip([*ys, *grads], want):
         assert (got.detach().double() - w).norm() <= rel * w.norm()
+
+
+class GemmProduct(ctypes.Structure):
+    """Mirror of `mlts_gemm_product`."""
+    _fields_ = [("form", ctypes.c_int32), ("segments", ctypes.c_int32), ("accumulate", ctypes.c_int32), ("M", ctypes.c_int64), ("N", ctypes.c_int64),
+                ("k", ctypes.c_int64 * 3), ("a", ctypes.c_void_p * 3), ("b", ctypes.c_void_p * 3), ("lda", ctypes.c_int64 * 3),
+                ("ldb", ctypes.c_int64 * 3), ("c", ctypes.c_void_p), ("ldc", ctypes.c_int64)]
+
+
+def run_products(products, dtype):
+    """mlts_gemm_multi of (form, [(a, b), ...], c, accumulate)."""
+    ps = (GemmProduct * len(products))()
+    for p, (form, segments, c, accumulate) in zip(ps, products):
+        p.form, p.segments, p.accumulate, (p.M, p.N), p.c, p.ldc = form, len(segments), accumulate, c.shape, c.data_ptr(), c.stride(0)
+        for i, (a, b) in enumerate(segments):
+            p.k[i] = a.size(0) if form == TN else a.size(1)
+            p.a[i], p.b[i], p.lda[i], p.ldb[i] = a.data_ptr(), b.data_ptr(), a.stride(0), b.stride(0)
+    code, L = {torch.bfloat16: _lib.MLTS_BF16, torch.float32: _lib.MLTS_F32}[dtype], _lib.lib()
+    ws = torch.empty(max(16, L.mlts_gemm_multi_workspace_bytes(ps, len(ps), code)), dtype=torch.uint8, device=products[0][2].device)
+    _lib.check(L.mlts_gemm_multi(ps, len(ps), code, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("plan", ["s", "ss", "sss", "nsts", "0s", "s0n", "tn"])
+def test_products_with_segments_in_one_call(dev, dtype, plan):
+    """s: a sum over three segments, alone and beside others; 0: one without rows; n, t: plain NN and TN products."""
+    gen = torch.Generator().manual_seed(len(plan))
+    rnd = lambda *shape: torch.randn(*shape, generator=gen).to(dtype).to(dev)
+    products, want = [], []
+    for i, kind in enumerate(plan):
+        M, N = 0 if kind == "0" else 72 + 32 * i, 64 + 8 * i
+        ks = {"s": (64, 136, 32), "0": (64, 32), "n": (200,), "t": (72,)}[kind]
+        form = TN if kind == "t" else NN
+        segments = [(rnd(k, M) if form == TN else rnd(M, k), rnd(k, N)) for k in ks]
+        c, accumulate = rnd(M, N), i % 2
+        want.append(sum((expected(form, a, b) for a, b in segments), c.double() * accumulate))
+        products.append((form, segments, c, accumulate))
+    run_products(products, dtype)
+    rel = 4e-3 if dtype == torch.bfloat16 else 2e-6
+    for (_, _, c, _), w in zip(products, want):
+        assert (c.double() - w).norm() <= (2 if dtype == torch.bfloat16 else 1) * rel * w.norm()   # bf16: each segment is rounded
