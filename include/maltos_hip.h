@@ -284,7 +284,8 @@ int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, cons
               void* c, int64_t ldc, int32_t accumulate, void* workspace, int64_t workspace_bytes, mlts_stream_t stream);
 /* Up to four products in one call, small ones in one launch.  A product of the NN form may be the sum over up to three
  * segments a[i] b[i] (the input gradient of layers that share their input), in bf16 with the roundings of separate products.
- * A launch takes the segments of one product: a call with more of them takes more launches. */
+ * A launch takes the segments of one product: a call with more of them takes more launches.  The outputs of a call must not
+ * overlap (MLTS_ERR_INVALID). */
 typedef struct {
   int32_t form, segments, accumulate;
   int64_t M, N;

@@ -638,6 +638,19 @@ const char* why_not(const mlts_gemm_product& p, int dtype) {
   return nullptr;
 }
 
+// Whether two outputs of a call share elements (the column ranges of one buffer interleave, but do not).  Products of a launch run at
+// the same time: they must not.
+bool outputs_overlap(const mlts_gemm_product& p, const mlts_gemm_product& q, int es) {
+  if (p.M == 0 || p.N == 0 || q.M == 0 || q.N == 0) return false;
+  const uintptr_t pa = reinterpret_cast<uintptr_t>(p.c), qa = reinterpret_cast<uintptr_t>(q.c);
+  if (pa > qa) return outputs_overlap(q, p, es);
+  const uintptr_t p_end = pa + static_cast<uintptr_t>((p.M - 1) * p.ldc + p.N) * es;
+  if (qa >= p_end) return false;
+  if (p.ldc != q.ldc || (qa - pa) % es) return true;  // (row by row they may still miss each other: not worth telling apart)
+  const int64_t column = static_cast<int64_t>((qa - pa) / es) % p.ldc;  // of p's row in which q starts
+  return column < p.N || column + q.N > p.ldc;
+}
+
 mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc,
                          int32_t accumulate) {
   mlts_gemm_product p{};
@@ -744,6 +757,8 @@ extern "C" int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count,
     for (int k = 0; k < p.segments; ++k)
       MLTS_REQUIRE(p.k[k] == 0 || (p.a[k] && p.b[k] && mlts_aligned16(p.a[k]) && mlts_aligned16(p.b[k])),
                    "mlts_gemm: pointers must be 16-byte aligned and not null");
+    for (int j = 0; j < i; ++j)
+      MLTS_REQUIRE(!outputs_overlap(products[j], p, dtype == MLTS_BF16 ? 2 : 4), "mlts_gemm: outputs %d and %d of the call overlap", j, i);
   }
   const int64_t need = mlts_gemm_multi_workspace_bytes(products, count, dtype);
   MLTS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && mlts_aligned16(workspace)), "mlts_gemm: workspace too small or unaligned");

@@ -377,6 +377,13 @@ Tensor project_all(const Tensor& x, const Adjacent& rows, const std::vector<Tens
   return y;
 }
 
+// whether two dense buffers share memory (the gradient of a parameter that is used twice)
+bool share_memory(const Tensor& a, const Tensor& b) {
+  if (!a.defined() || !b.defined()) return false;
+  const char *pa = static_cast<const char*>(a.const_data_ptr()), *pb = static_cast<const char*>(b.const_data_ptr());
+  return pa < pb + b.nbytes() && pb < pa + a.nbytes();
+}
+
 // The input gradient (if asked for), then one gradient per parameter: added into the gradient buffers where into_grad allows it,
 // and then undefined.  dy2: the outputs' gradients side by side.
 variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, bool need_dx, const Tensor& x, const Tensor& dy2) {
@@ -404,6 +411,8 @@ variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights
       ProductList list;
       for (size_t i = 0; i < weights.size(); ++i) {
         Tensor dw = into[i].defined() ? into[i] : at::empty(weights[i].sizes(), dy2.options());
+        // two projections with one weight add into the same buffer: one launch after the other
+        if (std::any_of(into.begin(), into.begin() + i, [&](const Tensor& before) { return share_memory(before, into[i]); })) list.run(), list = {};
         list.add(MLTS_GEMM_TN, parts[i], x2, dw, into[i].defined());
         if (!into[i].defined()) out[1 + i] = dw;
       }

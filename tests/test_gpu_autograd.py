@@ -3,7 +3,7 @@ shared parameters, second derivatives, tangents."""
 import pytest
 import torch
 
-from maltos_amd.llama import LlamaConfig, LlamaForCausalLM
+from maltos_amd.llama import LlamaConfig, LlamaForCausalLM, set_grad_accumulation_into_buffers
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +74,24 @@ def test_tangent_of_a_weight_is_not_dropped_by_the_model(dev, name):
     with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="forward-mode"):
         dual = torch.autograd.forward_ad.make_dual(weights[name].detach(), torch.ones_like(weights[name]))
         torch.func.functional_call(model, {name: dual}, (batch,))
+
+
+@pytest.mark.parametrize("pairs", [(("k_proj", "v_proj"),), (("q_proj", "k_proj"), ("k_proj", "v_proj")), (("gate_proj", "up_proj"),)])
+def test_projections_that_share_a_weight_add_both_gradients_into_its_buffer(dev, pairs):
+    def shared_model():
+        model = _model(dev, torch.float32, num_key_value_heads=4)
+        for layer in model.layers:
+            for a, b in pairs:
+                holder = layer.mlp if a == "gate_proj" else layer.self_attn
+                getattr(holder, b).weight = getattr(holder, a).weight
+        return model
+
+    plain, buffers, batch = shared_model(), shared_model(), _batch(dev)
+    set_grad_accumulation_into_buffers(buffers)
+    for model in (plain, buffers):
+        for p in model.parameters():
+            p.grad = torch.zeros_like(p)
+        for _ in range(2):
+            model(batch).backward()
+    for (name, p), q in zip(buffers.named_parameters(), plain.parameters()):
+        assert (p.grad - q.grad).norm() <= 1e-5 * q.grad.norm(), name   # fp32 sums in another order

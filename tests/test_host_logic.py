@@ -294,3 +294,30 @@ def test_shipped_gemm_selection_file_is_well_formed():
     if not torch.cuda.is_available():
         with pytest.raises(RuntimeError, match="needs a GPU"):
             use_tuned_gemms()
+
+
+def test_products_of_a_call_must_not_share_outputs():
+    """Products of one launch run at the same time: two that add to the same C would lose one of the sums.  Column ranges of one
+    buffer are served (here with a workspace that is refused afterwards: nothing is launched)."""
+    class Product(ctypes.Structure):
+        _fields_ = [("form", ctypes.c_int32), ("segments", ctypes.c_int32), ("accumulate", ctypes.c_int32), ("M", ctypes.c_int64), ("N", ctypes.c_int64),
+                    ("k", ctypes.c_int64 * 3), ("a", ctypes.c_void_p * 3), ("b", ctypes.c_void_p * 3), ("lda", ctypes.c_int64 * 3),
+                    ("ldb", ctypes.c_int64 * 3), ("c", ctypes.c_void_p), ("ldc", ctypes.c_int64)]
+
+    def message(*outputs):   # (address in elements, rows, columns, row stride) of each product
+        ps = (Product * (len(outputs) + 1))()
+        for p, (at, M, N, ld) in zip(ps, outputs):
+            p.form, p.segments, p.M, p.N, p.c, p.ldc = 2, 1, M, N, 0x100000 + 4 * at, ld
+            p.k[0], p.a[0], p.b[0], p.lda[0], p.ldb[0] = 64, 0x1000, 0x2000, M, N
+        # a last product that the check of the arguments always refuses: its row stride is shorter than its rows
+        last = ps[len(outputs)]
+        last.form, last.segments, last.M, last.N, last.c, last.ldc = 2, 1, 64, 64, 0x3000, 32
+        assert _lib.lib().mlts_gemm_multi(ps, len(ps), _lib.MLTS_F32, None, 0, None) == _lib.MLTS_ERR_INVALID
+        return _lib.last_error()
+
+    for shared in ([(0, 64, 64, 64), (0, 64, 64, 64)], [(0, 64, 64, 64), (4032, 64, 64, 64)], [(4032, 64, 64, 64), (0, 64, 64, 64)],
+                   [(0, 64, 64, 160), (60, 64, 64, 160)], [(64, 64, 64, 128), (124, 64, 68, 128)], [(0, 8, 64, 64), (1024, 8, 64, 64), (448, 16, 64, 64)]):
+        assert "overlap" in message(*shared), shared
+    for apart in ([(0, 64, 64, 64), (4096, 64, 64, 64)], [(0, 64, 64, 160), (64, 64, 64, 160), (128, 64, 32, 160)], [(64, 64, 64, 128), (0, 64, 64, 128)],
+                  [(0, 64, 64, 64), (0, 0, 64, 64)]):
+        assert "row strides" in message(*apart), apart
