@@ -208,7 +208,8 @@ __global__ __launch_bounds__(kCeThreads) void ce_row_stream_kernel(const T* logi
   float label_logit = 0.f;
   if (threadIdx.x == 0 && label_ok) label_logit = to_f32<T>(zr[label]);
   const float mx = block_max(m, red);
-  se = block_sum(m == -INFINITY ? 0.f : se * exp2f((m - mx) * kLog2e), red);
+  // (a lane without a maximum has seen nothing, only -inf, which add 0, or NaN, which is its sum and has to reach the loss)
+  se = block_sum(m == -INFINITY ? se : se * exp2f((m - mx) * kLog2e), red);
   const float lse = mx + logf(se);
   if (threadIdx.x == 0) row_loss[row] = label_ok ? lse - label_logit : NAN;
   const int cnt = *count;

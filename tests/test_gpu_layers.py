@@ -297,6 +297,27 @@ def test_cross_entropy_rows_at_any_alignment(dev, dtype, vocab):
         torch.testing.assert_close(grad.float(), ref.grad, **tol)
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("vocab", [1, 9, 300, 513, 4099, 65553])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_cross_entropy_of_a_row_with_nan_is_nan(dev, dtype, vocab, offset):
+    """Wherever the NaN stands, also as the only element of a lane; offset 1: buffers that are not 16-byte aligned."""
+    gen = torch.Generator().manual_seed(vocab)
+    values = torch.randn(3, vocab, generator=gen)
+    values[0, 1:] = -float("inf")   # what a lane with nothing but -inf adds is zero
+    labels = torch.tensor([0, vocab - 1, 0], device=dev)
+    for at in sorted({0, vocab // 2, vocab - 1}):
+        x = values.clone()
+        for nan in (False, True):
+            if nan:
+                x[1, at] = float("nan")
+            leaf = torch.empty(3 * vocab + offset, dtype=dtype, device=dev)[offset:].view(3, vocab).copy_(x).requires_grad_(True)
+            loss = ops.cross_entropy(leaf, labels)
+            (grad,) = torch.autograd.grad(loss, leaf)
+            assert loss.isnan().item() == nan and grad[1].isnan().all().item() == nan
+            assert grad[0].isfinite().all() and grad[2].isfinite().all()
+
+
 @pytest.mark.parametrize("rows", [1, 3, 5, 1023, 1025, 2049, 4097])
 @pytest.mark.parametrize("hidden", [768, 2048, 4096])
 def test_rmsnorm_backward_few_rows(dev, rows, hidden):
