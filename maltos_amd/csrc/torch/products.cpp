@@ -31,6 +31,8 @@ struct Sizes {
 bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
 bool plain(const Tensor& t) { return t.is_cuda() && t.dim() == 2 && (t.stride(1) == 1 || t.size(1) == 1) && !at::isTensorSubclassLike(t); }
 
+int64_t row_stride(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : t.size(1); }  // (a single row's stride means nothing)
+
 Tensor library_product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
   const Tensor x = form == MLTS_GEMM_TN ? a.t() : a, y = form == MLTS_GEMM_NT ? b.t() : b;
   if (!out.defined()) return at::mm(x, y);
@@ -49,19 +51,21 @@ bool own_product(int form, const Tensor& a, const Tensor& b) {
 }
 
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
-  if (!own_product(form, a, b) || (out.defined() && !own_output(out, a))) return library_product(form, a, b, out, accumulate);
   const Sizes z(form, a, b);
+  TORCH_CHECK_VALUE(!out.defined() || (out.dim() == 2 && out.size(0) == z.M && out.size(1) == z.N), "a product of shape [", z.M, ", ", z.N,
+                    "] cannot be written to a tensor of shape ", out.sizes());
+  if (!own_product(form, a, b) || (out.defined() && !own_output(out, a))) return library_product(form, a, b, out, accumulate);
   Tensor c = out.defined() ? out : at::empty({z.M, z.N}, a.options());
   const int dtype = dtype_code(a);
   const int64_t ws_bytes = mlts_gemm_workspace_bytes(form, dtype, z.M, z.N, z.K);
   Tensor ws = workspace(ws_bytes, a);
-  check(mlts_gemm(form, dtype, z.M, z.N, z.K, ptr(a), a.stride(0), ptr(b), b.stride(0), mptr(c), z.N, accumulate,
+  check(mlts_gemm(form, dtype, z.M, z.N, z.K, ptr(a), a.stride(0), ptr(b), b.stride(0), mptr(c), row_stride(c), accumulate,
                   ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
   return c;
 }
 
 bool own_output(const Tensor& out, const Tensor& a) {
-  return plain(out) && aligned(out) && out.scalar_type() == a.scalar_type() && out.stride(0) >= out.size(1);
+  return plain(out) && aligned(out) && out.scalar_type() == a.scalar_type() && row_stride(out) >= out.size(1);
 }
 
 void ProductList::add(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
@@ -69,7 +73,7 @@ void ProductList::add(int form, const Tensor& a, const Tensor& b, const Tensor& 
   mlts_gemm_product& p = items[count++];
   p = {};
   p.form = form, p.accumulate = accumulate;
-  p.M = z.M, p.N = z.N, p.c = mptr(out), p.ldc = out.size(0) > 1 ? out.stride(0) : z.N;
+  p.M = z.M, p.N = z.N, p.c = mptr(out), p.ldc = row_stride(out);
   add_segment(a, b);
   like = a;
 }

@@ -120,3 +120,22 @@ def test_products_with_segments_in_one_call(dev, dtype, plan):
     rel = 4e-3 if dtype == torch.bfloat16 else 2e-6
     for (_, _, c, _), w in zip(products, want):
         assert (c.double() - w).norm() <= (2 if dtype == torch.bfloat16 else 1) * rel * w.norm()   # bf16: each segment is rounded
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form,M,N,K", [(NT, 72, 64, 136), (NN, 64, 200, 40), (TN, 512, 512, 4096), (NN, 8, 2048, 1000), (NT, 1, 64, 64)])
+def test_product_into_rows_of_a_wider_buffer(dev, dtype, form, M, N, K):
+    """Outputs that are column ranges, also of products whose contraction is split where the output is dense; the columns beside them
+    are not touched.  An output of another shape is refused, on the host."""
+    a, b = operands(form, M, N, K, dtype, dev, K)
+    want, rel = expected(form, a, b), 4e-3 if dtype == torch.bfloat16 else 2e-6
+    for accumulate in (False, True):
+        wide = torch.randn(M, N + 96, generator=torch.Generator().manual_seed(1)).to(dtype).to(dev)
+        before = wide.clone()
+        total = want + before[:, 32:32 + N].double() * accumulate
+        native().product(form, a, b, wide[:, 32:32 + N], accumulate)
+        assert (wide[:, 32:32 + N].double() - total).norm() <= rel * total.norm()
+        assert torch.equal(wide[:, :32], before[:, :32]) and torch.equal(wide[:, 32 + N:], before[:, 32 + N:])
+    for shape in ((M, N + 8), (M + 1, N), (N * M,)):
+        with pytest.raises(ValueError, match="cannot be written"):
+            native().product(form, a, b, torch.zeros(shape, dtype=dtype, device=dev))
