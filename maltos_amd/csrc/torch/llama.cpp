@@ -204,7 +204,7 @@ struct LinearBackward final : Formula {
 bool ordinary(const Tensor& t) { return !has_tangent(t) && !at::isTensorSubclassLike(t); }
 
 Tensor linear(const Tensor& x, const Tensor& weight, bool into_grad) {
-  if (!ordinary(x) || !ordinary(weight)) return at::linear(x, weight);
+  if (!ordinary(x) || !ordinary(weight) || weight.dim() != 2) return at::linear(x, weight);
   std::shared_ptr<LinearBackward> fn;
   if (compute_requires_grad(x, weight)) {
     fn = make_formula<LinearBackward>();

@@ -23,13 +23,15 @@ bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K) {
 }
 
 struct Sizes {
-  int64_t M, N, K;
+  int64_t M, N, K;  // (K as the first operand has it)
   Sizes(int form, const Tensor& a, const Tensor& b)
       : M(form == MLTS_GEMM_TN ? a.size(1) : a.size(0)), N(form == MLTS_GEMM_NT ? b.size(0) : b.size(1)), K(form == MLTS_GEMM_TN ? a.size(0) : a.size(1)) {}
 };
 
 bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
 bool plain(const Tensor& t) { return t.is_cuda() && t.dim() == 2 && (t.stride(1) == 1 || t.size(1) == 1) && !at::isTensorSubclassLike(t); }
+
+bool same_contraction(int form, const Tensor& a, const Tensor& b) { return a.size(form == MLTS_GEMM_TN ? 0 : 1) == b.size(form == MLTS_GEMM_NT ? 1 : 0); }
 
 int64_t row_stride(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : t.size(1); }  // (a single row's stride means nothing)
 
@@ -43,14 +45,16 @@ Tensor library_product(int form, const Tensor& a, const Tensor& b, const Tensor&
 }  // namespace
 
 bool own_product(int form, const Tensor& a, const Tensor& b) {
+  if (!plain(a) || !plain(b) || !same_contraction(form, a, b)) return false;  // (operands that do not match: torch says so)
   const Sizes z(form, a, b);
-  return z.M > 0 && z.N > 0 && z.K > 0 && plain(a) && plain(b) && a.scalar_type() == b.scalar_type() &&
+  return z.M > 0 && z.N > 0 && z.K > 0 && a.scalar_type() == b.scalar_type() &&
          (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) && within_own_range(form, dtype_code(a), z.M, z.N, z.K) &&
          mlts_gemm_supports(form, dtype_code(a), z.M, z.N, z.K, a.stride(0), b.stride(0), z.N) == nullptr && aligned(a) && aligned(b) &&
          !c10::impl::dispatch_mode_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA);
 }
 
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out, bool accumulate) {
+  TORCH_CHECK_VALUE(a.dim() == 2 && b.dim() == 2, "a product takes two matrices, got ", a.sizes(), " and ", b.sizes());
   const Sizes z(form, a, b);
   TORCH_CHECK_VALUE(!out.defined() || (out.dim() == 2 && out.size(0) == z.M && out.size(1) == z.N), "a product of shape [", z.M, ", ", z.N,
                     "] cannot be written to a tensor of shape ", out.sizes());

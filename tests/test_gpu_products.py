@@ -139,3 +139,16 @@ def test_product_into_rows_of_a_wider_buffer(dev, dtype, form, M, N, K):
     for shape in ((M, N + 8), (M + 1, N), (N * M,)):
         with pytest.raises(ValueError, match="cannot be written"):
             native().product(form, a, b, torch.zeros(shape, dtype=dtype, device=dev))
+
+
+@pytest.mark.parametrize("form", [NT, NN, TN])
+@pytest.mark.parametrize("longer", [0, 1])
+def test_operands_that_do_not_match_are_refused(dev, form, longer):
+    """Contractions of different lengths (rows of a wider weight would be in bounds, and a wrong product)."""
+    a, _ = operands(form, 64, 64, 128 if longer == 0 else 64, torch.bfloat16, dev, 1)
+    _, b = operands(form, 64, 64, 128 if longer == 1 else 64, torch.bfloat16, dev, 2)
+    with pytest.raises(RuntimeError):
+        native().product(form, a, b)
+    if form == NT:
+        with pytest.raises(RuntimeError):
+            native().linear(a, b, False)
