@@ -3,9 +3,12 @@
 #include <torch/library.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <iterator>
 #include <list>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -73,10 +76,14 @@ struct PlanEntry {
   Ids ids;
   Tensor plan;
 };
-std::list<PlanEntry>& plan_cache = *new std::list<PlanEntry>;  // (never destroyed: its tensors must not outlive the runtime)
-size_t plan_cache_entries = 8;
+// Forward runs on the caller's thread, backward on autograd's device thread.  A thread that holds the mutex must not wait for Python's
+// interpreter lock, whose holder may be waiting for the mutex: no tensor is made, copied or released under it (one that Python has
+// an object of may need that lock), only references to entries move.
+typedef std::list<std::shared_ptr<const PlanEntry>> PlanList;
+PlanList& plan_cache = *new PlanList;  // (never destroyed: its tensors must not outlive the runtime)
+std::atomic<size_t> plan_cache_entries{8};
 constexpr int64_t kPlanCacheBytes = int64_t{1} << 30;  // most bytes of plans kept (a plan is B * Sq * Sk / 4 bytes)
-std::mutex plan_mutex;  // forward runs on the caller's thread, backward on autograd's device thread
+std::mutex plan_mutex;
 
 bool same_key(const PlanKey& a, const PlanKey& b) { return std::memcmp(&a, &b, sizeof(PlanKey)) == 0; }
 
@@ -98,10 +105,31 @@ PlanKey plan_key(const mlts_attn_shape& s, const Ids& ids, const Tensor& q) {
   return key;
 }
 
-int64_t cached_plan_bytes() {
-  int64_t n = 0;
-  for (const PlanEntry& e : plan_cache) n += e.plan.numel();
-  return n;
+std::shared_ptr<const PlanEntry> find_plan(const PlanKey& key) {
+  std::lock_guard<std::mutex> lock(plan_mutex);
+  for (auto it = plan_cache.begin(); it != plan_cache.end(); ++it)
+    if (same_key((*it)->key, key)) {
+      plan_cache.splice(plan_cache.begin(), plan_cache, it);
+      return *it;
+    }
+  return nullptr;
+}
+
+// the oldest entries beyond the limits, for the caller to release once it has let go of the mutex
+void evict_plans(PlanList& gone) {
+  auto bytes = [] {
+    int64_t n = 0;
+    for (const auto& e : plan_cache) n += e->plan.numel();
+    return n;
+  };
+  while (plan_cache.size() > plan_cache_entries || bytes() > kPlanCacheBytes) gone.splice(gone.begin(), plan_cache, std::prev(plan_cache.end()));
+}
+
+void keep_plan(std::shared_ptr<const PlanEntry> entry) {
+  PlanList gone;
+  std::lock_guard<std::mutex> lock(plan_mutex);
+  plan_cache.push_front(std::move(entry));
+  evict_plans(gone);
 }
 
 void point_at_ids(mlts_attn_shape& s, const Ids& ids) {
@@ -143,24 +171,20 @@ Tensor attach_document_ids(mlts_attn_shape& s, Ids& ids, const Tensor& q, const 
     convert();
     return Tensor();
   }
-  std::lock_guard<std::mutex> lock(plan_mutex);
   const PlanKey key = plan_key(s, ids, q);
-  for (auto it = plan_cache.begin(); it != plan_cache.end(); ++it) {
-    if (!same_key(it->key, key)) continue;
-    if (it != plan_cache.begin()) plan_cache.splice(plan_cache.begin(), plan_cache, it);
-    for (int i = 0; i < 4; ++i) ids.used[i] = it->ids.used[i];
+  if (const std::shared_ptr<const PlanEntry> kept = find_plan(key)) {
+    for (int i = 0; i < 4; ++i) ids.used[i] = kept->ids.used[i];
     point_at_ids(s, ids);
     check_supported(s, who);
-    s.doc_plan = it->plan.const_data_ptr();
-    return it->plan;
+    s.doc_plan = kept->plan.const_data_ptr();
+    return kept->plan;
   }
   convert();
   const int64_t bytes = mlts_attn_doc_plan_bytes(&s);
   if (bytes <= 0 || bytes > kPlanCacheBytes) return Tensor();
   Tensor plan = workspace(bytes, q);
   check(mlts_attn_doc_plan(&s, mptr(plan), bytes, current_stream()));
-  plan_cache.push_front(PlanEntry{key, ids, plan});
-  while (plan_cache.size() > plan_cache_entries || cached_plan_bytes() > kPlanCacheBytes) plan_cache.pop_back();
+  keep_plan(std::make_shared<const PlanEntry>(PlanEntry{key, ids, plan}));
   s.doc_plan = plan.const_data_ptr();
   return plan;
 }
@@ -1021,14 +1045,15 @@ Tensor py_cross_entropy(const Tensor& logits, const Tensor& labels, int64_t igno
 
 size_t set_doc_plan_cache_entries(int64_t n) {
   TORCH_CHECK_VALUE(n >= 0, "the number of cached plans is >= 0");
+  PlanList gone;
   std::lock_guard<std::mutex> lock(plan_mutex);
   const size_t previous = plan_cache_entries;
   plan_cache_entries = static_cast<size_t>(n);
-  while (plan_cache.size() > plan_cache_entries) plan_cache.pop_back();
+  evict_plans(gone);
   return previous;
 }
 void clear_doc_plan_cache() {
-  std::list<PlanEntry> gone;  // freed outside the lock
+  PlanList gone;
   std::lock_guard<std::mutex> lock(plan_mutex);
   gone.swap(plan_cache);
 }

@@ -801,3 +801,44 @@ def test_tensors_of_more_than_two_to_the_31_elements(dev):
     want_o, want_lse = oa.attention_with_lse(qf, kf, vf, oa.causal_mask(64, S, "cpu"))
     check(o[sl][:, :, -64:], want_o, torch.bfloat16, "last rows O")
     assert (lse[sl][:, :, -64:].cpu() - want_lse).abs().max() <= 1e-4
+
+
+def test_document_plans_are_evicted_while_another_thread_runs(dev):
+    """Two threads attend under ids of their own, more sets of them than plans are kept, and let go of the id tensors at once, so that
+    an evicted plan holds their last references.  Each releases the interpreter lock inside the calls (the backward, the allocator):
+    whoever evicts must not hold the cache's lock while it waits for the interpreter's."""
+    import threading
+
+    B, H, S, D, rounds = 1, 2, 64, 64, 40
+    failures = []
+
+    def work(seed):
+        try:
+            gen = torch.Generator().manual_seed(seed)
+            with torch.cuda.stream(torch.cuda.Stream(dev)):
+                q, k, v, do = (bshd(B, H, S, D, gen, torch.bfloat16).to(dev) for _ in range(4))
+                q, k, v = (t.requires_grad_(True) for t in (q, k, v))
+                first = None
+                for _ in range(rounds):
+                    pos, seq = torch.arange(S, device=dev).expand(B, S).contiguous(), torch.zeros(B, S, dtype=torch.long, device=dev)
+                    o = ops.attention(q, k, v, mask_mode=ops.MASK_DOC, q_pos=pos, k_pos=pos, q_seq=seq, k_seq=seq)
+                    del pos, seq
+                    (dq,) = torch.autograd.grad(o, q, do)
+                    first = dq if first is None else first
+                    assert torch.equal(dq, first)
+                torch.cuda.current_stream().synchronize()
+        except Exception as error:   # (reported by the test's own thread)
+            failures.append(error)
+
+    previous = ops.set_doc_plan_cache_entries(1)
+    try:
+        threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=40)
+        assert not any(t.is_alive() for t in threads), "a thread is stuck"
+        assert not failures, failures
+        assert len(ops._DOC_PLAN_CACHE) <= 1
+    finally:
+        ops.set_doc_plan_cache_entries(previous)
