@@ -61,7 +61,8 @@ OptTensor ids32(const OptTensor& t, int64_t batch, int64_t seq, const char* what
 // later calls with the same ids.  "The same" is judged without reading device memory: same address, dtype, shape, strides
 // and autograd version of the four id tensors as given by the caller, which are kept alive with the plan so that their
 // addresses cannot be handed to other tensors meanwhile (an in-place change of the ids through torch bumps the version;
-// writes behind torch's back are not seen: clear_doc_plan_cache()).  The int32 forms of the ids are kept with it.
+// writes behind torch's back are not seen: clear_doc_plan_cache()).  The int32 forms of the ids are kept with it, also for calls
+// that have no plan (fp32, other head dims), if they had to be made.
 struct PlanKey {
   int64_t shape[7];
   int64_t device;
@@ -119,7 +120,7 @@ std::shared_ptr<const PlanEntry> find_plan(const PlanKey& key) {
 void evict_plans(PlanList& gone) {
   auto bytes = [] {
     int64_t n = 0;
-    for (const auto& e : plan_cache) n += e->plan.numel();
+    for (const auto& e : plan_cache) n += e->plan.defined() ? e->plan.numel() : 0;
     return n;
   };
   while (plan_cache.size() > plan_cache_entries || bytes() > kPlanCacheBytes) gone.splice(gone.begin(), plan_cache, std::prev(plan_cache.end()));
@@ -176,12 +177,17 @@ Tensor attach_document_ids(mlts_attn_shape& s, Ids& ids, const Tensor& q, const 
     for (int i = 0; i < 4; ++i) ids.used[i] = kept->ids.used[i];
     point_at_ids(s, ids);
     check_supported(s, who);
-    s.doc_plan = kept->plan.const_data_ptr();
+    if (kept->plan.defined()) s.doc_plan = kept->plan.const_data_ptr();
     return kept->plan;
   }
   convert();
   const int64_t bytes = mlts_attn_doc_plan_bytes(&s);
-  if (bytes <= 0 || bytes > kPlanCacheBytes) return Tensor();
+  if (bytes <= 0 || bytes > kPlanCacheBytes) {
+    bool converted = false;
+    for (int i = 0; i < 4; ++i) converted = converted || !ids.used[i]->is_same(*ids.given[i]);
+    if (converted) keep_plan(std::make_shared<const PlanEntry>(PlanEntry{key, ids, Tensor()}));
+    return Tensor();
+  }
   Tensor plan = workspace(bytes, q);
   check(mlts_attn_doc_plan(&s, mptr(plan), bytes, current_stream()));
   keep_plan(std::make_shared<const PlanEntry>(PlanEntry{key, ids, plan}));
@@ -1059,7 +1065,7 @@ void clear_doc_plan_cache() {
 }
 size_t doc_plan_cache_size() {
   std::lock_guard<std::mutex> lock(plan_mutex);
-  return plan_cache.size();
+  return std::count_if(plan_cache.begin(), plan_cache.end(), [](const auto& e) { return e->plan.defined(); });
 }
 
 }  // namespace

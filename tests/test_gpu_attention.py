@@ -842,3 +842,34 @@ def test_document_plans_are_evicted_while_another_thread_runs(dev):
         assert len(ops._DOC_PLAN_CACHE) <= 1
     finally:
         ops.set_doc_plan_cache_entries(previous)
+
+
+@pytest.mark.parametrize("dtype,head_dim", [(torch.float32, 64), (torch.bfloat16, 32)])
+def test_int64_ids_are_converted_once_per_batch(dev, dtype, head_dim):
+    """Kernels without a document plan read the ids themselves: their int32 form is made once for all layers, forward and backward,
+    and made again when the ids change in place."""
+    from torch.profiler import ProfilerActivity, profile
+
+    from maltos_amd.llama import LlamaConfig, LlamaForCausalLM
+
+    cfg = LlamaConfig(vocab_size=128, hidden_size=2 * head_dim, intermediate_size=344, num_hidden_layers=3, num_attention_heads=2,
+                      max_position_embeddings=64)
+    torch.manual_seed(3)
+    model = LlamaForCausalLM(cfg).to(dev).to(dtype)
+    ids = torch.randint(0, 128, (2, 50), generator=torch.Generator().manual_seed(1)).to(dev)
+    batch = {"input_ids": ids, "labels": ids.clone(), "position_ids": (torch.arange(50, device=dev) % 20).expand(2, 50).contiguous(),
+             "sequence_ids": (torch.arange(50, device=dev) // 20).expand(2, 50).contiguous()}
+
+    def conversions():
+        with profile(activities=[ProfilerActivity.CPU]) as prof:
+            loss = model(batch)
+            loss.backward()
+        return sum(e.count for e in prof.key_averages() if e.key == "aten::_to_copy"), loss.item()
+
+    # positions and sequence ids for the attention, positions for the rotation
+    assert conversions()[0] <= 3
+    assert conversions()[0] == 0
+    first = conversions()[1]
+    batch["sequence_ids"].zero_()
+    count, loss = conversions()
+    assert 1 <= count <= 3 and loss != first
