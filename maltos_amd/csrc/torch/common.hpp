@@ -65,6 +65,8 @@ inline const void* ptr(const Tensor& t) { return t.const_data_ptr(); }
 inline void* mptr(const Tensor& t) { return t.mutable_data_ptr(); }
 inline const void* ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->const_data_ptr() : nullptr; }
 
+inline bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }  // to 16-byte accesses
+
 inline Tensor workspace(int64_t bytes, const Tensor& like) {
   if (bytes <= 0) return Tensor();
   return at::empty({bytes}, like.options().dtype(at::kByte));

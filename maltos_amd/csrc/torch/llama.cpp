@@ -231,10 +231,10 @@ struct EmbeddingBackward final : Formula {
     if (!g[0].defined()) return {Tensor()};
     const Tensor &w = s[W], ids = dense(s[IDS].scalar_type() == at::kLong ? s[IDS] : s[IDS].to(at::kLong)), dy = dense(g[0]);
     const int64_t n = ids.numel(), vocab = w.size(0), hidden = w.size(1);
-    if ((w.scalar_type() != at::kBFloat16 && w.scalar_type() != at::kFloat) || dy.scalar_type() != w.scalar_type() ||
-        mlts_embedding_bwd_supports(n, hidden, vocab, dtype_code(w)) != nullptr)
-      return {at::embedding_dense_backward(dy, ids, vocab, -1, false)};
     const Tensor grad = bound_grad(w, into_grad);
+    if ((w.scalar_type() != at::kBFloat16 && w.scalar_type() != at::kFloat) || dy.scalar_type() != w.scalar_type() ||
+        mlts_embedding_bwd_supports(n, hidden, vocab, dtype_code(w)) != nullptr || !aligned(dy) || (grad.defined() && !aligned(grad)))
+      return {at::embedding_dense_backward(dy, ids, vocab, -1, false)};
     Tensor dw = grad.defined() ? grad : at::zeros({vocab, hidden}, w.options());
     check(mlts_embedding_bwd(ids.const_data_ptr<int64_t>(), ptr(dy), mptr(dw), n, hidden, vocab, dtype_code(w), current_stream()));
     if (!grad.defined()) return {dw};

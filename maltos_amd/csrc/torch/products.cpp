@@ -28,7 +28,6 @@ struct Sizes {
       : M(form == MLTS_GEMM_TN ? a.size(1) : a.size(0)), N(form == MLTS_GEMM_NT ? b.size(0) : b.size(1)), K(form == MLTS_GEMM_TN ? a.size(0) : a.size(1)) {}
 };
 
-bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
 bool plain(const Tensor& t) { return t.is_cuda() && t.dim() == 2 && (t.stride(1) == 1 || t.size(1) == 1) && !at::isTensorSubclassLike(t); }
 
 bool same_contraction(int form, const Tensor& a, const Tensor& b) { return a.size(form == MLTS_GEMM_TN ? 0 : 1) == b.size(form == MLTS_GEMM_NT ? 1 : 0); }

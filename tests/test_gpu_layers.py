@@ -579,6 +579,25 @@ def test_embedding_gradient(dev, dtype, n, hidden, vocab, common):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("where", ["gradient", "buffer"])
+def test_embedding_gradient_at_any_alignment(dev, dtype, where):
+    """An incoming gradient or a bound buffer off a 16-byte boundary is served, by torch's kernel."""
+    from maltos_amd._native import native
+    gen = torch.Generator().manual_seed(7)
+    n, hidden, vocab = 100, 64, 40
+    ids, dy = torch.randint(0, vocab, (n,), generator=gen), torch.randn(n, hidden, generator=gen).to(dtype)
+    want = torch.zeros(vocab, hidden, dtype=torch.float64).index_add_(0, ids, dy.double())
+    off = lambda shape: torch.zeros(shape[0] * shape[1] + 1, dtype=dtype, device=dev)[1:].view(shape)
+    w = torch.zeros(vocab, hidden, dtype=dtype, device=dev, requires_grad=True)
+    if where == "buffer":
+        w.grad = off((vocab, hidden))
+        native().embedding(w, ids.to(dev), True).backward(dy.to(dev))
+    else:
+        native().embedding(w, ids.to(dev), False).backward(off((n, hidden)).copy_(dy))
+    assert (w.grad.cpu().double() - want).norm() <= (3e-3 if dtype == torch.bfloat16 else 1e-6) * want.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_norm_embedding_and_head_gradients_into_buffers(dev, dtype):
     """With gradient buffers bound, their gradients are autograd's; a weight with a tensor hook stays with autograd."""
     from maltos_amd.llama import LlamaConfig, LlamaForCausalLM, set_grad_accumulation_into_buffers
