@@ -152,9 +152,10 @@ Tensor project(const Tensor& x, const Tensor& weight) {
   return product(MLTS_GEMM_NT, rows2d(x), weight).view(shape);
 }
 
-// dx = dy2 w and dw = dy2^T x2 (added into `grad` if that is defined, and then not returned): in one launch where both run on
-// the own kernels, as neither fills the chip at the sizes they are used for
-std::pair<Tensor, Tensor> input_and_weight_grad(const Tensor& dy2, const Tensor& w, const Tensor& x2, const Tensor& grad) {
+// dx = dy2 w and dw = dy2^T x2 (added into `grad` if that is defined, and then not returned), those of them that are needed: in one
+// launch where both run on the own kernels, as neither fills the chip at the sizes they are used for
+std::pair<Tensor, Tensor> input_and_weight_grad(const Tensor& dy2, const Tensor& w, const Tensor& x2, const Tensor& grad, bool need_dx, bool need_dw) {
+  if (!need_dx || !need_dw) return {need_dx ? product(MLTS_GEMM_NN, dy2, w) : Tensor(), need_dw ? weight_grad(x2, dy2, grad) : Tensor()};
   if (own_product(MLTS_GEMM_NN, dy2, w) && own_product(MLTS_GEMM_TN, dy2, x2) && (!grad.defined() || own_output(grad, x2))) {
     Tensor dx = at::empty({dy2.size(0), w.size(1)}, dy2.options());
     Tensor dw = grad.defined() ? grad : at::empty(w.sizes(), dy2.options());
@@ -176,21 +177,11 @@ struct LinearBackward final : Formula {
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     const Tensor &x = s[X], &w = s[W], &dy = g[0];
     if (!dy.defined()) return {Tensor(), Tensor()};
-    Tensor dx, dw;
-    const Tensor dy2 = rows2d(dy);
     const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
     const Tensor grad = need_dw ? bound_grad(w, into_grad) : Tensor();
-    if (need_dx && need_dw) {
-      std::tie(dx, dw) = input_and_weight_grad(dy2, w, rows2d(x), grad);
-      dx = dx.view(x.sizes());
-    } else if (need_dx) {
-      dx = product(MLTS_GEMM_NN, dy2, w).view(x.sizes());
-    }
-    if (need_dw) {
-      if (!need_dx) dw = weight_grad(rows2d(x), dy2, grad);
-      if (grad.defined()) notify_grad_written(w);  // autograd's hooks on the weight see no gradient for what was added here
-    }
-    return {dx, dw};
+    auto [dx, dw] = input_and_weight_grad(rows2d(dy), w, rows2d(x), grad, need_dx, need_dw);
+    if (grad.defined()) notify_grad_written(w);  // autograd's hooks on the weight see no gradient for what was added here
+    return {need_dx ? dx.view(x.sizes()) : dx, dw};
   }
   variable_list recorded_backward(variable_list&& g, const std::vector<Tensor>& s) override {
     const Tensor &x = s[X], &w = s[W], &dy = g[0];
@@ -278,10 +269,11 @@ struct Adjacent {
   std::vector<size_t> order;         // parameters by output column
   int64_t width = 0;                 // their rows together
   bool similar = false;              // not adjacent, but of one input width and type: may run as a group
-  std::vector<std::pair<const void*, const void*>> key;  // addresses of the parameters and their gradients this was made for
+  typedef std::tuple<const void*, const void*, bool> Key;  // addresses of a parameter and its gradient, whether it is trained
+  std::vector<Key> key;                                    // what this was made for
 
   explicit Adjacent(const std::vector<Tensor>& params) {
-    for (const Tensor& p : params) key.push_back(addresses(p));
+    for (const Tensor& p : params) key.push_back(key_of(p));
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     const Tensor& p0 = params[0];
     for (const Tensor& p : params)
@@ -294,12 +286,12 @@ struct Adjacent {
     for (const Tensor& p : params)
       if (!p.requires_grad()) return;
     std::vector<size_t> in_order = order;
-    std::sort(in_order.begin(), in_order.end(), [&](size_t i, size_t j) { return key[i].first < key[j].first; });
+    std::sort(in_order.begin(), in_order.end(), [&](size_t i, size_t j) { return address(i) < address(j); });
     std::vector<int64_t> at(params.size());
     int64_t rows = 0;
-    const char* next = static_cast<const char*>(key[in_order[0]].first);
+    const char* next = static_cast<const char*>(address(in_order[0]));
     for (size_t i : in_order) {
-      if (key[i].first != next || !params[i].storage().is_alias_of(p0.storage())) return;
+      if (address(i) != next || !params[i].storage().is_alias_of(p0.storage())) return;
       at[i] = rows;
       rows += params[i].size(0);
       next += params[i].nbytes();
@@ -312,20 +304,21 @@ struct Adjacent {
     for (size_t i : order) {
       const Tensor& g = params[i].grad();
       if (!g.defined() || !g.is_contiguous() || g.scalar_type() != p0.scalar_type() || g.sizes() != params[i].sizes() ||
-          (next && key[i].second != next) || !g.storage().is_alias_of(g0.storage()))
+          (next && std::get<1>(key[i]) != next) || !g.storage().is_alias_of(g0.storage()))
         return;
-      next = static_cast<const char*>(key[i].second) + g.nbytes();
+      next = static_cast<const char*>(std::get<1>(key[i])) + g.nbytes();
     }
     grad = g0.as_strided(weight.sizes(), weight.strides(), g0.storage_offset());
   }
-  static std::pair<const void*, const void*> addresses(const Tensor& p) {
+  const void* address(size_t i) const { return std::get<0>(key[i]); }
+  static Key key_of(const Tensor& p) {
     const Tensor& g = p.grad();
-    return {p.const_data_ptr(), g.defined() ? g.const_data_ptr() : nullptr};
+    return {p.const_data_ptr(), g.defined() ? g.const_data_ptr() : nullptr, p.requires_grad()};
   }
   bool made_for(const std::vector<Tensor>& params) const {
     if (params.size() != key.size()) return false;
     for (size_t i = 0; i < params.size(); ++i)
-      if (addresses(params[i]) != key[i]) return false;
+      if (key_of(params[i]) != key[i]) return false;
     return true;
   }
 };
@@ -384,53 +377,61 @@ bool share_memory(const Tensor& a, const Tensor& b) {
   return pa < pb + b.nbytes() && pb < pa + a.nbytes();
 }
 
-// The input gradient (if asked for), then one gradient per parameter: added into the gradient buffers where into_grad allows it,
-// and then undefined.  dy2: the outputs' gradients side by side.
-variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, bool need_dx, const Tensor& x, const Tensor& dy2) {
+// Which gradients a pass asks for: of the input, of the weights that read it (frozen ones are not asked for)
+struct Needed {
+  bool input = false, any_weight = false, all_weights = true;
+  std::vector<bool> weight;
+};
+
+// The input gradient, then one gradient per parameter, as far as they are needed: added into the gradient buffers where into_grad
+// allows it, and then undefined.  dy2: the outputs' gradients side by side.
+variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, const Needed& need, const Tensor& x, const Tensor& dy2) {
   variable_list out(1 + weights.size());
   const Tensor x2 = rows2d(x);
-  if (a.weight.defined()) {
-    const Tensor grad = into_grad && !at::GradMode::is_enabled() ? a.grad : Tensor();
+  const bool one_matrix = a.weight.defined();
+  if (one_matrix && (need.all_weights || !need.any_weight)) {
+    const Tensor grad = need.any_weight && into_grad && !at::GradMode::is_enabled() ? a.grad : Tensor();
     Tensor dw;
-    if (need_dx) std::tie(out[0], dw) = input_and_weight_grad(dy2, a.weight, x2, grad);
-    else dw = weight_grad(x2, dy2, grad);
+    std::tie(out[0], dw) = input_and_weight_grad(dy2, a.weight, x2, grad, need.input, need.any_weight);
     for (size_t i = 0; i < weights.size(); ++i) {
       if (grad.defined()) notify_grad_written(weights[i]);
-      else out[1 + i] = dw.narrow(0, a.first[i], weights[i].size(0));
+      else if (dw.defined()) out[1 + i] = dw.narrow(0, a.first[i], weights[i].size(0));
     }
   } else {
     std::vector<Tensor> parts, into;
-    bool own = true;
+    bool own = !one_matrix;
     for (size_t i = 0; i < weights.size(); ++i) {
       parts.push_back(dy2.narrow(1, a.first[i], weights[i].size(0)));
-      into.push_back(bound_grad(weights[i], into_grad && weights[i].requires_grad()));
+      into.push_back(need.weight[i] ? bound_grad(weights[i], into_grad) : Tensor());
       own = own && own_product(MLTS_GEMM_NN, parts[i], weights[i]) && own_product(MLTS_GEMM_TN, parts[i], x2) &&
             (!into[i].defined() || own_output(into[i], x2));
     }
     if (own) {
       ProductList list;
       for (size_t i = 0; i < weights.size(); ++i) {
+        if (!need.weight[i]) continue;
         Tensor dw = into[i].defined() ? into[i] : at::empty(weights[i].sizes(), dy2.options());
         // two projections with one weight add into the same buffer: one launch after the other
         if (std::any_of(into.begin(), into.begin() + i, [&](const Tensor& before) { return share_memory(before, into[i]); })) list.run(), list = {};
         list.add(MLTS_GEMM_TN, parts[i], x2, dw, into[i].defined());
         if (!into[i].defined()) out[1 + i] = dw;
       }
-      if (need_dx) {
+      if (need.input) {
         out[0] = at::empty(x2.sizes(), dy2.options());
         for (size_t i = weights.size(); i-- > 0;) {  // last one first: the order in which autograd adds them up
           if (i + 1 == weights.size()) list.add(MLTS_GEMM_NN, parts[i], weights[i], out[0], false);
           else list.add_segment(parts[i], weights[i]);
         }
       }
-      list.run();
+      if (list.count) list.run();
     } else {
+      if (need.input && one_matrix) out[0] = product(MLTS_GEMM_NN, dy2, a.weight);
       for (size_t i = weights.size(); i-- > 0;) {
-        if (need_dx) {
+        if (need.input && !one_matrix) {
           Tensor dx = product(MLTS_GEMM_NN, parts[i], weights[i]);
           out[0] = out[0].defined() ? out[0].add_(dx) : dx;
         }
-        out[1 + i] = weight_grad(x2, parts[i], into[i]);
+        if (need.weight[i]) out[1 + i] = weight_grad(x2, parts[i], into[i]);
       }
     }
     for (size_t i = 0; i < weights.size(); ++i)
@@ -440,12 +441,26 @@ variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights
   return out;
 }
 
-struct AdjacentLinearsBackward final : Formula {
-  enum { X, COUNT };
+// A formula whose first outputs are the gradients of the shared input and of the weights that read it
+struct SharedInputFormula : public Formula {
   AdjacentPtr rows;
   bool into_grad = false;
   std::vector<Tensor> weights;
-  AdjacentLinearsBackward() : Formula(COUNT) {}
+  using Formula::Formula;
+  Needed needed() const {
+    Needed n;
+    n.input = task_should_compute_output(0);
+    for (size_t i = 0; i < weights.size(); ++i) {
+      n.weight.push_back(task_should_compute_output(1 + i));
+      n.any_weight = n.any_weight || n.weight[i], n.all_weights = n.all_weights && n.weight[i];
+    }
+    return n;
+  }
+};
+
+struct AdjacentLinearsBackward final : SharedInputFormula {
+  enum { X, COUNT };
+  AdjacentLinearsBackward() : SharedInputFormula(COUNT) {}
   std::string name() const override { return "MaltosAdjacentLinearsBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     bool all = true, any = false;
@@ -470,7 +485,7 @@ struct AdjacentLinearsBackward final : Formula {
         else part.zero_();
       }
     }
-    return grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dy2);
+    return grads_of_all(*rows, weights, into_grad, needed(), s[X], dy2);
   }
 };
 
@@ -516,18 +531,15 @@ std::vector<Tensor> adjacent_linears(const Tensor& x, const AdjacentPtr& rows, c
 
 // round(silu(x W_gate^T)) * (x W_up^T) (models/llama.py:205-206) with the two projections as one product; the backward
 // writes d gate and d up side by side, so that the input gradient is one product as well
-struct GateUpBackward final : Formula {
+struct GateUpBackward final : SharedInputFormula {
   enum { X, GU, COUNT };
-  AdjacentPtr rows;
-  bool into_grad = false;
-  std::vector<Tensor> weights;
-  GateUpBackward() : Formula(COUNT) {}
+  GateUpBackward() : SharedInputFormula(COUNT) {}
   std::string name() const override { return "MaltosGateUpBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(3);
     const Tensor dgu = swiglu_rows_backward(g[0], dense(s[GU]), rows->first[0], rows->first[1], weights[0].size(0));
     const Tensor dgu2 = rows2d(dgu);
-    return grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dgu2);
+    return grads_of_all(*rows, weights, into_grad, needed(), s[X], dgu2);
   }
 };
 
@@ -632,28 +644,33 @@ bool recorded(const Tensor& x, const BlockWeights& w) {
   return at::GradMode::is_enabled() && (compute_requires_grad(x, w.out) || any_requires_grad(w.in));
 }
 
-// The last projection of a block: the gradients of its input and weight
-std::pair<Tensor, Tensor> output_grads(const Tensor& dy, const Tensor& w, const Tensor& rows, bool into_grad) {
-  const Tensor grad = bound_grad(w, into_grad && w.requires_grad());
-  auto grads = input_and_weight_grad(rows2d(dense(dy)), w, rows, grad);
-  if (grad.defined()) notify_grad_written(w);
-  return grads;
-}
+// A formula of a whole block: the last output is the gradient of the last projection's weight
+struct BlockFormula : public SharedInputFormula {
+  bool into_grad_out = false;
+  using SharedInputFormula::SharedInputFormula;
+  // the last projection: the gradients of its input (if something in front of it needs one) and of its weight
+  std::pair<Tensor, Tensor> output_grads(const Tensor& dy, const Tensor& w, const Tensor& rows, const Needed& in) const {
+    const bool need_dw = task_should_compute_output(1 + weights.size());
+    const Tensor grad = need_dw ? bound_grad(w, into_grad_out) : Tensor();
+    auto grads = input_and_weight_grad(rows2d(dense(dy)), w, rows, grad, in.input || in.any_weight, need_dw);
+    if (grad.defined()) notify_grad_written(w);
+    return grads;
+  }
+};
 
-struct AttentionBlockBackward final : Formula {
+struct AttentionBlockBackward final : BlockFormula {
   enum { X, Q, K, V, OUT, LSE, COS, SIN, ROPE_POSITIONS, POSITIONS, SEQUENCES, OUT_W, COUNT };
-  AdjacentPtr rows;
-  std::vector<Tensor> weights;
-  bool into_grad = false, into_grad_out = false;
   int64_t position_offset = 0, mask_mode = 0;
   double scale = 0;
-  AttentionBlockBackward() : Formula(COUNT) {}
+  AttentionBlockBackward() : BlockFormula(COUNT) {}
   std::string name() const override { return "MaltosAttentionBlockBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(5);
     const Tensor &q = s[Q], &k = s[K];
     const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
-    auto [dvo, dwo] = output_grads(g[0], s[OUT_W], as_rows(s[OUT]), into_grad_out);
+    const Needed need = needed();
+    auto [dvo, dwo] = output_grads(g[0], s[OUT_W], as_rows(s[OUT]), need);
+    if (!dvo.defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), dwo};
     const OptTensor pos = optional_tensor(s[POSITIONS]), seq = optional_tensor(s[SEQUENCES]);
     auto [dq, dk, dv] = attention_backward(as_heads(dvo, B, S, H * D, 0, H, D), q, k, s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq);
     rope_pair(dq, dk, s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset, true, true);
@@ -664,7 +681,7 @@ struct AttentionBlockBackward final : Formula {
       for (size_t i : rows->order) ordered.push_back(parts[i]);
       dqkv = at::cat(ordered, 1);
     }
-    variable_list out = grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], dqkv);
+    variable_list out = grads_of_all(*rows, weights, into_grad, need, s[X], dqkv);
     out.push_back(dwo);
     return out;
   }
@@ -701,18 +718,17 @@ Tensor attention_block(const Tensor& x, const BlockWeights& w, int64_t heads, in
   return y;
 }
 
-struct MlpBlockBackward final : Formula {
+struct MlpBlockBackward final : BlockFormula {
   enum { X, GU, H, OUT_W, COUNT };
-  AdjacentPtr rows;
-  std::vector<Tensor> weights;
-  bool into_grad = false, into_grad_out = false;
-  MlpBlockBackward() : Formula(COUNT) {}
+  MlpBlockBackward() : BlockFormula(COUNT) {}
   std::string name() const override { return "MaltosMlpBlockBackward"; }
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(4);
-    auto [dh, dw] = output_grads(g[0], s[OUT_W], rows2d(s[H]), into_grad_out);
+    const Needed need = needed();
+    auto [dh, dw] = output_grads(g[0], s[OUT_W], rows2d(s[H]), need);
+    if (!dh.defined()) return {Tensor(), Tensor(), Tensor(), dw};
     const Tensor dgu = swiglu_rows_backward(dh.view(s[H].sizes()), dense(s[GU]), rows->first[0], rows->first[1], weights[0].size(0));
-    variable_list out = grads_of_all(*rows, weights, into_grad, task_should_compute_output(0), s[X], rows2d(dgu));
+    variable_list out = grads_of_all(*rows, weights, into_grad, need, s[X], rows2d(dgu));
     out.push_back(dw);
     return out;
   }

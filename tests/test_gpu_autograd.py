@@ -95,3 +95,80 @@ def test_projections_that_share_a_weight_add_both_gradients_into_its_buffer(dev,
             model(batch).backward()
     for (name, p), q in zip(buffers.named_parameters(), plain.parameters()):
         assert (p.grad - q.grad).norm() <= 1e-5 * q.grad.norm(), name   # fp32 sums in another order
+
+
+_FROZEN = {"all": lambda n: True, "projections": lambda n: "_proj" in n, "some": lambda n: "k_proj" in n or "up_proj" in n or "layers.0" in n,
+           "all-but-o": lambda n: "o_proj" not in n and "down_proj" not in n, "all-but-v": lambda n: "layers.1.self_attn.v_proj" not in n}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["layers-at-once", "modules", "into-buffers"])
+@pytest.mark.parametrize("frozen", _FROZEN)
+def test_frozen_weights_get_no_gradient_and_the_others_theirs(dev, dtype, form, frozen):
+    def gradients(model, x):
+        if form == "modules":
+            model.layers[0].register_forward_hook(lambda *a: None)
+        model({"hidden_states": x, "labels": _batch(dev)["labels"]}).backward()
+        return x.grad
+
+    trained, partly = _model(dev, dtype), _model(dev, dtype)
+    for name, p in partly.named_parameters():
+        p.requires_grad_(not _FROZEN[frozen](name))
+    if form == "into-buffers":   # a frozen weight's buffer is left alone
+        for model in (trained, partly):
+            set_grad_accumulation_into_buffers(model)
+            for name, p in model.named_parameters():
+                p.grad = torch.zeros_like(p)
+    hidden = torch.randn(2, 101, 256, generator=torch.Generator().manual_seed(2)).to(dev, dtype)
+    dx, want = (gradients(m, hidden.clone().requires_grad_(True)) for m in (partly, trained))
+    rel = 1e-2 if dtype == torch.bfloat16 else 1e-5   # (other launches add up in another order)
+    assert (dx.double() - want.double()).norm() <= rel * want.double().norm()
+    for (name, p), q in zip(partly.named_parameters(), trained.parameters()):
+        if not p.requires_grad:
+            assert p.grad is None or (p.grad == 0).all(), name
+        elif q.grad is not None:
+            assert (p.grad.double() - q.grad.double()).norm() <= rel * q.grad.double().norm(), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hook", [False, True], ids=["layers-at-once", "modules"])
+def test_frozen_weights_cost_no_products(dev, dtype, hook):
+    """Their gradients are not formed: the backward pass asks for at least their bytes less."""
+    taken = {}
+    for frozen in (False, True):
+        model = _model(dev, dtype)
+        model.layers.requires_grad_(not frozen)
+        if hook:
+            model.layers[0].register_forward_hook(lambda *a: None)
+        hidden = torch.randn(2, 101, 256, generator=torch.Generator().manual_seed(2)).to(dev, dtype).requires_grad_(True)
+        loss = model({"hidden_states": hidden, "labels": _batch(dev)["labels"]})
+        before = torch.cuda.memory_stats()["requested_bytes.all.allocated"]
+        loss.backward()
+        taken[frozen] = torch.cuda.memory_stats()["requested_bytes.all.allocated"] - before
+    size = sum(p.numel() * p.element_size() for p in model.layers.parameters() if p.dim() == 2)
+    assert taken[False] - taken[True] >= size, (taken, size)
+
+
+def test_gradients_of_some_weights_alone(dev):
+    """autograd.grad for one of several projections with adjacent weights: the others' buffers are not written."""
+    from maltos_amd.optim import FusedAdamW, MasterWeightsOptimizer
+
+    model, batch = _model(dev), _batch(dev)
+    opt = MasterWeightsOptimizer(model.parameters(), optimizer_factory=lambda ps: FusedAdamW(ps, lr=1e-3), flat=True)
+    model(batch).backward()
+    names = ["layers.0.self_attn.k_proj.weight", "layers.1.mlp.up_proj.weight", "layers.1.self_attn.o_proj.weight"]
+    weights = dict(model.named_parameters())
+    want = [weights[n].grad.clone() for n in names]
+    opt.zero_grad()
+    got = torch.autograd.grad(model(batch), [weights[n] for n in names])
+    assert (opt.flat_model_grad == 0).all()
+    for name, g, w in zip(names, got, want):
+        assert (g.double() - w.double()).norm() <= 1e-2 * w.double().norm(), name
+    set_grad_accumulation_into_buffers(model)
+    model(batch).backward(inputs=[weights[n] for n in names])
+    for name, p in weights.items():
+        if name in names:
+            w = want[names.index(name)]
+            assert (p.grad.double() - w.double()).norm() <= 1e-2 * w.double().norm(), name
+        else:
+            assert (p.grad == 0).all(), name
