@@ -7,8 +7,11 @@
 // layout of the next product once the contraction index is renumbered, which both operands agree on.
 //
 //  * fp32 runs on v_mfma_f32_16x16x4_f32, true fp32 products and sums at twice the rate of the vector ALU;
-//  * bf16 runs on v_mfma_f32_16x16x32_bf16.  Probabilities and dS enter their second product as the sum of two bf16 values
-//    (hi + lo, 16 significant bits), so results differ from fp32 probabilities only below the rounding of the output.
+//  * bf16 runs on v_mfma_f32_16x16x32_bf16.  Probabilities and dS enter their second product as the sum of three bf16 values of 8
+//    bits each, which is all of an fp32 number: products and sums as with fp32 probabilities.  (Two of them are enough for a bf16
+//    output, but not for gradients added in fp32: 2.5e-6 off the exact ones at S = 777, with three 0.3 to 0.5e-6.  The third
+//    costs a few percent where a kernel is short, 9 to 15 where it fills the chip: 8 x 8 heads x 1024, head_dim 32, forward and
+//    backward 27 + 68 us with two, 30 + 77 with three.)
 //
 // What bounds it: the matrix pipe for long rows (fp32: 32 cycles per 16x16x4; a 32-key unit is 2 * D / 2 of them), the chain
 // of tiles of one workgroup for short ones.  A workgroup is four wavefronts: 64 rows, or, when the grid would leave compute
@@ -70,13 +73,17 @@ struct Tile16<bf16_t, DP> {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
   }
   static __device__ __forceinline__ void accumulate(f32x4 (&acc)[DP / 16], const bf16_t* unit, const f32x4 (&x)[2], int, int l16, int g) {
-    bf16x8 hi, lo;
+    bf16x8 part[3];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        hi[4 * b + i] = static_cast<bf16_t>(x[b][i]);
-        lo[4 * b + i] = static_cast<bf16_t>(x[b][i] - static_cast<float>(hi[4 * b + i]));
+        float rest = x[b][i];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          part[n][4 * b + i] = static_cast<bf16_t>(rest);
+          rest -= static_cast<float>(part[n][4 * b + i]);
+        }
       }
     const bf16_t* src = unit + (4 * g + (l16 >> 2)) * LS + (l16 & 3) * 4;
 #pragma unroll
@@ -84,8 +91,8 @@ struct Tile16<bf16_t, DP> {
       const i16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src + 16 * db));
       const i16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src + 16 * LS + 16 * db));
       const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7));
-      acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, hi, acc[db], 0, 0, 0);
-      acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, lo, acc[db], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, part[n], acc[db], 0, 0, 0);
     }
   }
 };

@@ -873,3 +873,33 @@ def test_int64_ids_are_converted_once_per_batch(dev, dtype, head_dim):
     batch["sequence_ids"].zero_()
     count, loss = conversions()
     assert 1 <= count <= 3 and loss != first
+
+
+def _exact_attention(q, k, v, do, o, causal, scale):
+    """fp64 (lse, dq, dk, dv) on the device; delta from the output `o` that the kernels are handed."""
+    q, k, v, do, o = (t.double().contiguous() for t in (q, k, v, do, o))
+    group = q.size(1) // k.size(1)
+    ke, ve = (t.repeat_interleave(group, dim=1) for t in (k, v))
+    s = (q @ ke.transpose(2, 3).contiguous()) * scale
+    if causal:
+        s = s.masked_fill(torch.ones(s.shape[2:], dtype=torch.bool, device=s.device).triu(1 + s.size(3) - s.size(2)), -float("inf"))
+    p = torch.softmax(s, dim=-1)
+    ds = p * (do @ ve.transpose(2, 3).contiguous() - (do * o).sum(-1, keepdim=True))
+    per_kv = lambda t: t.unflatten(1, (-1, group)).sum(2)
+    return (torch.logsumexp(s, dim=-1), ds @ ke * scale, per_kv(ds.transpose(2, 3).contiguous() @ q) * scale,
+            per_kv(p.transpose(2, 3).contiguous() @ do))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D", [(1, 4, 4, 64, 64, 32), (2, 8, 4, 777, 777, 96), (1, 4, 1, 1024, 2048, 32), (8, 12, 12, 515, 515, 48)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_bf16_gradients_added_in_fp32_keep_fp32_probabilities(dev, B, Hq, Hkv, Sq, Sk, D, causal):
+    """Head dims of the 16-row kernels: probabilities and dS are fp32 numbers in their second product too.  Each term is off by a few
+    2^-24 (the exponential, its argument, the product); 20 of them bound the sums, two bf16 parts alone leave 40."""
+    gen = torch.Generator().manual_seed(Sq + D)
+    q, k, v, do = (bshd(B, h, s, D, gen, torch.bfloat16).to(dev) for h, s in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk), (Hq, Sq)))
+    mode = ops.MASK_CAUSAL if causal else ops.MASK_NONE
+    o, lse = ops.attention_forward(q, k, v, mask_mode=mode)
+    grads = [torch.zeros(t.shape, device=dev) for t in (q, k, v)]
+    ops.attention_backward_accumulate(do, q, k, v, o, lse, *grads, mask_mode=mode)
+    for name, got, want in zip(("dq", "dk", "dv"), grads, _exact_attention(q, k, v, do, o, causal, D ** -0.5)[1:]):
+        assert (got.double() - want).norm() <= 20 * 2.0 ** -24 * want.norm(), name
