@@ -903,3 +903,15 @@ def test_bf16_gradients_added_in_fp32_keep_fp32_probabilities(dev, B, Hq, Hkv, S
     ops.attention_backward_accumulate(do, q, k, v, o, lse, *grads, mask_mode=mode)
     for name, got, want in zip(("dq", "dk", "dv"), grads, _exact_attention(q, k, v, do, o, causal, D ** -0.5)[1:]):
         assert (got.double() - want).norm() <= 20 * 2.0 ** -24 * want.norm(), name
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.float32, 32), (torch.bfloat16, 32), (torch.bfloat16, 96)])
+@pytest.mark.parametrize("S", [64, 777])
+def test_log_sum_exp_of_exact_scores_is_rounded_once(dev, dtype, D, S):
+    """16-row kernels.  Small integers times 1/8: every score and row maximum is an fp32 number, so the LSE may be off by its own rounding
+    and by log(sum), of a sum of at most 777 terms with a few 2^-24 each."""
+    gen = torch.Generator().manual_seed(S + D)
+    q, k = (torch.randint(-9, 10, (2, S, 4, D), generator=gen).to(dtype).transpose(1, 2).to(dev) for _ in range(2))
+    lse = ops.attention_forward(q, k, k, mask_mode=ops.MASK_CAUSAL, scale=0.125)[1].double()
+    want = _exact_attention(q, k, k, q, q, True, 0.125)[0]
+    assert ((lse - want).abs() <= 2.0 ** -24 * want.abs() + 16 * 2.0 ** -24).all(), ((lse - want).abs() / want.abs()).max()
