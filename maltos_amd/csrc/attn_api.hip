@@ -11,8 +11,8 @@ int mlts_attn_bwd_dkdv_bf16_split(AttnBwdParams bp, int D, int mode, void* works
 int mlts_attn_bwd_dq_bf16_tr(const AttnBwdParams& bp, int D, int mode, hipStream_t st);                    // attn_bwd_dq_tr.hip
 int mlts_attn_tile16_fwd(AttnParams p, int D, int dtype, int mode, hipStream_t st);                        // attn_tile16.hip
 int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int dtype, int mode, hipStream_t st);                    // attn_tile16.hip
-int mlts_attn_delta(const void* dout, const int64_t* dos, const void* o, const int64_t* os, float* delta, int B, int H,
-                    int S, int D, int dtype, hipStream_t st);
+int mlts_attn_delta_bf16(const void* dout, const int64_t* dos, const void* o, const int64_t* os, float* delta, int B, int H, int S,
+                         int D, hipStream_t st);                                                            // attn_delta.hip
 
 namespace {
 
@@ -237,7 +237,7 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
   // the recomputing dQ kernel forms delta itself from 16-byte chunks of the O rows
   const bool stats_in_dq = s->Sk > 0 && mlts_aligned16(o) && strides_aligned(s->o_stride, 2);
   if (s->Sq > 0 && !stats_in_dq) {
-    int rc = mlts_attn_delta(dout, do_stride, o, s->o_stride, delta, s->B, s->Hq, s->Sq, s->D, s->dtype, st);
+    int rc = mlts_attn_delta_bf16(dout, do_stride, o, s->o_stride, delta, s->B, s->Hq, s->Sq, s->D, st);
     if (rc != MLTS_OK) return rc;
   }
   return attn_bwd_bf16(bp, s->D, s->mask_mode, delta, lse2_ws, stats_in_dq, st);

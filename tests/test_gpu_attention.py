@@ -915,3 +915,16 @@ def test_log_sum_exp_of_exact_scores_is_rounded_once(dev, dtype, D, S):
     lse = ops.attention_forward(q, k, k, mask_mode=ops.MASK_CAUSAL, scale=0.125)[1].double()
     want = _exact_attention(q, k, k, q, q, True, 0.125)[0]
     assert ((lse - want).abs() <= 2.0 ** -24 * want.abs() + 16 * 2.0 ** -24).all(), ((lse - want).abs() / want.abs()).max()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_output_rows_off_a_16_byte_boundary(dev, D):
+    """The backward of the 32-row kernels forms rowsum(dO * O) in a pass of its own then: fp32 sums in another order."""
+    gen = torch.Generator().manual_seed(D)
+    B, Hq, Hkv, S = 2, 4, 2, 333
+    q, k, v, do = (bshd(B, h, S, D, gen, torch.bfloat16).to(dev) for h in (Hq, Hkv, Hkv, Hq))
+    o, lse = ops.attention_forward(q, k, v, mask_mode=ops.MASK_CAUSAL)
+    moved = torch.empty(B * S * Hq * D + 1, dtype=torch.bfloat16, device=dev)[1:].view(B, S, Hq, D).transpose(1, 2).copy_(o)
+    for got, want in zip(ops.attention_backward(do, q, k, v, moved, lse, mask_mode=ops.MASK_CAUSAL),
+                         ops.attention_backward(do, q, k, v, o, lse, mask_mode=ops.MASK_CAUSAL)):
+        assert (got.double() - want.double()).norm() <= 2.0 ** -9 * want.double().norm()   # a bf16 result may round the other way
