@@ -9,17 +9,25 @@ namespace maltos {
 namespace {
 
 // M * N * K up to which the own kernels run.  A product through torch costs 18 us of host time, a call here 5, and that is what
-// small steps wait for: up to a few thousand rows of a 512-wide model the host is behind the GPU.  There the own kernels are
-// the faster ones on the GPU as well (1023 x 512 x 32000, dx: 45 us against the library's 145; 512-wide: 9 against 12).  From
-// 16384 x 512 x 512 on a step fills the GPU for longer than the host needs, and the library's kernels, with the shipped
-// per-shape selection, are ahead: a training step of that size took 90 us more of 9500 with its 512-wide products done here.
-constexpr double kOwnLimit = 4.0e9;
+// small steps wait for: up to a few thousand rows of a 512-wide model the host is behind the GPU.  On the GPU alone (both sides
+// captured; 256 to 4096 wide, 256 to 16384 rows, own over library's time for all products of a size together, the library's choice
+// untuned) they are ahead of it up to these lines, and behind from there:
+//   bf16  1 to 1.5e9  0.79 (y), 0.80 (dx), 0.79 (dW)    2.5 to 3e9  0.82, 0.85, 0.90    3 to 4e9  0.98, 1.02, 1.07
+//         4 to 5e9    1.14, 0.94, 0.97                  6 to 8e9    1.19, 1.28, 1.07    1.2 to 2e10  1.20, 1.14, 1.13
+//   fp32  0.5 to 1e9  0.86, 0.86, 0.82                  2.5 to 3e9  0.90, 0.92, 0.87    3 to 4e9  1.13, 1.15, 1.17
+// (16384 x 512 x 512: y 16.7 us against 16.1, or 17.6 against 15.0 with the shipped per-shape selection.)
+constexpr double kOwnLimitBf16 = 4.0e9, kOwnLimitF32 = 3.0e9;
 
-// Above it they still run for dx = dy W with so long a contraction that it is split over workgroups (dx of an lm_head): the
-// library does not split those (us, 512 wide, 32000 terms: 1024 rows 47 against 160, 8192 rows 270 against 346).
+// Above it they still run for dx = dy W in bf16 with so long a contraction that it is split over workgroups (dx of an lm_head, of a wide
+// MLP): the library does not split those.  Own over library's time, 256 to 8192 rows, 512 to 4096 wide: 32000 terms 0.17 to 0.79, 11008
+// terms 0.54 to 0.83, 8192 terms 0.42 to 0.98; with 4096 or 5504 terms 0.76 to 1.04 where fewer than 128 tiles of 256 x 128 leave more
+// than half of the CUs idle unsplit, but 1.05 and 1.12 for 128 tiles (2048 x 2048 x 5504 56.6 us against 53.8, 1024 x 4096 x 4096 46.1
+// against 41.1).
 bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K) {
-  return static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K) <= kOwnLimit ||
-         (form == MLTS_GEMM_NN && mlts_gemm_workspace_bytes(form, dtype, M, N, K) > 0);
+  const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
+  if (dtype == MLTS_F32) return size <= kOwnLimitF32;
+  if (size <= kOwnLimitBf16) return true;
+  return form == MLTS_GEMM_NN && (K >= 8192 || M * N < 128 * 256 * 128) && mlts_gemm_workspace_bytes(form, dtype, M, N, K) > 0;
 }
 
 struct Sizes {
