@@ -269,8 +269,10 @@ struct Adjacent {
   std::vector<size_t> order;         // parameters by output column
   int64_t width = 0;                 // their rows together
   bool similar = false;              // not adjacent, but of one input width and type: may run as a group
-  typedef std::tuple<const void*, const void*, bool> Key;  // addresses of a parameter and its gradient, whether it is trained
-  std::vector<Key> key;                                    // what this was made for
+  // of a parameter: its address and that of its gradient, whether it is trained, its shape and type (another one may come to lie at an
+  // address that was given back)
+  typedef std::tuple<const void*, const void*, bool, int64_t, int64_t, c10::ScalarType> Key;
+  std::vector<Key> key;  // what this was made for
 
   explicit Adjacent(const std::vector<Tensor>& params) {
     for (const Tensor& p : params) key.push_back(key_of(p));
@@ -313,7 +315,7 @@ struct Adjacent {
   const void* address(size_t i) const { return std::get<0>(key[i]); }
   static Key key_of(const Tensor& p) {
     const Tensor& g = p.grad();
-    return {p.const_data_ptr(), g.defined() ? g.const_data_ptr() : nullptr, p.requires_grad()};
+    return {p.const_data_ptr(), g.defined() ? g.const_data_ptr() : nullptr, p.requires_grad(), p.dim() == 2 ? p.size(0) : -1, p.numel(), p.scalar_type()};
   }
   bool made_for(const std::vector<Tensor>& params) const {
     if (params.size() != key.size()) return false;

@@ -118,3 +118,12 @@ def test_tangents_through_rotations_and_joint_projections_raise():
                      lambda: native().adjacent_linears(rows, group, [torch.empty(4, 6)], False), lambda: native().gate_up(rows, group, [torch.empty(4, 6)], False)):
             with pytest.raises(NotImplementedError, match="forward-mode"):
                 call()
+
+
+def test_kept_rows_belong_to_parameters_of_one_shape_and_type():
+    """What a module keeps about its projections is made anew when another parameter lies at the address of an old one."""
+    memory = torch.zeros(64)
+    group = native().Adjacent([memory.view(8, 8)])
+    assert group.made_for([memory.view(8, 8)])
+    for other in (memory.view(4, 16), memory.view(16, 4), memory[:32].view(4, 8), memory.view(torch.int32).view(8, 8), memory.view(8, 8).requires_grad_(True)):
+        assert not group.made_for([other])
