@@ -448,8 +448,13 @@ struct SharedInputFormula : public Formula {
   AdjacentPtr rows;
   bool into_grad = false;
   std::vector<Tensor> weights;
+  std::vector<int64_t> versions;  // of the weights as the forward pass read them
   using Formula::Formula;
   Needed needed() const {
+    for (size_t i = 0; i < versions.size(); ++i)
+      TORCH_CHECK(weights[i]._version() == versions[i], name(), ": a weight of shape ", weights[i].sizes(),
+                  " needed for gradient computation has been modified by an inplace operation: it is at version ", weights[i]._version(),
+                  "; expected version ", versions[i], " instead");
     Needed n;
     n.input = task_should_compute_output(0);
     for (size_t i = 0; i < weights.size(); ++i) {
@@ -512,6 +517,9 @@ std::shared_ptr<F> adjacent_formula(const Tensor& x, const AdjacentPtr& rows, co
   fn->set_next_edges(std::move(edges));
   fn->save(fn->X, x);
   fn->rows = rows, fn->weights = weights, fn->into_grad = into_grad;
+  // (adjacent parameters are views that flat optimizer layouts write to as one buffer: their versions say nothing)
+  if (!rows->weight.defined())
+    for (const Tensor& w : weights) fn->versions.push_back(w._version());
   return fn;
 }
 

@@ -172,3 +172,16 @@ def test_gradients_of_some_weights_alone(dev):
             assert (p.grad.double() - w.double()).norm() <= 1e-2 * w.double().norm(), name
         else:
             assert (p.grad == 0).all(), name
+
+
+@pytest.mark.parametrize("form", ["layers-at-once", "modules"])
+@pytest.mark.parametrize("name", ["self_attn.q_proj", "self_attn.o_proj", "mlp.up_proj", "mlp.down_proj", "input_layernorm"])
+def test_weights_modified_between_forward_and_backward_are_noticed(dev, form, name):
+    model, batch = _model(dev), _batch(dev)
+    if form == "modules":
+        model.layers[0].register_forward_hook(lambda *a: None)
+    loss = model(batch)
+    with torch.no_grad():
+        model.get_submodule("layers.1." + name).weight.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
