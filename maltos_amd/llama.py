@@ -70,8 +70,13 @@ def _fused_rows(holder: nn.Module, modules: list[nn.Module], params: list[nn.Par
         rows = holder.__dict__["_maltos_hip_fused_rows"] = native().Adjacent(params)
     if rows.adjacent:
         return rows
-    plain = all(type(m) is HipLinear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks) for m in modules)
-    return rows if plain and rows.runs_as_group(x, params) else None
+    return rows if all(_plain_linear(m) for m in modules) and rows.runs_as_group(x, params) else None
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """Whether calling the module is the product with its weight and nothing else."""
+    return (type(m) is HipLinear and HipLinear.forward is _STOCK_METHODS[HipLinear, "forward"] and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
 
 
 def _adjacent_columns(parts: list[torch.Tensor]) -> torch.Tensor | None:
@@ -322,6 +327,8 @@ class LlamaDecoderLayer(nn.Module):
 # what native().run_layers takes a layer apart into
 _STOCK_MODULES = {"layer": LlamaDecoderLayer, "attention": LlamaAttention, "core": HipAttentionCore, "rotary": LlamaRotaryEmbedding,
                   "mlp": LlamaMLP, "norm": LlamaRMSNorm, "linear": HipLinear}
+# ... as long as nobody has put another method in the place of one of theirs
+_STOCK_METHODS = {(cls, name): getattr(cls, name) for cls in _STOCK_MODULES.values() for name in ("forward", "row_ids", "tables") if hasattr(cls, name)}
 
 
 class LlamaForCausalLM(nn.Module):
@@ -394,6 +401,8 @@ class LlamaForCausalLM(nn.Module):
         """(x, pending) after all layers without leaving C++, or None: only layers of the modules above, as they are and with
         nothing hooked into them, can be run that way."""
         if type(self.layers) is not nn.ModuleList or x.dim() != 3 or torch.nn.modules.module._has_any_global_hook():
+            return None
+        if any(getattr(cls, name) is not method for (cls, name), method in _STOCK_METHODS.items()):
             return None
         rope_pos = sequences = None
         if position_ids is not None:

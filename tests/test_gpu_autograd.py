@@ -185,3 +185,26 @@ def test_weights_modified_between_forward_and_backward_are_noticed(dev, form, na
         model.get_submodule("layers.1." + name).weight.mul_(2)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         loss.backward()
+
+
+@pytest.mark.parametrize("cls", ["LlamaMLP", "LlamaDecoderLayer", "LlamaRMSNorm", "HipLinear", "HipAttentionCore", "LlamaAttention"])
+def test_a_replaced_forward_of_a_class_is_called(dev, cls, monkeypatch):
+    import maltos_amd.llama as llama
+
+    model, batch, calls = _model(dev), _batch(dev), []
+    original = getattr(llama, cls).forward
+    if cls == "HipAttentionCore":   # (only asked when rotation and attention are separate)
+        monkeypatch.setattr(llama.LlamaAttention, "fuse_rope_attention", False)
+    want = model(batch)
+    monkeypatch.setattr(getattr(llama, cls), "forward", lambda self, *a, **kw: (calls.append(1), original(self, *a, **kw))[1])
+    got = model(batch)
+    assert calls and torch.allclose(got, want, rtol=1e-3)
+
+
+def test_a_replaced_forward_of_a_projection_is_called(dev):
+    model, batch, calls = _model(dev), _batch(dev), []
+    projection = model.layers[0].self_attn.k_proj
+    original = projection.forward
+    projection.forward = lambda x: (calls.append(1), original(x))[1]
+    model(batch)
+    assert len(calls) == 1
