@@ -18,6 +18,7 @@
 
 #include <optional>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../../include/maltos_hip.h"
@@ -55,6 +56,13 @@ template <typename... T>
 void refuse_tangents(const char* what, const T&... tensors) {
   TORCH_CHECK_NOT_IMPLEMENTED(!(has_tangent(tensors) || ...), what, ": maltos_amd has no forward-mode derivative of this operator");
 }
+
+// tensors of function transforms (torch.func)
+inline bool of_transform(const Tensor& t) {
+  return t.defined() && (t.key_set().has(c10::DispatchKey::FuncTorchBatched) || t.key_set().has(c10::DispatchKey::FuncTorchGradWrapper));
+}
+// Whether something around the innermost transform differentiates this value: what a node records in there is not seen by it.
+bool differentiated_outside(Tensor t);
 
 inline mlts_stream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 inline bool stream_is_capturing() {
@@ -156,6 +164,9 @@ struct Formula : public Node {
   // The backward kernels have no derivatives: their results carry an error as history, so that a second derivative raises where
   // its terms would be missing.  Formulas made of differentiable operators override this.
   virtual variable_list recorded_backward(variable_list&& grads, const std::vector<Tensor>& saved) {
+    static const char* const refusal = ": maltos_amd has no second derivative of this operator";
+    for (const std::vector<Tensor>* values : {&std::as_const(grads), &saved})
+      for (const Tensor& t : *values) TORCH_CHECK(!differentiated_outside(t), name(), refusal);
     torch::autograd::edge_list sources;
     for (const Tensor& g : grads)
       if (g.defined() && g.requires_grad()) sources.push_back(torch::autograd::impl::gradient_edge(g));
@@ -168,7 +179,7 @@ struct Formula : public Node {
       for (Tensor& t : out)
         if (t.defined()) t = t.detach();  // (a result may be one of the gradients, or stand there twice)
     }
-    const auto error = std::shared_ptr<Node>(new torch::autograd::Error(name() + ": maltos_amd has no second derivative of this operator", std::move(sources)),
+    const auto error = std::shared_ptr<Node>(new torch::autograd::Error(name() + refusal, std::move(sources)),
                                              torch::autograd::deleteNode);
     for (const Tensor& t : out)
       if (t.defined()) torch::autograd::set_history(t, error);

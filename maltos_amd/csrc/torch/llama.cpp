@@ -498,10 +498,9 @@ struct AdjacentLinearsBackward final : SharedInputFormula {
 
 // the nodes of several projections have no counterpart in torch to fall back to
 void refuse_function_transforms(const char* what, const Tensor& x, const std::vector<Tensor>& weights = {}) {
-  auto wrapped = [](const Tensor& t) { return t.key_set().has(c10::DispatchKey::FuncTorchBatched) || t.key_set().has(c10::DispatchKey::FuncTorchGradWrapper); };
-  bool any = wrapped(x);
+  bool any = of_transform(x);
   refuse_tangents(what, x);
-  for (const Tensor& w : weights) refuse_tangents(what, w), any = any || wrapped(w);
+  for (const Tensor& w : weights) refuse_tangents(what, w), any = any || of_transform(w);
   TORCH_CHECK_NOT_IMPLEMENTED(!any, what, ": maltos_amd has no rule of this operator for function transforms");
 }
 

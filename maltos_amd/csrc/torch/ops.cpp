@@ -29,6 +29,17 @@ void raise_status(int status) {
   throw pybind11::error_already_set();
 }
 
+bool differentiated_outside(Tensor t) {
+  if (!of_transform(t)) return false;
+  pybind11::gil_scoped_acquire gil;
+  const pybind11::object unwrap = pybind11::module_::import("torch._C._functorch").attr("get_unwrapped");
+  while (of_transform(t)) {
+    t = unwrap(t).cast<Tensor>();
+    if (t.requires_grad() || t.key_set().has(c10::DispatchKey::FuncTorchGradWrapper)) return true;
+  }
+  return false;
+}
+
 namespace {
 
 void check_attn_inputs(const Tensor& q, const Tensor& k, const Tensor& v) {

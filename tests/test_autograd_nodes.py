@@ -127,3 +127,17 @@ def test_kept_rows_belong_to_parameters_of_one_shape_and_type():
     assert group.made_for([memory.view(8, 8)])
     for other in (memory.view(4, 16), memory.view(16, 4), memory[:32].view(4, 8), memory.view(torch.int32).view(8, 8), memory.view(8, 8).requires_grad_(True)):
         assert not group.made_for([other])
+
+
+@pytest.mark.parametrize("name", _OPS)
+def test_nested_function_transforms_raise_where_a_second_derivative_is_missing(name):
+    f, leaves = _OPS[name]()
+    values, total = [t.detach() for t in leaves], lambda *a: f(*a).sum()
+    every = tuple(range(len(values)))
+    first = torch.func.grad(total, argnums=every)
+    assert [g.shape for g in first(*values)] == [v.shape for v in values]
+    penalty = lambda *a: sum((g ** 2).sum() for g in first(*a))
+    with pytest.raises(RuntimeError, match="no second derivative"):
+        torch.func.grad(penalty, argnums=every)(*values)
+    with pytest.raises(RuntimeError, match="no second derivative"):
+        penalty(*leaves)   # (the leaves require gradients: torch's autograd around the transform)

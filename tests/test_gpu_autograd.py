@@ -208,3 +208,20 @@ def test_a_replaced_forward_of_a_projection_is_called(dev):
     projection.forward = lambda x: (calls.append(1), original(x))[1]
     model(batch)
     assert len(calls) == 1
+
+
+def test_second_derivative_of_a_rotation(dev):
+    """|R x|^2 has the gradient 2 x, and |2 x|^2 the gradient 8 x: by recorded passes and by nested function transforms."""
+    from maltos_amd import ops
+
+    gen = torch.Generator().manual_seed(6)
+    x = torch.randn(1, 2, 5, 8, generator=gen).to(dev)
+    angles = torch.rand(5, 4, generator=gen).to(dev)
+    cos, sin = angles.cos(), angles.sin()
+    for rotate in (lambda t: ops.rope(t, cos, sin), lambda t: ops.rope_pair(t, t, cos, sin)[1]):
+        first = torch.func.grad(lambda t: rotate(t).square().sum())
+        assert torch.allclose(torch.func.grad(lambda t: first(t).square().sum())(x), 8 * x, atol=1e-5)
+        leaf = x.clone().requires_grad_(True)
+        (g,) = torch.autograd.grad(rotate(leaf).square().sum(), leaf, create_graph=True)
+        (second,) = torch.autograd.grad(g.square().sum(), leaf)
+        assert torch.allclose(g.detach(), 2 * x, atol=1e-5) and torch.allclose(second, 8 * x, atol=1e-5)
