@@ -9,8 +9,10 @@ int mlts_attn_fwd_bf16_dma(const AttnParams& p, int D, int mode, hipStream_t st)
 int64_t mlts_attn_bwd_dkdv_split_workspace(int64_t B, int64_t Hq, int64_t Sq);                             // attn_bwd_split.hip
 int mlts_attn_bwd_dkdv_bf16_split(AttnBwdParams bp, int D, int mode, void* workspace, bool lse2_ready, hipStream_t st);    // attn_bwd_split.hip
 int mlts_attn_bwd_dq_bf16_tr(const AttnBwdParams& bp, int D, int mode, hipStream_t st);                    // attn_bwd_dq_tr.hip
-int mlts_attn_tile16_fwd(AttnParams p, int D, int dtype, int mode, hipStream_t st);                        // attn_tile16.hip
-int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int dtype, int mode, hipStream_t st);                    // attn_tile16.hip
+int mlts_attn_tile16_fwd(AttnParams p, int D, int mode, hipStream_t st);                                   // attn_tile16.hip
+int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int mode, hipStream_t st);                               // attn_tile16.hip
+int mlts_attn_f32_fwd(AttnParams p, int D, int mode, hipStream_t st);                                      // attn_f32_fwd.hip
+int mlts_attn_f32_bwd(AttnBwdParams bp, int D, int mode, hipStream_t st);                                  // attn_f32_bwd.hip
 int mlts_attn_delta_bf16(const void* dout, const int64_t* dos, const void* o, const int64_t* os, float* delta, int B, int H, int S,
                          int D, hipStream_t st);                                                            // attn_delta.hip
 
@@ -232,7 +234,8 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
   void* lse2_ws = ws;
   if (!uses_mfma(s)) {
     bp.delta_out = delta;
-    return mlts_attn_tile16_bwd(bp, s->D, s->dtype, s->mask_mode, st);
+    if (s->dtype == MLTS_F32) return mlts_attn_f32_bwd(bp, s->D, s->mask_mode, st);
+    return mlts_attn_tile16_bwd(bp, s->D, s->mask_mode, st);
   }
   // the recomputing dQ kernel forms delta itself from 16-byte chunks of the O rows
   const bool stats_in_dq = s->Sk > 0 && mlts_aligned16(o) && strides_aligned(s->o_stride, 2);
@@ -624,7 +627,8 @@ extern "C" int mlts_attn_fwd(const mlts_attn_shape* s, const void* q, const void
     setup_stats(p, s, false, static_cast<char*>(workspace), st);
     return mlts_attn_fwd_bf16_dma(p, s->D, s->mask_mode, st);
   }
-  return mlts_attn_tile16_fwd(p, s->D, s->dtype, s->mask_mode, st);
+  if (s->dtype == MLTS_F32) return mlts_attn_f32_fwd(p, s->D, s->mask_mode, st);
+  return mlts_attn_tile16_fwd(p, s->D, s->mask_mode, st);
 }
 
 extern "C" int mlts_attn_bwd(const mlts_attn_shape* s, const void* dout, const int64_t do_stride[3], const void* q,

@@ -1,4 +1,4 @@
-// Attention on 16-row wavefront tiles: fp32 at any head_dim <= 192, bf16 at head dims the 32-row kernels do not cover.
+// Attention on 16-row wavefront tiles: bf16 at head dims <= 192 that the 32-row kernels do not cover.
 //
 // A wavefront owns 16 rows (queries in the forward and dQ kernels, keys in the dK/dV kernel) and walks the other side in
 // units of 32, staged in LDS 64 at a time.  Everything is computed transposed, S^T = K Q^T and O^T = V^T P^T (dK/dV: S = Q K^T,
@@ -6,16 +6,15 @@
 // registers they were computed in: the 16 x 16 result layout (lane l: column l % 16, rows 4 (l / 16) ..+3) is the operand
 // layout of the next product once the contraction index is renumbered, which both operands agree on.
 //
-//  * fp32 runs on v_mfma_f32_16x16x4_f32, true fp32 products and sums at twice the rate of the vector ALU;
-//  * bf16 runs on v_mfma_f32_16x16x32_bf16.  Probabilities and dS enter their second product as the sum of three bf16 values of 8
-//    bits each, which is all of an fp32 number: products and sums as with fp32 probabilities.  (Two of them are enough for a bf16
-//    output, but not for gradients added in fp32: 2.5e-6 off the exact ones at S = 777, with three 0.3 to 0.5e-6.  The third
-//    costs a few percent where a kernel is short, 9 to 15 where it fills the chip: 8 x 8 heads x 1024, head_dim 32, forward and
-//    backward 27 + 68 us with two, 30 + 77 with three.)
+// Products run on v_mfma_f32_16x16x32_bf16.  Probabilities and dS enter their second product as the sum of three bf16 values of 8
+// bits each, which is all of an fp32 number: products and sums as with fp32 probabilities.  (Two of them are enough for a bf16
+// output, but not for gradients added in fp32: 2.5e-6 off the exact ones at S = 777, with three 0.3 to 0.5e-6.  The third
+// costs a few percent where a kernel is short, 9 to 15 where it fills the chip: 8 x 8 heads x 1024, head_dim 32, forward and
+// backward 27 + 68 us with two, 30 + 77 with three.)
 //
-// What bounds it: the matrix pipe for long rows (fp32: 32 cycles per 16x16x4; a 32-key unit is 2 * D / 2 of them), the chain
-// of tiles of one workgroup for short ones.  A workgroup is four wavefronts: 64 rows, or, when the grid would leave compute
-// units idle, 32 rows with the two halves of every tile on different wavefronts (joined in LDS at the end).
+// What bounds it: the matrix pipe for long rows, the chain of tiles of one workgroup for short ones.  A workgroup is four
+// wavefronts: 64 rows, or, when the grid would leave compute units idle, 32 rows with the two halves of every tile on different
+// wavefronts (joined in LDS at the end).
 #include "attn_common.hpp"
 
 namespace {
@@ -34,35 +33,6 @@ template <typename T, int DP>
 struct Tile16;
 
 template <int DP>
-struct Tile16<float, DP> {
-  static constexpr int STEP = 16;          // head_dim columns per own-row fragment
-  static constexpr int FRAGS = DP / STEP;
-  static constexpr int PER = 4;            // elements of a fragment per lane: columns STEP * j + 4 * (lane / 16) ..+3
-  static constexpr int LS = DP + 4;        // LDS row stride: 16-byte reads over 16 rows and 4-byte reads over 4 x 16 are conflict free
-  typedef f32x4 frag;
-  // acc[m = walked row, n = own row] += walked row . own row, one fragment
-  static __device__ __forceinline__ f32x4 dot(frag a, frag b, f32x4 acc) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c], b[c], acc, 0, 0, 0);
-    return acc;
-  }
-  // acc[db][m = column 16 db + ., n = own row] += sum over the 32 walked rows of a unit of tile[row][m] * x[row][n]; `blocks`:
-  // which of the unit's two 16-row blocks take part (x is zero in the other)
-  static __device__ __forceinline__ void accumulate(f32x4 (&acc)[DP / 16], const float* unit, const f32x4 (&x)[2], int blocks, int l16, int g) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      if (!(blocks & (1 << b))) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float* row = unit + (16 * b + 4 * g + i) * LS + l16;
-#pragma unroll
-        for (int db = 0; db < DP / 16; ++db) acc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(row[16 * db], x[b][i], acc[db], 0, 0, 0);
-      }
-    }
-  }
-};
-
-template <int DP>
 struct Tile16<bf16_t, DP> {
   static constexpr int STEP = 32;
   static constexpr int FRAGS = DP / STEP;
@@ -72,7 +42,7 @@ struct Tile16<bf16_t, DP> {
   static __device__ __forceinline__ f32x4 dot(frag a, frag b, f32x4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
   }
-  static __device__ __forceinline__ void accumulate(f32x4 (&acc)[DP / 16], const bf16_t* unit, const f32x4 (&x)[2], int, int l16, int g) {
+  static __device__ __forceinline__ void accumulate(f32x4 (&acc)[DP / 16], const bf16_t* unit, const f32x4 (&x)[2], int l16, int g) {
     bf16x8 part[3];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
@@ -141,16 +111,13 @@ struct Stage {
 };
 
 // e^x.  Scores, maxima and log-sum-exps stay in natural units and are subtracted first: what is rounded on the way into the hardware's
-// 2^x is then a difference that is near 0 wherever the probability counts, and not a score.  In fp32, against 64 bits (2-norms of 40
-// drawn inputs a size, head dims 32 to 128, 64 to 300 rows, N(0, 1) and three times that), the errors of O, LSE and the gradients are
-// 0.65 to 1.01 of those of kernels on the vector ALU with expf, and within 0.06 of what expf gives here (0.63 to 1.02), which takes 4
-// to 12 % of the kernels' time (4 x 8 heads x 1024, head_dim 64: forward 64 / 67 us, backward 211 / 219); in bf16 up to 60 %.  With the
-// scores multiplied by log2 e before the subtraction they were up to 1.25 times those errors.
+// 2^x is then a difference that is near 0 wherever the probability counts, and not a score (with the scores multiplied by log2 e
+// before the subtraction the errors were up to 1.25 times as large).  expf would take up to 60 % of the kernels' time.
 __device__ __forceinline__ float exponential(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
 struct Tile16Args {
   int D;
-  int row_waves;  // wavefronts over the owned rows: 4, 2 (the others split a tile's two units) or 1 (and a unit's two 16-row blocks)
+  int row_waves;  // wavefronts over the owned rows: 4, or 2 (the others work on the other of a tile's two units)
   bool vec;       // every row of every tensor is 16-byte aligned and D a multiple of the 16-byte vector
 };
 
@@ -238,7 +205,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row_wave = wave & (a.row_waves - 1), split = wave / a.row_waves, splits = kWaves / a.row_waves;
-  const int unit0 = splits == 4 ? split >> 1 : split, unit_step = splits == 1 ? 1 : 2, blocks = splits == 4 ? 1 << (split & 1) : 3;
+  const int unit0 = split, unit_step = splits;
   const int rows = a.row_waves * 16;
   // last blocks first: with a causal mask they are the long ones
   const int nbh = p.B * p.Hq, qt = p.nqt - 1 - static_cast<int>(blockIdx.x) / nbh, bh = static_cast<int>(blockIdx.x) % nbh;
@@ -312,10 +279,6 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (!(blocks & (1 << kb))) {
-          s[kb] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-          continue;
-        }
 #pragma unroll
         for (int j = 0; j < C::FRAGS; ++j)
           s[kb] = C::dot(*reinterpret_cast<const typename C::frag*>(ku_rows + 16 * kb * C::LS + C::STEP * j), qf[j], s[kb]);
@@ -357,7 +320,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
           s[kb][i] = exponential(s[kb][i] * p.scale - m_use);
           l += s[kb][i];
         }
-      C::accumulate(o, sV + 32 * u * C::LS, s, blocks, l16, g);
+      C::accumulate(o, sV + 32 * u * C::LS, s, l16, g);
     }
     k0 = kn;
   }
@@ -401,7 +364,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row_wave = wave & (a.row_waves - 1), split = wave / a.row_waves, splits = kWaves / a.row_waves;
-  const int unit0 = splits == 4 ? split >> 1 : split, unit_step = splits == 1 ? 1 : 2, blocks = splits == 4 ? 1 << (split & 1) : 3;
+  const int unit0 = split, unit_step = splits;
   const int rows = a.row_waves * 16;
   const int nbh = p.B * p.Hq, qt = p.nqt - 1 - static_cast<int>(blockIdx.x) / nbh, bh = static_cast<int>(blockIdx.x) % nbh;
   const int b = bh / p.Hq, hq = bh % p.Hq, hkv = hq / (p.Hq / p.Hkv);
@@ -487,7 +450,6 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         s[kb] = dp[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (!(blocks & (1 << kb))) continue;
 #pragma unroll
         for (int j = 0; j < C::FRAGS; ++j) {
           const int at = frag0 + 16 * kb * C::LS + C::STEP * j;
@@ -507,9 +469,9 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
           } else if (masked && ku + 16 * kb + 4 * g + i > klim) {
             pv = 0.f;
           }
-          s[kb][i] = (blocks & (1 << kb)) ? pv * (dp[kb][i] - delta) : 0.f;
+          s[kb][i] = pv * (dp[kb][i] - delta);
         }
-      C::accumulate(dq, sK + 32 * u * C::LS, s, blocks, l16, g);
+      C::accumulate(dq, sK + 32 * u * C::LS, s, l16, g);
     }
     k0 = kn;
   }
@@ -534,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row_wave = wave & (a.row_waves - 1), split = wave / a.row_waves, splits = kWaves / a.row_waves;
-  const int unit0 = splits == 4 ? split >> 1 : split, unit_step = splits == 1 ? 1 : 2, blocks = splits == 4 ? 1 << (split & 1) : 3;
+  const int unit0 = split, unit_step = splits;
   const int rows = a.row_waves * 16;
   // first blocks first: with a causal mask they are the long ones
   const int nbh = p.B * p.Hkv, kt = static_cast<int>(blockIdx.x) / nbh, bh = static_cast<int>(blockIdx.x) % nbh;
@@ -623,7 +585,6 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
         s[qb] = dp[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (!(blocks & (1 << qb))) continue;
 #pragma unroll
         for (int j = 0; j < C::FRAGS; ++j) {
           const int at = frag0 + 16 * qb * C::LS + C::STEP * j;
@@ -645,12 +606,11 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
           } else if (masked && q0 + r < qlim) {
             pv = 0.f;
           }
-          if (!(blocks & (1 << qb))) pv = 0.f;
           s[qb][i] = pv;
           dp[qb][i] = pv * (dp[qb][i] - st.y);
         }
-      C::accumulate(dv, sdO + 32 * u * C::LS, s, blocks, l16, g);
-      C::accumulate(dk, sQ + 32 * u * C::LS, dp, blocks, l16, g);
+      C::accumulate(dv, sdO + 32 * u * C::LS, s, l16, g);
+      C::accumulate(dk, sQ + 32 * u * C::LS, dp, l16, g);
     }
     hg = hn, q0 = qn;
   }
@@ -671,14 +631,13 @@ constexpr int lds_bytes() {
   return tiles > join ? tiles : join;
 }
 
-// Wavefronts over the owned rows (each 16 of them); the others of a workgroup's four split the tiles of the same rows.  64 rows
-// per workgroup stage a tile for four times as many products as 16 rows do, but short rows then leave compute units idle and
-// the kernel lasts as long as one workgroup's chain of tiles.  The lines, from forward + backward at 4, 2 and 1 (us):
-//   fp32 D=64 S=1024   16 heads (256 workgroups of 64 rows) 287 / 212 / 188     64 heads (1024) 471 / 547 / 773
-//   bf16 D=64 S=1024   16 heads 118 / 88 / 88    32 heads (512) 123 / 95 / 142    S=2048, 32 heads (1024) 248 / 267 / 427
-int row_waves_for(int64_t rows, int64_t heads, bool fp32) {
+// Wavefronts over the owned rows (each 16 of them); the others of a workgroup's four take the other half of every tile.  64 rows
+// per workgroup stage a tile for twice as many products as 32 rows do, but short rows then leave compute units idle and
+// the kernel lasts as long as one workgroup's chain of tiles.  The line, from forward + backward at 4 and 2 (us), D=64:
+//   S=1024   16 heads (256 workgroups of 64 rows) 118 / 88   32 heads (512) 123 / 95      S=2048, 32 heads (1024) 248 / 267
+int row_waves_for(int64_t rows, int64_t heads) {
   const int64_t blocks = (rows + 63) / 64 * heads;
-  return blocks >= 768 ? 4 : fp32 && blocks <= 256 ? 1 : 2;
+  return blocks >= 768 ? 4 : 2;
 }
 
 template <auto KERN, typename P>
@@ -702,7 +661,7 @@ bool rows_vec(const int64_t* s, const void* ptr, int per) {
 template <typename T, int DP, bool DOC>
 int fwd(AttnParams p, int D, hipStream_t st) {
   const int per = 16 / static_cast<int>(sizeof(T));
-  Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq, sizeof(T) == 4),
+  Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq),
                D % per == 0 && rows_vec(p.qs, p.q, per) && rows_vec(p.ks, p.k, per) && rows_vec(p.vs, p.v, per) && rows_vec(p.os, p.o, per)};
   p.nqt = (p.Sq + a.row_waves * 16 - 1) / (a.row_waves * 16);
   MltsKernelTimer timer("attn_fwd", st);
@@ -716,14 +675,14 @@ int bwd(AttnBwdParams bp, int D, hipStream_t st) {
   const bool in_vec = D % per == 0 && rows_vec(p.qs, p.q, per) && rows_vec(p.ks, p.k, per) && rows_vec(p.vs, p.v, per) &&
                       rows_vec(bp.dos, bp.dout, per) && rows_vec(p.os, p.o, per);
   if (p.Sq > 0) {
-    Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq, sizeof(T) == 4), in_vec && (bp.dq_f32 || rows_vec(bp.dqs, bp.dq_acc, per))};
+    Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq), in_vec && (bp.dq_f32 || rows_vec(bp.dqs, bp.dq_acc, per))};
     p.nqt = (p.Sq + a.row_waves * 16 - 1) / (a.row_waves * 16);
     MltsKernelTimer timer("attn_bwd_dq", st);
     if (int rc = launch<attn_tile16_bwd_dq<T, DP, DOC>>(lds_bytes<T, DP>(), static_cast<int64_t>(p.nqt) * p.B * p.Hq, st, bp, a, "mlts_attn_bwd"); rc != MLTS_OK)
       return rc;
   }
   if (p.Sk == 0) return MLTS_OK;
-  Tile16Args a{D, row_waves_for(p.Sk, static_cast<int64_t>(p.B) * p.Hkv, sizeof(T) == 4),
+  Tile16Args a{D, row_waves_for(p.Sk, static_cast<int64_t>(p.B) * p.Hkv),
                in_vec && (bp.accumulate_f32 || (rows_vec(bp.dks, bp.dk, per) && rows_vec(bp.dvs, bp.dv, per)))};
   const int64_t nkt = (p.Sk + a.row_waves * 16 - 1) / (a.row_waves * 16);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
@@ -746,23 +705,19 @@ void set_causal_off(AttnParams& p, int mode) {
   } while (0)
 #define MLTS_TILE16(FN, ...)                                              \
   do {                                                                    \
-    if (dtype == MLTS_BF16) {                                             \
-      if (mode == MLTS_MASK_DOC) MLTS_TILE16_DP(FN, bf16_t, true, __VA_ARGS__);  \
-      MLTS_TILE16_DP(FN, bf16_t, false, __VA_ARGS__);                     \
-    }                                                                     \
-    if (mode == MLTS_MASK_DOC) MLTS_TILE16_DP(FN, float, true, __VA_ARGS__);     \
-    MLTS_TILE16_DP(FN, float, false, __VA_ARGS__);                        \
+    if (mode == MLTS_MASK_DOC) MLTS_TILE16_DP(FN, bf16_t, true, __VA_ARGS__);    \
+    MLTS_TILE16_DP(FN, bf16_t, false, __VA_ARGS__);                       \
   } while (0)
 
 }  // namespace
 
-int mlts_attn_tile16_fwd(AttnParams p, int D, int dtype, int mode, hipStream_t st) {
+int mlts_attn_tile16_fwd(AttnParams p, int D, int mode, hipStream_t st) {
   set_causal_off(p, mode);
   MLTS_TILE16(fwd, p, D, st);
 }
 
 // bp.delta_out receives rowsum(dO * O); bp.delta must point at the same buffer
-int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int dtype, int mode, hipStream_t st) {
+int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
   MLTS_TILE16(bwd, bp, D, st);
 }

@@ -360,6 +360,28 @@ def test_sixteen_row_kernels_at_tile_edges(dev, dtype, D, B, H, Hkv, Sq, Sk):
         run_case(dev, dtype, B, H, Hkv, Sq, Sk, D, mode, seed=Sq + D)
 
 
+# 16-row blocks: 195, 1365 and 2145, i.e. eight, two and one wavefronts to a block, with a workgroup at the end that is partly empty
+@pytest.mark.parametrize("B,H", [(1, 3), (3, 7), (11, 3)])
+@pytest.mark.parametrize("D", [64, 60])
+def test_fp32_blocks_shared_by_wavefronts(dev, D, B, H):
+    for mode in (ops.MASK_CAUSAL, ops.MASK_DOC):
+        run_case(dev, torch.float32, B, H, H, 1030, 1030, D, mode, seed=B + D, max_doc=300)
+
+
+def test_fp32_rows_far_apart(dev):
+    """Row strides that no 24-bit offset reaches give the bits of the same rows close together."""
+    gen = torch.Generator().manual_seed(3)
+    q, k, v, do = (bshd(1, 2, 20, 64, gen, torch.float32).to(dev) for _ in range(4))
+    far = torch.zeros(20, 1 << 22, device=dev)[:, :128].unflatten(1, (2, 64)).transpose(0, 1).unsqueeze(0)
+    far.copy_(k)
+    want = got = None
+    for keys in (k, far):
+        qg, kg, vg = (t.detach().requires_grad_(True) for t in (q, keys, v))
+        o, lse = ops.attention(qg, kg, vg, mask_mode=ops.MASK_CAUSAL, return_lse=True)
+        want, got = got, (o, lse, *torch.autograd.grad(o, (qg, kg, vg), do))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_padding_rows_give_zeros_and_no_nan(dev, dtype):
     o, lse = run_case(dev, dtype, 2, 2, 2, 200, 200, 64, ops.MASK_DOC, seed=77, max_doc=50, pad_tail=37)
