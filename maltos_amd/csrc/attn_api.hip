@@ -11,6 +11,10 @@ int mlts_attn_bwd_dkdv_bf16_split(AttnBwdParams bp, int D, int mode, void* works
 int mlts_attn_bwd_dq_bf16_tr(const AttnBwdParams& bp, int D, int mode, hipStream_t st);                    // attn_bwd_dq_tr.hip
 int mlts_attn_tile16_fwd(AttnParams p, int D, int mode, hipStream_t st);                                   // attn_tile16.hip
 int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int mode, hipStream_t st);                               // attn_tile16.hip
+bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride);  // attn_small.hip
+int mlts_attn_small_fwd(AttnParams p, int D, int mode, hipStream_t st);                                    // attn_small.hip
+int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st);                             // attn_small.hip
+int mlts_attn_small_bwd_dkv(AttnBwdParams bp, int D, int mode, hipStream_t st);                            // attn_small.hip
 int mlts_attn_f32_fwd(AttnParams p, int D, int mode, hipStream_t st);                                      // attn_f32_fwd.hip
 int mlts_attn_f32_bwd(AttnBwdParams bp, int D, int mode, hipStream_t st);                                  // attn_f32_bwd.hip
 int mlts_attn_delta_bf16(const void* dout, const int64_t* dos, const void* o, const int64_t* os, float* delta, int B, int H, int S,
@@ -174,8 +178,8 @@ int64_t bwd_min_workspace(const mlts_attn_shape* s) {
   return stats_bytes(s, true) + delta + lse2;
 }
 
-// The recomputing dQ kernel first, which (stats_in_dq) also writes the row statistics (delta, lse2) into the workspace,
-// then the dK/dV kernel that reads them.
+// The dQ kernel first, which (stats_in_dq) also writes the row statistics (delta, lse2) into the workspace, then the dK/dV kernel
+// that reads them.
 int attn_bwd_bf16(AttnBwdParams bp, int D, int mode, float* delta_ws, void* lse2_ws, bool stats_in_dq, hipStream_t st) {
   const AttnParams& p = bp.a;
   bp.nkt = (p.Sk + 127) / 128;
@@ -183,9 +187,11 @@ int attn_bwd_bf16(AttnBwdParams bp, int D, int mode, float* delta_ws, void* lse2
     bp.delta_out = delta_ws;
     bp.lse2_out = static_cast<float*>(lse2_ws);
   }
-  int rc = mlts_attn_bwd_dq_bf16_tr(bp, D, mode, st);
+  const bool small_dq = stats_in_dq && p.Sq > 0 && mlts_attn_small_serves(ATTN_BWD_DQ, p, D, mode, bp.dos);
+  int rc = small_dq ? mlts_attn_small_bwd_dq(bp, D, mode, st) : mlts_attn_bwd_dq_bf16_tr(bp, D, mode, st);
   if (rc != MLTS_OK) return rc;
   bp.delta_out = bp.lse2_out = nullptr;
+  if (p.Sk > 0 && mlts_attn_small_serves(ATTN_BWD_DKV, p, D, mode, bp.dos)) return mlts_attn_small_bwd_dkv(bp, D, mode, st);
   return mlts_attn_bwd_dkdv_bf16_split(bp, D, mode, lse2_ws, stats_in_dq, st);
 }
 
@@ -237,7 +243,7 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
     if (s->dtype == MLTS_F32) return mlts_attn_f32_bwd(bp, s->D, s->mask_mode, st);
     return mlts_attn_tile16_bwd(bp, s->D, s->mask_mode, st);
   }
-  // the recomputing dQ kernel forms delta itself from 16-byte chunks of the O rows
+  // the dQ kernels form delta themselves from 16-byte chunks of the O rows
   const bool stats_in_dq = s->Sk > 0 && mlts_aligned16(o) && strides_aligned(s->o_stride, 2);
   if (s->Sq > 0 && !stats_in_dq) {
     int rc = mlts_attn_delta_bf16(dout, do_stride, o, s->o_stride, delta, s->B, s->Hq, s->Sq, s->D, st);
@@ -625,6 +631,7 @@ extern "C" int mlts_attn_fwd(const mlts_attn_shape* s, const void* q, const void
     MLTS_REQUIRE(mlts_aligned16(q) && mlts_aligned16(k) && mlts_aligned16(v) && mlts_aligned16(o),
                  "mlts_attn_fwd: q, k, v, o must be 16-byte aligned");
     setup_stats(p, s, false, static_cast<char*>(workspace), st);
+    if (mlts_attn_small_serves(ATTN_FWD, p, s->D, s->mask_mode, nullptr)) return mlts_attn_small_fwd(p, s->D, s->mask_mode, st);
     return mlts_attn_fwd_bf16_dma(p, s->D, s->mask_mode, st);
   }
   if (s->dtype == MLTS_F32) return mlts_attn_f32_fwd(p, s->D, s->mask_mode, st);

@@ -71,6 +71,8 @@ struct AttnBwdParams {
   float* lse2_out;
 };
 
+enum AttnPass { ATTN_FWD, ATTN_BWD_DQ, ATTN_BWD_DKV };
+
 enum TileClass { TILE_SKIP = 0, TILE_FULL = 1, TILE_MASKED = 2 };
 
 // Classification of a (64-query group, 64-key tile) pair from the statistics, MLTS_MASK_DOC.

@@ -6,18 +6,16 @@ namespace {
 // dQ: dq = scale * sum_j ds_ij k_j, ds = p (dp - delta), p = exp(scale s - lse).  Runs first in a backward pass and writes
 // delta = rowsum(dO * O) for the dK/dV kernel.  bp.dq_f32: dq is added to (1) or overwritten (0, 2).
 template <int DP, int R, bool DOC, int LAYOUT>
-__global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(const AttnBwdParams bp, const F32Args a) {
+__global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(const AttnBwdParams bp, const RowArgs a) {
   constexpr int FRAGS = DP / 16, NC = DP / 16, ROWS = 16 * R;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), splits = a.splits, split = wave & (splits - 1);
-  const int waves = static_cast<int>(blockDim.x) >> 6, slot = splits < kMinWaves ? wave >> (splits - 1) : 0;  // (one or two splits: shift by 0 or 1)
-  const int block = splits < kMinWaves ? static_cast<int>(blockIdx.x) * (waves >> (splits - 1)) + slot : static_cast<int>(blockIdx.x);
-  const bool there = block < a.blocks;  // else it only keeps the barriers
+  const Place at(a);
+  const int lane = at.lane, l16 = at.l16, g = at.g, splits = at.splits, split = at.split, slot = at.slot;
+  const bool there = at.there;
   // with a causal mask the last blocks are the long ones
   int bh, hq, member;
-  const int qt = p.nqt - 1 - a.rank(a.batch_heads.over(min(block, a.blocks - 1), &bh)), b = a.heads.over(bh, &hq), hkv = a.group.over(hq, &member);
+  const int qt = p.nqt - 1 - a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hq), hkv = a.group.over(hq, &member);
   const int q0 = qt * ROWS;
   const float* K = static_cast<const float*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
   const float* V = static_cast<const float*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
@@ -76,7 +74,7 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
 #pragma unroll
     for (int db = 0; db < NC; ++db) dq[r][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 kf[FRAGS], vf[FRAGS];
-  float* turn = lds + wave * Turn<DP>::FLOATS;
+  float* turn = lds + at.wave * Turn<DP>::FLOATS;
   int kp[4], ks[4], kp_now[4], ks_now[4];
   auto fetch = [&](int k) {
     const int safe = min(k + l16, p.Sk - 1);
@@ -154,18 +152,16 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
 
 // dK, dV of 16 key rows of one KV head, summed over the query heads of its group.
 template <int DP, bool DOC, int LAYOUT>
-__global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(const AttnBwdParams bp, const F32Args a) {
+__global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(const AttnBwdParams bp, const RowArgs a) {
   constexpr int FRAGS = DP / 16, NC = DP / 16;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), splits = a.splits, split = wave & (splits - 1);
-  const int waves = static_cast<int>(blockDim.x) >> 6, slot = splits < kMinWaves ? wave >> (splits - 1) : 0;  // (one or two splits: shift by 0 or 1)
-  const int block = splits < kMinWaves ? static_cast<int>(blockIdx.x) * (waves >> (splits - 1)) + slot : static_cast<int>(blockIdx.x);
-  const bool there = block < a.blocks;  // else it only keeps the barriers
+  const Place at(a);
+  const int lane = at.lane, l16 = at.l16, g = at.g, splits = at.splits, split = at.split, slot = at.slot;
+  const bool there = at.there;
   // with a causal mask the first blocks are the long ones
   int bh, hkv;
-  const int kt = a.rank(a.batch_heads.over(min(block, a.blocks - 1), &bh)), b = a.heads.over(bh, &hkv), group = static_cast<int>(a.group.d);
+  const int kt = a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hkv), group = static_cast<int>(a.group.d);
   const int kb0 = kt * 16, krow = kb0 + l16;
   const int64_t ksafe = min(krow, p.Sk - 1);
   const float* K = static_cast<const float*>(p.k) + b * p.ks[0] + hkv * p.ks[1] + ksafe * p.ks[2];
@@ -197,7 +193,7 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
 #pragma unroll
   for (int db = 0; db < NC; ++db) dkv[0][db] = dkv[1][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 qf[FRAGS], dof[FRAGS];
-  float *turn_q = lds + wave * 2 * Turn<DP>::FLOATS, *turn_do = turn_q + Turn<DP>::FLOATS;
+  float *turn_q = lds + at.wave * 2 * Turn<DP>::FLOATS, *turn_do = turn_q + Turn<DP>::FLOATS;
   float lse[4], delta[4];
   int qp[4], qs[4];
   const float* Q0 = static_cast<const float*>(p.q) + b * p.qs[0];
@@ -209,12 +205,12 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     const float *q_row = row_of<LAYOUT>(Q, safe, p.qs[2]), *do_row = row_of<LAYOUT>(dO, safe, bp.dos[2]);
 #pragma unroll
     for (int j = 0; j < FRAGS; ++j) qf[j] = load_dot<LAYOUT>(q_row, 16 * j + 4 * g, a.D), dof[j] = load_dot<LAYOUT>(do_row, 16 * j + 4 * g, a.D);
-    const int64_t at = (static_cast<int64_t>(b) * p.Hq + head) * p.Sq;
+    const int64_t stat = (static_cast<int64_t>(b) * p.Hq + head) * p.Sq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int ok = min(q + 4 * g + i, p.Sq - 1);
-      lse[i] = p.lse[at + ok];
-      delta[i] = bp.delta[at + ok];
+      lse[i] = p.lse[stat + ok];
+      delta[i] = bp.delta[stat + ok];
       if (DOC) qp[i] = units.pos[ok], qs[i] = units.seq[ok];
     }
   };
@@ -273,9 +269,9 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     accumulate(dkv[0], rows, dp);
     hg = hn, q0 = qn;
   }
-  const int64_t at = krow;
-  float* const row[2] = {there && krow < p.Sk ? static_cast<float*>(bp.dk) + b * bp.dks[0] + hkv * bp.dks[1] + at * bp.dks[2] : nullptr,
-                         there && krow < p.Sk ? static_cast<float*>(bp.dv) + b * bp.dvs[0] + hkv * bp.dvs[1] + at * bp.dvs[2] : nullptr};
+  const int64_t own = krow;
+  float* const row[2] = {there && krow < p.Sk ? static_cast<float*>(bp.dk) + b * bp.dks[0] + hkv * bp.dks[1] + own * bp.dks[2] : nullptr,
+                         there && krow < p.Sk ? static_cast<float*>(bp.dv) + b * bp.dvs[0] + hkv * bp.dvs[1] + own * bp.dvs[2] : nullptr};
   const float scale[2] = {p.scale, 1.f};
   join_and_store(dkv, lds + slot * splits * 2 * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0);
 }
@@ -285,10 +281,11 @@ int bwd_dq(AttnBwdParams bp, int D, hipStream_t st) {
   AttnParams& p = bp.a;
   p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
-  const F32Args a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dqs, bp.dq_acc), p.Hq, p.nqt);
+  const RowArgs a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dqs, bp.dq_acc), p.Hq, p.nqt);
   MltsKernelTimer timer("attn_bwd_dq", st);
-  return launch_splits<attn_f32_bwd_dq<DP, R, DOC, LAYOUT>, DP, R, max_splits(DP, LAYOUT)>(blocks, splits_for(blocks, (p.Sk + 15) / 16, max_splits(DP, LAYOUT)), 1, st, bp, a,
-                                                                   "mlts_attn_bwd");
+  const int splits = splits_for(blocks, (p.Sk + 15) / 16, max_splits(DP, LAYOUT));
+  return launch_splits<attn_f32_bwd_dq<DP, R, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, R * DP * 64, Turn<DP>::FLOATS * 4, st, bp, a,
+                                                                                    "mlts_attn_bwd");
 }
 
 template <int DP, bool DOC, int LAYOUT>
@@ -303,10 +300,11 @@ int bwd(AttnBwdParams bp, int D, hipStream_t st) {
   }
   if (p.Sk == 0) return MLTS_OK;
   const int64_t blocks = static_cast<int64_t>((p.Sk + 15) / 16) * p.B * p.Hkv;
-  const F32Args a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dks, bp.dk) && rows_vec(bp.dvs, bp.dv), p.Hkv, (p.Sk + 15) / 16);
+  const RowArgs a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dks, bp.dk) && rows_vec(bp.dvs, bp.dv), p.Hkv, (p.Sk + 15) / 16);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
-  return launch_splits<attn_f32_bwd_dkv<DP, DOC, LAYOUT>, DP, 2, max_splits(DP, LAYOUT)>(
-      blocks, splits_for(blocks, static_cast<int64_t>((p.Sq + 15) / 16) * (p.Hq / p.Hkv), max_splits(DP, LAYOUT)), 2, st, bp, a, "mlts_attn_bwd");
+  const int splits = splits_for(blocks, static_cast<int64_t>((p.Sq + 15) / 16) * (p.Hq / p.Hkv), max_splits(DP, LAYOUT));
+  return launch_splits<attn_f32_bwd_dkv<DP, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, 2 * DP * 64, 2 * Turn<DP>::FLOATS * 4, st, bp, a,
+                                                                                  "mlts_attn_bwd");
 }
 
 }  // namespace

@@ -5,17 +5,15 @@ namespace {
 
 // O and LSE of 16 query rows.  DP: head_dim rounded up to a multiple of 32 (the padding is zero in every dot product).
 template <int DP, bool DOC, int LAYOUT>
-__global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_fwd(const AttnParams p, const F32Args a) {
+__global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_fwd(const AttnParams p, const RowArgs a) {
   constexpr int FRAGS = DP / 16, NC = DP / 16;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), splits = a.splits, split = wave & (splits - 1);
-  const int waves = static_cast<int>(blockDim.x) >> 6, slot = splits < kMinWaves ? wave >> (splits - 1) : 0;  // (one or two splits: shift by 0 or 1)
-  const int block = splits < kMinWaves ? static_cast<int>(blockIdx.x) * (waves >> (splits - 1)) + slot : static_cast<int>(blockIdx.x);
-  const bool there = block < a.blocks;  // else it only keeps the barriers
+  const Place at(a);
+  const int lane = at.lane, l16 = at.l16, g = at.g, splits = at.splits, split = at.split, slot = at.slot;
+  const bool there = at.there;
   // with a causal mask the last blocks are the long ones
   int bh, hq, member;
-  const int qt = p.nqt - 1 - a.rank(a.batch_heads.over(min(block, a.blocks - 1), &bh)), b = a.heads.over(bh, &hq), hkv = a.group.over(hq, &member);
+  const int qt = p.nqt - 1 - a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hq), hkv = a.group.over(hq, &member);
   const int q0 = 16 * qt, qrow = q0 + l16;
   const float* K = static_cast<const float*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
   const float* V = static_cast<const float*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
@@ -132,7 +130,8 @@ int fwd(AttnParams p, int D, bool vec_out, hipStream_t st) {
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   const int splits = splits_for(blocks, (p.Sk + 15) / 16, max_splits(DP, LAYOUT));
   MltsKernelTimer timer("attn_fwd", st);
-  return launch_splits<attn_f32_fwd<DP, DOC, LAYOUT>, DP, 1, max_splits(DP, LAYOUT)>(blocks, splits, 0, st, p, F32Args(p, D, vec_out, p.Hq, p.nqt), "mlts_attn_fwd");
+  return launch_splits<attn_f32_fwd<DP, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, DP * 64, 0, st, p, RowArgs(p, D, vec_out, p.Hq, p.nqt),
+                                                                              "mlts_attn_fwd");
 }
 
 }  // namespace

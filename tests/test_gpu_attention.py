@@ -382,6 +382,17 @@ def test_fp32_rows_far_apart(dev):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("mode", [ops.MASK_NONE, ops.MASK_CAUSAL, ops.MASK_DOC])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D", [(1, 2, 2, 513, 513, 64), (1, 3, 1, 545, 545, 128), (1, 8, 4, 1030, 1030, 64), (3, 8, 8, 527, 527, 64),
+                                              (2, 8, 8, 527, 527, 128), (1, 4, 2, 1, 2049, 64), (1, 2, 2, 600, 17, 128), (2, 2, 1, 515, 1061, 64)])
+def test_long_rows_of_small_grids(dev, mode, B, Hq, Hkv, Sq, Sk, D):
+    """Blocks of 16 rows that eight, four and two wavefronts share, remainders of 16 and 32 rows, calls of which only the
+    forward and dQ passes or only dK/dV are long enough for them; the last of each kind at the limit of the grid."""
+    if mode == ops.MASK_DOC and Sq != Sk:
+        return
+    run_case(dev, torch.bfloat16, B, Hq, Hkv, Sq, Sk, D, mode, seed=Sq + Sk + D, max_doc=200, pad_tail=21 * (Sq & 1), share_ids=B == 1)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_padding_rows_give_zeros_and_no_nan(dev, dtype):
     o, lse = run_case(dev, dtype, 2, 2, 2, 200, 200, 64, ops.MASK_DOC, seed=77, max_doc=50, pad_tail=37)
