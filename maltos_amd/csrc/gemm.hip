@@ -149,12 +149,14 @@ struct TileShape {
   typedef Slab<T, BM, FORM != FORM_TN, THREADS, SETS> SA;
   typedef Slab<T, BN, FORM == FORM_NT, THREADS, SETS> SB;
   static constexpr int STAGE = SA::BYTES + SB::BYTES;
-  static constexpr int OUT = WAVES * 32 * (WN + 4) * 4 + (KG > 1 ? (WAVES - WAVES / KG) * MB * NB * 4096 : 0);
+  static constexpr int OUT = WAVES * 32 * (WN + 4) * 4;
+  static_assert(KG == 1 || WAVES == KG, "one wavefront to a group");
   static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
 };
 
-// One tile of one product.  KG > 1: the wavefronts form KG groups that share the tile and each multiply their part of every
-// slab; the groups' sums are joined through LDS in a fixed order.
+// One tile of one product.  KG > 1: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
+// LDS, where all of them add up and write out a part of the tile (us, one of them / all: fp32 NT 2048 x 256 x 256 7.2 / 6.7,
+// 500 x 512 x 512 8.0 / 7.0).
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS>
 __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs) {
   typedef TileShape<T, FORM, BM, BN, WM, WN, KG> S;
@@ -164,7 +166,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   constexpr int BK = Elem<T>::BK, STEPS = 4 / KG;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = KG > 1 ? wave / (S::WAVES / KG) : 0, member = KG > 1 ? wave % (S::WAVES / KG) : wave;
+  const int group = KG > 1 ? wave : 0, member = KG > 1 ? 0 : wave;
   const int wm = (member / WAVES_N) * WM, wn = (member % WAVES_N) * WN;
   const int slice = tile / (g.tiles_m * g.tiles_n);
   tile -= slice * (g.tiles_m * g.tiles_n);
@@ -228,17 +230,18 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   // What the result is added to, for small tiles: fetched here, behind the first slabs, where the end of the tile would wait for
   // it (a gradient that was last touched a step ago; dW and dx of a 512-wide layer at 1023 tokens: four launches a layer, 40 us
   // of a training step of 8 layers).
-  constexpr int LPR = WN / 4, RPP = 64 / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
-  constexpr bool EARLY = MB * NB == 1;
+  constexpr int OUT_LANES = KG > 1 ? S::THREADS : 64;  // that write a block of 32 rows of C
+  constexpr int LPR = WN / 4, RPP = OUT_LANES / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
+  constexpr bool EARLY = KG > 1 || MB * NB == 1;
   typedef T t4 __attribute__((ext_vector_type(4)));
-  t4 old[EARLY ? PASSES : 1];
-  const int c4 = (lane % LPR) * 4, col = n0 + wn + c4;
+  t4 old[EARLY ? MB * PASSES : 1];
+  const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + wn + c4;
   const bool whole = col + 4 <= g.N && (g.ldc & 3) == 0;
-  if (EARLY && g.accumulate && !g.partial && whole && group == 0) {
+  if (EARLY && g.accumulate && !g.partial && whole) {
 #pragma unroll
-    for (int r = 0; r < PASSES; ++r) {
-      const int row = m0 + wm + r * RPP + lane / LPR;
-      if (row < g.M) old[EARLY ? r : 0] = *reinterpret_cast<const t4*>(static_cast<const T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col);
+    for (int i = 0; i < (EARLY ? MB * PASSES : 0); ++i) {
+      const int row = m0 + wm + i * RPP + out_lane / LPR;
+      if (row < g.M) old[i] = *reinterpret_cast<const t4*>(static_cast<const T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col);
     }
   }
 #pragma unroll
@@ -304,12 +307,21 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   if constexpr (SETS == 1) {
     for (int s = 0; s < slabs; ++s) slab(s, 0);
   } else {
-    for (int s = 0; s < slabs; s += 2) {
-      slab(s, 1);
-      after(s);
-      if (s + 1 < slabs) {
-        slab(s + 1, 0);
-        after(s + 1);
+    // (Whole rounds of the sets with nothing to jump over: a way round one slab of a round leaves fewer loads behind, and the waits
+    // of the next round are set for that way.  1023 x 512 x 512 6.4 -> 5.7 us, x 1376 11.8 -> 10.2 us with weights out of HBM.)
+    int s = 0;
+    for (; s + SETS <= slabs; s += SETS) {
+#pragma unroll
+      for (int u = 0; u < SETS; ++u) {
+        slab(s + u, (u + 1) % SETS);
+        after(s + u);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < SETS - 1; ++u) {
+      if (s + u < slabs) {
+        slab(s + u, (u + 1) % SETS);
+        after(s + u);
       }
     }
   }
@@ -326,48 +338,24 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   // acc[i][j][4 q + r]: row wm + 32 i + l % 32 of C, column wn + 32 j + 8 q + 4 hh + r.  Out through LDS, 32 rows at a time.
   __syncthreads();
   constexpr int ROW = WN + 4;  // floats
-  if constexpr (KG > 1) {
-    f32x4* sums = reinterpret_cast<f32x4*>(lds + S::WAVES * 32 * ROW * 4);  // [group - 1][member][block][quad][lane]
-    if (group > 0) {
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            sums[(((wave - S::WAVES / KG) * MB * NB + i * NB + j) * 4 + q) * 64 + lane] =
-                f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-    }
-    __syncthreads();
-    if (group > 0) return;
-#pragma unroll
-    for (int o = 0; o < KG - 1; ++o)
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const f32x4 v = sums[(((o * (S::WAVES / KG) + member) * MB * NB + i * NB + j) * 4 + q) * 64 + lane];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] += v[r];
-          }
-  }
-  float* stage = reinterpret_cast<float*>(lds) + wave * 32 * ROW;
+  float* stage = reinterpret_cast<float*>(lds) + (KG > 1 ? 0 : wave * 32 * ROW);
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
+    if (KG > 1 && i > 0) __syncthreads();
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-        *reinterpret_cast<f32x4*>(stage + l32 * ROW + 32 * j + 8 * q + 4 * hh) = v;
+        *reinterpret_cast<f32x4*>(stage + (group * 32 + l32) * ROW + 32 * j + 8 * q + 4 * hh) = v;
       }
-    // (a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
+    if (KG > 1) __syncthreads();  // (alone, a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
 #pragma unroll
     for (int r = 0; r < PASSES; ++r) {
-      const int rr = r * RPP + lane / LPR, row = m0 + wm + 32 * i + rr;
+      const int rr = r * RPP + out_lane / LPR, row = m0 + wm + 32 * i + rr;
       f32x4 v = *reinterpret_cast<const f32x4*>(stage + rr * ROW + c4);
+#pragma unroll
+      for (int o = 1; o < KG; ++o) v += *reinterpret_cast<const f32x4*>(stage + (o * 32 + rr) * ROW + c4);
       if (row >= g.M || col >= g.N) continue;
       if (g.partial) {
         float* p = g.partial + (static_cast<int64_t>(slice) * g.M + row) * g.N + col;
@@ -381,7 +369,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
       T* p = static_cast<T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col;
       if (whole) {
         if (g.accumulate) {
-          const t4 before = EARLY ? old[EARLY ? r : 0] : *reinterpret_cast<const t4*>(p);
+          const t4 before = EARLY ? old[EARLY ? i * PASSES + r : 0] : *reinterpret_cast<const t4*>(p);
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] += to_f32<T>(before[e]);
         }
