@@ -19,6 +19,9 @@
 #include "attn_common.hpp"
 #include <type_traits>
 
+bool mlts_attn_bwd_dkv64_serves(const AttnParams& p, int mode);                                            // attn_bwd_dkv64.hip
+int mlts_attn_bwd_dkv64(const AttnBwdParams& bp, int mode, const float* lse2, hipStream_t st);              // attn_bwd_dkv64.hip
+
 namespace {
 
 constexpr int BQ = 64;
@@ -833,5 +836,6 @@ int mlts_attn_bwd_dkdv_bf16_split(AttnBwdParams bp, int D, int mode, void* works
   const int64_t n = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
   if (!lse2_ready)
     hipLaunchKernelGGL(lse2_kernel, dim3(static_cast<unsigned>((n + 256) / 256)), dim3(256), 0, st, p.lse, lse2, n);
+  if (D == 64 && mlts_attn_bwd_dkv64_serves(p, mode)) return mlts_attn_bwd_dkv64(bp, mode, lse2, st);
   return D == 128 ? launch_mode<128>(bp, mode, lse2, st) : launch_mode<64>(bp, mode, lse2, st);
 }

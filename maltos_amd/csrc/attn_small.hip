@@ -10,17 +10,12 @@
 // own row and the next product takes them, rounded to bf16 once, from the registers they are in.
 //
 // Documents: the plan's tile classes and visibility bits, as in the 32-row kernels.
-#include "attn_rows.hpp"
+#include "attn_bf16.hpp"
 
 namespace {
 
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-#define MLTS_LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
-
 constexpr int kUnit = 32;      // walked rows
 constexpr int kMaxSplits = 8;  // wavefronts to a row block
-
-__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 __device__ __forceinline__ const bf16_t* row_of(const bf16_t* base, int row, int64_t stride) {  // (near(): offsets fit 32 bits)
   const uint32_t offset = __umul24(static_cast<uint32_t>(row), static_cast<uint32_t>(stride) * 2u);
@@ -29,39 +24,19 @@ __device__ __forceinline__ const bf16_t* row_of(const bf16_t* base, int row, int
 
 // A unit of one operand: fetched, put to LDS, read as fragments.
 template <int D>
-struct Unit {
-  static constexpr int CHUNKS = D / 8, N = kUnit * CHUNKS / 64, STRIDE = D + 8, BYTES = kUnit * STRIDE * 2;  // (conflict-free reads of 16 rows)
+struct Unit : Rows<D> {
+  static constexpr int CHUNKS = D / 8, N = kUnit * CHUNKS / 64, BYTES = kUnit * Rows<D>::BYTES;
   bf16x8 raw[N];
   __device__ __forceinline__ void fetch(const bf16_t* base, int64_t stride, int row0, int last, int lane) {
 #pragma unroll
     for (int i = 0; i < N; ++i)
       raw[i] = *reinterpret_cast<const bf16x8*>(row_of(base, min(row0 + (64 / CHUNKS) * i + lane / CHUNKS, last), stride) + 8 * (lane % CHUNKS));
   }
-  __device__ __forceinline__ void put(bf16_t* lds, int lane) const {
+  __device__ __forceinline__ void put(unsigned char* lds, int lane) const {
 #pragma unroll
-    for (int i = 0; i < N; ++i) *reinterpret_cast<bf16x8*>(lds + ((64 / CHUNKS) * i + lane / CHUNKS) * STRIDE + 8 * (lane % CHUNKS)) = raw[i];
-  }
-  // rows 16 b + l16, columns 32 j + 8 g ..+7
-  static __device__ __forceinline__ bf16x8 dot(const bf16_t* lds, int b, int j, int l16, int g) {
-    return *reinterpret_cast<const bf16x8*>(lds + (16 * b + l16) * STRIDE + 32 * j + 8 * g);
-  }
-  // column 16 db + l16 of rows 4 g ..+3 and 16 + 4 g ..+3: in the order in which a lane holds scores
-  static __device__ __forceinline__ bf16x8 columns(const bf16_t* lds, int db, int l16, int g) {
-    const bf16_t* src = lds + (4 * g + (l16 >> 2)) * STRIDE + 16 * db + (l16 & 3) * 4;
-    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src));
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src + 16 * STRIDE));
-    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    for (int i = 0; i < N; ++i) *reinterpret_cast<bf16x8*>(lds + Rows<D>::at((64 / CHUNKS) * i + lane / CHUNKS, lane % CHUNKS)) = raw[i];
   }
 };
-
-__device__ __forceinline__ bf16x8 pack(const f32x4 (&x)[2]) {
-  bf16x8 v;
-#pragma unroll
-  for (int b = 0; b < 2; ++b)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[4 * b + i] = static_cast<bf16_t>(x[b][i]);
-  return v;
-}
 
 // The units a split works on, in order: every `splits`-th.  Documents: those of them whose tile of 64 rows the plan's statistics do not
 // rule out for the own rows' group of 64, 32 tiles at a time, a lane for each unit.
@@ -130,19 +105,6 @@ __device__ __forceinline__ void join_and_store(f32x4 (&acc)[N][NC], f32x4* lds, 
     }
 }
 
-// mode 0: bf16, overwritten; 1: fp32, added to; 2: fp32, overwritten
-__device__ __forceinline__ void store4(void* base, int64_t off, f32x4 v, int mode) {
-  if (mode == 0) {
-    bf16x4 w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = static_cast<bf16_t>(v[e]);
-    *reinterpret_cast<bf16x4*>(static_cast<bf16_t*>(base) + off) = w;
-  } else {
-    f32x4* p = reinterpret_cast<f32x4*>(static_cast<float*>(base) + off);
-    *p = mode == 1 ? *p + v : v;
-  }
-}
-
 // O and LSE of 16 query rows
 template <int D, bool DOC>
 __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnParams p, const RowArgs a) {
@@ -183,7 +145,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
 #pragma unroll
   for (int db = 0; db < NC; ++db) o[0][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   U keys, values;
-  bf16_t *lk = reinterpret_cast<bf16_t*>(lds_raw + at.wave * 2 * U::BYTES), *lv = lk + U::BYTES / 2;
+  unsigned char *lk = lds_raw + at.wave * 2 * U::BYTES, *lv = lk + U::BYTES;
   // (past the end the last key is fetched again: a branch around the loads would wait for all of them)
   unsigned long long word = 0, word_now = 0;
   bool masked = false, masked_now = false;
@@ -344,7 +306,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
 #pragma unroll
   for (int db = 0; db < NC; ++db) dq[0][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   U keys, values;
-  bf16_t *lk = reinterpret_cast<bf16_t*>(lds_raw + at.wave * 2 * U::BYTES), *lv = lk + U::BYTES / 2;
+  unsigned char *lk = lds_raw + at.wave * 2 * U::BYTES, *lv = lk + U::BYTES;
   unsigned long long word = 0, word_now = 0;
   bool masked = false, masked_now = false;
   auto fetch = [&](int k) {  // (past the end the last key again: a branch around the loads would wait for all of them)
@@ -444,7 +406,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
   for (int db = 0; db < NC; ++db) dkv[0][db] = dkv[1][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   U queries, grads;
   unsigned char* own = lds_raw + at.wave * (2 * U::BYTES + 256);
-  bf16_t *lq = reinterpret_cast<bf16_t*>(own), *ld = lq + U::BYTES / 2;
+  unsigned char *lq = own, *ld = own + U::BYTES;
   float* lstat = reinterpret_cast<float*>(own + 2 * U::BYTES);  // (lse, delta) of the unit's queries: a lane fetches one, and reads eight of each
   float stat = 0.f;
   unsigned long long word = 0, word_now = 0;

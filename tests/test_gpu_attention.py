@@ -393,6 +393,14 @@ def test_long_rows_of_small_grids(dev, mode, B, Hq, Hkv, Sq, Sk, D):
     run_case(dev, torch.bfloat16, B, Hq, Hkv, Sq, Sk, D, mode, seed=Sq + Sk + D, max_doc=200, pad_tail=21 * (Sq & 1), share_ids=B == 1)
 
 
+@pytest.mark.parametrize("mode,B,Hq,Hkv,Sq,Sk", [(ops.MASK_NONE, 32, 4, 4, 513, 300), (ops.MASK_CAUSAL, 20, 8, 8, 577, 415), (ops.MASK_CAUSAL, 20, 8, 8, 512, 513),
+                                                 (ops.MASK_CAUSAL, 43, 6, 3, 545, 545), (ops.MASK_DOC, 35, 6, 3, 545, 545), (ops.MASK_DOC, 16, 8, 8, 512, 512)])
+def test_dkv_of_large_grids(dev, mode, B, Hq, Hkv, Sq, Sk):
+    """head_dim 64, 128 keys to a workgroup of one-role wavefronts: remainders of tiles and key blocks, queries past the keys and
+    keys past the queries, padding, at the smallest grid of each mask."""
+    run_case(dev, torch.bfloat16, B, Hq, Hkv, Sq, Sk, 64, mode, seed=B + Sk, max_doc=200, pad_tail=21 * (Sq & 1), share_ids=bool(Sq & 1))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_padding_rows_give_zeros_and_no_nan(dev, dtype):
     o, lse = run_case(dev, dtype, 2, 2, 2, 200, 200, 64, ops.MASK_DOC, seed=77, max_doc=50, pad_tail=37)
