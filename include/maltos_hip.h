@@ -298,6 +298,12 @@ typedef struct {
 int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* products, int32_t count, int32_t dtype);
 int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
                     mlts_stream_t stream);
+/* gate = x W_gate^T, up = x W_up^T (W [N, K], x [M, K]) and h = round(silu(gate)) * up of the rounded gate and up (models/llama.py:205-206)
+ * in one launch: the values of two products and mlts_swiglu_fwd_rows.  gate and up may be null (nobody reads them).  Sizes whose products
+ * would be split, or are large, are not served: mlts_gemm_swiglu_supports says NULL, or why. */
+const char* mlts_gemm_swiglu_supports(int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldc, int64_t ldh);
+int mlts_gemm_swiglu(int32_t dtype, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx, const void* w_gate, const void* w_up,
+                     int64_t ldw, void* gate, void* up, int64_t ldc, void* h, int64_t ldh, mlts_stream_t stream);
 
 
 /* The norm, scaling and AdamW passes over a list of fp32 tensors (host arrays of device pointers and element counts) in one

@@ -83,6 +83,7 @@ template <typename T>
 __device__ __forceinline__ float round_to(float x) {
   return to_f32<T>(from_f32<T>(x));
 }
+__device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }  // the form ATen evaluates
 
 // 16-byte vector of T
 template <typename T>

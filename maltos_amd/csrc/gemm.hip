@@ -50,8 +50,9 @@ struct Elem<float> {
   }
 };
 
-// One operand's slab: ROWS rows (of C's rows or columns), KC: the contraction is its contiguous dimension.
-template <typename T, int ROWS, bool KC, int THREADS, int SETS>
+// One operand's slab: ROWS rows (of C's rows or columns), KC: the contraction is its contiguous dimension.  TWO: the upper half of the rows
+// are those of a second matrix.
+template <typename T, int ROWS, bool KC, int THREADS, int SETS, bool TWO = false>
 struct Slab {
   static constexpr int ES = static_cast<int>(sizeof(T));
   static constexpr int BK = Elem<T>::BK;
@@ -63,7 +64,7 @@ struct Slab {
   static constexpr int PER = LINES * CHUNKS / THREADS;         // chunks per lane
   static_assert(LINES * CHUNKS % THREADS == 0, "whole chunks per lane");
 
-  __amdgpu_buffer_rsrc_t rsrc;
+  __amdgpu_buffer_rsrc_t rsrc, rsrc2;
   uint32_t offset[PER];
   uint32_t advance;
   u32x4 reg[SETS][PER];
@@ -74,17 +75,23 @@ struct Slab {
     rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, static_cast<int>(bytes), 0x00020000);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int idx = i * THREADS + threadIdx.x;
+      const int idx = (TWO ? i % (PER / 2) : i) * THREADS + threadIdx.x;
       const int64_t line = idx / CHUNKS + (KC ? 0 : k_begin);
       offset[i] = static_cast<uint32_t>((line * ld + (KC ? k_begin : 0)) * ES + (idx % CHUNKS) * 16);
     }
     advance = static_cast<uint32_t>(KC ? 128 : BK * ld * ES);
   }
+  // of the second matrix, as many lines with the same stride
+  __device__ __forceinline__ void init_second(const T* base, int64_t ld, int64_t lines, int64_t line_elems) {
+    static_assert(!TWO || (KC && PER % 2 == 0), "a chunk is of one matrix");
+    const int64_t bytes = lines > 0 ? ((lines - 1) * ld + line_elems) * ES : 0;
+    rsrc2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, static_cast<int>(bytes), 0x00020000);
+  }
   // chunk i of the slab at the current offsets; k_left: contraction elements from there to the end
   __device__ __forceinline__ void fetch(int set, int i, int k_left) {
     const int idx = i * THREADS + threadIdx.x;
     const int k = KC ? (idx % CHUNKS) * (16 / ES) : idx / CHUNKS;
-    reg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, k < k_left ? offset[i] : kOutside, 0, 0);
+    reg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(TWO && i >= PER / 2 ? rsrc2 : rsrc, k < k_left ? offset[i] : kOutside, 0, 0);
     offset[i] += advance;
   }
   __device__ __forceinline__ void store(int set, int i, unsigned char* lds) const {
@@ -124,6 +131,13 @@ struct Product {
   int tiles_m, tiles_n, slices;
   int form, accumulate;
 };
+// Two NT products of one shape that share A and meet in the end (gate and up of an MLP): C = A B^T, C2 = A B2^T, h = round(silu(C)) * C2 of
+// the rounded C and C2; N, ldb and ldc are those of one of them.  C and C2 may be null.
+struct Pair {
+  const void* b2;
+  void *c2, *h;
+  int ldh;
+};
 // The contraction of the NN form may be a concatenation (dx = sum dy_i W_i of layers that share their input): what follows the
 // first part.  In bf16 each part is rounded, and added to the parts before it in bf16: the values of separate products whose
 // results are added, bit for bit.
@@ -141,25 +155,26 @@ __device__ __forceinline__ int tile_of(int block, int tiles) {
   return pos < per + (xcd < rest) ? xcd * per + min(xcd, rest) + pos : -1;
 }
 
-template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG>
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool PAIR = false>
 struct TileShape {
   static constexpr int WAVES_N = BN / WN, WAVES = (BM / WM) * WAVES_N * KG, THREADS = WAVES * 64;
   static constexpr int MB = WM / 32, NB = WN / 32;
   static constexpr int SETS = MB * NB >= 8 ? 1 : 2;  // (eight accumulator blocks leave no registers for a second set)
   typedef Slab<T, BM, FORM != FORM_TN, THREADS, SETS> SA;
-  typedef Slab<T, BN, FORM == FORM_NT, THREADS, SETS> SB;
+  typedef Slab<T, BN, FORM == FORM_NT, THREADS, SETS, PAIR> SB;
   static constexpr int STAGE = SA::BYTES + SB::BYTES;
   static constexpr int OUT = WAVES * 32 * (WN + 4) * 4;
   static_assert(KG == 1 || WAVES == KG, "one wavefront to a group");
+  static_assert(!PAIR || (FORM == FORM_NT && KG == 1 && WAVES_N == 2), "the products of a pair side by side in a tile, a wavefront of each");
   static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
 };
 
 // One tile of one product.  KG > 1: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
 // LDS, where all of them add up and write out a part of the tile (us, one of them / all: fp32 NT 2048 x 256 x 256 7.2 / 6.7,
 // 500 x 512 x 512 8.0 / 7.0).
-template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS>
-__device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs) {
-  typedef TileShape<T, FORM, BM, BN, WM, WN, KG> S;
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false>
+__device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr) {
+  typedef TileShape<T, FORM, BM, BN, WM, WN, KG, PAIR> S;
   constexpr int WAVES_N = S::WAVES_N, MB = S::MB, NB = S::NB, SETS = S::SETS, STAGE = S::STAGE;
   typedef typename S::SA SA;
   typedef typename S::SB SB;
@@ -170,7 +185,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   const int wm = (member / WAVES_N) * WM, wn = (member % WAVES_N) * WN;
   const int slice = tile / (g.tiles_m * g.tiles_n);
   tile -= slice * (g.tiles_m * g.tiles_n);
-  const int m0 = (tile / g.tiles_n) * BM, n0 = (tile % g.tiles_n) * BN;
+  const int m0 = (tile / g.tiles_n) * BM, n0 = (tile % g.tiles_n) * (PAIR ? BN / 2 : BN);
 
   SA sa;
   SB sb;
@@ -181,6 +196,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
     else sa.init(static_cast<const T*>(a) + m0 * lda, lda, g.M - m0, K, k_begin);
     if (FORM == FORM_NT) sb.init(static_cast<const T*>(b) + n0 * ldb, ldb, g.N - n0, K, k_begin);
     else sb.init(static_cast<const T*>(b) + n0, ldb, K, g.N - n0, k_begin);
+    if constexpr (PAIR) sb.init_second(static_cast<const T*>(pair->b2) + n0 * ldb, ldb, g.N - n0, K);
     k_left = static_cast<int>(k_end - k_begin);
     seg_slabs = (k_left + BK - 1) / BK;
   };
@@ -232,10 +248,10 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   // of a training step of 8 layers).
   constexpr int OUT_LANES = KG > 1 ? S::THREADS : 64;  // that write a block of 32 rows of C
   constexpr int LPR = WN / 4, RPP = OUT_LANES / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
-  constexpr bool EARLY = KG > 1 || MB * NB == 1;
+  constexpr bool EARLY = !PAIR && (KG > 1 || MB * NB == 1);
   typedef T t4 __attribute__((ext_vector_type(4)));
   t4 old[EARLY ? MB * PASSES : 1];
-  const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + wn + c4;
+  const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? 0 : wn) + c4;
   const bool whole = col + 4 <= g.N && (g.ldc & 3) == 0;
   if (EARLY && g.accumulate && !g.partial && whole) {
 #pragma unroll
@@ -341,7 +357,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   float* stage = reinterpret_cast<float*>(lds) + (KG > 1 ? 0 : wave * 32 * ROW);
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
-    if (KG > 1 && i > 0) __syncthreads();
+    if ((KG > 1 || PAIR) && i > 0) __syncthreads();
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
@@ -349,7 +365,26 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
         const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
         *reinterpret_cast<f32x4*>(stage + (group * 32 + l32) * ROW + 32 * j + 8 * q + 4 * hh) = v;
       }
-    if (KG > 1) __syncthreads();  // (alone, a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
+    if (KG > 1 || PAIR) __syncthreads();  // (alone, a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
+    if constexpr (PAIR) {  // the two wavefronts of a pair of blocks take half of the rows each
+      const float* first = reinterpret_cast<const float*>(lds) + (wave & ~1) * 32 * ROW;
+#pragma unroll
+      for (int r = 0; r < PASSES / 2; ++r) {
+        const int rr = (wave & 1) * 16 + r * RPP + lane / LPR, row = m0 + wm + 32 * i + rr;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(first + rr * ROW + c4), b = *reinterpret_cast<const f32x4*>(first + (32 + rr) * ROW + c4);
+        if (row >= g.M || col >= g.N) continue;
+        t4 gate, up, h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          gate[e] = from_f32<T>(a[e]), up[e] = from_f32<T>(b[e]);
+          h[e] = from_f32<T>(round_to<T>(silu(to_f32<T>(gate[e]))) * to_f32<T>(up[e]));
+        }
+        const int64_t at = static_cast<int64_t>(row) * g.ldc + col;
+        if (g.c) *reinterpret_cast<t4*>(static_cast<T*>(g.c) + at) = gate, *reinterpret_cast<t4*>(static_cast<T*>(pair->c2) + at) = up;
+        *reinterpret_cast<t4*>(static_cast<T*>(pair->h) + static_cast<int64_t>(row) * pair->ldh + col) = h;
+      }
+      continue;
+    }
 #pragma unroll
     for (int r = 0; r < PASSES; ++r) {
       const int rr = r * RPP + out_lane / LPR, row = m0 + wm + 32 * i + rr;
@@ -389,6 +424,16 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_kernel(c
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n * g.slices);
   if (tile >= 0) gemm_tile<T, FORM, BM, BN, WM, WN, KG, false>(g, tile, lds, MoreSegments{}, 0);
+}
+
+// us, one product and the pass over gate and up / the pair / without gate and up (weights out of HBM, x just written): 1376 + 1376 x 512 bf16
+// 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 16.1 + 5.8 / 19.2 / 17.4; 688 + 688 x 256 fp32 2048 rows
+// 20.1 + 4.8 / 20.9 / 18.9.
+template <typename T, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_pair_kernel(const Product g, const Pair pair) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n);
+  if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, WM, WN, 1, false, true>(g, tile, lds, MoreSegments{}, 0, &pair);
 }
 
 // Several small products in one launch: what a linear layer's backward needs (dx and dW), or projections that share their input.
@@ -716,6 +761,33 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hip
   return mlts_check_launch("mlts_gemm");
 }
 
+// The tile that two products of a pair take together, or -1: one after the other
+int pair_tile(int64_t M, int64_t N, int64_t K, int dtype) {
+  const mlts_gemm_product both = single(FORM_NT, M, 2 * N, K, nullptr, K, nullptr, K, nullptr, 2 * N, 0);
+  const LaunchPlan plan(&both, 1, dtype);
+  return plan.slices[0] > 1 || plan.tile[0] == 3 || (plan.tile[0] == kSmall && plan.shape.size != 64) ? -1 : plan.tile[0];
+}
+
+template <typename T, int BM, int BN, int WM, int WN>
+int launch_pair(Product& g, const Pair& pair, hipStream_t st) {
+  typedef TileShape<T, FORM_NT, BM, BN, WM, WN, 1, true> S;
+  g.tiles_m = (g.M + BM - 1) / BM, g.tiles_n = (g.N + BN / 2 - 1) / (BN / 2);
+  const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n;
+  MLTS_REQUIRE(tiles < (int64_t{1} << 30), "mlts_gemm_swiglu: too many tiles");
+  auto kern = gemm_pair_kernel<T, BM, BN, WM, WN>;
+  static MltsLdsOptIn once;
+  if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_swiglu"); rc != MLTS_OK) return rc;
+  MltsKernelTimer timer("gemm_swiglu", st);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(S::THREADS), S::LDS, st, g, pair);
+  return mlts_check_launch("mlts_gemm_swiglu");
+}
+template <typename T>
+int run_pair(int tile, Product& g, const Pair& pair, hipStream_t st) {
+  if (tile == 1) return launch_pair<T, 128, 128, 64, 64>(g, pair, st);
+  if (tile == 2) return launch_pair<T, 256, 128, 64, 64>(g, pair, st);
+  return launch_pair<T, 64, 64, 32, 32>(g, pair, st);
+}
+
 }  // namespace
 
 extern "C" const char* mlts_gemm_supports(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc) {
@@ -759,4 +831,30 @@ extern "C" int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int6
                          void* c, int64_t ldc, int32_t accumulate, void* workspace, int64_t workspace_bytes, mlts_stream_t stream) {
   const mlts_gemm_product p = single(form, M, N, K, a, lda, b, ldb, c, ldc, accumulate);
   return mlts_gemm_multi(&p, 1, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" const char* mlts_gemm_swiglu_supports(int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldc, int64_t ldh) {
+  if (dtype != MLTS_BF16 && dtype != MLTS_F32) return "dtype must be MLTS_F32 or MLTS_BF16";
+  if (const char* why = why_not(single(FORM_NT, M, N, K, nullptr, ldx, nullptr, ldw, nullptr, ldc, 0), dtype)) return why;
+  if (M <= 0 || N <= 0 || K <= 0) return "an empty product";
+  if (N % 4 || ldc % 4 || ldh % 4 || ldh < N || ldh > 0x7fffffff || 2 * N > 0x7fffffff) return "rows of gate, up and h are written four elements at a time";
+  return pair_tile(M, N, K, dtype) < 0 ? "products of this size are not made in one launch" : nullptr;
+}
+
+extern "C" int mlts_gemm_swiglu(int32_t dtype, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx, const void* w_gate, const void* w_up, int64_t ldw,
+                                void* gate, void* up, int64_t ldc, void* h, int64_t ldh, mlts_stream_t stream) {
+  const char* why = mlts_gemm_swiglu_supports(dtype, M, N, K, ldx, ldw, ldc, ldh);
+  MLTS_REQUIRE(why == nullptr, "mlts_gemm_swiglu: %s", why);
+  MLTS_REQUIRE(x && w_gate && w_up && h && !gate == !up, "mlts_gemm_swiglu: null pointer");
+  for (const void* p : {x, w_gate, w_up, static_cast<const void*>(gate), static_cast<const void*>(up), static_cast<const void*>(h)})
+    MLTS_REQUIRE(!p || mlts_aligned16(p), "mlts_gemm_swiglu: pointers must be 16-byte aligned");
+  Product g{};
+  g.a = x, g.b = w_gate, g.c = gate;
+  g.lda = static_cast<int>(ldx), g.ldb = static_cast<int>(ldw), g.ldc = static_cast<int>(ldc);
+  g.M = static_cast<int>(M), g.N = static_cast<int>(N), g.K = static_cast<int>(K);
+  g.form = FORM_NT, g.slices = 1, g.k_slice = static_cast<int>(K);
+  const Pair pair{w_up, up, h, static_cast<int>(ldh)};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int tile = pair_tile(M, N, K, dtype);
+  return dtype == MLTS_BF16 ? run_pair<bf16_t>(tile, g, pair, st) : run_pair<float>(tile, g, pair, st);
 }

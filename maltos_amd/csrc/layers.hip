@@ -300,7 +300,6 @@ __global__ __launch_bounds__(kThreads) void rope_pair_kernel(const RopeOperand a
 
 // ============================== SwiGLU ===================================================
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float siluf_(float x) { return x / (1.0f + expf(-x)); }  // the form ATen evaluates
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void swiglu_fwd_kernel(const T* __restrict__ gate, const T* __restrict__ up,
@@ -314,7 +313,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_fwd_kernel(const T* __restric
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const float gj = g.get(j);
-      const float act = round_to<T>(siluf_(gj));  // F.silu materialised in T
+      const float act = round_to<T>(silu(gj));  // F.silu materialised in T
       o.set(j, act * u.get(j));
     }
     reinterpret_cast<Vec16<T>*>(h)[i] = o;
@@ -358,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_fwd_rows_kernel(const T* __re
     Vec16<T> u = *reinterpret_cast<const Vec16<T>*>(up + in);
     Vec16<T> o;
 #pragma unroll
-    for (int j = 0; j < N; ++j) o.set(j, round_to<T>(siluf_(g.get(j))) * u.get(j));
+    for (int j = 0; j < N; ++j) o.set(j, round_to<T>(silu(g.get(j))) * u.get(j));
     *reinterpret_cast<Vec16<T>*>(h + static_cast<int64_t>(row) * ld_h + c * N) = o;
   }
 }
@@ -394,7 +393,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_fwd_tail(const T* gate, const
   int64_t i = start + static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (i >= n) return;
   const float gj = to_f32<T>(gate[i]);
-  const float act = round_to<T>(siluf_(gj));
+  const float act = round_to<T>(silu(gj));
   h[i] = from_f32<T>(act * to_f32<T>(up[i]));
 }
 template <typename T>

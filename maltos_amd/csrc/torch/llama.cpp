@@ -372,6 +372,32 @@ Tensor project_all(const Tensor& x, const Adjacent& rows, const std::vector<Tens
   return y;
 }
 
+// gate and up of an MLP side by side (undefined if nobody keeps them), and round(silu(gate)) * up: in one launch up to the sizes of the own
+// products, where the pass over gate and up costs as much for its launch as for its bytes.
+std::pair<Tensor, Tensor> gate_up_activation(const Tensor& x, const Adjacent& rows, const std::vector<Tensor>& weights, bool keep) {
+  const Tensor &wg = weights[0], &wu = weights[1], x2 = rows2d(x);
+  const int64_t cols = wg.size(0), es = x.element_size();
+  if (x.is_contiguous() && wu.sizes() == wg.sizes() && wu.stride(0) == wg.stride(0) && own_product(MLTS_GEMM_NT, x2, rows.weight.defined() ? rows.weight : wg) &&
+      own_product(MLTS_GEMM_NT, x2, wg) && own_product(MLTS_GEMM_NT, x2, wu) && (rows.first[0] * es) % 16 == 0 && (rows.first[1] * es) % 16 == 0 &&
+      mlts_gemm_swiglu_supports(dtype_code(x), x2.size(0), cols, x2.size(1), x2.stride(0), wg.stride(0), rows.width, cols) == nullptr) {
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = cols;
+    const Tensor h = at::empty(shape, x.options());
+    Tensor gu;
+    char *gate = nullptr, *up = nullptr;
+    if (keep) {
+      shape.back() = rows.width;
+      gu = at::empty(shape, x.options());
+      gate = static_cast<char*>(mptr(gu)) + rows.first[0] * es, up = static_cast<char*>(mptr(gu)) + rows.first[1] * es;
+    }
+    check(mlts_gemm_swiglu(dtype_code(x), x2.size(0), cols, x2.size(1), ptr(x2), x2.stride(0), ptr(wg), ptr(wu), wg.stride(0), gate, up, rows.width, mptr(h),
+                           cols, current_stream()));
+    return {gu, h};
+  }
+  const Tensor gu = project_all(x, rows, weights);
+  return {gu, swiglu_rows(gu, rows.first[0], rows.first[1], cols)};
+}
+
 // whether two dense buffers share memory (the gradient of a parameter that is used twice)
 bool share_memory(const Tensor& a, const Tensor& b) {
   if (!a.defined() || !b.defined()) return false;
@@ -554,13 +580,13 @@ struct GateUpBackward final : SharedInputFormula {
 
 Tensor gate_up(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tensor>& weights, bool into_grad) {
   refuse_function_transforms("gate_up", x, weights);
+  const bool recorded = at::GradMode::is_enabled() && (compute_requires_grad(x) || any_requires_grad(weights));
   Tensor gu, h;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    gu = project_all(x, *rows, weights);
-    h = swiglu_rows(gu, rows->first[0], rows->first[1], weights[0].size(0));
+    std::tie(gu, h) = gate_up_activation(x, *rows, weights, recorded);
   }
-  if (at::GradMode::is_enabled() && (compute_requires_grad(x) || any_requires_grad(weights))) {
+  if (recorded) {
     const auto fn = adjacent_formula<GateUpBackward>(x, rows, weights, into_grad);
     fn->save(fn->GU, gu);
     set_history(h, fn);
@@ -744,14 +770,14 @@ struct MlpBlockBackward final : BlockFormula {
 };
 
 Tensor mlp_block(const Tensor& x, const BlockWeights& w) {
+  const bool keep = recorded(x, w);
   Tensor gu, h, y;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    gu = project_all(x, *w.rows, w.in);
-    h = swiglu_rows(gu, w.rows->first[0], w.rows->first[1], w.in[0].size(0));
+    std::tie(gu, h) = gate_up_activation(x, *w.rows, w.in, keep);
     y = project(h, w.out);
   }
-  if (recorded(x, w)) {
+  if (keep) {
     auto fn = block_formula<MlpBlockBackward>(x, w);
     fn->save(fn->GU, gu), fn->save(fn->H, h);
     set_history(y, fn);

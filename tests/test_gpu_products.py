@@ -152,3 +152,28 @@ def test_operands_that_do_not_match_are_refused(dev, form, longer):
     if form == NT:
         with pytest.raises(RuntimeError):
             native().linear(a, b, False)
+
+
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 1, 8, 8), (torch.bfloat16, 65, 72, 136), (torch.bfloat16, 1016, 1376, 512),
+                                         (torch.bfloat16, 1100, 2056, 72), (torch.bfloat16, 4001, 1032, 64), (torch.float32, 700, 1028, 68),
+                                         (torch.float32, 2048, 1376, 40)])
+def test_gate_up_in_one_launch(dev, dtype, M, N, K, keep):
+    """Tiles of 64, 128 and 256 rows with remainders of rows, columns (of each of the two products) and slabs, operands with row
+    strides, gate and up wanted or not: the bits of the product with both weights and the pass over it."""
+    gen = torch.Generator().manual_seed(M + N)
+    rows = lambda n: torch.randn(n, K + 24, generator=gen).to(dtype).to(dev)[:, 16:16 + K]
+    x, wg, wu = rows(M), rows(N), rows(N)
+    gu, h = torch.full((M, 2 * N + 8), 7.0, dtype=dtype, device=dev), torch.full((M, N + 4), 7.0, dtype=dtype, device=dev)
+    es, st = x.element_size(), torch.cuda.current_stream().cuda_stream
+    up = gu.data_ptr() + (N + 8) * es
+    both = native().product(NT, x, torch.cat([wg, wu]))
+    want = native().swiglu_rows(both, 0, N, N)
+    L = _lib.lib()
+    _lib.check(L.mlts_gemm_swiglu(1 if dtype == torch.bfloat16 else 0, M, N, K, x.data_ptr(), x.stride(0), wg.data_ptr(), wu.data_ptr(), wg.stride(0),
+                                  gu.data_ptr() if keep else None, up if keep else None, gu.stride(0), h.data_ptr(), h.stride(0), st))
+    assert torch.equal(h[:, :N], want) and (h[:, N:] == 7).all() and (gu[:, N:N + 8] == 7).all()
+    if keep:
+        assert torch.equal(gu[:, :N], both[:, :N]) and torch.equal(gu[:, N + 8:], both[:, N:])
+    else:
+        assert (gu == 7).all()
