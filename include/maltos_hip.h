@@ -298,6 +298,18 @@ typedef struct {
 int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* products, int32_t count, int32_t dtype);
 int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
                     mlts_stream_t stream);
+/* NT products of one call, some of whose columns are heads that are rotated to their positions as they are written
+ * (models/llama.py:143-146): the values of mlts_gemm_multi followed by mlts_rope over them.  Row r is token r % seq of its batch row, at
+ * positions[r], or at position_offset + r % seq.  columns[i]: two ranges [begin, end) of whole heads of product i (empty: begin = end).
+ * Products that would be split are not served: mlts_gemm_rope_supports says NULL, or why. */
+typedef struct {
+  const void *cos, *sin; /* [max_pos, head_dim / 2], the products' dtype, 8-byte aligned */
+  const int32_t* positions;
+  int32_t max_pos, position_offset, seq, head_dim;
+  int64_t columns[4][4];
+} mlts_gemm_rotation;
+const char* mlts_gemm_rope_supports(const mlts_gemm_product* products, int32_t count, int32_t dtype, const mlts_gemm_rotation* rotation);
+int mlts_gemm_rope(const mlts_gemm_product* products, int32_t count, int32_t dtype, const mlts_gemm_rotation* rotation, mlts_stream_t stream);
 /* gate = x W_gate^T, up = x W_up^T (W [N, K], x [M, K]) and h = round(silu(gate)) * up of the rounded gate and up (models/llama.py:205-206)
  * in one launch: the values of two products and mlts_swiglu_fwd_rows.  gate and up may be null (nobody reads them).  Sizes whose products
  * would be split, or are large, are not served: mlts_gemm_swiglu_supports says NULL, or why. */

@@ -131,6 +131,7 @@ struct Product {
   int tiles_m, tiles_n, slices;
   int form, accumulate;
 };
+constexpr int kMaxProducts = 4;  // of a call
 // Two NT products of one shape that share A and meet in the end (gate and up of an MLP): C = A B^T, C2 = A B2^T, h = round(silu(C)) * C2 of
 // the rounded C and C2; N, ldb and ldc are those of one of them.  C and C2 may be null.
 struct Pair {
@@ -138,10 +139,32 @@ struct Pair {
   void *c2, *h;
   int ldh;
 };
+// Rotary positions on the way out of an NT product whose rows are tokens and whose columns are heads: rounded x_even, x_odd become
+// x_even cos - x_odd sin, x_even sin + x_odd cos with the roundings of the pass over them (mlts_rope).
+struct Rotation {
+  const void *cos, *sin;  // [max_pos][D / 2]
+  const int32_t* positions;
+  int max_pos, position_offset, seq, D;
+  int columns[kMaxProducts][4];  // of each product: two ranges of whole heads
+  template <typename T, typename C2>
+  __device__ __forceinline__ void angles(int row, int pair, C2* c, C2* s) const {
+    int pos = positions ? positions[row] : position_offset + static_cast<int>(static_cast<uint32_t>(row) % static_cast<uint32_t>(seq));
+    pos = pos < 0 ? 0 : pos >= max_pos ? max_pos - 1 : pos;  // host validated; keeps reads in bounds
+    const int64_t at = static_cast<int64_t>(pos) * (D / 2) + pair;
+    *c = *reinterpret_cast<const C2*>(static_cast<const T*>(cos) + at), *s = *reinterpret_cast<const C2*>(static_cast<const T*>(sin) + at);
+  }
+};
+template <typename T>
+__device__ __forceinline__ void rotate(float& even, float& odd, float c, float s) {
+#pragma clang fp contract(off)
+  const float xe = round_to<T>(even), xo = round_to<T>(odd);
+  even = round_to<T>(xe * c) - round_to<T>(xo * s);
+  odd = round_to<T>(xe * s) + round_to<T>(xo * c);
+}
 // The contraction of the NN form may be a concatenation (dx = sum dy_i W_i of layers that share their input): what follows the
 // first part.  In bf16 each part is rounded, and added to the parts before it in bf16: the values of separate products whose
 // results are added, bit for bit.
-constexpr int kMaxSegments = 3, kMaxProducts = 4;
+constexpr int kMaxSegments = 3;
 struct MoreSegments {
   const void *a[kMaxSegments - 1], *b[kMaxSegments - 1];
   int lda[kMaxSegments - 1], ldb[kMaxSegments - 1], K[kMaxSegments - 1];
@@ -172,8 +195,9 @@ struct TileShape {
 // One tile of one product.  KG > 1: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
 // LDS, where all of them add up and write out a part of the tile (us, one of them / all: fp32 NT 2048 x 256 x 256 7.2 / 6.7,
 // 500 x 512 x 512 8.0 / 7.0).
-template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false>
-__device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr) {
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false, bool ROPE = false>
+__device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr,
+                                          const Rotation* rot = nullptr, int product = 0) {
   typedef TileShape<T, FORM, BM, BN, WM, WN, KG, PAIR> S;
   constexpr int WAVES_N = S::WAVES_N, MB = S::MB, NB = S::NB, SETS = S::SETS, STAGE = S::STAGE;
   typedef typename S::SA SA;
@@ -248,7 +272,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   // of a training step of 8 layers).
   constexpr int OUT_LANES = KG > 1 ? S::THREADS : 64;  // that write a block of 32 rows of C
   constexpr int LPR = WN / 4, RPP = OUT_LANES / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
-  constexpr bool EARLY = !PAIR && (KG > 1 || MB * NB == 1);
+  constexpr bool EARLY = !PAIR && !ROPE && (KG > 1 || MB * NB == 1);
   typedef T t4 __attribute__((ext_vector_type(4)));
   t4 old[EARLY ? MB * PASSES : 1];
   const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? 0 : wn) + c4;
@@ -258,6 +282,21 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
     for (int i = 0; i < (EARLY ? MB * PASSES : 0); ++i) {
       const int row = m0 + wm + i * RPP + out_lane / LPR;
       if (row < g.M) old[i] = *reinterpret_cast<const t4*>(static_cast<const T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col);
+    }
+  }
+  // ... and what it is rotated by, likewise
+  constexpr bool EARLY_ANGLES = ROPE && MB * NB == 1;
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  t2 cosines[EARLY_ANGLES ? PASSES : 1], sines[EARLY_ANGLES ? PASSES : 1];
+  bool rotated = false;
+  int pair_of_head = 0;
+  if constexpr (ROPE) {
+    const int* range = rot->columns[product];
+    rotated = (col >= range[0] && col < range[1]) || (col >= range[2] && col < range[3]);
+    pair_of_head = static_cast<int>(static_cast<uint32_t>(col - (col >= range[2] && col < range[3] ? range[2] : range[0])) % static_cast<uint32_t>(rot->D)) / 2;
+    if (EARLY_ANGLES && rotated) {
+#pragma unroll
+      for (int r = 0; r < PASSES; ++r) rot->angles<T>(min(m0 + wm + r * RPP + out_lane / LPR, g.M - 1), pair_of_head, &cosines[EARLY_ANGLES ? r : 0], &sines[EARLY_ANGLES ? r : 0]);
     }
   }
 #pragma unroll
@@ -392,6 +431,18 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
 #pragma unroll
       for (int o = 1; o < KG; ++o) v += *reinterpret_cast<const f32x4*>(stage + (o * 32 + rr) * ROW + c4);
       if (row >= g.M || col >= g.N) continue;
+      if constexpr (ROPE) {
+        if (rotated) {
+          t2 c = cosines[EARLY_ANGLES ? r : 0], s = sines[EARLY_ANGLES ? r : 0];
+          if (!EARLY_ANGLES) rot->angles<T>(row, pair_of_head, &c, &s);
+#pragma unroll
+          for (int e = 0; e < 4; e += 2) {
+            float even = v[e], odd = v[e + 1];
+            rotate<T>(even, odd, to_f32<T>(c[e / 2]), to_f32<T>(s[e / 2]));
+            v[e] = even, v[e + 1] = odd;
+          }
+        }
+      }
       if (g.partial) {
         float* p = g.partial + (static_cast<int64_t>(slice) * g.M + row) * g.N + col;
         if (col + 4 <= g.N && (g.N & 3) == 0) {
@@ -426,6 +477,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_kernel(c
   if (tile >= 0) gemm_tile<T, FORM, BM, BN, WM, WN, KG, false>(g, tile, lds, MoreSegments{}, 0);
 }
 
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_rope_kernel(const Product g, const Rotation rot) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n);
+  if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, WM, WN, KG, false, false, true>(g, tile, lds, MoreSegments{}, 0, nullptr, &rot);
+}
+
 // us, one product and the pass over gate and up / the pair / without gate and up (weights out of HBM, x just written): 1376 + 1376 x 512 bf16
 // 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 16.1 + 5.8 / 19.2 / 17.4; 688 + 688 x 256 fp32 2048 rows
 // 20.1 + 4.8 / 20.9 / 18.9.
@@ -458,6 +516,19 @@ __global__ __launch_bounds__(256) void gemm_multi_kernel(const Products ps) {
   if (FORMS == FORMS_NT || (FORMS != FORMS_NN && g.form == FORM_NT)) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
   else if (FORMS == FORMS_NN || g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, 32, 32, KG, FORMS == FORMS_SEGMENTS>(g, tile, lds, ps.more, i == ps.more.product ? ps.more.count : 0);
   else gemm_tile<T, FORM_TN, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
+}
+
+template <typename T, int BM, int BN, int KG>
+__global__ __launch_bounds__(256) void gemm_multi_rope_kernel(const Products ps, const Rotation rot) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int block = static_cast<int>(blockIdx.x);
+  int i = 0, first = ps.first[0];
+#pragma unroll
+  for (int k = 1; k < kMaxProducts; ++k)
+    if (block >= ps.first[k]) i = k, first = ps.first[k];
+  const Product& g = ps.p[i];
+  const int tile = tile_of(block - first, g.tiles_m * g.tiles_n);
+  if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false, false, true>(g, tile, lds, ps.more, 0, nullptr, &rot, i);
 }
 
 // C (+)= sum of the slices' fp32 partial products, one rounding; up to kMaxProducts outputs
@@ -630,6 +701,35 @@ int launch_alone(int tile, const SmallShape& shape, const Product& g, hipStream_
   return g.form == FORM_NN ? launch_form<T, FORM_NN>(tile, shape, g, st) : launch_form<T, FORM_TN>(tile, shape, g, st);
 }
 
+template <typename T, int BM, int BN, int WM, int WN, int KG = 1>
+int launch_rope_tile(const Product& g, const Rotation& rot, hipStream_t st) {
+  typedef TileShape<T, FORM_NT, BM, BN, WM, WN, KG> S;
+  auto kern = gemm_rope_kernel<T, BM, BN, WM, WN, KG>;
+  static MltsLdsOptIn once;
+  if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_rope"); rc != MLTS_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g.tiles_m * g.tiles_n)), dim3(S::THREADS), S::LDS, st, g, rot);
+  return MLTS_OK;
+}
+template <typename T>
+int launch_rope_alone(int tile, const SmallShape& shape, const Product& g, const Rotation& rot, hipStream_t st) {
+  if (tile == 1) return launch_rope_tile<T, 128, 128, 64, 64>(g, rot, st);
+  if (tile == 2) return launch_rope_tile<T, 256, 128, 64, 64>(g, rot, st);
+  if (tile == 3) return launch_rope_tile<T, 256, 256, 128, 64>(g, rot, st);
+  if constexpr (sizeof(T) == 4) {
+    if (shape.size == 32) return launch_rope_tile<T, 32, 32, 32, 32, 4>(g, rot, st);
+  }
+  return launch_rope_tile<T, 64, 64, 32, 32>(g, rot, st);
+}
+template <typename T, int BM, int BN, int KG>
+int launch_rope_small(const Products& ps, const Rotation& rot, int blocks, hipStream_t st) {
+  typedef TileShape<T, FORM_NT, BM, BN, 32, 32, KG> S;
+  auto kern = gemm_multi_rope_kernel<T, BM, BN, KG>;
+  static MltsLdsOptIn once;
+  if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_rope"); rc != MLTS_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), S::LDS, st, ps, rot);
+  return MLTS_OK;
+}
+
 template <typename T, int FORMS, int BM, int BN, int KG>
 int launch_small(const Products& ps, int blocks, hipStream_t st) {
   constexpr int nt = TileShape<T, FORM_NT, BM, BN, 32, 32, KG>::LDS, nn = TileShape<T, FORM_NN, BM, BN, 32, 32, KG>::LDS,
@@ -693,9 +793,12 @@ mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const vo
   return p;
 }
 
+// rotation: of the outputs (products of the NT form, not split), or null
 template <typename T>
-int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hipStream_t st) {
+int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, const Rotation* rotation, hipStream_t st) {
   const LaunchPlan plan(ps, count, dtype);
+  Rotation rot{};
+  if (rotation) rot = *rotation;
   Products joint;
   Joins joins{};
   int blocks, join_blocks = 0, smalls;
@@ -707,6 +810,12 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hip
   };
   auto launch = [&] {  // what `joint` holds
     if (!smalls) return static_cast<int>(MLTS_OK);
+    if (rotation) {
+      if constexpr (sizeof(T) == 4) {
+        if (plan.shape.size == 32) return launch_rope_small<T, 32, 32, 4>(joint, rot, blocks, st);
+      }
+      return launch_rope_small<T, 64, 64, 1>(joint, rot, blocks, st);
+    }
     const int forms = joint.more.count ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
     if constexpr (sizeof(T) == 2) return launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
     else if (plan.shape.size == 64) return launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
@@ -750,8 +859,13 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, hip
     if (small && (count > 1 || p.segments > 1)) {
       all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN;
       joint.first[smalls] = blocks;
+      if (rotation) std::copy(rotation->columns[i], rotation->columns[i] + 4, rot.columns[smalls]);
       blocks += static_cast<int>((tiles + 7) / 8 * 8);  // (whole rounds over the XCDs, so that each product starts at the first)
       joint.p[smalls++] = g;
+    } else if (rotation) {
+      Rotation own = *rotation;
+      std::copy(rotation->columns[i], rotation->columns[i] + 4, own.columns[0]);
+      if (int rc = launch_rope_alone<T>(plan.tile[i], plan.shape, g, own, st); rc != MLTS_OK) return rc;
     } else if (int rc = launch_alone<T>(plan.tile[i], plan.shape, g, st); rc != MLTS_OK) {
       return rc;
     }
@@ -804,8 +918,7 @@ extern "C" int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* prod
   return count < 1 || count > kMaxProducts ? 0 : LaunchPlan(products, count, dtype).workspace;
 }
 
-extern "C" int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
-                               mlts_stream_t stream) {
+static int check_products(const mlts_gemm_product* products, int32_t count, int32_t dtype) {
   MLTS_REQUIRE(dtype == MLTS_BF16 || dtype == MLTS_F32, "mlts_gemm: unknown dtype %d", dtype);
   MLTS_REQUIRE(products && count >= 1 && count <= kMaxProducts, "mlts_gemm: 1 to %d products in a call", kMaxProducts);
   for (int i = 0; i < count; ++i) {
@@ -820,11 +933,17 @@ extern "C" int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count,
     for (int j = 0; j < i; ++j)
       MLTS_REQUIRE(!outputs_overlap(products[j], p, dtype == MLTS_BF16 ? 2 : 4), "mlts_gemm: outputs %d and %d of the call overlap", j, i);
   }
+  return MLTS_OK;
+}
+
+extern "C" int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
+                               mlts_stream_t stream) {
+  if (int rc = check_products(products, count, dtype); rc != MLTS_OK) return rc;
   const int64_t need = mlts_gemm_multi_workspace_bytes(products, count, dtype);
   MLTS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && mlts_aligned16(workspace)), "mlts_gemm: workspace too small or unaligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
   float* ws = static_cast<float*>(workspace);
-  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, ws, st) : run<float>(products, count, dtype, ws, st);
+  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, ws, nullptr, st) : run<float>(products, count, dtype, ws, nullptr, st);
 }
 
 extern "C" int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb,
@@ -857,4 +976,35 @@ extern "C" int mlts_gemm_swiglu(int32_t dtype, int64_t M, int64_t N, int64_t K, 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int tile = pair_tile(M, N, K, dtype);
   return dtype == MLTS_BF16 ? run_pair<bf16_t>(tile, g, pair, st) : run_pair<float>(tile, g, pair, st);
+}
+
+extern "C" const char* mlts_gemm_rope_supports(const mlts_gemm_product* products, int32_t count, int32_t dtype, const mlts_gemm_rotation* rotation) {
+  if (!products || !rotation || count < 1 || count > kMaxProducts) return "1 to 4 products in a call";
+  if (dtype != MLTS_BF16 && dtype != MLTS_F32) return "dtype must be MLTS_F32 or MLTS_BF16";
+  if (rotation->head_dim < 4 || rotation->head_dim % 4 || rotation->max_pos < 1 || rotation->seq < 1) return "bad rotation";
+  for (int i = 0; i < count; ++i) {
+    const mlts_gemm_product& p = products[i];
+    if (const char* why = why_not(p, dtype)) return why;
+    if (p.form != FORM_NT || p.accumulate || p.M <= 0 || p.N <= 0 || p.k[0] <= 0 || p.N % 4 || p.ldc % 4) return "products whose outputs are not rotated";
+    for (int r = 0; r < 4; r += 2) {
+      const int64_t a = rotation->columns[i][r], b = rotation->columns[i][r + 1];
+      if (a < 0 || b < a || b > p.N || a % 4 || (b - a) % rotation->head_dim) return "columns that are not whole heads";
+    }
+  }
+  return LaunchPlan(products, count, dtype).workspace ? "products that would be split" : nullptr;
+}
+
+extern "C" int mlts_gemm_rope(const mlts_gemm_product* products, int32_t count, int32_t dtype, const mlts_gemm_rotation* rotation, mlts_stream_t stream) {
+  const char* why = mlts_gemm_rope_supports(products, count, dtype, rotation);
+  MLTS_REQUIRE(why == nullptr, "mlts_gemm_rope: %s", why);
+  if (int rc = check_products(products, count, dtype); rc != MLTS_OK) return rc;
+  MLTS_REQUIRE(rotation->cos && rotation->sin && ((reinterpret_cast<uintptr_t>(rotation->cos) | reinterpret_cast<uintptr_t>(rotation->sin)) & 7) == 0,
+               "mlts_gemm_rope: the cos / sin tables must be 8-byte aligned and not null");
+  MLTS_REQUIRE(rotation->positions || (rotation->position_offset >= 0 && rotation->position_offset + static_cast<int64_t>(rotation->seq) <= rotation->max_pos),
+               "mlts_gemm_rope: positions exceed the table (%d rows)", rotation->max_pos);
+  Rotation r{rotation->cos, rotation->sin, rotation->positions, rotation->max_pos, rotation->position_offset, rotation->seq, rotation->head_dim, {}};
+  for (int i = 0; i < count; ++i)
+    for (int k = 0; k < 4; ++k) r.columns[i][k] = static_cast<int>(rotation->columns[i][k]);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, nullptr, &r, st) : run<float>(products, count, dtype, nullptr, &r, st);
 }

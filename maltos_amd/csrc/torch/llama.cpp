@@ -727,6 +727,40 @@ struct Positions {
   OptTensor rope, ids, sequences;  // int32 rotary positions; positions and sequence ids of a document mask
 };
 
+// q, k and v side by side with q and k rotated on the way out of their products, or undefined: sizes, layouts and positions that are left to
+// a pass of their own
+Tensor project_rotated(const Tensor& x, const BlockWeights& w, int64_t heads, int64_t kv_heads, const Tensor& cos, const Tensor& sin, const Positions& p) {
+  const Adjacent& rows = *w.rows;
+  const int64_t B = x.size(0), S = x.size(1), D = w.in[0].size(0) / heads, max_pos = cos.dim() == 2 ? cos.size(0) : 0;
+  const auto table = [&](const Tensor& t) {
+    return t.is_cuda() && t.is_contiguous() && t.dim() == 2 && t.size(0) == max_pos && t.size(1) * 2 == D && t.scalar_type() == x.scalar_type() && aligned(t);
+  };
+  const bool given = p.rope.has_value() && p.rope->defined();
+  if (!x.is_contiguous() || !table(cos) || !table(sin) || max_pos > 0x7fffffff || S > 0x7fffffff) return Tensor();
+  if (given ? !p.rope->is_cuda() || p.rope->scalar_type() != at::kInt || !p.rope->is_contiguous() || p.rope->sizes() != at::IntArrayRef({B, S})
+            : p.offset < 0 || p.offset + S > max_pos)
+    return Tensor();
+  const Tensor x2 = rows2d(x);
+  if (rows.weight.defined() && !own_product(MLTS_GEMM_NT, x2, rows.weight)) return Tensor();
+  const Tensor y = at::empty({B, S, rows.width}, x.options()), y2 = rows2d(y);
+  mlts_gemm_rotation r{};
+  r.cos = ptr(cos), r.sin = ptr(sin), r.positions = given ? p.rope->const_data_ptr<int32_t>() : nullptr;
+  r.max_pos = static_cast<int32_t>(max_pos), r.position_offset = given ? 0 : static_cast<int32_t>(p.offset);
+  r.seq = static_cast<int32_t>(S), r.head_dim = static_cast<int32_t>(D);
+  ProductList list;
+  if (rows.weight.defined()) {
+    list.add(MLTS_GEMM_NT, x2, rows.weight, y2, false);
+    r.columns[0][0] = rows.first[0], r.columns[0][1] = rows.first[0] + heads * D;
+    r.columns[0][2] = rows.first[1], r.columns[0][3] = rows.first[1] + kv_heads * D;
+  } else {
+    for (size_t i = 0; i < w.in.size(); ++i) list.add(MLTS_GEMM_NT, x2, w.in[i], y2.narrow(1, rows.first[i], w.in[i].size(0)), false);
+    r.columns[0][1] = heads * D, r.columns[1][1] = kv_heads * D;
+  }
+  if (mlts_gemm_rope_supports(list.items, list.count, dtype_code(x), &r) != nullptr) return Tensor();
+  check(mlts_gemm_rope(list.items, list.count, dtype_code(x), &r, current_stream()));
+  return y;
+}
+
 Tensor attention_block(const Tensor& x, const BlockWeights& w, int64_t heads, int64_t kv_heads, const Tensor& cos, const Tensor& sin, const Positions& p) {
   const int64_t B = x.size(0), S = x.size(1), D = w.in[0].size(0) / heads, width = w.rows->width;
   const int64_t mask_mode = p.ids.has_value() ? MLTS_MASK_DOC : MLTS_MASK_CAUSAL;
@@ -734,11 +768,14 @@ Tensor attention_block(const Tensor& x, const BlockWeights& w, int64_t heads, in
   Tensor q, k, v, qr, kr, out, lse, y;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    const Tensor qkv = project_all(x, *w.rows, w.in);
+    Tensor qkv = project_rotated(x, w, heads, kv_heads, cos, sin, p);
+    const bool rotated = qkv.defined();
+    if (!rotated) qkv = project_all(x, *w.rows, w.in);
     q = as_heads(qkv, B, S, width, w.rows->first[0], heads, D);
     k = as_heads(qkv, B, S, width, w.rows->first[1], kv_heads, D);
     v = as_heads(qkv, B, S, width, w.rows->first[2], kv_heads, D);
-    std::tie(qr, kr) = rope_pair(q, k, cos, sin, p.rope, p.offset, false, false);
+    if (rotated) qr = q, kr = k;
+    else std::tie(qr, kr) = rope_pair(q, k, cos, sin, p.rope, p.offset, false, false);
     std::tie(out, lse) = attention_forward(qr, kr, v, mask_mode, scale, p.ids, p.ids, p.sequences, p.sequences);
     y = product(MLTS_GEMM_NT, as_rows(out), w.out).view({B, S, w.out.size(0)});
   }

@@ -177,3 +177,46 @@ def test_gate_up_in_one_launch(dev, dtype, M, N, K, keep):
         assert torch.equal(gu[:, :N], both[:, :N]) and torch.equal(gu[:, N + 8:], both[:, N:])
     else:
         assert (gu == 7).all()
+
+
+class GemmRotation(ctypes.Structure):
+    """Mirror of `mlts_gemm_rotation`."""
+    _fields_ = [("cos", ctypes.c_void_p), ("sin", ctypes.c_void_p), ("positions", ctypes.c_void_p), ("max_pos", ctypes.c_int32),
+                ("position_offset", ctypes.c_int32), ("seq", ctypes.c_int32), ("head_dim", ctypes.c_int32), ("columns", (ctypes.c_int64 * 4) * 4)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,S,H,Hkv,D,K,joint,given", [(1, 1, 1, 1, 64, 8, False, False), (3, 77, 4, 2, 64, 136, False, True), (2, 65, 3, 1, 128, 72, True, False),
+                                                       (2, 333, 2, 2, 96, 264, True, True), (3, 701, 8, 8, 64, 64, False, True),
+                                                       (3, 777, 16, 4, 128, 40, False, False), (2, 3001, 16, 8, 96, 64, False, True)])
+def test_rotation_in_the_products(dev, dtype, B, S, H, Hkv, D, K, joint, given):
+    """q, k, v as one product or as three: every tile, remainders of rows and slabs, positions of packed rows, or an offset; the
+    bits of the products and the rotation one after the other."""
+    gen = torch.Generator().manual_seed(B * S + D)
+    rnd = lambda *s: torch.randn(*s, generator=gen).to(dtype).to(dev)
+    widths, max_pos, offset = [H * D, Hkv * D, Hkv * D], S + 9, 0 if given else 5
+    x, w, y = rnd(B * S, K), rnd(sum(widths), K), torch.empty(B * S, sum(widths), dtype=dtype, device=dev)
+    angles = torch.rand(max_pos, D // 2, generator=gen) * 6.3
+    cos, sin = angles.cos().to(dtype).to(dev), angles.sin().to(dtype).to(dev)
+    positions = torch.randint(0, max_pos, (B, S), generator=gen, dtype=torch.int32).to(dev) if given else None
+    ws, ys = w.split(widths), y.split(widths, 1)
+    parts = list(zip(ws, ys)) if joint else [(w, y)]
+    plain = [torch.empty_like(c) for _, c in parts]
+    run_products([(NT, [(x, b)], c, 0) for (b, _), c in zip(parts, plain)], dtype)
+    r = GemmRotation(cos.data_ptr(), sin.data_ptr(), positions.data_ptr() if given else None, max_pos, offset, S, D)
+    if joint:
+        r.columns[0][1], r.columns[1][1] = widths[0], widths[1]
+    else:
+        r.columns[0][:] = [0, widths[0], widths[0], widths[0] + widths[1]]
+    ps = (GemmProduct * len(parts))()
+    for p, (b, c) in zip(ps, parts):
+        p.form, p.segments, (p.M, p.N), p.c, p.ldc = NT, 1, c.shape, c.data_ptr(), c.stride(0)
+        p.k[0], p.a[0], p.b[0], p.lda[0], p.ldb[0] = K, x.data_ptr(), b.data_ptr(), x.stride(0), b.stride(0)
+    code = {torch.bfloat16: _lib.MLTS_BF16, torch.float32: _lib.MLTS_F32}[dtype]
+    _lib.check(_lib.lib().mlts_gemm_rope(ps, len(ps), code, ctypes.byref(r), torch.cuda.current_stream().cuda_stream))
+    q, k, v = torch.cat(plain, 1).split(widths, 1)
+    heads = lambda t: t.unflatten(0, (B, S)).unflatten(2, (-1, D)).transpose(1, 2)
+    q, k = native().rope_pair(heads(q), heads(k), cos, sin, positions, offset)
+    rows = lambda t: t.transpose(1, 2).flatten(2).flatten(0, 1)
+    for got, want in zip(ys, (rows(q), rows(k), v)):
+        assert torch.equal(got, want)
