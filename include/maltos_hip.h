@@ -298,6 +298,13 @@ typedef struct {
 int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* products, int32_t count, int32_t dtype);
 int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
                     mlts_stream_t stream);
+/* The backward pass of h W^T (W [K, N], h = round(silu(gate)) * up) in one launch: dW (+)= dy^T h (dense; null: not wanted), and d gate,
+ * d up of dh = dy W, which is not written: the values of two products and mlts_swiglu_bwd_rows.  supports: NULL and the workspace it takes, or why not. */
+const char* mlts_gemm_swiglu_bwd_supports(int32_t dtype, int32_t weight, int64_t M, int64_t N, int64_t K, int64_t ldy, int64_t ldw, int64_t ldh,
+                                          int64_t ldg, int64_t ldd, int64_t* workspace_bytes);
+int mlts_gemm_swiglu_bwd(int32_t dtype, int64_t M, int64_t N, int64_t K, const void* dy, int64_t ldy, const void* w, int64_t ldw, const void* h,
+                         int64_t ldh, void* dw, int32_t accumulate, const void* gate, const void* up, int64_t ldg, void* dgate, void* dup,
+                         int64_t ldd, void* workspace, int64_t workspace_bytes, mlts_stream_t stream);
 /* NT products of one call, some of whose columns are heads that are rotated to their positions as they are written
  * (models/llama.py:143-146): the values of mlts_gemm_multi followed by mlts_rope over them.  Row r is token r % seq of its batch row, at
  * positions[r], or at position_offset + r % seq.  columns[i]: two ranges [begin, end) of whole heads of product i (empty: begin = end).

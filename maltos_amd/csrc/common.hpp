@@ -84,6 +84,13 @@ __device__ __forceinline__ float round_to(float x) {
   return to_f32<T>(from_f32<T>(x));
 }
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }  // the form ATen evaluates
+// d gate and d up of silu(gate) * up
+__device__ __forceinline__ void swiglu_grads(float dh, float gate, float up, float* dgate, float* dup) {
+#pragma clang fp contract(off)
+  const float sg = 1.0f / (1.0f + expf(-gate));
+  *dup = dh * (gate * sg);
+  *dgate = dh * up * (sg * (1.0f + gate * (1.0f - sg)));
+}
 
 // 16-byte vector of T
 template <typename T>

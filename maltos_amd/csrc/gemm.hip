@@ -161,6 +161,13 @@ __device__ __forceinline__ void rotate(float& even, float& odd, float c, float s
   even = round_to<T>(xe * c) - round_to<T>(xo * s);
   odd = round_to<T>(xe * s) + round_to<T>(xo * c);
 }
+// What becomes of dh = dy W_down, an NN product, instead of being written: d gate and d up of the activation (mlts_swiglu_bwd_rows of the
+// rounded dh).  Strides in elements.
+struct Activation {
+  const void *gate, *up;
+  void *dgate, *dup;
+  int ld_in, ld_out;
+};
 // The contraction of the NN form may be a concatenation (dx = sum dy_i W_i of layers that share their input): what follows the
 // first part.  In bf16 each part is rounded, and added to the parts before it in bf16: the values of separate products whose
 // results are added, bit for bit.
@@ -195,9 +202,9 @@ struct TileShape {
 // One tile of one product.  KG > 1: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
 // LDS, where all of them add up and write out a part of the tile (us, one of them / all: fp32 NT 2048 x 256 x 256 7.2 / 6.7,
 // 500 x 512 x 512 8.0 / 7.0).
-template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false, bool ROPE = false>
+template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false, bool ROPE = false, bool ACT = false>
 __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr,
-                                          const Rotation* rot = nullptr, int product = 0) {
+                                          const Rotation* rot = nullptr, int product = 0, const Activation* act = nullptr) {
   typedef TileShape<T, FORM, BM, BN, WM, WN, KG, PAIR> S;
   constexpr int WAVES_N = S::WAVES_N, MB = S::MB, NB = S::NB, SETS = S::SETS, STAGE = S::STAGE;
   typedef typename S::SA SA;
@@ -272,7 +279,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   // of a training step of 8 layers).
   constexpr int OUT_LANES = KG > 1 ? S::THREADS : 64;  // that write a block of 32 rows of C
   constexpr int LPR = WN / 4, RPP = OUT_LANES / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
-  constexpr bool EARLY = !PAIR && !ROPE && (KG > 1 || MB * NB == 1);
+  constexpr bool EARLY = !PAIR && !ROPE && !ACT && (KG > 1 || MB * NB == 1);
   typedef T t4 __attribute__((ext_vector_type(4)));
   t4 old[EARLY ? MB * PASSES : 1];
   const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? 0 : wn) + c4;
@@ -284,7 +291,16 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
       if (row < g.M) old[i] = *reinterpret_cast<const t4*>(static_cast<const T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col);
     }
   }
-  // ... and what it is rotated by, likewise
+  // ... and the activation's operands, and what it is rotated by, likewise
+  static_assert(!ACT || MB * NB == 1, "small tiles");
+  t4 gates[ACT ? PASSES : 1], ups[ACT ? PASSES : 1];
+  if constexpr (ACT) {
+#pragma unroll
+    for (int r = 0; r < PASSES; ++r) {
+      const int64_t at = static_cast<int64_t>(min(m0 + wm + r * RPP + out_lane / LPR, g.M - 1)) * act->ld_in + min(col, g.N - 4);
+      gates[r] = *reinterpret_cast<const t4*>(static_cast<const T*>(act->gate) + at), ups[r] = *reinterpret_cast<const t4*>(static_cast<const T*>(act->up) + at);
+    }
+  }
   constexpr bool EARLY_ANGLES = ROPE && MB * NB == 1;
   typedef T t2 __attribute__((ext_vector_type(2)));
   t2 cosines[EARLY_ANGLES ? PASSES : 1], sines[EARLY_ANGLES ? PASSES : 1];
@@ -431,6 +447,18 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
 #pragma unroll
       for (int o = 1; o < KG; ++o) v += *reinterpret_cast<const f32x4*>(stage + (o * 32 + rr) * ROW + c4);
       if (row >= g.M || col >= g.N) continue;
+      if constexpr (ACT) {
+        t4 dgate, dup;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float dg, du;
+          swiglu_grads(round_to<T>(v[e]), to_f32<T>(gates[r][e]), to_f32<T>(ups[r][e]), &dg, &du);
+          dgate[e] = from_f32<T>(dg), dup[e] = from_f32<T>(du);
+        }
+        const int64_t at = static_cast<int64_t>(row) * act->ld_out + col;
+        *reinterpret_cast<t4*>(static_cast<T*>(act->dgate) + at) = dgate, *reinterpret_cast<t4*>(static_cast<T*>(act->dup) + at) = dup;
+        continue;
+      }
       if constexpr (ROPE) {
         if (rotated) {
           t2 c = cosines[EARLY_ANGLES ? r : 0], s = sines[EARLY_ANGLES ? r : 0];
@@ -529,6 +557,18 @@ __global__ __launch_bounds__(256) void gemm_multi_rope_kernel(const Products ps,
   const Product& g = ps.p[i];
   const int tile = tile_of(block - first, g.tiles_m * g.tiles_n);
   if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false, false, true>(g, tile, lds, ps.more, 0, nullptr, &rot, i);
+}
+
+// dW = dy^T h (if it is wanted), and dh = dy W on its way through the activation
+template <typename T, int BM, int BN, int KG>
+__global__ __launch_bounds__(256) void gemm_multi_act_kernel(const Products ps, const Activation act) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int block = static_cast<int>(blockIdx.x), i = block >= ps.first[1] ? 1 : 0;
+  const Product& g = ps.p[i];
+  const int tile = tile_of(block - ps.first[i], g.tiles_m * g.tiles_n * g.slices);
+  if (tile < 0) return;
+  if (g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, 32, 32, KG, false, false, false, true>(g, tile, lds, ps.more, 0, nullptr, nullptr, 0, &act);
+  else gemm_tile<T, FORM_TN, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
 }
 
 // C (+)= sum of the slices' fp32 partial products, one rounding; up to kMaxProducts outputs
@@ -730,6 +770,16 @@ int launch_rope_small(const Products& ps, const Rotation& rot, int blocks, hipSt
   return MLTS_OK;
 }
 
+template <typename T, int BM, int BN, int KG>
+int launch_act_small(const Products& ps, const Activation& act, int blocks, hipStream_t st) {
+  constexpr int bytes = std::max(TileShape<T, FORM_NN, BM, BN, 32, 32, KG>::LDS, TileShape<T, FORM_TN, BM, BN, 32, 32, KG>::LDS);
+  auto kern = gemm_multi_act_kernel<T, BM, BN, KG>;
+  static MltsLdsOptIn once;
+  if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), bytes, "mlts_gemm_swiglu_bwd"); rc != MLTS_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), bytes, st, ps, act);
+  return MLTS_OK;
+}
+
 template <typename T, int FORMS, int BM, int BN, int KG>
 int launch_small(const Products& ps, int blocks, hipStream_t st) {
   constexpr int nt = TileShape<T, FORM_NT, BM, BN, 32, 32, KG>::LDS, nn = TileShape<T, FORM_NN, BM, BN, 32, 32, KG>::LDS,
@@ -793,9 +843,10 @@ mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const vo
   return p;
 }
 
-// rotation: of the outputs (products of the NT form, not split), or null
+// rotation: of the outputs (products of the NT form, not split), or null.  activation: of the output of the NN product (small, not split),
+// alone or beside one of the TN form, or null.
 template <typename T>
-int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, const Rotation* rotation, hipStream_t st) {
+int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, const Rotation* rotation, const Activation* activation, hipStream_t st) {
   const LaunchPlan plan(ps, count, dtype);
   Rotation rot{};
   if (rotation) rot = *rotation;
@@ -810,6 +861,12 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
   };
   auto launch = [&] {  // what `joint` holds
     if (!smalls) return static_cast<int>(MLTS_OK);
+    if (activation) {
+      if constexpr (sizeof(T) == 4) {
+        if (plan.shape.size == 32) return launch_act_small<T, 32, 32, 4>(joint, *activation, blocks, st);
+      }
+      return launch_act_small<T, 64, 64, 1>(joint, *activation, blocks, st);
+    }
     if (rotation) {
       if constexpr (sizeof(T) == 4) {
         if (plan.shape.size == 32) return launch_rope_small<T, 32, 32, 4>(joint, rot, blocks, st);
@@ -856,7 +913,7 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
       joins.p[joins.count++] = {p.c, g.partial, g.slices, g.accumulate, join_blocks, p.M * p.N / 4};
       join_blocks += static_cast<int>((p.M * p.N / 4 + 255) / 256);
     }
-    if (small && (count > 1 || p.segments > 1)) {
+    if (small && (count > 1 || p.segments > 1 || activation)) {
       all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN;
       joint.first[smalls] = blocks;
       if (rotation) std::copy(rotation->columns[i], rotation->columns[i] + 4, rot.columns[smalls]);
@@ -943,7 +1000,7 @@ extern "C" int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count,
   MLTS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && mlts_aligned16(workspace)), "mlts_gemm: workspace too small or unaligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
   float* ws = static_cast<float*>(workspace);
-  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, ws, nullptr, st) : run<float>(products, count, dtype, ws, nullptr, st);
+  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, ws, nullptr, nullptr, st) : run<float>(products, count, dtype, ws, nullptr, nullptr, st);
 }
 
 extern "C" int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, const void* a, int64_t lda, const void* b, int64_t ldb,
@@ -1006,5 +1063,47 @@ extern "C" int mlts_gemm_rope(const mlts_gemm_product* products, int32_t count, 
   for (int i = 0; i < count; ++i)
     for (int k = 0; k < 4; ++k) r.columns[i][k] = static_cast<int>(rotation->columns[i][k]);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, nullptr, &r, st) : run<float>(products, count, dtype, nullptr, &r, st);
+  return dtype == MLTS_BF16 ? run<bf16_t>(products, count, dtype, nullptr, &r, nullptr, st) : run<float>(products, count, dtype, nullptr, &r, nullptr, st);
+}
+
+// the products of the last projection's backward pass: dW, if it is wanted, then dh
+static int swiglu_bwd_products(mlts_gemm_product (&ps)[2], int64_t M, int64_t N, int64_t K, const void* dy, int64_t ldy, const void* w, int64_t ldw,
+                               const void* h, int64_t ldh, void* dw, int32_t accumulate, bool weight) {
+  int count = 0;
+  if (weight) ps[count++] = single(FORM_TN, K, N, M, dy, ldy, h, ldh, dw, N, accumulate);
+  ps[count++] = single(FORM_NN, M, N, K, dy, ldy, w, ldw, nullptr, N, 0);
+  return count;
+}
+
+extern "C" const char* mlts_gemm_swiglu_bwd_supports(int32_t dtype, int32_t weight, int64_t M, int64_t N, int64_t K, int64_t ldy, int64_t ldw, int64_t ldh,
+                                                     int64_t ldg, int64_t ldd, int64_t* workspace_bytes) {
+  if (dtype != MLTS_BF16 && dtype != MLTS_F32) return "dtype must be MLTS_F32 or MLTS_BF16";
+  if (M <= 0 || N <= 0 || K <= 0) return "an empty product";
+  mlts_gemm_product ps[2];
+  const int count = swiglu_bwd_products(ps, M, N, K, nullptr, ldy, nullptr, ldw, nullptr, ldh, nullptr, 0, weight != 0);
+  for (int i = 0; i < count; ++i)
+    if (const char* why = why_not(ps[i], dtype)) return why;
+  if (N % 4 || ldg % 4 || ldd % 4 || ldg < N || ldd < N || ldg > 0x7fffffff || ldd > 0x7fffffff) return "rows of gate and up are taken four elements at a time";
+  const LaunchPlan plan(ps, count, dtype);
+  if (plan.smalls != count || plan.slices[count - 1] > 1) return "products of this size are not made in one launch";
+  *workspace_bytes = plan.workspace;
+  return nullptr;
+}
+
+extern "C" int mlts_gemm_swiglu_bwd(int32_t dtype, int64_t M, int64_t N, int64_t K, const void* dy, int64_t ldy, const void* w, int64_t ldw, const void* h,
+                                    int64_t ldh, void* dw, int32_t accumulate, const void* gate, const void* up, int64_t ldg, void* dgate, void* dup,
+                                    int64_t ldd, void* workspace, int64_t workspace_bytes, mlts_stream_t stream) {
+  int64_t need = 0;
+  const char* why = mlts_gemm_swiglu_bwd_supports(dtype, dw != nullptr, M, N, K, ldy, ldw, ldh, ldg, ldd, &need);
+  MLTS_REQUIRE(why == nullptr, "mlts_gemm_swiglu_bwd: %s", why);
+  for (const void* p : {dy, w, gate, up, static_cast<const void*>(dgate), static_cast<const void*>(dup)})
+    MLTS_REQUIRE(p && mlts_aligned16(p), "mlts_gemm_swiglu_bwd: pointers must be 16-byte aligned and not null");
+  MLTS_REQUIRE(!dw || (h && mlts_aligned16(h) && mlts_aligned16(dw)), "mlts_gemm_swiglu_bwd: pointers must be 16-byte aligned and not null");
+  MLTS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && mlts_aligned16(workspace)), "mlts_gemm_swiglu_bwd: workspace too small or unaligned");
+  mlts_gemm_product ps[2];
+  const int count = swiglu_bwd_products(ps, M, N, K, dy, ldy, w, ldw, h, ldh, dw, accumulate, dw != nullptr);
+  const Activation act{gate, up, dgate, dup, static_cast<int>(ldg), static_cast<int>(ldd)};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  float* ws = static_cast<float*>(workspace);
+  return dtype == MLTS_BF16 ? run<bf16_t>(ps, count, dtype, ws, nullptr, &act, st) : run<float>(ps, count, dtype, ws, nullptr, &act, st);
 }

@@ -299,7 +299,6 @@ __global__ __launch_bounds__(kThreads) void rope_pair_kernel(const RopeOperand a
 }
 
 // ============================== SwiGLU ===================================================
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void swiglu_fwd_kernel(const T* __restrict__ gate, const T* __restrict__ up,
@@ -333,10 +332,9 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_kernel(const T* __restric
     Vec16<T> og, ou;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const float gj = g.get(j), dj = d.get(j);
-      const float sg = sigmoidf_(gj);
-      ou.set(j, dj * (gj * sg));
-      og.set(j, dj * u.get(j) * (sg * (1.0f + gj * (1.0f - sg))));
+      float dg, du;
+      swiglu_grads(d.get(j), g.get(j), u.get(j), &dg, &du);
+      ou.set(j, du), og.set(j, dg);
     }
     reinterpret_cast<Vec16<T>*>(dgate)[i] = og;
     reinterpret_cast<Vec16<T>*>(dup)[i] = ou;
@@ -378,10 +376,9 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_rows_kernel(const T* __re
     Vec16<T> og, ou;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const float gj = g.get(j), dj = d.get(j);
-      const float sg = sigmoidf_(gj);
-      ou.set(j, dj * (gj * sg));
-      og.set(j, dj * u.get(j) * (sg * (1.0f + gj * (1.0f - sg))));
+      float dg, du;
+      swiglu_grads(d.get(j), g.get(j), u.get(j), &dg, &du);
+      ou.set(j, du), og.set(j, dg);
     }
     *reinterpret_cast<Vec16<T>*>(dgate + out) = og;
     *reinterpret_cast<Vec16<T>*>(dup + out) = ou;
@@ -401,10 +398,10 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_tail(const T* dh, const T
                                                             int64_t start, int64_t n) {
   int64_t i = start + static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (i >= n) return;
-  const float gj = to_f32<T>(gate[i]), dj = to_f32<T>(dh[i]);
-  const float sg = sigmoidf_(gj);
-  dup[i] = from_f32<T>(dj * (gj * sg));
-  dgate[i] = from_f32<T>(dj * to_f32<T>(up[i]) * (sg * (1.0f + gj * (1.0f - sg))));
+  float dg, du;
+  swiglu_grads(to_f32<T>(dh[i]), to_f32<T>(gate[i]), to_f32<T>(up[i]), &dg, &du);
+  dup[i] = from_f32<T>(du);
+  dgate[i] = from_f32<T>(dg);
 }
 
 int stream_grid(int64_t nvec) {

@@ -790,6 +790,31 @@ Tensor attention_block(const Tensor& x, const BlockWeights& w, int64_t heads, in
   return y;
 }
 
+// the gradients of an MLP's gate and up side by side, and (need_dw) of its last projection's weight, in one launch; undefined: sizes and
+// layouts that are left to the products and the pass over gate and up
+std::pair<Tensor, Tensor> activation_and_weight_grad(const Tensor& dy2, const Tensor& w, const Tensor& h2, const Tensor& gu, const Adjacent& rows,
+                                                     const Tensor& grad, bool need_dw) {
+  const int64_t cols = w.size(1), es = gu.element_size(), width = gu.size(-1);
+  if (width != 2 * cols || !gu.is_contiguous() || !aligned(gu) || (rows.first[0] * es) % 16 || (rows.first[1] * es) % 16 ||
+      !own_product(MLTS_GEMM_NN, dy2, w) || (need_dw && !own_product(MLTS_GEMM_TN, dy2, h2)) || gu.scalar_type() != dy2.scalar_type() || gu.numel() / width != dy2.size(0) ||
+      (grad.defined() && (!own_output(grad, h2) || !grad.is_contiguous())))
+    return {};
+  int64_t ws_bytes = 0;
+  const int dtype = dtype_code(dy2);
+  if (mlts_gemm_swiglu_bwd_supports(dtype, need_dw, dy2.size(0), cols, dy2.size(1), dy2.stride(0), w.stride(0), h2.stride(0), width, width,
+                                    &ws_bytes) != nullptr)
+    return {};
+  const Tensor dgu = at::empty(gu.sizes(), gu.options());
+  const Tensor dw = grad.defined() ? grad : need_dw ? at::empty(w.sizes(), dy2.options()) : Tensor();
+  const Tensor ws = workspace(ws_bytes, dy2);
+  const char* in = static_cast<const char*>(ptr(gu));
+  char* out = static_cast<char*>(mptr(dgu));
+  check(mlts_gemm_swiglu_bwd(dtype, dy2.size(0), cols, dy2.size(1), ptr(dy2), dy2.stride(0), ptr(w), w.stride(0), ptr(h2), h2.stride(0), need_dw ? mptr(dw) : nullptr,
+                             grad.defined(), in + rows.first[0] * es, in + rows.first[1] * es, width, out + rows.first[0] * es, out + rows.first[1] * es, width,
+                             ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
+  return {dgu, dw};
+}
+
 struct MlpBlockBackward final : BlockFormula {
   enum { X, GU, H, OUT_W, COUNT };
   MlpBlockBackward() : BlockFormula(COUNT) {}
@@ -797,9 +822,19 @@ struct MlpBlockBackward final : BlockFormula {
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(4);
     const Needed need = needed();
-    auto [dh, dw] = output_grads(g[0], s[OUT_W], rows2d(s[H]), need);
-    if (!dh.defined()) return {Tensor(), Tensor(), Tensor(), dw};
-    const Tensor dgu = swiglu_rows_backward(dh.view(s[H].sizes()), dense(s[GU]), rows->first[0], rows->first[1], weights[0].size(0));
+    Tensor dgu, dw;
+    if (need.input || need.any_weight) {
+      const bool need_dw = task_should_compute_output(1 + weights.size());
+      const Tensor grad = need_dw ? bound_grad(s[OUT_W], into_grad_out) : Tensor();
+      std::tie(dgu, dw) = activation_and_weight_grad(rows2d(dense(g[0])), s[OUT_W], rows2d(s[H]), dense(s[GU]), *rows, grad, need_dw);
+      if (dgu.defined() && grad.defined()) dw = Tensor(), notify_grad_written(s[OUT_W]);
+    }
+    if (!dgu.defined()) {
+      Tensor dh;
+      std::tie(dh, dw) = output_grads(g[0], s[OUT_W], rows2d(s[H]), need);
+      if (!dh.defined()) return {Tensor(), Tensor(), Tensor(), dw};
+      dgu = swiglu_rows_backward(dh.view(s[H].sizes()), dense(s[GU]), rows->first[0], rows->first[1], weights[0].size(0));
+    }
     variable_list out = grads_of_all(*rows, weights, into_grad, need, s[X], rows2d(dgu));
     out.push_back(dw);
     return out;

@@ -220,3 +220,25 @@ def test_rotation_in_the_products(dev, dtype, B, S, H, Hkv, D, K, joint, given):
     rows = lambda t: t.transpose(1, 2).flatten(2).flatten(0, 1)
     for got, want in zip(ys, (rows(q), rows(k), v)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("accumulate", [0, 1, None], ids=["written", "added", "frozen"])
+@pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 8, 8, 8), (torch.bfloat16, 136, 72, 200), (torch.bfloat16, 1016, 1376, 512),
+                                         (torch.float32, 100, 36, 72), (torch.float32, 2048, 688, 256), (torch.float32, 1000, 1376, 512)])
+def test_activation_gradients_in_the_products(dev, dtype, M, N, K, accumulate):
+    """dW and dh = dy W in one launch with dh going through the activation: remainders of tiles, split dW, added onto, written or not
+    wanted; the bits of the products and the pass over gate and up."""
+    gen = torch.Generator().manual_seed(M + N)
+    rnd = lambda *s: torch.randn(*s, generator=gen).to(dtype).to(dev)
+    dy, w, h, gu, dw = rnd(M, K), rnd(K, N), rnd(M, N), rnd(M, 2 * N), rnd(K, N)
+    want_dw, dh = dw.clone(), torch.empty(M, N, dtype=dtype, device=dev)
+    both = [] if accumulate is None else [(TN, [(dy, h)], want_dw, accumulate)]
+    run_products(both + [(NN, [(dy, w)], dh, 0)], dtype)
+    want = native().swiglu_rows_backward(dh, gu, 0, N, N)
+    code, es, L, need = {torch.bfloat16: _lib.MLTS_BF16, torch.float32: _lib.MLTS_F32}[dtype], gu.element_size(), _lib.lib(), ctypes.c_int64()
+    assert L.mlts_gemm_swiglu_bwd_supports(code, len(both), M, N, K, K, N, N, 2 * N, 2 * N, ctypes.byref(need)) is None
+    ws, dgu = torch.empty(max(16, need.value), dtype=torch.uint8, device=dev), torch.full_like(gu, 7.0)
+    _lib.check(L.mlts_gemm_swiglu_bwd(code, M, N, K, dy.data_ptr(), K, w.data_ptr(), N, h.data_ptr(), N, dw.data_ptr() if both else None, accumulate or 0, gu.data_ptr(),
+                                      gu.data_ptr() + N * es, 2 * N, dgu.data_ptr(), dgu.data_ptr() + N * es, 2 * N, ws.data_ptr(), need.value,
+                                      torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(dw, want_dw) and torch.equal(dgu, want)
