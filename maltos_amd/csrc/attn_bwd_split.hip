@@ -1,4 +1,4 @@
-// Attention backward, dK and dV, head_dim 64 and 128, bf16: two-role workgroup.
+// Attention backward, dK and dV, head_dim 64 and 128, bf16: two-role workgroup.  (head_dim 64 on large grids: attn_bwd_dkv64.hip)
 //
 // A workgroup owns 128 keys (small grids: 64) of one (batch, kv head) and walks the 64-row query tiles that can see them
 // (all query heads of the GQA group); its EIGHT (four) wavefronts come in two roles per 32-key block kb = wave % KB:

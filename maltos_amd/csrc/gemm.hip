@@ -505,6 +505,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_kernel(c
   if (tile >= 0) gemm_tile<T, FORM, BM, BN, WM, WN, KG, false>(g, tile, lds, MoreSegments{}, 0);
 }
 
+// us in a training step, product and pass / rotated here: q, k, v of 1023 rows as one 1536 x 512 product 7.5 + 3.7 / 9.1; of 2331 rows as
+// three 11.9 + 4.0 / 12.8; fp32 of 2048 rows as three 256 x 256 12.8 + 3.9 / 14.1.
 template <typename T, int BM, int BN, int WM, int WN, int KG>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_rope_kernel(const Product g, const Rotation rot) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -559,7 +561,8 @@ __global__ __launch_bounds__(256) void gemm_multi_rope_kernel(const Products ps,
   if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false, false, true>(g, tile, lds, ps.more, 0, nullptr, &rot, i);
 }
 
-// dW = dy^T h (if it is wanted), and dh = dy W on its way through the activation
+// dW = dy^T h (if it is wanted), and dh = dy W on its way through the activation (1023 rows, 1376 x 512: 13.4 us and 5.1 for the pass /
+// 16.3 here)
 template <typename T, int BM, int BN, int KG>
 __global__ __launch_bounds__(256) void gemm_multi_act_kernel(const Products ps, const Activation act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
