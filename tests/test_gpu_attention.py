@@ -344,6 +344,32 @@ def test_backward_accumulation_modes(dev, dtype, D, mode):
         assert torch.allclose(dk - 1, dk0, **tol) and torch.allclose(dv - 1, dv0, **tol)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,mode", [(1, 4, 2, 545, 64, ops.MASK_CAUSAL), (1, 4, 2, 530, 128, ops.MASK_DOC), (20, 8, 8, 530, 64, ops.MASK_CAUSAL),
+                                               (16, 8, 8, 513, 64, ops.MASK_DOC)])
+def test_backward_accumulation_modes_of_long_walks(dev, B, Hq, Hkv, S, D, mode):
+    """The same modes in the 16-row kernels and in dK/dV of large grids."""
+    gen = torch.Generator().manual_seed(S + D)
+    q, k, v, do = (bshd(B, h, S, D, gen, torch.bfloat16).to(dev) for h in (Hq, Hkv, Hkv, Hq))
+    kw = {}
+    if mode == ops.MASK_DOC:
+        pos, seq = (t.to(dev) for t in make_docs(B, S, gen, 190, pad_tail=7))
+        kw = dict(q_pos=pos, k_pos=pos, q_seq=seq, k_seq=seq)
+    o, lse = ops.attention_forward(q, k, v, mask_mode=mode, **kw)
+    dq0, dk0, dv0 = ops.attention_backward(do, q, k, v, o, lse, mask_mode=mode, **kw)
+    first = torch.full(q.shape, float("nan"), device=dev)
+    dk, dv = torch.full_like(k, float("nan")), torch.full_like(v, float("nan"))
+    ops.attention_backward_ring_block(do, q, k, v, o, lse, first, dk, dv, first=True, mask_mode=mode, **kw)
+    assert torch.equal(first.to(torch.bfloat16), dq0) and torch.equal(dk, dk0) and torch.equal(dv, dv0)
+    dq = first.clone()
+    ops.attention_backward_ring_block(do, q, k, v, o, lse, dq, dk, dv, first=False, mask_mode=mode, **kw)
+    assert torch.equal(dq, first + first) and torch.equal(dk, dk0) and torch.equal(dv, dv0)
+    grads = [torch.ones(t.shape, device=dev) for t in (q, k, v)]
+    ops.attention_backward_accumulate(do, q, k, v, o, lse, *grads, mask_mode=mode, **kw)
+    assert torch.allclose(grads[0], first + 1, rtol=1e-6, atol=1e-6)   # (the product and the addition may be one fused operation)
+    for got, want in zip(grads[1:], (dk0, dv0)):
+        assert torch.allclose(got - 1, want.float(), rtol=2.0 ** -7, atol=1e-5)
+
+
 @pytest.mark.parametrize("D", [1, 3, 24, 96, 192])
 def test_generic_head_dims(dev, D):
     run_case(dev, torch.float32, 1, 2, 1, 70, 70, D, ops.MASK_CAUSAL, seed=D)
