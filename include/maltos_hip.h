@@ -108,7 +108,12 @@ int mlts_attn_doc_plan(const mlts_attn_shape* s, void* plan, int64_t plan_bytes,
 /* O = softmax(scale * Q K^T + mask) V and LSE = logsumexp (natural log, fp32, [B, Hq, Sq]).
  * Replaces F.scaled_dot_product_attention (utils/attention_backend.py:60-64,109-116),
  * flash_attn_dense / flash_attn_dense_with_lse / flash_attn_varlen
- * (runtime/layers/flash_utils.py:180-215,266-276,493-520). */
+ * (runtime/layers/flash_utils.py:180-215,266-276,493-520).
+ *
+ * Bits (this call and mlts_attn_bwd): the same call gives the same bits every time.  A batch row in a call on more rows has
+ * the bits of a call on that row alone only for MLTS_BF16 at D 64 and 128 whose walk is shorter than 512 rows (O, LSE and dQ: Sk < 512;
+ * dK and dV: Sq < 512).  Otherwise the kernel, or how many wavefronts share a row's walk, follows the size of the whole
+ * call, and a row's last bits may change with B; so they may with the linear layers' products below. */
 int mlts_attn_fwd(const mlts_attn_shape* s, const void* q, const void* k, const void* v, void* o,
                   float* lse, void* workspace, int64_t workspace_bytes, mlts_stream_t stream);
 

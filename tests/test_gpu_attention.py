@@ -184,6 +184,43 @@ def test_small_grids_equal_large_ones(dev, D, mode, Hq, Hkv, Sq, Sk):
             assert torch.equal(got[row], want), (b, name)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mode", [ops.MASK_NONE, ops.MASK_CAUSAL, ops.MASK_DOC])
+@pytest.mark.parametrize("Hq,Hkv,Sq,Sk", [(8, 4, 511, 511), (4, 2, 511, 96), (12, 12, 40, 511)])
+def test_walks_of_511_rows_have_the_arithmetic_of_large_grids(dev, D, mode, Hq, Hkv, Sq, Sk):
+    """The longest walks of which a batch row still has the bits of a call on it alone."""
+    test_small_grids_equal_large_ones(dev, D, mode, Hq, Hkv, Sq, Sk)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mode", [ops.MASK_NONE, ops.MASK_CAUSAL, ops.MASK_DOC])
+def test_walks_of_512_rows_alone_and_in_a_batch(dev, D, mode):
+    """From 512 rows on a row alone and in a batch go to different kernels: each gives the same bits every time, and both are
+    within the bounds of a bf16 output (dQ, dK, dV and O of the other kernel in the place of the oracle's)."""
+    B, H, S = 20, 8, 512
+    gen = torch.Generator().manual_seed(S + D)
+    q, k, v, do = (bshd(B, H, S, D, gen, torch.bfloat16).to(dev) for _ in range(4))
+    ids = {}
+    if mode == ops.MASK_DOC:
+        pos, doc = (t.to(dev) for t in make_docs(B, S, gen, 200, pad_tail=3))
+        ids = dict(q_pos=pos, k_pos=pos, q_seq=doc, k_seq=doc)
+
+    def run(rows):
+        one = {name: t[rows] for name, t in ids.items()}
+        o, lse = ops.attention_forward(q[rows], k[rows], v[rows], mask_mode=mode, **one)
+        return (o, lse, *ops.attention_backward(do[rows], q[rows], k[rows], v[rows], o, lse, mask_mode=mode, **one))
+
+    row = slice(B // 2, B // 2 + 1)
+    alone, batch = run(row), run(slice(0, B))
+    for first, again in ((alone, run(row)), (batch, run(slice(0, B)))):
+        assert all(torch.equal(a, b) for a, b in zip(first, again))
+    for name, a, b in zip(("O", "LSE", "dQ", "dK", "dV"), alone, (t[row] for t in batch)):
+        if name == "LSE":
+            assert torch.equal(torch.isfinite(a), torch.isfinite(b)) and (a - b)[torch.isfinite(a)].abs().max() <= 1e-4
+        else:
+            check(a, b, torch.bfloat16, name)
+
+
 @pytest.mark.parametrize("seed", range(10))
 def test_document_mask_drawn_shapes(dev, seed):
     """Drawn batch sizes, head groupings (1, 2, 3, 4, 8 query heads per KV head: the forward and dQ workgroups take one,
