@@ -22,24 +22,19 @@ namespace {
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
 constexpr int kTile = 64;  // rows of the walked side per LDS stage: two units of 32
+constexpr int kVec = 8;    // elements of a 16-byte vector: a fragment
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 #define MLTS_LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
 
 // DP: head_dim rounded up to a multiple of 32 (the padding is zero in every operand)
-template <typename T, int DP>
-struct Tile16;
-
 template <int DP>
-struct Tile16<bf16_t, DP> {
+struct Tile16 {
   static constexpr int STEP = 32;
   static constexpr int FRAGS = DP / STEP;
-  static constexpr int PER = 8;
   static constexpr int LS = DP + 8;
-  typedef bf16x8 frag;
-  static __device__ __forceinline__ f32x4 dot(frag a, frag b, f32x4 acc) {
+  static __device__ __forceinline__ f32x4 dot(bf16x8 a, bf16x8 b, f32x4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
   }
   static __device__ __forceinline__ void accumulate(f32x4 (&acc)[DP / 16], const bf16_t* unit, const f32x4 (&x)[2], int l16, int g) {
@@ -67,45 +62,42 @@ struct Tile16<bf16_t, DP> {
   }
 };
 
-// columns d0 .. d0 + PER - 1 of a row, zero past D (and everywhere if the row does not exist)
-template <typename T, int DP>
-__device__ __forceinline__ typename Tile16<T, DP>::frag load_frag(const T* row, bool exists, int d0, int D, bool vec) {
-  typedef typename Tile16<T, DP>::frag frag;
-  frag f;
+// columns d0 .. d0 + kVec - 1 of a row, zero past D (and everywhere if the row does not exist)
+__device__ __forceinline__ bf16x8 load_frag(const bf16_t* row, bool exists, int d0, int D, bool vec) {
+  bf16x8 f;
 #pragma unroll
-  for (int e = 0; e < Tile16<T, DP>::PER; ++e) f[e] = static_cast<T>(0.f);
+  for (int e = 0; e < kVec; ++e) f[e] = static_cast<bf16_t>(0.f);
   if (!exists) return f;
   if (vec) {
-    if (d0 < D) f = *reinterpret_cast<const frag*>(row + d0);
+    if (d0 < D) f = *reinterpret_cast<const bf16x8*>(row + d0);
   } else {
 #pragma unroll
-    for (int e = 0; e < Tile16<T, DP>::PER; ++e)
+    for (int e = 0; e < kVec; ++e)
       if (d0 + e < D) f[e] = row[d0 + e];
   }
   return f;
 }
 
 // A [64][DP] tile on its way from global memory to LDS through registers: fetched while the tile before it is worked on.
-template <typename T, int DP>
+template <int DP>
 struct Stage {
-  static constexpr int PER = 16 / static_cast<int>(sizeof(T));
-  static constexpr int CHUNKS = DP / PER;                        // 16-byte chunks per row
+  static constexpr int CHUNKS = DP / kVec;                       // 16-byte chunks per row
   static constexpr int N = kTile * CHUNKS / kThreads;            // chunks per lane
   static_assert(kTile * CHUNKS % kThreads == 0, "whole chunks per lane");
-  typename Tile16<T, DP>::frag r[N];
-  __device__ __forceinline__ void fetch(const T* base, int64_t row_stride, int row0, int limit, int D, bool vec) {
+  bf16x8 r[N];
+  __device__ __forceinline__ void fetch(const bf16_t* base, int64_t row_stride, int row0, int limit, int D, bool vec) {
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       const int idx = n * kThreads + threadIdx.x;
       const int row = row0 + idx / CHUNKS;
-      r[n] = load_frag<T, DP>(base + static_cast<int64_t>(row) * row_stride, row < limit, (idx % CHUNKS) * PER, D, vec);
+      r[n] = load_frag(base + static_cast<int64_t>(row) * row_stride, row < limit, (idx % CHUNKS) * kVec, D, vec);
     }
   }
-  __device__ __forceinline__ void store(T* lds) const {
+  __device__ __forceinline__ void store(bf16_t* lds) const {
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       const int idx = n * kThreads + threadIdx.x;
-      *reinterpret_cast<typename Tile16<T, DP>::frag*>(lds + (idx / CHUNKS) * Tile16<T, DP>::LS + (idx % CHUNKS) * PER) = r[n];
+      *reinterpret_cast<bf16x8*>(lds + (idx / CHUNKS) * Tile16<DP>::LS + (idx % CHUNKS) * kVec) = r[n];
     }
   }
 };
@@ -130,25 +122,24 @@ __device__ __forceinline__ float max_groups(float x) {
   return fmaxf(x, __shfl_xor(x, 32, 64));
 }
 
-// One row's columns 16 db + 4 g ..+3 as they lie in the accumulators.  mode 0: T, overwritten; 1: fp32, added to; 2: fp32, overwritten.
-template <typename T, int DP>
+// One row's columns 16 db + 4 g ..+3 as they lie in the accumulators.  mode 0: bf16, overwritten; 1: fp32, added to; 2: fp32, overwritten.
+template <int DP>
 __device__ __forceinline__ void store_row(void* base, int64_t off, const f32x4 (&acc)[DP / 16], float scale, int g, int D, bool vec, int mode) {
 #pragma unroll
   for (int db = 0; db < DP / 16; ++db) {
     const int d = 16 * db + 4 * g;
     if (mode == 0 && vec) {
-      typedef T t4 __attribute__((ext_vector_type(4)));
-      t4 w;
+      bf16x4 w;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = from_f32<T>(acc[db][i] * scale);
-      if (d < D) *reinterpret_cast<t4*>(static_cast<T*>(base) + off + d) = w;
+      for (int i = 0; i < 4; ++i) w[i] = from_f32<bf16_t>(acc[db][i] * scale);
+      if (d < D) *reinterpret_cast<bf16x4*>(static_cast<bf16_t*>(base) + off + d) = w;
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if (d + i >= D) continue;
         const float x = acc[db][i] * scale;
         float* f = static_cast<float*>(base) + off + d + i;
-        if (mode == 0) static_cast<T*>(base)[off + d + i] = from_f32<T>(x);
+        if (mode == 0) static_cast<bf16_t*>(base)[off + d + i] = from_f32<bf16_t>(x);
         else if (mode == 1) *f += x;
         else *f = x;
       }
@@ -195,12 +186,12 @@ __device__ __forceinline__ void join_splits(f32x4 (&acc)[N], float* lds, int row
   }
 }
 
-template <typename T, int DP, bool DOC>
+template <int DP, bool DOC>
 __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, const Tile16Args a) {
-  typedef Tile16<T, DP> C;
+  typedef Tile16<DP> C;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  T* sK = reinterpret_cast<T*>(lds_raw);
-  T* sV = sK + kTile * C::LS;
+  bf16_t* sK = reinterpret_cast<bf16_t*>(lds_raw);
+  bf16_t* sV = sK + kTile * C::LS;
   int2* sIds = reinterpret_cast<int2*>(sV + kTile * C::LS);
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -211,14 +202,14 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
   const int nbh = p.B * p.Hq, qt = p.nqt - 1 - static_cast<int>(blockIdx.x) / nbh, bh = static_cast<int>(blockIdx.x) % nbh;
   const int b = bh / p.Hq, hq = bh % p.Hq, hkv = hq / (p.Hq / p.Hkv);
   const int q0 = qt * rows, qrow = q0 + row_wave * 16 + l16;
-  const T* Q = static_cast<const T*>(p.q) + b * p.qs[0] + hq * p.qs[1];
-  const T* K = static_cast<const T*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
-  const T* V = static_cast<const T*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
+  const bf16_t* Q = static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1];
+  const bf16_t* K = static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
+  const bf16_t* V = static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
 
-  typename C::frag qf[C::FRAGS];
+  bf16x8 qf[C::FRAGS];
 #pragma unroll
   for (int j = 0; j < C::FRAGS; ++j)
-    qf[j] = load_frag<T, DP>(Q + static_cast<int64_t>(min(qrow, p.Sq - 1)) * p.qs[2], true, C::STEP * j + C::PER * g, a.D, a.vec);
+    qf[j] = load_frag(Q + static_cast<int64_t>(min(qrow, p.Sq - 1)) * p.qs[2], true, C::STEP * j + kVec * g, a.D, a.vec);
   // keys this lane's query sees: up to klim (p.causal_off is Sk without a causal mask); documents also by their ids
   const int klim = qrow < p.Sq ? min(p.Sk - 1, qrow + p.causal_off) : -1;
   int kend = p.Sk, qpos = 0, qseq = -1;
@@ -254,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
   f32x4 o[DP / 16];
 #pragma unroll
   for (int db = 0; db < DP / 16; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Stage<T, DP> stK, stV;
+  Stage<DP> stK, stV;
   int2 ids = make_int2(0, -2);
   int k0 = next_tile(0);
   auto fetch = [&](int k) {
@@ -274,14 +265,14 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
     for (int u = unit0; u < 2; u += unit_step) {
       const int ku = k0 + 32 * u;
       if (ku >= p.Sk || ku > wave_kmax) continue;
-      const T* ku_rows = sK + (32 * u + l16) * C::LS + C::PER * g;
+      const bf16_t* ku_rows = sK + (32 * u + l16) * C::LS + kVec * g;
       f32x4 s[2];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < C::FRAGS; ++j)
-          s[kb] = C::dot(*reinterpret_cast<const typename C::frag*>(ku_rows + 16 * kb * C::LS + C::STEP * j), qf[j], s[kb]);
+          s[kb] = C::dot(*reinterpret_cast<const bf16x8*>(ku_rows + 16 * kb * C::LS + C::STEP * j), qf[j], s[kb]);
       }
       if (DOC) {
 #pragma unroll
@@ -346,20 +337,20 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_fwd(const AttnParams p, 
     if (split > 0) return;
   }
   if (qrow >= p.Sq) return;
-  store_row<T, DP>(p.o, b * p.os[0] + hq * p.os[1] + static_cast<int64_t>(qrow) * p.os[2], o, l > 0.f ? 1.0f / l : 0.f, g, a.D, a.vec, 0);
+  store_row<DP>(p.o, b * p.os[0] + hq * p.os[1] + static_cast<int64_t>(qrow) * p.os[2], o, l > 0.f ? 1.0f / l : 0.f, g, a.D, a.vec, 0);
   if (g == 0)
     p.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] = l > 0.f ? m + logf(l) : -INFINITY;
 }
 
 // dQ of 64 (32) query rows: dq = scale * sum_j ds_ij k_j, ds = p (dp - delta), p = exp(scale s - lse).  Runs first in a backward
-// pass and writes delta = rowsum(dO * O) for the dK/dV kernel.  bp.dq_f32: dq is fp32 and added to (1) or overwritten (2); 0: T.
-template <typename T, int DP, bool DOC>
+// pass and writes delta = rowsum(dO * O) for the dK/dV kernel.  bp.dq_f32: dq is fp32 and added to (1) or overwritten (2); 0: bf16.
+template <int DP, bool DOC>
 __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdParams bp, const Tile16Args a) {
-  typedef Tile16<T, DP> C;
+  typedef Tile16<DP> C;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  T* sK = reinterpret_cast<T*>(lds_raw);
-  T* sV = sK + kTile * C::LS;
+  bf16_t* sK = reinterpret_cast<bf16_t*>(lds_raw);
+  bf16_t* sV = sK + kTile * C::LS;
   int2* sIds = reinterpret_cast<int2*>(sV + kTile * C::LS);
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -369,22 +360,22 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
   const int nbh = p.B * p.Hq, qt = p.nqt - 1 - static_cast<int>(blockIdx.x) / nbh, bh = static_cast<int>(blockIdx.x) % nbh;
   const int b = bh / p.Hq, hq = bh % p.Hq, hkv = hq / (p.Hq / p.Hkv);
   const int q0 = qt * rows, qrow = q0 + row_wave * 16 + l16, qsafe = min(qrow, p.Sq - 1);
-  const T* Q = static_cast<const T*>(p.q) + b * p.qs[0] + hq * p.qs[1] + static_cast<int64_t>(qsafe) * p.qs[2];
-  const T* dO = static_cast<const T*>(bp.dout) + b * bp.dos[0] + hq * bp.dos[1] + static_cast<int64_t>(qsafe) * bp.dos[2];
-  const T* O = static_cast<const T*>(p.o) + b * p.os[0] + hq * p.os[1] + static_cast<int64_t>(qsafe) * p.os[2];
-  const T* K = static_cast<const T*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
-  const T* V = static_cast<const T*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
+  const bf16_t* Q = static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1] + static_cast<int64_t>(qsafe) * p.qs[2];
+  const bf16_t* dO = static_cast<const bf16_t*>(bp.dout) + b * bp.dos[0] + hq * bp.dos[1] + static_cast<int64_t>(qsafe) * bp.dos[2];
+  const bf16_t* O = static_cast<const bf16_t*>(p.o) + b * p.os[0] + hq * p.os[1] + static_cast<int64_t>(qsafe) * p.os[2];
+  const bf16_t* K = static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
+  const bf16_t* V = static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
 
-  typename C::frag qf[C::FRAGS], dof[C::FRAGS];
+  bf16x8 qf[C::FRAGS], dof[C::FRAGS];
   float delta = 0.f;
 #pragma unroll
   for (int j = 0; j < C::FRAGS; ++j) {
-    const int d0 = C::STEP * j + C::PER * g;
-    qf[j] = load_frag<T, DP>(Q, true, d0, a.D, a.vec);
-    dof[j] = load_frag<T, DP>(dO, true, d0, a.D, a.vec);
-    const typename C::frag of = load_frag<T, DP>(O, true, d0, a.D, a.vec);
+    const int d0 = C::STEP * j + kVec * g;
+    qf[j] = load_frag(Q, true, d0, a.D, a.vec);
+    dof[j] = load_frag(dO, true, d0, a.D, a.vec);
+    const bf16x8 of = load_frag(O, true, d0, a.D, a.vec);
 #pragma unroll
-    for (int e = 0; e < C::PER; ++e) delta += static_cast<float>(dof[j][e]) * static_cast<float>(of[e]);
+    for (int e = 0; e < kVec; ++e) delta += static_cast<float>(dof[j][e]) * static_cast<float>(of[e]);
   }
   delta = sum_groups(delta);
   const int64_t stat = (static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qsafe;
@@ -425,7 +416,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
   f32x4 dq[DP / 16];
 #pragma unroll
   for (int db = 0; db < DP / 16; ++db) dq[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Stage<T, DP> stK, stV;
+  Stage<DP> stK, stV;
   int2 ids = make_int2(0, -2);
   int k0 = next_tile(0);
   auto fetch = [&](int k) {
@@ -445,7 +436,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
     for (int u = unit0; u < 2; u += unit_step) {
       const int ku = k0 + 32 * u;
       if (ku >= p.Sk || ku > wave_kmax) continue;
-      const int frag0 = (32 * u + l16) * C::LS + C::PER * g;
+      const int frag0 = (32 * u + l16) * C::LS + kVec * g;
       f32x4 s[2], dp[2];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
@@ -453,8 +444,8 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
 #pragma unroll
         for (int j = 0; j < C::FRAGS; ++j) {
           const int at = frag0 + 16 * kb * C::LS + C::STEP * j;
-          s[kb] = C::dot(*reinterpret_cast<const typename C::frag*>(sK + at), qf[j], s[kb]);
-          dp[kb] = C::dot(*reinterpret_cast<const typename C::frag*>(sV + at), dof[j], dp[kb]);
+          s[kb] = C::dot(*reinterpret_cast<const bf16x8*>(sK + at), qf[j], s[kb]);
+          dp[kb] = C::dot(*reinterpret_cast<const bf16x8*>(sV + at), dof[j], dp[kb]);
         }
       }
       const bool masked = !DOC && ku + 31 > wave_klim;
@@ -480,17 +471,17 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dq(const AttnBwdPara
     if (split > 0) return;
   }
   if (qrow < p.Sq)
-    store_row<T, DP>(bp.dq_acc, b * bp.dqs[0] + hq * bp.dqs[1] + static_cast<int64_t>(qrow) * bp.dqs[2], dq, p.scale, g, a.D, a.vec, bp.dq_f32);
+    store_row<DP>(bp.dq_acc, b * bp.dqs[0] + hq * bp.dqs[1] + static_cast<int64_t>(qrow) * bp.dqs[2], dq, p.scale, g, a.D, a.vec, bp.dq_f32);
 }
 
 // dK, dV of 64 (32) key rows of one KV head, summed over the query heads of its group.
-template <typename T, int DP, bool DOC>
+template <int DP, bool DOC>
 __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdParams bp, const Tile16Args a) {
-  typedef Tile16<T, DP> C;
+  typedef Tile16<DP> C;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  T* sQ = reinterpret_cast<T*>(lds_raw);
-  T* sdO = sQ + kTile * C::LS;
+  bf16_t* sQ = reinterpret_cast<bf16_t*>(lds_raw);
+  bf16_t* sdO = sQ + kTile * C::LS;
   float2* sStat = reinterpret_cast<float2*>(sdO + kTile * C::LS);  // (lse, delta) of the tile's queries
   int2* sIds = reinterpret_cast<int2*>(sStat + kTile);
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
@@ -502,14 +493,14 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
   const int nbh = p.B * p.Hkv, kt = static_cast<int>(blockIdx.x) / nbh, bh = static_cast<int>(blockIdx.x) % nbh;
   const int b = bh / p.Hkv, hkv = bh % p.Hkv, group = p.Hq / p.Hkv;
   const int kb0 = kt * rows, krow = kb0 + row_wave * 16 + l16, ksafe = min(krow, p.Sk - 1);
-  const T* K = static_cast<const T*>(p.k) + b * p.ks[0] + hkv * p.ks[1] + static_cast<int64_t>(ksafe) * p.ks[2];
-  const T* V = static_cast<const T*>(p.v) + b * p.vs[0] + hkv * p.vs[1] + static_cast<int64_t>(ksafe) * p.vs[2];
-  typename C::frag kf[C::FRAGS], vf[C::FRAGS];
+  const bf16_t* K = static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1] + static_cast<int64_t>(ksafe) * p.ks[2];
+  const bf16_t* V = static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1] + static_cast<int64_t>(ksafe) * p.vs[2];
+  bf16x8 kf[C::FRAGS], vf[C::FRAGS];
 #pragma unroll
   for (int j = 0; j < C::FRAGS; ++j) {
-    const int d0 = C::STEP * j + C::PER * g;
-    kf[j] = load_frag<T, DP>(K, true, d0, a.D, a.vec);
-    vf[j] = load_frag<T, DP>(V, true, d0, a.D, a.vec);
+    const int d0 = C::STEP * j + kVec * g;
+    kf[j] = load_frag(K, true, d0, a.D, a.vec);
+    vf[j] = load_frag(V, true, d0, a.D, a.vec);
   }
   const int qlim = krow < p.Sk ? krow - p.causal_off : 0x7fffffff;          // first query that sees this lane's key
   const int wave_qall = min(kb0 + row_wave * 16 + 15, p.Sk - 1) - p.causal_off;  // from here on every row of the wavefront is seen
@@ -545,12 +536,12 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
   f32x4 dk[DP / 16], dv[DP / 16];
 #pragma unroll
   for (int db = 0; db < DP / 16; ++db) dk[db] = dv[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Stage<T, DP> stQ, stdO;
+  Stage<DP> stQ, stdO;
   float2 stat = make_float2(INFINITY, 0.f);
   int2 ids = make_int2(0, -1);
   auto fetch = [&](int hq, int q) {
-    stQ.fetch(static_cast<const T*>(p.q) + b * p.qs[0] + hq * p.qs[1], p.qs[2], q, p.Sq, a.D, a.vec);
-    stdO.fetch(static_cast<const T*>(bp.dout) + b * bp.dos[0] + hq * bp.dos[1], bp.dos[2], q, p.Sq, a.D, a.vec);
+    stQ.fetch(static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1], p.qs[2], q, p.Sq, a.D, a.vec);
+    stdO.fetch(static_cast<const bf16_t*>(bp.dout) + b * bp.dos[0] + hq * bp.dos[1], bp.dos[2], q, p.Sq, a.D, a.vec);
     if (tid < kTile) {
       stat = make_float2(INFINITY, 0.f);  // probability 0: rows past the end, rows that saw no key
       if (DOC) ids = make_int2(0, -1);
@@ -580,7 +571,7 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
     for (int u = unit0; u < 2; u += unit_step) {
       const int qu = q0 + 32 * u;
       if (qu >= p.Sq || (!DOC && qu + 31 < wave_qmin)) continue;
-      const int frag0 = (32 * u + l16) * C::LS + C::PER * g;
+      const int frag0 = (32 * u + l16) * C::LS + kVec * g;
       f32x4 s[2], dp[2];
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
@@ -588,8 +579,8 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
 #pragma unroll
         for (int j = 0; j < C::FRAGS; ++j) {
           const int at = frag0 + 16 * qb * C::LS + C::STEP * j;
-          s[qb] = C::dot(*reinterpret_cast<const typename C::frag*>(sQ + at), kf[j], s[qb]);
-          dp[qb] = C::dot(*reinterpret_cast<const typename C::frag*>(sdO + at), vf[j], dp[qb]);
+          s[qb] = C::dot(*reinterpret_cast<const bf16x8*>(sQ + at), kf[j], s[qb]);
+          dp[qb] = C::dot(*reinterpret_cast<const bf16x8*>(sdO + at), vf[j], dp[qb]);
         }
       }
       const bool masked = !DOC && (qu < wave_qall || ragged);
@@ -620,13 +611,13 @@ __global__ __launch_bounds__(kThreads) void attn_tile16_bwd_dkv(const AttnBwdPar
     if (split > 0) return;
   }
   if (krow >= p.Sk) return;
-  store_row<T, DP>(bp.dk, b * bp.dks[0] + hkv * bp.dks[1] + static_cast<int64_t>(krow) * bp.dks[2], dk, p.scale, g, a.D, a.vec, bp.accumulate_f32);
-  store_row<T, DP>(bp.dv, b * bp.dvs[0] + hkv * bp.dvs[1] + static_cast<int64_t>(krow) * bp.dvs[2], dv, 1.f, g, a.D, a.vec, bp.accumulate_f32);
+  store_row<DP>(bp.dk, b * bp.dks[0] + hkv * bp.dks[1] + static_cast<int64_t>(krow) * bp.dks[2], dk, p.scale, g, a.D, a.vec, bp.accumulate_f32);
+  store_row<DP>(bp.dv, b * bp.dvs[0] + hkv * bp.dvs[1] + static_cast<int64_t>(krow) * bp.dvs[2], dv, 1.f, g, a.D, a.vec, bp.accumulate_f32);
 }
 
-template <typename T, int DP>
+template <int DP>
 constexpr int lds_bytes() {
-  const int tiles = 2 * kTile * Tile16<T, DP>::LS * static_cast<int>(sizeof(T)) + kTile * 16;
+  const int tiles = 2 * kTile * Tile16<DP>::LS * static_cast<int>(sizeof(bf16_t)) + kTile * 16;
   const int join = 3 * (DP / 16) * 64 * 16;
   return tiles > join ? tiles : join;
 }
@@ -654,39 +645,37 @@ int launch(int lds, int64_t blocks, hipStream_t st, const P& params, const Tile1
   return mlts_check_launch(what);
 }
 
-bool rows_vec(const int64_t* s, const void* ptr, int per) {
-  return ((s[0] | s[1] | s[2]) & (per - 1)) == 0 && mlts_aligned16(ptr);
+bool rows_vec(const int64_t* s, const void* ptr) {
+  return ((s[0] | s[1] | s[2]) & (kVec - 1)) == 0 && mlts_aligned16(ptr);
 }
 
-template <typename T, int DP, bool DOC>
+template <int DP, bool DOC>
 int fwd(AttnParams p, int D, hipStream_t st) {
-  const int per = 16 / static_cast<int>(sizeof(T));
   Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq),
-               D % per == 0 && rows_vec(p.qs, p.q, per) && rows_vec(p.ks, p.k, per) && rows_vec(p.vs, p.v, per) && rows_vec(p.os, p.o, per)};
+               D % kVec == 0 && rows_vec(p.qs, p.q) && rows_vec(p.ks, p.k) && rows_vec(p.vs, p.v) && rows_vec(p.os, p.o)};
   p.nqt = (p.Sq + a.row_waves * 16 - 1) / (a.row_waves * 16);
   MltsKernelTimer timer("attn_fwd", st);
-  return launch<attn_tile16_fwd<T, DP, DOC>>(lds_bytes<T, DP>(), static_cast<int64_t>(p.nqt) * p.B * p.Hq, st, p, a, "mlts_attn_fwd");
+  return launch<attn_tile16_fwd<DP, DOC>>(lds_bytes<DP>(), static_cast<int64_t>(p.nqt) * p.B * p.Hq, st, p, a, "mlts_attn_fwd");
 }
 
-template <typename T, int DP, bool DOC>
+template <int DP, bool DOC>
 int bwd(AttnBwdParams bp, int D, hipStream_t st) {
   AttnParams& p = bp.a;
-  const int per = 16 / static_cast<int>(sizeof(T));
-  const bool in_vec = D % per == 0 && rows_vec(p.qs, p.q, per) && rows_vec(p.ks, p.k, per) && rows_vec(p.vs, p.v, per) &&
-                      rows_vec(bp.dos, bp.dout, per) && rows_vec(p.os, p.o, per);
+  const bool in_vec = D % kVec == 0 && rows_vec(p.qs, p.q) && rows_vec(p.ks, p.k) && rows_vec(p.vs, p.v) &&
+                      rows_vec(bp.dos, bp.dout) && rows_vec(p.os, p.o);
   if (p.Sq > 0) {
-    Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq), in_vec && (bp.dq_f32 || rows_vec(bp.dqs, bp.dq_acc, per))};
+    Tile16Args a{D, row_waves_for(p.Sq, static_cast<int64_t>(p.B) * p.Hq), in_vec && (bp.dq_f32 || rows_vec(bp.dqs, bp.dq_acc))};
     p.nqt = (p.Sq + a.row_waves * 16 - 1) / (a.row_waves * 16);
     MltsKernelTimer timer("attn_bwd_dq", st);
-    if (int rc = launch<attn_tile16_bwd_dq<T, DP, DOC>>(lds_bytes<T, DP>(), static_cast<int64_t>(p.nqt) * p.B * p.Hq, st, bp, a, "mlts_attn_bwd"); rc != MLTS_OK)
+    if (int rc = launch<attn_tile16_bwd_dq<DP, DOC>>(lds_bytes<DP>(), static_cast<int64_t>(p.nqt) * p.B * p.Hq, st, bp, a, "mlts_attn_bwd"); rc != MLTS_OK)
       return rc;
   }
   if (p.Sk == 0) return MLTS_OK;
   Tile16Args a{D, row_waves_for(p.Sk, static_cast<int64_t>(p.B) * p.Hkv),
-               in_vec && (bp.accumulate_f32 || (rows_vec(bp.dks, bp.dk, per) && rows_vec(bp.dvs, bp.dv, per)))};
+               in_vec && (bp.accumulate_f32 || (rows_vec(bp.dks, bp.dk) && rows_vec(bp.dvs, bp.dv)))};
   const int64_t nkt = (p.Sk + a.row_waves * 16 - 1) / (a.row_waves * 16);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
-  return launch<attn_tile16_bwd_dkv<T, DP, DOC>>(lds_bytes<T, DP>(), nkt * p.B * p.Hkv, st, bp, a, "mlts_attn_bwd");
+  return launch<attn_tile16_bwd_dkv<DP, DOC>>(lds_bytes<DP>(), nkt * p.B * p.Hkv, st, bp, a, "mlts_attn_bwd");
 }
 
 // p.causal_off: the last key query i sees is i + causal_off; without a causal mask it is past every key
@@ -694,19 +683,19 @@ void set_causal_off(AttnParams& p, int mode) {
   if (mode != MLTS_MASK_CAUSAL) p.causal_off = p.Sk > p.Sq ? p.Sk : p.Sq;
 }
 
-#define MLTS_TILE16_DP(FN, T, DOC, ...)                    \
-  do {                                                     \
-    if (D <= 32) return FN<T, 32, DOC>(__VA_ARGS__);       \
-    if (D <= 64) return FN<T, 64, DOC>(__VA_ARGS__);       \
-    if (D <= 96) return FN<T, 96, DOC>(__VA_ARGS__);       \
-    if (D <= 128) return FN<T, 128, DOC>(__VA_ARGS__);     \
-    if (D <= 160) return FN<T, 160, DOC>(__VA_ARGS__);     \
-    return FN<T, 192, DOC>(__VA_ARGS__);                   \
+#define MLTS_TILE16_DP(FN, DOC, ...)                \
+  do {                                              \
+    if (D <= 32) return FN<32, DOC>(__VA_ARGS__);   \
+    if (D <= 64) return FN<64, DOC>(__VA_ARGS__);   \
+    if (D <= 96) return FN<96, DOC>(__VA_ARGS__);   \
+    if (D <= 128) return FN<128, DOC>(__VA_ARGS__); \
+    if (D <= 160) return FN<160, DOC>(__VA_ARGS__); \
+    return FN<192, DOC>(__VA_ARGS__);               \
   } while (0)
-#define MLTS_TILE16(FN, ...)                                              \
-  do {                                                                    \
-    if (mode == MLTS_MASK_DOC) MLTS_TILE16_DP(FN, bf16_t, true, __VA_ARGS__);    \
-    MLTS_TILE16_DP(FN, bf16_t, false, __VA_ARGS__);                       \
+#define MLTS_TILE16(FN, ...)                                          \
+  do {                                                                \
+    if (mode == MLTS_MASK_DOC) MLTS_TILE16_DP(FN, true, __VA_ARGS__); \
+    MLTS_TILE16_DP(FN, false, __VA_ARGS__);                           \
   } while (0)
 
 }  // namespace
