@@ -1,4 +1,4 @@
-// fp32 attention without LDS in its loops: shared pieces of attn_f32_fwd.hip and attn_f32_bwd.hip.
+// fp32 attention without tiles that wavefronts share in LDS: pieces of attn_f32_fwd.hip and attn_f32_bwd.hip.
 //
 // A wavefront owns 16 or 32 rows (queries in the forward and dQ kernels, keys in the dK/dV kernel) and walks the other side in
 // units of 16 or 32 rows.  Everything is computed transposed, S^T = K Q^T and O^T = V^T P^T (dK/dV: S = Q K^T, dV^T = dO^T P), on
@@ -7,8 +7,10 @@
 // operand layout of the next product once the contraction index is renumbered, which both operands agree on.
 //
 // The wavefronts of a workgroup share their own rows and take every `splits`-th unit, so that no two of them read the same walked
-// rows: staging those in LDS would share nothing and cost two barriers a tile.  They come straight from memory in both forms a
-// product needs them in, all as 16-byte loads at head dims 64, 128 and 192:
+// rows: staging those for all of them in LDS would share nothing and cost two barriers a tile.  Each fetches its own straight from memory,
+// all as 16-byte loads at head dims 64, 128 and 192, and a product needs them in one of two forms.  The forward kernel fetches K in the
+// first and V in the second; the backward kernels, which need K, or Q and dO, in both, fetch the first and turn it into the second through
+// LDS of the wavefront's own (Turn below), without a barrier:
 //   dot          lane l: row l % 16, columns 16 j + 4 (l / 16) ..+3           (contraction over the columns)
 //   accumulate   lane l: row 4 (l / 16) + i, columns NC (l % 16) .. + NC - 1  (contraction over the rows; NC = head_dim / 16: column
 //                block db of a product is column NC (l % 16) + db, so that one load feeds NC products)
