@@ -16,8 +16,8 @@
 //                block db of a product is column NC (l % 16) + db, so that one load feeds NC products)
 // The unit behind the one that is multiplied is on its way meanwhile.  The splits' sums meet in LDS at the end.
 //
-// What bounds it: MFMA (32 cycles per 16x16x4) with the vector work between, 0.5 to 0.65 of the pipe where the chip is full; below that the
-// fixed 5 us of a launch, a chain of first loads and the join.  Before, four wavefronts staged whole 64-row tiles in LDS, which all of
+// What bounds it: MFMA (32 cycles per 16x16x4) with the vector work between, by counters 0.63 to 0.77 of the pipe where the chip is full
+// (8 x 8 x 1024 and 4 x 8 x 1024; 0.47 at 2 x 8 x 777); below that the fixed 5 us of a launch, a chain of first loads and the join.  Before, four wavefronts staged whole 64-row tiles in LDS, which all of
 // them waited for.  Before / now (us; forward, dQ, dK/dV): 2 x 8 heads (4 KV) x 777 causal, head_dim 64: 41 48 90 / 24 36 45;
 // 8 x 4 x 256: 15.5 18.8 19.4 / 9.6 13.4 14.6; 1 x 4 x 100: 8.8 10.5 10.2 / 6.0 7.2 8.3; 8 x 8 x 1024: 120 165 216 / 114 132 222;
 // 4 x 8 x 1024 unmasked: 132 175 220 / 92 120 192; 2 x 8 x 700, head_dim 96: 48 54 61 / 31 47 54; 4 x 8 x 500 x 1000, head_dim 128:
