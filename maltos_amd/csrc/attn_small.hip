@@ -548,6 +548,11 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 //   two query heads and more to a KV head: dK/dV walks all of them.  2 x 16 (4) heads x 777 53.8 -> 26.0, 1 x 16 (4) x 2048 121 -> 49
 // Without a mask a block's work is twice that of a causal one: head_dim 64 768 blocks 6 x 2048 32.7 36.4 33.5 -> 22.8 26.2 29.9, but 1024
 // blocks 8 x 2048 32.5 37.4 34.8 -> 30.8 34.7 43.5; head_dim 128 256 blocks 4 x 1024 22.9 38.4 32.2 -> 13.5 15.6 15.6.
+//
+// The lines are one number of blocks for every length of the walk, up to which no measured call is behind.  They are not the
+// break-even, which moves up with the length: of the calls above that are past their line, and so left to the 32-row kernels, these
+// would be ahead here: 1536 causal blocks, forward and dQ of 3 x 8 heads x 1024 (11 and 9 %) and of 12 x 2048 (26 and 18 %), dK/dV of
+// the latter (5 %); 1024 unmasked blocks, forward and dQ of 8 x 2048 (5 and 7 %).  The rule has no term for the length.
 bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride) {
   const bool keys = pass == ATTN_BWD_DKV;
   if ((keys ? p.Sq : p.Sk) < 512) return false;
