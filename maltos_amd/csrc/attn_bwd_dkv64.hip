@@ -7,7 +7,7 @@
 //
 // Against the two-role kernel of attn_bwd_split.hip, whose wavefronts hand the probabilities over in LDS (head_dim 128 has no registers for
 // anything else): no hand-over, no second barrier chain, and the arithmetic of one wavefront beside the products of another.  8 x 8 heads x
-// 2048 causal 114 -> 97 us, 4 x 16 x 4096 412 -> 329 us (290 on another box).  By counters the matrix cores are busy 37 % of that time (44 %
+// 2048 causal 114 -> 97 us, 4 x 16 x 4096 412 -> 329 us (290 on another card).  By counters the matrix cores are busy 37 % of that time (44 %
 // in the larger call) and the vector port 48 % (54 %): what is left is what of the two does not overlap.
 #include "attn_bf16.hpp"
 
