@@ -130,6 +130,7 @@ struct Product {
   int M, N;
   int tiles_m, tiles_n, slices;
   int form, accumulate;
+  int xcds;  // log2 of the parts its slices, tile rows and tile columns are divided into for the eight XCDs, four bits each
 };
 constexpr int kMaxProducts = 4;  // of a call
 // Two NT products of one shape that share A and meet in the end (gate and up of an MLP): C = A B^T, C2 = A B2^T, h = round(silu(C)) * C2 of
@@ -146,9 +147,17 @@ struct Rotation {
   const int32_t* positions;
   int max_pos, position_offset, seq, D;
   int columns[kMaxProducts][4];  // of each product: two ranges of whole heads
+  // of row + step; in_seq: row's place in its sequence, for calls without positions
   template <typename T, typename C2>
-  __device__ __forceinline__ void angles(int row, int pair, C2* c, C2* s) const {
-    int pos = positions ? positions[row] : position_offset + static_cast<int>(static_cast<uint32_t>(row) % static_cast<uint32_t>(seq));
+  __device__ __forceinline__ void angles(int row, int step, int in_seq, int last, int pair, C2* c, C2* s) const {
+    int pos;
+    if (positions) {
+      pos = positions[min(row + step, last)];
+    } else {
+      pos = in_seq + step;
+      if (pos >= seq) pos = pos < 2 * seq ? pos - seq : static_cast<int>(static_cast<uint32_t>(pos) % static_cast<uint32_t>(seq));  // (a division takes 30 instructions)
+      pos += position_offset;
+    }
     pos = pos < 0 ? 0 : pos >= max_pos ? max_pos - 1 : pos;  // host validated; keeps reads in bounds
     const int64_t at = static_cast<int64_t>(pos) * (D / 2) + pair;
     *c = *reinterpret_cast<const C2*>(static_cast<const T*>(cos) + at), *s = *reinterpret_cast<const C2*>(static_cast<const T*>(sin) + at);
@@ -161,6 +170,46 @@ __device__ __forceinline__ void rotate(float& even, float& odd, float c, float s
   even = round_to<T>(xe * c) - round_to<T>(xo * s);
   odd = round_to<T>(xe * s) + round_to<T>(xo * c);
 }
+// Where a tile's rows are read and written four columns at a time: the bounds check of a buffer descriptor stands for a branch over the rows and
+// columns past the end at every access, which all passes of a tile would wait behind.  (Rows too far apart for the descriptor's 32-bit
+// offsets: pointers.)
+template <typename T>
+struct Window {
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  static constexpr int ES = static_cast<int>(sizeof(T));
+  __amdgpu_buffer_rsrc_t rsrc;
+  T* at;  // of this lane's first row and column
+  int64_t ld;
+  uint32_t offset;
+  int rows;   // that exist, from this lane's first one on
+  bool near;
+  // base: the tile's first row; rows: of the tile that exist; row, col: this lane's first row in the tile and its column of `columns`
+  template <int BM>
+  __device__ __forceinline__ void init(const void* base, int64_t stride, int tile_rows, int columns, int row, int col) {
+    ld = stride, near = stride < (int64_t{1} << 31) / (BM * ES);
+    const int existing = min(tile_rows, BM);
+    const uint32_t bytes = near ? static_cast<uint32_t>(((existing - 1) * ld + columns) * ES) : 0;
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
+    offset = col < columns ? static_cast<uint32_t>(row * static_cast<uint32_t>(stride) + col) * ES : kOutside;
+    at = static_cast<T*>(const_cast<void*>(base)) + row * ld + col;
+    rows = col < columns ? existing - row : 0;
+  }
+  __device__ __forceinline__ void put(int row, t4 v) const {
+    if (near) {
+      if constexpr (ES == 2) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, 0);
+      else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, 0);
+    } else if (row < rows) {
+      *reinterpret_cast<t4*>(at + row * ld) = v;
+    }
+  }
+  __device__ __forceinline__ t4 get(int row) const {
+    if (near) {
+      if constexpr (ES == 2) return __builtin_bit_cast(t4, __builtin_amdgcn_raw_buffer_load_b64(rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, 0));
+      else return __builtin_bit_cast(t4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, 0));
+    }
+    return row < rows ? *reinterpret_cast<const t4*>(at + row * ld) : t4{};
+  }
+};
 // What becomes of dh = dy W_down, an NN product, instead of being written: d gate and d up of the activation (mlts_swiglu_bwd_rows of the
 // rounded dh).  Strides in elements.
 struct Activation {
@@ -178,12 +227,25 @@ struct MoreSegments {
   int count, product;  // how many, of which product
 };
 
-// Consecutive workgroups go to the eight XCDs in turn; each XCD gets a contiguous run of a product's tiles, walked along N, so
-// that the workgroups that share rows of A share an L2.
-__device__ __forceinline__ int tile_of(int block, int tiles) {
-  const int per = tiles >> 3, rest = tiles & 7, xcd = block & 7, pos = block >> 3;
-  return pos < per + (xcd < rest) ? xcd * per + min(xcd, rest) + pos : -1;
-}
+// The tile of a workgroup.  Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its own: an XCD gets a rectangle of a
+// product's tiles (split contractions: of some of the slices), so that it reads few rows of A and few columns of B (divide()), and walks it along N.
+struct Tile {
+  int slice, m, n;
+  bool there;
+  __device__ __forceinline__ Tile(const Product& g, int block) {
+    const int xcd = block & 7, ls = g.xcds & 15, lm = (g.xcds >> 4) & 15, ln = g.xcds >> 8;
+    const int xn = xcd & ((1 << ln) - 1), xm = (xcd >> ln) & ((1 << lm) - 1), xs = xcd >> (ln + lm);
+    const int n0 = (g.tiles_n * xn) >> ln, width = ((g.tiles_n * (xn + 1)) >> ln) - n0;
+    const int m0 = (g.tiles_m * xm) >> lm, height = ((g.tiles_m * (xm + 1)) >> lm) - m0;
+    const int s0 = (g.slices * xs) >> ls, depth = ((g.slices * (xs + 1)) >> ls) - s0;
+    int rest = block >> 3;
+    there = rest < width * height * depth;
+    const int row = there ? rest / width : 0;
+    n = n0 + rest - row * width;
+    slice = depth > 1 ? row / height : 0;
+    m = m0 + row - slice * height, slice += s0;
+  }
+};
 
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool PAIR = false>
 struct TileShape {
@@ -195,7 +257,7 @@ struct TileShape {
   static constexpr int STAGE = SA::BYTES + SB::BYTES;
   static constexpr int OUT = WAVES * 32 * (WN + 4) * 4;
   static_assert(KG == 1 || WAVES == KG, "one wavefront to a group");
-  static_assert(!PAIR || (FORM == FORM_NT && KG == 1 && WAVES_N == 2), "the products of a pair side by side in a tile, a wavefront of each");
+  static_assert(!PAIR || (FORM == FORM_NT && KG == 1 && WAVES_N % 2 == 0), "the products of a pair side by side in a tile, half of the wavefronts each");
   static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
 };
 
@@ -203,7 +265,7 @@ struct TileShape {
 // LDS, where all of them add up and write out a part of the tile (us, one of them / all: fp32 NT 2048 x 256 x 256 7.2 / 6.7,
 // 500 x 512 x 512 8.0 / 7.0).
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false, bool ROPE = false, bool ACT = false>
-__device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr,
+__device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr,
                                           const Rotation* rot = nullptr, int product = 0, const Activation* act = nullptr) {
   typedef TileShape<T, FORM, BM, BN, WM, WN, KG, PAIR> S;
   constexpr int WAVES_N = S::WAVES_N, MB = S::MB, NB = S::NB, SETS = S::SETS, STAGE = S::STAGE;
@@ -214,9 +276,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = KG > 1 ? wave : 0, member = KG > 1 ? 0 : wave;
   const int wm = (member / WAVES_N) * WM, wn = (member % WAVES_N) * WN;
-  const int slice = tile / (g.tiles_m * g.tiles_n);
-  tile -= slice * (g.tiles_m * g.tiles_n);
-  const int m0 = (tile / g.tiles_n) * BM, n0 = (tile % g.tiles_n) * (PAIR ? BN / 2 : BN);
+  const int slice = tile.slice, m0 = tile.m * BM, n0 = tile.n * (PAIR ? BN / 2 : BN);
 
   SA sa;
   SB sb;
@@ -279,41 +339,56 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
   // of a training step of 8 layers).
   constexpr int OUT_LANES = KG > 1 ? S::THREADS : 64;  // that write a block of 32 rows of C
   constexpr int LPR = WN / 4, RPP = OUT_LANES / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
-  constexpr bool EARLY = !PAIR && !ROPE && !ACT && (KG > 1 || MB * NB == 1);
+  constexpr bool EARLY = !PAIR && !ROPE && !ACT && (KG > 1 || MB * NB <= 2);
   typedef T t4 __attribute__((ext_vector_type(4)));
   t4 old[EARLY ? MB * PASSES : 1];
-  const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? 0 : wn) + c4;
-  const bool whole = col + 4 <= g.N && (g.ldc & 3) == 0;
-  if (EARLY && g.accumulate && !g.partial && whole) {
+  constexpr int HALF = WAVES_N / 2;  // PAIR: wavefronts of a row of blocks that have the first product; HALF further on is the second one of the same columns
+  const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? wn % (BN / 2) : wn) + c4;
+  const int tile_row = wm + out_lane / LPR, out_row = m0 + tile_row, rows_here = g.M - m0;  // out_row: of pass 0 of the first block
+  const bool vec = PAIR || ACT || ROPE || ((g.N & 3) == 0 && (g.ldc & 3) == 0);
+  Window<T> out;
+  if (!ACT) out.template init<BM>(static_cast<const T*>(g.c) + m0 * static_cast<int64_t>(g.ldc), g.ldc, rows_here, g.N, tile_row, col);
+  const bool add = !PAIR && !ROPE && !ACT && g.accumulate && !g.partial;
+  auto fetch_old = [&] {
+    if (EARLY && add && vec) {
 #pragma unroll
-    for (int i = 0; i < (EARLY ? MB * PASSES : 0); ++i) {
-      const int row = m0 + wm + i * RPP + out_lane / LPR;
-      if (row < g.M) old[i] = *reinterpret_cast<const t4*>(static_cast<const T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col);
+      for (int i = 0; i < (EARLY ? MB * PASSES : 0); ++i) old[i] = out.get(i * RPP);
     }
-  }
-  // ... and the activation's operands, and what it is rotated by, likewise
-  static_assert(!ACT || MB * NB == 1, "small tiles");
-  t4 gates[ACT ? PASSES : 1], ups[ACT ? PASSES : 1];
-  if constexpr (ACT) {
+  };
+  // ... and the activation's operands, and what it is rotated by, likewise.  Larger tiles fetch the activation's operands, and the old C, behind
+  // the last slab, where the registers of the slabs are free.
+  constexpr bool SMALL = MB * NB == 1;
+  t4 gates[ACT ? MB * PASSES : 1], ups[ACT ? MB * PASSES : 1];
+  auto fetch_gates = [&] {
+    if constexpr (ACT) {
+      Window<T> gate, up;
+      gate.template init<BM>(static_cast<const T*>(act->gate) + m0 * static_cast<int64_t>(act->ld_in), act->ld_in, rows_here, g.N, tile_row, col);
+      up.template init<BM>(static_cast<const T*>(act->up) + m0 * static_cast<int64_t>(act->ld_in), act->ld_in, rows_here, g.N, tile_row, col);
 #pragma unroll
-    for (int r = 0; r < PASSES; ++r) {
-      const int64_t at = static_cast<int64_t>(min(m0 + wm + r * RPP + out_lane / LPR, g.M - 1)) * act->ld_in + min(col, g.N - 4);
-      gates[r] = *reinterpret_cast<const t4*>(static_cast<const T*>(act->gate) + at), ups[r] = *reinterpret_cast<const t4*>(static_cast<const T*>(act->up) + at);
+      for (int r = 0; r < MB * PASSES; ++r) gates[r] = gate.get(r * RPP), ups[r] = up.get(r * RPP);
     }
-  }
-  constexpr bool EARLY_ANGLES = ROPE && MB * NB == 1;
+  };
+  if (SMALL) fetch_old(), fetch_gates();
   typedef T t2 __attribute__((ext_vector_type(2)));
-  t2 cosines[EARLY_ANGLES ? PASSES : 1], sines[EARLY_ANGLES ? PASSES : 1];
+  constexpr bool EARLY_ANGLES = SMALL, ALL_ANGLES = MB * NB <= 4;  // (the largest tiles: a block of rows at a time)
+  constexpr int ANGLES = (ALL_ANGLES ? MB : 1) * PASSES;
+  t2 cosines[ROPE ? ANGLES : 1], sines[ROPE ? ANGLES : 1];
   bool rotated = false;
-  int pair_of_head = 0;
+  int pair_of_head = 0, in_seq = 0;
+  auto fetch_angles = [&](int i) {
+    if constexpr (ROPE) {
+      if (rotated) {
+#pragma unroll
+        for (int r = 0; r < ANGLES; ++r) rot->angles<T>(out_row, 32 * i + r * RPP, in_seq, g.M - 1, pair_of_head, &cosines[r], &sines[r]);
+      }
+    }
+  };
   if constexpr (ROPE) {
     const int* range = rot->columns[product];
     rotated = (col >= range[0] && col < range[1]) || (col >= range[2] && col < range[3]);
     pair_of_head = static_cast<int>(static_cast<uint32_t>(col - (col >= range[2] && col < range[3] ? range[2] : range[0])) % static_cast<uint32_t>(rot->D)) / 2;
-    if (EARLY_ANGLES && rotated) {
-#pragma unroll
-      for (int r = 0; r < PASSES; ++r) rot->angles<T>(min(m0 + wm + r * RPP + out_lane / LPR, g.M - 1), pair_of_head, &cosines[EARLY_ANGLES ? r : 0], &sines[EARLY_ANGLES ? r : 0]);
-    }
+    if (!rot->positions) in_seq = static_cast<int>(static_cast<uint32_t>(out_row) % static_cast<uint32_t>(rot->seq));
+    if (EARLY_ANGLES) fetch_angles(0);
   }
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) store(0, c, lds);
@@ -406,6 +481,19 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
     }
   }
 
+  if (!SMALL) fetch_old(), fetch_gates();
+  if (!EARLY_ANGLES && ALL_ANGLES) fetch_angles(0);
+  Window<T> out2, out_h;
+  if constexpr (PAIR) {
+    out2.template init<BM>(static_cast<T*>(pair->c2) + m0 * static_cast<int64_t>(g.ldc), g.ldc, rows_here, g.N, tile_row, col);
+    out_h.template init<BM>(static_cast<T*>(pair->h) + m0 * static_cast<int64_t>(pair->ldh), pair->ldh, rows_here, g.N, tile_row, col);
+  }
+  if constexpr (ACT) {
+    out.template init<BM>(static_cast<T*>(act->dgate) + m0 * static_cast<int64_t>(act->ld_out), act->ld_out, rows_here, g.N, tile_row, col);
+    out2.template init<BM>(static_cast<T*>(act->dup) + m0 * static_cast<int64_t>(act->ld_out), act->ld_out, rows_here, g.N, tile_row, col);
+  }
+  Window<float> sums;
+  if (!PAIR && !ROPE && !ACT && g.partial) sums.template init<BM>(g.partial + (static_cast<int64_t>(slice) * g.M + m0) * g.N, g.N, rows_here, g.N, tile_row, col);
   // acc[i][j][4 q + r]: row wm + 32 i + l % 32 of C, column wn + 32 j + 8 q + 4 hh + r.  Out through LDS, 32 rows at a time.
   __syncthreads();
   constexpr int ROW = WN + 4;  // floats
@@ -413,6 +501,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
     if ((KG > 1 || PAIR) && i > 0) __syncthreads();
+    if (!ALL_ANGLES) fetch_angles(i);
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
@@ -422,77 +511,81 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
       }
     if (KG > 1 || PAIR) __syncthreads();  // (alone, a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
     if constexpr (PAIR) {  // the two wavefronts of a pair of blocks take half of the rows each
-      const float* first = reinterpret_cast<const float*>(lds) + (wave & ~1) * 32 * ROW;
+      const int second = wave % WAVES_N / HALF;
+      const float* first = reinterpret_cast<const float*>(lds) + (wave - second * HALF) * 32 * ROW;
 #pragma unroll
       for (int r = 0; r < PASSES / 2; ++r) {
-        const int rr = (wave & 1) * 16 + r * RPP + lane / LPR, row = m0 + wm + 32 * i + rr;
-        const f32x4 a = *reinterpret_cast<const f32x4*>(first + rr * ROW + c4), b = *reinterpret_cast<const f32x4*>(first + (32 + rr) * ROW + c4);
-        if (row >= g.M || col >= g.N) continue;
+        const int rr = second * 16 + r * RPP, at = (rr + lane / LPR) * ROW + c4;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(first + at), b = *reinterpret_cast<const f32x4*>(first + HALF * 32 * ROW + at);
         t4 gate, up, h;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           gate[e] = from_f32<T>(a[e]), up[e] = from_f32<T>(b[e]);
           h[e] = from_f32<T>(round_to<T>(silu(to_f32<T>(gate[e]))) * to_f32<T>(up[e]));
         }
-        const int64_t at = static_cast<int64_t>(row) * g.ldc + col;
-        if (g.c) *reinterpret_cast<t4*>(static_cast<T*>(g.c) + at) = gate, *reinterpret_cast<t4*>(static_cast<T*>(pair->c2) + at) = up;
-        *reinterpret_cast<t4*>(static_cast<T*>(pair->h) + static_cast<int64_t>(row) * pair->ldh + col) = h;
+        if (g.c) out.put(32 * i + rr, gate), out2.put(32 * i + rr, up);
+        out_h.put(32 * i + rr, h);
       }
       continue;
     }
 #pragma unroll
     for (int r = 0; r < PASSES; ++r) {
-      const int rr = r * RPP + out_lane / LPR, row = m0 + wm + 32 * i + rr;
-      f32x4 v = *reinterpret_cast<const f32x4*>(stage + rr * ROW + c4);
+      const int at = (r * RPP + out_lane / LPR) * ROW + c4, row = 32 * i + r * RPP;
+      f32x4 v = *reinterpret_cast<const f32x4*>(stage + at);
 #pragma unroll
-      for (int o = 1; o < KG; ++o) v += *reinterpret_cast<const f32x4*>(stage + (o * 32 + rr) * ROW + c4);
-      if (row >= g.M || col >= g.N) continue;
+      for (int o = 1; o < KG; ++o) v += *reinterpret_cast<const f32x4*>(stage + o * 32 * ROW + at);
       if constexpr (ACT) {
         t4 dgate, dup;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float dg, du;
-          swiglu_grads(round_to<T>(v[e]), to_f32<T>(gates[r][e]), to_f32<T>(ups[r][e]), &dg, &du);
+          swiglu_grads(round_to<T>(v[e]), to_f32<T>(gates[ACT ? i * PASSES + r : 0][e]), to_f32<T>(ups[ACT ? i * PASSES + r : 0][e]), &dg, &du);
           dgate[e] = from_f32<T>(dg), dup[e] = from_f32<T>(du);
         }
-        const int64_t at = static_cast<int64_t>(row) * act->ld_out + col;
-        *reinterpret_cast<t4*>(static_cast<T*>(act->dgate) + at) = dgate, *reinterpret_cast<t4*>(static_cast<T*>(act->dup) + at) = dup;
+        out.put(row, dgate), out2.put(row, dup);
         continue;
       }
       if constexpr (ROPE) {
-        if (rotated) {
-          t2 c = cosines[EARLY_ANGLES ? r : 0], s = sines[EARLY_ANGLES ? r : 0];
-          if (!EARLY_ANGLES) rot->angles<T>(row, pair_of_head, &c, &s);
+        if (__builtin_amdgcn_ballot_w64(rotated)) {
+          const t2 c = cosines[ROPE ? (i * PASSES + r) % ANGLES : 0], s = sines[ROPE ? (i * PASSES + r) % ANGLES : 0];
 #pragma unroll
           for (int e = 0; e < 4; e += 2) {
             float even = v[e], odd = v[e + 1];
             rotate<T>(even, odd, to_f32<T>(c[e / 2]), to_f32<T>(s[e / 2]));
-            v[e] = even, v[e + 1] = odd;
+            v[e] = rotated ? even : v[e], v[e + 1] = rotated ? odd : v[e + 1];
           }
         }
       }
-      if (g.partial) {
-        float* p = g.partial + (static_cast<int64_t>(slice) * g.M + row) * g.N + col;
-        if (col + 4 <= g.N && (g.N & 3) == 0) {
-          *reinterpret_cast<f32x4*>(p) = v;
-        } else {
+      if (!ROPE && g.partial) {
+        if ((g.N & 3) == 0) {
+          sums.put(row, v);
+        } else if (row + tile_row < rows_here) {
+          float* p = g.partial + (static_cast<int64_t>(slice) * g.M + out_row + row) * g.N + col;
           for (int e = 0; e < 4 && col + e < g.N; ++e) p[e] = v[e];
         }
         continue;
       }
-      T* p = static_cast<T*>(g.c) + static_cast<int64_t>(row) * g.ldc + col;
-      if (whole) {
-        if (g.accumulate) {
-          const t4 before = EARLY ? old[EARLY ? i * PASSES + r : 0] : *reinterpret_cast<const t4*>(p);
+      if (vec) {
+        if (add) {
+          const t4 before = EARLY ? old[EARLY ? i * PASSES + r : 0] : out.get(row);
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] += to_f32<T>(before[e]);
         }
         t4 w;
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = from_f32<T>(v[e]);
-        *reinterpret_cast<t4*>(p) = w;
-      } else {
-        for (int e = 0; e < 4 && col + e < g.N; ++e) p[e] = from_f32<T>(v[e] + (g.accumulate ? to_f32<T>(p[e]) : 0.f));
+        out.put(row, w);
+      } else if (row + tile_row < rows_here) {  // (columns that are not whole groups of four)
+        T* p = static_cast<T*>(g.c) + static_cast<int64_t>(out_row + row) * g.ldc + col;
+        if (col + 4 <= g.N && (g.ldc & 3) == 0) {
+          t4 w;
+          const t4 before = add ? *reinterpret_cast<const t4*>(p) : t4{};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = from_f32<T>(add ? v[e] + to_f32<T>(before[e]) : v[e]);
+          *reinterpret_cast<t4*>(p) = w;
+        } else {
+          for (int e = 0; e < 4 && col + e < g.N; ++e) p[e] = from_f32<T>(v[e] + (add ? to_f32<T>(p[e]) : 0.f));
+        }
       }
     }
   }
@@ -501,27 +594,27 @@ __device__ __forceinline__ void gemm_tile(const Product& g, int tile, unsigned c
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_kernel(const Product g) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n * g.slices);
-  if (tile >= 0) gemm_tile<T, FORM, BM, BN, WM, WN, KG, false>(g, tile, lds, MoreSegments{}, 0);
+  const Tile tile(g, static_cast<int>(blockIdx.x));
+  if (tile.there) gemm_tile<T, FORM, BM, BN, WM, WN, KG, false>(g, tile, lds, MoreSegments{}, 0);
 }
 
 // us in a training step, product and pass / rotated here: q, k, v of 1023 rows as one 1536 x 512 product 7.5 + 3.7 / 9.1; of 2331 rows as
-// three 11.9 + 4.0 / 12.8; fp32 of 2048 rows as three 256 x 256 12.8 + 3.9 / 14.1.
+// three 11.9 + 4.0 / 12.8; of 16384 rows as one 32 (the library's selected kernel) + 15 / 44; fp32 of 2048 rows as three 256 x 256 12.8 + 3.9 / 14.1.
 template <typename T, int BM, int BN, int WM, int WN, int KG>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_rope_kernel(const Product g, const Rotation rot) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n);
-  if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, WM, WN, KG, false, false, true>(g, tile, lds, MoreSegments{}, 0, nullptr, &rot);
+  const Tile tile(g, static_cast<int>(blockIdx.x));
+  if (tile.there) gemm_tile<T, FORM_NT, BM, BN, WM, WN, KG, false, false, true>(g, tile, lds, MoreSegments{}, 0, nullptr, &rot);
 }
 
 // us, one product and the pass over gate and up / the pair / without gate and up (weights out of HBM, x just written): 1376 + 1376 x 512 bf16
-// 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 16.1 + 5.8 / 19.2 / 17.4; 688 + 688 x 256 fp32 2048 rows
-// 20.1 + 4.8 / 20.9 / 18.9.
+// 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 15.5 + 5.8 / 17.7 / 16.1, 16384 rows 72 (library) + 23 / 76 /;
+// 688 + 688 x 256 fp32 2048 rows 20.1 + 4.8 / 20.9 / 18.9.
 template <typename T, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_pair_kernel(const Product g, const Pair pair) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int tile = tile_of(static_cast<int>(blockIdx.x), g.tiles_m * g.tiles_n);
-  if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, WM, WN, 1, false, true>(g, tile, lds, MoreSegments{}, 0, &pair);
+  const Tile tile(g, static_cast<int>(blockIdx.x));
+  if (tile.there) gemm_tile<T, FORM_NT, BM, BN, WM, WN, 1, false, true>(g, tile, lds, MoreSegments{}, 0, &pair);
 }
 
 // Several small products in one launch: what a linear layer's backward needs (dx and dW), or projections that share their input.
@@ -532,8 +625,8 @@ struct Products {
   Product p[kMaxProducts];
   MoreSegments more;
 };
-template <typename T, int FORMS, int BM, int BN, int KG>
-__global__ __launch_bounds__(256) void gemm_multi_kernel(const Products ps) {
+template <typename T, int FORMS, int BM, int BN, int WM, int WN, int KG>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_multi_kernel(const Products ps) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int block = static_cast<int>(blockIdx.x);
   int i = 0, first = ps.first[0];
@@ -541,15 +634,15 @@ __global__ __launch_bounds__(256) void gemm_multi_kernel(const Products ps) {
   for (int k = 1; k < kMaxProducts; ++k)
     if (block >= ps.first[k]) i = k, first = ps.first[k];
   const Product& g = ps.p[i];
-  const int tile = tile_of(block - first, g.tiles_m * g.tiles_n * g.slices);
-  if (tile < 0) return;
-  if (FORMS == FORMS_NT || (FORMS != FORMS_NN && g.form == FORM_NT)) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
-  else if (FORMS == FORMS_NN || g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, 32, 32, KG, FORMS == FORMS_SEGMENTS>(g, tile, lds, ps.more, i == ps.more.product ? ps.more.count : 0);
-  else gemm_tile<T, FORM_TN, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
+  const Tile tile(g, block - first);
+  if (!tile.there) return;
+  if (FORMS == FORMS_NT || (FORMS != FORMS_NN && g.form == FORM_NT)) gemm_tile<T, FORM_NT, BM, BN, WM, WN, KG, false>(g, tile, lds, ps.more, 0);
+  else if (FORMS == FORMS_NN || g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, WM, WN, KG, FORMS == FORMS_SEGMENTS>(g, tile, lds, ps.more, i == ps.more.product ? ps.more.count : 0);
+  else gemm_tile<T, FORM_TN, BM, BN, WM, WN, KG, false>(g, tile, lds, ps.more, 0);
 }
 
-template <typename T, int BM, int BN, int KG>
-__global__ __launch_bounds__(256) void gemm_multi_rope_kernel(const Products ps, const Rotation rot) {
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_multi_rope_kernel(const Products ps, const Rotation rot) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int block = static_cast<int>(blockIdx.x);
   int i = 0, first = ps.first[0];
@@ -557,21 +650,21 @@ __global__ __launch_bounds__(256) void gemm_multi_rope_kernel(const Products ps,
   for (int k = 1; k < kMaxProducts; ++k)
     if (block >= ps.first[k]) i = k, first = ps.first[k];
   const Product& g = ps.p[i];
-  const int tile = tile_of(block - first, g.tiles_m * g.tiles_n);
-  if (tile >= 0) gemm_tile<T, FORM_NT, BM, BN, 32, 32, KG, false, false, true>(g, tile, lds, ps.more, 0, nullptr, &rot, i);
+  const Tile tile(g, block - first);
+  if (tile.there) gemm_tile<T, FORM_NT, BM, BN, WM, WN, KG, false, false, true>(g, tile, lds, ps.more, 0, nullptr, &rot, i);
 }
 
-// dW = dy^T h (if it is wanted), and dh = dy W on its way through the activation (1023 rows, 1376 x 512: 13.4 us and 5.1 for the pass /
-// 16.3 here)
-template <typename T, int BM, int BN, int KG>
-__global__ __launch_bounds__(256) void gemm_multi_act_kernel(const Products ps, const Activation act) {
+// dW = dy^T h (if it is wanted), and dh = dy W on its way through the activation (1376 x 512, us: 1023 rows 13.4 and 5.1 for the pass /
+// 16.3 here; 16384 rows, dh alone, 34 to 50 (the library's) and 37 / 66)
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_multi_act_kernel(const Products ps, const Activation act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int block = static_cast<int>(blockIdx.x), i = block >= ps.first[1] ? 1 : 0;
   const Product& g = ps.p[i];
-  const int tile = tile_of(block - ps.first[i], g.tiles_m * g.tiles_n * g.slices);
-  if (tile < 0) return;
-  if (g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, 32, 32, KG, false, false, false, true>(g, tile, lds, ps.more, 0, nullptr, nullptr, 0, &act);
-  else gemm_tile<T, FORM_TN, BM, BN, 32, 32, KG, false>(g, tile, lds, ps.more, 0);
+  const Tile tile(g, block - ps.first[i]);
+  if (!tile.there) return;
+  if (g.form == FORM_NN) gemm_tile<T, FORM_NN, BM, BN, WM, WN, KG, false, false, false, true>(g, tile, lds, ps.more, 0, nullptr, nullptr, 0, &act);
+  else gemm_tile<T, FORM_TN, BM, BN, WM, WN, KG, false>(g, tile, lds, ps.more, 0);
 }
 
 // C (+)= sum of the slices' fp32 partial products, one rounding; up to kMaxProducts outputs
@@ -616,8 +709,8 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(const Joins js) {
 }
 
 // ---- which tile, which split ----------------------------------------------------------------------------------------------
-constexpr int kSmall = 0;  // a tile of the multi kernel; 1: 128 x 128, 2: 256 x 128, 3: 256 x 256
-constexpr int kTileM[4] = {64, 128, 256, 256}, kTileN[4] = {64, 128, 128, 256};
+constexpr int kSmall = 0, k128 = 1, k256x128 = 2, k256 = 3, k128x64 = 4, kTiles = 5;  // (small: 64 x 64, in fp32 also 32 x 32; 128 x 64: bf16)
+constexpr int kTileM[kTiles] = {64, 128, 256, 256, 128}, kTileN[kTiles] = {64, 128, 128, 256, 64};
 int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 int slab_of(int dtype) { return dtype == MLTS_BF16 ? 64 : 32; }
 int64_t slabs_of(const mlts_gemm_product& p, int bk) {
@@ -632,25 +725,16 @@ void set_slices(Product& g, int64_t slices, int64_t slabs, int bk) {
   g.slices = static_cast<int>(std::max<int64_t>(1, (slabs + part - 1) / part));
 }
 
-// A product that runs alone takes the largest tile that still gives every CU a workgroup; one with fewer tiles than CUs is split
-// along its contraction where that is long.  Best of all tiles and splits (us): NT 16384 x 512 x 512 256x128 15.6 (128x128 16.7,
-// 64x64 19.2, 256x256 21.6); NT 16384 x 2752 x 512 256x256 66 (76, 96, 77); NN 1023 x 512 x 32000 256x128 in 16 parts 45 (unsplit
-// 210); TN 512 x 512 x 16384 in 32 parts 24 (128x128 in 16: 23); TN 2752 x 512 x 16384 in 4 parts 70 (256x256 in 8: 68).
-int choose_tile(const mlts_gemm_product& p, int dtype, int64_t* slices) {
-  const int64_t slabs = slabs_of(p, slab_of(dtype)), t2 = tiles_of(p.M, p.N, 256, 128);
-  *slices = 1;
+// fp32: a product that runs alone takes the largest tile that still gives every CU a workgroup.
+int choose_f32_tile(const mlts_gemm_product& p) {
   if (p.segments > 1) return kSmall;
-  if (tiles_of(p.M, p.N, 256, 256) >= 240) return 3;
-  if (t2 >= 256) return 2;
-  if (dtype == MLTS_BF16 && slabs >= 64 && t2 * (slabs / 8) >= 192) {
-    while (t2 * *slices * 2 <= 256 && slabs / (*slices * 2) >= 8) *slices *= 2;
-    return 2;
-  }
-  return tiles_of(p.M, p.N, 128, 128) >= 256 ? 1 : kSmall;
+  if (tiles_of(p.M, p.N, 256, 256) >= 240) return k256;
+  if (tiles_of(p.M, p.N, 256, 128) >= 256) return k256x128;
+  return tiles_of(p.M, p.N, 128, 128) >= 256 ? k128 : kSmall;
 }
 bool splittable(const mlts_gemm_product& p) { return p.segments == 1 && p.N % 4 == 0 && p.ldc == p.N; }
 
-// The small products of a launch together: tiles of 64 x 64, or in fp32 also of 32 x 32, whose four wavefronts share a tile along
+// The small fp32 products of a launch together: tiles of 64 x 64, or of 32 x 32, whose four wavefronts share a tile along
 // the contraction (us, 64 x 64 / 32 x 32: NT 2048 x 256 x 256 8.2 / 6.3, NN 1000 x 512 x 1376 31.4 / 17.1, 500 x 256 x 256 7.9 /
 // 4.6, but 2048 x 1376 x 512 29.8 / 32.4).  chain: us a workgroup takes for a slab; busy: us of a CU for each slab when it has
 // several workgroups (measured).
@@ -658,15 +742,14 @@ struct SmallShape {
   int size;
   double chain, busy;
 };
-constexpr SmallShape kBf16Shape{64, 0.26, 0.16}, kF32Shape{64, 0.65, 0.5}, kF32Fine{32, 0.31, 0.16};
+constexpr SmallShape kBf16Shape{64, 0, 0}, kF32Shape{64, 0.65, 0.5}, kF32Fine{32, 0.31, 0.16};
 
 // Slices of each product, and the estimated time: the longest chain of slabs, or the product on all 256 CUs if that is longer, and
 // what a split costs: a launch that joins the slices and their fp32 sums written and read.  A weight gradient's split does not
-// depend on what shares its launch, so that its bits do not either.  (us: NN 1024 x 512 x 2752 whole 14.8, in
-// two 13.0, in four 14.5; TN 512 x 512 x 2048 whole 12.0, in four 9.5; TN 512 x 512 x 1024 whole 7.6, in two 8.3; fp32 TN 256 x 256 x
-// 2048 whole 20.5, in eight 8.9; fp32 NN 1000 x 512 x 1376 whole 17.1, in two 20.3.)
-double small_slices(const mlts_gemm_product* const* ps, int count, int dtype, const SmallShape& shape, int64_t* slices) {
-  const int bk = slab_of(dtype);
+// depend on what shares its launch, so that its bits do not either.  (us: TN 256 x 256 x 2048 whole 20.5, in eight 8.9; NN 1000 x 512 x
+// 1376 whole 17.1, in two 20.3.)
+double small_slices(const mlts_gemm_product* const* ps, int count, const SmallShape& shape, int64_t* slices) {
+  const int bk = slab_of(MLTS_F32);
   double longest = 0;
   for (int i = 0; i < count; ++i) {
     const int64_t slabs = slabs_of(*ps[i], bk), tiles = tiles_of(ps[i]->M, ps[i]->N, shape.size, shape.size);
@@ -684,27 +767,147 @@ double small_slices(const mlts_gemm_product* const* ps, int count, int dtype, co
   return longest;
 }
 
+// The rectangles of the eight XCDs (Tile), bm x bn the tile; returns the workgroups of the launch, eight times those of the largest one.
+int64_t divide(Product& g, int bm, int bn) {
+  auto part = [](int64_t n, int l) { return (n + (int64_t{1} << l) - 1) >> l; };
+  const int64_t mean = (static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices + 7) / 8;
+  int64_t most = 0;
+  double best = 0;
+  for (int ls = 0; ls <= 3; ++ls)
+    for (int lm = 0; lm + ls <= 3; ++lm) {
+      const int ln = 3 - ls - lm;
+      const int64_t depth = part(g.slices, ls), rows = part(g.tiles_m, lm), columns = part(g.tiles_n, ln), tiles = depth * rows * columns;
+      const double cost = static_cast<double>(depth * (rows * bm + columns * bn)) * static_cast<double>(std::max<int64_t>(tiles, 32)) / static_cast<double>(std::max<int64_t>(mean, 32));
+      if (most == 0 || cost < best) most = tiles, best = cost, g.xcds = ls | lm << 4 | ln << 8;
+    }
+  return most * 8;
+}
+
+// bf16: tile and split by estimated time (us).  A launch takes `fixed`, then the longer of the chain of slabs of a workgroup and its work
+// shared by 256 CUs, then what is written; a split also the launch that joins the slices and their fp32 sums.  Fitted to 1100 products of 100 to
+// 12000 rows, 256 to 32000 columns and 256 to 2752 terms in the three forms, weights out of HBM: off by 7 % (rms), and the choice by 0.5 %
+// from the best of all tiles and splits.  What a workgroup fetches decides: loads alone, with neither LDS nor matrix instructions, take as
+// long as the kernel (2048 x 2048 x 1536, tiles of 64 x 64: 29 us of 30.5), and a tile of 128 x 128 fetches half as much for its work
+// (us, 64 x 64 / 128 x 128: NT 2331 x 1536 x 512 12.0 / 9.4, 8192 x 2752 x 512 45.3 / 34.9, NN 16384 x 1376 x 512 48.8 / 36.5).
+struct TileCost {
+  double fixed, chain, busy, out;  // out: of a million elements
+};
+constexpr TileCost kBf16Cost[kTiles] = {{3.6, 0.285, 0.26, 0.26}, {4.5, 0.54, 0.68, 0.28}, {6.7, 0.73, 1.25, 0.42}, {9.7, 1.2, 2.1, 0.48}, {4.4, 0.38, 0.405, 0.4}};
+constexpr double kJoinFixed = 4.2, kJoinSums = 0.97;  // ... of a million partial sums
+// What a pass on the way out adds, on small tiles and on larger ones, whose fewer wavefronts have less to overlap its latency with: of a launch,
+// of a million elements.  (us, 64 x 64 / 128 x 128: three rotated products of 512 x 512, 300 rows 7.8 / 12.6, 2331 13.2 / 14.1, 4096 18.2 / 15.8;
+// gate, up and activation of 1376 x 512, 300 rows 6.7 / 10.3, 1536 15.3 / 15.9, 2331 19.4 / 17.7, 8192 50 / 42; d gate and d up of it 300 rows
+// 8.5 / 14.6, 4096 29.8 / 29.2, 8192 56 / 45)
+struct PassCost {
+  double fixed[2], out[2];
+};
+constexpr PassCost kRotationCost{{0.3, 2.5}, {0, 0}}, kPairCost{{1.8, 4.2}, {0, 0}}, kActivationCost{{2.0, 5.5}, {2.1, 1.6}};
+double pass_time(const PassCost& c, int tile, int64_t M, int64_t N) {
+  const int larger = tile != kSmall;
+  return c.fixed[larger] + c.out[larger] * 1e-6 * static_cast<double>(M) * static_cast<double>(N);
+}
+
+// The time of products in one launch, the slices of each given
+double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const int64_t* slices) {
+  const TileCost& c = kBf16Cost[tile];
+  double longest = 0, work = 0, out = 0, sums = 0;
+  for (int i = 0; i < count; ++i) {
+    const double part = static_cast<double>((slabs_of(*ps[i], 64) + slices[i] - 1) / slices[i]), elements = 1e-6 * static_cast<double>(ps[i]->M) * static_cast<double>(ps[i]->N);
+    longest = std::max(longest, part);
+    work += part * static_cast<double>(slices[i] * tiles_of(ps[i]->M, ps[i]->N, kTileM[tile], kTileN[tile]));
+    (slices[i] > 1 ? sums : out) += elements * static_cast<double>(slices[i] > 1 ? slices[i] : 1);
+  }
+  return c.fixed + std::max(longest * c.chain, work / 256 * c.busy) + out * c.out + (sums > 0 ? kJoinFixed + kJoinSums * sums : 0);
+}
+
+// The best tile and split of a product that runs alone.  (A contraction of 64 slabs and more on few tiles: 256 x 128 in as many parts as fill the
+// chip, which the estimate has no data for.  NN 1023 x 512 x 32000 in 16 parts 45 us, unsplit 210.)
+int choose_bf16_tile(const mlts_gemm_product& p, int64_t* slices) {
+  const int64_t slabs = slabs_of(p, 64), t2 = tiles_of(p.M, p.N, 256, 128);
+  *slices = 1;
+  if (p.segments > 1) return kSmall;
+  if (slabs >= 64 && t2 < 256 && t2 * (slabs / 8) >= 192 && p.form == FORM_NN) {
+    while (splittable(p) && t2 * *slices * 2 <= 256 && slabs / (*slices * 2) >= 8) *slices *= 2;
+    return k256x128;
+  }
+  const mlts_gemm_product* const one = &p;
+  int best = kSmall;
+  double least = 0;
+  for (int tile = 0; tile < kTiles; ++tile)
+    for (int64_t s = 1; s == 1 || (splittable(p) && s <= 16 && slabs / s >= 4); s *= 2) {
+      const double t = bf16_time(&one, 1, tile, &s);
+      if (least == 0 || t < least) least = t, best = tile, *slices = s;
+    }
+  return best;
+}
+
 struct LaunchPlan {
   int tile[kMaxProducts];
   int64_t slices[kMaxProducts];
-  const mlts_gemm_product* small[kMaxProducts];
-  int small_at[kMaxProducts], smalls = 0;
-  SmallShape shape;
-  int64_t workspace = 0;  // bytes
-  LaunchPlan(const mlts_gemm_product* ps, int count, int dtype) : shape(dtype == MLTS_BF16 ? kBf16Shape : kF32Shape) {
-    for (int i = 0; i < count; ++i) {
-      tile[i] = choose_tile(ps[i], dtype, &slices[i]);
-      if (tile[i] == kSmall) small_at[smalls] = i, small[smalls++] = &ps[i];
-      else if (!splittable(ps[i])) slices[i] = 1;
-    }
-    if (smalls) {
-      int64_t s[kMaxProducts], fine[kMaxProducts];
-      const double coarse = small_slices(small, smalls, dtype, shape, s);
-      if (dtype == MLTS_F32 && small_slices(small, smalls, dtype, kF32Fine, fine) < coarse) shape = kF32Fine, std::copy(fine, fine + smalls, s);
-      for (int i = 0; i < smalls; ++i) slices[small_at[i]] = s[i];
-    }
+  bool together[kMaxProducts] = {};  // in the launch of several products, all of one tile
+  SmallShape shape;                  // of the small tile
+  int64_t workspace = 0;             // bytes
+  // activation: an NN product that is not split, whose output goes through the activation
+  LaunchPlan(const mlts_gemm_product* ps, int count, int dtype, bool activation = false, bool rotation = false) : shape(dtype == MLTS_BF16 ? kBf16Shape : kF32Shape) {
+    if (dtype == MLTS_BF16) plan_bf16(ps, count, activation, rotation);
+    else plan_f32(ps, count, activation);
     for (int i = 0; i < count; ++i)
       if (slices[i] > 1) workspace += ps[i].M * ps[i].N * 4 * slices[i];
+  }
+
+ private:
+  void plan_f32(const mlts_gemm_product* ps, int count, bool activation) {
+    const mlts_gemm_product* small[kMaxProducts];
+    int small_at[kMaxProducts], smalls = 0;
+    for (int i = 0; i < count; ++i) {
+      tile[i] = choose_f32_tile(ps[i]), slices[i] = 1;
+      if (tile[i] == kSmall) small_at[smalls] = i, small[smalls++] = &ps[i];
+      together[i] = tile[i] == kSmall && (count > 1 || ps[i].segments > 1 || activation);
+    }
+    if (smalls == 0) return;
+    int64_t s[kMaxProducts], fine[kMaxProducts];
+    const double coarse = small_slices(small, smalls, shape, s);
+    if (small_slices(small, smalls, kF32Fine, fine) < coarse) shape = kF32Fine, std::copy(fine, fine + smalls, s);
+    for (int i = 0; i < smalls; ++i) slices[small_at[i]] = s[i];
+  }
+
+  // All products in one launch of small or of 128 x 128 tiles, or each by itself.  A weight gradient's split is the one it has alone, so that its
+  // bits do not depend on what shares its launch.
+  void plan_bf16(const mlts_gemm_product* ps, int count, bool activation, bool rotation) {
+    const mlts_gemm_product* all[kMaxProducts];
+    double apart = 0;
+    int joins = 0;
+    bool parts = false;
+    for (int i = 0; i < count; ++i) {
+      all[i] = &ps[i];
+      tile[i] = choose_bf16_tile(ps[i], &slices[i]);
+      apart += bf16_time(&all[i], 1, tile[i], &slices[i]) + (rotation ? pass_time(kRotationCost, tile[i], 0, 0) : 0);
+      joins += slices[i] > 1;
+      parts = parts || ps[i].segments > 1;
+    }
+    apart -= joins > 1 ? (joins - 1) * kJoinFixed : 0;  // one launch joins them all
+    if (count == 1 && !parts && !activation) {
+      if (rotation && slices[0] == 1)
+        for (int t = 0; t < kTiles; ++t) {
+          const auto time = [&](int at) { return bf16_time(all, 1, at, slices) + pass_time(kRotationCost, at, 0, 0); };
+          if (time(t) < time(tile[0])) tile[0] = t;
+        }
+      return;
+    }
+    double least = 0;
+    int best = -1;
+    int64_t best_slices[kMaxProducts], s[kMaxProducts];
+    for (int t : {kSmall, k128}) {
+      if (t != kSmall && parts) continue;
+      for (int64_t dx = 1; dx <= (activation ? 1 : 4); dx *= 2) {
+        for (int i = 0; i < count; ++i) s[i] = ps[i].form == FORM_TN ? slices[i] : ps[i].form == FORM_NN && splittable(ps[i]) && slabs_of(ps[i], 64) / dx >= 4 ? dx : 1;
+        double time = bf16_time(all, count, t, s) + (rotation ? pass_time(kRotationCost, t, 0, 0) : 0);
+        if (activation) time += pass_time(kActivationCost, t, ps[count - 1].M, ps[count - 1].N);
+        if (best < 0 || time < least) least = time, best = t, std::copy(s, s + count, best_slices);
+      }
+    }
+    if (!parts && !activation && apart < least) return;
+    std::fill(tile, tile + count, best), std::fill(together, together + count, true), std::copy(best_slices, best_slices + count, slices);
   }
 };
 
@@ -719,89 +922,100 @@ int opt_in_lds(MltsLdsOptIn& once, const void* kern, int bytes, S what) {
 }
 
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG = 1>
-int launch_tile(const Product& g, hipStream_t st) {
+int launch_tile(const Product& g, unsigned grid, hipStream_t st) {
   typedef TileShape<T, FORM, BM, BN, WM, WN, KG> S;
   static_assert(S::LDS <= 160 * 1024, "LDS");
   auto kern = gemm_kernel<T, FORM, BM, BN, WM, WN, KG>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm"); rc != MLTS_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g.tiles_m * g.tiles_n * g.slices)), dim3(S::THREADS), S::LDS, st, g);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(S::THREADS), S::LDS, st, g);
   return MLTS_OK;
 }
+// Columns of a wavefront of a 128 x 128 tile: in bf16 eight wavefronts of 128 registers, so that two tiles share a CU (us, four wavefronts /
+// eight: NT 2331 x 1536 x 512 10.6 / 9.4, NN 8192 x 1376 x 512 23.2 / 21.8)
+template <typename T>
+constexpr int k128Columns = sizeof(T) == 2 ? 32 : 64;
+
 template <typename T, int FORM>
-int launch_form(int tile, const SmallShape& shape, const Product& g, hipStream_t st) {
-  if (tile == 1) return launch_tile<T, FORM, 128, 128, 64, 64>(g, st);
-  if (tile == 2) return launch_tile<T, FORM, 256, 128, 64, 64>(g, st);
-  if (tile == 3) return launch_tile<T, FORM, 256, 256, 128, 64>(g, st);
+int launch_form(int tile, const SmallShape& shape, const Product& g, unsigned grid, hipStream_t st) {
+  if (tile == k128) return launch_tile<T, FORM, 128, 128, 64, k128Columns<T>>(g, grid, st);
+  if (tile == k256x128) return launch_tile<T, FORM, 256, 128, 64, 64>(g, grid, st);
+  if (tile == k256) return launch_tile<T, FORM, 256, 256, 128, 64>(g, grid, st);
   if constexpr (sizeof(T) == 4) {
-    if (shape.size == 32) return launch_tile<T, FORM, 32, 32, 32, 32, 4>(g, st);
+    if (shape.size == 32) return launch_tile<T, FORM, 32, 32, 32, 32, 4>(g, grid, st);
+  } else {
+    if (tile == k128x64) return launch_tile<T, FORM, 128, 64, 64, 32>(g, grid, st);
   }
-  return launch_tile<T, FORM, 64, 64, 32, 32>(g, st);
+  return launch_tile<T, FORM, 64, 64, 32, 32>(g, grid, st);
 }
 template <typename T>
-int launch_alone(int tile, const SmallShape& shape, const Product& g, hipStream_t st) {
-  if (g.form == FORM_NT) return launch_form<T, FORM_NT>(tile, shape, g, st);
-  return g.form == FORM_NN ? launch_form<T, FORM_NN>(tile, shape, g, st) : launch_form<T, FORM_TN>(tile, shape, g, st);
+int launch_alone(int tile, const SmallShape& shape, const Product& g, unsigned grid, hipStream_t st) {
+  if (g.form == FORM_NT) return launch_form<T, FORM_NT>(tile, shape, g, grid, st);
+  return g.form == FORM_NN ? launch_form<T, FORM_NN>(tile, shape, g, grid, st) : launch_form<T, FORM_TN>(tile, shape, g, grid, st);
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int KG = 1>
-int launch_rope_tile(const Product& g, const Rotation& rot, hipStream_t st) {
+int launch_rope_tile(const Product& g, const Rotation& rot, unsigned grid, hipStream_t st) {
   typedef TileShape<T, FORM_NT, BM, BN, WM, WN, KG> S;
   auto kern = gemm_rope_kernel<T, BM, BN, WM, WN, KG>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_rope"); rc != MLTS_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g.tiles_m * g.tiles_n)), dim3(S::THREADS), S::LDS, st, g, rot);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(S::THREADS), S::LDS, st, g, rot);
   return MLTS_OK;
 }
 template <typename T>
-int launch_rope_alone(int tile, const SmallShape& shape, const Product& g, const Rotation& rot, hipStream_t st) {
-  if (tile == 1) return launch_rope_tile<T, 128, 128, 64, 64>(g, rot, st);
-  if (tile == 2) return launch_rope_tile<T, 256, 128, 64, 64>(g, rot, st);
-  if (tile == 3) return launch_rope_tile<T, 256, 256, 128, 64>(g, rot, st);
+int launch_rope_alone(int tile, const SmallShape& shape, const Product& g, const Rotation& rot, unsigned grid, hipStream_t st) {
+  if (tile == k128) return launch_rope_tile<T, 128, 128, 64, k128Columns<T>>(g, rot, grid, st);
+  if (tile == k256x128) return launch_rope_tile<T, 256, 128, 64, 64>(g, rot, grid, st);
+  if (tile == k256) return launch_rope_tile<T, 256, 256, 128, 64>(g, rot, grid, st);
   if constexpr (sizeof(T) == 4) {
-    if (shape.size == 32) return launch_rope_tile<T, 32, 32, 32, 32, 4>(g, rot, st);
+    if (shape.size == 32) return launch_rope_tile<T, 32, 32, 32, 32, 4>(g, rot, grid, st);
+  } else {
+    if (tile == k128x64) return launch_rope_tile<T, 128, 64, 64, 32>(g, rot, grid, st);
   }
-  return launch_rope_tile<T, 64, 64, 32, 32>(g, rot, st);
+  return launch_rope_tile<T, 64, 64, 32, 32>(g, rot, grid, st);
 }
-template <typename T, int BM, int BN, int KG>
-int launch_rope_small(const Products& ps, const Rotation& rot, int blocks, hipStream_t st) {
-  typedef TileShape<T, FORM_NT, BM, BN, 32, 32, KG> S;
-  auto kern = gemm_multi_rope_kernel<T, BM, BN, KG>;
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+int launch_rope_joint(const Products& ps, const Rotation& rot, int blocks, hipStream_t st) {
+  typedef TileShape<T, FORM_NT, BM, BN, WM, WN, KG> S;
+  auto kern = gemm_multi_rope_kernel<T, BM, BN, WM, WN, KG>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_rope"); rc != MLTS_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), S::LDS, st, ps, rot);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(S::THREADS), S::LDS, st, ps, rot);
   return MLTS_OK;
 }
 
-template <typename T, int BM, int BN, int KG>
-int launch_act_small(const Products& ps, const Activation& act, int blocks, hipStream_t st) {
-  constexpr int bytes = std::max(TileShape<T, FORM_NN, BM, BN, 32, 32, KG>::LDS, TileShape<T, FORM_TN, BM, BN, 32, 32, KG>::LDS);
-  auto kern = gemm_multi_act_kernel<T, BM, BN, KG>;
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+int launch_act_joint(const Products& ps, const Activation& act, int blocks, hipStream_t st) {
+  typedef TileShape<T, FORM_NN, BM, BN, WM, WN, KG> S;
+  constexpr int bytes = std::max(S::LDS, TileShape<T, FORM_TN, BM, BN, WM, WN, KG>::LDS);
+  auto kern = gemm_multi_act_kernel<T, BM, BN, WM, WN, KG>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), bytes, "mlts_gemm_swiglu_bwd"); rc != MLTS_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), bytes, st, ps, act);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(S::THREADS), bytes, st, ps, act);
   return MLTS_OK;
 }
 
-template <typename T, int FORMS, int BM, int BN, int KG>
-int launch_small(const Products& ps, int blocks, hipStream_t st) {
-  constexpr int nt = TileShape<T, FORM_NT, BM, BN, 32, 32, KG>::LDS, nn = TileShape<T, FORM_NN, BM, BN, 32, 32, KG>::LDS,
-                tn = TileShape<T, FORM_TN, BM, BN, 32, 32, KG>::LDS;
-  constexpr int bytes = FORMS == FORMS_NT ? nt : FORMS == FORMS_NN ? nn : std::max(nt, std::max(nn, tn));
-  static_assert(TileShape<T, FORM_NT, BM, BN, 32, 32, KG>::THREADS == 256, "four wavefronts");
-  auto kern = gemm_multi_kernel<T, FORMS, BM, BN, KG>;
+template <typename T, int FORMS, int BM, int BN, int WM, int WN, int KG>
+int launch_joint(const Products& ps, int blocks, hipStream_t st) {
+  typedef TileShape<T, FORM_NT, BM, BN, WM, WN, KG> S;
+  constexpr int nn = TileShape<T, FORM_NN, BM, BN, WM, WN, KG>::LDS, tn = TileShape<T, FORM_TN, BM, BN, WM, WN, KG>::LDS;
+  constexpr int bytes = FORMS == FORMS_NT ? S::LDS : FORMS == FORMS_NN ? nn : std::max(S::LDS, std::max(nn, tn));
+  auto kern = gemm_multi_kernel<T, FORMS, BM, BN, WM, WN, KG>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), bytes, "mlts_gemm"); rc != MLTS_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), bytes, st, ps);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(S::THREADS), bytes, st, ps);
   return MLTS_OK;
 }
-template <typename T, int BM, int BN, int KG>
-int launch_small_forms(int forms, const Products& ps, int blocks, hipStream_t st) {
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+int launch_joint_forms(int forms, const Products& ps, int blocks, hipStream_t st) {
   switch (forms) {
-    case FORMS_NT: return launch_small<T, FORMS_NT, BM, BN, KG>(ps, blocks, st);
-    case FORMS_NN: return launch_small<T, FORMS_NN, BM, BN, KG>(ps, blocks, st);
-    case FORMS_ANY: return launch_small<T, FORMS_ANY, BM, BN, KG>(ps, blocks, st);
-    default: return launch_small<T, FORMS_SEGMENTS, BM, BN, KG>(ps, blocks, st);
+    case FORMS_NT: return launch_joint<T, FORMS_NT, BM, BN, WM, WN, KG>(ps, blocks, st);
+    case FORMS_NN: return launch_joint<T, FORMS_NN, BM, BN, WM, WN, KG>(ps, blocks, st);
+    case FORMS_ANY: return launch_joint<T, FORMS_ANY, BM, BN, WM, WN, KG>(ps, blocks, st);
+    default:
+      if constexpr (WM * WN == 32 * 32) return launch_joint<T, FORMS_SEGMENTS, BM, BN, WM, WN, KG>(ps, blocks, st);
+      else return MLTS_ERR_INVALID;  // (plans leave parts to the small tiles)
   }
 }
 
@@ -850,36 +1064,35 @@ mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const vo
 // alone or beside one of the TN form, or null.
 template <typename T>
 int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, const Rotation* rotation, const Activation* activation, hipStream_t st) {
-  const LaunchPlan plan(ps, count, dtype);
+  const LaunchPlan plan(ps, count, dtype, activation != nullptr, rotation != nullptr);
   Rotation rot{};
   if (rotation) rot = *rotation;
   Products joint;
   Joins joins{};
-  int blocks, join_blocks = 0, smalls;
+  int blocks, join_blocks = 0, together, joint_tile = kSmall;
   bool all_nt, all_nn;
   auto clear = [&] {
     joint = {};
     std::fill(joint.first, joint.first + kMaxProducts, 0x7fffffff);
-    blocks = smalls = 0, all_nt = all_nn = true;
+    blocks = together = 0, all_nt = all_nn = true;
   };
   auto launch = [&] {  // what `joint` holds
-    if (!smalls) return static_cast<int>(MLTS_OK);
-    if (activation) {
-      if constexpr (sizeof(T) == 4) {
-        if (plan.shape.size == 32) return launch_act_small<T, 32, 32, 4>(joint, *activation, blocks, st);
-      }
-      return launch_act_small<T, 64, 64, 1>(joint, *activation, blocks, st);
-    }
-    if (rotation) {
-      if constexpr (sizeof(T) == 4) {
-        if (plan.shape.size == 32) return launch_rope_small<T, 32, 32, 4>(joint, rot, blocks, st);
-      }
-      return launch_rope_small<T, 64, 64, 1>(joint, rot, blocks, st);
-    }
+    if (!together) return static_cast<int>(MLTS_OK);
     const int forms = joint.more.count ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
-    if constexpr (sizeof(T) == 2) return launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
-    else if (plan.shape.size == 64) return launch_small_forms<T, 64, 64, 1>(forms, joint, blocks, st);
-    else return launch_small_forms<T, 32, 32, 4>(forms, joint, blocks, st);
+    if constexpr (sizeof(T) == 4) {
+      if (plan.shape.size == 32) {
+        if (activation) return launch_act_joint<T, 32, 32, 32, 32, 4>(joint, *activation, blocks, st);
+        if (rotation) return launch_rope_joint<T, 32, 32, 32, 32, 4>(joint, rot, blocks, st);
+        return launch_joint_forms<T, 32, 32, 32, 32, 4>(forms, joint, blocks, st);
+      }
+    } else if (joint_tile == k128) {
+      if (activation) return launch_act_joint<T, 128, 128, 64, 32, 1>(joint, *activation, blocks, st);
+      if (rotation) return launch_rope_joint<T, 128, 128, 64, 32, 1>(joint, rot, blocks, st);
+      return launch_joint_forms<T, 128, 128, 64, 32, 1>(forms, joint, blocks, st);
+    }
+    if (activation) return launch_act_joint<T, 64, 64, 32, 32, 1>(joint, *activation, blocks, st);
+    if (rotation) return launch_rope_joint<T, 64, 64, 32, 32, 1>(joint, rot, blocks, st);
+    return launch_joint_forms<T, 64, 64, 32, 32, 1>(forms, joint, blocks, st);
   };
   clear();
   MltsKernelTimer timer("gemm", st);
@@ -895,8 +1108,8 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
     g.tiles_m = static_cast<int>((p.M + bm - 1) / bm), g.tiles_n = static_cast<int>((p.N + bn - 1) / bn);
     const int64_t slabs = slabs_of(p, slab_of(dtype));
     set_slices(g, plan.slices[i], slabs, slab_of(dtype));
-    const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices;
-    if (tiles == 0) continue;
+    if (g.tiles_m == 0 || g.tiles_n == 0) continue;
+    const int64_t grid = divide(g, bm, bn);
     if (p.segments > 1) {
       if (joint.more.count) {  // a launch has room for the segments of one product
         if (int rc = launch(); rc != MLTS_OK) return rc;
@@ -907,26 +1120,27 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
         joint.more.a[k - 1] = p.a[k], joint.more.b[k - 1] = p.b[k];
         joint.more.lda[k - 1] = static_cast<int>(p.lda[k]), joint.more.ldb[k - 1] = static_cast<int>(p.ldb[k]), joint.more.K[k - 1] = static_cast<int>(p.k[k]);
       }
-      joint.more.count = p.segments - 1, joint.more.product = smalls;
+      joint.more.count = p.segments - 1, joint.more.product = together;
     }
-    MLTS_REQUIRE(blocks + tiles < (int64_t{1} << 30), "mlts_gemm: too many tiles");
+    MLTS_REQUIRE(blocks + grid < (int64_t{1} << 30), "mlts_gemm: too many tiles");
     if (plan.slices[i] > 1) {
       g.partial = workspace;
       workspace += p.M * p.N * plan.slices[i];
       joins.p[joins.count++] = {p.c, g.partial, g.slices, g.accumulate, join_blocks, p.M * p.N / 4};
       join_blocks += static_cast<int>((p.M * p.N / 4 + 255) / 256);
     }
-    if (small && (count > 1 || p.segments > 1 || activation)) {
+    if (plan.together[i]) {
+      joint_tile = plan.tile[i];
       all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN;
-      joint.first[smalls] = blocks;
-      if (rotation) std::copy(rotation->columns[i], rotation->columns[i] + 4, rot.columns[smalls]);
-      blocks += static_cast<int>((tiles + 7) / 8 * 8);  // (whole rounds over the XCDs, so that each product starts at the first)
-      joint.p[smalls++] = g;
+      joint.first[together] = blocks;
+      if (rotation) std::copy(rotation->columns[i], rotation->columns[i] + 4, rot.columns[together]);
+      blocks += static_cast<int>(grid);  // (whole rounds over the XCDs, so that each product starts at the first)
+      joint.p[together++] = g;
     } else if (rotation) {
       Rotation own = *rotation;
       std::copy(rotation->columns[i], rotation->columns[i] + 4, own.columns[0]);
-      if (int rc = launch_rope_alone<T>(plan.tile[i], plan.shape, g, own, st); rc != MLTS_OK) return rc;
-    } else if (int rc = launch_alone<T>(plan.tile[i], plan.shape, g, st); rc != MLTS_OK) {
+      if (int rc = launch_rope_alone<T>(plan.tile[i], plan.shape, g, own, static_cast<unsigned>(grid), st); rc != MLTS_OK) return rc;
+    } else if (int rc = launch_alone<T>(plan.tile[i], plan.shape, g, static_cast<unsigned>(grid), st); rc != MLTS_OK) {
       return rc;
     }
   }
@@ -939,26 +1153,33 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
 int pair_tile(int64_t M, int64_t N, int64_t K, int dtype) {
   const mlts_gemm_product both = single(FORM_NT, M, 2 * N, K, nullptr, K, nullptr, K, nullptr, 2 * N, 0);
   const LaunchPlan plan(&both, 1, dtype);
-  return plan.slices[0] > 1 || plan.tile[0] == 3 || (plan.tile[0] == kSmall && plan.shape.size != 64) ? -1 : plan.tile[0];
+  if (plan.slices[0] > 1) return -1;
+  if (dtype == MLTS_F32) return plan.tile[0] == k256 || (plan.tile[0] == kSmall && plan.shape.size != 64) ? -1 : plan.tile[0];
+  const mlts_gemm_product* const one = &both;
+  const int64_t whole = 1;
+  const auto time = [&](int tile) { return bf16_time(&one, 1, tile, &whole) + pass_time(kPairCost, tile, M, N); };
+  return time(k128) < time(kSmall) ? k128 : kSmall;
 }
 
 template <typename T, int BM, int BN, int WM, int WN>
 int launch_pair(Product& g, const Pair& pair, hipStream_t st) {
   typedef TileShape<T, FORM_NT, BM, BN, WM, WN, 1, true> S;
   g.tiles_m = (g.M + BM - 1) / BM, g.tiles_n = (g.N + BN / 2 - 1) / (BN / 2);
-  const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n;
-  MLTS_REQUIRE(tiles < (int64_t{1} << 30), "mlts_gemm_swiglu: too many tiles");
+  const int64_t grid = divide(g, BM, BN);
+  MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm_swiglu: too many tiles");
   auto kern = gemm_pair_kernel<T, BM, BN, WM, WN>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_swiglu"); rc != MLTS_OK) return rc;
   MltsKernelTimer timer("gemm_swiglu", st);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(S::THREADS), S::LDS, st, g, pair);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(S::THREADS), S::LDS, st, g, pair);
   return mlts_check_launch("mlts_gemm_swiglu");
 }
 template <typename T>
 int run_pair(int tile, Product& g, const Pair& pair, hipStream_t st) {
-  if (tile == 1) return launch_pair<T, 128, 128, 64, 64>(g, pair, st);
-  if (tile == 2) return launch_pair<T, 256, 128, 64, 64>(g, pair, st);
+  if (tile == k128) return launch_pair<T, 128, 128, 64, k128Columns<T>>(g, pair, st);
+  if constexpr (sizeof(T) == 4) {
+    if (tile == k256x128) return launch_pair<T, 256, 128, 64, 64>(g, pair, st);
+  }
   return launch_pair<T, 64, 64, 32, 32>(g, pair, st);
 }
 
@@ -1087,8 +1308,9 @@ extern "C" const char* mlts_gemm_swiglu_bwd_supports(int32_t dtype, int32_t weig
   for (int i = 0; i < count; ++i)
     if (const char* why = why_not(ps[i], dtype)) return why;
   if (N % 4 || ldg % 4 || ldd % 4 || ldg < N || ldd < N || ldg > 0x7fffffff || ldd > 0x7fffffff) return "rows of gate and up are taken four elements at a time";
-  const LaunchPlan plan(ps, count, dtype);
-  if (plan.smalls != count || plan.slices[count - 1] > 1) return "products of this size are not made in one launch";
+  if (LaunchPlan(ps, count, dtype).slices[count - 1] > 1) return "a product that would be split";
+  const LaunchPlan plan(ps, count, dtype, true);
+  if (!std::all_of(plan.together, plan.together + count, [](bool t) { return t; }) || plan.slices[count - 1] > 1) return "products of this size are not made in one launch";
   *workspace_bytes = plan.workspace;
   return nullptr;
 }

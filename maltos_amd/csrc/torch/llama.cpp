@@ -372,8 +372,8 @@ Tensor project_all(const Tensor& x, const Adjacent& rows, const std::vector<Tens
   return y;
 }
 
-// gate and up of an MLP side by side (undefined if nobody keeps them), and round(silu(gate)) * up: in one launch up to the sizes of the own
-// products, where the pass over gate and up costs as much for its launch as for its bytes.
+// gate and up of an MLP side by side (undefined if nobody keeps them), and round(silu(gate)) * up: in one launch where the products run
+// on the own kernels: the pass over gate and up costs a launch in small calls and a read of both in large ones.
 std::pair<Tensor, Tensor> gate_up_activation(const Tensor& x, const Adjacent& rows, const std::vector<Tensor>& weights, bool keep) {
   const Tensor &wg = weights[0], &wu = weights[1], x2 = rows2d(x);
   const int64_t cols = wg.size(0), es = x.element_size();
@@ -413,6 +413,9 @@ struct Needed {
 
 // The input gradient, then one gradient per parameter, as far as they are needed: added into the gradient buffers where into_grad
 // allows it, and then undefined.  dy2: the outputs' gradients side by side.
+// M * N * K of each part up to which the input gradient of weights that are not adjacent is one contraction in parts: it runs on the small
+// tiles only, and beyond them the products and their sum one after the other are as fast
+constexpr double kOwnLimitParts = 4.0e9;
 variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, const Needed& need, const Tensor& x, const Tensor& dy2) {
   variable_list out(1 + weights.size());
   const Tensor x2 = rows2d(x);
@@ -432,7 +435,7 @@ variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights
       parts.push_back(dy2.narrow(1, a.first[i], weights[i].size(0)));
       into.push_back(need.weight[i] ? bound_grad(weights[i], into_grad) : Tensor());
       own = own && own_product(MLTS_GEMM_NN, parts[i], weights[i]) && own_product(MLTS_GEMM_TN, parts[i], x2) &&
-            (!into[i].defined() || own_output(into[i], x2));
+            static_cast<double>(x2.numel()) * weights[i].size(0) <= kOwnLimitParts && (!into[i].defined() || own_output(into[i], x2));
     }
     if (own) {
       ProductList list;
@@ -790,28 +793,31 @@ Tensor attention_block(const Tensor& x, const BlockWeights& w, int64_t heads, in
   return y;
 }
 
-// the gradients of an MLP's gate and up side by side, and (need_dw) of its last projection's weight, in one launch; undefined: sizes and
-// layouts that are left to the products and the pass over gate and up
+// the gradients of an MLP's gate and up side by side, and (need_dw) of its last projection's weight, in one launch where that runs on the own
+// kernels; undefined: sizes and layouts that are left to the products and the pass over gate and up
 std::pair<Tensor, Tensor> activation_and_weight_grad(const Tensor& dy2, const Tensor& w, const Tensor& h2, const Tensor& gu, const Adjacent& rows,
                                                      const Tensor& grad, bool need_dw) {
   const int64_t cols = w.size(1), es = gu.element_size(), width = gu.size(-1);
   if (width != 2 * cols || !gu.is_contiguous() || !aligned(gu) || (rows.first[0] * es) % 16 || (rows.first[1] * es) % 16 ||
-      !own_product(MLTS_GEMM_NN, dy2, w) || (need_dw && !own_product(MLTS_GEMM_TN, dy2, h2)) || gu.scalar_type() != dy2.scalar_type() || gu.numel() / width != dy2.size(0) ||
+      !own_product(MLTS_GEMM_NN, dy2, w) || gu.scalar_type() != dy2.scalar_type() || gu.numel() / width != dy2.size(0) ||
       (grad.defined() && (!own_output(grad, h2) || !grad.is_contiguous())))
     return {};
   int64_t ws_bytes = 0;
   const int dtype = dtype_code(dy2);
+  const bool apart = need_dw && !own_product(MLTS_GEMM_TN, dy2, h2);
+  if (apart) need_dw = false;
   if (mlts_gemm_swiglu_bwd_supports(dtype, need_dw, dy2.size(0), cols, dy2.size(1), dy2.stride(0), w.stride(0), h2.stride(0), width, width,
                                     &ws_bytes) != nullptr)
     return {};
   const Tensor dgu = at::empty(gu.sizes(), gu.options());
-  const Tensor dw = grad.defined() ? grad : need_dw ? at::empty(w.sizes(), dy2.options()) : Tensor();
+  Tensor dw = !need_dw ? Tensor() : grad.defined() ? grad : at::empty(w.sizes(), dy2.options());
   const Tensor ws = workspace(ws_bytes, dy2);
   const char* in = static_cast<const char*>(ptr(gu));
   char* out = static_cast<char*>(mptr(dgu));
   check(mlts_gemm_swiglu_bwd(dtype, dy2.size(0), cols, dy2.size(1), ptr(dy2), dy2.stride(0), ptr(w), w.stride(0), ptr(h2), h2.stride(0), need_dw ? mptr(dw) : nullptr,
                              grad.defined(), in + rows.first[0] * es, in + rows.first[1] * es, width, out + rows.first[0] * es, out + rows.first[1] * es, width,
                              ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
+  if (apart) dw = weight_grad(h2, dy2, grad);
   return {dgu, dw};
 }
 

@@ -8,17 +8,28 @@
 namespace maltos {
 namespace {
 
-// M * N * K up to which the own kernels run.  A product through torch costs 18 us of host time, a call here 5, and that is what
-// small steps wait for: up to a few thousand rows of a 512-wide model the host is behind the GPU.  On the GPU alone (both sides
-// captured; 256 to 4096 wide, 256 to 16384 rows, own over library's time for all products of a size together, the library's choice
-// untuned) they are ahead of it up to these lines, and behind from there:
-//   bf16  1 to 1.5e9  0.79 (y), 0.80 (dx), 0.79 (dW)    2.5 to 3e9  0.82, 0.85, 0.90    3 to 4e9  0.98, 1.02, 1.07
-//         4 to 5e9    1.14, 0.94, 0.97                  6 to 8e9    1.19, 1.28, 1.07    1.2 to 2e10  1.20, 1.14, 1.13
-//   fp32  0.5 to 1e9  0.86, 0.86, 0.82                  2.5 to 3e9  0.90, 0.92, 0.87    3 to 4e9  1.13, 1.15, 1.17
-// (16384 x 512 x 512: y 16.7 us against 16.1, or 17.6 against 15.0 with the shipped per-shape selection.)
+// Where the own kernels run, by M * N * K.  A product through torch costs 18 us of host time, a call here 5, and that is what
+// small steps wait for.  On the GPU alone (both sides timed with the weights out of HBM; rows from 100 to 16384; the library's choice
+// untuned, or with the shipped per-shape selection where that has the shape) they are ahead of the library
+//   fp32  0.5 to 1e9  0.86 of its time (y), 0.86 (dx), 0.82 (dW)    2.5 to 3e9  0.90, 0.92, 0.87    3 to 4e9  1.13, 1.15, 1.17
+//   bf16  up to 4e9   0.4 to 0.95
+//         above it, y and dx of 256 or 512 terms: 8192 x 2752 x 512 34.3 us against 61.7, 12000 x 2752 x 512 50 against 80, 16384 x 2752 x 512
+//         61 against 78, 16384 x 1376 x 512 36 against 50; but 16384 x 1536 x 512 38 against 32 with the shipped selection (rotated on
+//         its way out 39 against 32 + 15)
+//         1024 to 1536 terms: 12000 x 512 x 1376 31 against 36, 16384 x 512 x 1376 34 against 40, 16384 x 512 x 1536 32 against 35; but 6000 and
+//         12000 x 1024 x 1024 20.9 and 33.6 against 19.6 and 30.0
+//         2752 terms: 3000 x 512 21 against 26, 6000 x 512 31 against 33, 12000 x 512 50 against 46
+//         dW against a batch of row slices: 6000 rows 1536 x 512 27 against 44, 8192 rows 2752 x 512 46 against 52, 12000 rows 39 against 52
+//         and 58 against 95; but 16384 rows 47 against 41 and 73 against 63
+//         columns of a vocabulary (32000 x 512): 1023 rows 54 against 49, 3000 rows 136 against 131
 constexpr double kOwnLimitBf16 = 4.0e9, kOwnLimitF32 = 3.0e9;
+double larger_limit_bf16(int form, int64_t M, int64_t N, int64_t K) {
+  if (N >= 16384 || N % 8) return 0;
+  if (form == MLTS_GEMM_TN) return M < 16384 && K < 16384 ? 3.0e10 : 0;
+  return K <= 768 ? 3.0e10 : K <= 1536 ? 1.3e10 : K <= 2816 ? 8.5e9 : 0;
+}
 
-// Above it they still run for dx = dy W in bf16 with so long a contraction that it is split over workgroups (dx of an lm_head, of a wide
+// In bf16 they also run for dx = dy W with so long a contraction that it is split over workgroups (dx of an lm_head, of a wide
 // MLP): the library does not split those.  Own over library's time, 256 to 8192 rows, 512 to 4096 wide: 32000 terms 0.17 to 0.79, 11008
 // terms 0.54 to 0.83, 8192 terms 0.42 to 0.98; with 4096 or 5504 terms 0.76 to 1.04 where fewer than 128 tiles of 256 x 128 leave more
 // than half of the CUs idle unsplit, but 1.05 and 1.12 for 128 tiles (2048 x 2048 x 5504 56.6 us against 53.8, 1024 x 4096 x 4096 46.1
@@ -26,7 +37,7 @@ constexpr double kOwnLimitBf16 = 4.0e9, kOwnLimitF32 = 3.0e9;
 bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K) {
   const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
   if (dtype == MLTS_F32) return size <= kOwnLimitF32;
-  if (size <= kOwnLimitBf16) return true;
+  if (size <= std::max(kOwnLimitBf16, larger_limit_bf16(form, M, N, K))) return true;
   return form == MLTS_GEMM_NN && (K >= 8192 || M * N < 128 * 256 * 128) && mlts_gemm_workspace_bytes(form, dtype, M, N, K) > 0;
 }
 

@@ -242,3 +242,22 @@ def test_activation_gradients_in_the_products(dev, dtype, M, N, K, accumulate):
                                       gu.data_ptr() + N * es, 2 * N, dgu.data_ptr(), dgu.data_ptr() + N * es, 2 * N, ws.data_ptr(), need.value,
                                       torch.cuda.current_stream().cuda_stream))
     assert torch.equal(dw, want_dw) and torch.equal(dgu, want)
+
+
+@pytest.mark.parametrize("check,args", [
+    (test_product_forms, (NT, 2331, 1544, 512)), (test_product_forms, (NT, 3001, 1003, 264)), (test_product_forms, (NT, 129, 8200, 264)), (test_product_forms, (NN, 2331, 1384, 520)),
+    (test_product_forms, (NT, 4033, 504, 1384)), (test_product_forms, (NN, 4100, 520, 1528)), (test_product_forms, (NN, 16001, 1032, 72)), (test_product_forms, (TN, 520, 1384, 6008)),
+    (test_product_forms, (TN, 1544, 520, 4001)), (test_product_forms, (TN, 264, 264, 12001)), (test_group_of_projections, (6001, 512, (512, 256, 256))),
+    (test_product_into_rows_of_a_wider_buffer, (NN, 2331, 1376, 512)), (test_product_into_rows_of_a_wider_buffer, (TN, 520, 1384, 3008)),
+    (test_gate_up_in_one_launch, (2331, 1376, 512, True)), (test_gate_up_in_one_launch, (4097, 1384, 264, False)),
+    (test_rotation_in_the_products, (3, 1411, 8, 8, 64, 512, True, True)), (test_rotation_in_the_products, (40, 111, 8, 4, 64, 512, True, False)),
+    (test_rotation_in_the_products, (5, 1601, 8, 4, 64, 520, False, True)), (test_activation_gradients_in_the_products, (4097, 1376, 512, 1)),
+    (test_activation_gradients_in_the_products, (8200, 1384, 520, None))], ids=lambda v: v.__name__[5:] if callable(v) else "-".join(map(str, v)))
+def test_larger_bf16_tiles(dev, check, args):
+    """The tiles of 128 rows, alone, with others in a launch and with what follows the products in them: remainders of rows, columns and slabs,
+    rectangles of tiles that eight does not divide, columns that are not whole groups of four, split contractions, sequences shorter than
+    a tile."""
+    first = dict(form=args[0], M=args[1], N=args[2], K=args[3]) if check in (test_product_forms, test_product_into_rows_of_a_wider_buffer) else None
+    names = {test_group_of_projections: ("rows", "hidden", "widths"), test_gate_up_in_one_launch: ("M", "N", "K", "keep"),
+             test_rotation_in_the_products: ("B", "S", "H", "Hkv", "D", "K", "joint", "given"), test_activation_gradients_in_the_products: ("M", "N", "K", "accumulate")}
+    check(dev=dev, dtype=torch.bfloat16, **(first or dict(zip(names[check], args))))
