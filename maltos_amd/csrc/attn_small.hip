@@ -2,9 +2,10 @@
 // attn_bwd_dq_tr.hip, attn_bwd_split.hip).
 //
 // Those give a workgroup 128 or 256 rows and walk the other side 64 rows at a time, one tile behind the other at about a microsecond each:
-// with few rows and heads the kernel lasts as long as one workgroup's chain.  Here a wavefront owns 16 rows (queries in the forward and dQ
-// kernels, keys in the dK/dV kernel) and takes every `splits`-th unit of 32 rows of the other side, so that there are up to 64 times as many
-// wavefronts, with chains of a few units.  A unit arrives in whole lines, one unit ahead, and goes through LDS of its own wavefront to
+// with few rows and heads the kernel lasts as long as one workgroup's chain.  Here a wavefront owns R blocks of 16 rows (queries in the forward
+// and dQ kernels, keys in the dK/dV kernel) and takes every `splits`-th unit of 32 rows of the other side, so that there are up to 64 times as
+// many wavefronts, with chains of a few units.  Two blocks share what a wavefront fetches, puts to LDS and reads from there: on grids that fill the
+// chip that is most of a unit's time besides the softmax arithmetic (two_blocks()).  A unit arrives in whole lines, one unit ahead, and goes through LDS of its own wavefront to
 // the fragments of v_mfma_f32_16x16x32_bf16 (rows: 16-byte reads; contraction over the rows: transposing reads), without a barrier before
 // the splits' sums meet at the end.  Scores are computed transposed, as in the fp32 kernels, so that a lane holds the probabilities of one
 // own row and the next product takes them, rounded to bf16 once, from the registers they are in.
@@ -27,10 +28,19 @@ template <int D>
 struct Unit : Rows<D> {
   static constexpr int CHUNKS = D / 8, N = kUnit * CHUNKS / 64, BYTES = kUnit * Rows<D>::BYTES;
   bf16x8 raw[N];
-  __device__ __forceinline__ void fetch(const bf16_t* base, int64_t stride, int row0, int last, int lane) {
+  uint32_t stride, offset;  // bytes: between rows, of this lane's chunk in the first rows
+  __device__ __forceinline__ void init(int64_t elements, int lane) {
+    stride = static_cast<uint32_t>(elements) * 2u;
+    offset = static_cast<uint32_t>(lane / CHUNKS) * stride + 16u * static_cast<uint32_t>(lane % CHUNKS);
+  }
+  // rows row0 ..; rows past the last one are zeros, from the bounds check of the descriptor (near(): no offset wraps).  One addition a chunk:
+  // the row's part of the address is the same in all lanes.
+  __device__ __forceinline__ void fetch(const bf16_t* base, int row0, int last) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), 0, static_cast<uint32_t>(last) * stride + 2u * D, 0x00020000);
+    const uint32_t at = static_cast<uint32_t>(min(row0, last)) * stride;
 #pragma unroll
     for (int i = 0; i < N; ++i)
-      raw[i] = *reinterpret_cast<const bf16x8*>(row_of(base, min(row0 + (64 / CHUNKS) * i + lane / CHUNKS, last), stride) + 8 * (lane % CHUNKS));
+      raw[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset + (at + static_cast<uint32_t>(64 / CHUNKS * i) * stride), 0, 0));
   }
   __device__ __forceinline__ void put(unsigned char* lds, int lane) const {
 #pragma unroll
@@ -105,10 +115,11 @@ __device__ __forceinline__ void join_and_store(f32x4 (&acc)[N][NC], f32x4* lds, 
     }
 }
 
-// O and LSE of 16 query rows
-template <int D, bool DOC>
+// O and LSE of R * 16 query rows
+template <int D, bool DOC, int R>
 __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnParams p, const RowArgs a) {
   typedef Unit<D> U;
+  static_assert(!DOC || R == 1, "documents: one block of 16 rows to a wavefront");
   constexpr int FRAGS = D / 32, NC = D / 16;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const Place at(a);
@@ -116,15 +127,19 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
   // with a causal mask the last blocks are the long ones
   int bh, hq, member;
   const int qt = p.nqt - 1 - a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hq), hkv = a.group.over(hq, &member);
-  const int q0 = 16 * qt, qrow = q0 + l16;
+  const int q0 = 16 * R * qt;
   const bf16_t* K = static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
   const bf16_t* V = static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
-  const bf16_t* q_row = row_of(static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1], min(qrow, p.Sq - 1), p.qs[2]);
-  bf16x8 qf[FRAGS];
+  bf16x8 qf[R][FRAGS];
+  int klim[R];  // keys this lane's queries see: up to klim (causal_off is Sk without a causal mask); documents also by the plan's bits
 #pragma unroll
-  for (int j = 0; j < FRAGS; ++j) qf[j] = *reinterpret_cast<const bf16x8*>(q_row + 32 * j + 8 * g);
-  // keys this lane's query sees: up to klim (causal_off is Sk without a causal mask); documents also by the plan's bits
-  const int klim = DOC || qrow < p.Sq ? min(p.Sk - 1, DOC ? p.Sk : qrow + p.causal_off) : -1;
+  for (int r = 0; r < R; ++r) {
+    const int qrow = q0 + 16 * r + l16;
+    const bf16_t* q_row = row_of(static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1], min(qrow, p.Sq - 1), p.qs[2]);
+#pragma unroll
+    for (int j = 0; j < FRAGS; ++j) qf[r][j] = *reinterpret_cast<const bf16x8*>(q_row + 32 * j + 8 * g);
+    klim[r] = DOC || qrow < p.Sq ? min(p.Sk - 1, DOC ? p.Sk : qrow + p.causal_off) : -1;
+  }
   Walk<DOC, true> walk;
   walk.split = at.split, walk.splits = at.splits, walk.lane = lane;
   const unsigned long long* bits = nullptr;
@@ -132,59 +147,74 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
     const int group = q0 >> 6;
     walk.stats = p.k_stats + b * p.nk_stats;
     walk.own = p.q_stats[b * p.nq_stats + group];
-    bits = p.doc_bits + (static_cast<int64_t>(b) * p.nq_stats + group) * p.nk_stats * 64 + (qrow & 63);
+    bits = p.doc_bits + (static_cast<int64_t>(b) * p.nq_stats + group) * p.nk_stats * 64 + ((q0 + l16) & 63);
     walk.end = p.Sk;
   } else {
-    walk.end = max(0, min(p.Sk, min(q0 + 16, p.Sq) + p.causal_off));
+    walk.end = max(0, min(p.Sk, min(q0 + 16 * R, p.Sq) + p.causal_off));
   }
   const int kend = at.there ? walk.end : 0;
   const int all_klim = DOC ? p.Sk - 1 : min(p.Sk - 1, min(q0, p.Sq - 1) + p.causal_off);  // seen by every row (that exists)
 
-  float m = -INFINITY, l = 0.f;
-  f32x4 o[1][NC];
+  float m[R], l[R];
+  f32x4 o[R][NC];
 #pragma unroll
-  for (int db = 0; db < NC; ++db) o[0][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < R; ++r) {
+    m[r] = -INFINITY, l[r] = 0.f;
+#pragma unroll
+    for (int db = 0; db < NC; ++db) o[r][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   U keys, values;
+  keys.init(p.ks[2], lane), values.init(p.vs[2], lane);
   unsigned char *lk = lds_raw + at.wave * 2 * U::BYTES, *lv = lk + U::BYTES;
-  // (past the end the last key is fetched again: a branch around the loads would wait for all of them)
+  // (past the end some key is fetched again: a branch around the loads would wait for all of them)
   unsigned long long word = 0, word_now = 0;
   bool masked = false, masked_now = false;
   auto fetch_keys = [&](int k) {
-    keys.fetch(K, p.ks[2], k, p.Sk - 1, lane);
+    keys.fetch(K, k, p.Sk - 1);
     if (DOC) word = bits[static_cast<int64_t>(min(k, p.Sk - 1) >> 6) * 64], masked = walk.masked;
   };
   int k0 = walk.first(0), kn = k0;
   if (k0 < kend) {
     fetch_keys(k0);
-    values.fetch(V, p.vs[2], k0, p.Sk - 1, lane);
+    values.fetch(V, k0, p.Sk - 1);
     keys.put(lk, lane), values.put(lv, lane);
     word_now = word, masked_now = masked;
     kn = walk.next(k0);
     fetch_keys(kn);
-    values.fetch(V, p.vs[2], kn, p.Sk - 1, lane);
+    values.fetch(V, kn, p.Sk - 1);
   }
   while (k0 < kend) {
-    f32x4 s[2];
+    f32x4 s[R][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < FRAGS; ++j) s[u] = mfma32(U::dot(lk, u, j, l16, g), qf[j], s[u]);
+      for (int r = 0; r < R; ++r) s[r][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < FRAGS; ++j) {
+        const bf16x8 key = U::dot(lk, u, j, l16, g);
+#pragma unroll
+        for (int r = 0; r < R; ++r) s[r][u] = mfma32(key, qf[r][j], s[r][u]);
+      }
     }
     if (k0 + kUnit - 1 > all_klim) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (k0 + 16 * u + 4 * g + i > klim) s[u][i] = -INFINITY;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (k0 + 16 * u + 4 * g + i > klim[r]) s[r][u][i] = -INFINITY;
     }
     if (DOC && masked_now) {
-      const uint32_t w = static_cast<uint32_t>(word_now >> (k0 & 32));
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int r = 0; r < R; ++r) {
+        const uint32_t w = static_cast<uint32_t>(word_now >> (k0 & 32));
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (!((w >> (16 * u + 4 * g + i)) & 1)) s[u][i] = -INFINITY;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (!((w >> (16 * u + 4 * g + i)) & 1)) s[r][u][i] = -INFINITY;
+      }
     }
     const int kn2 = kn < kend ? walk.next(kn) : kn;
     const unsigned long long word_next = word;
@@ -192,66 +222,88 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
     keys.put(lk, lane);  // the next unit's, which have had one unit's time to arrive
     fetch_keys(kn2);
     __builtin_amdgcn_sched_barrier(0);
-    float mx = -INFINITY;
+    bf16x8 pr[R];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int r = 0; r < R; ++r) {
+      float mx = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[u][i]);
-    mx = max_groups(mx) * p.scale;
-    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
-      const float m_new = fmaxf(m, mx);
-      const float alpha = exponential(m - (m_new == -INFINITY ? 0.f : m_new));  // 1 for rows that do not rise, 0 from -inf
-      m = m_new;
-      l *= alpha;
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int db = 0; db < NC; ++db) o[0][db] *= alpha;
-    }
-    const float m_use = m == -INFINITY ? 0.f : m;
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[r][u][i]);
+      mx = max_groups(mx) * p.scale;
+      if (__builtin_amdgcn_ballot_w64(mx > m[r]) != 0) {
+        const float m_new = fmaxf(m[r], mx);
+        const float alpha = exponential(m[r] - (m_new == -INFINITY ? 0.f : m_new));  // 1 for rows that do not rise, 0 from -inf
+        m[r] = m_new;
+        l[r] *= alpha;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        s[u][i] = exponential(s[u][i] * p.scale - m_use);
-        l += s[u][i];
+        for (int db = 0; db < NC; ++db) o[r][db] *= alpha;
       }
-    const bf16x8 pr = pack(s);
+      const float m_use = m[r] == -INFINITY ? 0.f : m[r];
 #pragma unroll
-    for (int db = 0; db < NC; ++db) o[0][db] = mfma32(U::columns(lv, db, l16, g), pr, o[0][db]);
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s[r][u][i] = exponential(s[r][u][i] * p.scale - m_use);
+          l[r] += s[r][u][i];
+        }
+      pr[r] = pack(s[r]);
+    }
+#pragma unroll
+    for (int db = 0; db < NC; ++db) {
+      const bf16x8 column = U::columns(lv, db, l16, g);
+#pragma unroll
+      for (int r = 0; r < R; ++r) o[r][db] = mfma32(column, pr[r], o[r][db]);
+    }
     values.put(lv, lane);
-    values.fetch(V, p.vs[2], kn2, p.Sk - 1, lane);
+    values.fetch(V, kn2, p.Sk - 1);
     k0 = kn, kn = kn2, word_now = word_next, masked_now = masked_next;
   }
-  l = sum_groups(l);
+#pragma unroll
+  for (int r = 0; r < R; ++r) l[r] = sum_groups(l[r]);
   if (at.splits > 1) {  // every split holds some of the keys: all to the largest maximum
     __syncthreads();    // the units' LDS is free
-    float* ml = reinterpret_cast<float*>(lds_raw) + at.slot * at.splits * 32;
-    if (g == 0) ml[at.split * 32 + l16] = m, ml[at.split * 32 + 16 + l16] = l;
-    __syncthreads();
-    float m_new = -INFINITY;
-    for (int s = 0; s < at.splits; ++s) m_new = fmaxf(m_new, ml[s * 32 + l16]);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = exponential(m - m_use);
-    l = 0.f;
-    for (int s = 0; s < at.splits; ++s) l += ml[s * 32 + 16 + l16] * exponential(ml[s * 32 + l16] - m_use);
-    m = m_new;
+    float* ml = reinterpret_cast<float*>(lds_raw) + at.slot * at.splits * 32 * R;
+    if (g == 0) {
 #pragma unroll
-    for (int db = 0; db < NC; ++db) o[0][db] *= alpha;
+      for (int r = 0; r < R; ++r) ml[(at.split * R + r) * 32 + l16] = m[r], ml[(at.split * R + r) * 32 + 16 + l16] = l[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float* of = ml + r * 32 + l16;
+      float m_new = -INFINITY;
+      for (int s = 0; s < at.splits; ++s) m_new = fmaxf(m_new, of[s * R * 32]);
+      const float m_use = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = exponential(m[r] - m_use);
+      l[r] = 0.f;
+      for (int s = 0; s < at.splits; ++s) l[r] += of[s * R * 32 + 16] * exponential(of[s * R * 32] - m_use);
+      m[r] = m_new;
+#pragma unroll
+      for (int db = 0; db < NC; ++db) o[r][db] *= alpha;
+    }
   }
-  const bool mine = at.there && qrow < p.Sq;
-  if (mine && g == 0 && at.split == 0)
-    p.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] = l > 0.f ? m + logf(l) : -INFINITY;
-  const int64_t row = b * p.os[0] + hq * p.os[1] + static_cast<int64_t>(qrow) * p.os[2] + 4 * g;
-  const float scale = l > 0.f ? 1.0f / l : 0.f;
-  join_and_store(o, reinterpret_cast<f32x4*>(lds_raw), at, [&](int, int db, f32x4 v) {
-    if (mine) store4(p.o, row + 16 * db, v * scale, 0);
+  const int64_t row = b * p.os[0] + hq * p.os[1] + 4 * g;
+  float scale[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int qrow = q0 + 16 * r + l16;
+    if (at.there && qrow < p.Sq && g == 0 && at.split == 0)
+      p.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] = l[r] > 0.f ? m[r] + logf(l[r]) : -INFINITY;
+    scale[r] = l[r] > 0.f ? 1.0f / l[r] : 0.f;
+  }
+  join_and_store(o, reinterpret_cast<f32x4*>(lds_raw), at, [&](int r, int db, f32x4 v) {
+    const int qrow = q0 + 16 * r + l16;
+    if (at.there && qrow < p.Sq) store4(p.o, row + qrow * p.os[2] + 16 * db, v * (R == 1 || r == 0 ? scale[0] : scale[R - 1]), 0);
   });
 }
 
-// dQ of 16 query rows: dq = scale * sum_j ds_ij k_j, ds = p (dp - delta), p = exp(scale s - lse).  Runs first in a backward pass and writes
+// dQ of R * 16 query rows: dq = scale * sum_j ds_ij k_j, ds = p (dp - delta), p = exp(scale s - lse).  Runs first in a backward pass and writes
 // delta = rowsum(dO * O) for the dK/dV kernel.  bp.dq_f32: dq is fp32 and added to (1) or overwritten (2); 0: bf16.
-template <int D, bool DOC>
+template <int D, bool DOC, int R>
 __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnBwdParams bp, const RowArgs a) {
   typedef Unit<D> U;
+  static_assert(!DOC || R == 1, "documents: one block of 16 rows to a wavefront");
   constexpr int FRAGS = D / 32, NC = D / 16;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -260,33 +312,38 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
   // with a causal mask the last blocks are the long ones
   int bh, hq, member;
   const int qt = p.nqt - 1 - a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hq), hkv = a.group.over(hq, &member);
-  const int q0 = 16 * qt, qrow = q0 + l16, safe = min(qrow, p.Sq - 1);
+  const int q0 = 16 * R * qt;
   const bf16_t* K = static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1];
   const bf16_t* V = static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1];
-  const bf16_t* q_row = row_of(static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1], safe, p.qs[2]);
-  const bf16_t* do_row = row_of(static_cast<const bf16_t*>(bp.dout) + b * bp.dos[0] + hq * bp.dos[1], safe, bp.dos[2]);
-  const bf16_t* o_row = row_of(static_cast<const bf16_t*>(p.o) + b * p.os[0] + hq * p.os[1], safe, p.os[2]);
-  bf16x8 qf[FRAGS], dof[FRAGS];
-  float delta = 0.f;
+  bf16x8 qf[R][FRAGS], dof[R][FRAGS];
+  float delta[R], lse[R];
+  int klim[R];
 #pragma unroll
-  for (int j = 0; j < FRAGS; ++j) {
-    qf[j] = *reinterpret_cast<const bf16x8*>(q_row + 32 * j + 8 * g);
-    dof[j] = *reinterpret_cast<const bf16x8*>(do_row + 32 * j + 8 * g);
-    const bf16x8 of = *reinterpret_cast<const bf16x8*>(o_row + 32 * j + 8 * g);
+  for (int r = 0; r < R; ++r) {
+    const int qrow = q0 + 16 * r + l16, safe = min(qrow, p.Sq - 1);
+    const bf16_t* q_row = row_of(static_cast<const bf16_t*>(p.q) + b * p.qs[0] + hq * p.qs[1], safe, p.qs[2]);
+    const bf16_t* do_row = row_of(static_cast<const bf16_t*>(bp.dout) + b * bp.dos[0] + hq * bp.dos[1], safe, bp.dos[2]);
+    const bf16_t* o_row = row_of(static_cast<const bf16_t*>(p.o) + b * p.os[0] + hq * p.os[1], safe, p.os[2]);
+    float sum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) delta += static_cast<float>(dof[j][e]) * static_cast<float>(of[e]);
-  }
-  delta = sum_groups(delta);
-  const int64_t stat = (static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + safe;
-  float lse = p.lse[stat];
-  lse = qrow < p.Sq && lse != -INFINITY ? lse : INFINITY;  // rows that saw no key: every probability 0
-  const bool mine = at.there && qrow < p.Sq;
-  if (mine && g == 0 && at.split == 0) {  // the statistics of the backward pass, for whichever dK/dV kernel comes next
-    bp.delta_out[stat] = delta;
-    bp.lse2_out[stat] = lse * 1.44269504088896340736f;
+    for (int j = 0; j < FRAGS; ++j) {
+      qf[r][j] = *reinterpret_cast<const bf16x8*>(q_row + 32 * j + 8 * g);
+      dof[r][j] = *reinterpret_cast<const bf16x8*>(do_row + 32 * j + 8 * g);
+      const bf16x8 of = *reinterpret_cast<const bf16x8*>(o_row + 32 * j + 8 * g);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum += static_cast<float>(dof[r][j][e]) * static_cast<float>(of[e]);
+    }
+    delta[r] = sum_groups(sum);
+    const int64_t stat = (static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + safe;
+    lse[r] = p.lse[stat];
+    lse[r] = qrow < p.Sq && lse[r] != -INFINITY ? lse[r] : INFINITY;  // rows that saw no key: every probability 0
+    if (at.there && qrow < p.Sq && g == 0 && at.split == 0) {  // the statistics of the backward pass, for whichever dK/dV kernel comes next
+      bp.delta_out[stat] = delta[r];
+      bp.lse2_out[stat] = lse[r] * 1.44269504088896340736f;
+    }
+    klim[r] = DOC || qrow < p.Sq ? min(p.Sk - 1, DOC ? p.Sk : qrow + p.causal_off) : -1;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) bp.lse2_out[static_cast<int64_t>(p.B) * p.Hq * p.Sq] = INFINITY;
-  const int klim = DOC || qrow < p.Sq ? min(p.Sk - 1, DOC ? p.Sk : qrow + p.causal_off) : -1;
   Walk<DOC, true> walk;
   walk.split = at.split, walk.splits = at.splits, walk.lane = lane;
   const unsigned long long* bits = nullptr;
@@ -294,24 +351,27 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     const int group = q0 >> 6;
     walk.stats = p.k_stats + b * p.nk_stats;
     walk.own = p.q_stats[b * p.nq_stats + group];
-    bits = p.doc_bits + (static_cast<int64_t>(b) * p.nq_stats + group) * p.nk_stats * 64 + (qrow & 63);
+    bits = p.doc_bits + (static_cast<int64_t>(b) * p.nq_stats + group) * p.nk_stats * 64 + ((q0 + l16) & 63);
     walk.end = p.Sk;
   } else {
-    walk.end = max(0, min(p.Sk, min(q0 + 16, p.Sq) + p.causal_off));
+    walk.end = max(0, min(p.Sk, min(q0 + 16 * R, p.Sq) + p.causal_off));
   }
   const int kend = at.there ? walk.end : 0;
   const int all_klim = DOC ? p.Sk - 1 : min(p.Sk - 1, min(q0, p.Sq - 1) + p.causal_off);
 
-  f32x4 dq[1][NC];
+  f32x4 dq[R][NC];
 #pragma unroll
-  for (int db = 0; db < NC; ++db) dq[0][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int db = 0; db < NC; ++db) dq[r][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   U keys, values;
+  keys.init(p.ks[2], lane), values.init(p.vs[2], lane);
   unsigned char *lk = lds_raw + at.wave * 2 * U::BYTES, *lv = lk + U::BYTES;
   unsigned long long word = 0, word_now = 0;
   bool masked = false, masked_now = false;
   auto fetch = [&](int k) {  // (past the end the last key again: a branch around the loads would wait for all of them)
-    keys.fetch(K, p.ks[2], k, p.Sk - 1, lane);
-    values.fetch(V, p.vs[2], k, p.Sk - 1, lane);
+    keys.fetch(K, k, p.Sk - 1);
+    values.fetch(V, k, p.Sk - 1);
     if (DOC) word = bits[static_cast<int64_t>(min(k, p.Sk - 1) >> 6) * 64], masked = walk.masked;
   };
   auto put = [&] {
@@ -326,28 +386,50 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     fetch(kn);
   }
   while (k0 < kend) {
-    f32x4 s[2], dp[2];
+    f32x4 s[R][2], dp[R][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      s[u] = dp[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r][u] = dp[r][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < FRAGS; ++j) {
-        s[u] = mfma32(U::dot(lk, u, j, l16, g), qf[j], s[u]);
-        dp[u] = mfma32(U::dot(lv, u, j, l16, g), dof[j], dp[u]);
+        const bf16x8 key = U::dot(lk, u, j, l16, g), value = U::dot(lv, u, j, l16, g);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          s[r][u] = mfma32(key, qf[r][j], s[r][u]);
+          dp[r][u] = mfma32(value, dof[r][j], dp[r][u]);
+        }
       }
     }
     const bool edge = k0 + kUnit - 1 > all_klim;
-    const uint32_t w = DOC && masked_now ? static_cast<uint32_t>(word_now >> (k0 & 32)) : ~0u;
+    bf16x8 ds[R];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float pv = exponential(s[u][i] * p.scale - lse);
-        if (edge && k0 + 16 * u + 4 * g + i > klim) pv = 0.f;
-        if (DOC && !((w >> (16 * u + 4 * g + i)) & 1)) pv = 0.f;
-        s[u][i] = pv * (dp[u][i] - delta);
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[r][u][i] = exponential(s[r][u][i] * p.scale - lse[r]);
+      if (edge) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (k0 + 16 * u + 4 * g + i > klim[r]) s[r][u][i] = 0.f;
       }
-    const bf16x8 ds = pack(s);
+      if (DOC && masked_now) {
+        const uint32_t w = static_cast<uint32_t>(word_now >> (k0 & 32));
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (!((w >> (16 * u + 4 * g + i)) & 1)) s[r][u][i] = 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[r][u][i] *= dp[r][u][i] - delta[r];
+      ds[r] = pack(s[r]);
+    }
     bf16x8 kc[NC];
 #pragma unroll
     for (int db = 0; db < NC; ++db) kc[db] = U::columns(lk, db, l16, g);
@@ -356,19 +438,23 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     fetch(kn2);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int db = 0; db < NC; ++db) dq[0][db] = mfma32(kc[db], ds, dq[0][db]);
+    for (int db = 0; db < NC; ++db)
+#pragma unroll
+      for (int r = 0; r < R; ++r) dq[r][db] = mfma32(kc[db], ds[r], dq[r][db]);
     k0 = kn, kn = kn2;
   }
-  const int64_t row = b * bp.dqs[0] + hq * bp.dqs[1] + static_cast<int64_t>(qrow) * bp.dqs[2] + 4 * g;
-  join_and_store(dq, reinterpret_cast<f32x4*>(lds_raw), at, [&](int, int db, f32x4 v) {
-    if (mine) store4(bp.dq_acc, row + 16 * db, v * p.scale, bp.dq_f32);
+  const int64_t row = b * bp.dqs[0] + hq * bp.dqs[1] + 4 * g;
+  join_and_store(dq, reinterpret_cast<f32x4*>(lds_raw), at, [&](int r, int db, f32x4 v) {
+    const int qrow = q0 + 16 * r + l16;
+    if (at.there && qrow < p.Sq) store4(bp.dq_acc, row + qrow * bp.dqs[2] + 16 * db, v * p.scale, bp.dq_f32);
   });
 }
 
-// dK, dV of 16 key rows of one KV head, summed over the query heads of its group.
-template <int D, bool DOC>
+// dK, dV of R * 16 key rows of one KV head, summed over the query heads of its group.
+template <int D, bool DOC, int R>
 __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const AttnBwdParams bp, const RowArgs a) {
   typedef Unit<D> U;
+  static_assert(!DOC || R == 1, "documents: one block of 16 rows to a wavefront");
   constexpr int FRAGS = D / 32, NC = D / 16;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -377,17 +463,21 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
   // with a causal mask the first blocks are the long ones
   int bh, hkv;
   const int kt = a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hkv), group = static_cast<int>(a.group.d);
-  const int kb0 = kt * 16, krow = kb0 + l16, ksafe = min(krow, p.Sk - 1);
-  const bf16_t* k_row = row_of(static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1], ksafe, p.ks[2]);
-  const bf16_t* v_row = row_of(static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1], ksafe, p.vs[2]);
-  bf16x8 kf[FRAGS], vf[FRAGS];
+  const int kb0 = kt * 16 * R;
+  bf16x8 kf[R][FRAGS], vf[R][FRAGS];
 #pragma unroll
-  for (int j = 0; j < FRAGS; ++j) {
-    kf[j] = *reinterpret_cast<const bf16x8*>(k_row + 32 * j + 8 * g);
-    vf[j] = *reinterpret_cast<const bf16x8*>(v_row + 32 * j + 8 * g);
+  for (int r = 0; r < R; ++r) {
+    const int ksafe = min(kb0 + 16 * r + l16, p.Sk - 1);
+    const bf16_t* k_row = row_of(static_cast<const bf16_t*>(p.k) + b * p.ks[0] + hkv * p.ks[1], ksafe, p.ks[2]);
+    const bf16_t* v_row = row_of(static_cast<const bf16_t*>(p.v) + b * p.vs[0] + hkv * p.vs[1], ksafe, p.vs[2]);
+#pragma unroll
+    for (int j = 0; j < FRAGS; ++j) {
+      kf[r][j] = *reinterpret_cast<const bf16x8*>(k_row + 32 * j + 8 * g);
+      vf[r][j] = *reinterpret_cast<const bf16x8*>(v_row + 32 * j + 8 * g);
+    }
   }
-  const int qlim = DOC ? 0 : krow - p.causal_off;                               // first query that sees this lane's key
-  const int all_qmin = DOC ? 0 : min(kb0 + 15, p.Sk - 1) - p.causal_off;        // from here on every key that exists is seen
+  const int qlim = DOC ? 0 : kb0 + l16 - p.causal_off;                              // first query that sees this lane's first key
+  const int all_qmin = DOC ? 0 : min(kb0 + 16 * R - 1, p.Sk - 1) - p.causal_off;    // from here on every key that exists is seen
   Walk<DOC, false> walk;
   walk.split = at.split, walk.splits = at.splits, walk.lane = lane, walk.end = p.Sq;
   const unsigned long long* bits = nullptr;
@@ -396,15 +486,18 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
     const int tile = kb0 >> 6;
     walk.stats = p.q_stats + b * p.nq_stats;
     walk.own = p.k_stats[b * p.nk_stats + tile];
-    bits = p.doc_bits_k + (static_cast<int64_t>(b) * p.nk_stats + tile) * p.nq_stats * 64 + (krow & 63);
+    bits = p.doc_bits_k + (static_cast<int64_t>(b) * p.nk_stats + tile) * p.nq_stats * 64 + ((kb0 + l16) & 63);
   } else {
     qstart = max(0, kb0 - p.causal_off) / kUnit * kUnit;
   }
 
-  f32x4 dkv[2][NC];
+  f32x4 dkv[2 * R][NC];  // dK of each block, dV of each
 #pragma unroll
-  for (int db = 0; db < NC; ++db) dkv[0][db] = dkv[1][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int n = 0; n < 2 * R; ++n)
+#pragma unroll
+    for (int db = 0; db < NC; ++db) dkv[n][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   U queries, grads;
+  queries.init(p.qs[2], lane), grads.init(bp.dos[2], lane);
   unsigned char* own = lds_raw + at.wave * (2 * U::BYTES + 256);
   unsigned char *lq = own, *ld = own + U::BYTES;
   float* lstat = reinterpret_cast<float*>(own + 2 * U::BYTES);  // (lse, delta) of the unit's queries: a lane fetches one, and reads eight of each
@@ -416,8 +509,8 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
   int row_fetched = 0;
   auto fetch = [&](int hg, int q) {  // (past the end the last query again: a branch around the loads would wait for all of them)
     const int head = hkv * group + hg;
-    queries.fetch(Q0 + head * p.qs[1], p.qs[2], q, p.Sq - 1, lane);
-    grads.fetch(dO0 + head * bp.dos[1], bp.dos[2], q, p.Sq - 1, lane);
+    queries.fetch(Q0 + head * p.qs[1], q, p.Sq - 1);
+    grads.fetch(dO0 + head * bp.dos[1], q, p.Sq - 1);
     row_fetched = q + (lane & 31);
     stat = (lane < 32 ? p.lse : bp.delta)[(static_cast<int64_t>(b) * p.Hq + head) * p.Sq + min(row_fetched, p.Sq - 1)];
     if (DOC) word = bits[static_cast<int64_t>(min(q, p.Sq - 1) >> 6) * 64], masked = walk.masked;
@@ -443,36 +536,59 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
     fetch(min(hn, group - 1), qn);
   }
   while (hg < group) {
-    f32x4 s[2], dp[2], lse[2], delta[2];
+    f32x4 s[R][2], dp[R][2], lse[2], delta[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      s[u] = dp[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r][u] = dp[r][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < FRAGS; ++j) {
-        s[u] = mfma32(U::dot(lq, u, j, l16, g), kf[j], s[u]);
-        dp[u] = mfma32(U::dot(ld, u, j, l16, g), vf[j], dp[u]);
+        const bf16x8 query = U::dot(lq, u, j, l16, g), grad = U::dot(ld, u, j, l16, g);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          s[r][u] = mfma32(query, kf[r][j], s[r][u]);
+          dp[r][u] = mfma32(grad, vf[r][j], dp[r][u]);
+        }
       }
       lse[u] = *reinterpret_cast<const f32x4*>(lstat + 16 * u + 4 * g);
       delta[u] = *reinterpret_cast<const f32x4*>(lstat + 32 + 16 * u + 4 * g);
     }
     const bool edge = !DOC && q0 < all_qmin;
-    const uint32_t w = DOC && masked_now ? static_cast<uint32_t>(word_now >> (q0 & 32)) : ~0u;
+    bf16x8 pr[R], ds[R];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float pv = exponential(s[u][i] * p.scale - lse[u][i]);
-        if (edge && q0 + 16 * u + 4 * g + i < qlim) pv = 0.f;
-        if (DOC && !((w >> (16 * u + 4 * g + i)) & 1)) pv = 0.f;
-        s[u][i] = pv;
-        dp[u][i] = pv * (dp[u][i] - delta[u][i]);
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[r][u][i] = exponential(s[r][u][i] * p.scale - lse[u][i]);
+      if (edge) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (q0 + 16 * u + 4 * g + i < qlim + 16 * r) s[r][u][i] = 0.f;
       }
-    const bf16x8 pr = pack(s), ds = pack(dp);
+      if (DOC && masked_now) {
+        const uint32_t w = static_cast<uint32_t>(word_now >> (q0 & 32));
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (!((w >> (16 * u + 4 * g + i)) & 1)) s[r][u][i] = 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dp[r][u][i] = s[r][u][i] * (dp[r][u][i] - delta[u][i]);
+      pr[r] = pack(s[r]), ds[r] = pack(dp[r]);
+    }
     bf16x8 col[NC];
 #pragma unroll
     for (int db = 0; db < NC; ++db) col[db] = U::columns(ld, db, l16, g);
 #pragma unroll
-    for (int db = 0; db < NC; ++db) dkv[1][db] = mfma32(col[db], pr, dkv[1][db]);
+    for (int db = 0; db < NC; ++db)
+#pragma unroll
+      for (int r = 0; r < R; ++r) dkv[R + r][db] = mfma32(col[db], pr[r], dkv[R + r][db]);
 #pragma unroll
     for (int db = 0; db < NC; ++db) col[db] = U::columns(lq, db, l16, g);
     int hn2 = hn, qn2 = qn;
@@ -481,48 +597,50 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
     fetch(min(hn2, group - 1), qn2);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int db = 0; db < NC; ++db) dkv[0][db] = mfma32(col[db], ds, dkv[0][db]);
+    for (int db = 0; db < NC; ++db)
+#pragma unroll
+      for (int r = 0; r < R; ++r) dkv[r][db] = mfma32(col[db], ds[r], dkv[r][db]);
     hg = hn, q0 = qn, hn = hn2, qn = qn2;
   }
-  const bool mine = at.there && krow < p.Sk;
-  const int64_t dk_row = b * bp.dks[0] + hkv * bp.dks[1] + static_cast<int64_t>(krow) * bp.dks[2] + 4 * g;
-  const int64_t dv_row = b * bp.dvs[0] + hkv * bp.dvs[1] + static_cast<int64_t>(krow) * bp.dvs[2] + 4 * g;
+  const int64_t dk_row = b * bp.dks[0] + hkv * bp.dks[1] + 4 * g, dv_row = b * bp.dvs[0] + hkv * bp.dvs[1] + 4 * g;
   join_and_store(dkv, reinterpret_cast<f32x4*>(lds_raw), at, [&](int n, int db, f32x4 v) {
-    if (mine) store4(n == 0 ? bp.dk : bp.dv, (n == 0 ? dk_row : dv_row) + 16 * db, n == 0 ? v * p.scale : v, bp.accumulate_f32);
+    const int krow = kb0 + 16 * (n < R ? n : n - R) + l16;
+    if (at.there && krow < p.Sk)
+      store4(n < R ? bp.dk : bp.dv, (n < R ? dk_row + krow * bp.dks[2] : dv_row + krow * bp.dvs[2]) + 16 * db, n < R ? v * p.scale : v, bp.accumulate_f32);
   });
 }
 
 bool near(int64_t rows, const int64_t* stride) {  // offsets that row_of can form
-  return rows < (1 << 24) && stride[2] < (1 << 23) && ((rows - 1) * stride[2] + 128) * 2 < (int64_t{1} << 32);
+  return rows < (1 << 24) && stride[2] < (1 << 23) && ((rows - 1 + kUnit) * stride[2] + 128) * 2 < (int64_t{1} << 32);
 }
 
-template <int D, bool DOC>
+template <int D, bool DOC, int R>
 int fwd(AttnParams p, hipStream_t st) {
-  p.nqt = (p.Sq + 15) / 16;
+  p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   MltsKernelTimer timer("attn_fwd", st);
-  return launch_splits<attn_small_fwd<D, DOC>, kMaxSplits>(blocks, splits_for(blocks, (p.Sk + kUnit - 1) / kUnit, kMaxSplits), D * 64, 2 * Unit<D>::BYTES, st, p,
-                                                           RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_fwd");
+  return launch_splits<attn_small_fwd<D, DOC, R>, kMaxSplits>(blocks, splits_for(blocks, (p.Sk + kUnit - 1) / kUnit, kMaxSplits), R * D * 64, 2 * Unit<D>::BYTES, st, p,
+                                                              RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_fwd");
 }
 
-template <int D, bool DOC>
+template <int D, bool DOC, int R>
 int bwd_dq(AttnBwdParams bp, hipStream_t st) {
   AttnParams& p = bp.a;
-  p.nqt = (p.Sq + 15) / 16;
+  p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   MltsKernelTimer timer("attn_bwd_dq", st);
-  return launch_splits<attn_small_bwd_dq<D, DOC>, kMaxSplits>(blocks, splits_for(blocks, (p.Sk + kUnit - 1) / kUnit, kMaxSplits), D * 64, 2 * Unit<D>::BYTES, st, bp,
-                                                              RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_bwd");
+  return launch_splits<attn_small_bwd_dq<D, DOC, R>, kMaxSplits>(blocks, splits_for(blocks, (p.Sk + kUnit - 1) / kUnit, kMaxSplits), R * D * 64, 2 * Unit<D>::BYTES, st, bp,
+                                                                 RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_bwd");
 }
 
-template <int D, bool DOC>
+template <int D, bool DOC, int R>
 int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
   const AttnParams& p = bp.a;
-  const int tiles = (p.Sk + 15) / 16;
+  const int tiles = (p.Sk + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(tiles) * p.B * p.Hkv, units = static_cast<int64_t>((p.Sq + kUnit - 1) / kUnit) * (p.Hq / p.Hkv);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
-  return launch_splits<attn_small_bwd_dkv<D, DOC>, kMaxSplits>(blocks, splits_for(blocks, units, kMaxSplits), 2 * D * 64, 2 * Unit<D>::BYTES + 256, st, bp,
-                                                               RowArgs(p, D, true, p.Hkv, tiles), "mlts_attn_bwd");
+  return launch_splits<attn_small_bwd_dkv<D, DOC, R>, kMaxSplits>(blocks, splits_for(blocks, units, kMaxSplits), 2 * R * D * 64, 2 * Unit<D>::BYTES + 256, st, bp,
+                                                                  RowArgs(p, D, true, p.Hkv, tiles), "mlts_attn_bwd");
 }
 
 }  // namespace
@@ -533,51 +651,87 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 // calls differ by 3 us and less (4 heads x 2 x 200: 8.4 us there, 5.5 here), which launching them hides; they keep one arithmetic for all
 // batch sizes, which a number of splits that depends on the grid does not have.
 //
-// And the grid has to be small, for a 16-row block reads the other side for 16 rows only.  us there -> here, forward, dQ, dK/dV (causal):
-//   head_dim 64    512 blocks  8 heads x 1024      20.0 21.7 18.8 ->  9.5 10.4 10.8     4 x 2048       34.0 35.8 33.5 -> 13.8 14.4 17.0
-//                 1024 blocks  2 x 8 heads x 1024  20.1 21.9 19.4 -> 14.5 15.2 18.1     8 x 2048       35.0 36.9 35.0 -> 22.2 23.2 28.1
-//                 1176 blocks  3 x 8 heads x 777   16.8 18.3 18.0 -> 13.9 16.2 17.6
-//                 1536 blocks  3 x 8 heads x 1024  20.5 22.7 21.7 -> 18.2 20.7 22.2    12 x 2048       35.3 37.9 39.1 -> 26.0 31.2 37.1
-//                 2048 blocks  4 x 8 heads x 1024  20.8 23.5 24.0 -> 21.2 24.8 28.4     8 x 4096       67.6 71.0 78.1 -> 66.2 77.4 98.3
-//   head_dim 128   512 blocks  8 heads x 1024      24.8 38.5 33.1 -> 15.2 17.0 17.1     2 x 4096         85  129  113 ->   34   35   43
-//                  768 blocks  3 x 4 heads x 1024  24.8 38.6 33.5 -> 22.4 26.0 26.6
-//                 1024 blocks  8 x 4 heads x 512   16.1 24.6 20.7 -> 18.4 22.2 22.0
-//   documents     1280 blocks  20 heads x 1023      15.2 16.4      -> 15.2 17.3
-//                 1024 blocks  2 x 8 heads x 1023  15.3 16.1 17.0 -> 12.3 14.2 14.1  (a row of 1023, pieces of 1 to 255, 8 heads: 15.0 16.0
-//                                                                                      15.8 ->  9.9 11.0 10.6)
-//   two query heads and more to a KV head: dK/dV walks all of them.  2 x 16 (4) heads x 777 53.8 -> 26.0, 1 x 16 (4) x 2048 121 -> 49
-// Without a mask a block's work is twice that of a causal one: head_dim 64 768 blocks 6 x 2048 32.7 36.4 33.5 -> 22.8 26.2 29.9, but 1024
-// blocks 8 x 2048 32.5 37.4 34.8 -> 30.8 34.7 43.5; head_dim 128 256 blocks 4 x 1024 22.9 38.4 32.2 -> 13.5 15.6 15.6.
+// And the grid has to be small, for a block reads the other side for its 16 or 32 rows only.  us there -> here with one block of 16 rows to a
+// wavefront / with two, forward, dQ, dK/dV (causal; blocks: of 16 rows):
+//   head_dim 64    512 blocks  8 heads x 1023      22.7 -> 12.2 / 13.4   23.2 -> 12.5 / 14.3   21.5 -> 12.9 / 14.4
+//                  768         12 x 1024           22.3 -> 13.4 / 14.5   23.5 -> 14.4 / 17.3   21.2 -> 15.4 / 17.6
+//                  896         7 x 4 x 512         14.5 -> 12.1 / 12.1   16.1 -> 13.5 / 12.3   14.3 -> 14.7 / 12.8
+//                 1024         8 x 2048            37.4 -> 23.6 / 21.1   39.1 -> 21.5 / 20.4   37.4 -> 28.9 / 23.3
+//                 1176         3 x 8 x 777         18.5 -> 15.3 / 14.5   20.1 -> 17.5 / 16.3   20.5 -> 18.8 / 18.8
+//                 2048         4 x 8 x 1024        22.5 -> 22.0 / 20.5   24.0 -> 21.1 / 20.2   25.4 -> 28.3 / 23.1
+//                 2048         8 x 4096            67.4 -> 65.5 / 53.0   69.9 -> 60.2 / 47.4   76.7 -> 89.0 / 61.0
+//                 2560         10 x 8 x 512        15.8 -> 17.2 / 17.4   17.7 -> 20.5 / 19.2   18.5 -> 23.7 / 23.2
+//                 3072         3 x 8 x 2048        38.5 -> 46.6 / 36.5   41.1 -> 54.0 / 40.1   47.0 -> 76.3 / 48.5
+//                 4096         4 x 8 x 2048        39.7 -> 57.2 / 52.2   43.8 -> 65.7 / 47.6   53.3 -> 75.1 / 61.5
+//   head_dim 128   512         8 x 1023            27.4 -> 15.6 / 18.5   40.7 -> 17.1 / 21.2   35.7 -> 18.4
+//                 1024         2 x 8 x 1024        28.0 -> 21.9 / 20.5   40.7 -> 24.1 / 22.7   36.2 -> 27.1
+//                 1536         3 x 8 x 1024        28.4 -> 32.2 / 30.8   41.4 -> 35.8 / 34.9   36.9 -> 39.5
+//                 2048         2 x 8 x 2048        48.1 -> 58.5 / 45.7   71.7 -> 64.3 / 49.1   64.0 -> 80.1
+//                 3072         3 x 8 x 2048        54.8 -> 81.2 / 60.7   75.8 -> 93.4 / 69.4   68.8 ->  142
+// Without a mask a block's work is twice that of a causal one:
+//   head_dim 64    384         6 x 1024            20.4 -> 14.3 / 12.5   23.4 -> 14.9 / 12.8   20.2 -> 18.4 / 13.7
+//                 1024         2 x 8 x 1024        20.0 -> 18.7 / 16.9   23.0 -> 19.1 / 17.4   20.5 -> 23.7 / 20.2
+//                 1536         2 x 6 x 2048        35.8 -> 41.4 / 33.1   39.7 -> 44.4 / 33.9   46.9 -> 54.9 / 42.7
+//                 1536         6 x 8 x 512         14.1 -> 16.6 / 15.7   15.7 -> 17.9 / 16.9   17.6 -> 20.1 / 19.7
+//   head_dim 128   512         8 x 1024            25.3 -> 20.3 / 18.1   39.9 -> 21.7 / 20.5   34.6 -> 24.8
+//                 1024         8 x 2048            44.6 -> 50.7 / 38.9   69.9 -> 56.6 / 42.9   63.1 -> 68.0
+//                 1536         6 x 4096            84.9 ->  138 / 98.9    132 ->  153 /  107    122 ->  186
+// So two blocks from 832 (384 without a mask) on, and long walks, where a 32-row workgroup's chain is longest, up to larger grids.  Several
+// query heads to a KV head lengthen the walk of dK/dV: 2 x 16 (4) heads x 1500 96.1 -> 48.7 / 38.7, 16 (4) x 2048 123 -> 47.3 / 45.9.
+// (dK/dV of two blocks at head_dim 128 has no registers for its accumulators.)
 //
-// The lines are one number of blocks for every length of the walk, up to which no measured call is behind.  They are not the
-// break-even, which moves up with the length: of the calls above that are past their line, and so left to the 32-row kernels, these
-// would be ahead here: 1536 causal blocks, forward and dQ of 3 x 8 heads x 1024 (11 and 9 %) and of 12 x 2048 (26 and 18 %), dK/dV of
-// the latter (5 %); 1024 unmasked blocks, forward and dQ of 8 x 2048 (5 and 7 %).  The rule has no term for the length.
-bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride) {
+// Documents stay with one block and smaller grids: what a row sees is not known here.  head_dim 64, 2 x 8 x 1023, pieces of 1 to 255, 16.8 -> 13.2
+// / 14.0, 17.5 -> 14.5 / 14.7, 18.5 -> 16.1 / 15.6; 4 x 4 x 2000 in pieces of about 100 15.6 -> 16.9 / 20.1, of 500 (2 x 8) 33.9 -> 28.3 / 25.1.
+constexpr int kLongWalk = 1408;
+struct Lines {
+  int blocks, blocks_of_long_walks;  // up to which a call is served
+};
+constexpr Lines kLines[2][2][3] = {  // head_dim 128, causal, pass (forward, dQ, dK/dV)
+    {{{1024, 1536}, {1024, 1536}, {1024, 1536}}, {{2048, 3072}, {2048, 3072}, {2048, 2560}}},
+    {{{512, 1024}, {1024, 1536}, {512, 512}}, {{1024, 2048}, {2048, 3072}, {1024, 1024}}}};
+
+static bool half_walked(const AttnParams& p, int mode) { return mode == MLTS_MASK_CAUSAL && p.Sk <= p.Sq + p.Sq / 2; }
+static int64_t row_blocks(AttnPass pass, const AttnParams& p) {
   const bool keys = pass == ATTN_BWD_DKV;
-  if ((keys ? p.Sq : p.Sk) < 512) return false;
-  const int64_t blocks = static_cast<int64_t>(((keys ? p.Sk : p.Sq) + 15) / 16) * p.B * (keys ? p.Hkv : p.Hq);
-  const bool doc = mode == MLTS_MASK_DOC, half = doc || (mode == MLTS_MASK_CAUSAL && p.Sk <= p.Sq + p.Sq / 2);
-  if (blocks > (D == 64 ? (!half ? 768 : keys || doc ? 1024 : 1280) : (half ? 768 : 384))) return false;
+  return static_cast<int64_t>(((keys ? p.Sk : p.Sq) + 15) / 16) * p.B * (keys ? p.Hkv : p.Hq);
+}
+
+// Two blocks of 16 rows to a wavefront.  (Of half of the blocks whose walk is that long, eight splits each still fill the chip.)
+static bool two_blocks(AttnPass pass, const AttnParams& p, int mode) {
+  const int64_t blocks = row_blocks(pass, p), walk = pass == ATTN_BWD_DKV ? static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) : p.Sk;
+  return blocks >= (half_walked(p, mode) ? 832 : 384) || (blocks >= 512 && walk >= 4096);
+}
+
+bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride) {
+  const int walk = pass == ATTN_BWD_DKV ? p.Sq : p.Sk, which = pass == ATTN_FWD ? 0 : pass == ATTN_BWD_DQ ? 1 : 2;
+  if (walk < 512) return false;
+  const Lines& line = kLines[D == 128][half_walked(p, mode)][which];
+  const int limit = mode == MLTS_MASK_DOC ? (D == 64 ? 1024 : 768) : walk >= kLongWalk ? line.blocks_of_long_walks : line.blocks;
+  if (row_blocks(pass, p) > limit) return false;
   return near(p.Sq, p.qs) && near(p.Sk, p.ks) && near(p.Sk, p.vs) && near(p.Sq, p.os) && (!dout_stride || near(p.Sq, dout_stride));
 }
 
 int mlts_attn_small_fwd(AttnParams p, int D, int mode, hipStream_t st) {
   set_causal_off(p, mode);
-  if (mode == MLTS_MASK_DOC) return D == 64 ? fwd<64, true>(p, st) : fwd<128, true>(p, st);
-  return D == 64 ? fwd<64, false>(p, st) : fwd<128, false>(p, st);
+  if (mode == MLTS_MASK_DOC) return D == 64 ? fwd<64, true, 1>(p, st) : fwd<128, true, 1>(p, st);
+  const bool two = two_blocks(ATTN_FWD, p, mode);
+  if (D == 64) return two ? fwd<64, false, 2>(p, st) : fwd<64, false, 1>(p, st);
+  return two ? fwd<128, false, 2>(p, st) : fwd<128, false, 1>(p, st);
 }
 
 // bp.delta_out and bp.lse2_out receive the row statistics
 int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
-  if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dq<64, true>(bp, st) : bwd_dq<128, true>(bp, st);
-  return D == 64 ? bwd_dq<64, false>(bp, st) : bwd_dq<128, false>(bp, st);
+  if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dq<64, true, 1>(bp, st) : bwd_dq<128, true, 1>(bp, st);
+  const bool two = two_blocks(ATTN_BWD_DQ, bp.a, mode);
+  if (D == 64) return two ? bwd_dq<64, false, 2>(bp, st) : bwd_dq<64, false, 1>(bp, st);
+  return two ? bwd_dq<128, false, 2>(bp, st) : bwd_dq<128, false, 1>(bp, st);
 }
 
 // reads bp.delta
 int mlts_attn_small_bwd_dkv(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
-  if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dkv<64, true>(bp, st) : bwd_dkv<128, true>(bp, st);
-  return D == 64 ? bwd_dkv<64, false>(bp, st) : bwd_dkv<128, false>(bp, st);
+  if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dkv<64, true, 1>(bp, st) : bwd_dkv<128, true, 1>(bp, st);
+  if (D == 64) return two_blocks(ATTN_BWD_DKV, bp.a, mode) ? bwd_dkv<64, false, 2>(bp, st) : bwd_dkv<64, false, 1>(bp, st);
+  return bwd_dkv<128, false, 1>(bp, st);
 }
