@@ -22,6 +22,11 @@
 // 8 x 4 x 256: 15.5 18.8 19.4 / 9.6 13.4 14.6; 1 x 4 x 100: 8.8 10.5 10.2 / 6.0 7.2 8.3; 8 x 8 x 1024: 120 165 216 / 114 132 222;
 // 4 x 8 x 1024 unmasked: 132 175 220 / 92 120 192; 2 x 8 x 700, head_dim 96: 48 54 61 / 31 47 54; 4 x 8 x 500 x 1000, head_dim 128:
 // 191 352 277 / 81 115 165; packed, 1 x 8 (4) x 2048: 78 83 165 / 52 71 106.
+//
+// Two blocks of 16 rows to a wavefront in the backward kernels (head dims up to 64) share what is fetched and its way through LDS, for longer
+// and fewer chains (us, one / two; blocks of 16 own rows; head_dim 64, causal).  dQ: 8 x 8 heads x 1024, 4096 blocks, 161 / 122, 4 x 8 x 1024, 2048
+// blocks, 70 / 69, unmasked 126 / 116, 2 x 8 x 1024 42 / 43.  dK/dV, which fetches most for a row: 4096 blocks 207 / 174, 2048 119 / 93, 1024 63 / 53,
+// 704 (4 x 4 x 700) 40 / 36.5, 912 of short walks (6 x 8 x 300) 27.6 / 26, but 8 x 8 x 256 23.4 / 24.1 and 512 blocks (8 x 1024) 36 / 49.
 #pragma once
 #include "attn_rows.hpp"
 

@@ -150,10 +150,10 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
   join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1);
 }
 
-// dK, dV of 16 key rows of one KV head, summed over the query heads of its group.
-template <int DP, bool DOC, int LAYOUT>
+// dK, dV of R * 16 key rows of one KV head, summed over the query heads of its group.
+template <int DP, int R, bool DOC, int LAYOUT>
 __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(const AttnBwdParams bp, const RowArgs a) {
-  constexpr int FRAGS = DP / 16, NC = DP / 16;
+  constexpr int FRAGS = DP / 16, NC = DP / 16, ROWS = 16 * R;
   const AttnParams& p = bp.a;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const Place at(a);
@@ -162,36 +162,48 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
   // with a causal mask the first blocks are the long ones
   int bh, hkv;
   const int kt = a.rank(a.batch_heads.over(at.block, &bh)), b = a.heads.over(bh, &hkv), group = static_cast<int>(a.group.d);
-  const int kb0 = kt * 16, krow = kb0 + l16;
-  const int64_t ksafe = min(krow, p.Sk - 1);
-  const float* K = static_cast<const float*>(p.k) + b * p.ks[0] + hkv * p.ks[1] + ksafe * p.ks[2];
-  const float* V = static_cast<const float*>(p.v) + b * p.vs[0] + hkv * p.vs[1] + ksafe * p.vs[2];
-  f32x4 kf[FRAGS], vf[FRAGS];
+  const int kb0 = kt * ROWS;
+  f32x4 kf[R][FRAGS], vf[R][FRAGS];
+  int qlim[R], kpos[R], kseq[R];  // qlim: first query that sees this lane's key
 #pragma unroll
-  for (int j = 0; j < FRAGS; ++j) {
-    const int d = 16 * j + 4 * g;
-    kf[j] = inside<LAYOUT>(load_dot<LAYOUT>(K, d, a.D), d, a.D);
-    vf[j] = inside<LAYOUT>(load_dot<LAYOUT>(V, d, a.D), d, a.D);
+  for (int r = 0; r < R; ++r) {
+    const int krow = kb0 + 16 * r + l16;
+    const int64_t ksafe = min(krow, p.Sk - 1);
+    const float* K = static_cast<const float*>(p.k) + b * p.ks[0] + hkv * p.ks[1] + ksafe * p.ks[2];
+    const float* V = static_cast<const float*>(p.v) + b * p.vs[0] + hkv * p.vs[1] + ksafe * p.vs[2];
+#pragma unroll
+    for (int j = 0; j < FRAGS; ++j) {
+      const int d = 16 * j + 4 * g;
+      kf[r][j] = inside<LAYOUT>(load_dot<LAYOUT>(K, d, a.D), d, a.D);
+      vf[r][j] = inside<LAYOUT>(load_dot<LAYOUT>(V, d, a.D), d, a.D);
+    }
+    qlim[r] = krow < p.Sk ? krow - p.causal_off : 0x7fffffff;
+    kpos[r] = 0, kseq[r] = -2;
   }
-  const int qlim = krow < p.Sk ? krow - p.causal_off : 0x7fffffff;  // first query that sees this lane's key
-  const int all_qmin = min(kb0 + 15, p.Sk - 1) - p.causal_off;      // from here on every key that exists is seen
-  const bool ragged = kb0 + 16 > p.Sk;
+  const int all_qmin = min(kb0 + ROWS - 1, p.Sk - 1) - p.causal_off;  // from here on every key that exists is seen
+  const bool ragged = kb0 + ROWS > p.Sk;
   Units<DOC, false> units;
   units.split = split, units.splits = splits, units.lane = lane, units.end = p.Sq;
-  int kpos = 0, kseq = -2, qstart = 0;
+  int qstart = 0;
   if (DOC) {
     const int32_t *kp = p.k_pos + static_cast<int64_t>(b) * p.Sk, *ks = p.k_seq + static_cast<int64_t>(b) * p.Sk;
     units.pos = p.q_pos + static_cast<int64_t>(b) * p.Sq;
     units.seq = p.q_seq + static_cast<int64_t>(b) * p.Sq;
-    if (krow < p.Sk) kpos = kp[krow], kseq = ks[krow];
-    units.own = id_range(kp, ks, kb0, 16, p.Sk, lane);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int krow = kb0 + 16 * r + l16;
+      if (krow < p.Sk) kpos[r] = kp[krow], kseq[r] = ks[krow];
+    }
+    units.own = id_range(kp, ks, kb0, ROWS, p.Sk, lane);
   } else {
     qstart = max(0, kb0 - p.causal_off) / 16 * 16;
   }
 
-  f32x4 dkv[2][NC];
+  f32x4 dkv[2 * R][NC];  // dK of each block, dV of each
 #pragma unroll
-  for (int db = 0; db < NC; ++db) dkv[0][db] = dkv[1][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int n = 0; n < 2 * R; ++n)
+#pragma unroll
+    for (int db = 0; db < NC; ++db) dkv[n][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 qf[FRAGS], dof[FRAGS];
   float *turn_q = lds + at.wave * 2 * Turn<DP>::FLOATS, *turn_do = turn_q + Turn<DP>::FLOATS;
   float lse[4], delta[4];
@@ -224,17 +236,21 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
   while (hg < group) {
     int hn = hg, qn = units.next(q0);
     skip(hn, qn);
-    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, dp = s;
+    f32x4 s[R], dp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = dp[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < FRAGS; ++j) {
       const f32x4 q = inside<LAYOUT>(qf[j], 16 * j + 4 * g, a.D), o = inside<LAYOUT>(dof[j], 16 * j + 4 * g, a.D);
       Turn<DP>::put(turn_q, j, qf[j], l16, g);
       Turn<DP>::put(turn_do, j, dof[j], l16, g);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        s = mfma4(q[c], kf[j][c], s);
-        dp = mfma4(o[c], vf[j][c], dp);
-      }
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          s[r] = mfma4(q[c], kf[r][j][c], s[r]);
+          dp[r] = mfma4(o[c], vf[r][j][c], dp[r]);
+        }
     }
     float lse_now[4], delta_now[4];
     int qp_now[4], qs_now[4];
@@ -252,28 +268,46 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     __builtin_amdgcn_sched_barrier(0);
     const bool masked = !DOC && (q0 < all_qmin || ragged);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float pv = exponential(s[i] * p.scale - lse_now[i]);
-      if (DOC) {
-        if (!(kpos <= qp_now[i] && kseq == qs_now[i] && qs_now[i] >= 0)) pv = 0.f;
-      } else if (masked && q0 + 4 * g + i < qlim) {
-        pv = 0.f;
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float pv = exponential(s[r][i] * p.scale - lse_now[i]);
+        if (DOC) {
+          if (!(kpos[r] <= qp_now[i] && kseq[r] == qs_now[i] && qs_now[i] >= 0)) pv = 0.f;
+        } else if (masked && q0 + 4 * g + i < qlim[r]) {
+          pv = 0.f;
+        }
+        s[r][i] = pv;
+        dp[r][i] = pv * (dp[r][i] - delta_now[i]);
       }
-      s[i] = pv;
-      dp[i] = pv * (dp[i] - delta_now[i]);
-    }
     Columns<NC> rows[4];
     Turn<DP>::get(rows, turn_do, l16, g);
-    accumulate(dkv[1], rows, s);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int db = 0; db < NC; ++db)
+#pragma unroll
+        for (int r = 0; r < R; ++r) dkv[R + r][db] = mfma4(rows[i].v[db], s[r][i], dkv[R + r][db]);
     Turn<DP>::get(rows, turn_q, l16, g);
-    accumulate(dkv[0], rows, dp);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int db = 0; db < NC; ++db)
+#pragma unroll
+        for (int r = 0; r < R; ++r) dkv[r][db] = mfma4(rows[i].v[db], dp[r][i], dkv[r][db]);
     hg = hn, q0 = qn;
   }
-  const int64_t own = krow;
-  float* const row[2] = {there && krow < p.Sk ? static_cast<float*>(bp.dk) + b * bp.dks[0] + hkv * bp.dks[1] + own * bp.dks[2] : nullptr,
-                         there && krow < p.Sk ? static_cast<float*>(bp.dv) + b * bp.dvs[0] + hkv * bp.dvs[1] + own * bp.dvs[2] : nullptr};
-  const float scale[2] = {p.scale, 1.f};
-  join_and_store(dkv, lds + slot * splits * 2 * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0);
+  float* row[2 * R];
+  float scale[2 * R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t krow = kb0 + 16 * r + l16;
+    const bool mine = there && krow < p.Sk;
+    row[r] = mine ? static_cast<float*>(bp.dk) + b * bp.dks[0] + hkv * bp.dks[1] + krow * bp.dks[2] : nullptr;
+    row[R + r] = mine ? static_cast<float*>(bp.dv) + b * bp.dvs[0] + hkv * bp.dvs[1] + krow * bp.dvs[2] : nullptr;
+    scale[r] = p.scale, scale[R + r] = 1.f;
+  }
+  join_and_store(dkv, lds + slot * splits * 2 * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0);
 }
 
 template <int DP, int R, bool DOC, int LAYOUT>
@@ -288,23 +322,29 @@ int bwd_dq(AttnBwdParams bp, int D, hipStream_t st) {
                                                                                     "mlts_attn_bwd");
 }
 
-template <int DP, bool DOC, int LAYOUT>
-int bwd(AttnBwdParams bp, int D, hipStream_t st) {
-  AttnParams& p = bp.a;
-  if (p.Sq > 0) {
-    int rc;
-    // 32 rows a wavefront where they still make two wavefronts for every SIMD: half the loads and half the turns through LDS
-    if (DP <= 64 && static_cast<int64_t>((p.Sq + 31) / 32) * p.B * p.Hq >= kResident / 2) rc = bwd_dq<DP, DP <= 64 ? 2 : 1, DOC, LAYOUT>(bp, D, st);
-    else rc = bwd_dq<DP, 1, DOC, LAYOUT>(bp, D, st);
-    if (rc != MLTS_OK) return rc;
-  }
-  if (p.Sk == 0) return MLTS_OK;
-  const int64_t blocks = static_cast<int64_t>((p.Sk + 15) / 16) * p.B * p.Hkv;
-  const RowArgs a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dks, bp.dk) && rows_vec(bp.dvs, bp.dv), p.Hkv, (p.Sk + 15) / 16);
+template <int DP, int R, bool DOC, int LAYOUT>
+int bwd_dkv(const AttnBwdParams& bp, int D, hipStream_t st) {
+  const AttnParams& p = bp.a;
+  const int tiles = (p.Sk + 16 * R - 1) / (16 * R);
+  const int64_t blocks = static_cast<int64_t>(tiles) * p.B * p.Hkv;
+  const RowArgs a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dks, bp.dk) && rows_vec(bp.dvs, bp.dv), p.Hkv, tiles);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
   const int splits = splits_for(blocks, static_cast<int64_t>((p.Sq + 15) / 16) * (p.Hq / p.Hkv), max_splits(DP, LAYOUT));
-  return launch_splits<attn_f32_bwd_dkv<DP, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, 2 * DP * 64, 2 * Turn<DP>::FLOATS * 4, st, bp, a,
-                                                                                  "mlts_attn_bwd");
+  return launch_splits<attn_f32_bwd_dkv<DP, R, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, 2 * R * DP * 64, 2 * Turn<DP>::FLOATS * 4, st, bp, a,
+                                                                                     "mlts_attn_bwd");
+}
+
+template <int DP, bool DOC, int LAYOUT>
+int bwd(AttnBwdParams bp, int D, hipStream_t st) {
+  constexpr int TWO = DP <= 64 ? 2 : 1;  // blocks of 16 rows to a wavefront: attn_f32.hpp has both sides of the lines
+  const AttnParams& p = bp.a;
+  if (p.Sq > 0) {
+    const bool two = static_cast<int64_t>((p.Sq + 31) / 32) * p.B * p.Hq >= kResident / 2;
+    if (int rc = two ? bwd_dq<DP, TWO, DOC, LAYOUT>(bp, D, st) : bwd_dq<DP, 1, DOC, LAYOUT>(bp, D, st); rc != MLTS_OK) return rc;
+  }
+  if (p.Sk == 0) return MLTS_OK;
+  const bool two = static_cast<int64_t>((p.Sk + 31) / 32) * p.B * p.Hkv >= 352 && static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) > 256;
+  return two ? bwd_dkv<DP, TWO, DOC, LAYOUT>(bp, D, st) : bwd_dkv<DP, 1, DOC, LAYOUT>(bp, D, st);
 }
 
 }  // namespace

@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
   }
   join_and_store(o, reinterpret_cast<f32x4*>(lds_raw), at, [&](int r, int db, f32x4 v) {
     const int qrow = q0 + 16 * r + l16;
-    if (at.there && qrow < p.Sq) store4(p.o, row + qrow * p.os[2] + 16 * db, v * (R == 1 || r == 0 ? scale[0] : scale[R - 1]), 0);
+    if (at.there && qrow < p.Sq) store4(p.o, row + qrow * p.os[2] + 16 * db, v * scale[r], 0);
   });
 }
 
