@@ -12,6 +12,7 @@ int mlts_attn_bwd_dq_bf16_tr(const AttnBwdParams& bp, int D, int mode, hipStream
 int mlts_attn_tile16_fwd(AttnParams p, int D, int mode, hipStream_t st);                                   // attn_tile16.hip
 int mlts_attn_tile16_bwd(AttnBwdParams bp, int D, int mode, hipStream_t st);                               // attn_tile16.hip
 bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride);  // attn_small.hip
+bool mlts_attn_small_serves_parts(const AttnParams& p, int D, int mode, const AttnBwdParams* bp);                 // attn_small.hip
 int mlts_attn_small_fwd(AttnParams p, int D, int mode, hipStream_t st);                                    // attn_small.hip
 int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st);                             // attn_small.hip
 int mlts_attn_small_bwd_dkv(AttnBwdParams bp, int D, int mode, hipStream_t st);                            // attn_small.hip
@@ -241,6 +242,10 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
   if (!uses_mfma(s)) {
     bp.delta_out = delta;
     if (s->dtype == MLTS_F32) return mlts_attn_f32_bwd(bp, s->D, s->mask_mode, st);
+    if (mlts_attn_small_serves_parts(bp.a, s->D, s->mask_mode, &bp)) {
+      if (int rc = mlts_attn_small_bwd_dq(bp, s->D, s->mask_mode, st); rc != MLTS_OK) return rc;
+      return mlts_attn_small_bwd_dkv(bp, s->D, s->mask_mode, st);
+    }
     return mlts_attn_tile16_bwd(bp, s->D, s->mask_mode, st);
   }
   // the dQ kernels form delta themselves from 16-byte chunks of the O rows
@@ -635,6 +640,7 @@ extern "C" int mlts_attn_fwd(const mlts_attn_shape* s, const void* q, const void
     return mlts_attn_fwd_bf16_dma(p, s->D, s->mask_mode, st);
   }
   if (s->dtype == MLTS_F32) return mlts_attn_f32_fwd(p, s->D, s->mask_mode, st);
+  if (mlts_attn_small_serves_parts(p, s->D, s->mask_mode, nullptr)) return mlts_attn_small_fwd(p, s->D, s->mask_mode, st);
   return mlts_attn_tile16_fwd(p, s->D, s->mask_mode, st);
 }
 

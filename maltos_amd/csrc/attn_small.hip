@@ -10,7 +10,8 @@
 // the splits' sums meet at the end.  Scores are computed transposed, as in the fp32 kernels, so that a lane holds the probabilities of one
 // own row and the next product takes them, rounded to bf16 once, from the registers they are in.
 //
-// Documents: the plan's tile classes and visibility bits, as in the 32-row kernels.
+// Documents: the plan's tile classes and visibility bits, as in the 32-row kernels.  At head_dim 32 and 96, without documents, all grids
+// (mlts_attn_small_serves_parts()).
 #include "attn_bf16.hpp"
 
 namespace {
@@ -23,15 +24,18 @@ __device__ __forceinline__ const bf16_t* row_of(const bf16_t* base, int row, int
   return reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(base) + offset);
 }
 
-// A unit of one operand: fetched, put to LDS, read as fragments.
+// A unit of one operand: fetched, put to LDS, read as fragments.  A wavefront's 64 chunks of 16 bytes are whole rows, or those of three fetches are.
 template <int D>
 struct Unit : Rows<D> {
   static constexpr int CHUNKS = D / 8, N = kUnit * CHUNKS / 64, BYTES = kUnit * Rows<D>::BYTES;
+  static constexpr int PERIOD = 64 % CHUNKS == 0 ? 1 : 3, ROWS = 64 * PERIOD / CHUNKS;  // of that many fetches
+  static_assert(64 * PERIOD % CHUNKS == 0 && N % PERIOD == 0, "whole rows");
   bf16x8 raw[N];
-  uint32_t stride, offset;  // bytes: between rows, of this lane's chunk in the first rows
+  uint32_t stride, offset[PERIOD];  // bytes: between rows, of this lane's chunks in the first rows
   __device__ __forceinline__ void init(int64_t elements, int lane) {
     stride = static_cast<uint32_t>(elements) * 2u;
-    offset = static_cast<uint32_t>(lane / CHUNKS) * stride + 16u * static_cast<uint32_t>(lane % CHUNKS);
+#pragma unroll
+    for (int i = 0; i < PERIOD; ++i) offset[i] = static_cast<uint32_t>((64 * i + lane) / CHUNKS) * stride + 16u * static_cast<uint32_t>((64 * i + lane) % CHUNKS);
   }
   // rows row0 ..; rows past the last one are zeros, from the bounds check of the descriptor (near(): no offset wraps).  One addition a chunk:
   // the row's part of the address is the same in all lanes.
@@ -40,13 +44,59 @@ struct Unit : Rows<D> {
     const uint32_t at = static_cast<uint32_t>(min(row0, last)) * stride;
 #pragma unroll
     for (int i = 0; i < N; ++i)
-      raw[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset + (at + static_cast<uint32_t>(64 / CHUNKS * i) * stride), 0, 0));
+      raw[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset[i % PERIOD] + (at + static_cast<uint32_t>(i / PERIOD * ROWS) * stride), 0, 0));
   }
   __device__ __forceinline__ void put(unsigned char* lds, int lane) const {
 #pragma unroll
-    for (int i = 0; i < N; ++i) *reinterpret_cast<bf16x8*>(lds + Rows<D>::at((64 / CHUNKS) * i + lane / CHUNKS, lane % CHUNKS)) = raw[i];
+    for (int i = 0; i < N; ++i) {
+      const int chunk = 64 * (i % PERIOD) + lane;
+      *reinterpret_cast<bf16x8*>(lds + Rows<D>::at(i / PERIOD * ROWS + chunk / CHUNKS, chunk % CHUNKS)) = raw[i];
+    }
   }
 };
+
+// What a probability or dS goes into its second product as: at head_dim 64 and 128 rounded to bf16, as in the 32-row kernels; else the sum of three bf16
+// values of 8 bits each, which is all of an fp32 number, as in attn_tile16.hip.
+template <int D>
+constexpr int kParts = D == 64 || D == 128 ? 1 : 3;
+template <int PARTS>
+__device__ __forceinline__ void split(bf16x8 (&part)[PARTS], const f32x4 (&x)[2]) {
+  if constexpr (PARTS == 1) {
+    part[0] = pack(x);
+  } else {
+    f32x4 rest[2] = {x[0], x[1]};
+#pragma unroll
+    for (int n = 0; n < PARTS; ++n) {
+      part[n] = pack(rest);
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rest[b][i] -= static_cast<float>(part[n][4 * b + i]);
+    }
+  }
+}
+// acc[r][db] += columns x own rows; column(db): of the walked rows
+template <int R, int NC, int PARTS, typename F>
+__device__ __forceinline__ void add_products(f32x4 (&acc)[R][NC], const bf16x8 (&x)[R][PARTS], F column) {
+  if constexpr (PARTS == 1) {
+#pragma unroll
+    for (int db = 0; db < NC; ++db) {
+      const bf16x8 c = column(db);
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r][db] = mfma32(c, x[r][0], acc[r][db]);
+    }
+  } else {
+    bf16x8 c[NC];
+#pragma unroll
+    for (int db = 0; db < NC; ++db) c[db] = column(db);
+#pragma unroll
+    for (int n = 0; n < PARTS; ++n)
+#pragma unroll
+      for (int db = 0; db < NC; ++db)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r][db] = mfma32(c[db], x[r][n], acc[r][db]);
+  }
+}
 
 // The units a split works on, in order: every `splits`-th.  Documents: those of them whose tile of 64 rows the plan's statistics do not
 // rule out for the own rows' group of 64, 32 tiles at a time, a lane for each unit.
@@ -222,7 +272,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
     keys.put(lk, lane);  // the next unit's, which have had one unit's time to arrive
     fetch_keys(kn2);
     __builtin_amdgcn_sched_barrier(0);
-    bf16x8 pr[R];
+    bf16x8 pr[R][kParts<D>];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       float mx = -INFINITY;
@@ -247,14 +297,9 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
           s[r][u][i] = exponential(s[r][u][i] * p.scale - m_use);
           l[r] += s[r][u][i];
         }
-      pr[r] = pack(s[r]);
+      split(pr[r], s[r]);
     }
-#pragma unroll
-    for (int db = 0; db < NC; ++db) {
-      const bf16x8 column = U::columns(lv, db, l16, g);
-#pragma unroll
-      for (int r = 0; r < R; ++r) o[r][db] = mfma32(column, pr[r], o[r][db]);
-    }
+    add_products(o, pr, [&](int db) { return U::columns(lv, db, l16, g); });
     values.put(lv, lane);
     values.fetch(V, kn2, p.Sk - 1);
     k0 = kn, kn = kn2, word_now = word_next, masked_now = masked_next;
@@ -339,11 +384,11 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     lse[r] = qrow < p.Sq && lse[r] != -INFINITY ? lse[r] : INFINITY;  // rows that saw no key: every probability 0
     if (at.there && qrow < p.Sq && g == 0 && at.split == 0) {  // the statistics of the backward pass, for whichever dK/dV kernel comes next
       bp.delta_out[stat] = delta[r];
-      bp.lse2_out[stat] = lse[r] * 1.44269504088896340736f;
+      if (kParts<D> == 1) bp.lse2_out[stat] = lse[r] * 1.44269504088896340736f;
     }
     klim[r] = DOC || qrow < p.Sq ? min(p.Sk - 1, DOC ? p.Sk : qrow + p.causal_off) : -1;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) bp.lse2_out[static_cast<int64_t>(p.B) * p.Hq * p.Sq] = INFINITY;
+  if (kParts<D> == 1 && blockIdx.x == 0 && threadIdx.x == 0) bp.lse2_out[static_cast<int64_t>(p.B) * p.Hq * p.Sq] = INFINITY;
   Walk<DOC, true> walk;
   walk.split = at.split, walk.splits = at.splits, walk.lane = lane;
   const unsigned long long* bits = nullptr;
@@ -402,7 +447,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
       }
     }
     const bool edge = k0 + kUnit - 1 > all_klim;
-    bf16x8 ds[R];
+    bf16x8 ds[R][kParts<D>];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
@@ -428,7 +473,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) s[r][u][i] *= dp[r][u][i] - delta[r];
-      ds[r] = pack(s[r]);
+      split(ds[r], s[r]);
     }
     bf16x8 kc[NC];
 #pragma unroll
@@ -437,10 +482,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     put();  // the next unit's, which have had one unit's time to arrive
     fetch(kn2);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int db = 0; db < NC; ++db)
-#pragma unroll
-      for (int r = 0; r < R; ++r) dq[r][db] = mfma32(kc[db], ds[r], dq[r][db]);
+    add_products(dq, ds, [&](int db) { return kc[db]; });
     k0 = kn, kn = kn2;
   }
   const int64_t row = b * bp.dqs[0] + hq * bp.dqs[1] + 4 * g;
@@ -491,11 +533,11 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
     qstart = max(0, kb0 - p.causal_off) / kUnit * kUnit;
   }
 
-  f32x4 dkv[2 * R][NC];  // dK of each block, dV of each
+  f32x4 dk[R][NC], dv[R][NC];
 #pragma unroll
-  for (int n = 0; n < 2 * R; ++n)
+  for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int db = 0; db < NC; ++db) dkv[n][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < NC; ++db) dk[r][db] = dv[r][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   U queries, grads;
   queries.init(p.qs[2], lane), grads.init(bp.dos[2], lane);
   unsigned char* own = lds_raw + at.wave * (2 * U::BYTES + 256);
@@ -554,7 +596,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
       delta[u] = *reinterpret_cast<const f32x4*>(lstat + 32 + 16 * u + 4 * g);
     }
     const bool edge = !DOC && q0 < all_qmin;
-    bf16x8 pr[R], ds[R];
+    bf16x8 pr[R][kParts<D>], ds[R][kParts<D>];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
@@ -580,15 +622,10 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) dp[r][u][i] = s[r][u][i] * (dp[r][u][i] - delta[u][i]);
-      pr[r] = pack(s[r]), ds[r] = pack(dp[r]);
+      split(pr[r], s[r]), split(ds[r], dp[r]);
     }
+    add_products(dv, pr, [&](int db) { return U::columns(ld, db, l16, g); });
     bf16x8 col[NC];
-#pragma unroll
-    for (int db = 0; db < NC; ++db) col[db] = U::columns(ld, db, l16, g);
-#pragma unroll
-    for (int db = 0; db < NC; ++db)
-#pragma unroll
-      for (int r = 0; r < R; ++r) dkv[R + r][db] = mfma32(col[db], pr[r], dkv[R + r][db]);
 #pragma unroll
     for (int db = 0; db < NC; ++db) col[db] = U::columns(lq, db, l16, g);
     int hn2 = hn, qn2 = qn;
@@ -596,13 +633,15 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
     put();  // the next unit's, which have had one unit's time to arrive
     fetch(min(hn2, group - 1), qn2);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int db = 0; db < NC; ++db)
-#pragma unroll
-      for (int r = 0; r < R; ++r) dkv[r][db] = mfma32(col[db], ds[r], dkv[r][db]);
+    add_products(dk, ds, [&](int db) { return col[db]; });
     hg = hn, q0 = qn, hn = hn2, qn = qn2;
   }
   const int64_t dk_row = b * bp.dks[0] + hkv * bp.dks[1] + 4 * g, dv_row = b * bp.dvs[0] + hkv * bp.dvs[1] + 4 * g;
+  f32x4 dkv[2 * R][NC];
+#pragma unroll
+  for (int n = 0; n < 2 * R; ++n)
+#pragma unroll
+    for (int db = 0; db < NC; ++db) dkv[n][db] = n < R ? dk[n < R ? n : 0][db] : dv[n < R ? 0 : n - R][db];
   join_and_store(dkv, reinterpret_cast<f32x4*>(lds_raw), at, [&](int n, int db, f32x4 v) {
     const int krow = kb0 + 16 * (n < R ? n : n - R) + l16;
     if (at.there && krow < p.Sk)
@@ -676,7 +715,7 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 //   head_dim 128   512         8 x 1024            25.3 -> 20.3 / 18.1   39.9 -> 21.7 / 20.5   34.6 -> 24.8
 //                 1024         8 x 2048            44.6 -> 50.7 / 38.9   69.9 -> 56.6 / 42.9   63.1 -> 68.0
 //                 1536         6 x 4096            84.9 ->  138 / 98.9    132 ->  153 /  107    122 ->  186
-// So two blocks from 832 (384 without a mask) on, and long walks, where a 32-row workgroup's chain is longest, up to larger grids.  Several
+// So two blocks from 832 (384 without a mask) on, short walks apart (8 x 32 heads x 64, head_dim 32, forward 7.3 / 8.9), and long walks, where a 32-row workgroup's chain is longest, up to larger grids.  Several
 // query heads to a KV head lengthen the walk of dK/dV: 2 x 16 (4) heads x 1500 96.1 -> 48.7 / 38.7, 16 (4) x 2048 123 -> 47.3 / 45.9.
 // (dK/dV of two blocks at head_dim 128 has no registers for its accumulators.)
 //
@@ -699,7 +738,7 @@ static int64_t row_blocks(AttnPass pass, const AttnParams& p) {
 // Two blocks of 16 rows to a wavefront.  (Of half of the blocks whose walk is that long, eight splits each still fill the chip.)
 static bool two_blocks(AttnPass pass, const AttnParams& p, int mode) {
   const int64_t blocks = row_blocks(pass, p), walk = pass == ATTN_BWD_DKV ? static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) : p.Sk;
-  return blocks >= (half_walked(p, mode) ? 832 : 384) || (blocks >= 512 && walk >= 4096);
+  return walk >= 96 && (blocks >= (half_walked(p, mode) ? 832 : 384) || (blocks >= 512 && walk >= 4096));
 }
 
 bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride) {
@@ -711,10 +750,33 @@ bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode,
   return near(p.Sq, p.qs) && near(p.Sk, p.ks) && near(p.Sk, p.vs) && near(p.Sq, p.os) && (!dout_stride || near(p.Sq, dout_stride));
 }
 
+// Whole passes at head_dim 32 and 96 without documents; bp: of the backward pass.  attn_tile16.hip, which takes rows at any alignment, shares 64-row
+// tiles between four wavefronts, which wait for each other twice a tile and walk a row's whole length (us there -> here, forward, dQ, dK/dV, causal):
+//   head_dim 32   8 heads x 1024      20.1 -> 11.2   20.8 -> 11.1   26.3 -> 12.3     96   32.0 -> 17.5   31.5 -> 18.0   38.4 -> 18.5
+//                 4 x 8 x 1024        23.7 -> 21.0   24.8 -> 21.6   31.1 -> 26.7          37.8 -> 31.8   41.0 -> 36.4   62.7 -> 49.3
+//                 8 x 16 x 1024       55.9 -> 53.7   60.7 -> 53.0   85.7 -> 72.3          96.3 -> 86.8    105 -> 94.6    164 -> 154
+//                 8 x 32 x 64          8.2 -> 7.3     8.1 -> 7.6     7.9 -> 7.3           11.2 -> 9.5    11.3 -> 9.6    10.7 -> 10.1
+//                 8 x 32 (8) x 300    16.7 -> 17.6   19.8 -> 19.0   31.9 -> 25.0          31.9 -> 28.1   36.9 -> 33.6   48.8 -> 40.2
+//   unmasked      8 x 8 x 1024        55.1 -> 46.7   57.7 -> 45.2   82.0 -> 64.4          93.1 -> 72.3    101 -> 76.6    143 -> 131
+// Errors against 64 bits as there or up to a fifth smaller (dQ, dK, dV in fp32, 300 to 1024 rows).
+bool mlts_attn_small_serves_parts(const AttnParams& p, int D, int mode, const AttnBwdParams* bp) {
+  if ((D != 32 && D != 96) || mode == MLTS_MASK_DOC || p.Sq == 0 || p.Sk == 0) return false;
+  const auto rows = [](const void* t, const int64_t* stride, int es) {
+    return mlts_aligned16(t) && stride[0] * es % 16 == 0 && stride[1] * es % 16 == 0 && stride[2] * es % 16 == 0;
+  };
+  if (!rows(p.q, p.qs, 2) || !rows(p.k, p.ks, 2) || !rows(p.v, p.vs, 2) || !rows(p.o, p.os, 2)) return false;
+  if (bp && (!rows(bp->dout, bp->dos, 2) || !rows(bp->dq_acc, bp->dqs, bp->dq_f32 ? 4 : 2) || !rows(bp->dk, bp->dks, bp->accumulate_f32 ? 4 : 2) ||
+             !rows(bp->dv, bp->dvs, bp->accumulate_f32 ? 4 : 2) || !near(p.Sq, bp->dos)))
+    return false;
+  return near(p.Sq, p.qs) && near(p.Sk, p.ks) && near(p.Sk, p.vs) && near(p.Sq, p.os);
+}
+
 int mlts_attn_small_fwd(AttnParams p, int D, int mode, hipStream_t st) {
   set_causal_off(p, mode);
   if (mode == MLTS_MASK_DOC) return D == 64 ? fwd<64, true, 1>(p, st) : fwd<128, true, 1>(p, st);
   const bool two = two_blocks(ATTN_FWD, p, mode);
+  if (D == 32) return two ? fwd<32, false, 2>(p, st) : fwd<32, false, 1>(p, st);
+  if (D == 96) return two ? fwd<96, false, 2>(p, st) : fwd<96, false, 1>(p, st);
   if (D == 64) return two ? fwd<64, false, 2>(p, st) : fwd<64, false, 1>(p, st);
   return two ? fwd<128, false, 2>(p, st) : fwd<128, false, 1>(p, st);
 }
@@ -724,6 +786,8 @@ int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
   if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dq<64, true, 1>(bp, st) : bwd_dq<128, true, 1>(bp, st);
   const bool two = two_blocks(ATTN_BWD_DQ, bp.a, mode);
+  if (D == 32) return two ? bwd_dq<32, false, 2>(bp, st) : bwd_dq<32, false, 1>(bp, st);
+  if (D == 96) return two ? bwd_dq<96, false, 2>(bp, st) : bwd_dq<96, false, 1>(bp, st);
   if (D == 64) return two ? bwd_dq<64, false, 2>(bp, st) : bwd_dq<64, false, 1>(bp, st);
   return two ? bwd_dq<128, false, 2>(bp, st) : bwd_dq<128, false, 1>(bp, st);
 }
@@ -732,6 +796,8 @@ int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st) {
 int mlts_attn_small_bwd_dkv(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
   if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dkv<64, true, 1>(bp, st) : bwd_dkv<128, true, 1>(bp, st);
+  if (D == 32) return two_blocks(ATTN_BWD_DKV, bp.a, mode) ? bwd_dkv<32, false, 2>(bp, st) : bwd_dkv<32, false, 1>(bp, st);
+  if (D == 96) return bwd_dkv<96, false, 1>(bp, st);
   if (D == 64) return two_blocks(ATTN_BWD_DKV, bp.a, mode) ? bwd_dkv<64, false, 2>(bp, st) : bwd_dkv<64, false, 1>(bp, st);
   return bwd_dkv<128, false, 1>(bp, st);
 }

@@ -1,4 +1,5 @@
-// Attention on 16-row wavefront tiles: bf16 at head dims <= 192 that the 32-row kernels do not cover.
+// Attention on 16-row wavefront tiles: bf16 at head dims <= 192 that neither the 32-row kernels nor attn_small.hip cover (documents, rows at
+// any alignment, head dims other than 32, 64, 96 and 128).
 //
 // A wavefront owns 16 rows (queries in the forward and dQ kernels, keys in the dK/dV kernel) and walks the other side in
 // units of 32, staged in LDS 64 at a time.  Everything is computed transposed, S^T = K Q^T and O^T = V^T P^T (dK/dV: S = Q K^T,

@@ -423,6 +423,32 @@ def test_sixteen_row_kernels_at_tile_edges(dev, dtype, D, B, H, Hkv, Sq, Sk):
         run_case(dev, dtype, B, H, Hkv, Sq, Sk, D, mode, seed=Sq + D)
 
 
+# one and two blocks of 16 rows to a wavefront (832 causal blocks, 384 without a mask), a last one that is cut, walks that end inside a unit, rows that see nothing
+@pytest.mark.parametrize("mode", [ops.MASK_CAUSAL, ops.MASK_NONE])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk", [(1, 1, 1, 1, 1), (2, 4, 2, 33, 70), (1, 6, 3, 200, 95), (3, 8, 8, 300, 290), (5, 12, 4, 225, 337)])
+@pytest.mark.parametrize("D", [32, 96])
+def test_head_dims_between_the_tuned_ones(dev, D, B, Hq, Hkv, Sq, Sk, mode):
+    """Rows of whole 16-byte chunks against the oracle, and against the kernels that take rows at any alignment, in every form of a gradient."""
+    run_case(dev, torch.bfloat16, B, Hq, Hkv, Sq, Sk, D, mode, seed=Sq + D)
+    gen = torch.Generator().manual_seed(Sk + D)
+    q, k, v, do = (bshd(B, h, S, D, gen, torch.bfloat16).to(dev) for h, S in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk), (Hq, Sq)))
+    apart = lambda t: torch.nn.functional.pad(t, (0, 4))[..., :D]   # rows 8 bytes further apart
+    results = []
+    for tensors in ((q, k, v, do), tuple(apart(t) for t in (q, k, v, do))):
+        q1, k1, v1, do1 = tensors
+        o, lse = ops.attention_forward(q1, k1, v1, mask_mode=mode)
+        grads = [torch.full(t.shape, float("nan"), device=dev) for t in (q1,)] + [torch.full_like(t, float("nan")) for t in (k1, v1)]
+        ops.attention_backward_ring_block(do1, q1, k1, v1, o, lse, *grads, first=True, mask_mode=mode)
+        sums = [torch.ones(t.shape, device=dev) for t in (q1, k1, v1)]
+        ops.attention_backward_accumulate(do1, q1, k1, v1, o, lse, *sums, mask_mode=mode)
+        results.append((o, lse, *ops.attention_backward(do1, q1, k1, v1, o, lse, mask_mode=mode), *grads, *sums))
+    for i, (got, want) in enumerate(zip(*results)):
+        if i == 1:
+            torch.testing.assert_close(got, want, rtol=0, atol=1e-5)
+        else:
+            check(got, want, torch.bfloat16, f"result {i}")
+
+
 # 16-row blocks: 195, 1365 and 2145, i.e. eight, two and one wavefronts to a block, with a workgroup at the end that is partly empty
 @pytest.mark.parametrize("B,H", [(1, 3), (3, 7), (11, 3)])
 @pytest.mark.parametrize("D", [64, 60])
