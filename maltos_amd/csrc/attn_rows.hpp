@@ -83,9 +83,9 @@ constexpr int64_t kResident = 2048;
 // head_dim 64, causal): 2 x 8 heads x 777 (784 blocks, 25 units on the mean) forward 36 31 24 27, dQ 49 42 36 41; with four KV heads dK/dV
 // (392 blocks, 49 units) 137 81 54 45; 8 x 4 x 256 (512 blocks, 8 units) forward 14.3 10.7 9.5 11.8, dQ 18.6 13.7 13.6 18.3, dK/dV 26 17 15
 // 18; 4 x 8 x 1024 without a mask (2048 blocks) forward 87 - 97 99, dQ 127 - 148 151.
-inline int splits_for(int64_t blocks, int64_t units, int most) {
+inline int splits_for(int64_t blocks, int64_t units, int most, int64_t fill = kResident) {
   int s = 1;
-  while (s < most && ((blocks * s < kResident && units >= 8 * s) || (blocks * s < kResident / 2 && units >= 2 * s))) s *= 2;
+  while (s < most && ((blocks * s < fill && units >= 8 * s) || (blocks * s < kResident / 2 && units >= 2 * s))) s *= 2;
   return s;
 }
 

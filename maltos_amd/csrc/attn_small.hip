@@ -653,12 +653,20 @@ bool near(int64_t rows, const int64_t* stride) {  // offsets that row_of can for
   return rows < (1 << 24) && stride[2] < (1 << 23) && ((rows - 1 + kUnit) * stride[2] + 128) * 2 < (int64_t{1} << 32);
 }
 
+// Splits of two blocks: where they come out at just two wavefronts a SIMD, four of half the length are ahead if they all fit (forward at head_dim 64: 121
+// registers) or the walk is long (us, two / four: head_dim 64, 8 heads x 4096 forward 56 / 44, dQ 49 / 48, dK/dV 67 / 61, 16 (4) x 2048 forward 31 / 26,
+// but dQ 28 / 32, 4 x 8 x 1024 dQ 20 / 25; head_dim 128, 8 x 4096 forward 79 / 75).  From 2304 on they are not: 1504 blocks x 1500 forward 20.5 / 23.2.
+template <int R>
+int splits_of(int64_t blocks, int64_t units, bool all_fit) {
+  return splits_for(blocks, units, kMaxSplits, R == 2 && (all_fit || units >= 4096 / kUnit) ? 2304 : kResident);
+}
+
 template <int D, bool DOC, int R>
 int fwd(AttnParams p, hipStream_t st) {
   p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   MltsKernelTimer timer("attn_fwd", st);
-  return launch_splits<attn_small_fwd<D, DOC, R>, kMaxSplits>(blocks, splits_for(blocks, (p.Sk + kUnit - 1) / kUnit, kMaxSplits), R * D * 64, 2 * Unit<D>::BYTES, st, p,
+  return launch_splits<attn_small_fwd<D, DOC, R>, kMaxSplits>(blocks, splits_of<R>(blocks, (p.Sk + kUnit - 1) / kUnit, D == 64), R * D * 64, 2 * Unit<D>::BYTES, st, p,
                                                               RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_fwd");
 }
 
@@ -668,7 +676,7 @@ int bwd_dq(AttnBwdParams bp, hipStream_t st) {
   p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   MltsKernelTimer timer("attn_bwd_dq", st);
-  return launch_splits<attn_small_bwd_dq<D, DOC, R>, kMaxSplits>(blocks, splits_for(blocks, (p.Sk + kUnit - 1) / kUnit, kMaxSplits), R * D * 64, 2 * Unit<D>::BYTES, st, bp,
+  return launch_splits<attn_small_bwd_dq<D, DOC, R>, kMaxSplits>(blocks, splits_of<R>(blocks, (p.Sk + kUnit - 1) / kUnit, false), R * D * 64, 2 * Unit<D>::BYTES, st, bp,
                                                                  RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_bwd");
 }
 
@@ -678,7 +686,7 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
   const int tiles = (p.Sk + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(tiles) * p.B * p.Hkv, units = static_cast<int64_t>((p.Sq + kUnit - 1) / kUnit) * (p.Hq / p.Hkv);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
-  return launch_splits<attn_small_bwd_dkv<D, DOC, R>, kMaxSplits>(blocks, splits_for(blocks, units, kMaxSplits), 2 * R * D * 64, 2 * Unit<D>::BYTES + 256, st, bp,
+  return launch_splits<attn_small_bwd_dkv<D, DOC, R>, kMaxSplits>(blocks, splits_of<R>(blocks, units, false), 2 * R * D * 64, 2 * Unit<D>::BYTES + 256, st, bp,
                                                                   RowArgs(p, D, true, p.Hkv, tiles), "mlts_attn_bwd");
 }
 
@@ -698,7 +706,7 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 //                 1024         8 x 2048            37.4 -> 23.6 / 21.1   39.1 -> 21.5 / 20.4   37.4 -> 28.9 / 23.3
 //                 1176         3 x 8 x 777         18.5 -> 15.3 / 14.5   20.1 -> 17.5 / 16.3   20.5 -> 18.8 / 18.8
 //                 2048         4 x 8 x 1024        22.5 -> 22.0 / 20.5   24.0 -> 21.1 / 20.2   25.4 -> 28.3 / 23.1
-//                 2048         8 x 4096            67.4 -> 65.5 / 53.0   69.9 -> 60.2 / 47.4   76.7 -> 89.0 / 61.0
+//                 2048         8 x 4096            67.5 -> 65.5 / 44     69.9 -> 60.2 / 47.7   77.3 -> 89.0 / 61.5
 //                 2560         10 x 8 x 512        15.8 -> 17.2 / 17.4   17.7 -> 20.5 / 19.2   18.5 -> 23.7 / 23.2
 //                 3072         3 x 8 x 2048        38.5 -> 46.6 / 36.5   41.1 -> 54.0 / 40.1   47.0 -> 76.3 / 48.5
 //                 4096         4 x 8 x 2048        39.7 -> 57.2 / 52.2   43.8 -> 65.7 / 47.6   53.3 -> 75.1 / 61.5
