@@ -729,13 +729,17 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 //
 // Documents stay with one block and smaller grids: what a row sees is not known here.  head_dim 64, 2 x 8 x 1023, pieces of 1 to 255, 16.8 -> 13.2
 // / 14.0, 17.5 -> 14.5 / 14.7, 18.5 -> 16.1 / 15.6; 4 x 4 x 2000 in pieces of about 100 15.6 -> 16.9 / 20.1, of 500 (2 x 8) 33.9 -> 28.3 / 25.1.
-constexpr int kLongWalk = 1408;
+//
+// Walks below 704 rows, the 32-row kernels' chains being short: head_dim 64 causal 5 x 8 x 512, 1280 blocks, dK/dV 15.0 -> 17.7 with two, 4 x 8 x 600 16.6 -> 17.2; unmasked
+// forward of 768, 3 x 8 x 512, 12.0 with one, 12.8 with two, dQ of 384, 3 x 4 x 512, 10.2 / 11.0; head_dim 128 causal dQ of 1280, 5 x 8 x 512, 25.8 -> 27.5, but
+// unmasked of 768 25.0 -> 20.8 with two.
+constexpr int kShortWalk = 704, kLongWalk = 1408;
 struct Lines {
-  int blocks, blocks_of_long_walks;  // up to which a call is served
+  int blocks[3];  // up to which a call is served: of short walks, between, of long ones
 };
 constexpr Lines kLines[2][2][3] = {  // head_dim 128, causal, pass (forward, dQ, dK/dV)
-    {{{1024, 1536}, {1024, 1536}, {1024, 1536}}, {{2048, 3072}, {2048, 3072}, {2048, 2560}}},
-    {{{512, 1024}, {1024, 1536}, {512, 512}}, {{1024, 2048}, {2048, 3072}, {1024, 1024}}}};
+    {{{{768, 1024, 1536}}, {{768, 1024, 1536}}, {{768, 1024, 1536}}}, {{{2048, 2048, 3072}}, {{2048, 2048, 3072}}, {{1024, 2048, 2560}}}},
+    {{{{512, 512, 1024}}, {{1024, 1024, 1536}}, {{512, 512, 512}}}, {{{1024, 1024, 2048}}, {{1024, 2048, 3072}}, {{1024, 1024, 1024}}}}};
 
 static bool half_walked(const AttnParams& p, int mode) { return mode == MLTS_MASK_CAUSAL && p.Sk <= p.Sq + p.Sq / 2; }
 static int64_t row_blocks(AttnPass pass, const AttnParams& p) {
@@ -743,17 +747,22 @@ static int64_t row_blocks(AttnPass pass, const AttnParams& p) {
   return static_cast<int64_t>(((keys ? p.Sk : p.Sq) + 15) / 16) * p.B * (keys ? p.Hkv : p.Hq);
 }
 
+static int64_t walked(AttnPass pass, const AttnParams& p) { return pass == ATTN_BWD_DKV ? static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) : p.Sk; }
+
 // Two blocks of 16 rows to a wavefront.  (Of half of the blocks whose walk is that long, eight splits each still fill the chip.)
-static bool two_blocks(AttnPass pass, const AttnParams& p, int mode) {
-  const int64_t blocks = row_blocks(pass, p), walk = pass == ATTN_BWD_DKV ? static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) : p.Sk;
-  return walk >= 96 && (blocks >= (half_walked(p, mode) ? 832 : 384) || (blocks >= 512 && walk >= 4096));
+static bool two_blocks(AttnPass pass, const AttnParams& p, int D, int mode) {
+  const int64_t blocks = row_blocks(pass, p), walk = walked(pass, p);
+  if (walk < 96) return false;
+  if (half_walked(p, mode)) return blocks >= 832 || (blocks >= 512 && walk >= 4096);
+  if (walk < kShortWalk && (D == 64 || D == 128)) return D == 128 && blocks >= 512;
+  return blocks >= 384;
 }
 
 bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode, const int64_t* dout_stride) {
-  const int walk = pass == ATTN_BWD_DKV ? p.Sq : p.Sk, which = pass == ATTN_FWD ? 0 : pass == ATTN_BWD_DQ ? 1 : 2;
-  if (walk < 512) return false;
-  const Lines& line = kLines[D == 128][half_walked(p, mode)][which];
-  const int limit = mode == MLTS_MASK_DOC ? (D == 64 ? 1024 : 768) : walk >= kLongWalk ? line.blocks_of_long_walks : line.blocks;
+  if ((pass == ATTN_BWD_DKV ? p.Sq : p.Sk) < 512) return false;
+  const int64_t walk = walked(pass, p);
+  const int which = pass == ATTN_FWD ? 0 : pass == ATTN_BWD_DQ ? 1 : 2;
+  const int limit = mode == MLTS_MASK_DOC ? (D == 64 ? 1024 : 768) : kLines[D == 128][half_walked(p, mode)][which].blocks[walk >= kLongWalk ? 2 : walk >= kShortWalk ? 1 : 0];
   if (row_blocks(pass, p) > limit) return false;
   return near(p.Sq, p.qs) && near(p.Sk, p.ks) && near(p.Sk, p.vs) && near(p.Sq, p.os) && (!dout_stride || near(p.Sq, dout_stride));
 }
@@ -782,7 +791,7 @@ bool mlts_attn_small_serves_parts(const AttnParams& p, int D, int mode, const At
 int mlts_attn_small_fwd(AttnParams p, int D, int mode, hipStream_t st) {
   set_causal_off(p, mode);
   if (mode == MLTS_MASK_DOC) return D == 64 ? fwd<64, true, 1>(p, st) : fwd<128, true, 1>(p, st);
-  const bool two = two_blocks(ATTN_FWD, p, mode);
+  const bool two = two_blocks(ATTN_FWD, p, D, mode);
   if (D == 32) return two ? fwd<32, false, 2>(p, st) : fwd<32, false, 1>(p, st);
   if (D == 96) return two ? fwd<96, false, 2>(p, st) : fwd<96, false, 1>(p, st);
   if (D == 64) return two ? fwd<64, false, 2>(p, st) : fwd<64, false, 1>(p, st);
@@ -793,7 +802,7 @@ int mlts_attn_small_fwd(AttnParams p, int D, int mode, hipStream_t st) {
 int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
   if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dq<64, true, 1>(bp, st) : bwd_dq<128, true, 1>(bp, st);
-  const bool two = two_blocks(ATTN_BWD_DQ, bp.a, mode);
+  const bool two = two_blocks(ATTN_BWD_DQ, bp.a, D, mode);
   if (D == 32) return two ? bwd_dq<32, false, 2>(bp, st) : bwd_dq<32, false, 1>(bp, st);
   if (D == 96) return two ? bwd_dq<96, false, 2>(bp, st) : bwd_dq<96, false, 1>(bp, st);
   if (D == 64) return two ? bwd_dq<64, false, 2>(bp, st) : bwd_dq<64, false, 1>(bp, st);
@@ -804,8 +813,8 @@ int mlts_attn_small_bwd_dq(AttnBwdParams bp, int D, int mode, hipStream_t st) {
 int mlts_attn_small_bwd_dkv(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   set_causal_off(bp.a, mode);
   if (mode == MLTS_MASK_DOC) return D == 64 ? bwd_dkv<64, true, 1>(bp, st) : bwd_dkv<128, true, 1>(bp, st);
-  if (D == 32) return two_blocks(ATTN_BWD_DKV, bp.a, mode) ? bwd_dkv<32, false, 2>(bp, st) : bwd_dkv<32, false, 1>(bp, st);
+  if (D == 32) return two_blocks(ATTN_BWD_DKV, bp.a, D, mode) ? bwd_dkv<32, false, 2>(bp, st) : bwd_dkv<32, false, 1>(bp, st);
   if (D == 96) return bwd_dkv<96, false, 1>(bp, st);
-  if (D == 64) return two_blocks(ATTN_BWD_DKV, bp.a, mode) ? bwd_dkv<64, false, 2>(bp, st) : bwd_dkv<64, false, 1>(bp, st);
+  if (D == 64) return two_blocks(ATTN_BWD_DKV, bp.a, D, mode) ? bwd_dkv<64, false, 2>(bp, st) : bwd_dkv<64, false, 1>(bp, st);
   return bwd_dkv<128, false, 1>(bp, st);
 }

@@ -489,8 +489,8 @@ def test_long_rows_of_small_grids(dev, mode, B, Hq, Hkv, Sq, Sk, D):
     run_case(dev, torch.bfloat16, B, Hq, Hkv, Sq, Sk, D, mode, seed=Sq + Sk + D, max_doc=200, pad_tail=21 * (Sq & 1), share_ids=B == 1)
 
 
-@pytest.mark.parametrize("mode,B,Hq,Hkv,Sq,Sk,D", [(ops.MASK_CAUSAL, 4, 8, 8, 513, 513, 64), (ops.MASK_CAUSAL, 3, 10, 10, 545, 561, 128), (ops.MASK_NONE, 4, 8, 8, 512, 512, 64),
-                                                   (ops.MASK_NONE, 2, 8, 8, 527, 1040, 128), (ops.MASK_CAUSAL, 1, 16, 4, 2047, 2050, 64), (ops.MASK_CAUSAL, 2, 11, 11, 1430, 1409, 64)])
+@pytest.mark.parametrize("mode,B,Hq,Hkv,Sq,Sk,D", [(ops.MASK_CAUSAL, 2, 14, 14, 513, 513, 64), (ops.MASK_CAUSAL, 3, 9, 9, 545, 561, 128), (ops.MASK_NONE, 2, 8, 8, 707, 707, 64),
+                                                   (ops.MASK_NONE, 2, 7, 7, 527, 1040, 128), (ops.MASK_CAUSAL, 1, 16, 4, 2047, 2050, 64), (ops.MASK_CAUSAL, 2, 11, 11, 1430, 1409, 64)])
 def test_two_blocks_of_sixteen_rows_to_a_wavefront(dev, mode, B, Hq, Hkv, Sq, Sk, D):
     """A last wavefront whose second block is empty or cut, rows past the last key, walks that end inside a unit, a short and a long walk on
     either side of the grids' lines, dK/dV over the heads of a group; and the accumulation modes."""
