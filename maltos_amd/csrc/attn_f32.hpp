@@ -26,7 +26,12 @@
 // Two blocks of 16 rows to a wavefront in the backward kernels (head dims up to 64) share what is fetched and its way through LDS, for longer
 // and fewer chains (us, one / two; blocks of 16 own rows; head_dim 64, causal).  dQ: 8 x 8 heads x 1024, 4096 blocks, 161 / 122, 4 x 8 x 1024, 2048
 // blocks, 70 / 69, unmasked 126 / 116, 2 x 8 x 1024 42 / 43.  dK/dV, which fetches most for a row: 4096 blocks 207 / 174, 2048 119 / 93, 1024 63 / 53,
-// 704 (4 x 4 x 700) 40 / 36.5, 912 of short walks (6 x 8 x 300) 27.6 / 26, but 8 x 8 x 256 23.4 / 24.1 and 512 blocks (8 x 1024) 36 / 49.
+// 704 (4 x 4 x 700) 40 / 36.5, 912 of short walks (6 x 8 x 300) 27.6 / 26, but 8 x 8 x 256 23.4 / 24.1 and 512 blocks (8 x 1024) 36 / 49; head_dim 32, two of
+// whose eight-wavefront workgroups share a CU while others are idle, from 1024 blocks on (4 x 4 x 700 23.0 / 27.5).
+//
+// dK/dV takes the statistics of a unit's queries through LDS, a lane one of them, in place of eight loads a lane and their addresses (before / now):
+// 2 x 8 (4) x 777 46 / 42, 8 x 8 x 1024 174 / 159, 2 x 8 (2) x 1024 92 / 81, unmasked 8 x 1024 54.5 / 48.4.  (With registers for four wavefronts a SIMD, 16
+// of them spilled, 62, 159, 107, 61.)
 #pragma once
 #include "attn_rows.hpp"
 

@@ -150,6 +150,9 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
   join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1);
 }
 
+template <int DP>
+constexpr int kDkvFloats = 2 * Turn<DP>::FLOATS + 32;  // LDS of a wavefront
+
 // dK, dV of R * 16 key rows of one KV head, summed over the query heads of its group.
 template <int DP, int R, bool DOC, int LAYOUT>
 __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(const AttnBwdParams bp, const RowArgs a) {
@@ -205,8 +208,10 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
 #pragma unroll
     for (int db = 0; db < NC; ++db) dkv[n][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 qf[FRAGS], dof[FRAGS];
-  float *turn_q = lds + at.wave * 2 * Turn<DP>::FLOATS, *turn_do = turn_q + Turn<DP>::FLOATS;
-  float lse[4], delta[4];
+  float *turn_q = lds + at.wave * kDkvFloats<DP>, *turn_do = turn_q + Turn<DP>::FLOATS;
+  float* lstat = turn_do + Turn<DP>::FLOATS;  // lse and delta of the unit's queries: a lane fetches one, and reads four of each
+  float stat = 0.f;
+  int row_fetched = 0;
   int qp[4], qs[4];
   const float* Q0 = static_cast<const float*>(p.q) + b * p.qs[0];
   const float* dO0 = static_cast<const float*>(bp.dout) + b * bp.dos[0];
@@ -217,13 +222,14 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     const float *q_row = row_of<LAYOUT>(Q, safe, p.qs[2]), *do_row = row_of<LAYOUT>(dO, safe, bp.dos[2]);
 #pragma unroll
     for (int j = 0; j < FRAGS; ++j) qf[j] = load_dot<LAYOUT>(q_row, 16 * j + 4 * g, a.D), dof[j] = load_dot<LAYOUT>(do_row, 16 * j + 4 * g, a.D);
-    const int64_t stat = (static_cast<int64_t>(b) * p.Hq + head) * p.Sq;
+    row_fetched = q + l16;
+    stat = (lane & 16 ? bp.delta : p.lse)[(static_cast<int64_t>(b) * p.Hq + head) * p.Sq + min(row_fetched, p.Sq - 1)];
+    if (DOC) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ok = min(q + 4 * g + i, p.Sq - 1);
-      lse[i] = p.lse[stat + ok];
-      delta[i] = bp.delta[stat + ok];
-      if (DOC) qp[i] = units.pos[ok], qs[i] = units.seq[ok];
+      for (int i = 0; i < 4; ++i) {
+        const int ok = min(q + 4 * g + i, p.Sq - 1);
+        qp[i] = units.pos[ok], qs[i] = units.seq[ok];
+      }
     }
   };
   // the units of all heads of the group, one after the other
@@ -252,20 +258,19 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
           dp[r] = mfma4(o[c], vf[r][j][c], dp[r]);
         }
     }
-    float lse_now[4], delta_now[4];
+    // probability 0: rows past the end, rows that saw no key
+    lstat[lane & 31] = (lane & 16) == 0 && (row_fetched >= p.Sq || stat == -INFINITY) ? INFINITY : stat;
     int qp_now[4], qs_now[4];
+    if (DOC) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      // probability 0: rows past the end, rows that saw no key
-      lse_now[i] = q0 + 4 * g + i < p.Sq && lse[i] != -INFINITY ? lse[i] : INFINITY;
-      delta_now[i] = delta[i];
-      if (DOC) qp_now[i] = qp[i], qs_now[i] = qs[i];
+      for (int i = 0; i < 4; ++i) qp_now[i] = qp[i], qs_now[i] = qs[i];
     }
     // (past the end the last query is fetched again: a branch around the loads would wait for all of them; without the barriers the
     // compiler moves them behind the products that they would arrive under)
     __builtin_amdgcn_sched_barrier(0);
     fetch(min(hn, group - 1), qn);
     __builtin_amdgcn_sched_barrier(0);
+    const f32x4 lse_now = *reinterpret_cast<const f32x4*>(lstat + 4 * g), delta_now = *reinterpret_cast<const f32x4*>(lstat + 16 + 4 * g);
     const bool masked = !DOC && (q0 < all_qmin || ragged);
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -330,7 +335,7 @@ int bwd_dkv(const AttnBwdParams& bp, int D, hipStream_t st) {
   const RowArgs a(p, D, LAYOUT != ROWS_ANY && rows_vec(bp.dks, bp.dk) && rows_vec(bp.dvs, bp.dv), p.Hkv, tiles);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
   const int splits = splits_for(blocks, static_cast<int64_t>((p.Sq + 15) / 16) * (p.Hq / p.Hkv), max_splits(DP, LAYOUT));
-  return launch_splits<attn_f32_bwd_dkv<DP, R, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, 2 * R * DP * 64, 2 * Turn<DP>::FLOATS * 4, st, bp, a,
+  return launch_splits<attn_f32_bwd_dkv<DP, R, DOC, LAYOUT>, max_splits(DP, LAYOUT)>(blocks, splits, 2 * R * DP * 64, kDkvFloats<DP> * 4, st, bp, a,
                                                                                      "mlts_attn_bwd");
 }
 
@@ -343,7 +348,7 @@ int bwd(AttnBwdParams bp, int D, hipStream_t st) {
     if (int rc = two ? bwd_dq<DP, TWO, DOC, LAYOUT>(bp, D, st) : bwd_dq<DP, 1, DOC, LAYOUT>(bp, D, st); rc != MLTS_OK) return rc;
   }
   if (p.Sk == 0) return MLTS_OK;
-  const bool two = static_cast<int64_t>((p.Sk + 31) / 32) * p.B * p.Hkv >= 352 && static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) > 256;
+  const bool two = static_cast<int64_t>((p.Sk + 31) / 32) * p.B * p.Hkv >= (DP == 32 ? 512 : 352) && static_cast<int64_t>(p.Sq) * (p.Hq / p.Hkv) > 256;
   return two ? bwd_dkv<DP, TWO, DOC, LAYOUT>(bp, D, st) : bwd_dkv<DP, 1, DOC, LAYOUT>(bp, D, st);
 }
 

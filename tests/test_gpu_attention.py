@@ -457,9 +457,9 @@ def test_fp32_blocks_shared_by_wavefronts(dev, D, B, H):
         run_case(dev, torch.float32, B, H, H, 1030, 1030, D, mode, seed=B + D, max_doc=300)
 
 
-# blocks of 32 keys: 544, 420, 352 and 360; a last one of 1, 16 and 20 rows; several heads to a group, head dims inside their padding, unaligned rows
+# blocks of 32 keys: 544, 420, 352 and 520 (head_dim 32); a last one of 1, 16 and 20 rows; several heads to a group, head dims inside their padding, unaligned rows
 @pytest.mark.parametrize("B,H,Hkv,Sq,Sk,D,mode", [(16, 8, 2, 513, 513, 64, ops.MASK_CAUSAL), (20, 7, 7, 500, 80, 33, ops.MASK_NONE), (4, 8, 8, 257, 340, 60, ops.MASK_CAUSAL),
-                                                  (9, 4, 4, 304, 304, 32, ops.MASK_DOC)])
+                                                  (13, 4, 4, 304, 304, 32, ops.MASK_DOC)])
 def test_fp32_two_key_blocks_to_a_wavefront(dev, B, H, Hkv, Sq, Sk, D, mode):
     run_case(dev, torch.float32, B, H, Hkv, Sq, Sk, D, mode, seed=Sq + D, max_doc=100)
 
