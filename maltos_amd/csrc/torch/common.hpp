@@ -111,7 +111,10 @@ Tensor grad_sum_slices(const Tensor& parts, const OptTensor& out, bool accumulat
 Tensor rms_norm(const Tensor& x, const Tensor& w, double eps, bool into_grad);
 std::tuple<Tensor, Tensor> add_rms_norm(const Tensor& x, const Tensor& res, const Tensor& w, double eps, bool into_grad);  // (sum, its norm)
 
-bool own_product(int form, const Tensor& a, const Tensor& b);  // whether `product` runs on the own kernels: by size, type, layout
+int64_t weight_grad_splits(int64_t rows, int64_t out_features, int64_t in_features);  // products.cpp
+// What shares a product's launch: nothing; dx and dW of one layer each other; the rotation; the activation, gate and up being kept; the activation alone, or its gradient
+enum class Use { ALONE, WITH_WEIGHT_GRAD, ROTATION, GATE_AND_UP, ACTIVATION };
+bool own_product(int form, const Tensor& a, const Tensor& b, Use use = Use::ALONE);  // whether it runs on the own kernels: by size, type, layout
 // a, b as the form (MLTS_GEMM_*) says -> [M, N], written to `out` (or added onto it) if that is given
 Tensor product(int form, const Tensor& a, const Tensor& b, const Tensor& out = Tensor(), bool accumulate = false);  // products.cpp
 

@@ -117,16 +117,6 @@ struct FlatViews {
 };
 
 // ---- products -------------------------------------------------------------------------------------------------------------
-// Number of K-splits for dW = dY^T X.  The product has only out * in outputs but `rows` (= tokens) terms each: for the
-// LLaMA-50M projections (512..1536 wide, 16384 tokens) a single GEMM fills a quarter of the 256 CUs and runs at ~85
-// TFLOP/s, the same work as a batch of 8-16 row slices reaches 300-600 TFLOP/s on MI355X.
-int64_t weight_grad_splits(int64_t rows, int64_t out_features, int64_t in_features) {
-  const int64_t tiles = ((out_features + 255) / 256) * ((in_features + 255) / 256);
-  int64_t splits = 1;
-  while (splits < 16 && tiles * splits < 128 && rows % (splits * 2) == 0 && rows / (splits * 2) >= 1024) splits *= 2;
-  return splits;
-}
-
 Tensor rows2d(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
 
 // dW = dy2^T x2 for [rows, out] / [rows, in] operands, large ones as a batch of row-slice products where that fills the chip
@@ -156,7 +146,7 @@ Tensor project(const Tensor& x, const Tensor& weight) {
 // launch where both run on the own kernels, as neither fills the chip at the sizes they are used for
 std::pair<Tensor, Tensor> input_and_weight_grad(const Tensor& dy2, const Tensor& w, const Tensor& x2, const Tensor& grad, bool need_dx, bool need_dw) {
   if (!need_dx || !need_dw) return {need_dx ? product(MLTS_GEMM_NN, dy2, w) : Tensor(), need_dw ? weight_grad(x2, dy2, grad) : Tensor()};
-  if (own_product(MLTS_GEMM_NN, dy2, w) && own_product(MLTS_GEMM_TN, dy2, x2) && (!grad.defined() || own_output(grad, x2))) {
+  if (own_product(MLTS_GEMM_NN, dy2, w, Use::WITH_WEIGHT_GRAD) && own_product(MLTS_GEMM_TN, dy2, x2, Use::WITH_WEIGHT_GRAD) && (!grad.defined() || own_output(grad, x2))) {
     Tensor dx = at::empty({dy2.size(0), w.size(1)}, dy2.options());
     Tensor dw = grad.defined() ? grad : at::empty(w.sizes(), dy2.options());
     ProductList list;
@@ -377,8 +367,9 @@ Tensor project_all(const Tensor& x, const Adjacent& rows, const std::vector<Tens
 std::pair<Tensor, Tensor> gate_up_activation(const Tensor& x, const Adjacent& rows, const std::vector<Tensor>& weights, bool keep) {
   const Tensor &wg = weights[0], &wu = weights[1], x2 = rows2d(x);
   const int64_t cols = wg.size(0), es = x.element_size();
-  if (x.is_contiguous() && wu.sizes() == wg.sizes() && wu.stride(0) == wg.stride(0) && own_product(MLTS_GEMM_NT, x2, rows.weight.defined() ? rows.weight : wg) &&
-      own_product(MLTS_GEMM_NT, x2, wg) && own_product(MLTS_GEMM_NT, x2, wu) && (rows.first[0] * es) % 16 == 0 && (rows.first[1] * es) % 16 == 0 &&
+  const Use use = keep ? Use::GATE_AND_UP : Use::ACTIVATION;
+  if (x.is_contiguous() && wu.sizes() == wg.sizes() && wu.stride(0) == wg.stride(0) && own_product(MLTS_GEMM_NT, x2, rows.weight.defined() ? rows.weight : wg, use) &&
+      own_product(MLTS_GEMM_NT, x2, wg, use) && own_product(MLTS_GEMM_NT, x2, wu, use) && (rows.first[0] * es) % 16 == 0 && (rows.first[1] * es) % 16 == 0 &&
       mlts_gemm_swiglu_supports(dtype_code(x), x2.size(0), cols, x2.size(1), x2.stride(0), wg.stride(0), rows.width, cols) == nullptr) {
     c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = cols;
@@ -744,7 +735,7 @@ Tensor project_rotated(const Tensor& x, const BlockWeights& w, int64_t heads, in
             : p.offset < 0 || p.offset + S > max_pos)
     return Tensor();
   const Tensor x2 = rows2d(x);
-  if (rows.weight.defined() && !own_product(MLTS_GEMM_NT, x2, rows.weight)) return Tensor();
+  if (rows.weight.defined() && !own_product(MLTS_GEMM_NT, x2, rows.weight, Use::ROTATION)) return Tensor();
   const Tensor y = at::empty({B, S, rows.width}, x.options()), y2 = rows2d(y);
   mlts_gemm_rotation r{};
   r.cos = ptr(cos), r.sin = ptr(sin), r.positions = given ? p.rope->const_data_ptr<int32_t>() : nullptr;
@@ -799,25 +790,22 @@ std::pair<Tensor, Tensor> activation_and_weight_grad(const Tensor& dy2, const Te
                                                      const Tensor& grad, bool need_dw) {
   const int64_t cols = w.size(1), es = gu.element_size(), width = gu.size(-1);
   if (width != 2 * cols || !gu.is_contiguous() || !aligned(gu) || (rows.first[0] * es) % 16 || (rows.first[1] * es) % 16 ||
-      !own_product(MLTS_GEMM_NN, dy2, w) || gu.scalar_type() != dy2.scalar_type() || gu.numel() / width != dy2.size(0) ||
+      !own_product(MLTS_GEMM_NN, dy2, w, Use::ACTIVATION) || (need_dw && !own_product(MLTS_GEMM_TN, dy2, h2, Use::ACTIVATION)) || gu.scalar_type() != dy2.scalar_type() || gu.numel() / width != dy2.size(0) ||
       (grad.defined() && (!own_output(grad, h2) || !grad.is_contiguous())))
     return {};
   int64_t ws_bytes = 0;
   const int dtype = dtype_code(dy2);
-  const bool apart = need_dw && !own_product(MLTS_GEMM_TN, dy2, h2);
-  if (apart) need_dw = false;
   if (mlts_gemm_swiglu_bwd_supports(dtype, need_dw, dy2.size(0), cols, dy2.size(1), dy2.stride(0), w.stride(0), h2.stride(0), width, width,
                                     &ws_bytes) != nullptr)
     return {};
   const Tensor dgu = at::empty(gu.sizes(), gu.options());
-  Tensor dw = !need_dw ? Tensor() : grad.defined() ? grad : at::empty(w.sizes(), dy2.options());
+  const Tensor dw = !need_dw ? Tensor() : grad.defined() ? grad : at::empty(w.sizes(), dy2.options());
   const Tensor ws = workspace(ws_bytes, dy2);
   const char* in = static_cast<const char*>(ptr(gu));
   char* out = static_cast<char*>(mptr(dgu));
   check(mlts_gemm_swiglu_bwd(dtype, dy2.size(0), cols, dy2.size(1), ptr(dy2), dy2.stride(0), ptr(w), w.stride(0), ptr(h2), h2.stride(0), need_dw ? mptr(dw) : nullptr,
                              grad.defined(), in + rows.first[0] * es, in + rows.first[1] * es, width, out + rows.first[0] * es, out + rows.first[1] * es, width,
                              ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
-  if (apart) dw = weight_grad(h2, dy2, grad);
   return {dgu, dw};
 }
 

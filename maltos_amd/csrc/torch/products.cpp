@@ -6,27 +6,60 @@
 #include "common.hpp"
 
 namespace maltos {
+
+// Number of K-splits for dW = dY^T X.  The product has only out * in outputs but `rows` (= tokens) terms each: for the
+// LLaMA-50M projections (512..1536 wide, 16384 tokens) a single GEMM fills a quarter of the 256 CUs and runs at ~85
+// TFLOP/s, the same work as a batch of 8-16 row slices reaches 300-600 TFLOP/s on MI355X.
+int64_t weight_grad_splits(int64_t rows, int64_t out_features, int64_t in_features) {
+  const int64_t tiles = ((out_features + 255) / 256) * ((in_features + 255) / 256);
+  int64_t splits = 1;
+  while (splits < 16 && tiles * splits < 128 && rows % (splits * 2) == 0 && rows / (splits * 2) >= 1024) splits *= 2;
+  return splits;
+}
+
 namespace {
 
 // Where the own kernels run, by M * N * K.  A product through torch costs 18 us of host time, a call here 5, and that is what
 // small steps wait for.  On the GPU alone (both sides timed with the weights out of HBM; rows from 100 to 16384; the library's choice
-// untuned, or with the shipped per-shape selection where that has the shape) they are ahead of the library
+// untuned) they are ahead of the library
 //   fp32  0.5 to 1e9  0.86 of its time (y), 0.86 (dx), 0.82 (dW)    2.5 to 3e9  0.90, 0.92, 0.87    3 to 4e9  1.13, 1.15, 1.17
 //   bf16  up to 4e9   0.4 to 0.95
-//         above it, y and dx of 256 or 512 terms: 8192 x 2752 x 512 34.3 us against 61.7, 12000 x 2752 x 512 50 against 80, 16384 x 2752 x 512
-//         61 against 78, 16384 x 1376 x 512 36 against 50; but 16384 x 1536 x 512 38 against 32 with the shipped selection (rotated on
-//         its way out 39 against 32 + 15)
-//         1024 to 1536 terms: 12000 x 512 x 1376 31 against 36, 16384 x 512 x 1376 34 against 40, 16384 x 512 x 1536 32 against 35; but 6000 and
-//         12000 x 1024 x 1024 20.9 and 33.6 against 19.6 and 30.0
-//         2752 terms: 3000 x 512 21 against 26, 6000 x 512 31 against 33, 12000 x 512 50 against 46
-//         dW against a batch of row slices: 6000 rows 1536 x 512 27 against 44, 8192 rows 2752 x 512 46 against 52, 12000 rows 39 against 52
-//         and 58 against 95; but 16384 rows 47 against 41 and 73 against 63
-//         columns of a vocabulary (32000 x 512): 1023 rows 54 against 49, 3000 rows 136 against 131
 constexpr double kOwnLimitBf16 = 4.0e9, kOwnLimitF32 = 3.0e9;
-double larger_limit_bf16(int form, int64_t M, int64_t N, int64_t K) {
-  if (N >= 16384 || N % 8) return 0;
-  if (form == MLTS_GEMM_TN) return M < 16384 && K < 16384 ? 3.0e10 : 0;
-  return K <= 768 ? 3.0e10 : K <= 1536 ? 1.3e10 : K <= 2816 ? 8.5e9 : 0;
+
+// Larger bf16 products, by what running one of them on the own kernels adds to a layer's training step in which the library has the others (us; 145
+// layers of 21 shapes, 256 to 2048 wide, of 3000 to 32768 rows; two runs differ by 4 us).  These lines take 7 % off a layer's step on the mean, and the
+// one that is slower than with the library alone by more than half a percent is by 1.7 % (dW of 1024 x 1024, 10000 rows).
+//   terms of y and dx, either side of the lines
+//     up to 768, 3e10      y of 3 x 768 rotated, 16384 rows -33, 20020 +7; gate and up of 2 x 1376 x 512, 16384 rows -23; of 2 x 2048 x 768, 6000 rows -7, 24576 +91
+//     up to 1536, 1.3e10   y of 512 x 1376, 16384 rows -18; of 512 x 1536, 8192 rows -5, 16384 0, 20020 +10, 24576 +17
+//     up to 2816, 8.5e9    y of 512 x 2048, 4096 rows -15, 8192 +8, 20020 +27; of 896 x 2392, 4096 rows -3, 10000 +26
+//   1024 and more columns and terms, both whole tiles of 256 (the library's): y of 1024 x 1024, 6000 rows +2 to +27, 12000 -2 to +11 (alone, 6000 and 12000 rows:
+//     22 us against 18, 34 against 26).  With their dW in one launch up to 8.5e9: 3000 x 1280 x 1280 -22, 6000 x 1024 x 1024 -15 to +4, but 10000 rows +54 to +76.
+//   gate and up in one launch, kept for a backward pass, 257 to 512 terms, whole tiles whose 256 x 256 fill their rounds over the CUs: 2 x 2048 x 512, 8192 rows +13 and 10000
+//     +25, beside -15 and -17 for the product and the pass apart; but 12000 rows of 2 x 1536 x 512 (a quarter idle) -11.
+//   dW, which the library forms as a batch of row slices (weight_grad_splits).  Slices too few for 64 of its tiles: 1024 x 1024 of 20001 rows, alone, 56 us against 162.  Slices of
+//     whole 1024 rows, from 16384 rows on: 512 to 768 wide 16384 rows -14 to +20, 24576 -32 to +32, but 20020 rows -2 to -57; below, up to 2e10: 5456 x 1024 x 4096 +13 to +15,
+//     3072 x 1024 x 8192 +4 to +21; 64 tiles without slices: 6912 x 1280 x 3000 +21, 5456 x 1024 x 3000 -4 to -9; others up to 3e10: 1024 x 2728 x 10000 -55, 1280 x 1792 x 12000 -27.
+//     In one launch with dh = dy W and the activation -2 to -107 at all row counts up to 32768; that dh without its dW up to +74.
+// (With the shipped per-shape selection, 16384 rows, alone: y 512 x 512 19 us against 17, 1536 x 512 46 / 33, in a step rotated on its way out 47 / 32 + 15,
+// 512 x 1376 39 / 39, 2752 x 512 69 / 80; dW 512 x 1376 40 / 45, 1536 x 512 46 / 37, 2752 x 512 69 / 58.)  Products with the columns of a vocabulary (32000 x 512): 1023 rows
+// 54 / 49, 3000 rows 136 / 131.
+bool larger_own_range_bf16(int form, int64_t M, int64_t N, int64_t K, Use use) {
+  const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
+  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+  if (N >= 16384 || N % 8) return false;
+  if (form == MLTS_GEMM_TN) {
+    if (M >= 16384) return false;
+    if (use == Use::ACTIVATION) return true;
+    const bool few = tiles * weight_grad_splits(K, M, N) < 64, whole = !few && K % 1024 == 0;
+    return !(whole && K >= 16384) && size <= (whole || tiles >= 64 ? 2.0e10 : 3.0e10);
+  }
+  if (size > (K <= 768 ? 3.0e10 : K <= 1536 ? 1.3e10 : K <= 2816 ? 8.5e9 : 0)) return false;
+  if (K >= 1024 && N >= 1024 && N % 256 == 0 && K % 256 == 0) {
+    if (use == Use::ALONE) return false;
+    if (use == Use::WITH_WEIGHT_GRAD) return size <= 8.5e9;
+  }
+  return use != Use::GATE_AND_UP || N % 256 || K % 64 || K <= 256 || K > 512 || tiles <= 256 || 10 * tiles < 8 * ((tiles + 255) / 256 * 256);
 }
 
 // In bf16 they also run for dx = dy W with so long a contraction that it is split over workgroups (dx of an lm_head, of a wide
@@ -34,10 +67,10 @@ double larger_limit_bf16(int form, int64_t M, int64_t N, int64_t K) {
 // terms 0.54 to 0.83, 8192 terms 0.42 to 0.98; with 4096 or 5504 terms 0.76 to 1.04 where fewer than 128 tiles of 256 x 128 leave more
 // than half of the CUs idle unsplit, but 1.05 and 1.12 for 128 tiles (2048 x 2048 x 5504 56.6 us against 53.8, 1024 x 4096 x 4096 46.1
 // against 41.1).
-bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K) {
+bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K, Use use) {
   const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
   if (dtype == MLTS_F32) return size <= kOwnLimitF32;
-  if (size <= std::max(kOwnLimitBf16, larger_limit_bf16(form, M, N, K))) return true;
+  if (size <= kOwnLimitBf16 || larger_own_range_bf16(form, M, N, K, use)) return true;
   return form == MLTS_GEMM_NN && (K >= 8192 || M * N < 128 * 256 * 128) && mlts_gemm_workspace_bytes(form, dtype, M, N, K) > 0;
 }
 
@@ -62,11 +95,11 @@ Tensor library_product(int form, const Tensor& a, const Tensor& b, const Tensor&
 
 }  // namespace
 
-bool own_product(int form, const Tensor& a, const Tensor& b) {
+bool own_product(int form, const Tensor& a, const Tensor& b, Use use) {
   if (!plain(a) || !plain(b) || !same_contraction(form, a, b)) return false;  // (operands that do not match: torch says so)
   const Sizes z(form, a, b);
   return z.M > 0 && z.N > 0 && z.K > 0 && a.scalar_type() == b.scalar_type() &&
-         (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) && within_own_range(form, dtype_code(a), z.M, z.N, z.K) &&
+         (a.scalar_type() == at::kBFloat16 || a.scalar_type() == at::kFloat) && within_own_range(form, dtype_code(a), z.M, z.N, z.K, use) &&
          mlts_gemm_supports(form, dtype_code(a), z.M, z.N, z.K, a.stride(0), b.stride(0), z.N) == nullptr && aligned(a) && aligned(b) &&
          !c10::impl::dispatch_mode_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA);
 }

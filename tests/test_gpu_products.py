@@ -62,6 +62,23 @@ def test_products_left_to_the_library(dev):
     assert _lib.lib().mlts_gemm_supports(NT, _lib.MLTS_BF16, 64, 64, 33, 33, 33, 64) is not None
 
 
+@pytest.mark.parametrize("form,M,N,K,own", [
+    (NT, 6000, 1024, 1024, False), (NT, 12000, 1024, 1024, False), (NN, 12000, 1024, 1024, False), (NT, 4096, 1280, 1280, False), (NT, 6000, 1000, 1024, True),
+    (NT, 16384, 2304, 768, True), (NT, 17000, 2304, 768, False), (NN, 16384, 512, 1536, True), (NT, 17000, 512, 1536, False), (NT, 8000, 512, 2048, True), (NT, 8192, 512, 2048, False),
+    (TN, 1024, 1024, 12000, True), (TN, 1024, 1024, 16384, False), (TN, 1024, 1024, 20001, True), (TN, 512, 1376, 16384, False), (TN, 256, 680, 32768, True), (TN, 2752, 512, 12000, True),
+    (TN, 5456, 1024, 4096, False), (TN, 1024, 2728, 10000, True), (TN, 6912, 1280, 3000, False)])
+def test_which_large_products_the_own_kernels_take(dev, form, M, N, K, own):
+    """Both sides of each line between them and the library."""
+    a, b = (torch.zeros(s, dtype=torch.bfloat16, device=dev) for s in ((K, M) if form == TN else (M, K), (N, K) if form == NT else (K, N)))
+    _lib.kernel_timing(True)
+    try:
+        native().product(form, a, b)
+        torch.cuda.synchronize()
+        assert _lib.kernel_time_ms("gemm")[1] == int(own)
+    finally:
+        _lib.kernel_timing(False)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,hidden,widths", [(8, 64, (64, 32, 32)), (333, 136, (96, 72, 40)), (1023, 512, (512, 256, 256)), (2048, 256, (688, 688)), (4104, 512, (1376, 1376))])
 def test_group_of_projections(dev, dtype, rows, hidden, widths):
