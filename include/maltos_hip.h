@@ -303,6 +303,17 @@ typedef struct {
 int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* products, int32_t count, int32_t dtype);
 int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dtype, void* workspace, int64_t workspace_bytes,
                     mlts_stream_t stream);
+/* What a call would launch, decided on the host (nothing runs, no GPU is asked for): each product's tile, into how many slices its contraction is
+ * split, and whether it shares a launch with the others.  with: the products by themselves, or what mlts_gemm_rope, mlts_gemm_swiglu_bwd (dW and dh) or
+ * mlts_gemm_swiglu (one product, N of each of the two) makes of them. */
+#define MLTS_GEMM_WITH_NOTHING 0
+#define MLTS_GEMM_WITH_ROTATION 1
+#define MLTS_GEMM_WITH_ACTIVATION 2
+#define MLTS_GEMM_WITH_GATE_UP 3
+typedef struct {
+  int32_t tile_m, tile_n, slices, together;
+} mlts_gemm_tiles;
+int mlts_gemm_plan(const mlts_gemm_product* products, int32_t count, int32_t dtype, int32_t with, mlts_gemm_tiles* tiles);
 /* The backward pass of h W^T (W [K, N], h = round(silu(gate)) * up) in one launch: dW (+)= dy^T h (dense; null: not wanted), and d gate,
  * d up of dh = dy W, which is not written: the values of two products and mlts_swiglu_bwd_rows.  supports: NULL and the workspace it takes, or why not. */
 const char* mlts_gemm_swiglu_bwd_supports(int32_t dtype, int32_t weight, int64_t M, int64_t N, int64_t K, int64_t ldy, int64_t ldw, int64_t ldh,

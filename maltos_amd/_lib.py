@@ -115,6 +115,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "mlts_gemm_workspace_bytes": (C.c_int64, [C.c_int32, C.c_int32] + [C.c_int64] * 3),
     "mlts_gemm_multi_workspace_bytes": (C.c_int64, [_P, C.c_int32, C.c_int32]),
     "mlts_gemm_multi": (C.c_int, [_P, C.c_int32, C.c_int32, _P, C.c_int64, _P]),
+    "mlts_gemm_plan": (C.c_int, [_P, C.c_int32, C.c_int32, C.c_int32, _P]),
     "mlts_gemm_rope_supports": (C.c_char_p, [_P, C.c_int32, C.c_int32, _P]),
     "mlts_gemm_rope": (C.c_int, [_P, C.c_int32, C.c_int32, _P, _P]),
     "mlts_gemm_swiglu_bwd_supports": (C.c_char_p, [C.c_int32] * 2 + [C.c_int64] * 8 + [_P]),

@@ -1065,6 +1065,7 @@ mlts_gemm_product single(int32_t form, int64_t M, int64_t N, int64_t K, const vo
 template <typename T>
 int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, const Rotation* rotation, const Activation* activation, hipStream_t st) {
   const LaunchPlan plan(ps, count, dtype, activation != nullptr, rotation != nullptr);
+  MLTS_REQUIRE(plan.workspace == 0 || (workspace && !rotation), "mlts_gemm: a split that the call was not checked for");
   Rotation rot{};
   if (rotation) rot = *rotation;
   Products joint;
@@ -1199,6 +1200,25 @@ extern "C" int64_t mlts_gemm_multi_workspace_bytes(const mlts_gemm_product* prod
   return count < 1 || count > kMaxProducts ? 0 : LaunchPlan(products, count, dtype).workspace;
 }
 
+extern "C" int mlts_gemm_plan(const mlts_gemm_product* products, int32_t count, int32_t dtype, int32_t with, mlts_gemm_tiles* tiles) {
+  MLTS_REQUIRE(products && tiles && count >= 1 && count <= kMaxProducts, "mlts_gemm_plan: 1 to %d products in a call", kMaxProducts);
+  MLTS_REQUIRE(dtype == MLTS_BF16 || dtype == MLTS_F32, "mlts_gemm_plan: unknown dtype %d", dtype);
+  for (int i = 0; i < count; ++i)
+    if (const char* why = why_not(products[i], dtype)) MLTS_REQUIRE(false, "mlts_gemm_plan: %s", why);
+  if (with == MLTS_GEMM_WITH_GATE_UP) {
+    const int tile = pair_tile(products[0].M, products[0].N, products[0].k[0], dtype);
+    MLTS_REQUIRE(count == 1 && tile >= 0, "mlts_gemm_plan: gate and up of this size are not made in one launch");
+    tiles[0] = {kTileM[tile], kTileN[tile], 1, 0};
+    return MLTS_OK;
+  }
+  const LaunchPlan plan(products, count, dtype, with == MLTS_GEMM_WITH_ACTIVATION, with == MLTS_GEMM_WITH_ROTATION);
+  for (int i = 0; i < count; ++i) {
+    const bool small = plan.tile[i] == kSmall;
+    tiles[i] = {small ? plan.shape.size : kTileM[plan.tile[i]], small ? plan.shape.size : kTileN[plan.tile[i]], static_cast<int32_t>(plan.slices[i]), plan.together[i]};
+  }
+  return MLTS_OK;
+}
+
 static int check_products(const mlts_gemm_product* products, int32_t count, int32_t dtype) {
   MLTS_REQUIRE(dtype == MLTS_BF16 || dtype == MLTS_F32, "mlts_gemm: unknown dtype %d", dtype);
   MLTS_REQUIRE(products && count >= 1 && count <= kMaxProducts, "mlts_gemm: 1 to %d products in a call", kMaxProducts);
@@ -1272,7 +1292,7 @@ extern "C" const char* mlts_gemm_rope_supports(const mlts_gemm_product* products
       if (a < 0 || b < a || b > p.N || a % 4 || (b - a) % rotation->head_dim) return "columns that are not whole heads";
     }
   }
-  return LaunchPlan(products, count, dtype).workspace ? "products that would be split" : nullptr;
+  return LaunchPlan(products, count, dtype, false, true).workspace ? "products that would be split" : nullptr;
 }
 
 extern "C" int mlts_gemm_rope(const mlts_gemm_product* products, int32_t count, int32_t dtype, const mlts_gemm_rotation* rotation, mlts_stream_t stream) {

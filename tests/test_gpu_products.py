@@ -105,6 +105,11 @@ class GemmProduct(ctypes.Structure):
                 ("ldb", ctypes.c_int64 * 3), ("c", ctypes.c_void_p), ("ldc", ctypes.c_int64)]
 
 
+class GemmTiles(ctypes.Structure):
+    """Mirror of `mlts_gemm_tiles`."""
+    _fields_ = [("tile_m", ctypes.c_int32), ("tile_n", ctypes.c_int32), ("slices", ctypes.c_int32), ("together", ctypes.c_int32)]
+
+
 def run_products(products, dtype):
     """mlts_gemm_multi of (form, [(a, b), ...], c, accumulate)."""
     ps = (GemmProduct * len(products))()

@@ -3,6 +3,7 @@ argument validation raises before any launch, and the host-side mirrors of the r
 (ids, mask rule, zigzag layout, ring schedule, varlen metadata, backend names, optimizer plumbing)
 behave as the reference's tests expect.  No kernel is launched here."""
 import ctypes
+import random
 import re
 from pathlib import Path
 
@@ -18,6 +19,8 @@ from maltos_amd.flash_utils import varlen_prefix_metadata, varlen_qkv_metadata
 from maltos_amd.optim import FusedAdamW, MasterWeightsOptimizer
 from maltos_amd.ring_attention import zigzag_ring_schedule
 from maltos_amd.ring_layout import expected_zigzag_ring_positions, has_zigzag_ring_layout
+
+from .test_gpu_products import GemmProduct, GemmRotation, GemmTiles
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -321,3 +324,22 @@ def test_products_of_a_call_must_not_share_outputs():
     for apart in ([(0, 64, 64, 64), (4096, 64, 64, 64)], [(0, 64, 64, 160), (64, 64, 64, 160), (128, 64, 32, 160)], [(64, 64, 64, 128), (0, 64, 64, 128)],
                   [(0, 64, 64, 64), (0, 0, 64, 64)]):
         assert "row strides" in message(*apart), apart
+
+
+def test_rotated_products_are_planned_as_they_are_checked():
+    """mlts_gemm_rope has no workspace: a call it serves must be one that it launches without splitting a contraction."""
+    rng, L = random.Random(7), _lib.lib()
+    split = 0
+    for _ in range(4000):
+        count, dtype, D, K = rng.choice([1, 1, 2, 3]), rng.choice([_lib.MLTS_BF16, _lib.MLTS_F32]), rng.choice([32, 64, 96, 128]), 8 * rng.randint(1, rng.choice([32, 128, 1024, 4096]))
+        ps, r, M = (GemmProduct * count)(), GemmRotation(None, None, None, 64, 0, 64, D), min(int(2 ** rng.uniform(0, 15)), 2 ** 28 // K)
+        for i, p in enumerate(ps):
+            p.form, p.segments, p.M, p.N, p.k[0], p.lda[0], p.ldb[0] = 0, 1, M, D * rng.randint(1, 32), K, K, K
+            p.ldc, r.columns[i][1] = p.N, D
+        tiles = (GemmTiles * count)()
+        assert L.mlts_gemm_plan(ps, count, dtype, 1, tiles) == _lib.MLTS_OK
+        why = L.mlts_gemm_rope_supports(ps, count, dtype, ctypes.byref(r))
+        assert why in (None, b"products that would be split")
+        assert (why is None) == all(t.slices == 1 for t in tiles), (M, [p.N for p in ps], K, dtype)
+        split += why is not None
+    assert 50 < split < 3950
