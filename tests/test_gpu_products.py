@@ -181,7 +181,7 @@ def test_operands_that_do_not_match_are_refused(dev, form, longer):
                                          (torch.bfloat16, 1100, 2056, 72), (torch.bfloat16, 4001, 1032, 64), (torch.float32, 700, 1028, 68),
                                          (torch.float32, 2048, 1376, 40)])
 def test_gate_up_in_one_launch(dev, dtype, M, N, K, keep):
-    """Tiles of 64, 128 and 256 rows with remainders of rows, columns (of each of the two products) and slabs, operands with row
+    """Tiles of 64 and 128 rows, in fp32 also of 256, with remainders of rows, columns (of each of the two products) and slabs, operands with row
     strides, gate and up wanted or not: the bits of the product with both weights and the pass over it."""
     gen = torch.Generator().manual_seed(M + N)
     rows = lambda n: torch.randn(n, K + 24, generator=gen).to(dtype).to(dev)[:, 16:16 + K]
@@ -212,7 +212,7 @@ class GemmRotation(ctypes.Structure):
                                                        (2, 333, 2, 2, 96, 264, True, True), (3, 701, 8, 8, 64, 64, False, True),
                                                        (3, 777, 16, 4, 128, 40, False, False), (2, 3001, 16, 8, 96, 64, False, True)])
 def test_rotation_in_the_products(dev, dtype, B, S, H, Hkv, D, K, joint, given):
-    """q, k, v as one product or as three: every tile, remainders of rows and slabs, positions of packed rows, or an offset; the
+    """q, k, v as one product or as three: remainders of rows and slabs, positions of packed rows, or an offset; the
     bits of the products and the rotation one after the other."""
     gen = torch.Generator().manual_seed(B * S + D)
     rnd = lambda *s: torch.randn(*s, generator=gen).to(dtype).to(dev)
@@ -276,10 +276,58 @@ def test_activation_gradients_in_the_products(dev, dtype, M, N, K, accumulate):
     (test_rotation_in_the_products, (5, 1601, 8, 4, 64, 520, False, True)), (test_activation_gradients_in_the_products, (4097, 1376, 512, 1)),
     (test_activation_gradients_in_the_products, (8200, 1384, 520, None))], ids=lambda v: v.__name__[5:] if callable(v) else "-".join(map(str, v)))
 def test_larger_bf16_tiles(dev, check, args):
-    """The tiles of 128 rows, alone, with others in a launch and with what follows the products in them: remainders of rows, columns and slabs,
+    """The tiles of 128 rows (and of 64 where a size is planned on those: narrow contractions of 4001 and 12001 rows), alone, with others in a launch and
+    with what follows the products in them: remainders of rows, columns and slabs,
     rectangles of tiles that eight does not divide, columns that are not whole groups of four, split contractions, sequences shorter than
     a tile."""
     first = dict(form=args[0], M=args[1], N=args[2], K=args[3]) if check in (test_product_forms, test_product_into_rows_of_a_wider_buffer) else None
     names = {test_group_of_projections: ("rows", "hidden", "widths"), test_gate_up_in_one_launch: ("M", "N", "K", "keep"),
              test_rotation_in_the_products: ("B", "S", "H", "Hkv", "D", "K", "joint", "given"), test_activation_gradients_in_the_products: ("M", "N", "K", "accumulate")}
     check(dev=dev, dtype=torch.bfloat16, **(first or dict(zip(names[check], args))))
+
+
+def planned(items, dtype=_lib.MLTS_BF16, sharing=0):
+    """The tile (rows, columns) and the slices that a call takes for each (form, M, N, K[, row stride of C]); nothing is launched."""
+    ps, tiles = (GemmProduct * len(items))(), (GemmTiles * len(items))()
+    for p, (form, M, N, K, *ldc) in zip(ps, items):
+        p.form, p.segments, p.M, p.N, p.k[0], p.ldc = form, 1, M, N, K, ldc[0] if ldc else N
+        p.lda[0], p.ldb[0] = (M if form == TN else K), (K if form == NT else N)
+    _lib.check(_lib.lib().mlts_gemm_plan(ps, len(ps), dtype, sharing, tiles))
+    return [(t.tile_m, t.tile_n, t.slices) for t in tiles]
+
+
+# (form, M, N, K), the gap behind the rows of C, and the bf16 tile and slices that it is planned with: ragged rows, columns and slabs of each
+TILE_CASES = [
+    ((NN, 265, 2056, 4104), 0, (256, 128, 4)), ((NN, 521, 5464, 4104), 0, (256, 128, 1)), ((TN, 12008, 72, 8201), 0, (256, 128, 4)), ((TN, 136, 5464, 12001), 0, (256, 128, 4)),
+    ((TN, 4088, 2040, 3001), 48, (256, 128, 1)), ((NT, 12001, 76, 8200), 0, (256, 128, 4)), ((NT, 4547, 7657, 680), 0, (256, 256, 1)), ((NN, 4547, 7656, 680), 8, (256, 256, 1)),
+    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((NT, 12001, 140, 520), 4, (128, 64, 1)), ((NT, 3001, 260, 6008), 0, (128, 64, 2)), ((NN, 4033, 72, 2760), 0, (128, 64, 4)),
+    ((TN, 2336, 136, 4104), 0, (128, 64, 4)), ((NT, 2331, 1542, 512), 0, (128, 128, 1)), ((NN, 3001, 72, 6008), 0, (128, 128, 8)), ((TN, 520, 1384, 6008), 0, (128, 128, 4))]
+# (batch rows, tokens, heads, KV heads, head_dim, K, positions given) of q, k, v as one rotated product
+ROTATED_TILE_CASES = [((1, 863, 24, 8, 64, 2352, False), (128, 64, 1)), ((1, 5297, 12, 4, 64, 3000, False), (256, 128, 1)), ((11, 1091, 16, 4, 64, 1032, True), (256, 256, 1)),
+                      ((5, 1601, 8, 4, 64, 520, True), (128, 128, 1))]
+
+
+@pytest.mark.parametrize("product,gap,tile", TILE_CASES, ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_every_bf16_tile(dev, product, gap, tile):
+    """Each tile, whole and split, written and added onto, into dense rows and into rows of a wider buffer whose rest is not touched."""
+    form, M, N, K = product
+    assert planned([(*product, N + gap)]) == [tile]
+    a, b = operands(form, M, N, K, torch.bfloat16, dev, M + N)
+    want = expected(form, a, b)
+    for accumulate in (0, 1):
+        wide = torch.randn(M, N + gap, generator=torch.Generator().manual_seed(1)).bfloat16().to(dev)
+        before = wide.clone()
+        run_products([(form, [(a, b)], wide[:, :N], accumulate)], torch.bfloat16)
+        total = want + before[:, :N].double() * accumulate
+        assert (wide[:, :N].double() - total).norm() <= 4e-3 * total.norm() and torch.equal(wide[:, N:], before[:, N:])
+        first = wide.clone()
+        wide.copy_(before)
+        run_products([(form, [(a, b)], wide[:, :N], accumulate)], torch.bfloat16)
+        assert torch.equal(wide, first)
+
+
+@pytest.mark.parametrize("case,tile", ROTATED_TILE_CASES, ids=lambda v: "-".join(map(str, v)))
+def test_every_bf16_tile_rotated(dev, case, tile):
+    B, S, H, Hkv, D, K, given = case
+    assert planned([(NT, B * S, (H + 2 * Hkv) * D, K)], sharing=1) == [tile]
+    test_rotation_in_the_products(dev, torch.bfloat16, B, S, H, Hkv, D, K, False, given)

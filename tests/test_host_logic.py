@@ -20,7 +20,7 @@ from maltos_amd.optim import FusedAdamW, MasterWeightsOptimizer
 from maltos_amd.ring_attention import zigzag_ring_schedule
 from maltos_amd.ring_layout import expected_zigzag_ring_positions, has_zigzag_ring_layout
 
-from .test_gpu_products import GemmProduct, GemmRotation, GemmTiles
+from .test_gpu_products import ROTATED_TILE_CASES, TILE_CASES, GemmProduct, GemmRotation, GemmTiles, planned
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -343,3 +343,12 @@ def test_rotated_products_are_planned_as_they_are_checked():
         assert (why is None) == all(t.slices == 1 for t in tiles), (M, [p.N for p in ps], K, dtype)
         split += why is not None
     assert 50 < split < 3950
+
+
+def test_products_that_test_a_tile_are_planned_on_it():
+    """The sizes of the GPU tests of each bf16 tile, so that other costs in the plan cannot move them off it unnoticed; all tiles are among them."""
+    for (form, M, N, K), gap, tile in TILE_CASES:
+        assert planned([(form, M, N, K, N + gap)]) == [tile], (form, M, N, K)
+    for (B, S, H, Hkv, D, K, _), tile in ROTATED_TILE_CASES:
+        assert planned([(0, B * S, (H + 2 * Hkv) * D, K)], sharing=1) == [tile], (B, S, H, Hkv, D, K)
+    assert {t[:2] for _, _, t in TILE_CASES} == {t[:2] for _, t in ROTATED_TILE_CASES} == {(128, 64), (128, 128), (256, 128), (256, 256)}
