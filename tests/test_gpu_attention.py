@@ -449,6 +449,14 @@ def test_head_dims_between_the_tuned_ones(dev, D, B, Hq, Hkv, Sq, Sk, mode):
             check(got, want, torch.bfloat16, f"result {i}")
 
 
+# causal: 936 and 1872 blocks of 16 keys and queries, i.e. two to a wavefront in all three kernels (head_dim 96: in the first two), rows past the last key and query in
+# the second block, several heads to a group; a walk of 1300 keys, and of 2200 queries by the keys of a group
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk", [(9, 16, 8, 205, 197), (1, 2, 1, 1100, 1300)])
+@pytest.mark.parametrize("D", [32, 96])
+def test_head_dims_between_the_tuned_ones_causal(dev, D, B, Hq, Hkv, Sq, Sk):
+    test_head_dims_between_the_tuned_ones(dev, D, B, Hq, Hkv, Sq, Sk, ops.MASK_CAUSAL)
+
+
 # 16-row blocks: 195, 1365 and 2145, i.e. eight, two and one wavefronts to a block, with a workgroup at the end that is partly empty
 @pytest.mark.parametrize("B,H", [(1, 3), (3, 7), (11, 3)])
 @pytest.mark.parametrize("D", [64, 60])
