@@ -1,6 +1,6 @@
-// bf16 attention on v_mfma_f32_16x16x32_bf16, head_dim 64 and 128: what attn_small.hip and attn_bwd_dkv64.hip share.  Scores are computed
-// transposed, walked rows x own rows: a lane then holds the probabilities of one own row and the next product takes them, rounded to bf16
-// once, from the registers they are in.
+// bf16 attention on v_mfma_f32_16x16x32_bf16: what attn_small.hip (head_dim 32, 64, 96 and 128) and attn_bwd_dkv64.hip (64) share.  Scores are computed
+// transposed, walked rows x own rows: a lane then holds the probabilities of one own row and the next product takes them from the registers
+// they are in, rounded to bf16 once (attn_small.hip at head_dim 32 and 96: in three parts).
 #pragma once
 #include "attn_rows.hpp"
 

@@ -1,5 +1,5 @@
 // bf16 attention at head_dim 64 and 128 on grids that leave most of the chip to few workgroups of the 32-row kernels (attn_fwd_dma.hip,
-// attn_bwd_dq_tr.hip, attn_bwd_split.hip).
+// attn_bwd_dq_tr.hip, attn_bwd_split.hip), and at head_dim 32 and 96 without documents (mlts_attn_small_serves_parts()).
 //
 // Those give a workgroup 128 or 256 rows and walk the other side 64 rows at a time, one tile behind the other at about a microsecond each:
 // with few rows and heads the kernel lasts as long as one workgroup's chain.  Here a wavefront owns R blocks of 16 rows (queries in the forward
@@ -10,8 +10,7 @@
 // the splits' sums meet at the end.  Scores are computed transposed, as in the fp32 kernels, so that a lane holds the probabilities of one
 // own row and the next product takes them, rounded to bf16 once, from the registers they are in.
 //
-// Documents: the plan's tile classes and visibility bits, as in the 32-row kernels.  At head_dim 32 and 96, without documents, all grids
-// (mlts_attn_small_serves_parts()).
+// Documents: the plan's tile classes and visibility bits, as in the 32-row kernels.
 #include "attn_bf16.hpp"
 
 namespace {
@@ -695,44 +694,45 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 // Which calls of a pass come here; the others go to the 32-row kernels.
 //
 // The chain a 32-row workgroup walks has to be long: from 512 rows of the other side on, where those kernels take 12 us and more.  Shorter
-// calls differ by 3 us and less (4 heads x 2 x 200: 8.4 us there, 5.5 here), which launching them hides; they keep one arithmetic for all
-// batch sizes, which a number of splits that depends on the grid does not have.
+// kernels differ by 4 us and less (4 heads x 2 x 200, by events: 10.4, 11.6 and 10.2 us there, 7.5, 7.3 and 7.7 here), which launching them hides: a forward and a
+// backward call of that size take 41 us in a row of them and 51 alone with either, the host's time for one being 41; they keep one arithmetic
+// for all batch sizes, which a number of splits that depends on the grid does not have.
 //
 // And the grid has to be small, for a block reads the other side for its 16 or 32 rows only.  us there -> here with one block of 16 rows to a
-// wavefront / with two, forward, dQ, dK/dV (causal; blocks: of 16 rows):
-//   head_dim 64    512 blocks  8 heads x 1023      22.7 -> 12.2 / 13.4   23.2 -> 12.5 / 14.3   21.5 -> 12.9 / 14.4
-//                  768         12 x 1024           22.3 -> 13.4 / 14.5   23.5 -> 14.4 / 17.3   21.2 -> 15.4 / 17.6
-//                  896         7 x 4 x 512         14.5 -> 12.1 / 12.1   16.1 -> 13.5 / 12.3   14.3 -> 14.7 / 12.8
-//                 1024         8 x 2048            37.4 -> 23.6 / 21.1   39.1 -> 21.5 / 20.4   37.4 -> 28.9 / 23.3
-//                 1176         3 x 8 x 777         18.5 -> 15.3 / 14.5   20.1 -> 17.5 / 16.3   20.5 -> 18.8 / 18.8
-//                 2048         4 x 8 x 1024        22.5 -> 22.0 / 20.5   24.0 -> 21.1 / 20.2   25.4 -> 28.3 / 23.1
-//                 2048         8 x 4096            67.5 -> 65.5 / 44     69.9 -> 60.2 / 47.7   77.3 -> 89.0 / 61.5
-//                 2560         10 x 8 x 512        15.8 -> 17.2 / 17.4   17.7 -> 20.5 / 19.2   18.5 -> 23.7 / 23.2
-//                 3072         3 x 8 x 2048        38.5 -> 46.6 / 36.5   41.1 -> 54.0 / 40.1   47.0 -> 76.3 / 48.5
-//                 4096         4 x 8 x 2048        39.7 -> 57.2 / 52.2   43.8 -> 65.7 / 47.6   53.3 -> 75.1 / 61.5
-//   head_dim 128   512         8 x 1023            27.4 -> 15.6 / 18.5   40.7 -> 17.1 / 21.2   35.7 -> 18.4
-//                 1024         2 x 8 x 1024        28.0 -> 21.9 / 20.5   40.7 -> 24.1 / 22.7   36.2 -> 27.1
-//                 1536         3 x 8 x 1024        28.4 -> 32.2 / 30.8   41.4 -> 35.8 / 34.9   36.9 -> 39.5
-//                 2048         2 x 8 x 2048        48.1 -> 58.5 / 45.7   71.7 -> 64.3 / 49.1   64.0 -> 80.1
-//                 3072         3 x 8 x 2048        54.8 -> 81.2 / 60.7   75.8 -> 93.4 / 69.4   68.8 ->  142
+// wavefront / with two, forward, dQ, dK/dV (causal; blocks: of 16 rows; medians of three runs of 30 calls, all in turn on one GPU):
+//   head_dim 64   512 blocks  8 heads x 1023     22.2 -> 13.2 / 14.6   23.9 -> 14.3 / 15.6   22.1 -> 13.5 / 15.1
+//                 768         12 x 1024          21.5 -> 13.7 / 15.1   22.9 -> 15.1 / 17.5   21.2 -> 16.1 / 17.7
+//                 896         7 x 4 x 512        14.5 -> 11.6 / 11.6   15.6 -> 13.1 / 11.9   14.1 -> 14.3 / 12.3
+//                1024         8 x 2048           36.9 -> 23.5 / 21.6   38.4 -> 22.0 / 20.8   36.7 -> 29.2 / 24.2
+//                1176         3 x 8 x 777        18.9 -> 16.0 / 15.6   20.7 -> 18.0 / 17.7   21.1 -> 20.0 / 19.7
+//                2048         4 x 8 x 1024       22.5 -> 22.7 / 20.8   24.3 -> 21.9 / 21.1   25.4 -> 29.0 / 24.8
+//                2048         8 x 4096           67.9 -> 64.8 / 42.5   70.2 -> 60.2 / 46.4   76.2 -> 87.3 / 58.3
+//                2560         10 x 8 x 512       15.9 -> 17.0 / 16.2   17.6 -> 20.2 / 18.6   18.5 -> 23.7 / 22.8
+//                3072         3 x 8 x 2048       38.8 -> 45.2 / 36.2   41.2 -> 52.6 / 39.2   47.3 -> 74.7 / 48.1
+//                4096         4 x 8 x 2048       39.4 -> 55.3 / 42.3   43.8 -> 63.2 / 46.8   52.3 -> 72.3 / 62.2
+//   head_dim 128  512         8 x 1023           27.2 -> 16.0 / 18.2   39.8 -> 18.0 / 20.9   35.2 -> 18.5
+//                1024         2 x 8 x 1024       28.5 -> 23.1 / 21.4   41.5 -> 25.2 / 24.0   37.5 -> 27.7
+//                1536         3 x 8 x 1024       28.8 -> 33.1 / 31.9   42.2 -> 37.3 / 36.2   38.2 -> 40.8
+//                2048         2 x 8 x 2048       49.2 -> 58.3 / 45.6   72.3 -> 64.0 / 48.7   65.2 -> 77.2
+//                3072         3 x 8 x 2048       55.2 -> 79.7 / 60.0   75.4 -> 92.0 / 67.8   67.6 ->  141
 // Without a mask a block's work is twice that of a causal one:
-//   head_dim 64    384         6 x 1024            20.4 -> 14.3 / 12.5   23.4 -> 14.9 / 12.8   20.2 -> 18.4 / 13.7
-//                 1024         2 x 8 x 1024        20.0 -> 18.7 / 16.9   23.0 -> 19.1 / 17.4   20.5 -> 23.7 / 20.2
-//                 1536         2 x 6 x 2048        35.8 -> 41.4 / 33.1   39.7 -> 44.4 / 33.9   46.9 -> 54.9 / 42.7
-//                 1536         6 x 8 x 512         14.1 -> 16.6 / 15.7   15.7 -> 17.9 / 16.9   17.6 -> 20.1 / 19.7
-//   head_dim 128   512         8 x 1024            25.3 -> 20.3 / 18.1   39.9 -> 21.7 / 20.5   34.6 -> 24.8
-//                 1024         8 x 2048            44.6 -> 50.7 / 38.9   69.9 -> 56.6 / 42.9   63.1 -> 68.0
-//                 1536         6 x 4096            84.9 ->  138 / 98.9    132 ->  153 /  107    122 ->  186
-// So two blocks from 832 (384 without a mask) on, short walks apart (8 x 32 heads x 64, head_dim 32, forward 7.3 / 8.9), and long walks, where a 32-row workgroup's chain is longest, up to larger grids.  Several
-// query heads to a KV head lengthen the walk of dK/dV: 2 x 16 (4) heads x 1500 96.1 -> 48.7 / 38.7, 16 (4) x 2048 123 -> 47.3 / 45.9.
+//   head_dim 64   384         6 x 1024           20.3 -> 14.1 / 12.9   22.5 -> 15.2 / 13.1   20.1 -> 18.6 / 14.0
+//                1024         2 x 8 x 1024       20.3 -> 18.6 / 17.6   22.9 -> 20.3 / 17.9   21.0 -> 24.1 / 20.1
+//                1536         2 x 6 x 2048       35.5 -> 39.9 / 32.2   39.4 -> 42.8 / 33.5   45.6 -> 53.3 / 42.6
+//                1536         6 x 8 x 512        13.6 -> 16.5 / 16.3   15.9 -> 18.6 / 17.6   17.4 -> 20.8 / 20.8
+//   head_dim 128  512         8 x 1024           25.8 -> 20.1 / 18.8   40.1 -> 22.2 / 21.8   35.3 -> 24.7
+//                1024         8 x 2048           45.6 -> 50.2 / 38.3   70.5 -> 55.6 / 42.3   64.0 -> 66.2
+//                1536         6 x 4096           90.3 ->  143 / 103     137 ->  159 / 111     129 ->  191
+// So two blocks from 832 (384 without a mask) on, short walks apart (8 x 32 heads x 64, head_dim 32, forward 6.8 / 7.9), and long walks, where a 32-row workgroup's chain is longest, up to larger grids.  Several
+// query heads to a KV head lengthen the walk of dK/dV: 2 x 16 (4) heads x 1500 95.2 -> 47.9 / 37.8, 16 (4) x 2048 123 -> 46.9 / 47.1.
 // (dK/dV of two blocks at head_dim 128 has no registers for its accumulators.)
 //
-// Documents stay with one block and smaller grids: what a row sees is not known here.  head_dim 64, 2 x 8 x 1023, pieces of 1 to 255, 16.8 -> 13.2
-// / 14.0, 17.5 -> 14.5 / 14.7, 18.5 -> 16.1 / 15.6; 4 x 4 x 2000 in pieces of about 100 15.6 -> 16.9 / 20.1, of 500 (2 x 8) 33.9 -> 28.3 / 25.1.
+// Documents stay with one block and smaller grids: what a row sees is not known here.  head_dim 64, documents of 64 to 446 rows, 2 x 8 x 1023, 17.0 -> 13.7,
+// 17.5 -> 14.4, 18.5 -> 15.8; of 50 to 136, 4 x 4 x 2000, 15.4 -> 16.8, 16.8 -> 19.2, 17.4 -> 22.6; of 64 to 936, 2 x 8 x 2000, 34.0 -> 28.8, 34.0 -> 32.2, 37.4 -> 35.6.
 //
-// Walks below 704 rows, the 32-row kernels' chains being short: head_dim 64 causal 5 x 8 x 512, 1280 blocks, dK/dV 15.0 -> 17.7 with two, 4 x 8 x 600 16.6 -> 17.2; unmasked
-// forward of 768, 3 x 8 x 512, 12.0 with one, 12.8 with two, dQ of 384, 3 x 4 x 512, 10.2 / 11.0; head_dim 128 causal dQ of 1280, 5 x 8 x 512, 25.8 -> 27.5, but
-// unmasked of 768 25.0 -> 20.8 with two.
+// Walks below 704 rows, the 32-row kernels' chains being short: head_dim 64 causal 5 x 8 x 512, 1280 blocks, dK/dV 15.1 -> 17.2 with two; unmasked forward of 768,
+// 3 x 8 x 512, 12.4 with one, 13.2 with two, dQ of 384, 3 x 4 x 512, 10.6 / 11.2; head_dim 128 causal dQ of 1280, 5 x 8 x 512, 25.6 -> 27.5, but unmasked of 768 25.7 -> 20.8
+// with two.
 constexpr int kShortWalk = 704, kLongWalk = 1408;
 struct Lines {
   int blocks[3];  // up to which a call is served: of short walks, between, of long ones
@@ -768,13 +768,21 @@ bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode,
 }
 
 // Whole passes at head_dim 32 and 96 without documents; bp: of the backward pass.  attn_tile16.hip, which takes rows at any alignment, shares 64-row
-// tiles between four wavefronts, which wait for each other twice a tile and walk a row's whole length (us there -> here, forward, dQ, dK/dV, causal):
-//   head_dim 32   8 heads x 1024      20.1 -> 11.2   20.8 -> 11.1   26.3 -> 12.3     96   32.0 -> 17.5   31.5 -> 18.0   38.4 -> 18.5
-//                 4 x 8 x 1024        23.7 -> 21.0   24.8 -> 21.6   31.1 -> 26.7          37.8 -> 31.8   41.0 -> 36.4   62.7 -> 49.3
-//                 8 x 16 x 1024       55.9 -> 53.7   60.7 -> 53.0   85.7 -> 72.3          96.3 -> 86.8    105 -> 94.6    164 -> 154
-//                 8 x 32 x 64          8.2 -> 7.3     8.1 -> 7.6     7.9 -> 7.3           11.2 -> 9.5    11.3 -> 9.6    10.7 -> 10.1
-//                 8 x 32 (8) x 300    16.7 -> 17.6   19.8 -> 19.0   31.9 -> 25.0          31.9 -> 28.1   36.9 -> 33.6   48.8 -> 40.2
-//   unmasked      8 x 8 x 1024        55.1 -> 46.7   57.7 -> 45.2   82.0 -> 64.4          93.1 -> 72.3    101 -> 76.6    143 -> 131
+// tiles between four wavefronts, which wait for each other twice a tile and walk a row's whole length (us there -> here, forward, dQ, dK/dV; head_dim 32, then 96):
+//   causal     8 x 1024           19.3 ->  9.7   19.3 ->  9.8   24.8 -> 11.6      31.6 -> 15.6   30.9 -> 16.7   37.9 -> 17.7
+//              4 x 8 x 1024       21.6 -> 18.5   21.7 -> 18.2   29.5 -> 24.2      36.2 -> 29.5   39.4 -> 31.5   59.5 -> 45.7
+//              8 x 16 x 1024      51.3 -> 48.1   55.6 -> 46.4   78.4 -> 62.4      92.7 -> 80.5    101 -> 90.1    158 ->  144
+//              8 x 32 x 64         8.1 ->  6.9    8.1 ->  6.9    8.0 ->  7.2      10.2 ->  9.2   11.4 ->  9.7   10.9 -> 10.0
+//              8 x 32 (8) x 300   15.9 -> 16.0   18.7 -> 17.2   30.8 -> 23.4      31.0 -> 27.6   36.3 -> 32.8   48.0 -> 39.7
+//              4 x 32 (8) x 300   13.4 -> 13.1   13.4 -> 13.0   30.0 -> 16.8      23.1 -> 22.1   25.6 -> 26.5   46.2 -> 28.0
+//              8 x 16 x 2048       164 ->  138    175 ->  134    263 ->  212       313 ->  272    341 ->  283    561 ->  522
+//              2 x 32 (8) x 2048  84.9 -> 85.1   91.6 -> 81.9    165 ->  115       158 ->  134    175 ->  147    355 ->  299
+//              16 x 8192           302 ->  305    331 ->  303    498 ->  415       576 ->  508    647 ->  554   1004 ->  949
+//              4 x 16 x 8192      1153 ->  988   1259 ->  999   1958 -> 1546      2250 -> 1910   2501 -> 2012   4226 -> 3858
+//   unmasked   8 x 8 x 1024       53.0 -> 45.1   55.8 -> 43.3   79.4 -> 61.9      96.5 -> 76.3    103 -> 78.5    148 ->  136
+//              4 x 16 x 4096       611 ->  508    656 ->  509   1016 ->  787      1145 ->  944   1270 -> 1007   2076 -> 1880
+// No grid up to 4 x 16 heads x 8192 is behind as a pass: two blocks share what a wavefront fetches, and it waits for nobody.  Single kernels are: by 1 % the
+// forward at head_dim 32 of grids whose 4096 wavefronts are twice what is resident, by 3 % dQ at head_dim 96 of 4 x 32 (8) x 300.
 // Errors against 64 bits as there or up to a fifth smaller (dQ, dK, dV in fp32, 300 to 1024 rows).
 bool mlts_attn_small_serves_parts(const AttnParams& p, int D, int mode, const AttnBwdParams* bp) {
   if ((D != 32 && D != 96) || mode == MLTS_MASK_DOC || p.Sq == 0 || p.Sk == 0) return false;

@@ -599,7 +599,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_kernel(c
 }
 
 // us in a training step, product and pass / rotated here: q, k, v of 1023 rows as one 1536 x 512 product 7.5 + 3.7 / 9.1; of 2331 rows as
-// three 11.9 + 4.0 / 12.8; of 16384 rows as one 32 (the library's selected kernel) + 15 / 44; fp32 of 2048 rows as three 256 x 256 12.8 + 3.9 / 14.1.
+// three 11.9 + 4.0 / 12.8; of 16384 rows as one 32 (the library's selected kernel) + 15 / 48; fp32 of 2048 rows as three 256 x 256 12.8 + 3.9 / 14.1.
 template <typename T, int BM, int BN, int WM, int WN, int KG>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_rope_kernel(const Product g, const Rotation rot) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -608,7 +608,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_rope_ker
 }
 
 // us, one product and the pass over gate and up / the pair / without gate and up (weights out of HBM, x just written): 1376 + 1376 x 512 bf16
-// 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 15.5 + 5.8 / 17.7 / 16.1, 16384 rows 72 (library) + 23 / 76 /;
+// 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 15.5 + 5.8 / 17.7 / 16.1, 16384 rows in a training step 80 (the library's selected kernel) + 23 / 82;
 // 688 + 688 x 256 fp32 2048 rows 20.1 + 4.8 / 20.9 / 18.9.
 template <typename T, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_pair_kernel(const Product g, const Pair pair) {
@@ -655,7 +655,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_multi_ro
 }
 
 // dW = dy^T h (if it is wanted), and dh = dy W on its way through the activation (1376 x 512, us: 1023 rows 13.4 and 5.1 for the pass /
-// 16.3 here; 16384 rows, dh alone, 34 to 50 (the library's) and 37 / 66)
+// 16.3 here; 16384 rows in a training step, dh alone, 47 (the library's selected kernel) and 37 / 71, with dW 48 and 6 more (row slices and their sum) / 103)
 template <typename T, int BM, int BN, int WM, int WN, int KG>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_multi_act_kernel(const Products ps, const Activation act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -786,7 +786,9 @@ int64_t divide(Product& g, int bm, int bn) {
 // bf16: tile and split by estimated time (us).  A launch takes `fixed`, then the longer of the chain of slabs of a workgroup and its work
 // shared by 256 CUs, then what is written; a split also the launch that joins the slices and their fp32 sums.  Fitted to 1100 products of 100 to
 // 12000 rows, 256 to 32000 columns and 256 to 2752 terms in the three forms, weights out of HBM: off by 7 % (rms), and the choice by 0.5 %
-// from the best of all tiles and splits.  What a workgroup fetches decides: loads alone, with neither LDS nor matrix instructions, take as
+// from the best of all tiles and splits.  Of 147 products of 16384 to 32768 rows, to which nothing was fitted, the choice is 3.6 % from the best on the mean and 13 % in
+// the worst tenth, mostly for want of a tile of 256 x 256 (y 16384 x 640 x 1720 81 us, 54 there).  Products that share a launch, pairs and those whose output goes through the
+// activation have tiles of 64 and of 128 rows only.  What a workgroup fetches decides: loads alone, with neither LDS nor matrix instructions, take as
 // long as the kernel (2048 x 2048 x 1536, tiles of 64 x 64: 29 us of 30.5), and a tile of 128 x 128 fetches half as much for its work
 // (us, 64 x 64 / 128 x 128: NT 2331 x 1536 x 512 12.0 / 9.4, 8192 x 2752 x 512 45.3 / 34.9, NN 16384 x 1376 x 512 48.8 / 36.5).
 struct TileCost {

@@ -402,11 +402,12 @@ struct Needed {
   std::vector<bool> weight;
 };
 
-// The input gradient, then one gradient per parameter, as far as they are needed: added into the gradient buffers where into_grad
-// allows it, and then undefined.  dy2: the outputs' gradients side by side.
 // M * N * K of each part up to which the input gradient of weights that are not adjacent is one contraction in parts: it runs on the small
 // tiles only, and beyond them the products and their sum one after the other are as fast
 constexpr double kOwnLimitParts = 4.0e9;
+
+// The input gradient, then one gradient per parameter, as far as they are needed: added into the gradient buffers where into_grad
+// allows it, and then undefined.  dy2: the outputs' gradients side by side.
 variable_list grads_of_all(const Adjacent& a, const std::vector<Tensor>& weights, bool into_grad, const Needed& need, const Tensor& x, const Tensor& dy2) {
   variable_list out(1 + weights.size());
   const Tensor x2 = rows2d(x);
