@@ -312,6 +312,7 @@ int mlts_gemm_multi(const mlts_gemm_product* products, int32_t count, int32_t dt
 #define MLTS_GEMM_WITH_GATE_UP 3
 typedef struct {
   int32_t tile_m, tile_n, slices, together;
+  int32_t busiest; /* tiles of the launch that the XCD with the most of them gets */
 } mlts_gemm_tiles;
 int mlts_gemm_plan(const mlts_gemm_product* products, int32_t count, int32_t dtype, int32_t with, mlts_gemm_tiles* tiles);
 /* The backward pass of h W^T (W [K, N], h = round(silu(gate)) * up) in one launch: dW (+)= dy^T h (dense; null: not wanted), and d gate,

@@ -130,9 +130,10 @@ struct Product {
   int M, N;
   int tiles_m, tiles_n, slices;
   int form, accumulate;
-  int xcds;  // log2 of the parts its slices, tile rows and tile columns are divided into for the eight XCDs, four bits each
+  int xcds;  // log2 of the parts its slices, tile rows and tile columns are divided into for the eight XCDs, four bits each; kRuns: a run of its tiles each
 };
 constexpr int kMaxProducts = 4;  // of a call
+constexpr int kRuns = -1;
 // Two NT products of one shape that share A and meet in the end (gate and up of an MLP): C = A B^T, C2 = A B2^T, h = round(silu(C)) * C2 of
 // the rounded C and C2; N, ldb and ldc are those of one of them.  C and C2 may be null.
 struct Pair {
@@ -228,18 +229,26 @@ struct MoreSegments {
 };
 
 // The tile of a workgroup.  Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its own: an XCD gets a rectangle of a
-// product's tiles (split contractions: of some of the slices), so that it reads few rows of A and few columns of B (divide()), and walks it along N.
+// product's tiles (split contractions: of some of the slices), so that it reads few rows of A and few columns of B, or a run of them (spread()), and walks
+// them along N.
 struct Tile {
   int slice, m, n;
   bool there;
   __device__ __forceinline__ Tile(const Product& g, int block) {
-    const int xcd = block & 7, ls = g.xcds & 15, lm = (g.xcds >> 4) & 15, ln = g.xcds >> 8;
-    const int xn = xcd & ((1 << ln) - 1), xm = (xcd >> ln) & ((1 << lm) - 1), xs = xcd >> (ln + lm);
-    const int n0 = (g.tiles_n * xn) >> ln, width = ((g.tiles_n * (xn + 1)) >> ln) - n0;
-    const int m0 = (g.tiles_m * xm) >> lm, height = ((g.tiles_m * (xm + 1)) >> lm) - m0;
-    const int s0 = (g.slices * xs) >> ls, depth = ((g.slices * (xs + 1)) >> ls) - s0;
-    int rest = block >> 3;
-    there = rest < width * height * depth;
+    const int xcd = block & 7;
+    int rest = block >> 3, n0 = 0, m0 = 0, s0 = 0, width = g.tiles_n, height = g.tiles_m, depth = g.slices;
+    if (g.xcds == kRuns) {
+      const int tiles = width * height * depth, per = tiles >> 3, more = tiles & 7;
+      there = rest < per + (xcd < more);
+      rest += xcd * per + min(xcd, more);
+    } else {
+      const int ls = g.xcds & 15, lm = (g.xcds >> 4) & 15, ln = g.xcds >> 8;
+      const int xn = xcd & ((1 << ln) - 1), xm = (xcd >> ln) & ((1 << lm) - 1), xs = xcd >> (ln + lm);
+      n0 = (g.tiles_n * xn) >> ln, width = ((g.tiles_n * (xn + 1)) >> ln) - n0;
+      m0 = (g.tiles_m * xm) >> lm, height = ((g.tiles_m * (xm + 1)) >> lm) - m0;
+      s0 = (g.slices * xs) >> ls, depth = ((g.slices * (xs + 1)) >> ls) - s0;
+      there = rest < width * height * depth;
+    }
     const int row = there ? rest / width : 0;
     n = n0 + rest - row * width;
     slice = depth > 1 ? row / height : 0;
@@ -767,7 +776,7 @@ double small_slices(const mlts_gemm_product* const* ps, int count, const SmallSh
   return longest;
 }
 
-// The rectangles of the eight XCDs (Tile), bm x bn the tile; returns the workgroups of the launch, eight times those of the largest one.
+// The rectangles of the eight XCDs (Tile), bm x bn the tile; returns the tiles of the largest one.
 int64_t divide(Product& g, int bm, int bn) {
   auto part = [](int64_t n, int l) { return (n + (int64_t{1} << l) - 1) >> l; };
   const int64_t mean = (static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices + 7) / 8;
@@ -780,7 +789,21 @@ int64_t divide(Product& g, int bm, int bn) {
       const double cost = static_cast<double>(depth * (rows * bm + columns * bn)) * static_cast<double>(std::max<int64_t>(tiles, 32)) / static_cast<double>(std::max<int64_t>(mean, 32));
       if (most == 0 || cost < best) most = tiles, best = cost, g.xcds = ls | lm << 4 | ln << 8;
     }
-  return most * 8;
+  return most;
+}
+
+// Divides the products of a launch; each: the tiles of an XCD, returns their sum.  In runs of equal length where the largest rectangles would give a CU of their XCD
+// one tile more: that costs more than what they save in L2.  (us, rectangles / runs, 33 to 36 tiles for the 32 CUs of an XCD and 32: bf16 NN 5352 x 768 x 768
+// 15.9 / 11.8, 2678 x 384 x 1488 11.7 / 9.4, dx and dW of 1407 x 640 x 3408 34.6 / 26.4; four on a CU for three: fp32 NN 1206 x 640 x 640 14.7 / 12.4.  Elsewhere
+// rectangles are ahead: NT 541 x 2304 x 768 7.4 / 8.9, 524 x 5456 x 1024 12.2 / 13.7.)
+int64_t spread(Product* ps, int count, int bm, int bn, int64_t* each) {
+  constexpr int64_t cus = 32;  // of an XCD
+  int64_t rectangles = 0, runs = 0;
+  const auto run_of = [](const Product& g) { return (static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices + 7) / 8; };
+  for (int i = 0; i < count; ++i) rectangles += each[i] = divide(ps[i], bm, bn), runs += run_of(ps[i]);
+  if ((rectangles + cus - 1) / cus <= (runs + cus - 1) / cus) return rectangles;
+  for (int i = 0; i < count; ++i) each[i] = run_of(ps[i]), ps[i].xcds = kRuns;
+  return runs;
 }
 
 // bf16: tile and split by estimated time (us).  A launch takes `fixed`, then the longer of the chain of slabs of a workgroup and its work
@@ -849,6 +872,8 @@ struct LaunchPlan {
   bool together[kMaxProducts] = {};  // in the launch of several products, all of one tile
   SmallShape shape;                  // of the small tile
   int64_t workspace = 0;             // bytes
+  int rows_of(int t) const { return t == kSmall ? shape.size : kTileM[t]; }
+  int columns_of(int t) const { return t == kSmall ? shape.size : kTileN[t]; }
   // activation: an NN product that is not split, whose output goes through the activation
   LaunchPlan(const mlts_gemm_product* ps, int count, int dtype, bool activation = false, bool rotation = false) : shape(dtype == MLTS_BF16 ? kBf16Shape : kF32Shape) {
     if (dtype == MLTS_BF16) plan_bf16(ps, count, activation, rotation);
@@ -912,6 +937,13 @@ struct LaunchPlan {
     std::fill(tile, tile + count, best), std::fill(together, together + count, true), std::copy(best_slices, best_slices + count, slices);
   }
 };
+
+// a product's tiles and slices as product i of a plan
+void set_tiles(Product& g, const mlts_gemm_product& p, const LaunchPlan& plan, int i, int dtype) {
+  const int bm = plan.rows_of(plan.tile[i]), bn = plan.columns_of(plan.tile[i]);
+  g.tiles_m = static_cast<int>((p.M + bm - 1) / bm), g.tiles_n = static_cast<int>((p.N + bn - 1) / bn);
+  set_slices(g, plan.slices[i], slabs_of(p, slab_of(dtype)), slab_of(dtype));
+}
 
 template <typename S>
 int opt_in_lds(MltsLdsOptIn& once, const void* kern, int bytes, S what) {
@@ -1072,15 +1104,20 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
   if (rotation) rot = *rotation;
   Products joint;
   Joins joins{};
-  int blocks, join_blocks = 0, together, joint_tile = kSmall;
+  int join_blocks = 0, together, joint_tile = kSmall;
   bool all_nt, all_nn;
   auto clear = [&] {
     joint = {};
     std::fill(joint.first, joint.first + kMaxProducts, 0x7fffffff);
-    blocks = together = 0, all_nt = all_nn = true;
+    together = 0, all_nt = all_nn = true;
   };
   auto launch = [&] {  // what `joint` holds
     if (!together) return static_cast<int>(MLTS_OK);
+    int64_t tiles[kMaxProducts], at = 0;  // of an XCD
+    const int64_t grid = 8 * spread(joint.p, together, plan.rows_of(joint_tile), plan.columns_of(joint_tile), tiles);
+    MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm: too many tiles");
+    for (int i = 0; i < together; ++i) joint.first[i] = static_cast<int>(at), at += 8 * tiles[i];  // (whole rounds over the XCDs, so that each product starts at the first)
+    const int blocks = static_cast<int>(grid);
     const int forms = joint.more.count ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
     if constexpr (sizeof(T) == 4) {
       if (plan.shape.size == 32) {
@@ -1101,18 +1138,14 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
   MltsKernelTimer timer("gemm", st);
   for (int i = 0; i < count; ++i) {
     const mlts_gemm_product& p = ps[i];
-    const bool small = plan.tile[i] == kSmall;
-    const int bm = small ? plan.shape.size : kTileM[plan.tile[i]], bn = small ? plan.shape.size : kTileN[plan.tile[i]];
+    const int bm = plan.rows_of(plan.tile[i]), bn = plan.columns_of(plan.tile[i]);
     Product g{};
     g.a = p.a[0], g.b = p.b[0], g.c = p.c;
     g.lda = static_cast<int>(p.lda[0]), g.ldb = static_cast<int>(p.ldb[0]), g.ldc = static_cast<int>(p.ldc), g.K = static_cast<int>(p.k[0]);
     g.form = p.form, g.accumulate = p.accumulate != 0;
     g.M = static_cast<int>(p.M), g.N = static_cast<int>(p.N);
-    g.tiles_m = static_cast<int>((p.M + bm - 1) / bm), g.tiles_n = static_cast<int>((p.N + bn - 1) / bn);
-    const int64_t slabs = slabs_of(p, slab_of(dtype));
-    set_slices(g, plan.slices[i], slabs, slab_of(dtype));
+    set_tiles(g, p, plan, i, dtype);
     if (g.tiles_m == 0 || g.tiles_n == 0) continue;
-    const int64_t grid = divide(g, bm, bn);
     if (p.segments > 1) {
       if (joint.more.count) {  // a launch has room for the segments of one product
         if (int rc = launch(); rc != MLTS_OK) return rc;
@@ -1125,7 +1158,6 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
       }
       joint.more.count = p.segments - 1, joint.more.product = together;
     }
-    MLTS_REQUIRE(blocks + grid < (int64_t{1} << 30), "mlts_gemm: too many tiles");
     if (plan.slices[i] > 1) {
       g.partial = workspace;
       workspace += p.M * p.N * plan.slices[i];
@@ -1135,11 +1167,14 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
     if (plan.together[i]) {
       joint_tile = plan.tile[i];
       all_nt = all_nt && p.form == FORM_NT, all_nn = all_nn && p.form == FORM_NN;
-      joint.first[together] = blocks;
       if (rotation) std::copy(rotation->columns[i], rotation->columns[i] + 4, rot.columns[together]);
-      blocks += static_cast<int>(grid);  // (whole rounds over the XCDs, so that each product starts at the first)
       joint.p[together++] = g;
-    } else if (rotation) {
+      continue;
+    }
+    int64_t tiles;
+    const int64_t grid = 8 * spread(&g, 1, bm, bn, &tiles);
+    MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm: too many tiles");
+    if (rotation) {
       Rotation own = *rotation;
       std::copy(rotation->columns[i], rotation->columns[i] + 4, own.columns[0]);
       if (int rc = launch_rope_alone<T>(plan.tile[i], plan.shape, g, own, static_cast<unsigned>(grid), st); rc != MLTS_OK) return rc;
@@ -1168,7 +1203,8 @@ template <typename T, int BM, int BN, int WM, int WN>
 int launch_pair(Product& g, const Pair& pair, hipStream_t st) {
   typedef TileShape<T, FORM_NT, BM, BN, WM, WN, 1, true> S;
   g.tiles_m = (g.M + BM - 1) / BM, g.tiles_n = (g.N + BN / 2 - 1) / (BN / 2);
-  const int64_t grid = divide(g, BM, BN);
+  int64_t tiles;
+  const int64_t grid = 8 * spread(&g, 1, BM, BN, &tiles);
   MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm_swiglu: too many tiles");
   auto kern = gemm_pair_kernel<T, BM, BN, WM, WN>;
   static MltsLdsOptIn once;
@@ -1210,14 +1246,26 @@ extern "C" int mlts_gemm_plan(const mlts_gemm_product* products, int32_t count, 
   if (with == MLTS_GEMM_WITH_GATE_UP) {
     const int tile = pair_tile(products[0].M, products[0].N, products[0].k[0], dtype);
     MLTS_REQUIRE(count == 1 && tile >= 0, "mlts_gemm_plan: gate and up of this size are not made in one launch");
-    tiles[0] = {kTileM[tile], kTileN[tile], 1, 0};
+    Product g{};
+    int64_t each;
+    g.tiles_m = static_cast<int>((products[0].M + kTileM[tile] - 1) / kTileM[tile]), g.tiles_n = static_cast<int>((2 * products[0].N + kTileN[tile] - 1) / kTileN[tile]), g.slices = 1;
+    tiles[0] = {kTileM[tile], kTileN[tile], 1, 0, static_cast<int32_t>(std::min<int64_t>(spread(&g, 1, kTileM[tile], kTileN[tile], &each), 0x7fffffff))};
     return MLTS_OK;
   }
   const LaunchPlan plan(products, count, dtype, with == MLTS_GEMM_WITH_ACTIVATION, with == MLTS_GEMM_WITH_ROTATION);
+  Product joint[kMaxProducts];
+  int64_t each[kMaxProducts];
+  int together = 0, joint_tile = kSmall;
   for (int i = 0; i < count; ++i) {
-    const bool small = plan.tile[i] == kSmall;
-    tiles[i] = {small ? plan.shape.size : kTileM[plan.tile[i]], small ? plan.shape.size : kTileN[plan.tile[i]], static_cast<int32_t>(plan.slices[i]), plan.together[i]};
+    Product g{};
+    set_tiles(g, products[i], plan, i, dtype);
+    const int bm = plan.rows_of(plan.tile[i]), bn = plan.columns_of(plan.tile[i]);
+    tiles[i] = {bm, bn, static_cast<int32_t>(plan.slices[i]), plan.together[i], static_cast<int32_t>(std::min<int64_t>(spread(&g, 1, bm, bn, each), 0x7fffffff))};
+    if (plan.together[i] && g.tiles_m && g.tiles_n) joint[together++] = g, joint_tile = plan.tile[i];
   }
+  const int64_t busiest = spread(joint, together, plan.rows_of(joint_tile), plan.columns_of(joint_tile), each);
+  for (int i = 0; i < count; ++i)
+    if (plan.together[i]) tiles[i].busiest = static_cast<int32_t>(std::min<int64_t>(busiest, 0x7fffffff));
   return MLTS_OK;
 }
 

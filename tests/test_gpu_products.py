@@ -107,7 +107,7 @@ class GemmProduct(ctypes.Structure):
 
 class GemmTiles(ctypes.Structure):
     """Mirror of `mlts_gemm_tiles`."""
-    _fields_ = [("tile_m", ctypes.c_int32), ("tile_n", ctypes.c_int32), ("slices", ctypes.c_int32), ("together", ctypes.c_int32)]
+    _fields_ = [("tile_m", ctypes.c_int32), ("tile_n", ctypes.c_int32), ("slices", ctypes.c_int32), ("together", ctypes.c_int32), ("busiest", ctypes.c_int32)]
 
 
 def run_products(products, dtype):
@@ -286,14 +286,51 @@ def test_larger_bf16_tiles(dev, check, args):
     check(dev=dev, dtype=torch.bfloat16, **(first or dict(zip(names[check], args))))
 
 
-def planned(items, dtype=_lib.MLTS_BF16, sharing=0):
-    """The tile (rows, columns) and the slices that a call takes for each (form, M, N, K[, row stride of C]); nothing is launched."""
+def plan_of(items, dtype, sharing):
+    """`mlts_gemm_plan` of (form, M, N, K[, row stride of C]); nothing is launched."""
     ps, tiles = (GemmProduct * len(items))(), (GemmTiles * len(items))()
     for p, (form, M, N, K, *ldc) in zip(ps, items):
         p.form, p.segments, p.M, p.N, p.k[0], p.ldc = form, 1, M, N, K, ldc[0] if ldc else N
         p.lda[0], p.ldb[0] = (M if form == TN else K), (K if form == NT else N)
     _lib.check(_lib.lib().mlts_gemm_plan(ps, len(ps), dtype, sharing, tiles))
-    return [(t.tile_m, t.tile_n, t.slices) for t in tiles]
+    return tiles
+
+
+def planned(items, dtype=_lib.MLTS_BF16, sharing=0):
+    """The tile (rows, columns) and the slices that a call takes for each."""
+    return [(t.tile_m, t.tile_n, t.slices) for t in plan_of(items, dtype, sharing)]
+
+
+def tiles_of_an_xcd(items, dtype, sharing=0):
+    """What the busiest of the eight gets of a launch, and what equal shares would give it."""
+    tiles, bk, shares = plan_of(items, dtype, sharing), 64 if dtype == _lib.MLTS_BF16 else 32, []
+    for (_, M, N, K), t in zip(items, tiles):
+        slabs = -(-K // bk)
+        slices = -(-slabs // -(-slabs // t.slices))
+        shares.append(-(-(-(-M // t.tile_m) * -(-N // t.tile_n) * slices) // 8))
+    return (tiles[0].busiest, sum(shares)) if tiles[0].together else (max(t.busiest for t in tiles), max(shares))
+
+
+# products and launches of dW and dx whose rectangles would give an XCD's 32 CUs 33 to 36 tiles, or 98 to 132 for 93 to 128: remainders of rows, columns and slices
+RUNS = [(_lib.MLTS_BF16, [(NN, 5352, 768, 768)]), (_lib.MLTS_BF16, [(NN, 2678, 384, 1488)]), (_lib.MLTS_BF16, [(NT, 1099, 848, 320)]), (_lib.MLTS_BF16, [(NT, 817, 2320, 640)]),
+        (_lib.MLTS_F32, [(NN, 1206, 640, 640)]), (_lib.MLTS_F32, [(TN, 2688, 384, 1159)]), (_lib.MLTS_F32, [(NN, 774, 320, 848)]), (_lib.MLTS_BF16, [(TN, 3408, 640, 1407), (NN, 1407, 640, 3408)]),
+        (_lib.MLTS_BF16, [(TN, 1152, 384, 1521), (NN, 1521, 384, 1152)]), (_lib.MLTS_F32, [(TN, 1704, 640, 1497), (NN, 1497, 640, 1704)]), (_lib.MLTS_F32, [(TN, 384, 384, 2191), (NN, 2191, 384, 384)])]
+
+
+@pytest.mark.parametrize("dtype,items", RUNS, ids=lambda v: {_lib.MLTS_BF16: "bf16", _lib.MLTS_F32: "fp32"}[v] if isinstance(v, int) else "-".join("x".join(map(str, i[1:])) for i in v))
+def test_tiles_in_runs_of_equal_length(dev, dtype, items):
+    busiest, share = tiles_of_an_xcd(items, dtype)
+    assert busiest == share
+    t = torch.bfloat16 if dtype == _lib.MLTS_BF16 else torch.float32
+    products, want = [], []
+    for form, M, N, K in items:
+        a, b = operands(form, M, N, K, t, dev, M)
+        c = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(t).to(dev)
+        want.append(expected(form, a, b) + c.double())
+        products.append((form, [(a, b)], c, 1))
+    run_products(products, t)
+    for (*_, c, _), w in zip(products, want):
+        assert (c.double() - w).norm() <= (4e-3 if t == torch.bfloat16 else 2e-6) * w.norm()
 
 
 # (form, M, N, K), the gap behind the rows of C, and the bf16 tile and slices that it is planned with: ragged rows, columns and slabs of each

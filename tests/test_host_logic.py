@@ -20,7 +20,7 @@ from maltos_amd.optim import FusedAdamW, MasterWeightsOptimizer
 from maltos_amd.ring_attention import zigzag_ring_schedule
 from maltos_amd.ring_layout import expected_zigzag_ring_positions, has_zigzag_ring_layout
 
-from .test_gpu_products import ROTATED_TILE_CASES, TILE_CASES, GemmProduct, GemmRotation, GemmTiles, planned
+from .test_gpu_products import ROTATED_TILE_CASES, TILE_CASES, GemmProduct, GemmRotation, GemmTiles, planned, tiles_of_an_xcd
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -352,3 +352,14 @@ def test_products_that_test_a_tile_are_planned_on_it():
     for (B, S, H, Hkv, D, K, _), tile in ROTATED_TILE_CASES:
         assert planned([(0, B * S, (H + 2 * Hkv) * D, K)], sharing=1) == [tile], (B, S, H, Hkv, D, K)
     assert {t[:2] for _, _, t in TILE_CASES} == {t[:2] for _, t in ROTATED_TILE_CASES} == {(128, 64), (128, 128), (256, 128), (256, 256)}
+
+
+def test_no_xcd_gets_a_tile_a_cu_more_than_its_share():
+    """The eight XCDs get rectangles of a launch's tiles, but none whose 32 CUs would have to work off one tile each more than with equal shares (5352 x 768 x 768: 36
+    tiles for 32)."""
+    rng = random.Random(9)
+    for _ in range(4000):
+        dtype, rows, i, o = rng.choice([_lib.MLTS_BF16, _lib.MLTS_F32]), int(2 ** rng.uniform(0, 14)), 8 * rng.randint(1, 256), 8 * rng.randint(1, 512)
+        for items in ([(0, rows, o, i)], [(1, rows, i, o)], [(2, o, i, rows)], [(2, o, i, rows), (1, rows, i, o)]):
+            busiest, share = tiles_of_an_xcd(items, dtype)
+            assert -(-busiest // 32) <= -(-share // 32), (dtype, items, busiest, share)
