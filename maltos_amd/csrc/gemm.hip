@@ -806,61 +806,65 @@ int64_t spread(Product* ps, int count, int bm, int bn, int64_t* each) {
   return runs;
 }
 
-// bf16: tile and split by estimated time (us).  A launch takes `fixed`, then the longer of the chain of slabs of a workgroup and its work
-// shared by 256 CUs, then what is written; a split also the launch that joins the slices and their fp32 sums.  Fitted to 1100 products of 100 to
-// 12000 rows, 256 to 32000 columns and 256 to 2752 terms in the three forms, weights out of HBM: off by 7 % (rms), and the choice by 0.5 %
-// from the best of all tiles and splits.  Of 147 products of 16384 to 32768 rows, to which nothing was fitted, the choice is 3.6 % from the best on the mean and 13 % in
-// the worst tenth, mostly for want of a tile of 256 x 256 (y 16384 x 640 x 1720 81 us, 54 there).  Products that share a launch, pairs and those whose output goes through the
-// activation have tiles of 64 and of 128 rows only.  What a workgroup fetches decides: loads alone, with neither LDS nor matrix instructions, take as
+// bf16: tile and split by estimated time (us).  A launch takes `fixed`, then what the CU with the most workgroups takes for their slabs, one after the
+// other, then what is written; a split also the launch that joins the slices and their fp32 sums.  Fitted to 900 products in the three forms, 3 to 32000 rows, 64
+// to 4096 wide, 2e6 to 2.4e10 multiplications, each on all tiles and splits; of 900 others it is off by 9 % (rms), and the choice by 0.6 % from the best (1 % of them by
+// more than 11 %); of 500 launches of dW and dx by 2.3 %, 1.5 of them because a weight gradient keeps the split that it has alone.
+// What a workgroup fetches decides: loads alone, with neither LDS nor matrix instructions, take as
 // long as the kernel (2048 x 2048 x 1536, tiles of 64 x 64: 29 us of 30.5), and a tile of 128 x 128 fetches half as much for its work
 // (us, 64 x 64 / 128 x 128: NT 2331 x 1536 x 512 12.0 / 9.4, 8192 x 2752 x 512 45.3 / 34.9, NN 16384 x 1376 x 512 48.8 / 36.5).
 struct TileCost {
-  double fixed, chain, busy, out;  // out: of a million elements
+  double fixed, slab, out;  // out: of a million elements
 };
-constexpr TileCost kBf16Cost[kTiles] = {{3.6, 0.285, 0.26, 0.26}, {4.5, 0.54, 0.68, 0.28}, {6.7, 0.73, 1.25, 0.42}, {9.7, 1.2, 2.1, 0.48}, {4.4, 0.38, 0.405, 0.4}};
-constexpr double kJoinFixed = 4.2, kJoinSums = 0.97;  // ... of a million partial sums
-// What a pass on the way out adds, on small tiles and on larger ones, whose fewer wavefronts have less to overlap its latency with: of a launch,
-// of a million elements.  (us, 64 x 64 / 128 x 128: three rotated products of 512 x 512, 300 rows 7.8 / 12.6, 2331 13.2 / 14.1, 4096 18.2 / 15.8;
-// gate, up and activation of 1376 x 512, 300 rows 6.7 / 10.3, 1536 15.3 / 15.9, 2331 19.4 / 17.7, 8192 50 / 42; d gate and d up of it 300 rows
-// 8.5 / 14.6, 4096 29.8 / 29.2, 8192 56 / 45)
+constexpr TileCost kBf16Cost[kTiles] = {{2.5, 0.24, 0.55}, {3.2, 0.52, 0.55}, {3.95, 0.83, 0.69}, {6.2, 1.26, 0.56}, {3.1, 0.373, 0.71}};
+constexpr double kJoinFixed = 2.55, kJoinSums = 1.73;  // ... of a million partial sums
+// What a pass on the way out adds on each tile: of a launch, of a million elements; the larger ones have fewer wavefronts to overlap its latency with.  (Fitted to 250
+// rotated products, 170 launches of three, 400 pairs and 300 launches of dW and dh, the choice 0.3, 0.1, 0.3 and 0.9 % from the best.)
 struct PassCost {
-  double fixed[2], out[2];
+  double fixed[kTiles], out[kTiles];
 };
-constexpr PassCost kRotationCost{{0.3, 2.5}, {0, 0}}, kPairCost{{1.8, 4.2}, {0, 0}}, kActivationCost{{2.0, 5.5}, {2.1, 1.6}};
-double pass_time(const PassCost& c, int tile, int64_t M, int64_t N) {
-  const int larger = tile != kSmall;
-  return c.fixed[larger] + c.out[larger] * 1e-6 * static_cast<double>(M) * static_cast<double>(N);
-}
+constexpr PassCost kRotationCost{{1.0, 1.7, 3.9, 7.2, 1.8}, {0, 0.16, 0.35, 0.38, 0.06}},
+    kJointRotationCost{{1.0, 3.7}, {0, 0.16}}, kPairCost{{0.7, 1.5}, {0.5, 0.8}}, kActivationCost{{1.9, 4.0}, {1.8, 1.3}};
+constexpr TileCost kRotationApart{2.0, 0, 0.6};  // a launch of its own, after a split product (110 of the two, in a graph: 0.7 % from the best)
+double pass_time(const PassCost& c, int tile, int64_t M, int64_t N) { return c.fixed[tile] + c.out[tile] * 1e-6 * static_cast<double>(M) * static_cast<double>(N); }
 
 // The time of products in one launch, the slices of each given
 double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const int64_t* slices) {
   const TileCost& c = kBf16Cost[tile];
-  double longest = 0, work = 0, out = 0, sums = 0;
+  double longest = 0, work = 0, workgroups = 0, out = 0, sums = 0;
+  int64_t of_an_xcd = 0;
   for (int i = 0; i < count; ++i) {
-    const double part = static_cast<double>((slabs_of(*ps[i], 64) + slices[i] - 1) / slices[i]), elements = 1e-6 * static_cast<double>(ps[i]->M) * static_cast<double>(ps[i]->N);
-    longest = std::max(longest, part);
-    work += part * static_cast<double>(slices[i] * tiles_of(ps[i]->M, ps[i]->N, kTileM[tile], kTileN[tile]));
+    const int64_t slabs = slabs_of(*ps[i], 64), part = (slabs + slices[i] - 1) / slices[i];
+    const int64_t tiles = tiles_of(ps[i]->M, ps[i]->N, kTileM[tile], kTileN[tile]) * (part ? (slabs + part - 1) / part : 1);
+    const double elements = 1e-6 * static_cast<double>(ps[i]->M) * static_cast<double>(ps[i]->N);
+    longest = std::max(longest, static_cast<double>(part));
+    work += static_cast<double>(part) * static_cast<double>(tiles), workgroups += static_cast<double>(tiles);
+    of_an_xcd += (tiles + 7) / 8;
     (slices[i] > 1 ? sums : out) += elements * static_cast<double>(slices[i] > 1 ? slices[i] : 1);
   }
-  return c.fixed + std::max(longest * c.chain, work / 256 * c.busy) + out * c.out + (sums > 0 ? kJoinFixed + kJoinSums * sums : 0);
+  const double of_a_cu = static_cast<double>((of_an_xcd + 31) / 32);
+  const double slabs = workgroups > 0 ? std::max(longest, work / workgroups * of_a_cu) : 0;
+  return c.fixed + slabs * c.slab + out * c.out + (sums > 0 ? kJoinFixed + kJoinSums * sums : 0);
 }
 
-// The best tile and split of a product that runs alone.  (A contraction of 64 slabs and more on few tiles: 256 x 128 in as many parts as fill the
-// chip, which the estimate has no data for.  NN 1023 x 512 x 32000 in 16 parts 45 us, unsplit 210.)
-int choose_bf16_tile(const mlts_gemm_product& p, int64_t* slices) {
-  const int64_t slabs = slabs_of(p, 64), t2 = tiles_of(p.M, p.N, 256, 128);
+// ... of a product in a launch by itself, its outputs rotated on their way out (split, by a launch after it) or not
+double alone_time(const mlts_gemm_product& p, int tile, int64_t slices, bool rotation) {
+  const mlts_gemm_product* const one = &p;
+  const double time = bf16_time(&one, 1, tile, &slices);
+  if (!rotation) return time;
+  return time + (slices == 1 ? pass_time(kRotationCost, tile, p.M, p.N) : kRotationApart.fixed + kRotationApart.out * 1e-6 * static_cast<double>(p.M) * static_cast<double>(p.N));
+}
+
+// The best tile and split of a product that runs alone
+int choose_bf16_tile(const mlts_gemm_product& p, int64_t* slices, bool rotation) {
+  const int64_t slabs = slabs_of(p, 64);
   *slices = 1;
   if (p.segments > 1) return kSmall;
-  if (slabs >= 64 && t2 < 256 && t2 * (slabs / 8) >= 192 && p.form == FORM_NN) {
-    while (splittable(p) && t2 * *slices * 2 <= 256 && slabs / (*slices * 2) >= 8) *slices *= 2;
-    return k256x128;
-  }
-  const mlts_gemm_product* const one = &p;
   int best = kSmall;
   double least = 0;
   for (int tile = 0; tile < kTiles; ++tile)
     for (int64_t s = 1; s == 1 || (splittable(p) && s <= 16 && slabs / s >= 4); s *= 2) {
-      const double t = bf16_time(&one, 1, tile, &s);
+      const double t = alone_time(p, tile, s, rotation);
       if (least == 0 || t < least) least = t, best = tile, *slices = s;
     }
   return best;
@@ -904,23 +908,18 @@ struct LaunchPlan {
     const mlts_gemm_product* all[kMaxProducts];
     double apart = 0;
     int joins = 0;
+    int64_t columns = 0;  // of the products of a rotated call, which share their rows
     bool parts = false;
     for (int i = 0; i < count; ++i) {
       all[i] = &ps[i];
-      tile[i] = choose_bf16_tile(ps[i], &slices[i]);
-      apart += bf16_time(&all[i], 1, tile[i], &slices[i]) + (rotation ? pass_time(kRotationCost, tile[i], 0, 0) : 0);
+      tile[i] = choose_bf16_tile(ps[i], &slices[i], rotation);
+      apart += alone_time(ps[i], tile[i], slices[i], rotation);
+      columns += ps[i].N;
       joins += slices[i] > 1;
       parts = parts || ps[i].segments > 1;
     }
     apart -= joins > 1 ? (joins - 1) * kJoinFixed : 0;  // one launch joins them all
-    if (count == 1 && !parts && !activation) {
-      if (rotation && slices[0] == 1)
-        for (int t = 0; t < kTiles; ++t) {
-          const auto time = [&](int at) { return bf16_time(all, 1, at, slices) + pass_time(kRotationCost, at, 0, 0); };
-          if (time(t) < time(tile[0])) tile[0] = t;
-        }
-      return;
-    }
+    if (count == 1 && !parts && !activation) return;
     double least = 0;
     int best = -1;
     int64_t best_slices[kMaxProducts], s[kMaxProducts];
@@ -928,7 +927,7 @@ struct LaunchPlan {
       if (t != kSmall && parts) continue;
       for (int64_t dx = 1; dx <= (activation ? 1 : 4); dx *= 2) {
         for (int i = 0; i < count; ++i) s[i] = ps[i].form == FORM_TN ? slices[i] : ps[i].form == FORM_NN && splittable(ps[i]) && slabs_of(ps[i], 64) / dx >= 4 ? dx : 1;
-        double time = bf16_time(all, count, t, s) + (rotation ? pass_time(kRotationCost, t, 0, 0) : 0);
+        double time = bf16_time(all, count, t, s) + (rotation ? pass_time(kJointRotationCost, t, ps[0].M, columns) : 0);
         if (activation) time += pass_time(kActivationCost, t, ps[count - 1].M, ps[count - 1].N);
         if (best < 0 || time < least) least = time, best = t, std::copy(s, s + count, best_slices);
       }

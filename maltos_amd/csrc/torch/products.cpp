@@ -62,16 +62,20 @@ bool larger_own_range_bf16(int form, int64_t M, int64_t N, int64_t K, Use use) {
   return use != Use::GATE_AND_UP || N % 256 || K % 64 || K <= 256 || K > 512 || tiles <= 256 || 10 * tiles < 8 * ((tiles + 255) / 256 * 256);
 }
 
-// In bf16 they also run for dx = dy W with so long a contraction that it is split over workgroups (dx of an lm_head, of a wide
-// MLP): the library does not split those.  Own over library's time, 256 to 8192 rows, 512 to 4096 wide: 32000 terms 0.17 to 0.79, 11008
-// terms 0.54 to 0.83, 8192 terms 0.42 to 0.98; with 4096 or 5504 terms 0.76 to 1.04 where fewer than 128 tiles of 256 x 128 leave more
-// than half of the CUs idle unsplit, but 1.05 and 1.12 for 128 tiles (2048 x 2048 x 5504 56.6 us against 53.8, 1024 x 4096 x 4096 46.1
-// against 41.1).
+// In bf16 they also run for dx = dy W with a long contraction over few outputs (dx of an lm_head, of a wide MLP), which is split over
+// workgroups where the tiles leave CUs idle: the library does not split those.  Own over library's time, 605 products of 64 to 20001 rows,
+// 256 to 4096 columns, 4e9 to 3e11 terms, by tiles of 256 x 128 (geometric mean, largest):
+//   2816 to 6144 terms    up to 32 0.71, 0.99    33 to 64 0.74, 0.91    65 to 128 0.87, 0.99    129 to 160 0.97, 1.22    161 to 256 1.03, 1.15    more 1.07, 1.33
+//   8192 to 50264 terms   up to 32 0.38, 0.63    33 to 64 0.52, 0.73    65 to 128 0.71, 0.91    129 to 160 0.94, 1.21    161 to 255 1.04, 1.18    256 1.00, 1.05    more 1.09, 1.33
+bool long_contraction_bf16(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
+  return K >= 2816 && (tiles <= 128 || (K >= 8192 && tiles == 256));
+}
+
 bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K, Use use) {
   const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
   if (dtype == MLTS_F32) return size <= kOwnLimitF32;
-  if (size <= kOwnLimitBf16 || larger_own_range_bf16(form, M, N, K, use)) return true;
-  return form == MLTS_GEMM_NN && (K >= 8192 || M * N < 128 * 256 * 128) && mlts_gemm_workspace_bytes(form, dtype, M, N, K) > 0;
+  return size <= kOwnLimitBf16 || larger_own_range_bf16(form, M, N, K, use) || (form == MLTS_GEMM_NN && long_contraction_bf16(M, N, K));
 }
 
 struct Sizes {

@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from maltos_amd import _lib
+from maltos_amd import _lib, ops  # (ops: the schemas of the operators)
 from maltos_amd._native import native
 
 pytestmark = pytest.mark.gpu
@@ -66,7 +66,9 @@ def test_products_left_to_the_library(dev):
     (NT, 6000, 1024, 1024, False), (NT, 12000, 1024, 1024, False), (NN, 12000, 1024, 1024, False), (NT, 4096, 1280, 1280, False), (NT, 6000, 1000, 1024, True),
     (NT, 16384, 2304, 768, True), (NT, 17000, 2304, 768, False), (NN, 16384, 512, 1536, True), (NT, 17000, 512, 1536, False), (NT, 8000, 512, 2048, True), (NT, 8192, 512, 2048, False),
     (TN, 1024, 1024, 12000, True), (TN, 1024, 1024, 16384, False), (TN, 1024, 1024, 20001, True), (TN, 512, 1376, 16384, False), (TN, 256, 680, 32768, True), (TN, 2752, 512, 12000, True),
-    (TN, 5456, 1024, 4096, False), (TN, 1024, 2728, 10000, True), (TN, 6912, 1280, 3000, False)])
+    (TN, 5456, 1024, 4096, False), (TN, 1024, 2728, 10000, True), (TN, 6912, 1280, 3000, False),
+    (NN, 2048, 2048, 2816, True), (NN, 2048, 2176, 2816, False), (NN, 4096, 1024, 2808, False), (NN, 1000, 4096, 8192, True), (NN, 4096, 2048, 8192, True), (NN, 4352, 2048, 8192, False),
+    (NN, 4096, 2048, 8184, False)])
 def test_which_large_products_the_own_kernels_take(dev, form, M, N, K, own):
     """Both sides of each line between them and the library."""
     a, b = (torch.zeros(s, dtype=torch.bfloat16, device=dev) for s in ((K, M) if form == TN else (M, K), (N, K) if form == NT else (K, N)))
@@ -335,12 +337,13 @@ def test_tiles_in_runs_of_equal_length(dev, dtype, items):
 
 # (form, M, N, K), the gap behind the rows of C, and the bf16 tile and slices that it is planned with: ragged rows, columns and slabs of each
 TILE_CASES = [
-    ((NN, 265, 2056, 4104), 0, (256, 128, 4)), ((NN, 521, 5464, 4104), 0, (256, 128, 1)), ((TN, 12008, 72, 8201), 0, (256, 128, 4)), ((TN, 136, 5464, 12001), 0, (256, 128, 4)),
+    ((NN, 521, 2056, 8200), 0, (256, 128, 4)), ((NN, 1033, 5464, 520), 0, (256, 128, 1)), ((TN, 12008, 72, 8201), 0, (256, 128, 4)), ((TN, 136, 5464, 12001), 0, (256, 256, 8)),
     ((TN, 4088, 2040, 3001), 48, (256, 128, 1)), ((NT, 12001, 76, 8200), 0, (256, 128, 4)), ((NT, 4547, 7657, 680), 0, (256, 256, 1)), ((NN, 4547, 7656, 680), 8, (256, 256, 1)),
-    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((NT, 12001, 140, 520), 4, (128, 64, 1)), ((NT, 3001, 260, 6008), 0, (128, 64, 2)), ((NN, 4033, 72, 2760), 0, (128, 64, 4)),
-    ((TN, 2336, 136, 4104), 0, (128, 64, 4)), ((NT, 2331, 1542, 512), 0, (128, 128, 1)), ((NN, 3001, 72, 6008), 0, (128, 128, 8)), ((TN, 520, 1384, 6008), 0, (128, 128, 4))]
+    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((NN, 2336, 1032, 8200), 0, (256, 256, 4)), ((NT, 4033, 516, 8200), 0, (256, 256, 4)), ((NT, 1033, 1029, 520), 3, (128, 64, 1)),
+    ((NT, 3001, 260, 8200), 0, (128, 64, 2)), ((NN, 521, 520, 4104), 0, (128, 64, 4)), ((TN, 2336, 136, 8201), 0, (128, 64, 4)), ((TN, 1032, 136, 8201), 0, (128, 64, 8)),
+    ((NT, 2331, 1542, 512), 0, (128, 128, 1)), ((NN, 3001, 72, 6008), 0, (128, 128, 8)), ((TN, 520, 1384, 6008), 0, (128, 128, 4))]
 # (batch rows, tokens, heads, KV heads, head_dim, K, positions given) of q, k, v as one rotated product
-ROTATED_TILE_CASES = [((1, 863, 24, 8, 64, 2352, False), (128, 64, 1)), ((1, 5297, 12, 4, 64, 3000, False), (256, 128, 1)), ((11, 1091, 16, 4, 64, 1032, True), (256, 256, 1)),
+ROTATED_TILE_CASES = [((1, 863, 16, 4, 64, 1032, False), (128, 64, 1)), ((1, 5297, 12, 4, 64, 3000, False), (256, 128, 1)), ((7, 757, 24, 8, 64, 1032, True), (256, 256, 1)),
                       ((5, 1601, 8, 4, 64, 520, True), (128, 128, 1))]
 
 
