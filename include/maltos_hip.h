@@ -154,6 +154,10 @@ int mlts_attn_bwd_noalloc(const mlts_attn_shape* s, const void* dout, const int6
                           const int64_t dq_stride[3], void* dk, const int64_t dk_stride[3], void* dv,
                           const int64_t dv_stride[3], int accumulate_f32, mlts_stream_t stream);
 
+/* Which splits a pass of bf16 attention takes over wavefronts with two blocks of 16 rows each; host only.  pass: 0 forward, 1 dQ, 2 dK/dV;
+   blocks: pairs of row blocks, of all heads; units: of 32 rows, that each walks. */
+int32_t mlts_attn_small_splits(int32_t pass, int32_t head_dim, int64_t blocks, int64_t units);
+
 /* Log-sum-exp merge of one block into the running fp32 state, rows [q_off, q_off + q_len):
  *   lse' = logaddexp(lse, lse_b); out' = out * exp(lse - lse') + out_b * exp(lse_b - lse'),
  * with exp(-inf - x) := 0 (a row where both are -inf becomes 0 with lse -inf).  Replaces

@@ -652,12 +652,41 @@ bool near(int64_t rows, const int64_t* stride) {  // offsets that row_of can for
   return rows < (1 << 24) && stride[2] < (1 << 23) && ((rows - 1 + kUnit) * stride[2] + 128) * 2 < (int64_t{1} << 32);
 }
 
-// Splits of two blocks: where they come out at just two wavefronts a SIMD, four of half the length are ahead if they all fit (forward at head_dim 64: 121
-// registers) or the walk is long (us, two / four: head_dim 64, 8 heads x 4096 forward 56 / 44, dQ 49 / 48, dK/dV 67 / 61, 16 (4) x 2048 forward 31 / 26,
-// but dQ 28 / 32, 4 x 8 x 1024 dQ 20 / 25; head_dim 128, 8 x 4096 forward 79 / 75).  From 2304 on they are not: 1504 blocks x 1500 forward 20.5 / 23.2.
-template <int R>
-int splits_of(int64_t blocks, int64_t units, bool all_fit) {
-  return splits_for(blocks, units, kMaxSplits, R == 2 && (all_fit || units >= 4096 / kUnit) ? 2304 : kResident);
+// Splits of two blocks.  What counts is how many wavefronts are there at once: a second round of them takes as long as the first.  Four splits are one wavefront
+// a SIMD to a workgroup, of which two (dK/dV, all of head_dim 128), three (dQ at head_dim 64: 3072 wavefronts) or four (forward at head_dim 64) fit; somewhat more than fit are
+// still ahead of two splits of twice the length, and long walks at any number.  Eight splits are ahead only if all fit, two workgroups to a CU where registers do not allow more.
+// us, two / four splits (blocks: of 32 rows; units: of 32 rows walked)
+//   head_dim 64, causal   forward 1200 blocks, 75 units 39.1 / 33.2    1254, 57 31.5 / 30.2    dQ 768, 32 19.8 / 18.7    832, 64 28.4 / 26.1    832, 32 19.5 / 21.8    900, 50 24.2 / 27.1
+//                         dQ 980, 70 30.1 / 32.6    1200, 75 38.9 / 37.2    1450, 145 71.0 / 64.0    dK/dV 828, 69 40.2 / 35.0    864, 32 24.6 / 26.0    1040, 104 68.8 / 51.2    1254, 57 47.9 / 40.1
+//   head_dim 128, causal  forward 640, 64 46.7 / 35.7    798, 57 42.1 / 40.6    900, 50 38.5 / 40.2    1008, 48 37.8 / 53.4    dQ 644, 46 40.2 / 35.3    672, 28 30.1 / 31.8    860, 43 37.1 / 41.1
+//                         dQ 896, 128 82.6 / 78.9    1024, 256 148 / 142    900, 50 41.2 / 45.0    1008, 48 41.0 / 54.2    1328, 83 67.4 / 74.7    unmasked, 740, 47 53.1 / 49.0
+// four / eight
+//   head_dim 64           forward 384, 64 25.3 / 24.4    522, 58 20.4 / 20.3    dQ 260, 45 19.5 / 24.3    470, 72 21.7 / 26.0    dK/dV 285, 220 75.9 / 81.5    384, 64 30.3 / 33.5
+//   head_dim 128          forward 246, 41 22.2 / 20.4    320, 64 37.5 / 45.5    474, 79 44.9 / 51.3    dQ 246, 41 22.5 / 23.0    320, 64 40.8 / 50.8    490, 35 30.1 / 38.8
+//   head_dim 32           forward 322, 46 21.9 / 21.4    dQ 273, 91 31.5 / 29.6    dK/dV 265, 53 29.3 / 32.1
+// A causal walk of several heads is uneven: eight of 128 units and more (dK/dV of 2 x 12 (3) x 1836, 345 blocks, 61.8 / 48.1, of 32 (8) x 2048, 512 blocks, 62.2 / 57.6).
+struct SplitLines {  // up to how many wavefronts: four splits, four of walks of so many units and more, eight, eight of walks of 128 units and more
+  int four, units, four_long, eight, eight_long;
+};
+constexpr SplitLines split_lines(AttnPass pass, int D) {
+  if (pass == ATTN_BWD_DKV) return {3328, 48, 6144, 2048, 4096};
+  if (D == 32) return {4092, 128, 4092, 4088, 4088};
+  if (D == 96) return {4092, 128, 4092, 2048, 2048};
+  if (pass == ATTN_FWD) return D == 64 ? SplitLines{6144, 128, 6144, 4096, 4096} : SplitLines{3072, 56, 4608, 2048, 2048};
+  return D == 64 ? SplitLines{3328, 75, 6144, 2048, 2048} : SplitLines{2624, 45, 3584, 2048, 2048};
+}
+int splits_of_two(AttnPass pass, int D, int64_t blocks, int64_t units) {
+  const SplitLines at = split_lines(pass, D);
+  const bool long_walk = units >= 128;
+  const int least = splits_for(blocks, units, kMaxSplits, 0);  // (that fill half of the chip)
+  if (blocks >= (long_walk ? 2304 : kResident) || units < 8) return least;
+  const int four = units < at.units ? at.four : long_walk ? std::max(at.four_long, 4608) : at.four_long;
+  if (units < 16 || 4 * blocks > four) return std::max(least, 2);
+  return std::max(least, units >= 32 && 8 * blocks <= (long_walk ? at.eight_long : at.eight) ? 8 : 4);
+}
+template <AttnPass PASS, int D, int R>
+int splits_of(int64_t blocks, int64_t units) {
+  return R == 2 ? splits_of_two(PASS, D, blocks, units) : splits_for(blocks, units, kMaxSplits);
 }
 
 template <int D, bool DOC, int R>
@@ -665,7 +694,7 @@ int fwd(AttnParams p, hipStream_t st) {
   p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   MltsKernelTimer timer("attn_fwd", st);
-  return launch_splits<attn_small_fwd<D, DOC, R>, kMaxSplits>(blocks, splits_of<R>(blocks, (p.Sk + kUnit - 1) / kUnit, D == 64), R * D * 64, 2 * Unit<D>::BYTES, st, p,
+  return launch_splits<attn_small_fwd<D, DOC, R>, kMaxSplits>(blocks, splits_of<ATTN_FWD, D, R>(blocks, (p.Sk + kUnit - 1) / kUnit), R * D * 64, 2 * Unit<D>::BYTES, st, p,
                                                               RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_fwd");
 }
 
@@ -675,7 +704,7 @@ int bwd_dq(AttnBwdParams bp, hipStream_t st) {
   p.nqt = (p.Sq + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(p.nqt) * p.B * p.Hq;
   MltsKernelTimer timer("attn_bwd_dq", st);
-  return launch_splits<attn_small_bwd_dq<D, DOC, R>, kMaxSplits>(blocks, splits_of<R>(blocks, (p.Sk + kUnit - 1) / kUnit, false), R * D * 64, 2 * Unit<D>::BYTES, st, bp,
+  return launch_splits<attn_small_bwd_dq<D, DOC, R>, kMaxSplits>(blocks, splits_of<ATTN_BWD_DQ, D, R>(blocks, (p.Sk + kUnit - 1) / kUnit), R * D * 64, 2 * Unit<D>::BYTES, st, bp,
                                                                  RowArgs(p, D, true, p.Hq, p.nqt), "mlts_attn_bwd");
 }
 
@@ -685,7 +714,7 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
   const int tiles = (p.Sk + 16 * R - 1) / (16 * R);
   const int64_t blocks = static_cast<int64_t>(tiles) * p.B * p.Hkv, units = static_cast<int64_t>((p.Sq + kUnit - 1) / kUnit) * (p.Hq / p.Hkv);
   MltsKernelTimer timer("attn_bwd_dkdv", st);
-  return launch_splits<attn_small_bwd_dkv<D, DOC, R>, kMaxSplits>(blocks, splits_of<R>(blocks, units, false), 2 * R * D * 64, 2 * Unit<D>::BYTES + 256, st, bp,
+  return launch_splits<attn_small_bwd_dkv<D, DOC, R>, kMaxSplits>(blocks, splits_of<ATTN_BWD_DKV, D, R>(blocks, units), 2 * R * D * 64, 2 * Unit<D>::BYTES + 256, st, bp,
                                                                   RowArgs(p, D, true, p.Hkv, tiles), "mlts_attn_bwd");
 }
 
@@ -712,7 +741,7 @@ int bwd_dkv(const AttnBwdParams& bp, hipStream_t st) {
 //                4096         4 x 8 x 2048       39.4 -> 55.3 / 42.3   43.8 -> 63.2 / 46.8   52.3 -> 72.3 / 62.2
 //   head_dim 128  512         8 x 1023           27.2 -> 16.0 / 18.2   39.8 -> 18.0 / 20.9   35.2 -> 18.5
 //                1024         2 x 8 x 1024       28.5 -> 23.1 / 21.4   41.5 -> 25.2 / 24.0   37.5 -> 27.7
-//                1536         3 x 8 x 1024       28.8 -> 33.1 / 31.9   42.2 -> 37.3 / 36.2   38.2 -> 40.8
+//                1536         3 x 8 x 1024       28.8 -> 33.1 / 31.9   42.2 -> 37.3 / 31.9   38.2 -> 40.8
 //                2048         2 x 8 x 2048       49.2 -> 58.3 / 45.6   72.3 -> 64.0 / 48.7   65.2 -> 77.2
 //                3072         3 x 8 x 2048       55.2 -> 79.7 / 60.0   75.4 -> 92.0 / 67.8   67.6 ->  141
 // Without a mask a block's work is twice that of a causal one:
@@ -782,7 +811,7 @@ bool mlts_attn_small_serves(AttnPass pass, const AttnParams& p, int D, int mode,
 //   unmasked   8 x 8 x 1024       53.0 -> 45.1   55.8 -> 43.3   79.4 -> 61.9      96.5 -> 76.3    103 -> 78.5    148 ->  136
 //              4 x 16 x 4096       611 ->  508    656 ->  509   1016 ->  787      1145 ->  944   1270 -> 1007   2076 -> 1880
 // No grid up to 4 x 16 heads x 8192 is behind as a pass: two blocks share what a wavefront fetches, and it waits for nobody.  Single kernels are: by 1 % the
-// forward at head_dim 32 of grids whose 4096 wavefronts are twice what is resident, by 3 % dQ at head_dim 96 of 4 x 32 (8) x 300.
+// forward at head_dim 32 of grids whose 4096 wavefronts are twice what is resident, by 3 % dQ at head_dim 96 of 4 x 32 (8) x 300, by 7 and 9 % forward and dQ there of 5 x 32 (8) x 120 (12.2, 13.2 us).
 // Errors against 64 bits as there or up to a fifth smaller (dQ, dK, dV in fp32, 300 to 1024 rows).
 bool mlts_attn_small_serves_parts(const AttnParams& p, int D, int mode, const AttnBwdParams* bp) {
   if ((D != 32 && D != 96) || mode == MLTS_MASK_DOC || p.Sq == 0 || p.Sk == 0) return false;
@@ -825,4 +854,9 @@ int mlts_attn_small_bwd_dkv(AttnBwdParams bp, int D, int mode, hipStream_t st) {
   if (D == 96) return bwd_dkv<96, false, 1>(bp, st);
   if (D == 64) return two_blocks(ATTN_BWD_DKV, bp.a, D, mode) ? bwd_dkv<64, false, 2>(bp, st) : bwd_dkv<64, false, 1>(bp, st);
   return bwd_dkv<128, false, 1>(bp, st);
+}
+
+// The splits of a pass whose wavefronts have two blocks of 16 rows each (blocks: pairs of them), walking units of 32 rows; nothing is launched
+extern "C" int32_t mlts_attn_small_splits(int32_t pass, int32_t head_dim, int64_t blocks, int64_t units) {
+  return splits_of_two(pass == 0 ? ATTN_FWD : pass == 1 ? ATTN_BWD_DQ : ATTN_BWD_DKV, head_dim, blocks, units);
 }

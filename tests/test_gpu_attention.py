@@ -1083,3 +1083,11 @@ def test_output_rows_off_a_16_byte_boundary(dev, D):
     for got, want in zip(ops.attention_backward(do, q, k, v, moved, lse, mask_mode=ops.MASK_CAUSAL),
                          ops.attention_backward(do, q, k, v, o, lse, mask_mode=ops.MASK_CAUSAL)):
         assert (got.double() - want.double()).norm() <= 2.0 ** -9 * want.double().norm()   # a bf16 result may round the other way
+
+
+# causal, wavefronts with two blocks: forward with two, four and eight splits at head_dim 128 (1008, 640 and, unmasked, 246 blocks of 32 rows) and four at 64 (1232); dQ with
+# two and four; dK/dV with four of more wavefronts than are there at once; last blocks and units that are cut
+@pytest.mark.parametrize("B,H,S,D,mode", [(3, 7, 1518, 128, ops.MASK_CAUSAL), (1, 10, 2041, 128, ops.MASK_CAUSAL), (1, 6, 1307, 128, ops.MASK_NONE), (1, 16, 2459, 64, ops.MASK_CAUSAL),
+                                          (1, 10, 1489, 64, ops.MASK_NONE)])
+def test_splits_of_two_blocks(dev, B, H, S, D, mode):
+    test_two_blocks_of_sixteen_rows_to_a_wavefront(dev, mode, B, H, H, S, S, D)

@@ -362,6 +362,18 @@ def test_splits_that_were_measured(items, plan):
     assert planned(items) == plan
 
 
+FORWARD, DQ, DKDV = range(3)
+
+
+@pytest.mark.parametrize("which,D,blocks,units,splits", [
+    (FORWARD, 128, 1008, 48, 2), (FORWARD, 128, 798, 57, 4), (FORWARD, 128, 640, 64, 4), (FORWARD, 128, 320, 64, 4), (FORWARD, 128, 246, 41, 8), (FORWARD, 64, 1200, 75, 4), (FORWARD, 64, 384, 64, 8),
+    (DQ, 128, 1008, 48, 2), (DQ, 128, 644, 46, 4), (DQ, 128, 896, 128, 4), (DQ, 128, 1024, 256, 4), (FORWARD, 32, 1024, 128, 4), (DQ, 128, 490, 35, 4), (DQ, 64, 342, 37, 4), (DQ, 64, 260, 45, 4), (DQ, 64, 900, 50, 2), (DQ, 64, 832, 64, 4), (DQ, 32, 273, 91, 8), (FORWARD, 96, 1024, 32, 2), (DKDV, 32, 2048, 128, 2),
+    (DKDV, 64, 475, 76, 4), (DKDV, 64, 345, 230, 8), (DKDV, 64, 1040, 104, 4), (DKDV, 64, 864, 32, 2), (DKDV, 32, 265, 53, 4)])
+def test_splits_of_two_blocks_do_not_overshoot_the_chip(which, D, blocks, units, splits):
+    """Either side of each line, as measured: so many wavefronts that most of them are there at once (3 x 7 heads x 1518 at head_dim 128, 1008 blocks: four splits 53 us, two 38)."""
+    assert _lib.lib().mlts_attn_small_splits(which, D, blocks, units) == splits
+
+
 def test_no_xcd_gets_a_tile_a_cu_more_than_its_share():
     """The eight XCDs get rectangles of a launch's tiles, but none whose 32 CUs would have to work off one tile each more than with equal shares (5352 x 768 x 768: 36
     tiles for 32)."""
