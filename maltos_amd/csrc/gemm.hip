@@ -817,6 +817,10 @@ struct TileCost {
   double fixed, slab, out;  // out: of a million elements
 };
 constexpr TileCost kBf16Cost[kTiles] = {{2.5, 0.24, 0.55}, {3.2, 0.52, 0.55}, {3.95, 0.83, 0.69}, {6.2, 1.26, 0.56}, {3.1, 0.373, 0.71}};
+// A second workgroup on a CU overlaps the first on 64 x 64, by so much a slab (us, 64 x 64 / 128 x 64, of 37 and 19 tiles to an XCD: NT 2331 x 512 x 512 6.5 / 6.95, NN 6.5 /
+// 6.95, dW and dx of it on 64 x 64 / 128 x 128 12.4 / 13.5).  Of 600 products and 200 launches of dW and dx the choice is 0.51 and 0.74 % from the best, 0.74 and 0.86 %
+// without it.  Launches with a pass, fitted without it, go without it.
+constexpr double kSmallOverlap = 0.06;
 constexpr double kJoinFixed = 2.55, kJoinSums = 1.73;  // ... of a million partial sums
 // What a pass on the way out adds on each tile: of a launch, of a million elements; the larger ones have fewer wavefronts to overlap its latency with.  (Fitted to 250
 // rotated products, 170 launches of three, 400 pairs and 300 launches of dW and dh, the choice 0.3, 0.1, 0.3 and 0.9 % from the best.)
@@ -829,7 +833,7 @@ constexpr TileCost kRotationApart{2.0, 0, 0.6};  // a launch of its own, after a
 double pass_time(const PassCost& c, int tile, int64_t M, int64_t N) { return c.fixed[tile] + c.out[tile] * 1e-6 * static_cast<double>(M) * static_cast<double>(N); }
 
 // The time of products in one launch, the slices of each given
-double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const int64_t* slices) {
+double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const int64_t* slices, bool pass) {
   const TileCost& c = kBf16Cost[tile];
   double longest = 0, work = 0, workgroups = 0, out = 0, sums = 0;
   int64_t of_an_xcd = 0;
@@ -843,14 +847,15 @@ double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const 
     (slices[i] > 1 ? sums : out) += elements * static_cast<double>(slices[i] > 1 ? slices[i] : 1);
   }
   const double of_a_cu = static_cast<double>((of_an_xcd + 31) / 32);
-  const double slabs = workgroups > 0 ? std::max(longest, work / workgroups * of_a_cu) : 0;
-  return c.fixed + slabs * c.slab + out * c.out + (sums > 0 ? kJoinFixed + kJoinSums * sums : 0);
+  const double overlap = tile == kSmall && of_a_cu > 1 && !pass ? kSmallOverlap : 0;
+  const double slabs = workgroups > 0 ? std::max(longest * c.slab, work / workgroups * (of_a_cu * c.slab - overlap)) : 0;
+  return c.fixed + slabs + out * c.out + (sums > 0 ? kJoinFixed + kJoinSums * sums : 0);
 }
 
 // ... of a product in a launch by itself, its outputs rotated on their way out (split, by a launch after it) or not
 double alone_time(const mlts_gemm_product& p, int tile, int64_t slices, bool rotation) {
   const mlts_gemm_product* const one = &p;
-  const double time = bf16_time(&one, 1, tile, &slices);
+  const double time = bf16_time(&one, 1, tile, &slices, rotation);
   if (!rotation) return time;
   return time + (slices == 1 ? pass_time(kRotationCost, tile, p.M, p.N) : kRotationApart.fixed + kRotationApart.out * 1e-6 * static_cast<double>(p.M) * static_cast<double>(p.N));
 }
@@ -927,7 +932,7 @@ struct LaunchPlan {
       if (t != kSmall && parts) continue;
       for (int64_t dx = 1; dx <= (activation ? 1 : 4); dx *= 2) {
         for (int i = 0; i < count; ++i) s[i] = ps[i].form == FORM_TN ? slices[i] : ps[i].form == FORM_NN && splittable(ps[i]) && slabs_of(ps[i], 64) / dx >= 4 ? dx : 1;
-        double time = bf16_time(all, count, t, s) + (rotation ? pass_time(kJointRotationCost, t, ps[0].M, columns) : 0);
+        double time = bf16_time(all, count, t, s, rotation || activation) + (rotation ? pass_time(kJointRotationCost, t, ps[0].M, columns) : 0);
         if (activation) time += pass_time(kActivationCost, t, ps[count - 1].M, ps[count - 1].N);
         if (best < 0 || time < least) least = time, best = t, std::copy(s, s + count, best_slices);
       }
@@ -1194,7 +1199,7 @@ int pair_tile(int64_t M, int64_t N, int64_t K, int dtype) {
   if (dtype == MLTS_F32) return plan.tile[0] == k256 || (plan.tile[0] == kSmall && plan.shape.size != 64) ? -1 : plan.tile[0];
   const mlts_gemm_product* const one = &both;
   const int64_t whole = 1;
-  const auto time = [&](int tile) { return bf16_time(&one, 1, tile, &whole) + pass_time(kPairCost, tile, M, N); };
+  const auto time = [&](int tile) { return bf16_time(&one, 1, tile, &whole, true) + pass_time(kPairCost, tile, M, N); };
   return time(k128) < time(kSmall) ? k128 : kSmall;
 }
 

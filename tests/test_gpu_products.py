@@ -339,7 +339,7 @@ def test_tiles_in_runs_of_equal_length(dev, dtype, items):
 TILE_CASES = [
     ((NN, 521, 2056, 8200), 0, (256, 128, 4)), ((NN, 1033, 5464, 520), 0, (256, 128, 1)), ((TN, 12008, 72, 8201), 0, (256, 128, 4)), ((TN, 136, 5464, 12001), 0, (256, 256, 8)),
     ((TN, 4088, 2040, 3001), 48, (256, 128, 1)), ((NT, 12001, 76, 8200), 0, (256, 128, 4)), ((NT, 4547, 7657, 680), 0, (256, 256, 1)), ((NN, 4547, 7656, 680), 8, (256, 256, 1)),
-    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((NN, 2336, 1032, 8200), 0, (256, 256, 4)), ((NT, 4033, 516, 8200), 0, (256, 256, 4)), ((NT, 1033, 1029, 520), 3, (128, 64, 1)),
+    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((NN, 2336, 1032, 8200), 0, (256, 256, 4)), ((NT, 4033, 516, 8200), 0, (256, 256, 4)), ((NT, 1033, 1029, 1032), 3, (128, 64, 1)),
     ((NT, 3001, 260, 8200), 0, (128, 64, 2)), ((NN, 521, 520, 4104), 0, (128, 64, 4)), ((TN, 2336, 136, 8201), 0, (128, 64, 4)), ((TN, 1032, 136, 8201), 0, (128, 64, 8)),
     ((NT, 2331, 1542, 512), 0, (128, 128, 1)), ((NN, 3001, 72, 6008), 0, (128, 128, 8)), ((TN, 520, 1384, 6008), 0, (128, 128, 4))]
 # (batch rows, tokens, heads, KV heads, head_dim, K, positions given) of q, k, v as one rotated product
