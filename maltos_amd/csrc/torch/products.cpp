@@ -41,8 +41,9 @@ constexpr double kOwnLimitBf16 = 4.0e9, kOwnLimitF32 = 3.0e9;
 //     whole 1024 rows, from 16384 rows on: 512 to 768 wide 16384 rows -14 to +20, 24576 -32 to +32, but 20020 rows -2 to -57; below, up to 2e10: 5456 x 1024 x 4096 +13 to +15,
 //     3072 x 1024 x 8192 +4 to +21; 64 tiles without slices: 6912 x 1280 x 3000 +21, 5456 x 1024 x 3000 -4 to -9; others up to 3e10: 1024 x 2728 x 10000 -55, 1280 x 1792 x 12000 -27.
 //     In one launch with dh = dy W and the activation -2 to -107 at all row counts up to 32768; that dh without its dW up to +74.
-// (With the shipped per-shape selection, 16384 rows, alone: y 512 x 512 19 us against 17, 1536 x 512 46 / 33, in a step rotated on its way out 48 / 32 + 15,
-// 512 x 1376 39 / 39, 2752 x 512 69 / 80; dW 512 x 1376 40 / 45, 1536 x 512 46 / 37, 2752 x 512 69 / 58.)  Products with the columns of a vocabulary (32000 x 512): 1023 rows
+// These were measured on tiles of 128 x 128 where 256 x 128 is taken since (y of 512 x 1376, 16384 rows, 39 us, now 34).
+// (With the shipped per-shape selection, 16384 rows, alone: y 512 x 512 17 us against 16, 1536 x 512 42 / 32, in a step rotated on its way out 48 / 32 + 15,
+// 512 x 1376 34 / 40, 2752 x 512 65 / 73; dW 512 x 1376 41 / 45, 1536 x 512 41 / 37, 2752 x 512 63 / 58.)  Products with the columns of a vocabulary (32000 x 512): 1023 rows
 // 54 / 49, 3000 rows 136 / 131.
 bool larger_own_range_bf16(int form, int64_t M, int64_t N, int64_t K, Use use) {
   const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
