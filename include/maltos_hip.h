@@ -340,7 +340,7 @@ const char* mlts_gemm_rope_supports(const mlts_gemm_product* products, int32_t c
 int mlts_gemm_rope(const mlts_gemm_product* products, int32_t count, int32_t dtype, const mlts_gemm_rotation* rotation, mlts_stream_t stream);
 /* gate = x W_gate^T, up = x W_up^T (W [N, K], x [M, K]) and h = round(silu(gate)) * up of the rounded gate and up (models/llama.py:205-206)
  * in one launch: the values of two products and mlts_swiglu_fwd_rows.  gate and up may be null (nobody reads them).  Sizes whose products
- * would be split (fp32: or are large) are not served: mlts_gemm_swiglu_supports says NULL, or why. */
+ * would be split (fp32: or are faster with a pass behind them) are not served: mlts_gemm_swiglu_supports says NULL, or why. */
 const char* mlts_gemm_swiglu_supports(int32_t dtype, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldc, int64_t ldh);
 int mlts_gemm_swiglu(int32_t dtype, int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx, const void* w_gate, const void* w_up,
                      int64_t ldw, void* gate, void* up, int64_t ldc, void* h, int64_t ldh, mlts_stream_t stream);

@@ -2,7 +2,7 @@
 //   NT  y  = x W^T      A [M, K], B [N, K]     both contiguous along the contraction
 //   NN  dx = dy W       A [M, K], B [K, N]
 //   TN  dW = dy^T x     A [K, M], B [K, N]     optionally added onto C, the contraction split over workgroups
-// in bf16 (v_mfma_f32_32x32x16_bf16) and fp32 (v_mfma_f32_32x32x2_f32: true fp32 products and sums).  fp32 accumulation, one
+// in bf16 (v_mfma_f32_32x32x16_bf16) and fp32 (v_mfma_f32_32x32x2_f32, or the bf16 instruction on elements in three parts: Multiply).  fp32 accumulation, one
 // rounding at the end.
 //
 // Why not the vendor library for these: through torch a product costs 18 us of host time whatever its size (a launch is 4), and
@@ -12,7 +12,7 @@
 // stages: while a slab is multiplied the next one is written to the other stage and the one after that is on its way from
 // memory, with one barrier per slab.  Loads go through buffer descriptors, whose bounds check supplies the zeros past the end
 // of an operand.  Rows along the contraction are padded by 16 bytes in LDS (16-byte fragment reads conflict free); rows along
-// M or N by 64 (transpose reads, bf16) or 32 bytes (4-byte reads, fp32).  The product is computed with the operands swapped, so
+// M or N by 64 (transpose reads, bf16) or 32 bytes (4-byte reads, fp32); those of parts are permuted instead, so that two tiles of 128 x 64 fit a CU.  The product is computed with the operands swapped, so
 // that a lane holds four neighbouring columns of one row of C, and leaves through LDS in whole row segments.
 #include "common.hpp"
 
@@ -27,40 +27,54 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kOutside = 0x80000000u;  // an offset past every operand (operands are smaller than 2 GiB)
 
-template <typename T>
-struct Elem;
-template <>
-struct Elem<bf16_t> {
-  static constexpr int BK = 64;    // contraction elements per slab: 128 bytes
-  static constexpr int STEP = 16;  // ... per fragment
-  static constexpr int PAD = 64;   // bytes behind a row along M / N
+// How a tile multiplies.  bf16: as it is.  fp32 whole: by fp32 matrix instructions (true fp32 products and sums).  fp32 in three parts: every element is the sum of three
+// bf16 values, 24 bits, and a product of two elements the sum of the six products of parts above 2^-24 of it, by bf16 matrix instructions with fp32 sums, which take 192 cycles for
+// what the fp32 ones take 512.  The product of both first parts has a sum of its own, so that it is rounded once in sixteen terms.  Errors against 64 bits, in three parts / whole: N(0, 1)
+// operands, 64 terms 0.5e-7 / 1.4e-7, 256 0.9e-7 / 2.9e-7, 2048 2.7e-7 / 8.1e-7, 8192 5.7e-7 / 16e-7; likewise with positive operands, operands of very different size, and small ones (1e-30).
+enum { BF16, F32_WHOLE, F32_PARTS };
+template <int KIND>
+struct Multiply {
   typedef bf16x8 frag;
+  static constexpr int STEP = 16;  // contraction elements of a fragment
   static __device__ __forceinline__ f32x16 mma(frag a, frag b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 };
 template <>
-struct Elem<float> {
-  static constexpr int BK = 32;
-  static constexpr int STEP = 8;
-  static constexpr int PAD = 32;
+struct Multiply<F32_WHOLE> {
   typedef f32x4 frag;
+  static constexpr int STEP = 8;
   static __device__ __forceinline__ f32x16 mma(frag a, frag b, f32x16 c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], c, 0, 0, 0);
     return c;
   }
 };
+// v as its parts: their sum is v, unless v is infinite, NaN or rounded to infinity in bf16
+__device__ __forceinline__ void split(f32x4 v, u32x2 (&parts)[3]) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    f32x2 rest = {v[2 * i], v[2 * i + 1]};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2));
+      parts[p][i] = pair;
+      if (p < 2) rest[0] -= __builtin_bit_cast(float, pair << 16), rest[1] -= __builtin_bit_cast(float, pair & 0xffff0000u);
+    }
+  }
+}
 
 // One operand's slab: ROWS rows (of C's rows or columns), KC: the contraction is its contiguous dimension.  TWO: the upper half of the rows
 // are those of a second matrix.
-template <typename T, int ROWS, bool KC, int THREADS, int SETS, bool TWO = false>
+template <typename T, int KIND, int ROWS, bool KC, int THREADS, int SETS, bool TWO = false>
 struct Slab {
   static constexpr int ES = static_cast<int>(sizeof(T));
-  static constexpr int BK = Elem<T>::BK;
+  static constexpr int BK = 128 / ES;                          // contraction elements: 128 bytes
+  static constexpr int PARTS = KIND == F32_PARTS ? 3 : 1, LS = KIND == F32_PARTS ? 2 : ES;  // LS: bytes of an element in LDS
   static constexpr int LINES = KC ? ROWS : BK;                 // lines in memory order
-  static constexpr int LINE_BYTES = KC ? 128 : ROWS * ES;
-  static constexpr int STRIDE = LINE_BYTES + (KC ? 16 : Elem<T>::PAD);
-  static constexpr int BYTES = LINES * STRIDE;
-  static constexpr int CHUNKS = LINE_BYTES / 16;               // 16-byte chunks per line
+  static constexpr int PAD = PARTS > 1 ? 0 : KC ? 16 : ES == 2 ? 64 : 32;  // bytes behind a line in LDS
+  static constexpr int STRIDE = (KC ? BK : ROWS) * LS + PAD;   // bytes of a line of a part in LDS
+  static constexpr int PART_BYTES = LINES * STRIDE, BYTES = PARTS * PART_BYTES;
+  static constexpr int CHUNKS = (KC ? BK : ROWS) * ES / 16;    // 16-byte chunks per line in memory
   static constexpr int PER = LINES * CHUNKS / THREADS;         // chunks per lane
   static_assert(LINES * CHUNKS % THREADS == 0, "whole chunks per lane");
 
@@ -69,21 +83,33 @@ struct Slab {
   uint32_t advance;
   u32x4 reg[SETS][PER];
 
+  // Lines without padding: what the place of a byte in line i is changed by, so that the lines that are read together lie in different banks (a function of i % 16 for KC,
+  // of i % 4 otherwise)
+  static __device__ __forceinline__ int moved(int i) {
+    if constexpr (PAD != 0) return 0;
+    else if constexpr (KC) return (i >> 2 & 3) << 4;
+    else return ROWS >= 128 ? (i & 3) << 6 : ROWS == 64 ? (i >> 1 & 1) << 6 : 0;
+  }
+
   // base: first element of the slab's first row (KC) or column; ld: elements between lines; lines / line_elems: what exists
   __device__ __forceinline__ void init(const T* base, int64_t ld, int64_t lines, int64_t line_elems, int64_t k_begin) {
     const int64_t bytes = lines > 0 ? ((lines - 1) * ld + line_elems) * ES : 0;
     rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, static_cast<int>(bytes), 0x00020000);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int idx = (TWO ? i % (PER / 2) : i) * THREADS + threadIdx.x;
+      const int idx = i * THREADS + threadIdx.x - (second(i) ? LINES / 2 * CHUNKS : 0);
       const int64_t line = idx / CHUNKS + (KC ? 0 : k_begin);
       offset[i] = static_cast<uint32_t>((line * ld + (KC ? k_begin : 0)) * ES + (idx % CHUNKS) * 16);
     }
     advance = static_cast<uint32_t>(KC ? 128 : BK * ld * ES);
   }
+  static __device__ __forceinline__ bool second(int i) {
+    if constexpr (TWO && PER == 1) return __builtin_amdgcn_readfirstlane(threadIdx.x) >= THREADS / 2;
+    return TWO && i >= PER / 2;
+  }
   // of the second matrix, as many lines with the same stride
   __device__ __forceinline__ void init_second(const T* base, int64_t ld, int64_t lines, int64_t line_elems) {
-    static_assert(!TWO || (KC && PER % 2 == 0), "a chunk is of one matrix");
+    static_assert(!TWO || (KC && (PER == 1 || PER % 2 == 0)), "a wavefront's chunk is of one matrix");
     const int64_t bytes = lines > 0 ? ((lines - 1) * ld + line_elems) * ES : 0;
     rsrc2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, static_cast<int>(bytes), 0x00020000);
   }
@@ -91,21 +117,30 @@ struct Slab {
   __device__ __forceinline__ void fetch(int set, int i, int k_left) {
     const int idx = i * THREADS + threadIdx.x;
     const int k = KC ? (idx % CHUNKS) * (16 / ES) : idx / CHUNKS;
-    reg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(TWO && i >= PER / 2 ? rsrc2 : rsrc, k < k_left ? offset[i] : kOutside, 0, 0);
+    reg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(second(i) ? rsrc2 : rsrc, k < k_left ? offset[i] : kOutside, 0, 0);
     offset[i] += advance;
   }
   __device__ __forceinline__ void store(int set, int i, unsigned char* lds) const {
     const int idx = i * THREADS + threadIdx.x;
-    *reinterpret_cast<u32x4*>(lds + (idx / CHUNKS) * STRIDE + (idx % CHUNKS) * 16) = reg[set][i];
+    const int line = idx / CHUNKS;
+    unsigned char* at = lds + line * STRIDE + ((idx % CHUNKS) * (16 / ES * LS) ^ moved(line));
+    if constexpr (PARTS == 1) {
+      *reinterpret_cast<u32x4*>(at) = reg[set][i];
+    } else {
+      u32x2 parts[3];
+      split(__builtin_bit_cast(f32x4, reg[set][i]), parts);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(at + p * PART_BYTES) = parts[p];
+    }
   }
-  // fragment of rows row0 .. row0 + 31, contraction step ks; lane: row l % 32, contraction STEP * ks + (STEP / 2) * (l / 32) ..
-  static __device__ __forceinline__ typename Elem<T>::frag fragment(const unsigned char* lds, int row0, int ks, int lane) {
+  // fragment of rows row0 .. row0 + 31 (of a part), contraction step ks; lane: row l % 32, contraction STEP * ks + (STEP / 2) * (l / 32) ..
+  static __device__ __forceinline__ typename Multiply<KIND>::frag fragment(const unsigned char* lds, int row0, int ks, int lane) {
     const int l32 = lane & 31, hh = lane >> 5;
     if constexpr (KC) {
-      return *reinterpret_cast<const typename Elem<T>::frag*>(lds + (row0 + l32) * STRIDE + (2 * ks + hh) * 16);
-    } else if constexpr (ES == 2) {
+      return *reinterpret_cast<const typename Multiply<KIND>::frag*>(lds + (row0 + l32) * STRIDE + ((2 * ks + hh) * 16 ^ moved(l32)));
+    } else if constexpr (LS == 2) {
       const int l16 = lane & 15;
-      const unsigned char* src = lds + (16 * ks + 8 * hh + (l16 >> 2)) * STRIDE + (row0 + (l32 >> 4) * 16 + (l16 & 3) * 4) * 2;
+      const unsigned char* src = lds + (16 * ks + 8 * hh + (l16 >> 2)) * STRIDE + ((row0 + (l32 >> 4) * 16 + (l16 & 3) * 4) * 2 ^ moved(l16 >> 2));
       const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src));
       const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src + 4 * STRIDE));
       return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -260,19 +295,22 @@ template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool PAI
 struct TileShape {
   static constexpr int WAVES_N = BN / WN, WAVES = (BM / WM) * WAVES_N * KG, THREADS = WAVES * 64;
   static constexpr int MB = WM / 32, NB = WN / 32;
+  static constexpr bool SHARED = KG > 1 && WAVES == KG, GROUPS = KG > 1 && WAVES > KG;  // one wavefront to a group; several
+  static constexpr int KIND = sizeof(T) == 2 ? BF16 : SHARED ? F32_WHOLE : F32_PARTS;  // (in a tile of 32 x 32 the parts are more work than they save)
   static constexpr int SETS = MB * NB >= 8 ? 1 : 2;  // (eight accumulator blocks leave no registers for a second set)
-  typedef Slab<T, BM, FORM != FORM_TN, THREADS, SETS> SA;
-  typedef Slab<T, BN, FORM == FORM_NT, THREADS, SETS, PAIR> SB;
+  typedef Slab<T, KIND, BM, FORM != FORM_TN, THREADS, SETS> SA;
+  typedef Slab<T, KIND, BN, FORM == FORM_NT, THREADS, SETS, PAIR> SB;
   static constexpr int STAGE = SA::BYTES + SB::BYTES;
-  static constexpr int OUT = WAVES * 32 * (WN + 4) * 4;
-  static_assert(KG == 1 || WAVES == KG, "one wavefront to a group");
-  static_assert(!PAIR || (FORM == FORM_NT && KG == 1 && WAVES_N % 2 == 0), "the products of a pair side by side in a tile, half of the wavefronts each");
+  static constexpr int OUT = WAVES / (GROUPS ? KG : 1) * 32 * (WN + 4) * 4;
+  static_assert(!GROUPS || (KG - 1) * BM * BN * 4 <= 2 * STAGE, "the groups' sums meet where the slabs were");
+  static_assert(!PAIR || (FORM == FORM_NT && !SHARED && WAVES_N % 2 == 0), "the products of a pair side by side in a tile, half of the wavefronts each");
   static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
 };
 
-// One tile of one product.  KG > 1: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
+// One tile of one product.  KG > 1, SHARED: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
 // LDS, where all of them add up and write out a part of the tile (us, one of them / all: fp32 NT 2048 x 256 x 256 7.2 / 6.7,
-// 500 x 512 x 512 8.0 / 7.0).
+// 500 x 512 x 512 8.0 / 7.0).  GROUPS: KG groups of wavefronts each multiply their part of every slab (64 x 64 of parts, one / two: NT 2048 x 256 x 688 14.5 / 12.3, TN 1376 x 256 x 2048
+// whole 36 / 30; four or eight tiles to a CU the same).
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG, bool SEGMENTS, bool PAIR = false, bool ROPE = false, bool ACT = false>
 __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, unsigned char* lds, const MoreSegments& more, int segs, const Pair* pair = nullptr,
                                           const Rotation* rot = nullptr, int product = 0, const Activation* act = nullptr) {
@@ -280,10 +318,13 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
   constexpr int WAVES_N = S::WAVES_N, MB = S::MB, NB = S::NB, SETS = S::SETS, STAGE = S::STAGE;
   typedef typename S::SA SA;
   typedef typename S::SB SB;
-  constexpr int BK = Elem<T>::BK, STEPS = 4 / KG;
+  typedef Multiply<S::KIND> Mul;
+  constexpr int BK = SA::BK, PARTS = SA::PARTS, STEPS = BK / Mul::STEP / KG;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = KG > 1 ? wave : 0, member = KG > 1 ? 0 : wave;
+  constexpr int MEMBERS = S::WAVES / KG;  // wavefronts of a group
+  constexpr bool SHARED = S::SHARED, GROUPS = S::GROUPS;
+  const int group = wave / MEMBERS, member = wave % MEMBERS;
   const int wm = (member / WAVES_N) * WM, wn = (member % WAVES_N) * WN;
   const int slice = tile.slice, m0 = tile.m * BM, n0 = tile.n * (PAIR ? BN / 2 : BN);
 
@@ -301,10 +342,22 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
     seg_slabs = (k_left + BK - 1) / BK;
   };
   const int k_begin = slice * g.k_slice;
-  open(g.a, g.lda, g.b, g.ldb, g.K, k_begin, min(g.K, k_begin + g.k_slice));
-  int slabs = seg_slabs;
-  if constexpr (SEGMENTS)
-    for (int i = 0; i < segs; ++i) slabs += (more.K[i] + BK - 1) / BK;
+  int slabs;
+  if constexpr (SEGMENTS) {  // a slice is a run of the slabs of all segments
+    int skip = k_begin / BK, left = (g.K + BK - 1) / BK;
+    slabs = left - skip;
+    for (int i = 0; i < segs; ++i) {
+      const int more_slabs = (more.K[i] + BK - 1) / BK;
+      slabs += more_slabs;
+      if (seg == i && skip >= left) skip -= left, left = more_slabs, ++seg;
+    }
+    slabs = min(slabs, g.k_slice / BK);
+    if (seg == 0) open(g.a, g.lda, g.b, g.ldb, g.K, skip * BK, g.K);
+    else open(more.a[seg - 1], more.lda[seg - 1], more.b[seg - 1], more.ldb[seg - 1], more.K[seg - 1], skip * BK, more.K[seg - 1]);
+  } else {
+    open(g.a, g.lda, g.b, g.ldb, g.K, k_begin, min(g.K, k_begin + g.k_slice));
+    slabs = seg_slabs;
+  }
   auto next_slab = [&] {  // before the first chunk of a slab is fetched
     if constexpr (SEGMENTS) {
       while (seg_slabs == 0 && seg < segs) {
@@ -315,13 +368,13 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
     }
   };
 
-  f32x16 acc[MB][NB];
+  f32x16 acc[MB][NB], low[PARTS > 1 ? MB : 1][PARTS > 1 ? NB : 1];  // low: the products of all but both first parts
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f, low[PARTS > 1 ? i : 0][PARTS > 1 ? j : 0][e] = 0.f;
 
   // One slab ahead in LDS, the next SETS in registers: chunk c of slab s + 1 goes to the other stage and its registers fetch
   // chunk c of slab s + 1 + SETS, spread behind the products of the fragment steps.  (Past the end: zeros, never multiplied.)
@@ -346,13 +399,13 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
   // What the result is added to, for small tiles: fetched here, behind the first slabs, where the end of the tile would wait for
   // it (a gradient that was last touched a step ago; dW and dx of a 512-wide layer at 1023 tokens: four launches a layer, 40 us
   // of a training step of 8 layers).
-  constexpr int OUT_LANES = KG > 1 ? S::THREADS : 64;  // that write a block of 32 rows of C
+  constexpr int OUT_LANES = SHARED ? S::THREADS : 64;  // that write a block of 32 rows of C
   constexpr int LPR = WN / 4, RPP = OUT_LANES / LPR, PASSES = 32 / RPP;  // out: lanes per row, four columns each, rows per pass
-  constexpr bool EARLY = !PAIR && !ROPE && !ACT && (KG > 1 || MB * NB <= 2);
+  constexpr bool EARLY = !PAIR && !ROPE && !ACT && (SHARED || MB * NB <= 2);
   typedef T t4 __attribute__((ext_vector_type(4)));
   t4 old[EARLY ? MB * PASSES : 1];
   constexpr int HALF = WAVES_N / 2;  // PAIR: wavefronts of a row of blocks that have the first product; HALF further on is the second one of the same columns
-  const int out_lane = KG > 1 ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? wn % (BN / 2) : wn) + c4;
+  const int out_lane = SHARED ? tid : lane, c4 = (out_lane % LPR) * 4, col = n0 + (PAIR ? wn % (BN / 2) : wn) + c4;
   const int tile_row = wm + out_lane / LPR, out_row = m0 + tile_row, rows_here = g.M - m0;  // out_row: of pass 0 of the first block
   const bool vec = PAIR || ACT || ROPE || ((g.N & 3) == 0 && (g.ldc & 3) == 0);
   Window<T> out;
@@ -428,12 +481,15 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
     const unsigned char* la = lds + (s & 1) * STAGE;
     const unsigned char* lb = la + SA::BYTES;
     unsigned char* next = lds + (~s & 1) * STAGE;
-    typename Elem<T>::frag fa[2][MB], fb[2][NB];  // (reading the whole slab's first instead changes nothing)
+    typename Mul::frag fa[2][MB][PARTS], fb[2][NB][PARTS];  // (reading the whole slab's first instead changes nothing)
     auto read = [&](int ks) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) fb[ks & 1][j] = SB::fragment(lb, wn + 32 * j, group * STEPS + ks, lane);
+      for (int p = PARTS - 1; p >= 0; --p) {
 #pragma unroll
-      for (int i = 0; i < MB; ++i) fa[ks & 1][i] = SA::fragment(la, wm + 32 * i, group * STEPS + ks, lane);
+        for (int j = 0; j < NB; ++j) fb[ks & 1][j][p] = SB::fragment(lb + p * SB::PART_BYTES, wn + 32 * j, group * STEPS + ks, lane);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fa[ks & 1][i][p] = SA::fragment(la + p * SA::PART_BYTES, wm + 32 * i, group * STEPS + ks, lane);
+      }
     };
     read(0);
 #pragma unroll
@@ -442,7 +498,15 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[i][j] = Elem<T>::mma(fb[ks & 1][j], fa[ks & 1][i], acc[i][j]);
+        for (int j = 0; j < NB; ++j) {
+          if constexpr (PARTS > 1) {
+#pragma unroll
+            for (int sum = 2; sum > 0; --sum)  // smallest products first; those of 2^-24 and less are left out
+#pragma unroll
+              for (int p = 0; p <= sum; ++p) low[i][j] = Mul::mma(fb[ks & 1][j][p], fa[ks & 1][i][sum - p], low[i][j]);
+          }
+          acc[i][j] = Mul::mma(fb[ks & 1][j][0], fa[ks & 1][i][0], acc[i][j]);
+        }
 #pragma unroll
       for (int c = ks * CHUNKS / STEPS; c < (ks + 1) * CHUNKS / STEPS; ++c) {
         store(set, c, next);
@@ -490,6 +554,71 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
     }
   }
 
+  if constexpr (PARTS > 1) {
+    float finite = 0.f;  // NaN if a sum is not
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        acc[i][j] += low[i][j];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
+      }
+    if (__builtin_amdgcn_ballot_w64(finite != 0.f)) {
+      // Infinities, NaN, and numbers that bf16 rounds to infinity have no parts: this wavefront's blocks once more, by fp32 matrix instructions straight from memory
+      // (a tenth of the speed or less).
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int row = m0 + wm + 32 * i + l32, block = wn + 32 * j, in_pair = block % (BN / 2);
+          const bool second = PAIR && block >= BN / 2;
+          const int column = n0 + (PAIR ? in_pair : block) + l32;
+          f32x16 sum;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+          for (int part = 0, before = 0; part <= (SEGMENTS ? segs : 0); ++part) {
+            const float* a = static_cast<const float*>(part ? more.a[part - 1] : g.a);
+            const float* b = static_cast<const float*>(part ? more.b[part - 1] : second ? pair->b2 : g.b);
+            const int64_t lda = part ? more.lda[part - 1] : g.lda, ldb = part ? more.ldb[part - 1] : g.ldb;
+            const int K = part ? more.K[part - 1] : g.K, from = max(0, k_begin - before), to = min(K, k_begin + g.k_slice - before);
+            before += (K + BK - 1) / BK * BK;
+            for (int k0 = from; k0 < to; k0 += 8) {
+              if (GROUPS && (k0 - from) / Mul::STEP % KG != group) continue;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int k = k0 + 4 * hh + e;
+                const float x = row < g.M && k < to ? a[FORM == FORM_TN ? k * lda + row : row * lda + k] : 0.f;
+                const float y = column < g.N && k < to ? b[FORM == FORM_NT ? column * ldb + k : k * ldb + column] : 0.f;
+                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(y, x, sum, 0, 0, 0);
+              }
+            }
+          }
+          acc[i][j] = sum;
+        }
+    }
+  }
+
+  if constexpr (GROUPS) {  // the first group takes the others' sums, and writes the tile
+    static_assert(MB * NB == 1);
+    f32x4* sums = reinterpret_cast<f32x4*>(lds) + member * 256 + lane;
+    __syncthreads();
+    if (group > 0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sums[(group - 1) * MEMBERS * 256 + q * 64] = f32x4{acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]};
+    }
+    __syncthreads();
+    if (group > 0) return;  // (a barrier waits for the wavefronts that are left)
+#pragma unroll
+    for (int o = 0; o < KG - 1; ++o)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 v = sums[o * MEMBERS * 256 + q * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[0][0][4 * q + e] += v[e];
+      }
+  }
+
   if (!SMALL) fetch_old(), fetch_gates();
   if (!EARLY_ANGLES && ALL_ANGLES) fetch_angles(0);
   Window<T> out2, out_h;
@@ -506,19 +635,19 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
   // acc[i][j][4 q + r]: row wm + 32 i + l % 32 of C, column wn + 32 j + 8 q + 4 hh + r.  Out through LDS, 32 rows at a time.
   __syncthreads();
   constexpr int ROW = WN + 4;  // floats
-  float* stage = reinterpret_cast<float*>(lds) + (KG > 1 ? 0 : wave * 32 * ROW);
+  float* stage = reinterpret_cast<float*>(lds) + (SHARED ? 0 : wave * 32 * ROW);
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
-    if ((KG > 1 || PAIR) && i > 0) __syncthreads();
+    if ((SHARED || PAIR) && i > 0) __syncthreads();
     if (!ALL_ANGLES) fetch_angles(i);
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-        *reinterpret_cast<f32x4*>(stage + (group * 32 + l32) * ROW + 32 * j + 8 * q + 4 * hh) = v;
+        *reinterpret_cast<f32x4*>(stage + ((SHARED ? group : 0) * 32 + l32) * ROW + 32 * j + 8 * q + 4 * hh) = v;
       }
-    if (KG > 1 || PAIR) __syncthreads();  // (alone, a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
+    if (SHARED || PAIR) __syncthreads();  // (alone, a wavefront reads only what it wrote: LDS operations of a wavefront complete in order)
     if constexpr (PAIR) {  // the two wavefronts of a pair of blocks take half of the rows each
       const int second = wave % WAVES_N / HALF;
       const float* first = reinterpret_cast<const float*>(lds) + (wave - second * HALF) * 32 * ROW;
@@ -542,7 +671,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
       const int at = (r * RPP + out_lane / LPR) * ROW + c4, row = 32 * i + r * RPP;
       f32x4 v = *reinterpret_cast<const f32x4*>(stage + at);
 #pragma unroll
-      for (int o = 1; o < KG; ++o) v += *reinterpret_cast<const f32x4*>(stage + o * 32 * ROW + at);
+      for (int o = 1; o < (SHARED ? KG : 1); ++o) v += *reinterpret_cast<const f32x4*>(stage + o * 32 * ROW + at);
       if constexpr (ACT) {
         t4 dgate, dup;
 #pragma unroll
@@ -619,11 +748,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_rope_ker
 // us, one product and the pass over gate and up / the pair / without gate and up (weights out of HBM, x just written): 1376 + 1376 x 512 bf16
 // 200 rows 5.8 + 4.2 / 6.3 / 6.0, 1023 rows 11.0 + 4.4 / 12.0 / 10.9, 2331 rows 15.5 + 5.8 / 17.7 / 16.1, 16384 rows in a training step 80 (the library's selected kernel) + 23 / 82;
 // 688 + 688 x 256 fp32 2048 rows 20.1 + 4.8 / 20.9 / 18.9.
-template <typename T, int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_pair_kernel(const Product g, const Pair pair) {
+template <typename T, int BM, int BN, int WM, int WN, int KG>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KG * 64) void gemm_pair_kernel(const Product g, const Pair pair) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const Tile tile(g, static_cast<int>(blockIdx.x));
-  if (tile.there) gemm_tile<T, FORM_NT, BM, BN, WM, WN, 1, false, true>(g, tile, lds, MoreSegments{}, 0, &pair);
+  if (tile.there) gemm_tile<T, FORM_NT, BM, BN, WM, WN, KG, false, true>(g, tile, lds, MoreSegments{}, 0, &pair);
 }
 
 // Several small products in one launch: what a linear layer's backward needs (dx and dW), or projections that share their input.
@@ -718,8 +847,8 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(const Joins js) {
 }
 
 // ---- which tile, which split ----------------------------------------------------------------------------------------------
-constexpr int kSmall = 0, k128 = 1, k256x128 = 2, k256 = 3, k128x64 = 4, kTiles = 5;  // (small: 64 x 64, in fp32 also 32 x 32; 128 x 64: bf16)
-constexpr int kTileM[kTiles] = {64, 128, 256, 256, 128}, kTileN[kTiles] = {64, 128, 128, 256, 64};
+constexpr int kSmall = 0, k128 = 1, k256x128 = 2, k256 = 3, k128x64 = 4, k32 = 5, kTiles = 6;  // (small: 64 x 64; the 256s: bf16; 32: fp32)
+constexpr int kTileM[kTiles] = {64, 128, 256, 256, 128, 32}, kTileN[kTiles] = {64, 128, 128, 256, 64, 32};
 int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 int slab_of(int dtype) { return dtype == MLTS_BF16 ? 64 : 32; }
 int64_t slabs_of(const mlts_gemm_product& p, int bk) {
@@ -734,47 +863,8 @@ void set_slices(Product& g, int64_t slices, int64_t slabs, int bk) {
   g.slices = static_cast<int>(std::max<int64_t>(1, (slabs + part - 1) / part));
 }
 
-// fp32: a product that runs alone takes the largest tile that still gives every CU a workgroup.
-int choose_f32_tile(const mlts_gemm_product& p) {
-  if (p.segments > 1) return kSmall;
-  if (tiles_of(p.M, p.N, 256, 256) >= 240) return k256;
-  if (tiles_of(p.M, p.N, 256, 128) >= 256) return k256x128;
-  return tiles_of(p.M, p.N, 128, 128) >= 256 ? k128 : kSmall;
-}
-bool splittable(const mlts_gemm_product& p) { return p.segments == 1 && p.N % 4 == 0 && p.ldc == p.N; }
-
-// The small fp32 products of a launch together: tiles of 64 x 64, or of 32 x 32, whose four wavefronts share a tile along
-// the contraction (us, 64 x 64 / 32 x 32: NT 2048 x 256 x 256 8.2 / 6.3, NN 1000 x 512 x 1376 31.4 / 17.1, 500 x 256 x 256 7.9 /
-// 4.6, but 2048 x 1376 x 512 29.8 / 32.4).  chain: us a workgroup takes for a slab; busy: us of a CU for each slab when it has
-// several workgroups (measured).
-struct SmallShape {
-  int size;
-  double chain, busy;
-};
-constexpr SmallShape kBf16Shape{64, 0, 0}, kF32Shape{64, 0.65, 0.5}, kF32Fine{32, 0.31, 0.16};
-
-// Slices of each product, and the estimated time: the longest chain of slabs, or the product on all 256 CUs if that is longer, and
-// what a split costs: a launch that joins the slices and their fp32 sums written and read.  A weight gradient's split does not
-// depend on what shares its launch, so that its bits do not either.  (us: TN 256 x 256 x 2048 whole 20.5, in eight 8.9; NN 1000 x 512 x
-// 1376 whole 17.1, in two 20.3.)
-double small_slices(const mlts_gemm_product* const* ps, int count, const SmallShape& shape, int64_t* slices) {
-  const int bk = slab_of(MLTS_F32);
-  double longest = 0;
-  for (int i = 0; i < count; ++i) {
-    const int64_t slabs = slabs_of(*ps[i], bk), tiles = tiles_of(ps[i]->M, ps[i]->N, shape.size, shape.size);
-    const int company = count > 1 && ps[i]->form == FORM_NN ? 2 : 1;  // beside dx runs a dW of the same size
-    const double whole = static_cast<double>(tiles * slabs * company) * shape.busy / 256;
-    auto cost = [&](int64_t s) {
-      return std::max(shape.chain * static_cast<double>(slabs) / static_cast<double>(s), whole) +
-             (s > 1 ? 2.5 + 8.0 * static_cast<double>(s * ps[i]->M * ps[i]->N) / 3.5e6 : 0.0);
-    };
-    slices[i] = 1;
-    for (int64_t s = 2; splittable(*ps[i]) && s <= 16 && slabs / s >= 4; s *= 2)
-      if (cost(s) < cost(slices[i])) slices[i] = s;
-    longest = std::max(longest, cost(slices[i]));
-  }
-  return longest;
-}
+// (the parts of a bf16 sum are rounded one by one)
+bool splittable(const mlts_gemm_product& p, int dtype) { return (p.segments == 1 || dtype == MLTS_F32) && p.N % 4 == 0 && p.ldc == p.N; }
 
 // The rectangles of the eight XCDs (Tile), bm x bn the tile; returns the tiles of the largest one.
 int64_t divide(Product& g, int bm, int bn) {
@@ -794,51 +884,68 @@ int64_t divide(Product& g, int bm, int bn) {
 
 // Divides the products of a launch; each: the tiles of an XCD, returns their sum.  In runs of equal length where the largest rectangles would give a CU of their XCD
 // one tile more: that costs more than what they save in L2.  (us, rectangles / runs, 33 to 36 tiles for the 32 CUs of an XCD and 32: bf16 NN 5352 x 768 x 768
-// 15.9 / 11.8, 2678 x 384 x 1488 11.7 / 9.4, dx and dW of 1407 x 640 x 3408 34.6 / 26.4; four on a CU for three: fp32 NN 1206 x 640 x 640 14.7 / 12.4.  Elsewhere
-// rectangles are ahead: NT 541 x 2304 x 768 7.4 / 8.9, 524 x 5456 x 1024 12.2 / 13.7.)
-int64_t spread(Product* ps, int count, int bm, int bn, int64_t* each) {
+// 15.9 / 11.8, 2678 x 384 x 1488 11.7 / 9.4, dx and dW of 1407 x 640 x 3408 34.6 / 26.4.  Elsewhere
+// rectangles are ahead: NT 541 x 2304 x 768 7.4 / 8.9, 524 x 5456 x 1024 12.2 / 13.7.)  In fp32, whose tiles are bound by their arithmetic, in runs wherever the largest rectangle has a tile more
+// (60 products and launches of dW and dx: equal, 0.4 % on the mean; tiles of 32 x 32, four on a CU for three: NN 1206 x 640 x 640 14.7 / 12.4).
+int64_t spread(Product* ps, int count, int tile, int dtype, int64_t* each) {
   constexpr int64_t cus = 32;  // of an XCD
   int64_t rectangles = 0, runs = 0;
   const auto run_of = [](const Product& g) { return (static_cast<int64_t>(g.tiles_m) * g.tiles_n * g.slices + 7) / 8; };
-  for (int i = 0; i < count; ++i) rectangles += each[i] = divide(ps[i], bm, bn), runs += run_of(ps[i]);
-  if ((rectangles + cus - 1) / cus <= (runs + cus - 1) / cus) return rectangles;
+  for (int i = 0; i < count; ++i) rectangles += each[i] = divide(ps[i], kTileM[tile], kTileN[tile]), runs += run_of(ps[i]);
+  if (dtype == MLTS_BF16 ? (rectangles + cus - 1) / cus <= (runs + cus - 1) / cus : rectangles <= runs) return rectangles;
   for (int i = 0; i < count; ++i) each[i] = run_of(ps[i]), ps[i].xcds = kRuns;
   return runs;
 }
 
-// bf16: tile and split by estimated time (us).  A launch takes `fixed`, then what the CU with the most workgroups takes for their slabs, one after the
-// other, then what is written; a split also the launch that joins the slices and their fp32 sums.  Fitted to 900 products in the three forms, 3 to 32000 rows, 64
+// Tile and split by estimated time (us).  A launch takes `fixed`, then what the CU with the most workgroups takes for their slabs (`busy` each, one after the
+// other; alone, a workgroup takes `chain`), then what is written; a split also the launch that joins the slices and their fp32 sums.
+struct TileCost {
+  double fixed, chain, busy, out;  // out: of a million elements
+};
+struct Costs {
+  TileCost tile[kTiles];
+  int tiles[5], count;           // that there are
+  double join_fixed, join_sums;  // ... of a million partial sums
+};
+// bf16: fitted to 900 products in the three forms, 3 to 32000 rows, 64
 // to 4096 wide, 2e6 to 2.4e10 multiplications, each on all tiles and splits; of 900 others it is off by 9 % (rms), and the choice by 0.6 % from the best (1 % of them by
 // more than 11 %); of 500 launches of dW and dx by 2.3 %, 1.5 of them because a weight gradient keeps the split that it has alone.
 // What a workgroup fetches decides: loads alone, with neither LDS nor matrix instructions, take as
 // long as the kernel (2048 x 2048 x 1536, tiles of 64 x 64: 29 us of 30.5), and a tile of 128 x 128 fetches half as much for its work
 // (us, 64 x 64 / 128 x 128: NT 2331 x 1536 x 512 12.0 / 9.4, 8192 x 2752 x 512 45.3 / 34.9, NN 16384 x 1376 x 512 48.8 / 36.5).
-struct TileCost {
-  double fixed, slab, out;  // out: of a million elements
-};
-constexpr TileCost kBf16Cost[kTiles] = {{2.5, 0.24, 0.55}, {3.2, 0.52, 0.55}, {3.95, 0.83, 0.69}, {6.2, 1.26, 0.56}, {3.1, 0.373, 0.71}};
-// A second workgroup on a CU overlaps the first on 64 x 64, by so much a slab (us, 64 x 64 / 128 x 64, of 37 and 19 tiles to an XCD: NT 2331 x 512 x 512 6.5 / 6.95, NN 6.5 /
+constexpr Costs kBf16Costs{{{2.5, 0.24, 0.24, 0.55}, {3.2, 0.52, 0.52, 0.55}, {3.95, 0.83, 0.83, 0.69}, {6.2, 1.26, 1.26, 0.56}, {3.1, 0.373, 0.373, 0.71}, {}},
+                           {kSmall, k128, k256x128, k256, k128x64}, 5, 2.55, 1.73};
+// fp32: fitted to 400 products in the three forms, 64 to 4096 rows, 64 to 2048 wide (and vocabularies of 8192 to 32000), 2e6 to 2.5e10 multiplications, each on all tiles and splits:
+// off by 4 to 6 % (rms), the choice by 0.4 % from the best.  32 x 32, whose four wavefronts share the contraction and multiply whole elements, has the
+// shortest chain; where CUs have several of them, the tiles of elements in three parts are ahead, larger ones the more so (us, 32 x 32 / 64 x 64 / 128 x 128, and the larger of these in fp32 matrix
+// instructions before: NT 2048 x 256 x 256 5.9 / 7.1 / 12, 2048 x 1376 x 256 20 / 14.3 / 13.8, before 16.7; 2048 x 8192 x 256 - / 64 / 55, before 75; 4096 x 2048 x 2048 - / 216 / 172, before 245).  Of the 400 the time
+// is 0.92 of that before on the geometric mean, from 5e8 multiplications on 0.55 to 0.85, and there 0.6 to 1.09 of the library's, 0.75 on the mean.
+// What bounds the parts: a slab of 128 x 128 takes a CU 1.0 us, of which the matrix instructions are 1536 cycles, the LDS 1000 (192 KB) and a wavefront's splitting and addresses 500; vector
+// and matrix instructions of a SIMD's wavefronts hardly overlap.  (No change: vector instructions spread between matrix instructions; twice the slabs in flight 7.1 -> 7.5.)
+constexpr Costs kF32Costs{{{3.29, 0.4, 0.384, 1.22}, {4.16, 0.99, 0.99, 1.33}, {}, {}, {3.87, 0.796, 0.663, 1.13}, {2.71, 0.191, 0.15, 1.02}}, {kSmall, k128, k128x64, k32}, 4, 2.44, 2.26};
+const Costs& costs_of(int dtype) { return dtype == MLTS_BF16 ? kBf16Costs : kF32Costs; }
+// A second workgroup on a CU overlaps the first on 64 x 64 in bf16, by so much a slab (us, 64 x 64 / 128 x 64, of 37 and 19 tiles to an XCD: NT 2331 x 512 x 512 6.5 / 6.95, NN 6.5 /
 // 6.95, dW and dx of it on 64 x 64 / 128 x 128 12.4 / 13.5).  Of 600 products and 200 launches of dW and dx the choice is 0.51 and 0.74 % from the best, 0.74 and 0.86 %
 // without it.  Launches with a pass, fitted without it, go without it.
 constexpr double kSmallOverlap = 0.06;
-constexpr double kJoinFixed = 2.55, kJoinSums = 1.73;  // ... of a million partial sums
-// What a pass on the way out adds on each tile: of a launch, of a million elements; the larger ones have fewer wavefronts to overlap its latency with.  (Fitted to 250
+// What a pass on the way out adds in bf16 on each tile: of a launch, of a million elements; the larger ones have fewer wavefronts to overlap its latency with.  (Fitted to 250
 // rotated products, 170 launches of three, 400 pairs and 300 launches of dW and dh, the choice 0.3, 0.1, 0.3 and 0.9 % from the best.)
 struct PassCost {
   double fixed[kTiles], out[kTiles];
 };
 constexpr PassCost kRotationCost{{1.0, 1.7, 3.9, 7.2, 1.8}, {0, 0.16, 0.35, 0.38, 0.06}},
     kJointRotationCost{{1.0, 3.7}, {0, 0.16}}, kPairCost{{0.7, 1.5}, {0.5, 0.8}}, kActivationCost{{1.9, 4.0}, {1.8, 1.3}};
-constexpr TileCost kRotationApart{2.0, 0, 0.6};  // a launch of its own, after a split product (110 of the two, in a graph: 0.7 % from the best)
+constexpr TileCost kRotationApart{2.0, 0, 0, 0.6};  // a launch of its own, after a split product (110 of the two, in a graph: 0.7 % from the best)
 double pass_time(const PassCost& c, int tile, int64_t M, int64_t N) { return c.fixed[tile] + c.out[tile] * 1e-6 * static_cast<double>(M) * static_cast<double>(N); }
 
 // The time of products in one launch, the slices of each given
-double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const int64_t* slices, bool pass) {
-  const TileCost& c = kBf16Cost[tile];
+double launch_time(int dtype, const mlts_gemm_product* const* ps, int count, int tile, const int64_t* slices, bool pass) {
+  const Costs& costs = costs_of(dtype);
+  const TileCost& c = costs.tile[tile];
   double longest = 0, work = 0, workgroups = 0, out = 0, sums = 0;
   int64_t of_an_xcd = 0;
   for (int i = 0; i < count; ++i) {
-    const int64_t slabs = slabs_of(*ps[i], 64), part = (slabs + slices[i] - 1) / slices[i];
+    const int64_t slabs = slabs_of(*ps[i], slab_of(dtype)), part = (slabs + slices[i] - 1) / slices[i];
     const int64_t tiles = tiles_of(ps[i]->M, ps[i]->N, kTileM[tile], kTileN[tile]) * (part ? (slabs + part - 1) / part : 1);
     const double elements = 1e-6 * static_cast<double>(ps[i]->M) * static_cast<double>(ps[i]->N);
     longest = std::max(longest, static_cast<double>(part));
@@ -847,31 +954,37 @@ double bf16_time(const mlts_gemm_product* const* ps, int count, int tile, const 
     (slices[i] > 1 ? sums : out) += elements * static_cast<double>(slices[i] > 1 ? slices[i] : 1);
   }
   const double of_a_cu = static_cast<double>((of_an_xcd + 31) / 32);
-  const double overlap = tile == kSmall && of_a_cu > 1 && !pass ? kSmallOverlap : 0;
-  const double slabs = workgroups > 0 ? std::max(longest * c.slab, work / workgroups * (of_a_cu * c.slab - overlap)) : 0;
-  return c.fixed + slabs + out * c.out + (sums > 0 ? kJoinFixed + kJoinSums * sums : 0);
+  const double overlap = dtype == MLTS_BF16 && tile == kSmall && of_a_cu > 1 && !pass ? kSmallOverlap : 0;
+  const double slabs = workgroups > 0 ? std::max(longest * c.chain, work / workgroups * (of_a_cu * c.busy - overlap)) : 0;
+  return c.fixed + slabs + out * c.out + (sums > 0 ? costs.join_fixed + costs.join_sums * sums : 0);
 }
 
 // ... of a product in a launch by itself, its outputs rotated on their way out (split, by a launch after it) or not
-double alone_time(const mlts_gemm_product& p, int tile, int64_t slices, bool rotation) {
+double alone_time(int dtype, const mlts_gemm_product& p, int tile, int64_t slices, bool rotation) {
   const mlts_gemm_product* const one = &p;
-  const double time = bf16_time(&one, 1, tile, &slices, rotation);
+  const double time = launch_time(dtype, &one, 1, tile, &slices, rotation);
   if (!rotation) return time;
-  return time + (slices == 1 ? pass_time(kRotationCost, tile, p.M, p.N) : kRotationApart.fixed + kRotationApart.out * 1e-6 * static_cast<double>(p.M) * static_cast<double>(p.N));
+  if (slices > 1) return time + kRotationApart.fixed + kRotationApart.out * 1e-6 * static_cast<double>(p.M) * static_cast<double>(p.N);
+  return time + (dtype == MLTS_BF16 ? pass_time(kRotationCost, tile, p.M, p.N) : 0);
 }
 
-// The best tile and split of a product that runs alone
-int choose_bf16_tile(const mlts_gemm_product& p, int64_t* slices, bool rotation) {
-  const int64_t slabs = slabs_of(p, 64);
+// The best tile (or `only` that) and split of a product that runs alone
+int choose_tile(int dtype, const mlts_gemm_product& p, int64_t* slices, bool rotation, int only = -1) {
+  const Costs& costs = costs_of(dtype);
+  const int64_t slabs = slabs_of(p, slab_of(dtype));
   *slices = 1;
-  if (p.segments > 1) return kSmall;
+  if (p.segments > 1 && only < 0) return kSmall;
   int best = kSmall;
   double least = 0;
-  for (int tile = 0; tile < kTiles; ++tile)
-    for (int64_t s = 1; s == 1 || (splittable(p) && s <= 16 && slabs / s >= 4); s *= 2) {
-      const double t = alone_time(p, tile, s, rotation);
-      if (least == 0 || t < least) least = t, best = tile, *slices = s;
+  for (int t = 0; t < costs.count; ++t) {
+    if (only >= 0 && costs.tiles[t] != only) continue;
+    // (32 x 32 equal within what the fit is off by: the parts, whose errors are a third)
+    const double weight = costs.tiles[t] == k32 ? 1.07 : 1;
+    for (int64_t s = 1; s == 1 || (splittable(p, dtype) && s <= 16 && slabs / s >= 4); s *= 2) {
+      const double time = weight * alone_time(dtype, p, costs.tiles[t], s, rotation);
+      if (least == 0 || time < least) least = time, best = costs.tiles[t], *slices = s;
     }
+  }
   return best;
 }
 
@@ -879,37 +992,12 @@ struct LaunchPlan {
   int tile[kMaxProducts];
   int64_t slices[kMaxProducts];
   bool together[kMaxProducts] = {};  // in the launch of several products, all of one tile
-  SmallShape shape;                  // of the small tile
   int64_t workspace = 0;             // bytes
-  int rows_of(int t) const { return t == kSmall ? shape.size : kTileM[t]; }
-  int columns_of(int t) const { return t == kSmall ? shape.size : kTileN[t]; }
-  // activation: an NN product that is not split, whose output goes through the activation
-  LaunchPlan(const mlts_gemm_product* ps, int count, int dtype, bool activation = false, bool rotation = false) : shape(dtype == MLTS_BF16 ? kBf16Shape : kF32Shape) {
-    if (dtype == MLTS_BF16) plan_bf16(ps, count, activation, rotation);
-    else plan_f32(ps, count, activation);
-    for (int i = 0; i < count; ++i)
-      if (slices[i] > 1) workspace += ps[i].M * ps[i].N * 4 * slices[i];
-  }
 
- private:
-  void plan_f32(const mlts_gemm_product* ps, int count, bool activation) {
-    const mlts_gemm_product* small[kMaxProducts];
-    int small_at[kMaxProducts], smalls = 0;
-    for (int i = 0; i < count; ++i) {
-      tile[i] = choose_f32_tile(ps[i]), slices[i] = 1;
-      if (tile[i] == kSmall) small_at[smalls] = i, small[smalls++] = &ps[i];
-      together[i] = tile[i] == kSmall && (count > 1 || ps[i].segments > 1 || activation);
-    }
-    if (smalls == 0) return;
-    int64_t s[kMaxProducts], fine[kMaxProducts];
-    const double coarse = small_slices(small, smalls, shape, s);
-    if (small_slices(small, smalls, kF32Fine, fine) < coarse) shape = kF32Fine, std::copy(fine, fine + smalls, s);
-    for (int i = 0; i < smalls; ++i) slices[small_at[i]] = s[i];
-  }
-
-  // All products in one launch of small or of 128 x 128 tiles, or each by itself.  A weight gradient's split is the one it has alone, so that its
-  // bits do not depend on what shares its launch.
-  void plan_bf16(const mlts_gemm_product* ps, int count, bool activation, bool rotation) {
+  // All products in one launch of small (in fp32 also 32 x 32) or of 128 x 128 tiles, or each by itself.  A weight gradient's split is the one it has alone (in fp32, on these tiles), so that
+  // in bf16 its bits do not depend on what shares its launch.  activation: an NN product that is not split, whose output goes through the activation
+  LaunchPlan(const mlts_gemm_product* ps, int count, int dtype, bool activation = false, bool rotation = false) {
+    const Costs& costs = costs_of(dtype);
     const mlts_gemm_product* all[kMaxProducts];
     double apart = 0;
     int joins = 0;
@@ -917,34 +1005,41 @@ struct LaunchPlan {
     bool parts = false;
     for (int i = 0; i < count; ++i) {
       all[i] = &ps[i];
-      tile[i] = choose_bf16_tile(ps[i], &slices[i], rotation);
-      apart += alone_time(ps[i], tile[i], slices[i], rotation);
+      tile[i] = choose_tile(dtype, ps[i], &slices[i], rotation);
+      apart += alone_time(dtype, ps[i], tile[i], slices[i], rotation);
       columns += ps[i].N;
       joins += slices[i] > 1;
       parts = parts || ps[i].segments > 1;
     }
-    apart -= joins > 1 ? (joins - 1) * kJoinFixed : 0;  // one launch joins them all
-    if (count == 1 && !parts && !activation) return;
-    double least = 0;
-    int best = -1;
-    int64_t best_slices[kMaxProducts], s[kMaxProducts];
-    for (int t : {kSmall, k128}) {
-      if (t != kSmall && parts) continue;
-      for (int64_t dx = 1; dx <= (activation ? 1 : 4); dx *= 2) {
-        for (int i = 0; i < count; ++i) s[i] = ps[i].form == FORM_TN ? slices[i] : ps[i].form == FORM_NN && splittable(ps[i]) && slabs_of(ps[i], 64) / dx >= 4 ? dx : 1;
-        double time = bf16_time(all, count, t, s, rotation || activation) + (rotation ? pass_time(kJointRotationCost, t, ps[0].M, columns) : 0);
-        if (activation) time += pass_time(kActivationCost, t, ps[count - 1].M, ps[count - 1].N);
-        if (best < 0 || time < least) least = time, best = t, std::copy(s, s + count, best_slices);
+    apart -= joins > 1 ? (joins - 1) * costs.join_fixed : 0;  // one launch joins them all
+    if (count > 1 || parts || activation) {
+      double least = 0;
+      int best = -1;
+      int64_t best_slices[kMaxProducts], s[kMaxProducts];
+      for (int t : {kSmall, k128, k32}) {
+        if ((t == k128 && parts) || (t == k32 && dtype == MLTS_BF16)) continue;
+        int64_t weight[kMaxProducts];
+        std::copy(slices, slices + count, weight);
+        if (dtype == MLTS_F32)
+          for (int i = 0; i < count; ++i) choose_tile(dtype, ps[i], &weight[i], false, t);
+        for (int64_t dx = 1; dx <= (activation ? 1 : 4); dx *= 2) {
+          for (int i = 0; i < count; ++i) s[i] = ps[i].form == FORM_TN ? weight[i] : ps[i].form == FORM_NN && splittable(ps[i], dtype) && slabs_of(ps[i], slab_of(dtype)) / dx >= 4 ? dx : 1;
+          double time = launch_time(dtype, all, count, t, s, rotation || activation);
+          if (dtype == MLTS_BF16 && rotation) time += pass_time(kJointRotationCost, t, ps[0].M, columns);
+          if (dtype == MLTS_BF16 && activation) time += pass_time(kActivationCost, t, ps[count - 1].M, ps[count - 1].N);
+          if (best < 0 || time < least) least = time, best = t, std::copy(s, s + count, best_slices);
+        }
       }
+      if (parts || activation || least <= apart) std::fill(tile, tile + count, best), std::fill(together, together + count, true), std::copy(best_slices, best_slices + count, slices);
     }
-    if (!parts && !activation && apart < least) return;
-    std::fill(tile, tile + count, best), std::fill(together, together + count, true), std::copy(best_slices, best_slices + count, slices);
+    for (int i = 0; i < count; ++i)
+      if (slices[i] > 1) workspace += ps[i].M * ps[i].N * 4 * slices[i];
   }
 };
 
 // a product's tiles and slices as product i of a plan
 void set_tiles(Product& g, const mlts_gemm_product& p, const LaunchPlan& plan, int i, int dtype) {
-  const int bm = plan.rows_of(plan.tile[i]), bn = plan.columns_of(plan.tile[i]);
+  const int bm = kTileM[plan.tile[i]], bn = kTileN[plan.tile[i]];
   g.tiles_m = static_cast<int>((p.M + bm - 1) / bm), g.tiles_n = static_cast<int>((p.N + bn - 1) / bn);
   set_slices(g, plan.slices[i], slabs_of(p, slab_of(dtype)), slab_of(dtype));
 }
@@ -959,6 +1054,10 @@ int opt_in_lds(MltsLdsOptIn& once, const void* kern, int bytes, S what) {
   return MLTS_OK;
 }
 
+// 64 x 64 in fp32: two groups of four wavefronts, a half of every slab each
+template <typename T>
+constexpr int kGroups = sizeof(T) == 4 ? 2 : 1;
+
 template <typename T, int FORM, int BM, int BN, int WM, int WN, int KG = 1>
 int launch_tile(const Product& g, unsigned grid, hipStream_t st) {
   typedef TileShape<T, FORM, BM, BN, WM, WN, KG> S;
@@ -969,27 +1068,25 @@ int launch_tile(const Product& g, unsigned grid, hipStream_t st) {
   hipLaunchKernelGGL(kern, dim3(grid), dim3(S::THREADS), S::LDS, st, g);
   return MLTS_OK;
 }
-// Columns of a wavefront of a 128 x 128 tile: in bf16 eight wavefronts of 128 registers, so that two tiles share a CU (us, four wavefronts /
-// eight: NT 2331 x 1536 x 512 10.6 / 9.4, NN 8192 x 1376 x 512 23.2 / 21.8)
-template <typename T>
-constexpr int k128Columns = sizeof(T) == 2 ? 32 : 64;
+// (128 x 128 in eight wavefronts: in bf16 of 128 registers, so that two tiles share a CU (us, four wavefronts / eight: NT 2331 x 1536 x 512 10.6 / 9.4, NN
+// 8192 x 1376 x 512 23.2 / 21.8))
 
 template <typename T, int FORM>
-int launch_form(int tile, const SmallShape& shape, const Product& g, unsigned grid, hipStream_t st) {
-  if (tile == k128) return launch_tile<T, FORM, 128, 128, 64, k128Columns<T>>(g, grid, st);
-  if (tile == k256x128) return launch_tile<T, FORM, 256, 128, 64, 64>(g, grid, st);
-  if (tile == k256) return launch_tile<T, FORM, 256, 256, 128, 64>(g, grid, st);
+int launch_form(int tile, const Product& g, unsigned grid, hipStream_t st) {
+  if (tile == k128) return launch_tile<T, FORM, 128, 128, 64, 32>(g, grid, st);
+  if (tile == k128x64) return launch_tile<T, FORM, 128, 64, 64, 32>(g, grid, st);
   if constexpr (sizeof(T) == 4) {
-    if (shape.size == 32) return launch_tile<T, FORM, 32, 32, 32, 32, 4>(g, grid, st);
+    if (tile == k32) return launch_tile<T, FORM, 32, 32, 32, 32, 4>(g, grid, st);
   } else {
-    if (tile == k128x64) return launch_tile<T, FORM, 128, 64, 64, 32>(g, grid, st);
+    if (tile == k256x128) return launch_tile<T, FORM, 256, 128, 64, 64>(g, grid, st);
+    if (tile == k256) return launch_tile<T, FORM, 256, 256, 128, 64>(g, grid, st);
   }
-  return launch_tile<T, FORM, 64, 64, 32, 32>(g, grid, st);
+  return launch_tile<T, FORM, 64, 64, 32, 32, kGroups<T>>(g, grid, st);
 }
 template <typename T>
-int launch_alone(int tile, const SmallShape& shape, const Product& g, unsigned grid, hipStream_t st) {
-  if (g.form == FORM_NT) return launch_form<T, FORM_NT>(tile, shape, g, grid, st);
-  return g.form == FORM_NN ? launch_form<T, FORM_NN>(tile, shape, g, grid, st) : launch_form<T, FORM_TN>(tile, shape, g, grid, st);
+int launch_alone(int tile, const Product& g, unsigned grid, hipStream_t st) {
+  if (g.form == FORM_NT) return launch_form<T, FORM_NT>(tile, g, grid, st);
+  return g.form == FORM_NN ? launch_form<T, FORM_NN>(tile, g, grid, st) : launch_form<T, FORM_TN>(tile, g, grid, st);
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int KG = 1>
@@ -1002,16 +1099,16 @@ int launch_rope_tile(const Product& g, const Rotation& rot, unsigned grid, hipSt
   return MLTS_OK;
 }
 template <typename T>
-int launch_rope_alone(int tile, const SmallShape& shape, const Product& g, const Rotation& rot, unsigned grid, hipStream_t st) {
-  if (tile == k128) return launch_rope_tile<T, 128, 128, 64, k128Columns<T>>(g, rot, grid, st);
-  if (tile == k256x128) return launch_rope_tile<T, 256, 128, 64, 64>(g, rot, grid, st);
-  if (tile == k256) return launch_rope_tile<T, 256, 256, 128, 64>(g, rot, grid, st);
+int launch_rope_alone(int tile, const Product& g, const Rotation& rot, unsigned grid, hipStream_t st) {
+  if (tile == k128) return launch_rope_tile<T, 128, 128, 64, 32>(g, rot, grid, st);
+  if (tile == k128x64) return launch_rope_tile<T, 128, 64, 64, 32>(g, rot, grid, st);
   if constexpr (sizeof(T) == 4) {
-    if (shape.size == 32) return launch_rope_tile<T, 32, 32, 32, 32, 4>(g, rot, grid, st);
+    if (tile == k32) return launch_rope_tile<T, 32, 32, 32, 32, 4>(g, rot, grid, st);
   } else {
-    if (tile == k128x64) return launch_rope_tile<T, 128, 64, 64, 32>(g, rot, grid, st);
+    if (tile == k256x128) return launch_rope_tile<T, 256, 128, 64, 64>(g, rot, grid, st);
+    if (tile == k256) return launch_rope_tile<T, 256, 256, 128, 64>(g, rot, grid, st);
   }
-  return launch_rope_tile<T, 64, 64, 32, 32>(g, rot, grid, st);
+  return launch_rope_tile<T, 64, 64, 32, 32, kGroups<T>>(g, rot, grid, st);
 }
 template <typename T, int BM, int BN, int WM, int WN, int KG>
 int launch_rope_joint(const Products& ps, const Rotation& rot, int blocks, hipStream_t st) {
@@ -1118,31 +1215,32 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
   auto launch = [&] {  // what `joint` holds
     if (!together) return static_cast<int>(MLTS_OK);
     int64_t tiles[kMaxProducts], at = 0;  // of an XCD
-    const int64_t grid = 8 * spread(joint.p, together, plan.rows_of(joint_tile), plan.columns_of(joint_tile), tiles);
+    const int64_t grid = 8 * spread(joint.p, together, joint_tile, dtype, tiles);
     MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm: too many tiles");
     for (int i = 0; i < together; ++i) joint.first[i] = static_cast<int>(at), at += 8 * tiles[i];  // (whole rounds over the XCDs, so that each product starts at the first)
     const int blocks = static_cast<int>(grid);
     const int forms = joint.more.count ? FORMS_SEGMENTS : all_nt ? FORMS_NT : all_nn ? FORMS_NN : FORMS_ANY;
     if constexpr (sizeof(T) == 4) {
-      if (plan.shape.size == 32) {
+      if (joint_tile == k32) {
         if (activation) return launch_act_joint<T, 32, 32, 32, 32, 4>(joint, *activation, blocks, st);
         if (rotation) return launch_rope_joint<T, 32, 32, 32, 32, 4>(joint, rot, blocks, st);
         return launch_joint_forms<T, 32, 32, 32, 32, 4>(forms, joint, blocks, st);
       }
-    } else if (joint_tile == k128) {
+    }
+    if (joint_tile == k128) {
       if (activation) return launch_act_joint<T, 128, 128, 64, 32, 1>(joint, *activation, blocks, st);
       if (rotation) return launch_rope_joint<T, 128, 128, 64, 32, 1>(joint, rot, blocks, st);
       return launch_joint_forms<T, 128, 128, 64, 32, 1>(forms, joint, blocks, st);
     }
-    if (activation) return launch_act_joint<T, 64, 64, 32, 32, 1>(joint, *activation, blocks, st);
-    if (rotation) return launch_rope_joint<T, 64, 64, 32, 32, 1>(joint, rot, blocks, st);
-    return launch_joint_forms<T, 64, 64, 32, 32, 1>(forms, joint, blocks, st);
+    if (activation) return launch_act_joint<T, 64, 64, 32, 32, kGroups<T>>(joint, *activation, blocks, st);
+    if (rotation) return launch_rope_joint<T, 64, 64, 32, 32, kGroups<T>>(joint, rot, blocks, st);
+    return launch_joint_forms<T, 64, 64, 32, 32, kGroups<T>>(forms, joint, blocks, st);
   };
   clear();
   MltsKernelTimer timer("gemm", st);
   for (int i = 0; i < count; ++i) {
     const mlts_gemm_product& p = ps[i];
-    const int bm = plan.rows_of(plan.tile[i]), bn = plan.columns_of(plan.tile[i]);
+    const int bm = kTileM[plan.tile[i]], bn = kTileN[plan.tile[i]];
     Product g{};
     g.a = p.a[0], g.b = p.b[0], g.c = p.c;
     g.lda = static_cast<int>(p.lda[0]), g.ldb = static_cast<int>(p.ldb[0]), g.ldc = static_cast<int>(p.ldc), g.K = static_cast<int>(p.k[0]);
@@ -1155,7 +1253,6 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
         if (int rc = launch(); rc != MLTS_OK) return rc;
         clear();
       }
-      g.k_slice = g.K;
       for (int k = 1; k < p.segments; ++k) {
         joint.more.a[k - 1] = p.a[k], joint.more.b[k - 1] = p.b[k];
         joint.more.lda[k - 1] = static_cast<int>(p.lda[k]), joint.more.ldb[k - 1] = static_cast<int>(p.ldb[k]), joint.more.K[k - 1] = static_cast<int>(p.k[k]);
@@ -1176,13 +1273,13 @@ int run(const mlts_gemm_product* ps, int count, int dtype, float* workspace, con
       continue;
     }
     int64_t tiles;
-    const int64_t grid = 8 * spread(&g, 1, bm, bn, &tiles);
+    const int64_t grid = 8 * spread(&g, 1, plan.tile[i], dtype, &tiles);
     MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm: too many tiles");
     if (rotation) {
       Rotation own = *rotation;
       std::copy(rotation->columns[i], rotation->columns[i] + 4, own.columns[0]);
-      if (int rc = launch_rope_alone<T>(plan.tile[i], plan.shape, g, own, static_cast<unsigned>(grid), st); rc != MLTS_OK) return rc;
-    } else if (int rc = launch_alone<T>(plan.tile[i], plan.shape, g, static_cast<unsigned>(grid), st); rc != MLTS_OK) {
+      if (int rc = launch_rope_alone<T>(plan.tile[i], g, own, static_cast<unsigned>(grid), st); rc != MLTS_OK) return rc;
+    } else if (int rc = launch_alone<T>(plan.tile[i], g, static_cast<unsigned>(grid), st); rc != MLTS_OK) {
       return rc;
     }
   }
@@ -1196,21 +1293,23 @@ int pair_tile(int64_t M, int64_t N, int64_t K, int dtype) {
   const mlts_gemm_product both = single(FORM_NT, M, 2 * N, K, nullptr, K, nullptr, K, nullptr, 2 * N, 0);
   const LaunchPlan plan(&both, 1, dtype);
   if (plan.slices[0] > 1) return -1;
-  if (dtype == MLTS_F32) return plan.tile[0] == k256 || (plan.tile[0] == kSmall && plan.shape.size != 64) ? -1 : plan.tile[0];
   const mlts_gemm_product* const one = &both;
   const int64_t whole = 1;
-  const auto time = [&](int tile) { return bf16_time(&one, 1, tile, &whole, true) + pass_time(kPairCost, tile, M, N); };
-  return time(k128) < time(kSmall) ? k128 : kSmall;
+  const auto time = [&](int tile) { return launch_time(dtype, &one, 1, tile, &whole, true) + (dtype == MLTS_BF16 ? pass_time(kPairCost, tile, M, N) : 0); };
+  if (dtype == MLTS_BF16) return time(k128) < time(kSmall) ? k128 : kSmall;
+  if (plan.tile[0] != k32) return plan.tile[0] == kSmall ? kSmall : k128;  // (these sum in one order: the bits of the product with both weights)
+  const double pass = 2.5 + 2.4e-6 * static_cast<double>(M) * static_cast<double>(N);  // (32 x 32 has no pair: the pass over gate and up is then a launch of its own)
+  return time(k32) + pass < time(kSmall) ? -1 : kSmall;
 }
 
-template <typename T, int BM, int BN, int WM, int WN>
+template <typename T, int BM, int BN, int WM, int WN, int KG = 1>
 int launch_pair(Product& g, const Pair& pair, hipStream_t st) {
-  typedef TileShape<T, FORM_NT, BM, BN, WM, WN, 1, true> S;
+  typedef TileShape<T, FORM_NT, BM, BN, WM, WN, KG, true> S;
   g.tiles_m = (g.M + BM - 1) / BM, g.tiles_n = (g.N + BN / 2 - 1) / (BN / 2);
   int64_t tiles;
-  const int64_t grid = 8 * spread(&g, 1, BM, BN, &tiles);
+  const int64_t grid = 8 * spread(&g, 1, BM == 128 ? k128 : kSmall, sizeof(T) == 2 ? MLTS_BF16 : MLTS_F32, &tiles);
   MLTS_REQUIRE(grid < (int64_t{1} << 30), "mlts_gemm_swiglu: too many tiles");
-  auto kern = gemm_pair_kernel<T, BM, BN, WM, WN>;
+  auto kern = gemm_pair_kernel<T, BM, BN, WM, WN, KG>;
   static MltsLdsOptIn once;
   if (int rc = opt_in_lds(once, reinterpret_cast<const void*>(kern), S::LDS, "mlts_gemm_swiglu"); rc != MLTS_OK) return rc;
   MltsKernelTimer timer("gemm_swiglu", st);
@@ -1219,11 +1318,8 @@ int launch_pair(Product& g, const Pair& pair, hipStream_t st) {
 }
 template <typename T>
 int run_pair(int tile, Product& g, const Pair& pair, hipStream_t st) {
-  if (tile == k128) return launch_pair<T, 128, 128, 64, k128Columns<T>>(g, pair, st);
-  if constexpr (sizeof(T) == 4) {
-    if (tile == k256x128) return launch_pair<T, 256, 128, 64, 64>(g, pair, st);
-  }
-  return launch_pair<T, 64, 64, 32, 32>(g, pair, st);
+  if (tile == k128) return launch_pair<T, 128, 128, 64, 32>(g, pair, st);
+  return launch_pair<T, 64, 64, 32, 32, kGroups<T>>(g, pair, st);
 }
 
 }  // namespace
@@ -1253,7 +1349,7 @@ extern "C" int mlts_gemm_plan(const mlts_gemm_product* products, int32_t count, 
     Product g{};
     int64_t each;
     g.tiles_m = static_cast<int>((products[0].M + kTileM[tile] - 1) / kTileM[tile]), g.tiles_n = static_cast<int>((2 * products[0].N + kTileN[tile] - 1) / kTileN[tile]), g.slices = 1;
-    tiles[0] = {kTileM[tile], kTileN[tile], 1, 0, static_cast<int32_t>(std::min<int64_t>(spread(&g, 1, kTileM[tile], kTileN[tile], &each), 0x7fffffff))};
+    tiles[0] = {kTileM[tile], kTileN[tile], 1, 0, static_cast<int32_t>(std::min<int64_t>(spread(&g, 1, tile, dtype, &each), 0x7fffffff))};
     return MLTS_OK;
   }
   const LaunchPlan plan(products, count, dtype, with == MLTS_GEMM_WITH_ACTIVATION, with == MLTS_GEMM_WITH_ROTATION);
@@ -1263,11 +1359,11 @@ extern "C" int mlts_gemm_plan(const mlts_gemm_product* products, int32_t count, 
   for (int i = 0; i < count; ++i) {
     Product g{};
     set_tiles(g, products[i], plan, i, dtype);
-    const int bm = plan.rows_of(plan.tile[i]), bn = plan.columns_of(plan.tile[i]);
-    tiles[i] = {bm, bn, static_cast<int32_t>(plan.slices[i]), plan.together[i], static_cast<int32_t>(std::min<int64_t>(spread(&g, 1, bm, bn, each), 0x7fffffff))};
+    const int bm = kTileM[plan.tile[i]], bn = kTileN[plan.tile[i]];
+    tiles[i] = {bm, bn, static_cast<int32_t>(plan.slices[i]), plan.together[i], static_cast<int32_t>(std::min<int64_t>(spread(&g, 1, plan.tile[i], dtype, each), 0x7fffffff))};
     if (plan.together[i] && g.tiles_m && g.tiles_n) joint[together++] = g, joint_tile = plan.tile[i];
   }
-  const int64_t busiest = spread(joint, together, plan.rows_of(joint_tile), plan.columns_of(joint_tile), each);
+  const int64_t busiest = spread(joint, together, joint_tile, dtype, each);
   for (int i = 0; i < count; ++i)
     if (plan.together[i]) tiles[i].busiest = static_cast<int32_t>(std::min<int64_t>(busiest, 0x7fffffff));
   return MLTS_OK;

@@ -21,10 +21,8 @@ namespace {
 
 // Where the own kernels run, by M * N * K.  A product through torch costs 18 us of host time, a call here 5, and that is what
 // small steps wait for.  On the GPU alone (both sides timed with the weights out of HBM; rows from 100 to 16384; the library's choice
-// untuned) they are ahead of the library
-//   fp32  0.5 to 1e9  0.86 of its time (y), 0.86 (dx), 0.82 (dW)    2.5 to 3e9  0.90, 0.92, 0.87    3 to 4e9  1.13, 1.15, 1.17
-//   bf16  up to 4e9   0.4 to 0.95
-constexpr double kOwnLimitBf16 = 4.0e9, kOwnLimitF32 = 3.0e9;
+// untuned) they are ahead of the library in fp32 at every size (0.6 to 0.9 of its time from 5e8 to 2.5e10, and its errors are larger), in bf16 up to 4e9 (0.4 to 0.95)
+constexpr double kOwnLimitBf16 = 4.0e9;
 
 // Larger bf16 products, by what running one of them on the own kernels adds to a layer's training step in which the library has the others (us; 145
 // layers of 21 shapes, 256 to 2048 wide, of 3000 to 32768 rows; two runs differ by 4 us).  These lines take 7 % off a layer's step on the mean, and the
@@ -75,8 +73,7 @@ bool long_contraction_bf16(int64_t M, int64_t N, int64_t K) {
 
 bool within_own_range(int form, int dtype, int64_t M, int64_t N, int64_t K, Use use) {
   const double size = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K);
-  if (dtype == MLTS_F32) return size <= kOwnLimitF32;
-  return size <= kOwnLimitBf16 || larger_own_range_bf16(form, M, N, K, use) || (form == MLTS_GEMM_NN && long_contraction_bf16(M, N, K));
+  return dtype == MLTS_F32 || size <= kOwnLimitBf16 || larger_own_range_bf16(form, M, N, K, use) || (form == MLTS_GEMM_NN && long_contraction_bf16(M, N, K));
 }
 
 struct Sizes {

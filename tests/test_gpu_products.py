@@ -371,3 +371,50 @@ def test_every_bf16_tile_rotated(dev, case, tile):
     B, S, H, Hkv, D, K, given = case
     assert planned([(NT, B * S, (H + 2 * Hkv) * D, K)], sharing=1) == [tile]
     test_rotation_in_the_products(dev, torch.bfloat16, B, S, H, Hkv, D, K, False, given)
+
+
+# fp32 products and the tile and slices that each is planned with: ragged rows, columns and slabs of the tiles of elements in three parts
+PARTS_CASES = [((NT, 901, 2052, 396), (64, 64, 1)), ((NN, 777, 1324, 516), (64, 64, 1)), ((TN, 1324, 252, 2047), (64, 64, 2)), ((NT, 2111, 2652, 332), (128, 64, 1)),
+               ((NT, 2047, 4100, 260), (128, 128, 1)), ((NN, 2041, 260, 8196), (128, 128, 4)), ((TN, 8196, 260, 1999), (128, 128, 1))]
+
+
+@pytest.mark.parametrize("product,tile", PARTS_CASES, ids=lambda v: "-".join(map(str, v)))
+def test_fp32_in_three_parts(dev, product, tile):
+    """Errors of one rounding in sixteen terms (a random walk of 2^-24 steps) and of the parts that are left out, which fp32 matrix instructions exceed; and operands that have
+    no parts: infinities, NaN and numbers that bf16 rounds to infinity give what fp32 gives, in their rows and columns alone."""
+    form, M, N, K = product
+    assert planned([product], _lib.MLTS_F32) == [tile]
+    a, b = operands(form, M, N, K, torch.float32, dev, M + N)
+    want = expected(form, a, b)
+    out = torch.empty(M, N, device=dev)
+    run_products([(form, [(a, b)], out, 0)], torch.float32)
+    assert (out.double() - want).norm() <= 2.0**-24 * (3 + (K / 16) ** 0.5) * want.norm()
+    run_products([(form, [(a, b)], out, 1)], torch.float32)
+    assert (out.double() - 2 * want).norm() <= 2.0**-23 * (4 + (K / 16) ** 0.5) * want.norm()
+    rows, columns = a.t() if form == TN else a, b.t() if form == NT else b   # [M, K], [K, N]
+    rows[3, 5], rows[M - 1, K - 1], rows[70, 0] = float("inf"), float("nan"), 3.4e38
+    columns[:, 7] *= 1e-3
+    columns[2, N - 1], columns[0, N - 1] = float("-inf"), 0.5   # (row 70 stays in range there, on its way to -inf)
+    run_products([(form, [(a, b)], out, 0)], torch.float32)
+    want = expected(form, a, b)
+    exact = want.float().double()   # (beyond fp32's range: infinite)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out == float("inf"), exact == float("inf")) and torch.equal(out == float("-inf"), exact == float("-inf"))
+    fine = exact.isfinite()
+    fine[70] = False
+    assert (out.double() - want)[fine].norm() <= 2.0**-24 * (3 + K**0.5) * want[fine].norm()   # (whole fp32 elements beside those: a rounding a term)
+    assert abs(out[70, 7].double() / want[70, 7] - 1) <= 1e-6
+
+
+def test_fp32_sum_over_segments_in_slices(dev):
+    """A sum over segments whose slabs are split over workgroups, alone and beside a weight gradient: slices that begin and end within segments."""
+    gen = torch.Generator().manual_seed(8)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen).to(dev)
+    for M, N, ks in ((200, 64, (520, 1000, 72)), (777, 132, (40, 1376)), (64, 256, (2000, 36, 516))):
+        segments = [(rnd(M, k), rnd(k, N)) for k in ks]
+        want, K = sum(expected(NN, a, b) for a, b in segments), sum(ks)
+        for others in (0, 1):
+            c, dw, dy = rnd(M, N), torch.empty(ks[0], N, device=dev), rnd(M, N)
+            total = want + c.double()
+            run_products([(NN, segments, c, 1)] + [(TN, [(segments[0][0], dy)], dw, 0)] * others, torch.float32)
+            assert (c.double() - total).norm() <= 2.0**-24 * (4 + K**0.5) * total.norm()
+            assert not others or (dw.double() - expected(TN, segments[0][0], dy)).norm() <= 2.0**-24 * (4 + M**0.5) * dw.double().norm()
