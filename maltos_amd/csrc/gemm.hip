@@ -175,6 +175,7 @@ struct Pair {
   const void* b2;
   void *c2, *h;
   int ldh;
+  bool large;  // gate and up are kept, and h does not fit the L2s
 };
 // Rotary positions on the way out of an NT product whose rows are tokens and whose columns are heads: rounded x_even, x_odd become
 // x_even cos - x_odd sin, x_even sin + x_odd cos with the roundings of the pass over them (mlts_rope).
@@ -206,6 +207,11 @@ __device__ __forceinline__ void rotate(float& even, float& odd, float c, float s
   even = round_to<T>(xe * c) - round_to<T>(xo * s);
   odd = round_to<T>(xe * s) + round_to<T>(xo * c);
 }
+// Buffer stores past the caches: of what is not read again before more than they hold was written.  Gate and up that are kept for a backward pass are (16384 x 2 x 688 x 384 48 -> 35 us,
+// 8192 x 2 x 1376 x 512 46 -> 40, 4096 x 2 x 1024 x 256 14.1 -> 12.9); so is h beside them where it exceeds the 32 MB of the eight L2s (16384 x 2 x 1376 x 512 94 -> 92 without it,
+// -> 74; a training step of 16384 tokens of the 50M model 8777 -> 8674, of 4000 tokens 3201 -> 3188).  Below that, and where gate and up are not kept, the product behind reads h out of the
+// caches (evaluation of 2331 tokens with h past them 617 -> 649).  No gain, or a loss, in steps: the rotated q, k, v, dense C, d gate and d up likewise, gate and up read so.
+constexpr int kNontemporal = 2;
 // Where a tile's rows are read and written four columns at a time: the bounds check of a buffer descriptor stands for a branch over the rows and
 // columns past the end at every access, which all passes of a tile would wait behind.  (Rows too far apart for the descriptor's 32-bit
 // offsets: pointers.)
@@ -230,10 +236,11 @@ struct Window {
     at = static_cast<T*>(const_cast<void*>(base)) + row * ld + col;
     rows = col < columns ? existing - row : 0;
   }
+  template <int POLICY = 0>
   __device__ __forceinline__ void put(int row, t4 v) const {
     if (near) {
-      if constexpr (ES == 2) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, 0);
-      else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, 0);
+      if constexpr (ES == 2) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, POLICY);
+      else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, offset + row * static_cast<uint32_t>(ld * ES), 0, POLICY);
     } else if (row < rows) {
       *reinterpret_cast<t4*>(at + row * ld) = v;
     }
@@ -661,8 +668,9 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
           gate[e] = from_f32<T>(a[e]), up[e] = from_f32<T>(b[e]);
           h[e] = from_f32<T>(round_to<T>(silu(to_f32<T>(gate[e]))) * to_f32<T>(up[e]));
         }
-        if (g.c) out.put(32 * i + rr, gate), out2.put(32 * i + rr, up);
-        out_h.put(32 * i + rr, h);
+        if (g.c) out.template put<kNontemporal>(32 * i + rr, gate), out2.template put<kNontemporal>(32 * i + rr, up);
+        if (pair->large) out_h.template put<kNontemporal>(32 * i + rr, h);
+        else out_h.put(32 * i + rr, h);
       }
       continue;
     }
@@ -1423,7 +1431,7 @@ extern "C" int mlts_gemm_swiglu(int32_t dtype, int64_t M, int64_t N, int64_t K, 
   g.lda = static_cast<int>(ldx), g.ldb = static_cast<int>(ldw), g.ldc = static_cast<int>(ldc);
   g.M = static_cast<int>(M), g.N = static_cast<int>(N), g.K = static_cast<int>(K);
   g.form = FORM_NT, g.slices = 1, g.k_slice = static_cast<int>(K);
-  const Pair pair{w_up, up, h, static_cast<int>(ldh)};
+  const Pair pair{w_up, up, h, static_cast<int>(ldh), up && M * N * (dtype == MLTS_BF16 ? 2 : 4) > int64_t{32} << 20};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int tile = pair_tile(M, N, K, dtype);
   return dtype == MLTS_BF16 ? run_pair<bf16_t>(tile, g, pair, st) : run_pair<float>(tile, g, pair, st);
