@@ -139,6 +139,20 @@ int mlts_attn_bwd(const mlts_attn_shape* s, const void* dout, const int64_t do_s
                   const int64_t dv_stride[3], int accumulate_f32, void* workspace, int64_t workspace_bytes,
                   mlts_stream_t stream);
 
+/* mlts_attn_bwd with MLTS_BWD_OVERWRITE of queries and keys that were rotated (mlts_rope_pair, mlts_gemm_rope), and mlts_rope_pair with `inverse` over dq
+ * and dk in place: the same values (bf16: the same bits), where a kernel of this shape can without a pass of its own.  Sq and Sk are equal.  cos, sin, max_pos,
+ * positions and position_offset as mlts_rope takes them, and refused as there. */
+typedef struct {
+  const void *cos, *sin;
+  const int32_t* positions;
+  int32_t max_pos, position_offset;
+} mlts_attn_rotation;
+int mlts_attn_bwd_rope(const mlts_attn_shape* s, const void* dout, const int64_t do_stride[3], const void* q,
+                       const void* k, const void* v, const void* o, const float* lse, void* dq,
+                       const int64_t dq_stride[3], void* dk, const int64_t dk_stride[3], void* dv,
+                       const int64_t dv_stride[3], const mlts_attn_rotation* rotation, void* workspace,
+                       int64_t workspace_bytes, mlts_stream_t stream);
+
 /* mlts_attn_bwd for callers that cannot allocate device memory or bring a workspace (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments and
  * results as mlts_attn_bwd with a workspace of exactly mlts_attn_bwd_workspace_bytes (the recomputing backward); the

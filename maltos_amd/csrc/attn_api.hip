@@ -199,7 +199,7 @@ int attn_bwd_bf16(AttnBwdParams bp, int D, int mode, float* delta_ws, void* lse2
 int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, const int64_t do_stride[3], const void* q,
                   const void* k, const void* v, const void* o, const float* lse, void* dq, const int64_t dq_stride[3],
                   void* dk, const int64_t dk_stride[3], void* dv, const int64_t dv_stride[3], int accumulate_f32,
-                  void* workspace, int64_t workspace_bytes, hipStream_t st) {
+                  const mlts_attn_rotation* rotation, void* workspace, int64_t workspace_bytes, hipStream_t st) {
   MLTS_REQUIRE(dout && q && k && v && o && lse && dq && dk && dv, "%s: null tensor pointer", who);
   MLTS_REQUIRE(do_stride && dq_stride && dk_stride && dv_stride, "%s: null stride pointer", who);
   MLTS_REQUIRE(accumulate_f32 >= MLTS_BWD_OVERWRITE && accumulate_f32 <= MLTS_BWD_DQ_STORE, "%s: unknown accumulate_f32 mode %d", who,
@@ -229,6 +229,8 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
   bp.dq_f32 = dq_f32;
   bp.nkt = 0;
   bp.delta_out = bp.lse2_out = nullptr;
+  bp.rot = {};
+  if (rotation) bp.rot = {rotation->cos, rotation->sin, rotation->positions, rotation->max_pos, rotation->position_offset, static_cast<int>(s->Sq), static_cast<int>(s->D / 2)};
   if (uses_mfma(s)) {
     MLTS_REQUIRE(mlts_aligned16(dout) && mlts_aligned16(q) && mlts_aligned16(k) && mlts_aligned16(v) &&
                      mlts_aligned16(dq) && mlts_aligned16(dk) && mlts_aligned16(dv),
@@ -246,7 +248,10 @@ int attn_bwd_impl(const char* who, const mlts_attn_shape* s, const void* dout, c
       if (int rc = mlts_attn_small_bwd_dq(bp, s->D, s->mask_mode, st); rc != MLTS_OK) return rc;
       return mlts_attn_small_bwd_dkv(bp, s->D, s->mask_mode, st);
     }
-    return mlts_attn_tile16_bwd(bp, s->D, s->mask_mode, st);
+    if (int rc = mlts_attn_tile16_bwd(bp, s->D, s->mask_mode, st); rc != MLTS_OK || !rotation) return rc;
+    // (the general kernels rotate nothing)
+    return mlts_rope_pair(dq, dq_stride, dq, dq_stride, s->Hq, dk, dk_stride, dk, dk_stride, s->Hkv, rotation->cos, rotation->sin, rotation->max_pos, rotation->positions,
+                          rotation->position_offset, s->B, s->Sq, s->D, s->dtype, 1, st);
   }
   // the dQ kernels form delta themselves from 16-byte chunks of the O rows
   const bool stats_in_dq = s->Sk > 0 && mlts_aligned16(o) && strides_aligned(s->o_stride, 2);
@@ -653,7 +658,28 @@ extern "C" int mlts_attn_bwd(const mlts_attn_shape* s, const void* dout, const i
   MLTS_REQUIRE(why == nullptr, "mlts_attn_bwd: %s", why);
   if (s->B == 0 || (s->Sq == 0 && s->Sk == 0)) return MLTS_OK;
   return attn_bwd_impl("mlts_attn_bwd", s, dout, do_stride, q, k, v, o, lse, dq, dq_stride, dk, dk_stride, dv, dv_stride,
-                       accumulate_f32, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+                       accumulate_f32, nullptr, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mlts_attn_bwd_rope(const mlts_attn_shape* s, const void* dout, const int64_t do_stride[3], const void* q,
+                                  const void* k, const void* v, const void* o, const float* lse, void* dq,
+                                  const int64_t dq_stride[3], void* dk, const int64_t dk_stride[3], void* dv,
+                                  const int64_t dv_stride[3], const mlts_attn_rotation* rotation, void* workspace,
+                                  int64_t workspace_bytes, mlts_stream_t stream) {
+  const char* why = shape_problem(s);
+  MLTS_REQUIRE(why == nullptr, "mlts_attn_bwd_rope: %s", why);
+  MLTS_REQUIRE(rotation, "mlts_attn_bwd_rope: null rotation");
+  MLTS_REQUIRE(s->Sq == s->Sk, "mlts_attn_bwd_rope: queries and keys have one set of positions (%lld and %lld rows)", (long long)s->Sq, (long long)s->Sk);
+  const mlts_attn_rotation& r = *rotation;
+  if (int rc = mlts_rope_check("mlts_attn_bwd_rope", dq, dq_stride, dq, dq_stride, r.cos, r.sin, r.max_pos, r.positions, r.position_offset, s->B, s->Hq, s->Sq, s->D,
+                               s->dtype); rc != MLTS_OK)
+    return rc;
+  if (int rc = mlts_rope_check("mlts_attn_bwd_rope", dk, dk_stride, dk, dk_stride, r.cos, r.sin, r.max_pos, r.positions, r.position_offset, s->B, s->Hkv, s->Sk, s->D,
+                               s->dtype); rc != MLTS_OK)
+    return rc;
+  if (s->B == 0 || s->Sq == 0) return MLTS_OK;
+  return attn_bwd_impl("mlts_attn_bwd_rope", s, dout, do_stride, q, k, v, o, lse, dq, dq_stride, dk, dk_stride, dv, dv_stride,
+                       MLTS_BWD_OVERWRITE, rotation, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mlts_attn_bwd_noalloc(const mlts_attn_shape* s, const void* dout, const int64_t do_stride[3], const void* q,
@@ -686,7 +712,7 @@ extern "C" int mlts_attn_bwd_noalloc(const mlts_attn_shape* s, const void* dout,
     }
   }
   rc = attn_bwd_impl("mlts_attn_bwd_noalloc", s, dout, do_stride, q, k, v, o, lse, dq, dq_stride, dk, dk_stride, dv,
-                     dv_stride, accumulate_f32, ws, need, st);
+                     dv_stride, accumulate_f32, nullptr, ws, need, st);
   if (ordered) {
     if (hipEventRecord(g_scratch_event[dev], st) == hipSuccess) {
       g_scratch_stream[dev] = st;

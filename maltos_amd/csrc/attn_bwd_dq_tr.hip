@@ -528,6 +528,13 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_bwd_dq_tr_kernel(const Att
   if (!bp.dq_f32 && rows16) {
     // bf16 rows through LDS (each wavefront owns 32 rows x RB bytes, tile-row swizzle), so that global stores are
     // 16 bytes per lane and cover whole rows
+    constexpr int CHUNKS = 32 * CPR / 64;
+    const RotateBack rot = rotation_of_kernel();
+    RotateBack::Angles<bf16_t, 4> angles[CHUNKS];  // fetched behind the last tile
+    if (rot.cos) {
+#pragma unroll
+      for (int i = 0; i < CHUNKS; ++i) angles[i] = rot.angles<bf16_t, 4>(rot.row(b, wq0 + (i * 64 + lane) / CPR), lane % CPR * 4);
+    }
     drain_and_barrier();  // every wavefront has finished reading the last K/V tile
     unsigned char* ebase = smem + wave * (32 * RB);
 #pragma unroll
@@ -542,10 +549,11 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_bwd_dq_tr_kernel(const Att
     }
     bf16_t* obase = reinterpret_cast<bf16_t*>(bp.dq_acc) + b * bp.dqs[0] + hq * bp.dqs[1];
 #pragma unroll
-    for (int i = 0; i < 32 * CPR / 64; ++i) {
+    for (int i = 0; i < CHUNKS; ++i) {
       const int idx = i * 64 + lane;
       const int row = idx / CPR, chunk = idx % CPR;
-      const v4i32 x = *reinterpret_cast<const v4i32*>(ebase + row * RB + ((chunk ^ swz<D>(row & 15)) << 4));
+      v4i32 x = *reinterpret_cast<const v4i32*>(ebase + row * RB + ((chunk ^ swz<D>(row & 15)) << 4));
+      if (rot.cos) x = __builtin_bit_cast(v4i32, RotateBack::back(__builtin_bit_cast(bf16x8, x), angles[i]));
       if (wq0 + row < p.Sq) *reinterpret_cast<v4i32*>(obase + static_cast<int64_t>(wq0 + row) * bp.dqs[2] + chunk * 8) = x;
     }
   } else if (qrow < p.Sq && bp.dq_f32) {

@@ -725,6 +725,14 @@ __global__ __launch_bounds__(KB * 128, 2) void attn_bwd_dkdv_split_kernel(const 
       // 32 rows x RB bytes of a stage that nobody reads any more (role 0: last_stage + 1, role 1: last_stage + 2);
       // chunk ^ (4 if row & 4) keeps the two half-wavefronts (rows 4 apart) on different banks
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      constexpr int CHUNKS = 32 * CPR / 64;
+      const RotateBack rot = rotation_of_kernel();
+      const bool rotated = role == 1 && rot.cos;
+      RotateBack::Angles<bf16_t, 4> angles[CHUNKS];
+      if (rotated) {
+#pragma unroll
+        for (int i = 0; i < CHUNKS; ++i) angles[i] = rot.angles<bf16_t, 4>(rot.row(b, wkv0 + (i * 64 + lane) / CPR), lane % CPR * 4);
+      }
       int es = last_stage + 1 + role;
       es = es >= STAGES ? es - STAGES : es;
       unsigned char* ebase = smem + es * STAGE_BYTES + kb * (32 * RB);
@@ -740,10 +748,11 @@ __global__ __launch_bounds__(KB * 128, 2) void attn_bwd_dkdv_split_kernel(const 
       }
       bf16_t* obase = static_cast<bf16_t*>(optr) + b * os[0] + hkv * os[1];
 #pragma unroll
-      for (int i = 0; i < 32 * CPR / 64; ++i) {
+      for (int i = 0; i < CHUNKS; ++i) {
         const int idx = i * 64 + lane;
         const int row = idx / CPR, chunk = idx % CPR;
-        const v4i32 x = *reinterpret_cast<const v4i32*>(ebase + row * RB + ((chunk ^ (((row >> 2) & 1) << 2)) << 4));
+        v4i32 x = *reinterpret_cast<const v4i32*>(ebase + row * RB + ((chunk ^ (((row >> 2) & 1) << 2)) << 4));
+        if (rotated) x = __builtin_bit_cast(v4i32, RotateBack::back(__builtin_bit_cast(bf16x8, x), angles[i]));
         if (wkv0 + row < p.Sk) *reinterpret_cast<v4i32*>(obase + static_cast<int64_t>(wkv0 + row) * os[2] + chunk * 8) = x;
       }
     } else if (bp.accumulate_f32) {

@@ -3,6 +3,8 @@
 #pragma once
 #include "common.hpp"
 
+#include <stddef.h>
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -50,6 +52,62 @@ struct AttnParams {
   const int* qblock_order;
 };
 
+// dQ and dK of rotated queries and keys, rotated back on their way out (mlts_attn_bwd_rope): the roundings of mlts_rope with `inverse`, over the
+// gradients as they would be stored.  A pass of its own reads and writes both once more (us, the kernels and the pass / here: 8 x 8 heads x 2048 of 64 in bf16 165.7 + 14.9 / 172.1,
+// 8 heads x 1023 packed 21.7 + 4.0 / 22.0, fp32 8 x 4 x 256 26.5 + 4.3 / 28.2).
+struct RotateBack {
+  const void *cos, *sin;  // [max_pos][D / 2] of the gradients' type; null: nothing is rotated
+  const int32_t* positions;  // [B, S], or null
+  int max_pos, offset, S, half;
+  // the table row of a gradient row, as an offset; rows past the end have that of the last one
+  __device__ __forceinline__ int64_t row(int b, int s) const {
+    s = min(s, S - 1);
+    int pos = positions ? positions[static_cast<int64_t>(b) * S + s] : offset + s;
+    pos = pos < 0 ? 0 : pos >= max_pos ? max_pos - 1 : pos;  // host validated; keeps reads in bounds
+    return static_cast<int64_t>(pos) * half;
+  }
+  template <typename T, int N>  // entries `pair` .. pair + N - 1 of a table row
+  struct Angles {
+    typedef T vec __attribute__((ext_vector_type(N)));
+    vec c, s;
+  };
+  template <typename T, int N>
+  __device__ __forceinline__ Angles<T, N> angles(int64_t row, int pair) const {
+    typedef typename Angles<T, N>::vec vec;
+    return {*reinterpret_cast<const vec*>(static_cast<const T*>(cos) + row + pair), *reinterpret_cast<const vec*>(static_cast<const T*>(sin) + row + pair)};
+  }
+  template <typename T>
+  static __device__ __forceinline__ void back(float& even, float& odd, T cosine, T sine) {
+#pragma clang fp contract(off)
+    const float xe = round_to<T>(even), xo = round_to<T>(odd), c = to_f32<T>(cosine), s = to_f32<T>(sine);
+    even = round_to<T>(xe * c) + round_to<T>(xo * s);
+    odd = round_to<T>(xo * c) - round_to<T>(xe * s);
+  }
+  template <typename T>
+  static __device__ __forceinline__ f32x4 back(f32x4 v, Angles<T, 2> a) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      float even = v[2 * e], odd = v[2 * e + 1];
+      back<T>(even, odd, a.c[e], a.s[e]);
+      v[2 * e] = even, v[2 * e + 1] = odd;
+    }
+    return v;
+  }
+  // eight stored values
+  static __device__ __forceinline__ bf16x8 back(bf16x8 v, Angles<bf16_t, 4> a) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float even = to_f32<bf16_t>(v[2 * e]), odd = to_f32<bf16_t>(v[2 * e + 1]);
+      back<bf16_t>(even, odd, a.c[e], a.s[e]);
+      v[2 * e] = from_f32<bf16_t>(even), v[2 * e + 1] = from_f32<bf16_t>(odd);
+    }
+    return v;
+  }
+};
+// of mlts_rope and what rotates besides (layers.hip)
+int mlts_rope_check(const char* who, const void* x, const int64_t* x_stride, const void* y, const int64_t* y_stride, const void* cos_tab, const void* sin_tab,
+                    int32_t max_pos, const int32_t* positions, int32_t position_offset, int32_t B, int32_t H, int32_t S, int32_t D, int32_t dtype);
+
 // Backward-only extras.
 struct AttnBwdParams {
   AttnParams a;
@@ -69,7 +127,26 @@ struct AttnBwdParams {
   // lse2_out[B * Hq * Sq + 1] = lse * log2(e) with +inf for rows that saw no key and in the last entry.
   float* delta_out;
   float* lse2_out;
+  RotateBack rot;  // of dq and dk; overwritten ones of the input dtype only
 };
+
+// `rot` of a kernel whose first argument is an AttnBwdParams, fetched where this is called: as a member of the argument it is in scalar registers from the
+// kernel's start, which its loop then lacks (dK/dV at head_dim 64, 8 x 8 x 2048 causal, 103 us, 108 with twelve more).
+__device__ __forceinline__ RotateBack rotation_of_kernel() {
+  RotateBack rot{};
+#ifdef __HIP_DEVICE_COMPILE__
+  typedef const __attribute__((address_space(4))) uint64_t* words;
+  static_assert(sizeof(RotateBack) == 40 && offsetof(AttnBwdParams, rot) % 8 == 0);
+  auto args = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(args));
+  const words at = reinterpret_cast<words>(args + offsetof(AttnBwdParams, rot));
+  uint64_t w[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) w[i] = at[i];
+  __builtin_memcpy(&rot, w, sizeof(rot));
+#endif
+  return rot;
+}
 
 enum AttnPass { ATTN_FWD, ATTN_BWD_DQ, ATTN_BWD_DKV };
 

@@ -112,37 +112,60 @@ __device__ __forceinline__ void accumulate(f32x4 (&acc)[NC], const Columns<NC> (
     for (int db = 0; db < NC; ++db) acc[db] = mfma4(rows[i].v[db], x[i], acc[db]);
 }
 
+// What a row's result becomes before it is stored: nothing else, or rotated back (columns d ..+1 or ..+3; D is then a multiple of 4)
+struct AsIs {
+  __device__ __forceinline__ void operator()(int, int, float&, float&) const {}
+  __device__ __forceinline__ f32x4 operator()(int, int, f32x4 v) const { return v; }
+};
+template <int N>
+struct Back {
+  const RotateBack& rot;
+  int64_t table[N];  // negative: not rotated
+  __device__ __forceinline__ void operator()(int n, int d, float& even, float& odd) const {
+    if (table[n] < 0 || d >= 2 * rot.half) return;
+    const auto a = rot.angles<float, 1>(table[n], d / 2);
+    RotateBack::back<float>(even, odd, a.c[0], a.s[0]);
+  }
+  __device__ __forceinline__ f32x4 operator()(int n, int d, f32x4 v) const {
+    return table[n] < 0 || d >= 2 * rot.half ? v : RotateBack::back<float>(v, rot.angles<float, 2>(table[n], d / 2));
+  }
+};
+
 // A row's result as it lies in the accumulators: acc[db][r] is column NC (4 g + r) + db.  Times scale, overwritten or added to.
-template <int NC>
-__device__ __forceinline__ void store_row(float* row, const f32x4 (&acc)[NC], float scale, int g, int D, bool vec, bool add) {
+template <int NC, typename F>
+__device__ __forceinline__ void store_row(float* row, const f32x4 (&acc)[NC], float scale, int g, int D, bool vec, bool add, int n, const F& finish) {
+  f32x4 w[NC];
+#pragma unroll
+  for (int t = 0; t < NC; ++t) {  // (what is loaded, in front of the first store)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[t][e] = acc[(4 * t + e) % NC][(4 * t + e) / NC] * scale;
+    w[t] = finish(n, 4 * NC * g + 4 * t, w[t]);
+  }
 #pragma unroll
   for (int t = 0; t < NC; ++t) {
     const int d = 4 * NC * g + 4 * t;
-    f32x4 w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = acc[(4 * t + e) % NC][(4 * t + e) / NC] * scale;
     if (vec) {
       if (d >= D) continue;
       f32x4* at = reinterpret_cast<f32x4*>(row + d);
-      *at = add ? *at + w : w;
+      *at = add ? *at + w[t] : w[t];
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (d + e < D) row[d + e] = add ? row[d + e] + w[e] : w[e];
+        if (d + e < D) row[d + e] = add ? row[d + e] + w[t][e] : w[t][e];
     }
   }
 }
 
 // N results of 16 rows each, spread over the splits: summed through LDS (N * DP / 16 KiB a split) and stored, every wavefront a part of
 // the columns.  lds: of these splits.  scale, row: as for store_row; row null: not stored.
-template <int NC, int N>
+template <int NC, int N, typename F>
 __device__ __forceinline__ void join_and_store(const f32x4 (&acc)[N][NC], float* lds, int split, int splits, float* const (&row)[N], const float (&scale)[N],
-                                               int lane, int D, bool vec, bool add) {
+                                               int lane, int D, bool vec, bool add, const F& finish) {
   const int g = lane >> 4;
   if (splits == 1) {
 #pragma unroll
     for (int n = 0; n < N; ++n)
-      if (row[n]) store_row(row[n], acc[n], scale[n], g, D, vec, add);
+      if (row[n]) store_row(row[n], acc[n], scale[n], g, D, vec, add, n, finish);
     return;
   }
   __syncthreads();  // nobody needs what the LDS holds any more
@@ -166,6 +189,17 @@ __device__ __forceinline__ void join_and_store(const f32x4 (&acc)[N][NC], float*
       const int d = NC * (4 * g + e);
 #pragma unroll
       for (int db = 0; db < NC; ++db) v[db] *= scale[n];
+      if constexpr (NC % 4 == 0) {
+#pragma unroll
+        for (int t = 0; t < NC; t += 4) {
+          const f32x4 w = finish(n, d + t, f32x4{v[t], v[t + 1], v[t + 2], v[t + 3]});
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[t + e] = w[e];
+        }
+      } else {
+#pragma unroll
+        for (int db = 0; db < NC; db += 2) finish(n, d + db, v[db], v[db + 1]);
+      }
       if (vec && NC % 4 == 0) {
 #pragma unroll
         for (int t = 0; t < NC / 4; ++t) {

@@ -147,7 +147,11 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
     row[r] = there && qrow < p.Sq ? dQ + static_cast<int64_t>(qrow) * bp.dqs[2] : nullptr;
     scale[r] = p.scale;
   }
-  join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1);
+  const RotateBack rot = rotation_of_kernel();
+  Back<R> back{rot, {}};
+#pragma unroll
+  for (int r = 0; r < R; ++r) back.table[r] = rot.cos ? rot.row(b, q0 + 16 * r + l16) : -1;
+  join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1, back);
 }
 
 template <int DP>
@@ -312,7 +316,11 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     row[R + r] = mine ? static_cast<float*>(bp.dv) + b * bp.dvs[0] + hkv * bp.dvs[1] + krow * bp.dvs[2] : nullptr;
     scale[r] = p.scale, scale[R + r] = 1.f;
   }
-  join_and_store(dkv, lds + slot * splits * 2 * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0);
+  const RotateBack rot = rotation_of_kernel();
+  Back<2 * R> back{rot, {}};
+#pragma unroll
+  for (int r = 0; r < R; ++r) back.table[r] = rot.cos ? rot.row(b, kb0 + 16 * r + l16) : -1, back.table[R + r] = -1;
+  join_and_store(dkv, lds + slot * splits * 2 * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0, back);
 }
 
 template <int DP, int R, bool DOC, int LAYOUT>

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_fwd(cons
     p.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] = l > 0.f ? m + logf(l) : -INFINITY;
   float* const row[1] = {there && qrow < p.Sq ? static_cast<float*>(p.o) + b * p.os[0] + hq * p.os[1] + static_cast<int64_t>(qrow) * p.os[2] : nullptr};
   const float scale[1] = {l > 0.f ? 1.0f / l : 0.f};
-  join_and_store(o, lds + slot * splits * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, false);
+  join_and_store(o, lds + slot * splits * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, false, AsIs{});
 }
 
 template <int DP, bool DOC, int LAYOUT>

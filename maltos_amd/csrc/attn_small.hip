@@ -138,10 +138,15 @@ struct Walk {
   }
 };
 
-// The splits' sums of N results of 16 rows, and what becomes of them: acc[n][db] are columns 16 db + 4 g ..+3 of this lane's row
-template <int NC, int N, typename F>
-__device__ __forceinline__ void join_and_store(f32x4 (&acc)[N][NC], f32x4* lds, const Place& at, F store) {
+// The splits' sums of N results of 16 rows, and what becomes of them: acc[n][db] are columns 16 db + 4 g ..+3 of this lane's row.  finish: what a sum
+// becomes before it is stored, which may load (ahead of the first store)
+template <int NC, int N, typename F, typename G>
+__device__ __forceinline__ void join_and_store(f32x4 (&acc)[N][NC], f32x4* lds, const Place& at, G finish, F store) {
   if (at.splits == 1) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+      for (int db = 0; db < NC; ++db) acc[n][db] = finish(n, db, acc[n][db]);
 #pragma unroll
     for (int n = 0; n < N; ++n)
 #pragma unroll
@@ -160,7 +165,7 @@ __device__ __forceinline__ void join_and_store(f32x4 (&acc)[N][NC], f32x4* lds, 
     for (int db = (at.split - n * NC) & (at.splits - 1); db < NC; db += at.splits) {
       f32x4 v = lds[(n * NC + db) * 64];
       for (int s = 1; s < at.splits; ++s) v += lds[((s * N + n) * NC + db) * 64];
-      store(n, db, v);
+      store(n, db, finish(n, db, v));
     }
 }
 
@@ -336,9 +341,9 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_fwd(const AttnPara
       p.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] = l[r] > 0.f ? m[r] + logf(l[r]) : -INFINITY;
     scale[r] = l[r] > 0.f ? 1.0f / l[r] : 0.f;
   }
-  join_and_store(o, reinterpret_cast<f32x4*>(lds_raw), at, [&](int r, int db, f32x4 v) {
+  join_and_store(o, reinterpret_cast<f32x4*>(lds_raw), at, [&](int r, int, f32x4 v) { return v * scale[r]; }, [&](int r, int db, f32x4 v) {
     const int qrow = q0 + 16 * r + l16;
-    if (at.there && qrow < p.Sq) store4(p.o, row + qrow * p.os[2] + 16 * db, v * scale[r], 0);
+    if (at.there && qrow < p.Sq) store4(p.o, row + qrow * p.os[2] + 16 * db, v, 0);
   });
 }
 
@@ -485,9 +490,18 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     k0 = kn, kn = kn2;
   }
   const int64_t row = b * bp.dqs[0] + hq * bp.dqs[1] + 4 * g;
-  join_and_store(dq, reinterpret_cast<f32x4*>(lds_raw), at, [&](int r, int db, f32x4 v) {
+  const RotateBack rot = rotation_of_kernel();
+  int64_t table[R];
+  if (rot.cos) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) table[r] = rot.row(b, q0 + 16 * r + l16);
+  }
+  const auto finish = [&](int r, int db, f32x4 v) {
+    return rot.cos ? RotateBack::back<bf16_t>(v * p.scale, rot.angles<bf16_t, 2>(table[r], 8 * db + 2 * g)) : v * p.scale;
+  };
+  join_and_store(dq, reinterpret_cast<f32x4*>(lds_raw), at, finish, [&](int r, int db, f32x4 v) {
     const int qrow = q0 + 16 * r + l16;
-    if (at.there && qrow < p.Sq) store4(bp.dq_acc, row + qrow * bp.dqs[2] + 16 * db, v * p.scale, bp.dq_f32);
+    if (at.there && qrow < p.Sq) store4(bp.dq_acc, row + qrow * bp.dqs[2] + 16 * db, v, bp.dq_f32);
   });
 }
 
@@ -641,10 +655,20 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
   for (int n = 0; n < 2 * R; ++n)
 #pragma unroll
     for (int db = 0; db < NC; ++db) dkv[n][db] = n < R ? dk[n < R ? n : 0][db] : dv[n < R ? 0 : n - R][db];
-  join_and_store(dkv, reinterpret_cast<f32x4*>(lds_raw), at, [&](int n, int db, f32x4 v) {
+  const RotateBack rot = rotation_of_kernel();
+  int64_t table[R];
+  if (rot.cos) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) table[r] = rot.row(b, kb0 + 16 * r + l16);
+  }
+  const auto finish = [&](int n, int db, f32x4 v) {
+    if (n >= R) return v;
+    return rot.cos ? RotateBack::back<bf16_t>(v * p.scale, rot.angles<bf16_t, 2>(table[n < R ? n : 0], 8 * db + 2 * g)) : v * p.scale;
+  };
+  join_and_store(dkv, reinterpret_cast<f32x4*>(lds_raw), at, finish, [&](int n, int db, f32x4 v) {
     const int krow = kb0 + 16 * (n < R ? n : n - R) + l16;
     if (at.there && krow < p.Sk)
-      store4(n < R ? bp.dk : bp.dv, (n < R ? dk_row + krow * bp.dks[2] : dv_row + krow * bp.dvs[2]) + 16 * db, n < R ? v * p.scale : v, bp.accumulate_f32);
+      store4(n < R ? bp.dk : bp.dv, (n < R ? dk_row + krow * bp.dks[2] : dv_row + krow * bp.dvs[2]) + 16 * db, v, bp.accumulate_f32);
   });
 }
 

@@ -641,10 +641,10 @@ extern "C" int mlts_rmsnorm_bwd_accumulate(const void* dy, const void* x, const 
                              hidden, dtype, stream);
 }
 
-// validation shared by mlts_rope and mlts_rope_pair
-static int rope_check(const char* who, const void* x, const int64_t* x_stride, const void* y, const int64_t* y_stride,
-                      const void* cos_tab, const void* sin_tab, int32_t max_pos, const int32_t* positions,
-                      int32_t position_offset, int32_t B, int32_t H, int32_t S, int32_t D, int32_t dtype) {
+// validation shared by mlts_rope, mlts_rope_pair and mlts_attn_bwd_rope
+int mlts_rope_check(const char* who, const void* x, const int64_t* x_stride, const void* y, const int64_t* y_stride,
+                    const void* cos_tab, const void* sin_tab, int32_t max_pos, const int32_t* positions,
+                    int32_t position_offset, int32_t B, int32_t H, int32_t S, int32_t D, int32_t dtype) {
   MLTS_REQUIRE(known_dtype(dtype), "%s: unknown dtype %d", who, dtype);
   MLTS_REQUIRE(B >= 0 && H >= 0 && S >= 0 && D > 0, "%s: bad shape", who);
   const int n = elem_per_vec(dtype);
@@ -668,7 +668,7 @@ extern "C" int mlts_rope(const void* x, const int64_t x_stride[3], void* y, cons
                          const void* cos_tab, const void* sin_tab, int32_t max_pos, const int32_t* positions,
                          int32_t position_offset, int32_t B, int32_t H, int32_t S, int32_t D, int32_t dtype,
                          int32_t inverse, mlts_stream_t stream) {
-  if (int rc = rope_check("mlts_rope", x, x_stride, y, y_stride, cos_tab, sin_tab, max_pos, positions, position_offset, B,
+  if (int rc = mlts_rope_check("mlts_rope", x, x_stride, y, y_stride, cos_tab, sin_tab, max_pos, positions, position_offset, B,
                           H, S, D, dtype); rc != MLTS_OK)
     return rc;
   if (B == 0 || H == 0 || S == 0) return MLTS_OK;
@@ -700,10 +700,10 @@ extern "C" int mlts_rope_pair(const void* xa, const int64_t xa_stride[3], void* 
                               const void* cos_tab, const void* sin_tab, int32_t max_pos, const int32_t* positions,
                               int32_t position_offset, int32_t B, int32_t S, int32_t D, int32_t dtype, int32_t inverse,
                               mlts_stream_t stream) {
-  if (int rc = rope_check("mlts_rope_pair", xa, xa_stride, ya, ya_stride, cos_tab, sin_tab, max_pos, positions,
+  if (int rc = mlts_rope_check("mlts_rope_pair", xa, xa_stride, ya, ya_stride, cos_tab, sin_tab, max_pos, positions,
                           position_offset, B, Ha, S, D, dtype); rc != MLTS_OK)
     return rc;
-  if (int rc = rope_check("mlts_rope_pair", xb, xb_stride, yb, yb_stride, cos_tab, sin_tab, max_pos, positions,
+  if (int rc = mlts_rope_check("mlts_rope_pair", xb, xb_stride, yb, yb_stride, cos_tab, sin_tab, max_pos, positions,
                           position_offset, B, Hb, S, D, dtype); rc != MLTS_OK)
     return rc;
   if (B == 0 || S == 0 || (Ha == 0 && Hb == 0)) return MLTS_OK;

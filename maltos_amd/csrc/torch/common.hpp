@@ -101,6 +101,15 @@ std::tuple<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, c
 std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
                                                       const Tensor& lse, int64_t mask_mode, double scale, const OptTensor& q_pos,
                                                       const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq);
+// rotary positions that q and k were rotated by (rope_pair): their gradients come back rotated back
+struct RotatedBy {
+  const Tensor &cos, &sin;
+  OptTensor positions;
+  int64_t offset;
+};
+std::tuple<Tensor, Tensor, Tensor> rotated_attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                                              const Tensor& lse, int64_t mask_mode, double scale, const OptTensor& q_pos,
+                                                              const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq, const RotatedBy& rotated);
 std::tuple<Tensor, Tensor> rope_pair(const Tensor& xa, const Tensor& xb, const Tensor& cos, const Tensor& sin, const OptTensor& positions,
                                      int64_t position_offset, bool inverse, bool in_place);
 Tensor swiglu_rows(const Tensor& gu, int64_t gate_col, int64_t up_col, int64_t cols);

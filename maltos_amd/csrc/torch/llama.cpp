@@ -591,8 +591,7 @@ Tensor gate_up(const Tensor& x, const AdjacentPtr& rows, const std::vector<Tenso
 
 // ---- attention(rotary(q), rotary(k), v) (models/llama.py:143-150) as one node ---------------------------------------------
 // The same kernels as the separate ops, hence the same values.  What the node adds is the layout of its backward: dQ, dK and
-// dV are head ranges of one [B, S, Hq + 2 Hkv, D] buffer and the rotation of dQ / dK back is done in place there (the buffer
-// is the node's own until it returns), so the gradient of q/k/v projections that run as one product arrives as one matrix.
+// dV are head ranges of one [B, S, Hq + 2 Hkv, D] buffer, dQ and dK rotated back on their way there, so the gradient of q/k/v projections that run as one product arrives as one matrix.
 struct RopeAttentionBackward final : Formula {
   enum { Q, K, V, OUT, LSE, COS, SIN, ROPE_POSITIONS, POSITIONS, SEQUENCES, COUNT };
   int64_t position_offset = 0, mask_mode = 0;
@@ -602,8 +601,8 @@ struct RopeAttentionBackward final : Formula {
   variable_list backward(variable_list&& g, const std::vector<Tensor>& s) override {
     if (!g[0].defined()) return variable_list(3);
     const OptTensor pos = optional_tensor(s[POSITIONS]), seq = optional_tensor(s[SEQUENCES]);
-    auto [dq, dk, dv] = attention_backward(g[0], s[Q], s[K], s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq);
-    rope_pair(dq, dk, s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset, true, true);
+    auto [dq, dk, dv] =
+        rotated_attention_backward(g[0], s[Q], s[K], s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq, {s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset});
     return {dq, dk, dv};
   }
 };
@@ -702,8 +701,8 @@ struct AttentionBlockBackward final : BlockFormula {
     auto [dvo, dwo] = output_grads(g[0], s[OUT_W], as_rows(s[OUT]), need);
     if (!dvo.defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), dwo};
     const OptTensor pos = optional_tensor(s[POSITIONS]), seq = optional_tensor(s[SEQUENCES]);
-    auto [dq, dk, dv] = attention_backward(as_heads(dvo, B, S, H * D, 0, H, D), q, k, s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq);
-    rope_pair(dq, dk, s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset, true, true);
+    auto [dq, dk, dv] =
+        rotated_attention_backward(as_heads(dvo, B, S, H * D, 0, H, D), q, k, s[V], s[OUT], s[LSE], mask_mode, scale, pos, pos, seq, seq, {s[COS], s[SIN], optional_tensor(s[ROPE_POSITIONS]), position_offset});
     const std::vector<Tensor> parts = {as_rows(dq), as_rows(dk), as_rows(dv)};
     Tensor dqkv = adjacent_columns(parts, rows->order);
     if (!dqkv.defined()) {

@@ -67,6 +67,15 @@ OptTensor ids32(const OptTensor& t, int64_t batch, int64_t seq, const char* what
   return t->to(at::kInt).contiguous();
 }
 
+void check_tables(const Tensor& x, const Tensor& cos, const Tensor& sin) {
+  const int64_t half = x.size(3) / 2;
+  TORCH_CHECK_VALUE(cos.sizes() == sin.sizes() && cos.dim() == 2 && cos.size(1) * 2 == x.size(3), "cos/sin tables must be [max_pos, ", half,
+                    "], got ", cos.sizes());
+  TORCH_CHECK_VALUE(cos.scalar_type() == x.scalar_type() && sin.scalar_type() == x.scalar_type(),
+                    "cos/sin tables must have the activation dtype (the reference casts them first)");
+}
+const int32_t* ids_ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->const_data_ptr<int32_t>() : nullptr; }
+
 // ---- document-mask plans (mlts_attn_doc_plan) -----------------------------------------------------------------------
 // Every layer of a model, forward and backward, attends under the same ids, so the plan of a call is kept and handed to
 // later calls with the same ids.  "The same" is judged without reading device memory: same address, dtype, shape, strides
@@ -251,7 +260,7 @@ namespace {
 // dq / dk / dv written or added to as `mode` (MLTS_BWD_*) says
 void attention_backward_into(const Tensor& dout_in, const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& o_in,
                              const Tensor& lse_in, Tensor& dq, Tensor& dk, Tensor& dv, int mode, int64_t mask_mode, double scale,
-                             const OptTensor& q_pos, const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq) {
+                             const OptTensor& q_pos, const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq, const RotatedBy* rotated = nullptr) {
   check_attn_inputs(q_in, k_in, v_in);
   for (const Tensor* t : {&dout_in, &q_in, &k_in, &v_in, &o_in, &lse_in}) require_gpu(*t);
   for (const Tensor* t : {&dq, &dk, &dv}) require_gpu(*t);
@@ -275,18 +284,27 @@ void attention_backward_into(const Tensor& dout_in, const Tensor& q_in, const Te
   const int64_t ws_bytes = mlts_attn_bwd_workspace_bytes(&s, mode);
   Tensor ws = workspace(ws_bytes, q);
   const Strides3 dos(dout), dqs(dq), dks(dk), dvs(dv);
+  if (rotated) {
+    require_gpu(rotated->cos), require_gpu(rotated->sin), require_gpu(rotated->positions);
+    check_tables(q, rotated->cos, rotated->sin);
+    const Tensor cos = dense(rotated->cos), sin = dense(rotated->sin);
+    const OptTensor pos = ids32(rotated->positions, B, Sq, "position_ids");
+    const mlts_attn_rotation r{ptr(cos), ptr(sin), ids_ptr(pos), static_cast<int32_t>(cos.size(0)), static_cast<int32_t>(rotated->offset)};
+    check(mlts_attn_bwd_rope(&s, ptr(dout), dos.v, ptr(q), ptr(k), ptr(v), ptr(o), lse.const_data_ptr<float>(), mptr(dq), dqs.v, mptr(dk), dks.v,
+                             mptr(dv), dvs.v, &r, ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
+    return;
+  }
   check(mlts_attn_bwd(&s, ptr(dout), dos.v, ptr(q), ptr(k), ptr(v), ptr(o), lse.const_data_ptr<float>(), mptr(dq), dqs.v, mptr(dk), dks.v,
                       mptr(dv), dvs.v, mode, ws.defined() ? mptr(ws) : nullptr, ws_bytes, current_stream()));
 }
 
-}  // namespace
-
 // dq, dk, dv in the input dtype, as [B, H, S, D] views of [B, S, H, D] storage.  For self-attention (queries and keys of
 // one length) the three are the head ranges [0, Hq), [Hq, Hq + Hkv), [Hq + Hkv, Hq + 2 Hkv) of ONE [B, S, Hq + 2 Hkv, D]
 // buffer: next to each other exactly as the input gradient of projections that run as one product wants them.
-std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+std::tuple<Tensor, Tensor, Tensor> attention_gradients(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
                                                       const Tensor& lse, int64_t mask_mode, double scale, const OptTensor& q_pos,
-                                                      const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq) {
+                                                      const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq,
+                                                       const RotatedBy* rotated) {
   check_attn_inputs(q, k, v);
   require_gpu(q);
   const int64_t B = q.size(0), Hq = q.size(1), Sq = q.size(2), D = q.size(3), Hkv = k.size(1), Sk = k.size(2);
@@ -303,8 +321,21 @@ std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& dout, const 
     dk = bshd_empty(B, Hkv, Sk, D, k.options());
     dv = bshd_empty(B, Hkv, Sk, D, v.options());
   }
-  attention_backward_into(dout, q, k, v, o, lse, dq, dk, dv, MLTS_BWD_OVERWRITE, mask_mode, scale, q_pos, k_pos, q_seq, k_seq);
+  attention_backward_into(dout, q, k, v, o, lse, dq, dk, dv, MLTS_BWD_OVERWRITE, mask_mode, scale, q_pos, k_pos, q_seq, k_seq, rotated);
   return {dq, dk, dv};
+}
+
+}  // namespace
+
+std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                                      const Tensor& lse, int64_t mask_mode, double scale, const OptTensor& q_pos,
+                                                      const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq) {
+  return attention_gradients(dout, q, k, v, o, lse, mask_mode, scale, q_pos, k_pos, q_seq, k_seq, nullptr);
+}
+std::tuple<Tensor, Tensor, Tensor> rotated_attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                                              const Tensor& lse, int64_t mask_mode, double scale, const OptTensor& q_pos,
+                                                              const OptTensor& k_pos, const OptTensor& q_seq, const OptTensor& k_seq, const RotatedBy& rotated) {
+  return attention_gradients(dout, q, k, v, o, lse, mask_mode, scale, q_pos, k_pos, q_seq, k_seq, &rotated);
 }
 
 namespace {
@@ -425,15 +456,6 @@ Tensor rmsnorm_bwd_into(const Tensor& dy_in, const Tensor& dres_in, const Tensor
 }
 
 // ---- RoPE -----------------------------------------------------------------------------------------------------------
-void check_tables(const Tensor& x, const Tensor& cos, const Tensor& sin) {
-  const int64_t half = x.size(3) / 2;
-  TORCH_CHECK_VALUE(cos.sizes() == sin.sizes() && cos.dim() == 2 && cos.size(1) * 2 == x.size(3), "cos/sin tables must be [max_pos, ", half,
-                    "], got ", cos.sizes());
-  TORCH_CHECK_VALUE(cos.scalar_type() == x.scalar_type() && sin.scalar_type() == x.scalar_type(),
-                    "cos/sin tables must have the activation dtype (the reference casts them first)");
-}
-const int32_t* ids_ptr(const OptTensor& t) { return t.has_value() && t->defined() ? t->const_data_ptr<int32_t>() : nullptr; }
-
 Tensor rope(const Tensor& x_in, const Tensor& cos_in, const Tensor& sin_in, const OptTensor& positions, int64_t position_offset, bool inverse) {
   for (const Tensor* t : {&x_in, &cos_in, &sin_in}) require_gpu(*t);
   require_gpu(positions);

@@ -160,3 +160,43 @@ def test_layers_at_once_equal_the_modules_one_by_one(dev, dtype, flat, packed):
         assert torch.equal(p.grad, q[1].grad), name
     if not flat:   # what the modules keep does not stand in the way of a copy
         assert copy.deepcopy(at_once)(batch).equal(at_once(batch))
+
+
+def _rotation_cases():
+    bf16, fp32 = torch.bfloat16, torch.float32
+    yield from ((bf16, 1, 4, 2, 70, 64, False), (bf16, 1, 4, 2, 200, 64, True), (bf16, 2, 4, 4, 513, 64, False))   # 16-row kernels, split
+    yield from ((bf16, 4, 8, 8, 1000, 64, True), (bf16, 16, 8, 8, 777, 64, False), (bf16, 8, 8, 4, 2047, 64, True))   # 128 and 256 rows, one-role dK/dV
+    yield from ((bf16, 1, 2, 1, 33, 128, False), (bf16, 8, 8, 8, 1100, 128, False), (bf16, 4, 8, 2, 2100, 128, True))
+    yield from ((bf16, 2, 3, 3, 130, 32, False), (bf16, 1, 4, 4, 301, 96, False), (bf16, 1, 2, 2, 90, 96, True), (bf16, 1, 2, 2, 65, 40, False))
+    yield from ((fp32, 2, 4, 2, 77, 64, False), (fp32, 8, 4, 4, 256, 64, True), (fp32, 1, 2, 2, 100, 32, False), (fp32, 1, 2, 1, 50, 96, True),
+                (fp32, 1, 2, 2, 130, 128, False), (fp32, 1, 2, 2, 33, 20, False))
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,S,D,documents", list(_rotation_cases()))
+def test_gradients_rotated_on_their_way_out_equal_a_rotation_after_them(dev, dtype, B, Hq, Hkv, S, D, documents):
+    from maltos_amd import ops
+    from maltos_amd._native import native
+
+    gen = torch.Generator().manual_seed(S + D)
+    rows = lambda heads: torch.randn(B, S, heads, D, generator=gen).to(dtype).to(dev).transpose(1, 2)
+    q, k, v, dout = rows(Hq), rows(Hkv), rows(Hkv), rows(Hq)
+    ang = torch.arange(S + 9).float()[:, None] * (1.0 / (10000.0 ** (torch.arange(0, D, 2).float() / D)))[None]
+    cos, sin = ang.cos().to(dtype).to(dev), ang.sin().to(dtype).to(dev)
+    ids = [None, None]
+    if documents:
+        doc = (torch.arange(S) * 3 // S).int().expand(B, S).contiguous()
+        first = torch.stack([torch.nonzero(doc[0] == d)[0, 0] for d in doc[0]])
+        ids = [(torch.arange(S) - first).int().expand(B, S).contiguous().to(dev), doc.to(dev)]
+    rope_ids, offset = (torch.randint(0, S + 9, (B, S), generator=gen).int().to(dev), 0) if documents else (None, 7)
+    leaves = [t.clone().transpose(1, 2).contiguous().transpose(1, 2).requires_grad_(True) for t in (q, k, v)]
+    got = torch.autograd.grad(native().rope_attention(*leaves, cos, sin, rope_ids, offset, *ids), leaves, dout)
+    qr, kr = torch.ops.maltos.rope_pair(q, k, cos, sin, rope_ids, offset, False)
+    turned = [t.detach().requires_grad_(True) for t in (qr, kr, v)]
+    out = ops.attention(*turned, mask_mode=ops.MASK_DOC if documents else ops.MASK_CAUSAL, q_pos=ids[0], k_pos=ids[0], q_seq=ids[1], k_seq=ids[1])
+    dq, dk, dv = torch.autograd.grad(out, turned, dout)
+    want = (*torch.ops.maltos.rope_pair(dq, dk, cos, sin, rope_ids, offset, True), dv)
+    for name, a, b in zip(("dQ", "dK", "dV"), got, want):
+        if dtype == torch.bfloat16:
+            assert torch.equal(a, b), name
+        else:   # two products and a sum, whether or not one product is fused into the sum: each rounded to 2^-24 of the largest at most
+            assert (a - b).abs().max() <= 3 * 2.0 ** -24 * 1.5 * b.abs().max(), name
