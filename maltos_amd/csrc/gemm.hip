@@ -154,6 +154,109 @@ struct Slab {
   }
 };
 
+// The slabs of a 256 x 256 tile of bf16 in the TN form, eight wavefronts of 128 x 64: 32 contraction elements a stage, five stages, straight from memory to LDS: no
+// registers hold them, so that three to four stages are on their way at any time (a slab of 64 in registers beside eight accumulator blocks: one), and there are no LDS
+// writes through registers.  One barrier a stage.  Bound by the matrix pipes' clock under load (0.54 PFLOP in 448 us, where the largest products reach 1.21 PFLOP/s).
+// us, slabs through registers / here: dW of 32000 x 512, 16384 rows 502 / 475, in a training step 502 (the library) / 448; 2752 x 512, 16384 rows 70 / 65; 2752 x 3072, 8192 rows 174 / 154; 70
+// products 0.95 on the mean, 0.88 to 1.02.  Operands with the contraction contiguous have 64 bytes a line and stage, half a cache line: of 40 NT products half are slower, by up to
+// 13 % (16384 x 1536 x 872 55.6 / 63.1), NN ones of long contractions by 3 to 5 % (12000 x 512 x 8192 112 / 116).
+struct Ring {
+  static constexpr int BK = 32, STAGES = 5, THREADS = 512, LINE = 256 * 2, OPERAND = BK * LINE, STAGE = 2 * OPERAND, BYTES = STAGES * STAGE, LOADS = 4;  // LOADS: of a lane a stage
+  struct Operand {
+    u32x4 rsrc;
+    uint32_t offset[2], advance;
+    int k[2];  // a chunk's contraction element in the stage
+    // Chunks of 16 bytes lie in LDS in the order of the lanes that fetch them.  Which chunk of its line that is depends on the line, so that the four lines a fragment is read from
+    // together lie in different banks.
+    __device__ __forceinline__ void init(const bf16_t* base, int64_t ld, int64_t lines, int64_t line_elems, int64_t k_begin) {
+      const uint64_t address = reinterpret_cast<uint64_t>(base);
+      const int64_t bytes = lines > 0 ? ((lines - 1) * ld + line_elems) * 2 : 0;
+      rsrc = u32x4{static_cast<uint32_t>(address), static_cast<uint32_t>(address >> 32) & 0xffff, static_cast<uint32_t>(bytes), 0x00020000};  // (as Slab's)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rsrc[e] = __builtin_amdgcn_readfirstlane(rsrc[e]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int slot = i * THREADS + static_cast<int>(threadIdx.x), line = slot >> 5, chunk = (slot & 31) ^ ((line & 3) << 2);
+        offset[i] = static_cast<uint32_t>((line + k_begin) * ld * 2 + chunk * 16);
+        k[i] = line;
+      }
+      advance = static_cast<uint32_t>(BK * ld * 2);
+    }
+    // the next stage, to LDS address `to` (of the wavefront's first chunk); k_left: contraction elements from there to the end
+    __device__ __forceinline__ void fetch(uint32_t to, int k_left) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t from = k[i] < k_left ? offset[i] : kOutside;
+        // (through the builtin the compiler would wait for all loads before any read of LDS)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(to + i * THREADS * 16), "v"(from), "s"(rsrc) : "memory", "m0");
+#pragma clang diagnostic pop
+        offset[i] += advance;
+      }
+    }
+  };
+  // as Slab::fragment
+  static __device__ __forceinline__ bf16x8 fragment(const unsigned char* lds, int row0, int ks, int lane) {
+    const int l32 = lane & 31, hh = lane >> 5, l16 = lane & 15;
+    const unsigned char* src = lds + (16 * ks + 8 * hh + (l16 >> 2)) * LINE + ((row0 + (l32 >> 4) * 16 + (l16 & 3) * 4) * 2 ^ (l16 >> 2) << 6);
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(MLTS_LDS_PTR(i16x4, src + 4 * LINE));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+  // Of this wavefront all but the last N loads to LDS are there and nothing that it reads there is outstanding; then likewise of all wavefronts of the workgroup.  (Reads carried over
+  // the barrier, which their slot allows: 475 -> 498 us; matrix instructions at a higher priority: no change.)
+  template <int N>
+  static __device__ __forceinline__ void wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+  // acc += the tile's product over k_left contraction elements
+  static __device__ __forceinline__ void multiply(Operand a, Operand b, int k_left, unsigned char* lds, int wm, int wn, f32x16 (&acc)[4][2]) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const uint32_t own = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(MLTS_LDS_PTR(unsigned char, lds))) + wave * 1024);
+    const int stages = (k_left + BK - 1) / BK;
+    uint32_t to = 0;  // the stage that is written next
+    auto fetch = [&] {  // (past the end: zeros)
+      a.fetch(own + to, k_left), b.fetch(own + to + OPERAND, k_left);
+      k_left -= BK;
+      to = to + STAGE == BYTES ? 0 : to + STAGE;
+    };
+    bf16x8 fa[2][4], fb[2][2];
+    auto read = [&](uint32_t stage, int ks) {
+      const unsigned char* from = lds + stage;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) fb[ks][j] = fragment(from + OPERAND, wn + 32 * j, ks, lane);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fa[ks][i] = fragment(from, wm + 32 * i, ks, lane);
+    };
+    auto products = [&](int ks) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = Multiply<BF16>::mma(fb[ks][j], fa[ks][i], acc[i][j]);
+    };
+#pragma unroll
+    for (int f = 0; f < STAGES - 1; ++f) fetch();
+    wait<2 * LOADS>();
+    uint32_t from = 0;
+    read(from, 0);
+    for (int s = 0; s < stages; ++s) {
+      // here stages s and s + 1 are in LDS, s + 2 and s + 3 on their way, and s - 1 is read by nobody any more: s + 4 takes its place
+      fetch();
+      const uint32_t next = from + STAGE == BYTES ? 0 : from + STAGE;
+      read(from, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      products(0);
+      __builtin_amdgcn_sched_barrier(0);
+      read(next, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      products(1);
+      from = next;
+      wait<2 * LOADS>();
+    }
+    wait<0>();  // (the zeros past the end)
+  }
+};
+
 // One product of a launch, as small as can be: kernel arguments are read from host memory.  (Operands are smaller than 2 GiB, so
 // their strides and lengths fit 32 bits.)
 struct Product {
@@ -304,6 +407,7 @@ struct TileShape {
   static constexpr int MB = WM / 32, NB = WN / 32;
   static constexpr bool SHARED = KG > 1 && WAVES == KG, GROUPS = KG > 1 && WAVES > KG;  // one wavefront to a group; several
   static constexpr int KIND = sizeof(T) == 2 ? BF16 : SHARED ? F32_WHOLE : F32_PARTS;  // (in a tile of 32 x 32 the parts are more work than they save)
+  static constexpr bool RING = KIND == BF16 && BM == 256 && BN == 256 && FORM == FORM_TN;  // (Ring)
   static constexpr int SETS = MB * NB >= 8 ? 1 : 2;  // (eight accumulator blocks leave no registers for a second set)
   typedef Slab<T, KIND, BM, FORM != FORM_TN, THREADS, SETS> SA;
   typedef Slab<T, KIND, BN, FORM == FORM_NT, THREADS, SETS, PAIR> SB;
@@ -311,7 +415,8 @@ struct TileShape {
   static constexpr int OUT = WAVES / (GROUPS ? KG : 1) * 32 * (WN + 4) * 4;
   static_assert(!GROUPS || (KG - 1) * BM * BN * 4 <= 2 * STAGE, "the groups' sums meet where the slabs were");
   static_assert(!PAIR || (FORM == FORM_NT && !SHARED && WAVES_N % 2 == 0), "the products of a pair side by side in a tile, half of the wavefronts each");
-  static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
+  static constexpr int SLABS = RING ? Ring::BYTES : 2 * STAGE;
+  static constexpr int LDS = SLABS > OUT ? SLABS : OUT;
 };
 
 // One tile of one product.  KG > 1, SHARED: the wavefronts share the tile and each multiply their part of every slab; their sums meet in
@@ -397,7 +502,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
     else sb.fetch(set, c - SA::PER, k_left);
   };
 #pragma unroll
-  for (int f = 0; f < SETS; ++f) {
+  for (int f = 0; f < (S::RING ? 0 : SETS); ++f) {
     next_slab();
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) fetch(f, c);
@@ -459,11 +564,13 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
     if (!rot->positions) in_seq = static_cast<int>(static_cast<uint32_t>(out_row) % static_cast<uint32_t>(rot->seq));
     if (EARLY_ANGLES) fetch_angles(0);
   }
+  if constexpr (!S::RING) {
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) store(0, c, lds);
-  next_slab();
+    for (int c = 0; c < CHUNKS; ++c) store(0, c, lds);
+    next_slab();
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) fetch(0, c);
+    for (int c = 0; c < CHUNKS; ++c) fetch(0, c);
+  }
   constexpr bool FOLD = SEGMENTS && sizeof(T) == 2;
   f32x16 parts[FOLD ? MB : 1][FOLD ? NB : 1];  // sum of the parts before
   int part = 0, part_end = FOLD ? (g.K + BK - 1) / BK : 0;
@@ -530,7 +637,12 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
       }
   };
   if constexpr (FOLD) after(-1);
-  if constexpr (SETS == 1) {
+  if constexpr (S::RING) {
+    Ring::Operand a, b;
+    a.init(static_cast<const bf16_t*>(g.a) + m0, g.lda, g.K, g.M - m0, k_begin);
+    b.init(static_cast<const bf16_t*>(g.b) + n0, g.ldb, g.K, g.N - n0, k_begin);
+    Ring::multiply(a, b, k_left, lds, wm, wn, acc);
+  } else if constexpr (SETS == 1) {
     for (int s = 0; s < slabs; ++s) slab(s, 0);
   } else {
     // (Whole rounds of the sets with nothing to jump over: a way round one slab of a round leaves fewer loads behind, and the waits

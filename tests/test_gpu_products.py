@@ -67,6 +67,8 @@ def test_products_left_to_the_library(dev):
     (NT, 16384, 2304, 768, True), (NT, 17000, 2304, 768, False), (NN, 16384, 512, 1536, True), (NT, 17000, 512, 1536, False), (NT, 8000, 512, 2048, True), (NT, 8192, 512, 2048, False),
     (TN, 1024, 1024, 12000, True), (TN, 1024, 1024, 16384, False), (TN, 1024, 1024, 20001, True), (TN, 512, 1376, 16384, False), (TN, 256, 680, 32768, True), (TN, 2752, 512, 12000, True),
     (TN, 5456, 1024, 4096, False), (TN, 1024, 2728, 10000, True), (TN, 6912, 1280, 3000, False),
+    (TN, 8192, 768, 12000, True), (TN, 8192, 776, 12000, False), (TN, 8192, 1024, 10000, True), (TN, 8192, 1024, 9992, False), (TN, 12000, 1024, 12000, False), (TN, 32000, 128, 4096, True),
+    (TN, 32000, 136, 4096, False), (TN, 32000, 512, 10000, True), (TN, 32000, 512, 9992, False),
     (NN, 2048, 2048, 2816, True), (NN, 2048, 2176, 2816, False), (NN, 4096, 1024, 2808, False), (NN, 1000, 4096, 8192, True), (NN, 4096, 2048, 8192, True), (NN, 4352, 2048, 8192, False),
     (NN, 4096, 2048, 8184, False)])
 def test_which_large_products_the_own_kernels_take(dev, form, M, N, K, own):
@@ -339,7 +341,7 @@ def test_tiles_in_runs_of_equal_length(dev, dtype, items):
 TILE_CASES = [
     ((NN, 521, 2056, 8200), 0, (256, 128, 4)), ((NN, 1033, 5464, 520), 0, (256, 128, 1)), ((TN, 12008, 72, 8201), 0, (256, 128, 4)), ((TN, 136, 5464, 12001), 0, (256, 256, 8)),
     ((TN, 4088, 2040, 3001), 48, (256, 128, 1)), ((NT, 12001, 76, 8200), 0, (256, 128, 4)), ((NT, 4547, 7657, 680), 0, (256, 256, 1)), ((NN, 4547, 7656, 680), 8, (256, 256, 1)),
-    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((NN, 2336, 1032, 8200), 0, (256, 256, 4)), ((NT, 4033, 516, 8200), 0, (256, 256, 4)), ((NT, 1033, 1029, 1032), 3, (128, 64, 1)),
+    ((TN, 4552, 7656, 681), 0, (256, 256, 1)), ((TN, 8200, 8200, 65), 0, (256, 256, 1)), ((TN, 8200, 8200, 97), 8, (256, 256, 1)), ((TN, 8200, 8200, 161), 0, (256, 256, 1)), ((NN, 2336, 1032, 8200), 0, (256, 256, 4)), ((NT, 4033, 516, 8200), 0, (256, 256, 4)), ((NT, 1033, 1029, 1032), 3, (128, 64, 1)),
     ((NT, 3001, 260, 8200), 0, (128, 64, 2)), ((NN, 521, 520, 4104), 0, (128, 64, 4)), ((TN, 2336, 136, 8201), 0, (128, 64, 4)), ((TN, 1032, 136, 8201), 0, (128, 64, 8)),
     ((NT, 2331, 1542, 512), 0, (128, 128, 1)), ((NN, 3001, 72, 6008), 0, (128, 128, 8)), ((TN, 520, 1384, 6008), 0, (128, 128, 4))]
 # (batch rows, tokens, heads, KV heads, head_dim, K, positions given) of q, k, v as one rotated product
