@@ -48,7 +48,10 @@ struct Multiply<F32_WHOLE> {
     return c;
   }
 };
-// v as its parts: their sum is v, unless v is infinite, NaN or rounded to infinity in bf16
+// Sums below 2^-70 are computed whole.  The parts of an element miss it by 2^-134 at most, half of bf16's smallest number (the matrix instructions keep denormal ones): 2^-64 of such a
+// sum times the other operand's elements, less than fp32's rounding where those are below 2^40.  (Without this, relative errors at elements of 1e-35 2.6e-6, at 1e-37 2.7e-4, as at any size 4e-7 now.)
+constexpr uint32_t kPartsFloor = (127u - 70u) << 24;  // (a float's bits shifted by one)
+// v as its parts: their sum is v, unless v is infinite, NaN, rounded to infinity in bf16 or below 2^-110
 __device__ __forceinline__ void split(f32x4 v, u32x2 (&parts)[3]) {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -674,18 +677,22 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
   }
 
   if constexpr (PARTS > 1) {
-    float finite = 0.f;  // NaN if a sum is not
+    float finite = 0.f;       // NaN if a sum is not
+    uint32_t smallest = ~0u;  // twice the bits of the smallest magnitude but zero, less one
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         acc[i][j] += low[i][j];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
+        for (int e = 0; e < 16; ++e) {
+          finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
+          smallest = min(smallest, (__builtin_bit_cast(uint32_t, acc[i][j][e]) << 1) - 1u);
+        }
       }
-    if (__builtin_amdgcn_ballot_w64(finite != 0.f)) {
-      // Infinities, NaN, and numbers that bf16 rounds to infinity have no parts: this wavefront's blocks once more, by fp32 matrix instructions straight from memory
-      // (a tenth of the speed or less).
+    if (__builtin_amdgcn_ballot_w64(finite != 0.f || smallest < kPartsFloor)) {
+      // Infinities, NaN, and numbers that bf16 rounds to infinity have no parts, and numbers below 2^-110 lose bits of their third one, which is below bf16's range: this
+      // wavefront's blocks once more, by fp32 matrix instructions straight from memory (a tenth of the speed or less).
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll

@@ -407,6 +407,22 @@ def test_fp32_in_three_parts(dev, product, tile):
     assert abs(out[70, 7].double() / want[70, 7] - 1) <= 1e-6
 
 
+@pytest.mark.parametrize("product,tile", PARTS_CASES, ids=lambda v: "-".join(map(str, v)))
+@pytest.mark.parametrize("size,other", [(1e-28, 1.0), (1e-31, 1.0), (1e-33, 1.0), (1e-35, 1.0), (1e-36, 1e10), (1e-20, 1e-12)])
+def test_fp32_of_small_elements(dev, product, tile, size, other):
+    """Elements whose third part is below bf16's range: as exact as fp32 instructions (a rounding a term), also where only some rows are that small."""
+    form, M, N, K = product
+    a, b = operands(form, M, N, K, torch.float32, dev, M + K)
+    rows = a.t() if form == TN else a
+    rows[::2] *= size
+    b *= other
+    out = torch.empty(M, N, device=dev)
+    run_products([(form, [(a, b)], out, 0)], torch.float32)
+    want = expected(form, a, b)
+    for part in (slice(0, M, 2), slice(1, M, 2)):
+        assert (out.double() - want)[part].norm() <= 2.0**-24 * (3 + K**0.5) * want[part].norm()
+
+
 def test_fp32_sum_over_segments_in_slices(dev):
     """A sum over segments whose slabs are split over workgroups, alone and beside a weight gradient: slices that begin and end within segments."""
     gen = torch.Generator().manual_seed(8)
