@@ -147,10 +147,14 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
     row[r] = there && qrow < p.Sq ? dQ + static_cast<int64_t>(qrow) * bp.dqs[2] : nullptr;
     scale[r] = p.scale;
   }
+  if (!bp.rot.cos) {  // (known from the start, unlike what rotation_of_kernel fetches: forward and backward of 2 x 8 (4) x 777 of 64, us: 93.4 / 92.3)
+    join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1, AsIs{});
+    return;
+  }
   const RotateBack rot = rotation_of_kernel();
   Back<R> back{rot, {}};
 #pragma unroll
-  for (int r = 0; r < R; ++r) back.table[r] = rot.cos ? rot.row(b, q0 + 16 * r + l16) : -1;
+  for (int r = 0; r < R; ++r) back.table[r] = rot.row(b, q0 + 16 * r + l16);
   join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1, back);
 }
 
@@ -316,10 +320,14 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     row[R + r] = mine ? static_cast<float*>(bp.dv) + b * bp.dvs[0] + hkv * bp.dvs[1] + krow * bp.dvs[2] : nullptr;
     scale[r] = p.scale, scale[R + r] = 1.f;
   }
+  if (!bp.rot.cos) {
+    join_and_store(dkv, lds + slot * splits * 2 * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0, AsIs{});
+    return;
+  }
   const RotateBack rot = rotation_of_kernel();
   Back<2 * R> back{rot, {}};
 #pragma unroll
-  for (int r = 0; r < R; ++r) back.table[r] = rot.cos ? rot.row(b, kb0 + 16 * r + l16) : -1, back.table[R + r] = -1;
+  for (int r = 0; r < R; ++r) back.table[r] = rot.row(b, kb0 + 16 * r + l16), back.table[R + r] = -1;
   join_and_store(dkv, lds + slot * splits * 2 * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0, back);
 }
 
