@@ -48,20 +48,24 @@ struct Multiply<F32_WHOLE> {
     return c;
   }
 };
-// Sums below 2^-70 are computed whole.  The parts of an element miss it by 2^-134 at most, half of bf16's smallest number (the matrix instructions keep denormal ones): 2^-64 of such a
-// sum times the other operand's elements, less than fp32's rounding where those are below 2^40.  (Without this, relative errors at elements of 1e-35 2.6e-6, at 1e-37 2.7e-4, as at any size 4e-7 now.)
-constexpr uint32_t kPartsFloor = (127u - 70u) << 24;  // (a float's bits shifted by one)
-// v as its parts: their sum is v, unless v is infinite, NaN, rounded to infinity in bf16 or below 2^-110
+// Elements are split times 2^24 and the sums taken back by 2^-48: every fp32 number but zero is then a multiple of 2^-125, and so is each of its parts, which bf16 holds without denormal numbers.
+// (Without it an element below 2^-110 loses bits of its third part and one below 2^-134 all of them, which a large enough other operand lifts into the result: 2.7e-4 relative
+// at 1e-37 times 1e25, zero for 3e-41 times 1e20.)  Elements from 2^104 and sums from 2^80 on leave the range instead, and are computed whole (gemm_tile).  us, without the scale / with it: NT 2048 x
+// 256 x 256 5.93 / 5.92, 2048 x 768 x 256 11.0 / 11.7, 4096 x 2048 x 2048 178.5 / 180.8, TN 688 x 256 x 2048 13.9 / 14.5.
+constexpr float kPartsScale = 0x1p24f, kPartsUnscale = 0x1p-48f;
+// v times kPartsScale as its parts: their sum is that, unless it is infinite, NaN or rounded to infinity in bf16
 __device__ __forceinline__ void split(f32x4 v, u32x2 (&parts)[3]) {
 #pragma clang fp contract(off)
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    f32x2 rest = {v[2 * i], v[2 * i + 1]};
+    f32x2 rest = {v[2 * i] * kPartsScale, v[2 * i + 1] * kPartsScale};
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2));
-      parts[p][i] = pair;
-      if (p < 2) rest[0] -= __builtin_bit_cast(float, pair << 16), rest[1] -= __builtin_bit_cast(float, pair & 0xffff0000u);
+      const uint32_t pair = parts[p][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2));
+      const float lo = __builtin_bit_cast(float, pair << 16), hi = __builtin_bit_cast(float, pair & 0xffff0000u);
+      // (from v again: 180.8 us for 184.9 of the third product above, with the scaled elements kept)
+      if (p == 0) rest[0] = __builtin_fmaf(v[2 * i], kPartsScale, -lo), rest[1] = __builtin_fmaf(v[2 * i + 1], kPartsScale, -hi);
+      if (p == 1) rest[0] -= lo, rest[1] -= hi;
     }
   }
 }
@@ -677,21 +681,17 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
   }
 
   if constexpr (PARTS > 1) {
-    float finite = 0.f;       // NaN if a sum is not
-    uint32_t smallest = ~0u;  // twice the bits of the smallest magnitude but zero, less one
+    float finite = 0.f;  // NaN if a sum is not
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
-        acc[i][j] += low[i][j];
+        acc[i][j] = (acc[i][j] + low[i][j]) * kPartsUnscale;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
-          smallest = min(smallest, (__builtin_bit_cast(uint32_t, acc[i][j][e]) << 1) - 1u);
-        }
+        for (int e = 0; e < 16; ++e) finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
       }
-    if (__builtin_amdgcn_ballot_w64(finite != 0.f || smallest < kPartsFloor)) {
-      // Infinities, NaN, and numbers that bf16 rounds to infinity have no parts, and numbers below 2^-110 lose bits of their third one, which is below bf16's range: this
+    if (__builtin_amdgcn_ballot_w64(finite != 0.f)) {
+      // Infinities, NaN, and numbers that leave the range of the scaled parts or of their sums: this
       // wavefront's blocks once more, by fp32 matrix instructions straight from memory (a tenth of the speed or less).
 #pragma unroll
       for (int i = 0; i < MB; ++i)

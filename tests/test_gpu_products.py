@@ -423,6 +423,27 @@ def test_fp32_of_small_elements(dev, product, tile, size, other):
         assert (out.double() - want)[part].norm() <= 2.0**-24 * (3 + K**0.5) * want[part].norm()
 
 
+@pytest.mark.parametrize("product,tile", PARTS_CASES, ids=lambda v: "-".join(map(str, v)))
+@pytest.mark.parametrize("size,other", [(1e-36, 1e20), (1e-37, 1e25), (1e-38, 1e20), (1e-38, 1e30), (3e-41, 1e10), (3e-41, 1e20), (1e-44, 1e30), (1e-12, 1e33), (1e13, 1e13), (1e-30, 1e37)])
+def test_fp32_of_elements_far_apart(dev, product, tile, size, other):
+    """Small elements, also below the normal numbers, against large ones, either operand's, all rows or some: as exact as fp32 instructions (a rounding a term).  And what leaves the range of the
+    parts or of their sums at the other end."""
+    form, M, N, K = product
+    x, y = operands(form, M, N, K, torch.float32, dev, M + K)
+    for swapped in (False, True):
+        for some in (False, True):
+            a, b = (x * other, y * size) if swapped else (x * size, y * other)
+            if some:   # of the small ones every other row or column such that its sums are about 1
+                rows = (b if form == NT else b.t()) if swapped else (a.t() if form == TN else a)
+                rows[1::2] = ((y if form == NT else y.t()) if swapped else (x.t() if form == TN else x))[1::2] * (1 / other)
+            out = torch.empty(M, N, device=dev)
+            run_products([(form, [(a, b)], out, 0)], torch.float32)
+            got, want = out.double(), expected(form, a, b)
+            got, want = (got.t(), want.t()) if swapped else (got, want)
+            for part in (slice(0, None, 2), slice(1, None, 2)):
+                assert (got - want)[part].norm() <= 2.0**-24 * (3 + K**0.5) * want[part].norm(), (swapped, some)
+
+
 def test_fp32_sum_over_segments_in_slices(dev):
     """A sum over segments whose slabs are split over workgroups, alone and beside a weight gradient: slices that begin and end within segments."""
     gen = torch.Generator().manual_seed(8)
