@@ -50,7 +50,7 @@ struct Multiply<F32_WHOLE> {
 };
 // Elements are split times 2^24 and the sums taken back by 2^-48: every fp32 number but zero is then a multiple of 2^-125, and so is each of its parts, which bf16 holds without denormal numbers.
 // (Without it an element below 2^-110 loses bits of its third part and one below 2^-134 all of them, which a large enough other operand lifts into the result: 2.7e-4 relative
-// at 1e-37 times 1e25, zero for 3e-41 times 1e20.)  Elements from 2^104 and sums from 2^80 on leave the range instead, and are computed whole (gemm_tile).  us, without the scale / with it: NT 2048 x
+// at 1e-37 times 1e25, zero for 3e-41 times 1e20.)  Elements from 2^104 and sums from 2^80 on leave the range instead, and are computed whole one by one (gemm_tile).  us, without the scale / with it: NT 2048 x
 // 256 x 256 5.93 / 5.92, 2048 x 768 x 256 11.0 / 11.7, 4096 x 2048 x 2048 178.5 / 180.8, TN 688 x 256 x 2048 13.9 / 14.5.
 constexpr float kPartsScale = 0x1p24f, kPartsUnscale = 0x1p-48f;
 // v times kPartsScale as its parts: their sum is that, unless it is infinite, NaN or rounded to infinity in bf16
@@ -691,8 +691,9 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
         for (int e = 0; e < 16; ++e) finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
       }
     if (__builtin_amdgcn_ballot_w64(finite != 0.f)) {
-      // Infinities, NaN, and numbers that leave the range of the scaled parts or of their sums: this
-      // wavefront's blocks once more, by fp32 matrix instructions straight from memory (a tenth of the speed or less).
+      // Infinities, NaN, and numbers that leave the range of the scaled parts or of their sums: blocks of this wavefront that have such elements once more, by fp32 matrix instructions straight
+      // from memory (a tenth of the speed or less).  The others of a block stay as they are, so that an element's bits depend on its own row and column alone; and what lies beside the operands in
+      // memory, which lanes past the last row or column may hold, is no reason.
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -700,6 +701,11 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
           const int row = m0 + wm + 32 * i + l32, block = wn + 32 * j, in_pair = block % (BN / 2);
           const bool second = PAIR && block >= BN / 2;
           const int column = n0 + (PAIR ? in_pair : block) + l32;
+          const auto in_range = [&](int e) { return __builtin_fabsf(acc[i][j][e]) < INFINITY; };
+          bool all = true;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) all = all && (in_range(e) || row >= g.M || column - l32 + 8 * (e / 4) + 4 * hh + e % 4 >= g.N);
+          if (!__builtin_amdgcn_ballot_w64(!all)) continue;
           f32x16 sum;
 #pragma unroll
           for (int e = 0; e < 16; ++e) sum[e] = 0.f;
@@ -720,7 +726,8 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
               }
             }
           }
-          acc[i][j] = sum;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = in_range(e) ? acc[i][j][e] : sum[e];
         }
     }
   }

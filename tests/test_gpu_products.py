@@ -444,6 +444,31 @@ def test_fp32_of_elements_far_apart(dev, product, tile, size, other):
                 assert (got - want)[part].norm() <= 2.0**-24 * (3 + K**0.5) * want[part].norm(), (swapped, some)
 
 
+@pytest.mark.parametrize("product,tile", PARTS_CASES, ids=lambda v: "-".join(map(str, v)))
+def test_fp32_bits_of_an_element_are_those_of_its_row_and_column(dev, product, tile):
+    """Whatever other rows and columns of the operands hold, and what lies beside them in memory."""
+    form, M, N, K = product
+    a, b = operands(form, M, N, K, torch.float32, dev, M + N)
+    out, other = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    run_products([(form, [(a, b)], out, 0)], torch.float32)
+    x, y = a.clone(), b.clone()
+    rows, columns = x.t() if form == TN else x, y if form != NT else y.t()
+    rows[3, 5], rows[M - 1, K - 1], rows[70, 0], rows[37] = float("inf"), float("nan"), 3.4e38, 1e-38
+    columns[2, N - 1], columns[0, 65], columns[1, 6] = float("-inf"), float("nan"), 2e32
+    run_products([(form, [(x, y)], other, 0)], torch.float32)
+    row, column = torch.ones(M, dtype=torch.bool, device=dev), torch.ones(N, dtype=torch.bool, device=dev)
+    row[[3, M - 1, 70, 37]], column[[N - 1, 65, 6]] = False, False
+    assert torch.equal(other[row][:, column], out[row][:, column])
+    # as ranges of wider buffers, of dW's rows and dx's columns an odd number
+    M, N, results = M - (form == TN), N - (form == NN), []
+    for beside in (1.0, float("nan")):
+        x, y = (torch.full((t.size(0), t.size(1) + 72), beside, device=dev)[:, :t.size(1) - odd] for t, odd in ((a, form == TN), (b, form == NN)))
+        x.copy_(a[:, :x.size(1)]), y.copy_(b[:, :y.size(1)])
+        results.append(torch.empty(M, N, device=dev))
+        run_products([(form, [(x, y)], results[-1], 0)], torch.float32)
+    assert torch.equal(*results)
+
+
 def test_fp32_sum_over_segments_in_slices(dev):
     """A sum over segments whose slabs are split over workgroups, alone and beside a weight gradient: slices that begin and end within segments."""
     gen = torch.Generator().manual_seed(8)
