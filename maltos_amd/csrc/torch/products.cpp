@@ -38,9 +38,12 @@ constexpr double kOwnLimitBf16 = 4.0e9;
 //   dW, which the library forms as a batch of row slices (weight_grad_splits).  Slices too few for 64 of its tiles: 1024 x 1024 of 20001 rows, alone, 56 us against 162.  Slices of
 //     whole 1024 rows, from 16384 rows on: 512 to 768 wide 16384 rows -14 to +20, 24576 -32 to +32, but 20020 rows -2 to -57; below, up to 2e10: 5456 x 1024 x 4096 +13 to +15,
 //     3072 x 1024 x 8192 +4 to +21; 64 tiles without slices: 6912 x 1280 x 3000 +21, 5456 x 1024 x 3000 -4 to -9; others up to 3e10: 1024 x 2728 x 10000 -55, 1280 x 1792 x 12000 -27.
-//   dW of 8192 rows and more (of a vocabulary), own over library's time, in terms (alone, added onto a gradient, 1023 to 16384): up to 128 wide 0.43 to 0.88; up to 96 tiles of 256 x 256 0.46 to 0.97
-//     from 4092 terms on; whole tiles and 10000 terms on 32000 x 256 0.90, x 512 0.95, 16000 x 512 0.89, 50264 x 256 0.86, 32000 x 768 0.75, up to 16384 wide 8192 x 1024 0.92, but 12000 x 1024 1.04
-//     (a quarter of the CUs idle in the last round); 32000 x 512 0.93 to 1.06 below, x 384 1.09 to 1.26.
+//   dW of 8192 rows and more (of a vocabulary), own over library's time, alone, added onto a gradient, 640 to 20001 terms, by tiles of 256 x 256
+//     up to 64                       0.45 to 1.07, 8192 x 512 0.64 to 0.94, 16384 x 256 0.59 to 0.99
+//     65 to 95 (20000 x 256)         from 2048 terms on 0.40 to 1.08; 1536 terms 0.87 to 1.20; 96, whole ones (8192 x 768, 24576 x 256) 0.84 to 1.31
+//     up to 128 wide                 up to 128 tiles 0.40 to 1.14; 157 and 197 tiles (40000 x 128, 50264 x 64 and x 128) 0.79 to 1.40
+//     whole ones, 10000 terms on     up to 128 tiles 0.65 to 1.07; 129 to 192 (16384 x 768, 40000 x 256: part of the CUs idle in the last round) 0.73 to 1.11; more 0.73 to 0.98
+//     others                         16384 x 384 and x 512 below 10000 terms 0.91 to 1.22; 20000 x 512, 24576 x 384, 40000 x 256, 50264 x 256 0.82 to 1.57; 32000 x 512 0.93 to 1.06
 //     In one launch with dh = dy W and the activation -2 to -107 at all row counts up to 32768; that dh without its dW up to +74.
 // These were measured on tiles of 128 x 128 where 256 x 128 is taken since (y of 512 x 1376, 16384 rows, 39 us, now 34).
 // (With the shipped per-shape selection, 16384 rows, alone: y 512 x 512 17 us against 16, 1536 x 512 42 / 32, in a step rotated on its way out 48 / 32 + 15,
@@ -51,7 +54,8 @@ bool larger_own_range_bf16(int form, int64_t M, int64_t N, int64_t K, Use use) {
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
   if (N >= 16384 || N % 8) return false;
   if (form == MLTS_GEMM_TN) {
-    if (M >= 8192 && (N <= 128 || tiles <= 96 || (N % 256 == 0 && K >= 10000 && (M >= 16384 || tiles <= 128)))) return true;
+    if (M >= 8192 && (tiles <= 64 || (tiles < 96 && K >= 2048) || (N <= 128 && tiles <= 128))) return true;
+    if (M >= 8192 && N % 256 == 0 && K >= 10000 && (tiles <= 128 || (M >= 16384 && tiles > 192))) return true;
     if (M >= 16384) return false;
     if (use == Use::ACTIVATION) return true;
     const bool few = tiles * weight_grad_splits(K, M, N) < 64, whole = !few && K % 1024 == 0;

@@ -69,6 +69,8 @@ def test_products_left_to_the_library(dev):
     (TN, 5456, 1024, 4096, False), (TN, 1024, 2728, 10000, True), (TN, 6912, 1280, 3000, False),
     (TN, 8192, 768, 12000, True), (TN, 8192, 776, 12000, False), (TN, 8192, 1024, 10000, True), (TN, 8192, 1024, 9992, False), (TN, 12000, 1024, 12000, False), (TN, 32000, 128, 4096, True),
     (TN, 32000, 136, 4096, False), (TN, 32000, 512, 10000, True), (TN, 32000, 512, 9992, False),
+    (TN, 16384, 256, 1023, True), (TN, 20480, 256, 2048, True), (TN, 20480, 256, 2040, False), (TN, 24576, 256, 2048, False), (TN, 32768, 128, 1023, True), (TN, 32776, 128, 1023, False),
+    (TN, 33024, 256, 12000, False), (TN, 32768, 256, 12000, True), (TN, 49152, 256, 12000, False), (TN, 49160, 256, 12000, True),
     (NN, 2048, 2048, 2816, True), (NN, 2048, 2176, 2816, False), (NN, 4096, 1024, 2808, False), (NN, 1000, 4096, 8192, True), (NN, 4096, 2048, 8192, True), (NN, 4352, 2048, 8192, False),
     (NN, 4096, 2048, 8184, False)])
 def test_which_large_products_the_own_kernels_take(dev, form, M, N, K, own):
