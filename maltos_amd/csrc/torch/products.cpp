@@ -21,7 +21,8 @@ namespace {
 
 // Where the own kernels run, by M * N * K.  A product through torch costs 18 us of host time, a call here 5, and that is what
 // small steps wait for.  On the GPU alone (both sides timed with the weights out of HBM; rows from 100 to 16384; the library's choice
-// untuned) they are ahead of the library in fp32 at every size (0.6 to 0.9 of its time from 5e8 to 2.5e10, and its errors are larger), in bf16 up to 4e9 (0.4 to 0.95)
+// untuned) they are ahead of the library in bf16 up to 4e9 (0.4 to 0.95), and in fp32 without a limit: 0.6 to 1.09 of its time from 5e8 to 2.5e10, 0.75 on the mean, and 0.73 to 0.82 from there
+// to 3.2e11 (logits of 16384 x 32000 x 512 3165 us for 3843, their dx 2695 / 3493, dW 2842 / 3578), with smaller errors
 constexpr double kOwnLimitBf16 = 4.0e9;
 
 // Larger bf16 products, by what running one of them on the own kernels adds to a layer's training step in which the library has the others (us; 145
