@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv64_kernel(const AttnBwdPar
 
   const int64_t dk0 = b * bp.dks[0] + hkv * bp.dks[1] + 4 * g, dv0 = b * bp.dvs[0] + hkv * bp.dvs[1] + 4 * g;
   if constexpr (ROTATED) {  // (dk and dv in bf16, overwritten)
-    const RotateBack rot = rotation_of_kernel();
+    const RotateBack rot = rotation_of_kernel<decltype(attn_bwd_dkv64_kernel<MODE, ROTATED>)>();
     // A quarter of a table row each for the lanes of a gradient row, on its way while dV is written; transposed it is every lane's own pairs.  8 x 8 heads x
     // 2048 causal, us: not rotated 96.7, so 99.2, fetched as the pairs are used (sixteen loads of 4 bytes) 103.8; the pass over dQ and dK took 14.9, of which dQ here keeps 3.9.
     uint32_t quarter[R][2][NC];

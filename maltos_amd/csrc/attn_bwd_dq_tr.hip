@@ -529,7 +529,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_bwd_dq_tr_kernel(const Att
     // bf16 rows through LDS (each wavefront owns 32 rows x RB bytes, tile-row swizzle), so that global stores are
     // 16 bytes per lane and cover whole rows
     constexpr int CHUNKS = 32 * CPR / 64;
-    const RotateBack rot = rotation_of_kernel();
+    const RotateBack rot = rotation_of_kernel<decltype(attn_bwd_dq_tr_kernel<D, MODE, WAVES>)>();
     RotateBack::Angles<bf16_t, 4> angles[CHUNKS];  // fetched behind the last tile
     if (rot.cos) {
 #pragma unroll

@@ -726,7 +726,7 @@ __global__ __launch_bounds__(KB * 128, 2) void attn_bwd_dkdv_split_kernel(const 
       // chunk ^ (4 if row & 4) keeps the two half-wavefronts (rows 4 apart) on different banks
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       constexpr int CHUNKS = 32 * CPR / 64;
-      const RotateBack rot = rotation_of_kernel();
+      const RotateBack rot = rotation_of_kernel<decltype(attn_bwd_dkdv_split_kernel<D, MODE, KB>)>();
       const bool rotated = role == 1 && rot.cos;
       RotateBack::Angles<bf16_t, 4> angles[CHUNKS];
       if (rotated) {

@@ -131,8 +131,14 @@ struct AttnBwdParams {
 };
 
 // `rot` of a kernel whose first argument is an AttnBwdParams, fetched where this is called: as a member of the argument it is in scalar registers from the
-// kernel's start, which its loop then lacks (dK/dV at head_dim 64, 8 x 8 x 2048 causal, 103 us, 108 with twelve more).
+// kernel's start, which its loop then lacks (dK/dV at head_dim 64, 8 x 8 x 2048 causal, 103 us, 108 with twelve more).  Kernel: the type of the kernel that calls it.
+template <typename Kernel>
+constexpr bool kTakesBwdParams = false;
+template <typename... Rest>
+constexpr bool kTakesBwdParams<void(AttnBwdParams, Rest...)> = true;
+template <typename Kernel>
 __device__ __forceinline__ RotateBack rotation_of_kernel() {
+  static_assert(kTakesBwdParams<Kernel>, "the first argument, which is read here as bytes");
   RotateBack rot{};
 #ifdef __HIP_DEVICE_COMPILE__
   typedef const __attribute__((address_space(4))) uint64_t* words;

@@ -151,7 +151,7 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dq(c
     join_and_store(dq, lds + slot * splits * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.dq_f32 == 1, AsIs{});
     return;
   }
-  const RotateBack rot = rotation_of_kernel();
+  const RotateBack rot = rotation_of_kernel<decltype(attn_f32_bwd_dq<DP, R, DOC, LAYOUT>)>();
   Back<R> back{rot, {}};
 #pragma unroll
   for (int r = 0; r < R; ++r) back.table[r] = rot.row(b, q0 + 16 * r + l16);
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(max_splits(DP, LAYOUT) * 64) void attn_f32_bwd_dkv(
     join_and_store(dkv, lds + slot * splits * 2 * R * NC * 256, split, splits, row, scale, lane, a.D, a.vec_out, bp.accumulate_f32 != 0, AsIs{});
     return;
   }
-  const RotateBack rot = rotation_of_kernel();
+  const RotateBack rot = rotation_of_kernel<decltype(attn_f32_bwd_dkv<DP, R, DOC, LAYOUT>)>();
   Back<2 * R> back{rot, {}};
 #pragma unroll
   for (int r = 0; r < R; ++r) back.table[r] = rot.row(b, kb0 + 16 * r + l16), back.table[R + r] = -1;

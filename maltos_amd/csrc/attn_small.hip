@@ -490,7 +490,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dq(const AttnB
     k0 = kn, kn = kn2;
   }
   const int64_t row = b * bp.dqs[0] + hq * bp.dqs[1] + 4 * g;
-  const RotateBack rot = rotation_of_kernel();
+  const RotateBack rot = rotation_of_kernel<decltype(attn_small_bwd_dq<D, DOC, R>)>();
   int64_t table[R];
   if (rot.cos) {
 #pragma unroll
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(kMaxSplits * 64) void attn_small_bwd_dkv(const Attn
   for (int n = 0; n < 2 * R; ++n)
 #pragma unroll
     for (int db = 0; db < NC; ++db) dkv[n][db] = n < R ? dk[n < R ? n : 0][db] : dv[n < R ? 0 : n - R][db];
-  const RotateBack rot = rotation_of_kernel();
+  const RotateBack rot = rotation_of_kernel<decltype(attn_small_bwd_dkv<D, DOC, R>)>();
   int64_t table[R];
   if (rot.cos) {
 #pragma unroll
