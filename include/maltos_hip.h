@@ -308,7 +308,9 @@ int mlts_gemm(int32_t form, int32_t dtype, int64_t M, int64_t N, int64_t K, cons
 /* Up to four products in one call, small ones in one launch.  A product of the NN form may be the sum over up to three
  * segments a[i] b[i] (the input gradient of layers that share their input), in bf16 with the roundings of separate products.
  * A launch takes the segments of one product: a call with more of them takes more launches.  The outputs of a call must not
- * overlap (MLTS_ERR_INVALID). */
+ * overlap (MLTS_ERR_INVALID).  Bits: the same call gives the same every time.  An element's depend on its own row and column, the sizes of the product, and in MLTS_F32
+ * also on what shares the call, which the tile is chosen for: small tiles multiply fp32 numbers whole, larger ones in three bf16 parts (24 bits, exact for every fp32
+ * number), with a third of the error.  An MLTS_BF16 weight gradient keeps the split it has alone. */
 typedef struct {
   int32_t form, segments, accumulate;
   int64_t M, N;

@@ -53,8 +53,8 @@ struct AttnParams {
 };
 
 // dQ and dK of rotated queries and keys, rotated back on their way out (mlts_attn_bwd_rope): the roundings of mlts_rope with `inverse`, over the
-// gradients as they would be stored.  A pass of its own reads and writes both once more (us, the kernels and the pass / here: 8 x 8 heads x 2048 of 64 in bf16 165.7 + 14.9 / 172.1,
-// 8 heads x 1023 packed 21.7 + 4.0 / 22.0, fp32 8 x 4 x 256 26.5 + 4.3 / 28.2).
+// gradients as they would be stored.  A pass of its own reads and writes both once more (us of dQ and dK/dV and the pass / here: 8 x 8 heads x 2048 of 64 in bf16 162.1 + 14.1 / 166.7,
+// 4 x 16 x 4096 493.6 + 23.4 / 506.8, 8 x 1024 19.2 + 3.3 / 19.4, 3 x 8 x 777 31.0 + 4.5 / 31.8, fp32 8 x 8 x 1024 275.7 + 11.6 / 281.7, 2 x 8 (4) x 777 75.7 + 4.6 / 76.0).
 struct RotateBack {
   const void *cos, *sin;  // [max_pos][D / 2] of the gradients' type; null: nothing is rotated
   const int32_t* positions;  // [B, S], or null

@@ -318,7 +318,8 @@ __device__ __forceinline__ void rotate(float& even, float& odd, float c, float s
   odd = round_to<T>(xe * s) + round_to<T>(xo * c);
 }
 // Buffer stores past the caches: of what is not read again before more than they hold was written.  Gate and up that are kept for a backward pass are (16384 x 2 x 688 x 384 48 -> 35 us,
-// 8192 x 2 x 1376 x 512 46 -> 40, 4096 x 2 x 1024 x 256 14.1 -> 12.9); so is h beside them where it exceeds the 32 MB of the eight L2s (16384 x 2 x 1376 x 512 94 -> 92 without it,
+// 8192 x 2 x 1376 x 512 46 -> 40, 4096 x 2 x 1024 x 256 14.1 -> 12.9), also where the last-level cache would hold them until then (the training step of the 50M model from a graph, gate and up cached /
+// past the caches: 512 tokens 1421 / 1421, 1023 1761 / 1751, 2046 2329 / 2317, 3000 2863 / 2853, 4092 3326 / 3305, 6000 4485 / 4425, 8192 5601 / 5548, 16384 8870 / 8783); so is h beside them where it exceeds the 32 MB of the eight L2s (16384 x 2 x 1376 x 512 94 -> 92 without it,
 // -> 74; a training step of 16384 tokens of the 50M model 8777 -> 8674, of 4000 tokens 3201 -> 3188).  Below that, and where gate and up are not kept, the product behind reads h out of the
 // caches (evaluation of 2331 tokens with h past them 617 -> 649).  No gain, or a loss, in steps: the rotated q, k, v, dense C, d gate and d up likewise, gate and up read so.
 constexpr int kNontemporal = 2;
@@ -692,7 +693,7 @@ __device__ __forceinline__ void gemm_tile(const Product& g, const Tile& tile, un
       }
     if (__builtin_amdgcn_ballot_w64(finite != 0.f)) {
       // Infinities, NaN, and numbers that leave the range of the scaled parts or of their sums: blocks of this wavefront that have such elements once more, by fp32 matrix instructions straight
-      // from memory (a tenth of the speed or less).  The others of a block stay as they are, so that an element's bits depend on its own row and column alone; and what lies beside the operands in
+      // from memory (us, 4096 x 2048 x 2048: 183, with a row of NaN 335, all NaN 1908; elements of 1e-36 192).  The others of a block stay as they are, so that an element's bits depend on its own row and column alone; and what lies beside the operands in
       // memory, which lanes past the last row or column may hold, is no reason.
 #pragma unroll
       for (int i = 0; i < MB; ++i)
@@ -1129,7 +1130,7 @@ struct LaunchPlan {
   int64_t workspace = 0;             // bytes
 
   // All products in one launch of small (in fp32 also 32 x 32) or of 128 x 128 tiles, or each by itself.  A weight gradient's split is the one it has alone (in fp32, on these tiles), so that
-  // in bf16 its bits do not depend on what shares its launch.  activation: an NN product that is not split, whose output goes through the activation
+  // in bf16 its bits do not depend on what shares its launch; in fp32 they may, with the tile (mlts_gemm_multi says so).  activation: an NN product that is not split, whose output goes through the activation
   LaunchPlan(const mlts_gemm_product* ps, int count, int dtype, bool activation = false, bool rotation = false) {
     const Costs& costs = costs_of(dtype);
     const mlts_gemm_product* all[kMaxProducts];

@@ -46,7 +46,7 @@ constexpr double kOwnLimitBf16 = 4.0e9;
 //     whole ones, 10000 terms on     up to 128 tiles 0.65 to 1.07; 129 to 192 (16384 x 768, 40000 x 256: part of the CUs idle in the last round) 0.73 to 1.11; more 0.73 to 0.98
 //     others                         16384 x 384 and x 512 below 10000 terms 0.91 to 1.22; 20000 x 512, 24576 x 384, 40000 x 256, 50264 x 256 0.82 to 1.57; 32000 x 512 0.93 to 1.06
 //     In one launch with dh = dy W and the activation -2 to -107 at all row counts up to 32768; that dh without its dW up to +74.
-// These were measured on tiles of 128 x 128 where 256 x 128 is taken since (y of 512 x 1376, 16384 rows, 39 us, now 34).
+// These were measured on tiles of 128 x 128 where 256 x 128 is taken since (y of 512 x 1376, 16384 rows, 39 us, now 34), and dW of fewer than 8192 rows before its 256 x 256 had a ring of stages.
 // (With the shipped per-shape selection, 16384 rows, alone: y 512 x 512 17 us against 16, 1536 x 512 42 / 32, in a step rotated on its way out 48 / 32 + 15,
 // 512 x 1376 34 / 40, 2752 x 512 65 / 73; dW 512 x 1376 41 / 45, 1536 x 512 41 / 37, 2752 x 512 63 / 58.)  Products with the columns of a vocabulary (32000 x 512): 1023 rows
 // 54 / 49, 3000 rows 136 / 131.
