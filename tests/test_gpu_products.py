@@ -471,6 +471,28 @@ def test_fp32_bits_of_an_element_are_those_of_its_row_and_column(dev, product, t
     assert torch.equal(*results)
 
 
+@pytest.mark.parametrize("M,N,K", [(700, 1028, 68), (2047, 1380, 36), (2048, 1376, 40)])
+def test_fp32_gate_up_out_of_the_range_of_the_parts(dev, M, N, K):
+    """Elements of x and of either weight without parts, in ragged tiles: the bits of the product with both weights, where those of the others stay."""
+    x, w = operands(NT, M, 2 * N, K, torch.float32, dev, M + N)
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    results = []
+    for out_of_range in (False, True):
+        if out_of_range:
+            x[3, 5], x[M - 1, K - 1], x[70, 0] = float("inf"), float("nan"), 3.4e38
+            w[7, 2], w[N - 1, 0], w[N + 65, 1], w[2 * N - 1, 3] = 2e32, float("-inf"), float("nan"), 3.4e38
+        wg, wu = w[:N], w[N:]
+        gate, up, h, both = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev), torch.empty(M, N, device=dev), torch.empty(M, 2 * N, device=dev)
+        assert L.mlts_gemm_swiglu_supports(_lib.MLTS_F32, M, N, K, K, K, N, N) is None and planned([(NT, M, N, K)], _lib.MLTS_F32, 3)[0][0] >= 64
+        _lib.check(L.mlts_gemm_swiglu(_lib.MLTS_F32, M, N, K, x.data_ptr(), K, wg.data_ptr(), wu.data_ptr(), K, gate.data_ptr(), up.data_ptr(), N, h.data_ptr(), N, st))
+        run_products([(NT, [(x, w)], both, 0)], torch.float32)
+        results.append((both, torch.cat([gate, up], 1)))
+        assert torch.equal(results[-1][0].nan_to_num(), results[-1][1].nan_to_num()) and torch.equal(both.isnan(), results[-1][1].isnan())
+    rows, columns = torch.ones(M, dtype=torch.bool, device=dev), torch.ones(2 * N, dtype=torch.bool, device=dev)
+    rows[[3, M - 1, 70]], columns[[7, N - 1, N + 65, 2 * N - 1]] = False, False
+    assert torch.equal(results[0][1][rows][:, columns], results[1][1][rows][:, columns])
+
+
 def test_fp32_sum_over_segments_in_slices(dev):
     """A sum over segments whose slabs are split over workgroups, alone and beside a weight gradient: slices that begin and end within segments."""
     gen = torch.Generator().manual_seed(8)
